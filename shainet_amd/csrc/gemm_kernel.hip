@@ -3,26 +3,26 @@
 // reference's GPU branch calls cuBLAS SGEMM (llama_block.cr:726-768, cuda.cr:237-247) and its CPU
 // branch SimpleMatrix#* (simple_matrix.cr:61-74).
 //
-// A workgroup of four wavefronts owns a 128 x 128 tile of y; each wavefront owns 32 of its rows
-// and all 128 columns (four blocks of v_mfma_f32_32x32x2_f32) and the workgroup walks K in steps
-// of 32; two workgroups share a compute unit, so that each SIMD holds two wavefronts and one's
-// barrier and memory waits hide behind the other's MFMAs (256 x 128 tiles, one workgroup per
-// compute unit and twice the MFMAs per LDS read, were 7 % slower: 128 against 137 TFLOP/s).  Both operands go global memory -> registers -> LDS (two LDS stages, one barrier per
-// step) and are read from LDS with ds_read_b128:
-//   x tile [rows][32 k], row stride 36 floats: a lane reads four consecutive k of its row;
-//   W tile [32 k][128 columns] as it lies in memory: lane n of a block owns columns 4 n + b of
-//     the four blocks b, so one 16-byte read of a W row feeds the four blocks, and a lane's
-//     results for one row of y are four neighbouring columns (16-byte stores).
-// An MFMA may visit the contraction index in any order as long as both operands agree: MFMA i of
-// a k step of 8 takes k = 8 s + 4 j + i from lane half j, on both sides.
-// MFMA 32x32x2 layout (lane l): A[m = l % 32][k = l / 32], B[k = l / 32][n = l % 32],
-// D[m = 8 (r / 4) + 4 (l / 32) + r % 4][n = l % 32] for accumulator register r.
-// Tile loads take a scalar base that moves along K plus a per-thread 32-bit offset, so the loop
-// holds next to no vector instructions besides the MFMAs (fp32 MFMAs run on the vector ALU's
-// lanes: every other vector instruction is paid in matrix throughput).
+// The product runs on the bf16 matrix cores, each operand as the exact sum of three bf16 numbers
+// (split_mfma.hpp).  A workgroup of 2 x WN wavefronts owns a tile of 64 MB rows and 64 WN columns of y; each
+// wavefront owns MB x 2 blocks of 32 x 32 and the workgroup walks K in steps of 16.
+// A step's tiles go global memory -> registers (one or two steps ahead) -> split -> LDS (two stages, one
+// barrier per step), where the fragments of an MFMA lie as it takes them: unit [part][octet of k][row or
+// column] of 16 bytes, so that 32 lanes read 512 consecutive bytes.
+//   x: a thread takes an octet of k of a row, or half of one;
+//   W: a thread takes 8 rows of one column, so that the pairs of k that share a register come from two of
+//      its registers and nothing has to be transposed.  Column c of a wavefront's 64 lies in block c % 2 at
+//      place c / 2: a lane's two blocks are neighbouring columns of y (8-byte stores, 256 bytes a row).
+// Tile loads take a scalar base that moves along K plus a per-thread 32-bit offset.
+// What bounds it: large shapes the power the card may draw.  4096 rows of 2048 -> 16384 run at 232 TFLOP/s
+// with N(0, 1) operands and at 295 with zeros (71 % of the six products' rate); with four wavefronts on
+// 128 x 128 tiles it was 183 and 252, so the large tile, which reads LDS 3/4 as often and splits half as much
+// per product, is worth more than a better schedule (an order forced between MFMAs and splits, three
+// workgroups per compute unit: 1 to 6 % slower).  The fp32 instruction it replaces, in tiles of 128 x 128,
+// reached 137.  Small shapes: a launch, the first loads' way, and the kernel that adds the pieces.
 //
 // Work is counted in units of one K step of one tile.  When the tiles do not fill whole rounds of
-// the chip (512 workgroups run at once), the units are dealt out evenly instead: a workgroup takes
+// the chip, the units are dealt out evenly instead: a workgroup takes
 // a contiguous run of units, which may end inside a tile (it leaves that piece as a partial product
 // in its own slot of a scratch array and marks the slot's flag word) and may begin inside one (it
 // then finishes that tile: waits for the flag words of the workgroups that hold the tile's earlier
@@ -37,6 +37,8 @@
 // kernel, with the whole chip, adds the pieces in a fixed order (and the residual).
 #include "gemm_kernel.hpp"
 
+#include "split_mfma.hpp"
+
 #include <stdint.h>
 #include <stdlib.h>
 
@@ -44,13 +46,7 @@ namespace shainet {
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int TN = 128, TK = 32;
-constexpr int AS = TK + 4;  // padded row stride of the x tile: conflict-free 16-byte reads down a column of rows
-
-#define ORDER_LDS_AND_MFMA() __builtin_amdgcn_sched_barrier(0x7)
+constexpr int TK = 16;
 
 // A partial product is read by a workgroup that may sit on another XCD, whose L2 is not kept
 // coherent with this one's for ordinary accesses: the store is written through to memory.
@@ -69,13 +65,13 @@ struct GemmArgs {
   const float *res;  // nullable: y = res + x W
   const float *bias;  // nullable: y = act(x W + bias)
   Activation act;
-  float *partials;   // [workgroups][128 * 128]: the piece a workgroup leaves unfinished
+  float *partials;   // [workgroups][a tile]: the piece a workgroup leaves unfinished
   unsigned *flags;   // [workgroups], zero between launches
   unsigned *flag_set;  // where a piece is marked complete: `flags`, or elsewhere in the test of the give-up path
   int spin_limit;    // polls before a wait for a flag word is given up
   int *error;        // set to 1 then
   int T, K, N, tiles_m;
-  int steps;            // K steps of 32 per tile
+  int steps;            // K steps of 16 per tile
   int group_bits;       // workgroup id -> group id & (groups - 1), place id >> group_bits
   int tiles_per_group;  // a group's workgroups share a contiguous run of tiles (row tiles fastest)
   int quota;            // units per workgroup
@@ -83,20 +79,40 @@ struct GemmArgs {
                         // is cut into this many pieces of `quota` steps, a workgroup each, all left in their slots
 };
 
-// v: four neighbouring columns from `col` on
-__device__ __forceinline__ f32x4 add_bias(const GemmArgs &g, f32x4 v, int col) {
-  const f32x4 b = *(const f32x4 *)(g.bias + col);
-  return f32x4{activate(g.act, v.x + b.x), activate(g.act, v.y + b.y), activate(g.act, v.z + b.z), activate(g.act, v.w + b.w)};
+// v: columns col and col + 1 of x W; rows past the last one are dropped
+__device__ __forceinline__ void store_pair(const GemmArgs &g, int row, int col, f32x2 v) {
+  if (row >= g.T) return;
+  const long long o = (long long)row * g.N + col;
+  if (g.bias) {
+    const f32x2 b = *(const f32x2 *)(g.bias + col);
+    v = f32x2{activate(g.act, v.x + b.x), activate(g.act, v.y + b.y)};
+  }
+  if (g.res) {
+    const f32x2 r = *(const f32x2 *)(g.res + o);
+    v = f32x2{r.x + v.x, r.y + v.y};
+  }
+  *(f32x2 *)(g.y + o) = v;
 }
 
-// GUARD: K need not be a multiple of 32 (pieces beyond its end are loaded as zeros); without it
-// every load of the loop is unconditional.
-template <bool GUARD>
-__global__ __launch_bounds__(256, 2) void sgemm_mfma_kernel(const GemmArgs g) {
-  constexpr int TM = 128;
-  constexpr int NA = 4;  // float4 of the x tile per thread
-  __shared__ __attribute__((aligned(16))) float As[2][TM * AS];
-  __shared__ __attribute__((aligned(16))) float Bs[2][TK * TN];
+// Units of 16 bytes in a stage of LDS.  A part of x: two octets of TM rows, four units apart from a multiple
+// of 16 (a wavefront writes both octets of 32 rows); a part of W: two octets of two wavefronts' two blocks of 32
+// columns, four units of padding behind each (neighbouring columns lie in two blocks).
+template <int MB, int WN>
+struct Stage {
+  static constexpr int kOctX = 64 * MB + 4, kPartX = 2 * kOctX;
+  static constexpr int kOctW = 2 * WN * 36, kPartW = 2 * kOctW;
+  static constexpr int kUnits = 3 * (kPartX + kPartW);
+};
+
+// GUARD: K need not be a multiple of 16 (pieces beyond its end are zeros).
+template <int MB, int WN, bool GUARD>
+__global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs g) {
+  constexpr int TM = 64 * MB, TN = 64 * WN;
+  constexpr int NX = 2 * MB / WN;  // float4 of the x tile per thread
+  constexpr int kSets = MB == 4 ? 1 : 2;
+  using S = Stage<MB, WN>;
+  static_assert(NX == 2 || NX == 1, "a thread stages an octet of x, or half of one");
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2][S::kUnits];
 
   // Workgroups go to the eight XCDs round-robin by index: the workgroups of a group (index modulo
   // the group count, a power of two up to 8) stay on the same XCDs and share a run of tiles, whose
@@ -115,26 +131,19 @@ __global__ __launch_bounds__(256, 2) void sgemm_mfma_kernel(const GemmArgs g) {
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ln = lane & 31, j = lane >> 5;
+  const int ln = lane & 31, j = lane >> 5, wm = wave / WN, wn = wave % WN;
   const int T = g.T, K = g.K, N = g.N;
 
-  // staging: x tile, NA float4 per thread: row = idx / 8, k piece = idx % 8 (rows past the last
-  // one repeat it: their products are never stored); W tile, 4 float4 per thread: row = idx / 32,
-  // columns 4 (idx % 32) .. + 3 (columns past the last one repeat the last four: never stored)
-  int a_lds[NA], b_lds[4];
-#pragma unroll
-  for (int u = 0; u < NA; ++u) {
-    const int idx = threadIdx.x + 256 * u;
-    a_lds[u] = (idx >> 3) * AS + 4 * (idx & 7);
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int idx = threadIdx.x + 256 * u;
-    b_lds[u] = (idx >> 5) * TN + 4 * (idx & 31);
-  }
-  // operand fragments of one k step of 8: x rows (four k each), W rows per MFMA i (four columns =
-  // the four blocks each)
-  const int a_off = (wave * 32 + ln) * AS + 4 * j, b_off = 4 * j * TN + 4 * ln;
+  // staging: x: octet tid % 2 of row tid / 2, or half an octet, quarter tid % 4 of row tid / 4; W: octet tid / TN
+  // of column tid % TN
+  const int xrow = NX == 1 ? threadIdx.x >> 2 : threadIdx.x >> 1;
+  const int xk = NX == 1 ? 4 * (threadIdx.x & 3) : 8 * (threadIdx.x & 1);
+  const int wcol = threadIdx.x & (TN - 1), wk = 8 * (threadIdx.x / TN);
+  const int x_unit = (xk >> 3) * S::kOctX + xrow;
+  const int w_unit = 3 * S::kPartX + (wk >> 3) * S::kOctW + (wcol >> 6) * 72 + (wcol & 1) * 36 + ((wcol & 63) >> 1);
+  // fragments
+  const int a_unit = j * S::kOctX + wm * 32 * MB + ln;
+  const int b_unit = 3 * S::kPartX + j * S::kOctW + wn * 72 + ln;
   const long long w_step = (long long)TK * N * 4;
 
   for (int visit = 0; visit <= t_last - t_first; ++visit) {
@@ -148,128 +157,163 @@ __global__ __launch_bounds__(256, 2) void sgemm_mfma_kernel(const GemmArgs g) {
     const int k_begin = s_begin * TK, k_end = min(K, s_end * TK);
     const int nk = s_end - s_begin;
 
-    unsigned x_off[NA], w_off[4];
-#pragma unroll
-    for (int u = 0; u < NA; ++u) {
-      const int idx = threadIdx.x + 256 * u;
-      x_off[u] = (unsigned)(((long long)min(m0 + (idx >> 3), T - 1) * g.xs + 4 * (idx & 7)) * 4);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int idx = threadIdx.x + 256 * u;
-      w_off[u] = (unsigned)(((long long)(idx >> 5) * N + min(n0 + 4 * (idx & 31), N - 4)) * 4);
-    }
+    // (rows past the last one repeat it and columns likewise: their products are never stored)
+    const unsigned x_off = (unsigned)(((long long)min(m0 + xrow, T - 1) * g.xs + xk) * 4);
+    const unsigned w_off = (unsigned)(((long long)wk * N + min(n0 + wcol, N - 1)) * 4);
     const char *x_base = (const char *)(g.x + k_begin);
     const char *w_base = (const char *)(g.w + (long long)k_begin * N);
 
     // two register sets: the tiles of step t travel in set t & 1 and are requested two steps ahead
-    // (one step, 1.7 us of MFMAs, is not always enough for a load to come back: 114 against 125 TFLOP/s)
-    f32x4 sa[2][NA], sb[2][4];
-    int k_next = k_begin;
-    auto load_tiles = [&](f32x4 (&ra)[NA], f32x4 (&rb)[4]) {
+    f32x4 sx[kSets][NX];
+    float sw[kSets][8];
+    int k_next = k_begin, to_load = nk;
+    auto load_tiles = [&](f32x4 (&rx)[NX], float (&rw)[8]) {
 #pragma unroll
-      for (int u = 0; u < NA; ++u) {
-        const int c4 = (threadIdx.x + 256 * u) & 7;
-        if (GUARD)  // a piece beyond the end of K contributes nothing: zero on the x side is enough
-          ra[u] = k_next + 4 * c4 < k_end ? *(const f32x4 *)(x_base + x_off[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
-        else
-          ra[u] = *(const f32x4 *)(x_base + x_off[u]);
+      for (int u = 0; u < NX; ++u) {
+        const int kk = k_next + xk + 4 * u;
+        const char *p = x_base + x_off + 16 * u;
+        rx[u] = !GUARD || kk < k_end ? *(const f32x4 *)p : f32x4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int row = (threadIdx.x + 256 * u) >> 5;
-        if (GUARD)
-          rb[u] = k_next + row < k_end ? *(const f32x4 *)(w_base + w_off[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
-        else
-          rb[u] = *(const f32x4 *)(w_base + w_off[u]);
+      for (int i = 0; i < 8; ++i)
+        rw[i] = !GUARD || k_next + wk + i < k_end ? *(const float *)(w_base + (long long)i * N * 4 + w_off) : 0.f;
+      if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
+        x_base += TK * 4;
+        w_base += w_step;
+        k_next += TK;
       }
-      x_base += TK * 4;
-      w_base += w_step;
-      k_next += TK;
     };
-    auto park_tiles = [&](const f32x4 (&ra)[NA], const f32x4 (&rb)[4], int buf) {
+    auto park_tiles = [&](const f32x4 (&rx)[NX], const float (&rw)[8], u32x4 *stage) {
+      u32x4 h, m, l;
 #pragma unroll
-      for (int u = 0; u < NA; ++u) *(f32x4 *)&As[buf][a_lds[u]] = ra[u];
+      for (int i = 0; i < 4; ++i) {
+        unsigned a, b, c;
+        split_pair(rw[2 * i], rw[2 * i + 1], a, b, c);
+        h[i] = a, m[i] = b, l[i] = c;
+      }
+      stage[w_unit] = h;
+      stage[w_unit + S::kPartW] = m;
+      stage[w_unit + 2 * S::kPartW] = l;
+      if (NX == 1) {
+        unsigned a[2], b[2], c[2];
+        split_pair(rx[0].x, rx[0].y, a[0], b[0], c[0]);
+        split_pair(rx[0].z, rx[0].w, a[1], b[1], c[1]);
+        u32x2 *half = (u32x2 *)(stage + x_unit) + ((xk >> 2) & 1);
+        half[0] = u32x2{a[0], a[1]};
+        half[2 * S::kPartX] = u32x2{b[0], b[1]};
+        half[4 * S::kPartX] = u32x2{c[0], c[1]};
+      } else {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) *(f32x4 *)&Bs[buf][b_lds[u]] = rb[u];
+        for (int i = 0; i < 4; ++i) {
+          const f32x4 v = rx[i >> 1];
+          unsigned a, b, c;
+          split_pair(i & 1 ? v.z : v.x, i & 1 ? v.w : v.y, a, b, c);
+          h[i] = a, m[i] = b, l[i] = c;
+        }
+        stage[x_unit] = h;
+        stage[x_unit + S::kPartX] = m;
+        stage[x_unit + 2 * S::kPartX] = l;
+      }
     };
 
-    f32x16 acc[4];
+    f32x16 acc[MB][2];
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
-
-    f32x4 af[2], bf[2][4];  // [k step parity]
-    auto fetch = [&](int par, int buf, int s) {
-      af[par] = *(const f32x4 *)&As[buf][a_off + 8 * s];
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) bf[par][i] = *(const f32x4 *)&Bs[buf][b_off + (8 * s + i) * TN];
-    };
+        for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
     // (after the last barrier of the tile before this one nobody reads LDS any more)
-    load_tiles(sa[0], sb[0]);
-    if (nk > 1) load_tiles(sa[1], sb[1]);
-    park_tiles(sa[0], sb[0], 0);
-    if (nk > 2) load_tiles(sa[0], sb[0]);
+    load_tiles(sx[0], sw[0]);
+    if (kSets == 2) load_tiles(sx[kSets - 1], sw[kSets - 1]);
+    park_tiles(sx[0], sw[0], lds[0]);
+    load_tiles(sx[0], sw[0]);
     __syncthreads();
-    fetch(0, 0, 0);
 
-    // Per step of 32 along K: the MFMAs of the four k steps of 8 run with the fragments of each
-    // fetched one k step ahead; before the last of them (its fragments are in registers by then)
-    // the next step's tiles go from their registers to the other LDS stage, the one barrier of the
-    // step follows, the tiles of a later step are requested into the registers just freed, and the
-    // first fragments of the next step are fetched: neither the barrier nor an LDS round trip
-    // stands between two steps' MFMAs.
-    auto step = [&](const int kt, f32x4 (&ra)[NA], f32x4 (&rb)[4]) {  // ra, rb: the set that holds step kt + 1
-      const int buf = kt & 1;
-      const bool more = kt + 1 < nk;
+    // Per step of 16 along K: the fragments are fetched, the next step's tiles are split and go to the other
+    // stage while the MFMAs run, the tiles of a later step are requested into the registers just freed, one barrier.
+    auto step = [&](const int kt, f32x4 (&rx)[NX], float (&rw)[8]) {  // rx, rw: the set that holds step kt + 1
+      const u32x4 *stage = lds[kt & 1];
+      u32x4 af[3][MB], bf[3][2];
 #pragma unroll
-      for (int s = 0; s < TK / 8; ++s) {
-        const int cur = s & 1, nxt = cur ^ 1;
-        if (s + 1 < TK / 8) {
-          fetch(nxt, buf, s + 1);
-        } else {
-          if (more) park_tiles(ra, rb, buf ^ 1);
-          __syncthreads();
-          if (kt + 3 < nk) load_tiles(ra, rb);
-          if (more) fetch(nxt, buf ^ 1, 0);
-        }
-        ORDER_LDS_AND_MFMA();
-        // the accumulators take turns: no MFMA waits for the one before it
+      for (int p = 0; p < 3; ++p) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * S::kPartX + 32 * a];
 #pragma unroll
-          for (int b = 0; b < 4; ++b)
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[cur][i], bf[cur][i][b], acc[b], 0, 0, 0);
-        ORDER_LDS_AND_MFMA();
+        for (int b = 0; b < 2; ++b) bf[p][b] = stage[b_unit + p * S::kPartW + 36 * b];
       }
+      park_tiles(rx, rw, lds[(kt & 1) ^ 1]);
+      load_tiles(rx, rw);
+      // smallest products first; the blocks take turns, no MFMA waits for the one before it
+      constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int a = 0; a < MB; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[pa[p]][a], bf[pb[p]][b], acc[a][b]);
+      __syncthreads();
     };
     for (int kt = 0; kt < nk; kt += 2) {
-      step(kt, sa[1], sb[1]);
-      if (kt + 1 < nk) step(kt + 1, sa[0], sb[0]);
+      step(kt, sx[kSets - 1], sw[kSets - 1]);
+      if (kt + 1 < nk) step(kt + 1, sx[0], sw[0]);
     }
 
-    // A piece travels as [register r][thread] float4: consecutive threads, consecutive 16 bytes.
-    constexpr long long kSlot = (long long)TM * TN;
-    f32x4 out[16];
+    const int row0 = m0 + wm * 32 * MB + 4 * j, col = n0 + wn * 64 + 2 * ln;
+    // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which
+    float probe = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) out[r] = f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
-    // (the thread's offset is taken afresh per tile, or the compiler computes all sixteen addresses
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) probe = fmaf(acc[a][b][r], 0.f, probe);
+    if (__any(probe != 0.f)) {
+#pragma unroll
+      for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+#pragma clang loop unroll(disable)
+      for (int k = k_begin; k < k_end; ++k) {
+        const float *wr = g.w + (long long)k * N;
+        const float w0 = wr[min(col, N - 1)], w1 = wr[min(col + 1, N - 1)];
+#pragma unroll
+        for (int a = 0; a < MB; ++a)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const float xv = g.x[(long long)min(row0 + 32 * a + 8 * (r >> 2) + (r & 3), T - 1) * g.xs + k];
+            acc[a][0][r] = fmaf(xv, w0, acc[a][0][r]);
+            acc[a][1][r] = fmaf(xv, w1, acc[a][1][r]);
+          }
+      }
+    }
+
+    // A piece travels as [pair of rows][thread] float4: consecutive threads, consecutive 16 bytes.
+    constexpr long long kSlot = (long long)TM * TN;
+    f32x4 out[8 * MB];
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]};
+    // (the thread's offset is taken afresh per tile, or the compiler computes all addresses
     // before the loops and keeps them in scratch memory)
     int in_slot = 4 * threadIdx.x;
     asm volatile("" : "+v"(in_slot));
     if (g.pieces) {  // the second kernel adds the pieces
       float *slot = g.partials + blockIdx.x * kSlot + in_slot;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) *(f32x4 *)(slot + r * 1024) = out[r];
+      for (int r = 0; r < 8 * MB; ++r) *(f32x4 *)(slot + r * 512 * WN) = out[r];
       return;
     }
     if (s_end < steps) {
       float *slot = g.partials + blockIdx.x * kSlot + in_slot;
       __builtin_amdgcn_sched_barrier(0);  // all of out[] is in place before the first store is issued
 #pragma unroll
-      for (int r = 0; r < 16; ++r) coherent_store4(slot + r * 1024, out[r]);
+      for (int r = 0; r < 8 * MB; ++r) coherent_store4(slot + r * 512 * WN, out[r]);
       // the stores are acknowledged (s_waitcnt vmcnt(0): the barrier alone does not wait for them)
       // before the piece is marked complete
       __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -305,52 +349,45 @@ __global__ __launch_bounds__(256, 2) void sgemm_mfma_kernel(const GemmArgs g) {
       const float *piece = g.partials + (long long)((p_first << g.group_bits) | group) * kSlot + in_slot;
       const long long piece_step = kSlot << g.group_bits;
       for (int i = 0; i < n_before; ++i) {
-        f32x4 v[16];
+        f32x4 v[8 * MB];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = *(const f32x4 *)(piece + i * piece_step + r * 1024);
-        __builtin_amdgcn_sched_barrier(0);  // all sixteen loads in flight before the first sum waits
+        for (int r = 0; r < 8 * MB; ++r) v[r] = *(const f32x4 *)(piece + i * piece_step + r * 512 * WN);
+        __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first sum waits
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[r] += v[r];
+        for (int r = 0; r < 8 * MB; ++r) out[r] += v[r];
       }
     }
-    const int col = n0 + 4 * ln;
-    if (col < N) {  // N is a multiple of 4: a lane's four columns are inside together
+    if (col < N) {  // N is a multiple of 4: a lane's two columns are inside together
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wave * 32 + 8 * (r >> 2) + 4 * j + (r & 3);
-        if (row < T) {
-          const long long o = (long long)row * N + col;
-          f32x4 v = out[r];
-          if (g.bias) v = add_bias(g, v, col);
-          if (g.res) v = *(const f32x4 *)(g.res + o) + v;
-          *(f32x4 *)(g.y + o) = v;
-        }
+      for (int r = 0; r < 8 * MB; ++r) {
+        const int row = row0 + 32 * (r >> 3) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
+        store_pair(g, row, col, f32x2{out[r].x, out[r].y});
+        store_pair(g, row + 1, col, f32x2{out[r].z, out[r].w});
       }
     }
   }
 }
 
 // y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order.  A piece lies in its
-// workgroup's slot as [register r][thread] float4, the layout of the product kernel's accumulators.
-__global__ __launch_bounds__(256) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
-  const int tile = blockIdx.x >> 4, r = blockIdx.x & 15;  // sixteen workgroups per tile, a register each
+// workgroup's slot as [pair of rows][thread] float4, the layout of the product kernel's accumulators.
+template <int MB, int WN>
+__global__ __launch_bounds__(128 * WN) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
+  const int tile = blockIdx.x / (8 * MB), r = blockIdx.x % (8 * MB);  // 8 MB workgroups per tile, a pair of rows of each thread each
   if (tile >= tiles) return;
   const int group = tile / g.tiles_per_group, t = tile - group * g.tiles_per_group;
-  constexpr long long kSlot = 128LL * TN;
-  const float *piece = g.partials + (long long)(((t * g.pieces) << g.group_bits) | group) * kSlot + r * 1024 + 4 * threadIdx.x;
+  constexpr int TN = 64 * WN;
+  constexpr long long kSlot = 64LL * MB * TN;
+  const float *piece = g.partials + (long long)(((t * g.pieces) << g.group_bits) | group) * kSlot + r * 512 * WN + 4 * threadIdx.x;
   const long long piece_step = kSlot << g.group_bits;
   const int n = min(g.pieces, (g.steps + g.quota - 1) / g.quota);  // pieces that hold any steps
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = (tile % g.tiles_m) * 64 * MB + (wave / WN) * 32 * MB + 32 * (r >> 3) + 4 * (lane >> 5) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
+  const int col = (tile / g.tiles_m) * TN + (wave % WN) * 64 + 2 * (lane & 31);
+  if (row >= g.T || col >= g.N) return;
   f32x4 acc = *(const f32x4 *)piece;
   for (int c = 1; c < n; ++c) acc += *(const f32x4 *)(piece + c * piece_step);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = (tile % g.tiles_m) * 128 + wave * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-  const int col = (tile / g.tiles_m) * TN + 4 * (lane & 31);
-  if (row < g.T && col < g.N) {
-    const long long o = (long long)row * g.N + col;
-    if (g.bias) acc = add_bias(g, acc, col);
-    if (g.res) acc = *(const f32x4 *)(g.res + o) + acc;
-    *(f32x4 *)(g.y + o) = acc;
-  }
+  store_pair(g, row, col, f32x2{acc.x, acc.y});
+  store_pair(g, row + 1, col, f32x2{acc.z, acc.w});
 }
 
 // Any shape (K or N not a multiple of 4, unaligned rows): one thread per element of y, W read
@@ -373,17 +410,50 @@ __global__ __launch_bounds__(256) void sgemm_plain_kernel(const float *__restric
 
 }  // namespace
 
+namespace {
+
+// workgroups the chip runs at once: two of four wavefronts per compute unit, or one of eight
+int slots_of(int wn) { return wn == 4 ? 256 : 512; }
+
+// The tile, by what was measured (us, 2048 -> 3072 | 2048 -> 2048 | 2048 -> 16384 | 8192 -> 2048 | 1024 -> 8192):
+//   rows   64 x 128                    128 x 128                  128 x 256                  256 x 256
+//     45   19 | 17 | 42 | 31 | 19      23 | 19 | 59 | 37 | 24
+//    100   22 | 21 | 69 | 41 | 24      23 | 20 | 62 | 39 | 26
+//    256   31 | 25 | 125 | 68 | 40     33 | 28 | 106 | 62 | 37    31 | 27 | 108 | 59 | 37
+//    512                               47 | 37 | 185 | 106 | 57   45 | 36 | 177 | 102 | 58   52 | 44 | 192 | 100 | 64
+//   1024                               87 | 58 | 360 | 197 | 96   82 | 57 | 342 | 186 | 88   80 | 63 | 315 | 173 | 116
+//   2048                               148 | 100 | 717 | 372 | 187  143 | 99 | 674 | 346 | 181  144 | 100 | 619 | 323 | 164
+// A low tile wastes least on few rows; where the weights are small it is also the faster one in two rounds.
+// The largest needs long runs: at least 36 steps a workgroup, and no tile that two of them share by waiting.
+void choose_tile(GemmPlan &p, int T, int K, int N) {
+  p.wn = 2;
+  if (T <= 64 || (T <= 128 && (long long)K * N <= 12 << 20)) {
+    p.mb = 1;
+    return;
+  }
+  p.mb = 2;
+  if (T <= 256) return;
+  p.wn = 4;
+  const long long rows2 = (T + 127) / 128 * 128LL, rows4 = (T + 255) / 256 * 256LL;
+  const long long tiles = rows4 / 256 * ((N + 255) / 256), run = tiles * p.steps / slots_of(4);
+  if (rows4 * 100 <= rows2 * 115 && run >= 36 && (tiles >= slots_of(4) || 2 * run < p.steps)) p.mb = 4;
+}
+
+}  // namespace
+
 GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
   GemmPlan p = {};
   // (the kernel addresses the rows of x by 32-bit byte offsets from a base that moves along K)
   p.mfma = T >= 1 && K >= 4 && N >= 4 && (K & 3) == 0 && (N & 3) == 0 && (x_stride & 3) == 0 &&
            (long long)T * x_stride * 4 < 0xffffffffLL && (long long)TK * N * 4 < 0xffffffffLL;
-  p.tiles_m = (T + 127) / 128;
+  p.steps = (K + TK - 1) / TK;
+  choose_tile(p, T, K, N);
+  const int TN = 64 * p.wn;
+  p.tiles_m = (T + 64 * p.mb - 1) / (64 * p.mb);
   p.tiles_n = (N + TN - 1) / TN;
   if (!p.mfma) return p;
-  const int slots = 512;  // workgroups the chip runs at once: two per compute unit
+  const int slots = slots_of(p.wn);
   const int tiles = p.tiles_m * p.tiles_n;
-  p.steps = (K + TK - 1) / TK;
   // groups of workgroups that stay on the same XCDs: as many (of 8, 4, 2, 1) as divide the tiles evenly
   p.group_bits = 3;
   while (tiles & ((1 << p.group_bits) - 1)) --p.group_bits;
@@ -396,9 +466,10 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
   }
   // Otherwise one round of workgroups shares the K steps of all tiles evenly.
   const long long units = (long long)p.tiles_per_group * p.steps;
+  const int least = 16;  // steps of 16: a workgroup's start and end must not outweigh its loop
   int places = slots / groups;
   int quota = (int)((units + places - 1) / places);
-  if (quota < 8) quota = p.steps < 8 ? p.steps : 8;  // a workgroup's start and end must not outweigh its loop
+  if (quota < least) quota = p.steps < least ? p.steps : least;
   if (2 * quota >= p.steps) {  // a tile is shared by two or three workgroups: the one that ends it adds the pieces
     p.quota = quota;
     p.workgroups = (int)((units + quota - 1) / quota) * groups;
@@ -408,7 +479,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
     // second kernel adds them
     int pieces = slots / tiles;
     static const int pieces_knob = getenv("SHAINET_HIP_GEMM_PIECES") ? atoi(getenv("SHAINET_HIP_GEMM_PIECES")) : 0;
-    if (pieces > 16) pieces = 16;  // (128 rows of 8192 -> 2048: 32 pieces 56 us, 16 pieces 48.5 us)
+    if (pieces > 16) pieces = 16;  // (45 rows of 8192 -> 2048: 32 pieces 35.2 us, 16 pieces 30.7 us)
     if (pieces_knob > 0) pieces = pieces_knob;  // SHAINET_HIP_GEMM_PIECES: a tuning knob
     if (pieces > p.steps / 8) pieces = p.steps / 8;
     if (pieces < 1) pieces = 1;
@@ -417,9 +488,27 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
     p.workgroups = tiles * pieces;
     if (pieces == 1) return p;  // (short K: a workgroup per tile after all)
   }
-  p.partial_floats = (size_t)p.workgroups * 128 * TN;
+  p.partial_floats = (size_t)p.workgroups * 64 * p.mb * TN;
   return p;
 }
+
+namespace {
+
+template <int MB, int WN>
+hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+  const dim3 grid((unsigned)p.workgroups);
+  if (g.K % TK != 0)
+    hipLaunchKernelGGL((sgemm_split_kernel<MB, WN, true>), grid, dim3(128 * WN), 0, stream, g);
+  else
+    hipLaunchKernelGGL((sgemm_split_kernel<MB, WN, false>), grid, dim3(128 * WN), 0, stream, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !g.pieces) return e;
+  const int tiles = p.tiles_m * p.tiles_n;
+  hipLaunchKernelGGL((sgemm_reduce_kernel<MB, WN>), dim3((unsigned)tiles * 8 * MB), dim3(128 * WN), 0, stream, g, tiles);
+  return hipGetLastError();
+}
+
+}  // namespace
 
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
                        unsigned *flags, int *error, int T, int K, int N, const GemmPlan &p, hipStream_t stream,
@@ -455,16 +544,8 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   g.tiles_per_group = p.tiles_per_group;
   g.quota = p.quota;
   g.pieces = p.pieces > 1 ? p.pieces : 0;
-  const dim3 grid((unsigned)p.workgroups);
-  if (K % TK != 0)
-    hipLaunchKernelGGL(sgemm_mfma_kernel<true>, grid, dim3(256), 0, stream, g);
-  else
-    hipLaunchKernelGGL(sgemm_mfma_kernel<false>, grid, dim3(256), 0, stream, g);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !g.pieces) return e;
-  const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL(sgemm_reduce_kernel, dim3((unsigned)tiles * 16), dim3(256), 0, stream, g, tiles);
-  return hipGetLastError();
+  if (p.wn == 4) return p.mb == 4 ? launch_tiles<4, 4>(g, p, stream) : launch_tiles<2, 4>(g, p, stream);
+  return p.mb == 2 ? launch_tiles<2, 2>(g, p, stream) : launch_tiles<1, 2>(g, p, stream);
 }
 
 }  // namespace shainet

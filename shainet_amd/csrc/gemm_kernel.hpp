@@ -8,8 +8,9 @@ namespace shainet {
 
 struct GemmPlan {
   bool mfma;              // false: K, N or the row stride of x is not a multiple of 4 -> the plain kernel
-  int tiles_m, tiles_n;   // 128 x 128 tiles of y
-  int steps;              // K steps of 32 per tile; a unit of work is one step of one tile
+  int mb, wn;             // tiles of y have 64 mb rows and 64 wn columns
+  int tiles_m, tiles_n;
+  int steps;              // K steps of 16 per tile; a unit of work is one step of one tile
   int group_bits;         // 2^group_bits groups of workgroups, each with an equal run of the tiles
   int tiles_per_group;
   int quota;              // consecutive units per workgroup (= steps: a workgroup per tile, nothing shared)

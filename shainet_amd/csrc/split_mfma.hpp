@@ -1,0 +1,47 @@
+// fp32 products on the bf16 matrix cores.  A float is the exact sum of three bf16 numbers, its value
+// rounded to bf16, the rest rounded to bf16, and the rest of that (8 + 8 + 8 mantissa bits with signs of
+// their own; a bf16 has a float's exponents).  Of the nine products of two such sums the six largest make
+// up the product to 2^-26 of itself; the three left out are at most 2^-27 of it each.  Six
+// v_mfma_f32_32x32x16_bf16 of 32 cycles do what eight v_mfma_f32_32x32x2_f32 of 64 do (192 against 512
+// cycles per 32 x 32 x 16; a loop of nothing else: 1876 TFLOP/s of bf16 = 312 of fp32, against 155), they
+// leave the vector ALU free meanwhile, which the fp32 instruction does not, and round the accumulator
+// 6/16 times per term instead of 1/2: measured against 64 bits the error is 0.8 to 0.95 of the fp32
+// instruction's for sums of 64 to 8192 terms.
+// What is not finite in an operand (or rounds to infinity: above 3.39e38) makes NaN of the sums it enters;
+// callers look for sums that are not finite and take those again in fp32.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace shainet {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// two floats rounded to bf16, the first in the low half
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+
+// the three parts of two floats, packed
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &high, unsigned &mid, unsigned &low) {
+  high = pack_bf16(a, b);
+  a -= __builtin_bit_cast(float, high << 16);
+  b -= __builtin_bit_cast(float, high & 0xffff0000u);
+  mid = pack_bf16(a, b);
+  a -= __builtin_bit_cast(float, mid << 16);
+  b -= __builtin_bit_cast(float, mid & 0xffff0000u);
+  low = pack_bf16(a, b);
+}
+
+// acc += a b; operands as 16-byte fragments: lane l holds k = 8 (l / 32) .. + 7 of row (column) l % 32.
+// D[m = 8 (r / 4) + 4 (l / 32) + r % 4][n = l % 32] in register r.
+__device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+}
+
+}  // namespace shainet

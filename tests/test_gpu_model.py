@@ -749,3 +749,50 @@ def test_load_llama_bf16_f16_sharded_qwen_style(hip, tmp_path):
     (tmp_path / "config.json").write_text(json.dumps(cfg))
     with pytest.raises(hip.ArgumentError, match="mixture-of-experts"):
         hip.HFLoader.load_llama(str(tmp_path))
+
+
+@pytest.mark.parametrize("T,K,N", [
+    (17, 4, 4), (64, 16, 132), (65, 20, 124),            # 64 x 128 tiles: one step, ragged columns, the guarded loads
+    (70, 2048, 6400), (129, 36, 128), (256, 528, 260),   # 128 x 128
+    (257, 16, 256), (300, 2052, 1028), (640, 512, 512),  # 128 x 256: whole and ragged, one step, pieces
+    (1024, 2048, 2308), (1000, 1040, 8192),              # 256 x 256: pieces and the kernel that adds them; whole tiles
+])
+def test_matmul_split_tiles(hip, T, K, N):
+    """Each tile of the product over split operands.  A sum is rounded 6 K / 16 times, each time by at most 2^-24 of
+    what has been added up, and the parts left out of a product are under 2^-24 of it; adding up to 16 pieces and
+    the residual rounds 17 times more."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    g = torch.Generator(device="cuda").manual_seed(T * K + N)
+    x = torch.randn((T, K), generator=g, device="cuda") * 10 ** (8 * torch.rand((T, 1), generator=g, device="cuda") - 4)
+    w = torch.randn((K, N), generator=g, device="cuda") / K ** 0.5
+    res = torch.randn((T, N), generator=g, device="cuda")
+    got = binding.matmul(x, w, res)
+    want = x.double() @ w.double() + res.double()
+    size = x.double().abs() @ w.double().abs() + res.double().abs()
+    off = (got.double() - want).abs()
+    assert bool((off <= 2.0 ** -24 * (6 * K / 16 + 18) * size).all()), float((off / size).max())
+    assert torch.equal(got, binding.matmul(x, w, res))
+
+
+@pytest.mark.parametrize("T", [40, 200, 300, 1100])
+def test_matmul_split_tiles_keep_what_is_not_finite(hip, T):
+    """Infinities, NaN and values that a bf16 would round to infinity come out as fp32 arithmetic has them."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn((T, 640), generator=g, device="cuda")
+    w = torch.randn((640, 8200), generator=g, device="cuda")
+    x[3, 5], x[T - 1, 639], w[7, 130], w[600, 8199] = float("inf"), float("-inf"), float("inf"), float("nan")
+    x[9], x[10, 1:], x[10, 0] = 0.0, 0.0, 3.4e38
+    w[0, :50] = 0.5
+    got, want = binding.matmul(x, w).cpu(), (x.double() @ w.double()).cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf() | (want.abs() > 3.4028235e38))
+    fine = got.isfinite()
+    assert bool(((got.double() - want).abs()[fine] <= 1e-4 * (1 + want.abs()[fine])).all())
+    assert got[10, 0].item() == np.float32(3.4e38) * np.float32(0.5)
