@@ -111,6 +111,16 @@ __global__ __launch_bounds__(256) void embed_kernel(const float *__restrict__ ta
   for (int j = threadIdx.x; j < d_model; j += 256) dst[j] = positions ? src[j] * scale + pos[j] : src[j] * scale;
 }
 
+// the same for ids that travel in the kernel's arguments
+__global__ __launch_bounds__(256) void embed_list_kernel(const float *__restrict__ table, const IdList list,
+                                                         float *__restrict__ out, int d_model, float scale,
+                                                         const float *__restrict__ positions) {
+  const float *src = table + (long long)list.id[blockIdx.x] * d_model;
+  float *dst = out + (long long)blockIdx.x * d_model;
+  const float *pos = positions + (positions ? (long long)blockIdx.x * d_model : 0);
+  for (int j = threadIdx.x; j < d_model; j += 256) dst[j] = positions ? src[j] * scale + pos[j] : src[j] * scale;
+}
+
 // Dynamic Tanh: no statistics over the row, so a workgroup takes 1024 columns of one row.
 __global__ __launch_bounds__(256) void dyn_tanh_kernel(const float *__restrict__ x, long long x_stride,
                                                        const float *__restrict__ gamma, const float *__restrict__ beta,
@@ -134,17 +144,31 @@ __global__ __launch_bounds__(256) void add_bias_row_kernel(float *__restrict__ l
   if (i < n) logits[i] = (float)((double)logits[i] + (double)bias[i]);
 }
 
-// The reference walks the ids in order and rewrites the logit once per occurrence,
-// so an id that repeats is penalised repeatedly; one thread keeps that order.
-__global__ void repetition_penalty_kernel(float *logits, int vocab, const int *ids, int n, double p) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  for (int i = 0; i < n; ++i) {
-    const int id = ids[i];
-    if (id >= 0 && id < vocab) {
-      const float v = logits[id];
-      logits[id] = (float)(v > 0.f ? (double)v / p : (double)v * p);
-    }
-  }
+// The reference walks the ids in order and rewrites the logit once per occurrence, so an id that repeats is
+// penalised repeatedly.  Different ids do not meet: the thread of an id's first place does all its occurrences.
+// The ids (a few dozen) travel in the kernel's arguments where they fit, without a copy to the device first.
+// 64 ids: 5 us; one thread that walks them, a memory round trip each, 22 us.
+__device__ __forceinline__ void penalise(float *__restrict__ logits, int vocab, const int *ids, int n, double p) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int id = i < n ? ids[i] : -1;
+  if (id < 0 || id >= vocab) return;
+  for (int j = 0; j < i; ++j)
+    if (ids[j] == id) return;
+  float v = logits[id];
+  for (int j = i; j < n; ++j)
+    if (ids[j] == id) v = (float)(v > 0.f ? (double)v / p : (double)v * p);
+  logits[id] = v;
+}
+__global__ __launch_bounds__(256) void repetition_penalty_kernel(float *__restrict__ logits, int vocab,
+                                                                 const int *__restrict__ ids, int n, double p) {
+  penalise(logits, vocab, ids, n, p);
+}
+__global__ __launch_bounds__(256) void repetition_penalty_list_kernel(float *__restrict__ logits, int vocab, const IdList list,
+                                                                      int n, double p) {
+  __shared__ int ids[kIdList];
+  if ((int)threadIdx.x < n) ids[threadIdx.x] = list.id[threadIdx.x];
+  __syncthreads();
+  penalise(logits, vocab, ids, n, p);
 }
 
 // ---- top-k ------------------------------------------------------------------
@@ -174,112 +198,179 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long v) {
   return v;
 }
 
-constexpr int kTopkChunk = 2048;  // logits per workgroup in the first pass; 8 keys per thread
+constexpr int kTopkChunk = 2048;   // logits per workgroup in the first pass; 8 keys per thread
+constexpr int kTopkThreads = 256;  // >= kMaxTopK
 
-// k rounds of "take the largest key and retire it" over keys held in registers.
-// n_mine keys per thread; writes the k winners (descending) to `dst`.
-template <int PER_THREAD>
-__device__ __forceinline__ void select_k(unsigned long long (&keys)[PER_THREAD], int k, unsigned long long *dst) {
-  __shared__ unsigned long long red[4];
-  for (int round = 0; round < k; ++round) {
-    unsigned long long best = 0ull;
-#pragma unroll
-    for (int u = 0; u < PER_THREAD; ++u) best = keys[u] > best ? keys[u] : best;
-    best = wave_max(best);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
-    __syncthreads();
-    unsigned long long w = red[0];
-#pragma unroll
-    for (int i = 1; i < 4; ++i) w = red[i] > w ? red[i] : w;
-    __syncthreads();
-    if (threadIdx.x == 0) dst[round] = w;
-    if (w == 0ull) {  // nothing left: the remaining rounds are empty too
-      for (int r = round + 1 + (int)threadIdx.x; r < k; r += 256) dst[r] = 0ull;
-      return;
-    }
-#pragma unroll
-    for (int u = 0; u < PER_THREAD; ++u)
-      if (keys[u] == w) keys[u] = 0ull;  // keys are unique (the index is part of them)
+struct TopkLds {
+  unsigned long long best[kTopkThreads];   // every thread's largest key
+  unsigned long long pool[kTopkChunk];     // keys at or above the threshold, in no order
+  unsigned long long win[kMaxTopK];        // the k largest, descending
+  unsigned long long threshold;
+  int pooled;
+};
+
+// The k-th largest of the threads' largest keys has at least k keys at or above it, and hardly more when the
+// large keys are spread over the threads.  (Keys are unique but for 0, so equal logits do not crowd the pool.)
+__device__ __forceinline__ void topk_threshold(TopkLds &s, unsigned long long mine, int k) {
+  s.best[threadIdx.x] = mine;
+  if (threadIdx.x == 0) s.threshold = 0ull, s.pooled = 0;
+  __syncthreads();
+  int above = 0;
+#pragma unroll 8
+  for (int j = 0; j < kTopkThreads; ++j) above += s.best[j] > mine;
+  if (above == k - 1) s.threshold = mine;  // (several threads only where mine is 0)
+  __syncthreads();
+}
+__device__ __forceinline__ void topk_pool(TopkLds &s, unsigned long long key) {
+  if (key != 0ull && key >= s.threshold) {
+    const int at = atomicAdd(&s.pooled, 1);
+    if (at < kTopkChunk) s.pool[at] = key;
   }
 }
+// win = the k largest of the pool in order (0 behind the last one)
+__device__ __forceinline__ void topk_rank(TopkLds &s, int k) {
+  __syncthreads();
+  const int n = s.pooled;
+  for (int i = threadIdx.x; i < n; i += kTopkThreads) {
+    const unsigned long long key = s.pool[i];
+    int above = 0;
+    for (int j = 0; j < n; ++j) above += s.pool[j] > key;
+    if (above < k) s.win[above] = key;
+  }
+  for (int r = n + (int)threadIdx.x; r < k; r += kTopkThreads) s.win[r] = 0ull;
+  __syncthreads();
+}
 
-__global__ __launch_bounds__(256) void topk_chunk_kernel(const float *__restrict__ logits, int vocab, int k,
-                                                         int finite_only, unsigned long long *__restrict__ cand) {
-  unsigned long long keys[8];
+// cand[r * chunks + c]: the r-th largest key of chunk c.  Rounds of "take the largest key" took 32 us for
+// k = 40 (two barriers a round); a threshold and ranks 7 us, whatever k is.
+__global__ __launch_bounds__(kTopkThreads) void topk_chunk_kernel(const float *__restrict__ logits, int vocab, int k,
+                                                                  int finite_only, unsigned long long *__restrict__ cand) {
+  __shared__ TopkLds s;
+  unsigned long long keys[8], mine = 0ull;
   const int base = blockIdx.x * kTopkChunk;
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
-    const int idx = base + u * 256 + threadIdx.x;
+    const int idx = base + u * kTopkThreads + threadIdx.x;
     keys[u] = idx < vocab ? make_key(logits[idx], idx, finite_only != 0) : 0ull;
+    mine = keys[u] > mine ? keys[u] : mine;
   }
-  select_k<8>(keys, k, cand + (long long)blockIdx.x * k);
-}
-
-// One workgroup merges the chunks' candidates (n_cand keys), 2048 at a time, keeping
-// the running top-k among them.
-__global__ __launch_bounds__(256) void topk_merge_kernel(const float *__restrict__ logits,
-                                                         unsigned long long *__restrict__ cand, int n_cand, int k,
-                                                         unsigned long long *__restrict__ winners,
-                                                         int *__restrict__ out_ids, float *__restrict__ out_vals,
-                                                         int *__restrict__ out_count, int fallback_id) {
-  // winners[0..k) holds the best so far; each pass selects among them and the next 2048 - 256 candidates
-  for (int r = threadIdx.x; r < k; r += 256) winners[r] = 0ull;
-  __syncthreads();
-  constexpr int kStep = 7 * 256;
-  for (int c0 = 0; c0 < n_cand || c0 == 0; c0 += kStep) {
-    unsigned long long keys[8];
-    keys[0] = (int)threadIdx.x < k ? winners[threadIdx.x] : 0ull;  // k <= 256
+  topk_threshold(s, mine, k);
 #pragma unroll
-    for (int u = 1; u < 8; ++u) {
-      const int i = c0 + (u - 1) * 256 + threadIdx.x;
-      keys[u] = i < n_cand ? cand[i] : 0ull;
-    }
-    __syncthreads();
-    select_k<8>(keys, k, winners);
-    __syncthreads();
-  }
-  int count = 0;
-  for (int r = threadIdx.x; r < k; r += 256) {
-    const unsigned long long key = winners[r];
-    if (key != 0ull) {
-      out_ids[r] = (int)(~(unsigned)(key & 0xffffffffu));
-      if (out_vals) out_vals[r] = key_value(key, logits);
-    } else {
-      out_ids[r] = fallback_id;
-      if (out_vals) out_vals[r] = 0.f;
-    }
-  }
-  if (threadIdx.x == 0 && out_count) {
-    while (count < k && winners[count] != 0ull) ++count;
-    *out_count = count;
-  }
+  for (int u = 0; u < 8; ++u) topk_pool(s, keys[u]);
+  topk_rank(s, k);
+  if ((int)threadIdx.x < k) cand[(long long)threadIdx.x * gridDim.x + blockIdx.x] = s.win[threadIdx.x];
 }
 
-// Sampler#sample after its top-k selection (text/sampler.cr:118-150): the temperature softmax over
-// the survivors and the inverse-CDF pick for the uniform draw r, one lane, in the reference's order
-// and number types (fp64 throughout).  ids / vals: the selection, descending; *count entries.
-__global__ void sample_pick_kernel(const int *__restrict__ ids, const float *__restrict__ vals,
-                                   const int *__restrict__ count, double temperature, double r, int *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const int n = *count;
+// One workgroup merges the chunks' candidates: their first ones come first, so the largest keys are spread over
+// the threads.  With `pick`, the rest of Sampler#sample follows (text/sampler.cr:118-150): the temperature softmax
+// over the survivors and the inverse-CDF pick for the uniform draw r, in fp64, its sums in the reference's order.
+__global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const float *__restrict__ logits,
+                                                                  const unsigned long long *__restrict__ cand, int n_cand, int k,
+                                                                  int *__restrict__ out_ids, float *__restrict__ out_vals,
+                                                                  int *__restrict__ out_count, int fallback_id,
+                                                                  int *__restrict__ pick, double temperature, double r) {
+  __shared__ TopkLds s;
+  __shared__ double weight[kMaxTopK];
+  unsigned long long mine = 0ull;
+  for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) mine = cand[i] > mine ? cand[i] : mine;
+  topk_threshold(s, mine, k);
+  for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) topk_pool(s, cand[i]);
+  __syncthreads();
+  if (s.pooled > kTopkChunk) {  // too many for the pool: the threshold is raised to the k-th largest key, a bit at a time
+    unsigned long long low = 0ull;
+    for (int bit = 63; bit >= 0; --bit) {
+      const unsigned long long tried = low | (1ull << bit);
+      __syncthreads();
+      if (threadIdx.x == 0) s.pooled = 0;
+      __syncthreads();
+      int here = 0;
+      for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) here += cand[i] >= tried;
+      atomicAdd(&s.pooled, here);
+      __syncthreads();
+      if (s.pooled >= k) low = tried;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) s.threshold = low, s.pooled = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) topk_pool(s, cand[i]);
+  }
+  topk_rank(s, k);
+  const int n = s.pooled < k ? s.pooled : k, t = threadIdx.x;
+  const unsigned long long key = t < k ? s.win[t] : 0ull;
+  const float v = key ? key_value(key, logits) : 0.f;
+  if (t < k) {
+    if (out_ids) out_ids[t] = key ? (int)(~(unsigned)(key & 0xffffffffu)) : fallback_id;
+    if (out_vals) out_vals[t] = v;
+  }
+  if (t == 0 && out_count) *out_count = n;
+  if (!pick) return;
+  // descending order: element 0 is the maximum
+  if (t < n) weight[t] = exp((double)v / temperature - (double)key_value(s.win[0], logits) / temperature);
+  __syncthreads();
+  if (t != 0) return;
   if (n <= 0) {  // all-NaN row: nothing to sample (sampler.cr:121)
-    *out = 0;
+    *pick = 0;
     return;
   }
-  const double max_val = (double)vals[0] / temperature;  // descending order: element 0 is the maximum
   double sum = 0.0;
-  for (int i = 0; i < n; ++i) sum += exp((double)vals[i] / temperature - max_val);
+  for (int i = 0; i < n; ++i) sum += weight[i];
   const double inv_sum = 1.0 / sum;
   double cumulative = 0.0;
-  int best = ids[n - 1];
+  int best = n - 1;
   for (int i = 0; i < n; ++i) {
-    cumulative += exp((double)vals[i] / temperature - max_val) * inv_sum;
+    cumulative += weight[i] * inv_sum;
     if (r <= cumulative) {
-      best = ids[i];
+      best = i;
       break;
     }
   }
-  *out = best;
+  *pick = (int)(~(unsigned)(s.win[best] & 0xffffffffu));
+}
+
+// Sampler.greedy and the next step's embedding lookup in one launch of one workgroup: *id = the largest finite
+// logit's place (0: none), out = its row of the table.  cand null: the logits themselves are read here, 128 KB of
+// them (vocabulary of 32000) in about 2 us; from 65536 on the chunks' largest keys are (n of them).
+__global__ __launch_bounds__(1024) void greedy_embed_kernel(const float *__restrict__ logits, int vocab,
+                                                            const unsigned long long *__restrict__ cand, int n,
+                                                            int *__restrict__ id, const float *__restrict__ table,
+                                                            float *__restrict__ out, int d_model, float scale,
+                                                            const float *__restrict__ position) {
+  __shared__ unsigned long long red[16];
+  unsigned long long best = 0ull;
+  if (cand) {
+    for (int i = threadIdx.x; i < n; i += 1024) best = cand[i] > best ? cand[i] : best;
+  } else {
+    const int whole = vocab & ~3;
+    for (int i0 = 0; i0 < whole; i0 += 8 * 4096) {
+      f32x4 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i = i0 + u * 4096 + 4 * (int)threadIdx.x;
+        v[u] = i < whole ? *(const f32x4 *)(logits + i) : f32x4{NAN, NAN, NAN, NAN};
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const unsigned long long key = make_key(v[u][c], i0 + u * 4096 + 4 * (int)threadIdx.x + c, true);
+          best = key > best ? key : best;
+        }
+    }
+    if (whole + (int)threadIdx.x < vocab) {
+      const unsigned long long key = make_key(logits[whole + threadIdx.x], whole + threadIdx.x, true);
+      best = key > best ? key : best;
+    }
+  }
+  best = wave_max(best);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
+  __syncthreads();
+  best = red[0];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) best = red[i] > best ? red[i] : best;
+  const int token = best ? (int)(~(unsigned)(best & 0xffffffffu)) : 0;
+  if (threadIdx.x == 0) *id = token;
+  const float *src = table + (long long)token * d_model;
+  for (int j = threadIdx.x; j < d_model; j += 1024) out[j] = position ? src[j] * scale + position[j] : src[j] * scale;
 }
 
 // RoPE.apply (rope.cr:7-33): one lane per (row, pair).  Everything in fp64 as the reference has
@@ -398,6 +489,14 @@ hipError_t launch_embed(const float *table, const int *tokens, float *out, int n
   return hipGetLastError();
 }
 
+hipError_t launch_embed_list(const float *table, const IdList &tokens, float *out, int n_tokens, int d_model,
+                             hipStream_t stream, float scale, const float *positions) {
+  if (n_tokens < 1 || n_tokens > kIdList || d_model < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(embed_list_kernel, dim3((unsigned)n_tokens), dim3(256), 0, stream, table, tokens, out, d_model, scale,
+                     positions);
+  return hipGetLastError();
+}
+
 hipError_t launch_add_bias_row(float *logits, const float *bias, int n, hipStream_t stream) {
   if (n < 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(add_bias_row_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, logits, bias, n);
@@ -407,7 +506,16 @@ hipError_t launch_add_bias_row(float *logits, const float *bias, int n, hipStrea
 hipError_t launch_repetition_penalty(float *logits, int vocab, const int *ids, int n, double penalty,
                                      hipStream_t stream) {
   if (n < 1) return hipSuccess;
-  hipLaunchKernelGGL(repetition_penalty_kernel, dim3(1), dim3(64), 0, stream, logits, vocab, ids, n, penalty);
+  hipLaunchKernelGGL(repetition_penalty_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, logits, vocab, ids, n,
+                     penalty);
+  return hipGetLastError();
+}
+
+hipError_t launch_repetition_penalty_list(float *logits, int vocab, const IdList &ids, int n, double penalty,
+                                          hipStream_t stream) {
+  if (n < 1) return hipSuccess;
+  if (n > kIdList) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(repetition_penalty_list_kernel, dim3(1), dim3(256), 0, stream, logits, vocab, ids, n, penalty);
   return hipGetLastError();
 }
 
@@ -422,30 +530,38 @@ hipError_t launch_rope_apply(const float *x, float *out, int seq_len, int head_d
   return hipGetLastError();
 }
 
-hipError_t launch_sample_pick(const int *ids, const float *vals, const int *count, double temperature, double r,
-                              int *out, hipStream_t stream) {
-  if (!ids || !vals || !count || !out || !(temperature > 0.0)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(sample_pick_kernel, dim3(1), dim3(64), 0, stream, ids, vals, count, temperature, r, out);
-  return hipGetLastError();
-}
-
 size_t topk_scratch_bytes(int vocab, int k) {
-  const size_t chunks = (size_t)(vocab + kTopkChunk - 1) / kTopkChunk;
-  return (chunks * k + k) * sizeof(unsigned long long);
+  return (size_t)((vocab + kTopkChunk - 1) / kTopkChunk) * k * sizeof(unsigned long long);
 }
 
 hipError_t launch_topk(const float *logits, int vocab, int k, bool finite_only, void *scratch, int *out_ids,
-                       float *out_vals, int *out_count, hipStream_t stream, int fallback_id) {
-  if (vocab < 1 || k < 1 || k > kMaxTopK || !scratch) return hipErrorInvalidValue;
+                       float *out_vals, int *out_count, hipStream_t stream, int fallback_id, int *pick, double temperature,
+                       double r) {
+  if (vocab < 1 || k < 1 || k > kMaxTopK || !scratch || (pick && !(temperature > 0.0))) return hipErrorInvalidValue;
   const int chunks = (vocab + kTopkChunk - 1) / kTopkChunk;
   unsigned long long *cand = (unsigned long long *)scratch;
-  unsigned long long *winners = cand + (size_t)chunks * k;
-  hipLaunchKernelGGL(topk_chunk_kernel, dim3((unsigned)chunks), dim3(256), 0, stream, logits, vocab, k,
+  hipLaunchKernelGGL(topk_chunk_kernel, dim3((unsigned)chunks), dim3(kTopkThreads), 0, stream, logits, vocab, k,
                      finite_only ? 1 : 0, cand);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(topk_merge_kernel, dim3(1), dim3(256), 0, stream, logits, cand, chunks * k, k, winners, out_ids,
-                     out_vals, out_count, fallback_id);
+  hipLaunchKernelGGL(topk_merge_kernel, dim3(1), dim3(kTopkThreads), 0, stream, logits, cand, chunks * k, k, out_ids, out_vals,
+                     out_count, fallback_id, pick, temperature, r);
+  return hipGetLastError();
+}
+
+hipError_t launch_greedy_embed(const float *logits, int vocab, void *scratch, int *id, const float *table, float *out, int d_model,
+                               float scale, const float *position, hipStream_t stream) {
+  if (!logits || vocab < 1 || !scratch || !id || !table || !out || d_model < 1) return hipErrorInvalidValue;
+  unsigned long long *cand = nullptr;
+  int chunks = 0;
+  if (vocab > 65536) {
+    chunks = (vocab + kTopkChunk - 1) / kTopkChunk;
+    cand = (unsigned long long *)scratch;
+    hipLaunchKernelGGL(topk_chunk_kernel, dim3((unsigned)chunks), dim3(kTopkThreads), 0, stream, logits, vocab, 1, 1, cand);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(greedy_embed_kernel, dim3(1), dim3(1024), 0, stream, logits, vocab, (const unsigned long long *)cand, chunks, id,
+                     table, out, d_model, scale, position);
   return hipGetLastError();
 }
 

@@ -26,6 +26,13 @@ hipError_t launch_swiglu_act(const float *gate_up, float *hidden, int rows, int 
 // out[t, :] = table[tokens[t], :] * scale (+ positions[t, :]);  the caller has checked 0 <= tokens[t] < vocab
 hipError_t launch_embed(const float *table, const int *tokens, float *out, int n_tokens, int d_model,
                         hipStream_t stream, float scale = 1.f, const float *positions = nullptr);
+// The same for up to kIdList ids on the host: they travel in the kernel's arguments.
+constexpr int kIdList = 256;
+struct IdList {
+  int id[kIdList];
+};
+hipError_t launch_embed_list(const float *table, const IdList &tokens, float *out, int n_tokens, int d_model,
+                             hipStream_t stream, float scale = 1.f, const float *positions = nullptr);
 // out[i, :] = x[rows[i], :], n rows of `cols` floats
 hipError_t launch_gather_rows(const float *x, const int *rows, float *out, int n, int cols, hipStream_t stream);
 // logits[j] += bias[j]
@@ -33,6 +40,8 @@ hipError_t launch_add_bias_row(float *logits, const float *bias, int n, hipStrea
 // Sampler#apply_repetition_penalty! : ids in order, duplicates penalised once per occurrence
 hipError_t launch_repetition_penalty(float *logits, int vocab, const int *ids, int n, double penalty,
                                      hipStream_t stream);
+hipError_t launch_repetition_penalty_list(float *logits, int vocab, const IdList &ids, int n, double penalty,
+                                          hipStream_t stream);
 
 // RoPE.apply (rope.cr:7-33) on [seq_len, head_dim] rows: half-split rotation by
 // (row + start_pos) * theta^(-2i/head_dim), frequency, angle, cosine, sine and the products in
@@ -44,17 +53,17 @@ hipError_t launch_rope_apply(const float *x, float *out, int seq_len, int head_d
 // selected (Sampler#sample's selection); with finite_only also +-inf are skipped
 // (Sampler.greedy).  scratch: topk_scratch_bytes(vocab, k) bytes.  out_ids /
 // out_vals: k entries; *out_count = entries found (< k when the row has fewer
-// eligible values); the unused ids are set to fallback_id.  out_vals and out_count
-// may be null.
+// eligible values); the unused ids are set to fallback_id.  out_ids, out_vals and out_count may be null.
+// pick (nullable; may be pinned host memory): the rest of Sampler#sample (text/sampler.cr:118-150), the softmax of
+// the values / temperature over the survivors and the choice for the uniform draw r in [0, 1) (0: nothing eligible).
 constexpr int kMaxTopK = 256;
 size_t topk_scratch_bytes(int vocab, int k);
 hipError_t launch_topk(const float *logits, int vocab, int k, bool finite_only, void *scratch, int *out_ids,
-                       float *out_vals, int *out_count, hipStream_t stream, int fallback_id = -1);
-
-// The rest of Sampler#sample (text/sampler.cr:118-150) on a selection launch_topk made: softmax of
-// vals / temperature over the *count survivors and the pick for the uniform draw r in [0, 1);
-// *out = the chosen id (0 when nothing was eligible).
-hipError_t launch_sample_pick(const int *ids, const float *vals, const int *count, double temperature, double r,
-                              int *out, hipStream_t stream);
+                       float *out_vals, int *out_count, hipStream_t stream, int fallback_id = -1, int *pick = nullptr,
+                       double temperature = 1.0, double r = 0.0);
+// *id = Sampler.greedy of the logits (0 when none is finite) and out = row *id of table * scale (+ position);
+// scratch: topk_scratch_bytes(vocab, 1) bytes.
+hipError_t launch_greedy_embed(const float *logits, int vocab, void *scratch, int *id, const float *table, float *out, int d_model,
+                               float scale, const float *position, hipStream_t stream);
 
 }  // namespace shainet

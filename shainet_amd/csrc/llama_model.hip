@@ -96,6 +96,7 @@ struct shainet_llama_model {
   size_t topk_scratch_cap = 0;
   int *d_ids = nullptr;    // kMaxTopK ids, then the count
   float *d_vals = nullptr;
+  int *h_pick = nullptr;   // pinned host word the sampled id is written to
   int *d_gen = nullptr;    // generated ids of one chunk of shainet_llama_model_generate_greedy
   ModelStep step;
 };
@@ -193,7 +194,7 @@ int run_topk(shainet_llama_model *m, int k, bool finite_only, int *ids, float *v
     m->topk_scratch_cap = need;
   }
   if (!m->d_ids) {
-    if (hipMalloc((void **)&m->d_ids, (kMaxTopK + 2) * sizeof(int)) != hipSuccess ||
+    if (hipMalloc((void **)&m->d_ids, (kMaxTopK + 1) * sizeof(int)) != hipSuccess ||
         hipMalloc((void **)&m->d_vals, kMaxTopK * sizeof(float)) != hipSuccess)
       return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   }
@@ -262,12 +263,16 @@ void plan_model_step(shainet_llama_model *m) {
   st.plan = p;
 }
 
+bool takes_one_launch_step(shainet_llama_model *m) {
+  if (!m->step.planned) plan_model_step(m);
+  return m->step.plan.ok;
+}
+
 // One new token through all blocks in one launch; m->act[0] receives the last block's output row.
 // Returns -1 when this step has to take the launch-per-product path instead.
 int run_step(shainet_llama_model *m, const int *d_token) {
   ModelStep &st = m->step;
-  if (!st.planned) plan_model_step(m);
-  if (!st.plan.ok) return -1;
+  if (!takes_one_launch_step(m)) return -1;
   const size_t n_layers = m->blocks.size();
   std::vector<StepLayer> now(n_layers);
   int pos = -1, rc;
@@ -340,18 +345,25 @@ int head_rows(shainet_llama_model *m, const float *x, int n, float *logits) {
   return SHAINET_HIP_OK;
 }
 
+int check_positions(const shainet_llama_model *m, int start, int T) {
+  if (!m->positions || (long long)start + T <= m->max_positions) return SHAINET_HIP_OK;
+  return fail(SHAINET_HIP_ERR_CAPACITY, std::to_string(start) + " + " + std::to_string(T) + " positions: this model has " +
+                                            std::to_string(m->max_positions));
+}
+
 // Network#run on token ids that already sit in device memory; asynchronous.  no_cache: every block's
 // LlamaBlock#forward instead of forward_cached (network_run.cr:199-204 with use_kv_cache off): the
 // rows attend among themselves from position 0 and the caches stay as they are.
 // last_block (nullable): receives the last block's output, all T rows, as long as the next run lasts.
+// list (nullable): the ids on the host, in place of d_tokens; embedded: act[0] holds the ids' embedding rows already.
 int run_device_tokens(shainet_llama_model *m, const int *d_tokens, int T, bool no_cache = false,
-                      const float **last_block = nullptr) {
+                      const float **last_block = nullptr, const IdList *list = nullptr, bool embedded = false) {
   const int d = m->d_model;
   if (!m->act[0].reserve((size_t)T * d) || !m->act[1].reserve((size_t)T * d) || !m->logits.reserve((size_t)m->vocab))
     return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   m->have_logits = false;
   int cur = 0, rc = -1;
-  if (T == 1 && !no_cache) {
+  if (T == 1 && !no_cache && !embedded) {
     rc = run_step(m, d_tokens);
     if (rc > 0) return rc;
     if (rc < 0 && m->step.mode == SHAINET_HIP_DECODE_PERSISTENT)
@@ -359,11 +371,11 @@ int run_device_tokens(shainet_llama_model *m, const int *d_tokens, int T, bool n
   }
   if (rc < 0) {
     const int start = no_cache ? 0 : shainet_llama_model_cache_len(m);
-    if (m->positions && (long long)start + T > m->max_positions)
-      return fail(SHAINET_HIP_ERR_CAPACITY, std::to_string(start) + " + " + std::to_string(T) + " positions: this model has " +
-                                                std::to_string(m->max_positions));
-    hipError_t e = launch_embed(m->embedding, d_tokens, m->act[0].p, T, d, m->stream, m->embedding_scale,
-                                m->positions ? m->positions + (size_t)start * d : nullptr);
+    if ((rc = check_positions(m, start, T))) return rc;
+    const float *positions = m->positions ? m->positions + (size_t)start * d : nullptr;
+    const hipError_t e = embedded ? hipSuccess
+                         : list   ? launch_embed_list(m->embedding, *list, m->act[0].p, T, d, m->stream, m->embedding_scale, positions)
+                                  : launch_embed(m->embedding, d_tokens, m->act[0].p, T, d, m->stream, m->embedding_scale, positions);
     if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("embedding launch: ") + hipGetErrorString(e));
     BlockCarry carry;
     for (shainet_llama_block *b : m->blocks) {
@@ -435,6 +447,7 @@ int shainet_llama_model_destroy(shainet_llama_model *m) {
   if (m->d_tokens) (void)hipFree(m->d_tokens);
   if (m->d_ids) (void)hipFree(m->d_ids);
   if (m->d_gen) (void)hipFree(m->d_gen);
+  if (m->h_pick) (void)hipHostFree(m->h_pick);
   if (m->topk_scratch) (void)hipFree(m->topk_scratch);
   m->proj.release();
   m->step.release();
@@ -521,9 +534,15 @@ static int run_host_tokens(shainet_llama_model *m, const int *tokens, int n_toke
     if (tokens[i] < 0 || tokens[i] >= m->vocab) return fail(SHAINET_HIP_ERR_ARGUMENT, "token id outside the vocabulary");
   if (!m->stream && hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess)
     return fail(SHAINET_HIP_ERR_RUNTIME, "hipStreamCreate failed");
+  m->have_logits = false;
+  // a few ids travel in the embedding launch itself (the one-launch step reads its id from memory)
+  if (n_tokens <= kIdList && !(n_tokens == 1 && !no_cache && takes_one_launch_step(m))) {
+    IdList list;
+    memcpy(list.id, tokens, (size_t)n_tokens * sizeof(int));
+    return run_device_tokens(m, nullptr, n_tokens, no_cache, last_block, &list);
+  }
   int rc = reserve_ints(&m->d_tokens, &m->d_tokens_cap, (size_t)n_tokens);
   if (rc) return rc;
-  m->have_logits = false;
   // pageable source: the copy has left the host buffer when the call returns
   if (hipMemcpyAsync(m->d_tokens, tokens, (size_t)n_tokens * sizeof(int), hipMemcpyHostToDevice, m->stream) !=
       hipSuccess)
@@ -595,11 +614,21 @@ int shainet_llama_model_generate_greedy(shainet_llama_model *m, int max_tokens, 
         if (int rc = shainet_llama_block_save_state(b)) return rc;
     }
     for (int i = 0; i < steps; ++i) {
-      // best_id = Sampler.greedy(logits) into d_gen[i]; then net.run([best_id]) reading it from there
-      hipError_t e = launch_topk(m->logits.p, m->vocab, 1, true, m->topk_scratch, m->d_gen + i, nullptr, nullptr,
-                                 m->stream, 0);
+      // best_id = Sampler.greedy(logits) into d_gen[i]; then net.run([best_id]), whose embedding row the same launch
+      // looks up (the one-launch step reads the id itself)
+      const bool embedded = !takes_one_launch_step(m);
+      hipError_t e;
+      if (embedded) {
+        const int start = shainet_llama_model_cache_len(m);
+        if (int rc = check_positions(m, start, 1)) return rc;
+        if (!m->act[0].reserve((size_t)m->d_model)) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
+        e = launch_greedy_embed(m->logits.p, m->vocab, m->topk_scratch, m->d_gen + i, m->embedding, m->act[0].p, m->d_model,
+                                m->embedding_scale, m->positions ? m->positions + (size_t)start * m->d_model : nullptr, m->stream);
+      } else {
+        e = launch_topk(m->logits.p, m->vocab, 1, true, m->topk_scratch, m->d_gen + i, nullptr, nullptr, m->stream, 0);
+      }
       if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("argmax launch: ") + hipGetErrorString(e));
-      int rc = run_device_tokens(m, m->d_gen + i, 1);
+      int rc = run_device_tokens(m, m->d_gen + i, 1, false, nullptr, nullptr, embedded);
       if (rc) return rc;
     }
     if (hipMemcpyAsync(host_ids, m->d_gen, steps * sizeof(int), hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
@@ -676,6 +705,13 @@ int shainet_llama_model_repetition_penalty(shainet_llama_model *m, const int *re
   if (!m || (n > 0 && !recent_ids)) return fail(SHAINET_HIP_ERR_ARGUMENT, "null argument");
   if (!m->have_logits) return fail(SHAINET_HIP_ERR_ARGUMENT, "no logits: call shainet_llama_model_run first");
   if (penalty == 1.0 || n < 1) return SHAINET_HIP_OK;  // sampler.cr:64
+  if (n <= kIdList) {
+    IdList list;
+    memcpy(list.id, recent_ids, (size_t)n * sizeof(int));
+    const hipError_t e = launch_repetition_penalty_list(m->logits.p, m->vocab, list, n, penalty, m->stream);
+    if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("penalty launch: ") + hipGetErrorString(e));
+    return SHAINET_HIP_OK;
+  }
   int rc = reserve_ints(&m->d_tokens, &m->d_tokens_cap, (size_t)n);
   if (rc) return rc;
   if (hipMemcpyAsync(m->d_tokens, recent_ids, (size_t)n * sizeof(int), hipMemcpyHostToDevice, m->stream) != hipSuccess)
@@ -703,22 +739,18 @@ int shainet_llama_model_sample(shainet_llama_model *m, int k, double temperature
     if (hipMalloc(&m->topk_scratch, need) != hipSuccess) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     m->topk_scratch_cap = need;
   }
-  if (!m->d_ids) {
-    if (hipMalloc((void **)&m->d_ids, (kMaxTopK + 2) * sizeof(int)) != hipSuccess ||
-        hipMalloc((void **)&m->d_vals, kMaxTopK * sizeof(float)) != hipSuccess)
-      return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-  }
+  if (!m->h_pick && hipHostMalloc((void **)&m->h_pick, sizeof(int), hipHostMallocDefault) != hipSuccess)
+    return fail(SHAINET_HIP_ERR_ALLOC, "hipHostMalloc failed");
   // dividing by a positive temperature keeps the order of the logits: the selection over v / t
   // (sampler.cr:100-115) is the selection over v
-  hipError_t e = launch_topk(m->logits.p, m->vocab, k, false, m->topk_scratch, m->d_ids, m->d_vals,
-                             m->d_ids + kMaxTopK, m->stream);
-  if (e == hipSuccess)
-    e = launch_sample_pick(m->d_ids, m->d_vals, m->d_ids + kMaxTopK, temperature, r, m->d_ids + kMaxTopK + 1, m->stream);
+  const hipError_t e = launch_topk(m->logits.p, m->vocab, k, false, m->topk_scratch, nullptr, nullptr, nullptr, m->stream, -1, m->h_pick,
+                                   temperature, r);
   if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("sample launch: ") + hipGetErrorString(e));
-  if (hipMemcpyAsync(token, m->d_ids + kMaxTopK + 1, sizeof(int), hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
-      hipStreamSynchronize(m->stream) != hipSuccess)
-    return fail(SHAINET_HIP_ERR_RUNTIME, "copying the sampled id back failed");
-  return check_error_word(m->error);
+  if (hipStreamSynchronize(m->stream) != hipSuccess)
+    return fail(SHAINET_HIP_ERR_RUNTIME, "waiting for the sampled id failed");
+  if (int rc = check_error_word(m->error)) return rc;
+  *token = *(volatile int *)m->h_pick;
+  return SHAINET_HIP_OK;
 }
 
 int shainet_llama_model_write_logits(shainet_llama_model *m, const float *logits) {

@@ -796,3 +796,58 @@ def test_matmul_split_tiles_keep_what_is_not_finite(hip, T):
     fine = got.isfinite()
     assert bool(((got.double() - want).abs()[fine] <= 1e-4 * (1 + want.abs()[fine])).all())
     assert got[10, 0].item() == np.float32(3.4e38) * np.float32(0.5)
+
+
+@pytest.mark.parametrize("vocab", [31, 2049, 131072])
+def test_device_topk_of_crowded_and_tied_rows(hip, vocab):
+    """Rows that a threshold over the threads' largest values does not thin out: all equal, a few allowed among masked
+    ones, everything large in one chunk, the k-th value tied, fewer than k eligible; selections are exact."""
+    m = hip.LlamaModel(vocab, 8, 1, 1, 8)
+    r = np.random.default_rng(vocab)
+    base = r.standard_normal(vocab).astype(np.float32)
+    masked = np.full(vocab, np.finfo(np.float32).min, np.float32)
+    masked[r.integers(0, vocab, 10)] = 1.5
+    one_chunk = base.copy()
+    one_chunk[:min(vocab, 2048)] += 100
+    stairs = np.floor(base * 2).astype(np.float32)
+    few = np.full(vocab, NAN, np.float32)
+    few[r.integers(0, vocab, 7)] = -INF
+    for name, row in (("equal", np.zeros(vocab, np.float32)), ("masked", masked), ("one chunk", one_chunk),
+                      ("rising", np.sort(base)), ("falling", -np.sort(base)), ("stairs", stairs), ("few", few)):
+        m.set_logits(row)
+        for k in (1, 40, 255, 256):
+            ids, vals = hip.Sampler(top_k=k).top_candidates(m)
+            want_ids, want_vals = orc.topk(row, k, 1.0)
+            np.testing.assert_array_equal(ids, want_ids, f"{name} k={k}")
+            np.testing.assert_array_equal(vals.astype(np.float64), want_vals, f"{name} k={k}")
+        assert hip.Sampler.greedy(m) == orc.greedy(row), name
+    ids = list(r.integers(0, vocab, 300)) + [3, 3, 3, -1, vocab]  # more ids than fit a launch's arguments
+    for part in (ids, ids[-200:]):
+        m.set_logits(base)
+        hip.Sampler(repetition_penalty=1.3).apply_repetition_penalty(m, part)
+        np.testing.assert_array_equal(m.logits(), orc.repetition_penalty(base.copy(), part, 1.3))
+    m.close()
+
+
+@pytest.mark.parametrize("vocab", [30, 4097, 70001])
+def test_generate_greedy_equals_steps(hip, vocab):
+    # the argmax that looks up the next row: one launch (below 65536 logits) or two, whole and ragged vocabularies
+    r = np.random.default_rng(vocab)
+    m = hip.LlamaModel(vocab, 64, 2, 2, 96, num_kv_heads=1)
+    m.set_embedding(r.standard_normal((vocab, 64)).astype(np.float32))
+    m.set_lm_head(r.standard_normal((64, vocab)).astype(np.float32))
+    for b in m.blocks:
+        b.set_weights(*[(0.1 * r.standard_normal(s)).astype(np.float32) for s in ((64, 64), (64, 32), (64, 32), (64, 64))])
+        b.set_ffn(*[(0.1 * r.standard_normal(s)).astype(np.float32) for s in ((64, 96), (64, 96), (96, 64))])
+    prompt = [int(t) for t in r.integers(0, vocab, 5)]
+    m.run(prompt, want_logits=False)
+    got = m.generate_greedy(20)
+    row = m.logits()
+    m.clear_cache()
+    want, last = [], m.run(prompt)
+    for _ in range(20):
+        want.append(orc.greedy(last))
+        last = m.run(want[-1:])
+    assert got == want
+    np.testing.assert_array_equal(row, last)
+    m.close()
