@@ -195,13 +195,8 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       stage[w_unit + S::kPartW] = m;
       stage[w_unit + 2 * S::kPartW] = l;
       if (NX == 1) {
-        unsigned a[2], b[2], c[2];
-        split_pair(rx[0].x, rx[0].y, a[0], b[0], c[0]);
-        split_pair(rx[0].z, rx[0].w, a[1], b[1], c[1]);
         u32x2 *half = (u32x2 *)(stage + x_unit) + ((xk >> 2) & 1);
-        half[0] = u32x2{a[0], a[1]};
-        half[2 * S::kPartX] = u32x2{b[0], b[1]};
-        half[4 * S::kPartX] = u32x2{c[0], c[1]};
+        split_quad(rx[0], half[0], half[2 * S::kPartX], half[4 * S::kPartX]);
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -246,13 +241,12 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       park_tiles(rx, rw, lds[(kt & 1) ^ 1]);
       load_tiles(rx, rw);
       // smallest products first; the blocks take turns, no MFMA waits for the one before it
-      constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
       for (int p = 0; p < 6; ++p)
 #pragma unroll
         for (int a = 0; a < MB; ++a)
 #pragma unroll
-          for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[pa[p]][a], bf[pb[p]][b], acc[a][b]);
+          for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p]][b], acc[a][b]);
       __syncthreads();
     };
     for (int kt = 0; kt < nk; kt += 2) {

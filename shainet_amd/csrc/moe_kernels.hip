@@ -1,5 +1,6 @@
 // A mixture of experts on gfx950 (moe_kernels.hpp says what is computed), fp32.
 #include "moe_kernels.hpp"
+#include "split_mfma.hpp"
 
 #include <math.h>
 #include <stdint.h>
@@ -8,11 +9,6 @@
 namespace shainet {
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-#define ORDER_LDS_AND_MFMA() __builtin_amdgcn_sched_barrier(0x7)
 
 __device__ __forceinline__ float swiglu1(float g, float u) { return g / (1.f + expf(-g)) * u; }
 __device__ __forceinline__ float wave_sum(float v) {
@@ -421,11 +417,13 @@ __global__ __launch_bounds__(256) void moe_scatter_kernel(int n, int top, int ex
 }
 
 // Rows of x (gathered, or as they lie) times the matrices of their groups, [N, K] (SWIGLU: [2N, K], gate
-// rows and up rows): the layout of a product whose operands both run along K.  A workgroup of four
-// wavefronts takes TM rows and TN matrix rows; both tiles go global memory -> registers -> LDS, two stages,
-// row stride 36 floats, and are read 16 bytes at a time down a column of rows.  v_mfma_f32_32x32x2: MFMA i of
-// a k step of 8 takes k = 8 s + 4 half + i on both sides.  With SWIGLU even blocks of 32 matrix rows are gates and
-// the odd ones behind them their partners, so that a lane holds both halves of its outputs.
+// rows and up rows): a product whose operands both run along K, on the bf16 matrix cores with every operand as
+// the exact sum of three bf16 numbers (split_mfma.hpp).  A workgroup of four wavefronts, two by two, takes 64 MB
+// rows and 128 matrix rows, a wavefront MB x 2 blocks of 32 x 32.  Per step of 16 along K both tiles go
+// global memory -> registers (two steps ahead) -> split -> LDS (two stages), where 16-byte units [part][octet of
+// k][row] are the fragments of an MFMA.  With SWIGLU a wavefront's first block of matrix rows is gates and the second
+// their partners, so that a lane holds both halves of its outputs.
+// 777 tokens, 145 rows an expert, 1024 -> 512: 155 -> 44 us against the fp32 instruction in tiles as large.
 struct GroupedArgs {
   const float *x;
   const int *gather;       // row r of the product is row gather[r] of x; null: row r
@@ -434,12 +432,12 @@ struct GroupedArgs {
   float *y;                // [rows, N]
   int rows, groups, K, N;
 };
-template <int TM, bool SWIGLU, bool VEC>
+template <int MB, bool SWIGLU, bool VEC>
 __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g) {
-  constexpr int TK = 32, AS = TK + 4, RW = TM / 32, CW = 4 / RW, NB = TM == 128 ? 4 : 2, TN = 32 * NB * CW;
-  constexpr int NA = TM / 32, NW = TN / 32;  // 16-byte pieces per thread and stage
-  extern __shared__ __attribute__((aligned(16))) float smem[];
-  float *As = smem, *Bs = smem + 2 * TM * AS;
+  constexpr int TK = 16, TM = 64 * MB, TN = 128;
+  constexpr int NA = TM / 64, NW = TN / 64;  // 16-byte pieces per thread and step
+  constexpr int kOctX = TM + 4, kOctW = TN + 4, kPartX = 2 * kOctX, kPartW = 2 * kOctW;  // units of 16 bytes
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2][3 * (kPartX + kPartW)];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int grp = 0, tm = blockIdx.x, r0 = 0, r1 = g.rows;
   if (g.tile_off) {
@@ -455,20 +453,22 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
   if (m0 >= r1) return;
   const int K = g.K, N = g.N, o0 = blockIdx.y * (SWIGLU ? TN / 2 : TN);
   const float *w = g.w + (long long)grp * (SWIGLU ? 2 : 1) * N * K;
+  // the matrix row behind row i of the tile
+  auto matrix_row = [&](int i) {
+    return SWIGLU ? (i >> 5 & 1) * N + min(o0 + (i >> 6) * 32 + (i & 31), N - 1) : min(o0 + i, N - 1);
+  };
 
-  const int srow = threadIdx.x >> 3, k4 = 4 * (threadIdx.x & 7);
+  // piece u of a thread: quarter tid % 4 of tile row tid / 4 + 64 u
+  const int srow = threadIdx.x >> 2, k4 = 4 * (threadIdx.x & 3);
   const float *ap[NA], *bp[NW];
 #pragma unroll
   for (int u = 0; u < NA; ++u) {
-    const int r = min(m0 + srow + 32 * u, r1 - 1);
+    const int r = min(m0 + srow + 64 * u, r1 - 1);
     ap[u] = g.x + (long long)(g.gather ? g.gather[r] : r) * K;
   }
 #pragma unroll
-  for (int u = 0; u < NW; ++u) {  // u is the block of 32 matrix rows
-    const int r = SWIGLU ? (u & 1) * N + min(o0 + (u >> 1) * 32 + srow, N - 1) : min(o0 + 32 * u + srow, N - 1);
-    bp[u] = w + (long long)r * K;
-  }
-  f32x4 sa[NA], sb[NW];
+  for (int u = 0; u < NW; ++u) bp[u] = w + (long long)matrix_row(srow + 64 * u) * K;
+  f32x4 sa[2][NA], sb[2][NW];
   auto piece = [&](const float *p, int k) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if constexpr (VEC) {
@@ -481,79 +481,108 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
     }
     return v;
   };
-  auto load = [&](int k0) {
+  auto load = [&](int set, int k0) {  // (steps behind the last one are zeros, which nobody reads)
 #pragma unroll
-    for (int u = 0; u < NA; ++u) sa[u] = piece(ap[u], k0 + k4);
+    for (int u = 0; u < NA; ++u)
+      sa[set][u] = piece(ap[u], k0 + k4);
 #pragma unroll
-    for (int u = 0; u < NW; ++u) sb[u] = piece(bp[u], k0 + k4);
+    for (int u = 0; u < NW; ++u) sb[set][u] = piece(bp[u], k0 + k4);
   };
-  auto park = [&](int buf) {
+  auto park = [&](int set, u32x4 *stage) {
+    u32x2 *at = (u32x2 *)(stage + (k4 >> 3) * kOctX + srow) + (k4 >> 2 & 1);
 #pragma unroll
-    for (int u = 0; u < NA; ++u) *(f32x4 *)(As + (buf * TM + srow + 32 * u) * AS + k4) = sa[u];
+    for (int u = 0; u < NA; ++u)
+      split_quad(sa[set][u], at[128 * u], at[128 * u + 2 * kPartX], at[128 * u + 4 * kPartX]);
+    at = (u32x2 *)(stage + 3 * kPartX + (k4 >> 3) * kOctW + srow) + (k4 >> 2 & 1);
 #pragma unroll
-    for (int u = 0; u < NW; ++u) *(f32x4 *)(Bs + (buf * TN + srow + 32 * u) * AS + k4) = sb[u];
+    for (int u = 0; u < NW; ++u) split_quad(sb[set][u], at[128 * u], at[128 * u + 2 * kPartW], at[128 * u + 4 * kPartW]);
   };
-  const int n = lane & 31, half = lane >> 5, rw = wave % RW, cw = wave / RW;
-  const float *af_p = As + (rw * 32 + n) * AS + 4 * half, *bf_p = Bs + (cw * NB * 32 + n) * AS + 4 * half;
-  f32x4 af[2], bf[2][NB];
-  auto fetch = [&](int par, int buf, int s) {
-    af[par] = *(const f32x4 *)(af_p + buf * TM * AS + 8 * s);
+  const int n = lane & 31, half = lane >> 5, rw = wave & 1, cw = wave >> 1;
+  const int a_unit = half * kOctX + rw * 32 * MB + n, b_unit = 3 * kPartX + half * kOctW + cw * 64 + n;
+  f32x16 acc[MB][2];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) bf[par][b] = *(const f32x4 *)(bf_p + (buf * TN + b * 32) * AS + 8 * s);
-  };
-  f32x16 acc[NB];
+  for (int a = 0; a < MB; ++a)
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
   const int steps = (K + TK - 1) / TK;
-  load(0);
-  park(0);
-  if (steps > 1) load(TK);
+  load(0, 0);
+  load(1, TK);
+  park(0, lds[0]);
+  load(0, 2 * TK);
   __syncthreads();
-  fetch(0, 0, 0);
-  for (int kt = 0; kt < steps; ++kt) {
-    const int buf = kt & 1;
-    const bool more = kt + 1 < steps;
+  auto step = [&](int kt, int set) {  // set: holds step kt + 1
+    const u32x4 *stage = lds[kt & 1];
+    u32x4 af[3][MB], bf[3][2];
 #pragma unroll
-    for (int s = 0; s < TK / 8; ++s) {
-      const int cur = s & 1, nxt = cur ^ 1;
-      if (s + 1 < TK / 8) {
-        fetch(nxt, buf, s + 1);
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * kPartX + 32 * a];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) bf[p][b] = stage[b_unit + p * kPartW + 32 * b];
+    }
+    park(set, lds[(kt & 1) ^ 1]);
+    load(set, (kt + 3) * TK);
+#pragma unroll
+    for (int p = 0; p < 6; ++p)
+#pragma unroll
+      for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p]][b], acc[a][b]);
+    __syncthreads();
+  };
+  for (int kt = 0; kt < steps; kt += 2) {
+    step(kt, 1);
+    if (kt + 1 < steps) step(kt + 1, 0);
+  }
+
+  // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which
+  const int row0 = m0 + rw * 32 * MB + 4 * half;
+  float probe = 0.f;
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) probe = fmaf(acc[a][b][r], 0.f, probe);
+  if (__any(probe != 0.f)) {
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = min(row0 + 32 * a + 8 * (r >> 2) + (r & 3), r1 - 1);
+        const float *xr = g.x + (long long)(g.gather ? g.gather[row] : row) * K;
+        const float *w0 = w + (long long)matrix_row(cw * 64 + n) * K, *w1 = w + (long long)matrix_row(cw * 64 + 32 + n) * K;
+        float s0 = 0.f, s1 = 0.f;
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < K; ++k) {
+          s0 = fmaf(xr[k], w0[k], s0);
+          s1 = fmaf(xr[k], w1[k], s1);
+        }
+        acc[a][0][r] = s0;
+        acc[a][1][r] = s1;
+      }
+  }
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = row0 + 32 * a + 8 * (r >> 2) + (r & 3);
+      if (row >= r1) continue;
+      float *yr = g.y + (long long)row * N;
+      if constexpr (SWIGLU) {
+        const int col = o0 + cw * 32 + n;
+        if (col < N) yr[col] = swiglu1(acc[a][0][r], acc[a][1][r]);
       } else {
-        if (more) park(buf ^ 1);
-        __syncthreads();
-        if (kt + 2 < steps) load((kt + 2) * TK);
-        if (more) fetch(nxt, buf ^ 1, 0);
-      }
-      ORDER_LDS_AND_MFMA();
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[cur][i], bf[cur][b][i], acc[b], 0, 0, 0);
-      ORDER_LDS_AND_MFMA();
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = m0 + rw * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-    if (row >= r1) continue;
-    float *yr = g.y + (long long)row * N;
-    if constexpr (SWIGLU) {
-#pragma unroll
-      for (int b = 0; b < NB; b += 2) {
-        const int col = o0 + ((cw * NB + b) >> 1) * 32 + n;
-        if (col < N) yr[col] = swiglu1(acc[b][r], acc[b + 1][r]);
-      }
-    } else {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const int col = o0 + (cw * NB + b) * 32 + n;
-        if (col < N) yr[col] = acc[b][r];
+        for (int b = 0; b < 2; ++b) {
+          const int col = o0 + cw * 64 + 32 * b + n;
+          if (col < N) yr[col] = acc[a][b][r];
+        }
       }
     }
-  }
 }
 
 // y[t] (+)= sum over the slots of weight * the expert's row, in the slots' order
@@ -602,38 +631,27 @@ ManyLayout many_layout(const MoeShape &m, int T) {
   return l;
 }
 
-template <int TM>
+template <int MB>
 hipError_t launch_product_tm(const GroupedArgs &g, bool swiglu, hipStream_t stream) {
-  constexpr int TN = TM == 32 ? 256 : 128;
+  constexpr int TM = 64 * MB, TN = 128;
   const long long tiles = g.tile_off ? (long long)g.rows / TM + (g.groups < g.rows ? g.groups : g.rows) : ((long long)g.rows + TM - 1) / TM;
   const int cols = swiglu ? TN / 2 : TN, ny = (g.N + cols - 1) / cols;
   if (tiles < 1 || tiles > 0x7fffffff || ny > 65535) return hipErrorInvalidValue;
   const dim3 grid((unsigned)tiles, (unsigned)ny);
-  const size_t lds = (size_t)2 * (TM + TN) * 36 * sizeof(float);
   const bool vec = (g.K & 3) == 0 && !(((uintptr_t)g.x | (uintptr_t)g.w) & 15);
-#define SHAINET_LAUNCH_PRODUCT(S_, V_)                                                                           \
-  do {                                                                                                           \
-    static const hipError_t e_ = hipFuncSetAttribute((const void *)moe_product_kernel<TM, S_, V_>,               \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);    \
-    if (e_ != hipSuccess) return e_;                                                                             \
-    hipLaunchKernelGGL((moe_product_kernel<TM, S_, V_>), grid, dim3(256), lds, stream, g);                       \
-  } while (0)
   if (swiglu && vec)
-    SHAINET_LAUNCH_PRODUCT(true, true);
+    hipLaunchKernelGGL((moe_product_kernel<MB, true, true>), grid, dim3(256), 0, stream, g);
   else if (swiglu)
-    SHAINET_LAUNCH_PRODUCT(true, false);
+    hipLaunchKernelGGL((moe_product_kernel<MB, true, false>), grid, dim3(256), 0, stream, g);
   else if (vec)
-    SHAINET_LAUNCH_PRODUCT(false, true);
+    hipLaunchKernelGGL((moe_product_kernel<MB, false, true>), grid, dim3(256), 0, stream, g);
   else
-    SHAINET_LAUNCH_PRODUCT(false, false);
-#undef SHAINET_LAUNCH_PRODUCT
+    hipLaunchKernelGGL((moe_product_kernel<MB, false, false>), grid, dim3(256), 0, stream, g);
   return hipGetLastError();
 }
 
 hipError_t launch_product(const GroupedArgs &g, int tm, bool swiglu, hipStream_t stream) {
-  return tm == 128 ? launch_product_tm<128>(g, swiglu, stream)
-         : tm == 64 ? launch_product_tm<64>(g, swiglu, stream)
-                    : launch_product_tm<32>(g, swiglu, stream);
+  return tm == 128 ? launch_product_tm<2>(g, swiglu, stream) : launch_product_tm<1>(g, swiglu, stream);
 }
 
 }  // namespace
@@ -699,9 +717,11 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
   hipLaunchKernelGGL(moe_select_kernel, dim3((unsigned)((T + tokens - 1) / tokens)), dim3(256), lds, stream, m, w.correction, logits,
                      stride, T, tokens, ids, weights, rank, counts);
   // rows an expert gets if the router spreads them evenly
-  const int per_expert = slots / n, best_tm = per_expert > 1024 ? 128 : per_expert > 32 ? 64 : 32;
-  static const int tile_knob = getenv("SHAINET_HIP_MOE_TILE") ? atoi(getenv("SHAINET_HIP_MOE_TILE")) : 0;  // a tuning knob: 32, 64 or 128
-  const int tm = tile_knob == 32 || tile_knob == 64 || tile_knob == 128 ? tile_knob : best_tm;
+  // (tiles of 64 | 128 rows, us a prompt: width 1024, 145 rows an expert 1347 | 1347, 281: 1904 | 2043, 384: 2310 | 2317;
+  // width 2048, 194: 3249 | 3169, 375: 5196 | 5053, 512: 6139 | 5725; tiles of 32 lose 4 to 23 % everywhere, one row included)
+  const int per_expert = slots / n, best_tm = per_expert > 320 ? 128 : 64;
+  static const int tile_knob = getenv("SHAINET_HIP_MOE_TILE") ? atoi(getenv("SHAINET_HIP_MOE_TILE")) : 0;  // a tuning knob: 64 or 128
+  const int tm = tile_knob == 64 || tile_knob == 128 ? tile_knob : best_tm;
   hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, stream, m.experts, tm, counts, off, tile_off);
   hipLaunchKernelGGL(moe_scatter_kernel, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, stream, slots, m.top, m.experts,
                      ids, rank, off, rows);

@@ -38,6 +38,19 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &high, uns
   low = pack_bf16(a, b);
 }
 
+// the three parts of four floats
+__device__ __forceinline__ void split_quad(f32x4 v, u32x2 &high, u32x2 &mid, u32x2 &low) {
+  unsigned a[2], b[2], c[2];
+  split_pair(v.x, v.y, a[0], b[0], c[0]);
+  split_pair(v.z, v.w, a[1], b[1], c[1]);
+  high = u32x2{a[0], a[1]};
+  mid = u32x2{b[0], b[1]};
+  low = u32x2{c[0], c[1]};
+}
+
+// The parts of the two factors in the six products that are taken, smallest first.
+constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
+
 // acc += a b; operands as 16-byte fragments: lane l holds k = 8 (l / 32) .. + 7 of row (column) l % 32.
 // D[m = 8 (r / 4) + 4 (l / 32) + r % 4][n = l % 32] in register r.
 __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {

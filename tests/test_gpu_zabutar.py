@@ -339,6 +339,19 @@ def test_experts(hip, tmp_path, name):
         close(block_cut(b, x, cuts), want)
 
 
+@pytest.mark.parametrize("name", ["plain", "one", "odd"])
+def test_experts_keep_rows_apart(hip, tmp_path, name):
+    """A row that is not a number shares tiles of an expert (64 and 128 rows, whole and ragged) with rows before it that are."""
+    g = MOE[name]
+    p = Pair(hip, tmp_path, zm.config([zm.layer(zm.hgrn2(heads=1, dim=4, vdim=4), zm.moe(**g["moe"]))], width=g["width"]), seed=3)
+    x = (2 * np.random.default_rng(4).standard_normal((420, g["width"]))).astype(np.float32)
+    want = p.layer(0, x)[:384]  # (a chunk of the HGRN2 mixer, 64 rows, is not kept apart)
+    x[384] = np.nan
+    got = p.model.blocks[0].forward_cached(x)
+    close(got[:384], want)
+    assert np.isnan(got[384:]).all()
+
+
 def test_optional_parts_left_out(hip, tmp_path):
     """No groups, scale, identity or shared expert in the configuration; a layer without a feed-forward."""
     cfg = zm.config([zm.layer(zm.attention(), zm.moe(experts=5, identity=0, top=2, groups=1, keep=1, scale=1.0, shared=0)),
