@@ -6,17 +6,17 @@
 //
 //   prefill_mfma_kernel   many new rows.  Query rows and the heads of a group
 //       are flattened into "virtual rows"; a wavefront owns 32 of them, a
-//       workgroup 128.  K/V tiles of 32 keys are staged through LDS (double
-//       buffered) and consumed by v_mfma_f32_32x32x2_f32.
+//       workgroup 128.  K/V tiles of 32 keys are split into bf16 parts on their way
+//       to LDS and consumed by v_mfma_f32_32x32x16_bf16.
 //   generic_attn_kernel   any head_dim; one wavefront per (row, head).  Used for
 //       head dims other than 64 and 128.
 //
 // The MFMA kernels compute S^T = K Q^T so that the probabilities come out of the MFMA
 // accumulator already laid out as the B operand of O^T = V^T P^T: no transpose,
 // no LDS round trip for P.  The contraction index of an MFMA may be visited in
-// any order as long as A and B agree, which lets every lane fetch 16-byte
-// pieces of K rows.
+// any order as long as A and B agree.
 #include "attn_kernels.hpp"
+#include "split_mfma.hpp"
 
 #include <math.h>
 #include <stdlib.h>
@@ -26,15 +26,7 @@ namespace shainet {
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// Scheduling fence that scalar and vector ALU instructions may cross but LDS,
-// MFMA and global-memory instructions may not: keeps operand fetches ahead of the
-// MFMAs that use them, where the source puts them, instead of next to them.
-#define ORDER_LDS_AND_MFMA() __builtin_amdgcn_sched_barrier(0x7)
 
 __device__ __forceinline__ int find_seq(const SeqTable &st, int item, const int *off) {
   int s = 0;
@@ -43,13 +35,12 @@ __device__ __forceinline__ int find_seq(const SeqTable &st, int item, const int 
 }
 
 // ---------------------------------------------------------------------------
-// Prefill: MFMA 32x32x2, K/V tiles staged through LDS.
+// Prefill: MFMA 32x32x16, K/V tiles staged through LDS.
 //
 // Virtual row v of a (sequence, kv head): query row v / g, head kvh*g + v % g.
-// MFMA 32x32x2 layout (lane l): A[m = l%32][k = l/32], B[k = l/32][n = l%32],
-// D[m = 8*(r/4) + 4*(l/32) + r%4][n = l%32] for accumulator register r = 0..15.
-//   scores:  m = key within the tile, n = virtual row; k-step s of lane half
-//            j = l/32 covers d = 8*(s/4) + 4*j + s%4 (float4 pieces of a K row).
+// MFMA layout (lane l, j = l/32): A[m = l%32][k = 8j .. 8j+7], B[k = 8j .. 8j+7][n = l%32],
+// D[m = 8*(r/4) + 4*j + r%4][n = l%32] for accumulator register r = 0..15.
+//   scores:  m = key within the tile, n = virtual row, k = d.
 //   output:  tile t, m = d index (d = NT*m + t), contraction over the tile's keys in
 //            the order the score accumulator holds them.
 // Row block number `rank` in dispatch order -> (sequence, block).  Level 0 is every
@@ -72,12 +63,24 @@ __device__ __forceinline__ void locate_block(const SeqTable &st, int rank, int &
   vb = st.work_off[s] - 1 - level;
 }
 
+// Units of 16 bytes (eight bf16, one MFMA operand of a lane) that one key tile takes in LDS.  K: [part][octet of
+// d][key], an octet's 32 keys one unit apart from a multiple of 16 (a row's octets are written side by side).  V:
+// [part][group of eight keys][column], column d at place d / NT of block d % NT, four units of padding a block; group
+// 2 u + j holds the keys 16 u + 4 j + {0 .. 3, 8 .. 11}, the ones whose probabilities lane half j has in its
+// registers 8 u .. 8 u + 7.
+template <int HD>
+struct TileUnits {
+  static constexpr int NT = HD / 32;
+  static constexpr int kOctK = 33, kPartK = HD / 8 * kOctK;
+  static constexpr int kGroupV = NT * 36, kPartV = 4 * kGroupV;
+  static constexpr int kK = 3 * kPartK, kTile = kK + 3 * kPartV;
+};
+
 // G = 1: four wavefronts, each with 32 virtual rows, walk the key tiles together.
 // G = 2: eight wavefronts; wavefronts 4..7 own the same rows as 0..3 and take every
 // second key tile, so that each SIMD holds two wavefronts of one workgroup and the
-// waits of one (barrier, LDS and memory latencies) hide behind the work of the other
-// even when a launch puts a single workgroup on a compute unit (vector instructions
-// do not hide: fp32 MFMAs and vector instructions share the SIMD's lanes).  The two
+// waits and vector instructions of one hide behind the MFMAs of the other
+// even when a launch puts a single workgroup on a compute unit.  The two
 // halves merge through LDS.
 // One workgroup's work: the row block (and key chunk) number `bid` of the launch.
 // PAD: the head dimension of the data (sh.hd, a multiple of 4) is smaller than HD, the one the
@@ -85,6 +88,15 @@ __device__ __forceinline__ void locate_block(const SeqTable &st, int rank, int &
 // there does not reach the scores), output elements beyond it are not stored, and a tile's
 // pieces beyond it repeat the row's first piece (a cache hit, no HBM traffic).
 // BIAS (with PAD): scores gain a value by distance (DistanceBias), value rows have a width of their own.
+//
+// Queries, keys, values and probabilities enter the MFMAs as exact sums of three bf16 numbers
+// (split_mfma.hpp): the queries once, a key tile by the workgroup on its way to LDS, the probabilities in
+// the registers the scores came in.  A tile costs a wavefront HD / 16 x 6 + HD / 16 x 6 MFMAs of 32 cycles (64:
+// 1536) where the fp32 instruction took HD x 64 (4096), and about as many cycles of vector instructions, which run
+// beside them.  Kernel times, the fp32 instruction before (us): 2048 rows, 32 / 8 heads of 64, 99 (146), 8192 rows 1324
+// (2050); 512 rows on 16384 cached, 32 / 4 heads of 128, 684 (1056); 2048 rows, 32 / 8 heads of 128, 186 (279).
+// Bound by the power the card may draw, as the large products are; raising one group's priority changes nothing and
+// parking V between the score MFMAs costs 5 to 16 %.
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS>
 __device__ __forceinline__ void prefill_block(const int bid, const float *__restrict__ q_rot,
                                               const float *__restrict__ kc, const float *__restrict__ vc,
@@ -92,14 +104,12 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
                                               float *__restrict__ part_ml, const SeqTable &st, const Shape &sh,
                                               int ns, float c, const DistanceBias &db) {
   static_assert(PAD || !BIAS, "sizes of their own come with padding");
-  constexpr int NK4 = HD / 8;   // float4 pieces of a K row per lane
+  using U = TileUnits<HD>;
+  constexpr int KS = HD / 16;   // MFMA steps along d of the scores
   constexpr int NT = HD / 32;   // d tiles of the output
-  constexpr int KSTR = HD + 4;  // padded K row stride in LDS: conflict-free 16-byte reads down a column
-  constexpr int LD4 = HD / 32;  // float4 per thread to stage the G K (or V) tiles of one step
+  constexpr int NI = HD / 64;   // items per thread to stage the G K (or V) tiles of one step
   constexpr int NTHREADS = 256 * G;
-  constexpr int TILE4 = 32 * (HD / 4);  // float4 per tile
-  __shared__ float Ks[2][G][32 * KSTR];
-  __shared__ float Vs[2][G][32 * HD];
+  __shared__ __attribute__((aligned(16))) u32x4 lds[G * U::kTile];
 
   // Workgroups are numbered so that the hardware dispatcher, which hands them out in
   // index order, starts the row blocks with the longest key ranges first; the kv
@@ -113,8 +123,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   int s, vb;
   locate_block(st, item, s, vb);
   // These are the same for all lanes of a wavefront, which the compiler cannot see: said so,
-  // tile counts, loop conditions and address bases live in scalar registers and their
-  // arithmetic leaves the vector ALU, which the MFMAs need
+  // tile counts, loop conditions and address bases live in scalar registers
   auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
   s = uniform(s);
   vb = uniform(vb);
@@ -147,200 +156,130 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   // entry of key row k: bias_row[k]
   const float *bias_row = BIAS ? db.tab + (long long)(kvh * g + hg) * db.stride + (db.origin - lim) : nullptr;
 
-  float qr[HD / 2];
-  {
-    const float *qp = q_rot + q_off + 4 * j;
+  // what a thread stages of a step's G tiles: K, an octet of d of a row; V, eight rows of a column
+  unsigned k_off[NI], v_off[NI];
+  int k_row[NI], v_row[NI], k_unit[NI], v_unit[NI];
+  bool k_second[NI];  // the octet's second half lies within the row
 #pragma unroll
-    for (int i = 0; i < NK4; ++i) {
-      // (lanes past the last virtual row repeat the last row: their results are never used,
-      // and not touching the loaded values here lets the first K and V loads go out behind
-      // these instead of after their arrival)
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      if (!PAD || 8 * i + 4 * j < hd) t = *(const f32x4 *)(qp + 8 * i);
-      qr[4 * i + 0] = t.x;
-      qr[4 * i + 1] = t.y;
-      qr[4 * i + 2] = t.z;
-      qr[4 * i + 3] = t.w;
+  for (int u = 0; u < NI; ++u) {
+    const int idx = threadIdx.x + NTHREADS * u;
+    const int oct = idx % (HD / 8), r = idx / (HD / 8);
+    k_row[u] = r;
+    k_off[u] = PAD && 8 * oct >= hd ? 0u : 32u * oct;
+    k_second[u] = !PAD || 8 * oct + 4 < hd;
+    k_unit[u] = (r >> 5) * U::kTile + oct * U::kOctK + (r & 31);
+    const int d = idx % HD, group = idx / HD & 3, ts = idx / (4 * HD);
+    v_row[u] = 32 * ts + 16 * (group >> 1) + 4 * (group & 1);
+    v_off[u] = PAD && d >= vhd ? 0u : 4u * d;
+    v_unit[u] = ts * U::kTile + U::kK + group * U::kGroupV + d % NT * 36 + d / NT;
+  }
+  const unsigned k_stride = (unsigned)hd * 4, v_stride = (unsigned)vhd * 4;
+  f32x4 stage_k[NI][2];
+  float stage_v[NI][8];
+  // a scalar base and a 32-bit byte offset per lane (a head's rows span less than 4 GiB: checked
+  // at launch); rows past the last one repeat it
+  auto load_k = [&](int sp) {
+    const int first = (kt0 + G * sp) * 32;
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      const char *p = (const char *)kbase + ((unsigned)min(first + k_row[u], L - 1) * k_stride + k_off[u]);
+      stage_k[u][0] = *(const f32x4 *)p;
+      stage_k[u][1] = *(const f32x4 *)(p + (k_second[u] ? 16 : 0));
     }
+  };
+  auto load_v = [&](int sp) {
+    const int first = (kt0 + G * sp) * 32;
+    if (first + 32 * G <= L) {
+      const char *base = (const char *)vbase + (unsigned long long)first * v_stride;
+#pragma unroll
+      for (int u = 0; u < NI; ++u) {
+        const unsigned off = (unsigned)v_row[u] * v_stride + v_off[u];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) stage_v[u][i] = *(const float *)(base + (unsigned long long)((i & 3) + 8 * (i >> 2)) * v_stride + off);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < NI; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          stage_v[u][i] = *(const float *)((const char *)vbase +
+                                           ((unsigned)min(first + v_row[u] + (i & 3) + 8 * (i >> 2), L - 1) * v_stride + v_off[u]));
+    }
+  };
+  auto park_k = [&]() {
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      u32x4 h, m, l;
+      split_octet(stage_k[u][0], stage_k[u][1], h, m, l);
+      lds[k_unit[u]] = h;
+      lds[k_unit[u] + U::kPartK] = m;
+      lds[k_unit[u] + 2 * U::kPartK] = l;
+    }
+  };
+  auto park_v = [&]() {
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      u32x4 h, m, l;
+      split_octet(f32x4{stage_v[u][0], stage_v[u][1], stage_v[u][2], stage_v[u][3]},
+                  f32x4{stage_v[u][4], stage_v[u][5], stage_v[u][6], stage_v[u][7]}, h, m, l);
+      lds[v_unit[u]] = h;
+      lds[v_unit[u] + U::kPartV] = m;
+      lds[v_unit[u] + 2 * U::kPartV] = l;
+    }
+  };
+
+  // steps of G tiles, one per group of wavefronts; below "tile sp" is this group's tile of step sp
+  const int n_sp = kt0 < kt1 ? (kt1 - kt0 + G - 1) / G : 0;
+  if (n_sp > 0) {
+    load_k(0);
+    load_v(0);
+  }
+  // the row's query, scaled by scale * log2(e): scores come out in log2 units
+  u32x4 qf[KS][3];
+  {
+    f32x4 t[KS][2];
+    const float *qp = q_rot + q_off + 8 * j;
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // (lanes past the last virtual row repeat the last row: their results are never used)
+        t[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!PAD || 16 * i + 8 * j + 4 * h < hd) t[i][h] = *(const f32x4 *)(qp + 16 * i + 4 * h);
+      }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) split_octet(t[i][0] * c, t[i][1] * c, qf[i][0], qf[i][1], qf[i][2]);
   }
 
-  // Online softmax against a reference value per virtual row instead of the running maximum.
-  // The fp32 MFMAs run on the lanes of the vector ALU (a wavefront's vector instructions and
-  // MFMAs, its own or its SIMD neighbour's, never overlap: measured, 6 cycles per fma and 12
-  // per exp2 added to a stream of 64-cycle MFMAs), so every vector instruction of the tile loop
-  // is paid in matrix throughput.  Hence:
-  //   * the query rows are scaled by scale * log2(e) once, so scores come out in log2 units;
-  //   * the score accumulator starts at -m_ref instead of 0, so the MFMAs deliver s - m_ref;
-  //   * m_ref is only moved (and l, O rescaled) when a score exceeds it by more than kTau, or
-  //     for a row's first visible key; probabilities are then at most 2^kTau, no overflow.
-  // A tile on the common path costs a maximum, 16 exp2 and 16 adds per lane.
+  // Online softmax against a reference value per virtual row instead of the running maximum: m_ref is only moved
+  // (and l, O rescaled) when a score exceeds it by more than kTau, or for a row's first visible key;
+  // probabilities are then at most 2^kTau, no overflow.  A tile on the common path costs a maximum, 16
+  // subtractions, exp2 and adds per lane.
   constexpr float kTau = 8.f;
   float m_ref = 0.f, l = 0.f;
-  float thr = -INFINITY;  // a row's scores move m_ref when above this: anything finite until its first key, kTau after
-  // -m_ref as the score MFMAs' initial accumulator: sixteen registers that hold it, or, where
-  // registers are short (head_dim 128), one more MFMA per tile that multiplies it by a column
-  // of ones
-  constexpr bool kRefByMfma = HD == 128;
-  f32x16 neg_m;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) neg_m[r] = 0.f;
-  const float ones_col = j == 0 ? 1.f : 0.f;  // A[key][k]: 1 for k = 0
+  float thr = -INFINITY;  // a row's scores move m_ref when above this: anything finite until its first key, m_ref + kTau after
   f32x16 o[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
 
-  // Staging registers: the G tiles of a step (tiles kt0 + G*sp .. + G-1, one per
-  // group of wavefronts) travel global memory -> registers during one iteration and
-  // registers -> LDS at the start of the next.
-  f32x4 stage_k[LD4], stage_v[LD4];
-  // what a thread fetches of a step's G tiles does not change from step to step: row
-  // row_in_step[u] of the step's 32 G rows, columns col4 .. col4 + 3
-  int row_in_step[LD4];
-#pragma unroll
-  for (int u = 0; u < LD4; ++u) {
-    const int idx = threadIdx.x + NTHREADS * u;
-    const int ts = idx / TILE4, rem = idx - ts * TILE4;
-    row_in_step[u] = ts * 32 + rem / (HD / 4);
-  }
-  // NTHREADS is a multiple of HD / 4
-  const unsigned col_bytes = PAD && 4 * (threadIdx.x % (HD / 4)) >= (unsigned)hd ? 0u : 16u * (threadIdx.x % (HD / 4));
-  const unsigned v_col_bytes = PAD && 4 * (threadIdx.x % (HD / 4)) >= (unsigned)vhd ? 0u : 16u * (threadIdx.x % (HD / 4));
-  static_assert(NTHREADS % (HD / 4) == 0, "a thread keeps its columns");
-  // a scalar base and a 32-bit byte offset per lane (a head's rows span less than 4 GiB: checked
-  // at launch); rows past the last one repeat it
-  auto load_tiles = [&](f32x4 (&dst)[LD4], const float *base, int sp, int width, unsigned col) {
-    const int first_row = (kt0 + G * sp) * 32;
-#pragma unroll
-    for (int u = 0; u < LD4; ++u) {
-      const unsigned off = (unsigned)min(first_row + row_in_step[u], L - 1) * (unsigned)(width * 4) + col;
-      dst[u] = *(const f32x4 *)((const char *)base + off);
-    }
-  };
-  auto park_k = [&](const f32x4 (&src)[LD4], int buf) {
-#pragma unroll
-    for (int u = 0; u < LD4; ++u) {
-      const int idx = threadIdx.x + NTHREADS * u;
-      const int ts = idx / TILE4, rem = idx - ts * TILE4;
-      const int r = rem / (HD / 4), c4 = rem - r * (HD / 4);
-      *(f32x4 *)&Ks[buf][ts][r * KSTR + 4 * c4] = src[u];
-    }
-  };
-  auto park_v = [&](const f32x4 (&src)[LD4], int buf) {
-#pragma unroll
-    for (int u = 0; u < LD4; ++u) {
-      const int idx = threadIdx.x + NTHREADS * u;
-      const int ts = idx / TILE4, rem = idx - ts * TILE4;
-      const int r = rem / (HD / 4), c4 = rem - r * (HD / 4);
-      *(f32x4 *)&Vs[buf][ts][r * HD + 4 * c4] = src[u];
-    }
-  };
-  auto load_k = [&](int sp) { load_tiles(stage_k, kbase, sp, hd, col_bytes); };
-  auto load_v = [&](int sp) { load_tiles(stage_v, vbase, sp, vhd, v_col_bytes); };
-  auto store_k = [&](int buf) { park_k(stage_k, buf); };
-  auto store_v = [&](int buf) { park_v(stage_v, buf); };
-
-  // S^T of one key tile: 32 keys x 32 virtual rows, K from LDS stage `buf`
-  // MFMA operands come from LDS; every fetch is issued PF steps before the MFMAs
-  // that use it, so that the matrix pipe never waits for an LDS round trip.
-  auto scores = [&](int buf) {
-    constexpr int PF = 2;
-    f32x16 sacc;
-    if constexpr (kRefByMfma) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-      sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ones_col, -m_ref, sacc, 0, 0, 0);
-    } else {
-      sacc = neg_m;
-    }
-    const float *kl = &Ks[buf][gidx][n * KSTR + 4 * j];
-    f32x4 kv[NK4];
-#pragma unroll
-    for (int i = 0; i < PF && i < NK4; ++i) kv[i] = *(const f32x4 *)(kl + 8 * i);
-#pragma unroll
-    for (int i = 0; i < NK4; ++i) {
-      if (i + PF < NK4) kv[i + PF] = *(const f32x4 *)(kl + 8 * (i + PF));
-      ORDER_LDS_AND_MFMA();
-      sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].x, qr[4 * i + 0], sacc, 0, 0, 0);
-      sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].y, qr[4 * i + 1], sacc, 0, 0, 0);
-      sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].z, qr[4 * i + 2], sacc, 0, 0, 0);
-      sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].w, qr[4 * i + 3], sacc, 0, 0, 0);
-      ORDER_LDS_AND_MFMA();
-    }
-    return sacc;
-  };
-
-  // Software pipeline over the key tiles, in steps of G tiles (one per group of
-  // wavefronts; below "tile sp" is this group's tile of step sp).  Step sp issues the
-  // MFMAs of S^T(sp+1) before the softmax arithmetic of tile sp (its scores are then a
-  // step old and certainly there), then O^T += V^T(sp) P^T(sp).  K runs two steps ahead of V:
-  //   LDS at the start of step sp:  K(sp+1) in Ks[(sp+1)&1], V(sp) in Vs[sp&1];
-  //   registers:                     K(sp+2), V(sp+1), fetched during step sp-1.
-  // The step first parks those registers in the two LDS stages nobody reads any
-  // more (Ks[sp&1] held K(sp), Vs[(sp+1)&1] held V(sp-1); both were last read in
-  // step sp-1), then fetches K(sp+3) and V(sp+2).  One barrier per step, at its
-  // end, orders all of this.
-  const int n_sp = kt0 < kt1 ? (kt1 - kt0 + G - 1) / G : 0;
-  f32x16 s_cur, s_next;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) s_cur[r] = s_next[r] = 0.f;
+  // One stage of LDS for K and one for V.  Step sp: scores and softmax of tile sp from K(sp), V(sp) is parked
+  // meanwhile; a barrier; O^T += V^T(sp) P^T(sp), K(sp + 1) is parked meanwhile; a barrier.  What is parked was
+  // requested a step before.
+  const u32x4 *tile = lds + gidx * U::kTile;
   if (n_sp > 0) {
-    // everything the first step needs is requested at once, with registers of its own for
-    // the tiles that go to LDS right away: one memory round trip before the first MFMA
-    // instead of three
-    f32x4 k0[LD4], v0[LD4], k1[LD4];
-    load_tiles(k0, kbase, 0, hd, col_bytes);
-    load_tiles(v0, vbase, 0, vhd, v_col_bytes);
-    if (n_sp > 1) {
-      load_tiles(k1, kbase, 1, hd, col_bytes);
-      load_v(1);
-    }
-    if (n_sp > 2) load_k(2);
-    park_k(k0, 0);
-    park_v(v0, 0);
-    if (n_sp > 1) park_k(k1, 1);
+    park_k();
+    if (n_sp > 1) load_k(1);
   }
-#pragma unroll
-  for (int i = 0; i < HD / 2; ++i) qr[i] *= c;
   __syncthreads();
-  if (kt0 + gidx < kt1 && (kt0 + gidx) * 32 <= wave_hi) s_cur = scores(0);
-  __syncthreads();  // step 0 overwrites Ks[0]
-
-  // O^T += V^T P^T of one tile; the probabilities are the registers of `p`
-  auto accumulate = [&](const f32x16 &p, int buf) {
-    constexpr int PF = NT == 2 ? 4 : 2;
-    const float *vl = &Vs[buf][gidx][4 * j * HD + NT * n];
-    typedef float vrow_t __attribute__((ext_vector_type(NT)));
-    vrow_t vv[16];
-#pragma unroll
-    for (int r = 0; r < PF; ++r) vv[r] = *(const vrow_t *)(vl + (8 * (r >> 2) + (r & 3)) * HD);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      if (r + PF < 16) vv[r + PF] = *(const vrow_t *)(vl + (8 * ((r + PF) >> 2) + ((r + PF) & 3)) * HD);
-      ORDER_LDS_AND_MFMA();
-#pragma unroll
-      for (int t = 0; t < NT; ++t) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[r][t], p[r], o[t], 0, 0, 0);
-      ORDER_LDS_AND_MFMA();
-    }
-  };
-
-  // One step; `cur` holds this step's scores, `nxt` receives the next step's.  The loop below
-  // calls it with the two register sets swapping roles, so that nothing is copied between
-  // steps (T = 2048: 161 -> 154 us).
-  auto step = [&](const int sp, f32x16 &cur, f32x16 &nxt) {
-    const int buf = sp & 1;
-    const int kt = kt0 + G * sp + gidx, kt_next = kt + G;  // this group's tile now and in the next step
-    if (sp + 2 < n_sp) store_k(buf);
-    if (sp + 1 < n_sp) store_v(buf ^ 1);
-    if (sp + 3 < n_sp) load_k(sp + 3);
-    if (sp + 2 < n_sp) load_v(sp + 2);
-    const bool have_next = kt_next < kt1 && kt_next * 32 <= wave_hi;
-    const bool have_cur = kt < kt1 && kt * 32 <= wave_hi;
-    // the tile's values by distance are asked for in front of the next tile's MFMAs; a tile that lies
+  for (int sp = 0; sp < n_sp; ++sp) {
+    const int kt = kt0 + G * sp + gidx;  // this group's tile
+    const bool have = kt < kt1 && kt * 32 <= wave_hi;
+    // the tile's values by distance are asked for in front of its MFMAs; a tile that lies
     // `reach` or more behind all rows of the wavefront has none
     f32x4 near_bias[BIAS ? 4 : 1];
-    const bool near = BIAS && have_cur && wave_lo - (kt * 32 + 31) < db.reach;
+    const bool near = BIAS && have && wave_lo - (kt * 32 + 31) < db.reach;
     if constexpr (BIAS) {
       if (near) {
         struct __attribute__((packed, aligned(4))) Four { f32x4 v; };
@@ -348,63 +287,133 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
         for (int r = 0; r < 4; ++r) near_bias[r] = ((const Four *)(bias_row + kt * 32 + 8 * r + 4 * j))->v;
       }
     }
-    if (have_next) nxt = scores(buf ^ 1);
-    if (have_cur) {
-      f32x16 &sacc = cur;            // scores of tile kt minus m_ref, log2 units; not needed after this step
+    f32x16 p;
+    if (have) {
+      // S^T of the key tile: 32 keys x 32 virtual rows
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = 0.f;
+      const u32x4 *kl = tile + j * U::kOctK + n;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        u32x4 kf[3];
+#pragma unroll
+        for (int w = 0; w < 3; ++w) kf[w] = kl[w * U::kPartK + 2 * i * U::kOctK];
+#pragma unroll
+        for (int w = 0; w < 6; ++w) p = mfma_bf16(kf[kPartA[w]], qf[i][kPartB[w]], p);
+      }
+    }
+    park_v();
+    if (sp + 1 < n_sp) load_v(sp + 1);
+    if (have) {
       if constexpr (BIAS) {
         if (near) {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) sacc[r] += near_bias[r >> 2][r & 3];
+          for (int r = 0; r < 16; ++r) p[r] += near_bias[r >> 2][r & 3];
         }
       }
       if (kt * 32 + 31 > wave_lo) {  // tile crosses the diagonal for some row of this wavefront
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = kt * 32 + 8 * (r >> 2) + 4 * j + (r & 3);
-          if (key > lim) sacc[r] = -INFINITY;
+          if (key > lim) p[r] = -INFINITY;
         }
       }
-      float mx = fmaxf(fmaxf(sacc[0], sacc[1]), sacc[2]);
+      float mx = fmaxf(fmaxf(p[0], p[1]), p[2]);
 #pragma unroll
-      for (int r = 3; r < 15; r += 2) mx = fmaxf(fmaxf(mx, sacc[r]), sacc[r + 1]);
-      mx = fmaxf(mx, sacc[15]);
+      for (int r = 3; r < 15; r += 2) mx = fmaxf(fmaxf(mx, p[r]), p[r + 1]);
+      mx = fmaxf(mx, p[15]);
       // mx covers this lane's half of the row's keys in the tile; the row's maximum is above thr
       // exactly when one of the two halves' is (never for a row without a visible key here:
       // -inf), so the halves only exchange their maxima once a move is certain
       if (__builtin_amdgcn_ballot_w64(mx > thr) != 0) {
         // rare after a row's first tiles: move the reference to this tile's maximum
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const bool move = mx > thr;
-        const float delta = move ? mx : 0.f;
-        const float alpha = (move && thr != -INFINITY) ? fast_exp2(-delta) : 1.f;  // nothing to rescale before a row's first key
-        m_ref += delta;
-        l *= alpha;
+        if (mx > thr) {
+          const float alpha = thr != -INFINITY ? fast_exp2(m_ref - mx) : 1.f;  // nothing to rescale before a row's first key
+          m_ref = mx;
+          thr = mx + kTau;
+          l *= alpha;
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+          for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          sacc[r] -= delta;
-          nxt[r] -= delta;     // computed against the old reference (unused if there is no next tile)
-          if constexpr (!kRefByMfma) neg_m[r] = -m_ref;
+            for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
         }
-        if (move) thr = kTau;
       }
       float psum = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        sacc[r] = fast_exp2(sacc[r]);
-        psum += sacc[r];
+        p[r] = fast_exp2(p[r] - m_ref);
+        psum += p[r];
       }
       l += psum;
-      accumulate(sacc, buf);
     }
-    __syncthreads();
-  };
-  for (int sp = 0; sp < n_sp; sp += 2) {
-    step(sp, s_cur, s_next);
-    if (sp + 1 < n_sp) step(sp + 1, s_next, s_cur);
+    __syncthreads();  // V(sp) is there, nobody reads K(sp) any more
+    if (have) {
+      // O^T += V^T P^T; the probabilities are where the scores were
+      const u32x4 *vl = tile + U::kK + j * U::kGroupV + n;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        u32x4 pf[3];
+        split_octet(f32x4{p[8 * u], p[8 * u + 1], p[8 * u + 2], p[8 * u + 3]},
+                    f32x4{p[8 * u + 4], p[8 * u + 5], p[8 * u + 6], p[8 * u + 7]}, pf[0], pf[1], pf[2]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          u32x4 vf[3];
+#pragma unroll
+          for (int w = 0; w < 3; ++w) vf[w] = vl[w * U::kPartV + 2 * u * U::kGroupV + 36 * t];
+#pragma unroll
+          for (int w = 0; w < 6; ++w) o[t] = mfma_bf16(vf[kPartA[w]], pf[kPartB[w]], o[t]);
+        }
+      }
+    }
+    if (sp + 1 < n_sp) park_k();
+    if (sp + 2 < n_sp) load_k(sp + 2);
+    __syncthreads();  // K(sp + 1) is there, nobody reads V(sp) any more
+  }
+
+  // Results that are not finite come from operands that are not (or from values that round to infinity as bf16):
+  // the wavefront takes its tiles again in fp32, which says which.
+  {
+    float probe = l * 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
+    if (__any(probe != 0.f)) {
+      m_ref = 0.f, l = 0.f, thr = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+#pragma clang loop unroll(disable)
+      for (int kt = kt0 + gidx; kt < kt1 && kt * 32 <= wave_hi; kt += G)
+#pragma clang loop unroll(disable)
+        for (int key = kt * 32; key < kt * 32 + 32 && key <= wave_hi; ++key) {
+          if (key > lim) continue;
+          float sc = 0.f;
+#pragma clang loop unroll(disable)
+          for (int d = 0; d < hd; ++d) sc = fmaf(q_rot[q_off + d] * c, kbase[(long long)key * hd + d], sc);
+          if (BIAS && lim - key < db.reach) sc += bias_row[key];
+          if (sc > thr) {  // here the reference is the running maximum
+            const float alpha = thr == -INFINITY ? 0.f : fast_exp2(thr - sc);
+            m_ref = thr = sc;
+            l *= alpha;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+          }
+          const float e = sc == -INFINITY ? 0.f : fast_exp2(sc - m_ref);
+          l += 0.5f * e;  // (both lane halves of a row count every key)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const int d = NT * (8 * (r >> 2) + 4 * j + (r & 3)) + t;
+              o[t][r] = fmaf(e, vbase[(long long)key * vhd + (PAD && d >= vhd ? 0 : d)], o[t][r]);
+            }
+        }
+    }
   }
 
   l += __shfl_xor(l, 32);
@@ -414,8 +423,9 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   if constexpr (G == 2) {
     // the second group hands its (max, sum, O) to the first through the tile stages
     // (every wavefront is past the last step's barrier: nobody reads tiles any more)
-    float *xo = &Ks[0][0][0];  // [4 row chunks][16 * NT registers][64 lanes]
-    float *xm = &Vs[0][0][0];  // [4][64] max, then [4][64] sum
+    float *xo = (float *)lds;                   // [4 row chunks][16 * NT registers][64 lanes]
+    float *xm = (float *)lds + 4 * 16 * NT * 64;  // [4][64] max, then [4][64] sum
+    static_assert(sizeof lds >= (4 * 16 * NT * 64 + 512) * sizeof(float), "the merge fits the tiles");
     if (gidx == 1) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
@@ -467,8 +477,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   }
 }
 
+// (three workgroups of four wavefronts on a compute unit where the registers allow: 8192 rows, 32 / 8 heads of 64,
+// 1377 -> 1324 us)
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS = false>
-__global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void prefill_mfma_kernel(const float *__restrict__ q_rot,
+__global__ __launch_bounds__(256 * G, G == 1 ? (HD == 64 && !PAD ? 3 : 2) : 1) void prefill_mfma_kernel(const float *__restrict__ q_rot,
                                                               const float *__restrict__ kc,
                                                               const float *__restrict__ vc,
                                                               float *__restrict__ out,
@@ -539,8 +551,8 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float *__res
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        // 0 for a chunk that saw no visible key, and for the clamped repeats past the last chunk
-        const float f = k0 + u < ns ? fast_exp2((mk[u] - mm) * c) : 0.f;
+        if (k0 + u >= ns) break;  // (repeats of the last chunk: 0 times what is not finite would not be 0)
+        const float f = fast_exp2((mk[u] - mm) * c);  // 0 for a chunk that saw no visible key
         acc += f * x[u];
         ls += f * lk[u];
       }
@@ -725,9 +737,9 @@ PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_pe
   // once: run one workgroup per compute unit (below) and give it eight wavefronts,
   // two per SIMD (G = 2).  Larger launches already have several workgroups per unit.
   p.groups = groups == 1 || groups == 2 ? groups : (p.n_wgs <= 768 ? 2 : 1);
-  // static LDS of the kernel: two stages of `groups` padded K tiles and V tiles
+  // static LDS of the kernel: `groups` K tiles and V tiles
   const int tile_hd = prefill_tile_head_dim(widest(sh, v_hd));
-  const size_t static_lds = (size_t)2 * p.groups * (32 * (tile_hd + 4) + 32 * tile_hd) * sizeof(float);
+  const size_t static_lds = (size_t)16 * p.groups * (tile_hd == 64 ? TileUnits<64>::kTile : TileUnits<128>::kTile);
   p.pad = 0;
   // With fewer workgroups than three per compute unit everything is resident at
   // once and the dispatcher cannot balance the triangular work: one workgroup per

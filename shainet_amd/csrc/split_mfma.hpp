@@ -48,6 +48,16 @@ __device__ __forceinline__ void split_quad(f32x4 v, u32x2 &high, u32x2 &mid, u32
   low = u32x2{c[0], c[1]};
 }
 
+// the three parts of eight floats: a fragment of each
+__device__ __forceinline__ void split_octet(f32x4 a, f32x4 b, u32x4 &high, u32x4 &mid, u32x4 &low) {
+  u32x2 h[2], m[2], l[2];
+  split_quad(a, h[0], m[0], l[0]);
+  split_quad(b, h[1], m[1], l[1]);
+  high = u32x4{h[0].x, h[0].y, h[1].x, h[1].y};
+  mid = u32x4{m[0].x, m[0].y, m[1].x, m[1].y};
+  low = u32x4{l[0].x, l[0].y, l[1].x, l[1].y};
+}
+
 // The parts of the two factors in the six products that are taken, smallest first.
 constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
 

@@ -906,3 +906,50 @@ def test_prefill_random_shapes(hip, seed, monkeypatch):
     assert check_step(ctx, cache, blocks, r, first, what=f"{what} new {first}") < 1e-4
     assert check_step(ctx, cache, blocks, r, second, what=f"{what} then {second}") < 1e-4
     check_cache_bits(cache, blocks)
+
+
+@pytest.mark.parametrize("hd,KV,T,cached", [(64, 2, 300, 0), (128, 2, 70, 100), (96, 4, 40, 33), (128, 8, 700, 0), (64, 8, 2300, 0)])
+def test_prefill_keeps_what_is_not_finite(hip, hd, KV, T, cached):
+    """Infinities, NaN and values that round to infinity as bf16, in queries, keys and values: the rows that meet them
+    come out as fp32 arithmetic has them, the others (rows before them, tile-mates among those) as ever."""
+    import torch
+
+    H, S = 2 * KV, cached + T
+    g = torch.Generator(device="cuda").manual_seed(hd + T)
+    q, k, v = (torch.randn((T, n * hd), generator=g, device="cuda") for n in (H, KV, KV))
+    kc, vc = (torch.randn((KV, max(cached, 1), hd), generator=g, device="cuda") for _ in range(2))
+    ctx = hip.AttnContext(H, KV, hd, max_positions=S)
+    t = [T // 4, T // 3, T // 2, 2 * T // 3, T - 2]
+    v.view(T, KV, hd)[t[0], 0, 3] = float("inf")
+    v.view(T, KV, hd)[t[1], 0, 5] = 3.4e38
+    v.view(T, KV, hd)[t[2], 1, 7] = float("nan")
+    q.view(T, H, hd)[t[3], H - 1, 1] = float("nan")
+    k.view(T, KV, hd)[t[4], KV - 1, 0] = float("inf")
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, S)
+    if cached:
+        cache.fill(0, kc, vc)
+    ctx.sync()
+    got = ctx.forward(cache, q, k, v, [T])
+    ctx.sync()
+    rows = np.stack([np.stack([cache.read(0, c, 0, S)[i] for c in range(KV)]) for i in (0, 1)]).astype(np.float64)
+    qr = ctx.last_q_rot(T).astype(np.float64).reshape(T, H, hd)
+    got = got.cpu().numpy().reshape(T, H, hd)
+    want = np.empty((T, H, hd))
+    with np.errstate(all="ignore"):
+        for h in range(H):
+            s = qr[:, h] @ rows[0, h // 2].T / np.sqrt(hd)
+            s[np.arange(S)[None] > cached + np.arange(T)[:, None]] = -np.inf
+            p = np.exp(s - s.max(-1, keepdims=True))
+            p /= p.sum(-1, keepdims=True)
+            full = rows[1, h // 2]
+            bad = ~np.isfinite(full).all(-1)
+            o = p[:, ~bad] @ full[~bad]
+            for j in np.flatnonzero(bad):  # keys a row does not see add nothing, whatever their values are
+                seen = cached + np.arange(T) >= j
+                o[seen] += p[seen, j:j + 1] * full[j]
+            want[:, h] = o
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    fine = np.isfinite(want)
+    assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-3 * np.abs(want[fine]))
