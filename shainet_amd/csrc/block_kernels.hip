@@ -147,28 +147,36 @@ __global__ __launch_bounds__(256) void add_bias_row_kernel(float *__restrict__ l
 // The reference walks the ids in order and rewrites the logit once per occurrence, so an id that repeats is
 // penalised repeatedly.  Different ids do not meet: the thread of an id's first place does all its occurrences.
 // The ids (a few dozen) travel in the kernel's arguments where they fit, without a copy to the device first.
-// 64 ids: 5 us; one thread that walks them, a memory round trip each, 22 us.
-__device__ __forceinline__ void penalise(float *__restrict__ logits, int vocab, const int *ids, int n, double p) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const int id = i < n ? ids[i] : -1;
+// 64 ids: 6 us; one thread that walks them, a memory round trip each, 22 us.
+__device__ __forceinline__ void penalise(float *__restrict__ logits, int vocab, const int *ids, int padded, int i, double p) {
+  const int id = ids[i];
   if (id < 0 || id >= vocab) return;
-  for (int j = 0; j < i; ++j)
-    if (ids[j] == id) return;
-  float v = logits[id];
-  for (int j = i; j < n; ++j)
-    if (ids[j] == id) v = (float)(v > 0.f ? (double)v / p : (double)v * p);
+  float v = logits[id];  // (asked for before it is known whether the place is the first: it is in flight meanwhile)
+  int times = 0;
+  bool first = true;
+#pragma unroll 4
+  for (int j = 0; j < padded; j += 4) {
+    const int4 other = *(const int4 *)(ids + j);
+    first = first && !((other.x == id && j < i) || (other.y == id && j + 1 < i) || (other.z == id && j + 2 < i) ||
+                       (other.w == id && j + 3 < i));
+    times += (other.x == id) + (other.y == id) + (other.z == id) + (other.w == id);
+  }
+  if (!first) return;
+  for (; times > 0; --times) v = (float)(v > 0.f ? (double)v / p : (double)v * p);
   logits[id] = v;
 }
+// (ids: n of them and -1 up to a multiple of 4)
 __global__ __launch_bounds__(256) void repetition_penalty_kernel(float *__restrict__ logits, int vocab,
                                                                  const int *__restrict__ ids, int n, double p) {
-  penalise(logits, vocab, ids, n, p);
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) penalise(logits, vocab, ids, (n + 3) & ~3, i, p);
 }
 __global__ __launch_bounds__(256) void repetition_penalty_list_kernel(float *__restrict__ logits, int vocab, const IdList list,
                                                                       int n, double p) {
-  __shared__ int ids[kIdList];
-  if ((int)threadIdx.x < n) ids[threadIdx.x] = list.id[threadIdx.x];
+  __shared__ __attribute__((aligned(16))) int ids[kIdList];
+  ids[threadIdx.x] = (int)threadIdx.x < n ? list.id[threadIdx.x] : -1;
   __syncthreads();
-  penalise(logits, vocab, ids, n, p);
+  if ((int)threadIdx.x < n) penalise(logits, vocab, ids, (n + 3) & ~3, threadIdx.x, p);
 }
 
 // ---- top-k ------------------------------------------------------------------
@@ -212,13 +220,23 @@ struct TopkLds {
 // The k-th largest of the threads' largest keys has at least k keys at or above it, and hardly more when the
 // large keys are spread over the threads.  (Keys are unique but for 0, so equal logits do not crowd the pool.)
 __device__ __forceinline__ void topk_threshold(TopkLds &s, unsigned long long mine, int k) {
-  s.best[threadIdx.x] = mine;
+  // (up to 48 of them: the largest keys of four threads each are enough, and a quarter of the comparisons)
+  const bool few = k <= 48;
+  if (few) {
+#pragma unroll
+    for (int o = 1; o <= 2; o <<= 1) {
+      const unsigned long long other = __shfl_xor(mine, o);
+      mine = other > mine ? other : mine;
+    }
+  }
+  const int groups = few ? kTopkThreads / 4 : kTopkThreads;
+  if (!few || (threadIdx.x & 3) == 0) s.best[few ? threadIdx.x >> 2 : threadIdx.x] = mine;
   if (threadIdx.x == 0) s.threshold = 0ull, s.pooled = 0;
   __syncthreads();
   int above = 0;
 #pragma unroll 8
-  for (int j = 0; j < kTopkThreads; ++j) above += s.best[j] > mine;
-  if (above == k - 1) s.threshold = mine;  // (several threads only where mine is 0)
+  for (int j = 0; j < groups; ++j) above += s.best[j] > mine;
+  if (above == k - 1) s.threshold = mine;  // (of several threads only where they hold the same)
   __syncthreads();
 }
 __device__ __forceinline__ void topk_pool(TopkLds &s, unsigned long long key) {

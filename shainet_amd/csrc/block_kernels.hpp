@@ -37,7 +37,8 @@ hipError_t launch_embed_list(const float *table, const IdList &tokens, float *ou
 hipError_t launch_gather_rows(const float *x, const int *rows, float *out, int n, int cols, hipStream_t stream);
 // logits[j] += bias[j]
 hipError_t launch_add_bias_row(float *logits, const float *bias, int n, hipStream_t stream);
-// Sampler#apply_repetition_penalty! : ids in order, duplicates penalised once per occurrence
+// Sampler#apply_repetition_penalty! : ids in order, duplicates penalised once per occurrence; ids has room for
+// a multiple of 4, -1 behind the n ids
 hipError_t launch_repetition_penalty(float *logits, int vocab, const int *ids, int n, double penalty,
                                      hipStream_t stream);
 hipError_t launch_repetition_penalty_list(float *logits, int vocab, const IdList &ids, int n, double penalty,

@@ -435,10 +435,13 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvArgs a) {
 // A workgroup takes two pairs: wavefronts 0 and 1 their lower rows, 2 and 3 their upper rows, and
 // the sums meet in LDS (a wavefront per pair, two rows each, took 0.85 us longer for 3072 rows).
 // DYT: the prologue is Dynamic Tanh instead: x becomes tanh(alpha x) gamma + beta where it is staged.
-template <int KV4, int NACC, int SP, bool MULTI, bool PREP = false, bool DYT = false>
+// TAIL: rows of a.K values, a multiple of 4 below 256 KV4; the pieces beyond are zeros (one row of 384 -> 1536, in
+// front of which the split product took 7.8 us: 3.9).
+template <int KV4, int NACC, int SP, bool MULTI, bool PREP = false, bool DYT = false, bool TAIL = false>
 __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   static_assert(!PREP || (NACC == 1 && SP == 1 && !MULTI), "the q | k | v epilogue: one row per wavefront");
   static_assert(!DYT || (SP == 1 && !PREP), "rows shared by two wavefronts come without a norm");
+  static_assert(!TAIL || (SP == 1 && !PREP && !DYT), "odd row lengths: no norm or RMSNorm");
   const bool rms_norm = !DYT && a.norm;
   // x: up to 2048 values stay in registers.  Longer (half) rows: a wavefront with one output reads
   // them again from memory (the L2), eight 16-byte pieces at a time, where they are used; one with
@@ -464,6 +467,10 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   const int seg = wave % SP;
   constexpr int KW = 256 * KV4;  // values per wavefront and row
   constexpr int K = KW * SP;
+  const int Kr = TAIL ? a.K : K;             // values of a row
+  constexpr int XO = (K + 1023) / 1024;      // pieces of a thread's share of x
+  auto within = [&](int k) { return !TAIL || k < Kr; };
+  constexpr f32x4 kZero = {0.f, 0.f, 0.f, 0.f};
   // (with SP = 2 both wavefronts of a pair see the same n0: they are live or not together; XSH:
   // wavefronts without an output stay for the workgroup's x and leave after its barrier)
   if (!PREP && !XSH && !live) return;
@@ -474,55 +481,59 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
 #pragma unroll
     for (int c = 0; c < NACC; ++c) {
       const long long wrow = PREP ? (long long)n + (((n >> half_shift) + upper) << half_shift) : (long long)c * N + n;
-      const float *row = a.w + wrow * K + seg * KW + 4 * lane;
+      const float *row = a.w + wrow * Kr + seg * KW + 4 * lane;
 #pragma unroll
-      for (int i = 0; i < KV4; ++i) w[c][i] = __builtin_nontemporal_load((const f32x4 *)(row + 256 * i));
+      for (int i = 0; i < KV4; ++i)
+        w[c][i] = within(4 * lane + 256 * i) ? __builtin_nontemporal_load((const f32x4 *)(row + 256 * i)) : kZero;
     }
   };
   f32x4 wa[NACC][KV4], wb[MULTI ? NACC : 1][MULTI ? KV4 : 1];
   float rms = 1.0f;  // 1 / the root mean square
   constexpr bool NORMS = SP == 1;  // (rows shared by two wavefronts come without the norm: gemvt_takes)
-  f32x4 b_own[XSH && DYT ? K / 1024 : 1];  // its share of beta
-  f32x4 x_own[XSH ? K / 1024 : 1], g_own[XSH && NORMS ? K / 1024 : 1];  // this thread's share of x (and gamma) on its way to LDS
+  f32x4 b_own[XSH && DYT ? XO : 1];  // its share of beta
+  f32x4 x_own[XSH ? XO : 1], g_own[XSH && NORMS ? XO : 1];  // this thread's share of x (and gamma) on its way to LDS
   if constexpr (XSH) {
 #pragma unroll
-    for (int i = 0; i < K / 1024; ++i) x_own[i] = *(const f32x4 *)(a.x + 4 * threadIdx.x + 1024 * i);
+    for (int i = 0; i < XO; ++i)
+      x_own[i] = within(4 * threadIdx.x + 1024 * i) ? *(const f32x4 *)(a.x + 4 * threadIdx.x + 1024 * i) : kZero;
     if (NORMS && a.norm && a.gamma) {
 #pragma unroll
-      for (int i = 0; i < K / 1024; ++i) g_own[i] = *(const f32x4 *)(a.gamma + 4 * threadIdx.x + 1024 * i);
+      for (int i = 0; i < XO; ++i)
+        g_own[i] = within(4 * threadIdx.x + 1024 * i) ? *(const f32x4 *)(a.gamma + 4 * threadIdx.x + 1024 * i) : kZero;
     }
     if constexpr (DYT) {
 #pragma unroll
-      for (int i = 0; i < K / 1024; ++i) b_own[i] = *(const f32x4 *)(a.beta + 4 * threadIdx.x + 1024 * i);
+      for (int i = 0; i < XO; ++i) b_own[i] = *(const f32x4 *)(a.beta + 4 * threadIdx.x + 1024 * i);
     }
   }
   if (live || PREP) load_row(wa, n0);
   if constexpr (XSH) {
     if constexpr (DYT) {
 #pragma unroll
-      for (int i = 0; i < K / 1024; ++i) x_own[i] = dyn_tanh4(x_own[i], a.alpha, g_own[i], b_own[i]);
+      for (int i = 0; i < XO; ++i) x_own[i] = dyn_tanh4(x_own[i], a.alpha, g_own[i], b_own[i]);
     }
     if (NORMS && rms_norm) {
       // squares, their sums and the root in fp32 (a reciprocal square root and one Newton step):
       // within a few 1e-7 of the fp64 factor of rms_norm.cr:18-37
       f32x4 q = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < K / 1024; ++i) q += x_own[i] * x_own[i];
+      for (int i = 0; i < XO; ++i) q += x_own[i] * x_own[i];
       float sq = (q.x + q.y) + (q.z + q.w);
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
       if (lane == 0) sq_s[wave] = sq;
       if (a.gamma) {
 #pragma unroll
-        for (int i = 0; i < K / 1024; ++i) x_own[i] = x_own[i] * g_own[i];  // (1 / rms multiplies the finished sum)
+        for (int i = 0; i < XO; ++i) x_own[i] = x_own[i] * g_own[i];  // (1 / rms multiplies the finished sum)
       }
     }
 #pragma unroll
-    for (int i = 0; i < K / 1024; ++i) *(f32x4 *)(xsh + 4 * threadIdx.x + 1024 * i) = x_own[i];
+    for (int i = 0; i < XO; ++i)
+      if (K >= 1024 || 4 * threadIdx.x < K) *(f32x4 *)(xsh + 4 * threadIdx.x + 1024 * i) = x_own[i];
     __syncthreads();
     if (!PREP && !live) return;
     if (NORMS && rms_norm) {
-      const float m = ((sq_s[0] + sq_s[1]) + (sq_s[2] + sq_s[3])) / (float)K + (float)a.eps;
+      const float m = ((sq_s[0] + sq_s[1]) + (sq_s[2] + sq_s[3])) / (float)Kr + (float)a.eps;
       float r = rsqrtf(m);
       rms = r * (1.5f - 0.5f * m * r * r);
     }
@@ -543,7 +554,7 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   f32x4 xv[XREG ? KV4 : 1];
   if constexpr (XREG) {  // x is loaded once, into the registers it stays in
 #pragma unroll
-    for (int i = 0; i < KV4; ++i) xv[i] = *(const f32x4 *)(xp + 256 * i);
+    for (int i = 0; i < KV4; ++i) xv[i] = within(4 * lane + 256 * i) ? *(const f32x4 *)(xp + 256 * i) : kZero;
   }
   if (!XSH && rms_norm) {
     // every wavefront of the launch runs this, so it is kept short: squares, their sums and the
@@ -555,14 +566,14 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
     for (int c0 = 0; c0 < KV4; c0 += XC) {
       f32x4 t[XC];
 #pragma unroll
-      for (int i = 0; i < XC; ++i) t[i] = XREG ? xv[c0 + i] : *(const f32x4 *)(xp + 256 * (c0 + i));
+      for (int i = 0; i < XC; ++i) t[i] = XREG ? xv[c0 + i] : within(4 * lane + 256 * (c0 + i)) ? *(const f32x4 *)(xp + 256 * (c0 + i)) : kZero;
 #pragma unroll
       for (int i = 0; i < XC; ++i) q += t[i] * t[i];
     }
     float sq = (q.x + q.y) + (q.z + q.w);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
-    const float m = sq / (float)K + (float)a.eps;
+    const float m = sq / (float)Kr + (float)a.eps;
     float r = rsqrtf(m);
     r = r * (1.5f - 0.5f * m * r * r);
     rms = r;
@@ -570,7 +581,7 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   // pieces c0 .. c0 + XC - 1 of x times gamma (for the copy of XLDS)
   auto x_pieces = [&](f32x4 (&t)[XC], int c0) {
 #pragma unroll
-    for (int i = 0; i < XC; ++i) t[i] = *(const f32x4 *)(xp + 256 * (c0 + i));
+    for (int i = 0; i < XC; ++i) t[i] = within(4 * lane + 256 * (c0 + i)) ? *(const f32x4 *)(xp + 256 * (c0 + i)) : kZero;
     if constexpr (DYT) {
 #pragma unroll
       for (int i = 0; i < XC; ++i) {
@@ -581,7 +592,7 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
 #pragma unroll
       for (int i = 0; i < XC; ++i) {
         f32x4 g = {1.f, 1.f, 1.f, 1.f};
-        if (a.gamma) g = *(const f32x4 *)(a.gamma + seg * KW + 4 * lane + 256 * (c0 + i));
+        if (a.gamma && within(4 * lane + 256 * (c0 + i))) g = *(const f32x4 *)(a.gamma + seg * KW + 4 * lane + 256 * (c0 + i));
         t[i] = t[i] * g;  // (1 / rms multiplies the finished sum instead of every element)
       }
     }
@@ -593,7 +604,8 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   } else if constexpr (XREG) {
     if (a.norm && a.gamma) {
 #pragma unroll
-      for (int i = 0; i < KV4; ++i) xv[i] = xv[i] * *(const f32x4 *)(a.gamma + 4 * lane + 256 * i);
+      for (int i = 0; i < KV4; ++i)
+        if (within(4 * lane + 256 * i)) xv[i] = xv[i] * *(const f32x4 *)(a.gamma + 4 * lane + 256 * i);
     }
   } else if constexpr (XLDS) {
 #pragma unroll
@@ -776,7 +788,8 @@ bool gemvt_takes(int T, int K, int N, int epilogue, int norm, const GemvPrep *pr
   }
   // rows of 8192: two wavefronts per output, which leaves out the norm prologue and SwiGLU
   if (K == 8192) return !norm && !(N & 1) && (epilogue == kGemvPlain || epilogue == kGemvResidual || epilogue == kGemvBias);
-  if (K != 1024 && K != 2048 && K != 4096) return false;
+  // other lengths: padded to 512, 1024, 2048 or 4096 (below 257 values the split product has as little to wait for)
+  if (K != 1024 && K != 2048 && K != 4096 && ((K & 3) || K <= 256 || K > 4096 || norm == kNormDynTanh)) return false;
   return epilogue == kGemvPlain || epilogue == kGemvResidual || epilogue == kGemvSwiglu || epilogue == kGemvBias;
 }
 
@@ -833,17 +846,38 @@ hipError_t launch_gemvt(const GemvArgs &args, hipStream_t stream) {
     else                                     \
       SHAINET_LAUNCH_GEMVT_N(KV4_, false);   \
   } while (0)
+#define SHAINET_LAUNCH_GEMVT_TAIL(KV4_)                                                                           \
+  do {                                                                                                            \
+    if (two && rpw > 1)                                                                                           \
+      hipLaunchKernelGGL((gemvt_kernel<KV4_, 2, 1, true, false, false, true>), grid, dim3(256), 0, stream, a);    \
+    else if (two)                                                                                                 \
+      hipLaunchKernelGGL((gemvt_kernel<KV4_, 2, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);   \
+    else if (rpw > 1)                                                                                             \
+      hipLaunchKernelGGL((gemvt_kernel<KV4_, 1, 1, true, false, false, true>), grid, dim3(256), 0, stream, a);    \
+    else                                                                                                          \
+      hipLaunchKernelGGL((gemvt_kernel<KV4_, 1, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);   \
+  } while (0)
   switch (a.K) {
     case 1024: SHAINET_LAUNCH_GEMVT(4); break;
     case 2048: SHAINET_LAUNCH_GEMVT(8); break;
     case 4096: SHAINET_LAUNCH_GEMVT(16); break;
-    default:  // 8192: two wavefronts per output
+    case 8192:  // two wavefronts per output
       if (rpw > 1)
         hipLaunchKernelGGL((gemvt_kernel<16, 1, 2, true>), grid, dim3(256), 0, stream, a);
       else
         hipLaunchKernelGGL((gemvt_kernel<16, 1, 2, false>), grid, dim3(256), 0, stream, a);
       break;
+    default:
+      if (a.K <= 512)
+        SHAINET_LAUNCH_GEMVT_TAIL(2);
+      else if (a.K < 1024)
+        SHAINET_LAUNCH_GEMVT_TAIL(4);
+      else if (a.K < 2048)
+        SHAINET_LAUNCH_GEMVT_TAIL(8);
+      else
+        SHAINET_LAUNCH_GEMVT_TAIL(16);
   }
+#undef SHAINET_LAUNCH_GEMVT_TAIL
 #undef SHAINET_LAUNCH_GEMVT
 #undef SHAINET_LAUNCH_GEMVT_N
   return hipGetLastError();

@@ -150,7 +150,29 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
   // q_full, k_new, v_new (llama_block.cr:253-255) as the three column blocks of one product
   const int hd = l->head_dim;
   static const bool fuse_off = getenv("SHAINET_HIP_NO_FUSED_PREP") != nullptr;
-  if (!fuse_off && T <= 16 && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
+  // the copy carries the weights of the norm this product follows (a layer used with another
+  // norm, or with none, gets its copy made again)
+  auto take_transposed = [&](Fused &f) {
+    const float *gamma = f.norm == kNormRms ? f.gamma : nullptr;
+    if (gamma != l->w_qkv_t_gamma) l->w_qkv_t_stale = true;
+    f.w_t = transposed_twin(&l->w_qkv_t, &l->w_qkv_t_stale, l->w_qkv, l->d_model, wide, stream, gamma);
+    l->w_qkv_t_gamma = f.w_t ? gamma : nullptr;
+    f.w_t_has_gamma = f.w_t && gamma;
+  };
+  // One row with QK-norm: the sum of squares needs the whole head, which the product over transposed weights does not
+  // hold in one place; it and the prep kernel behind it take 4 + 3.5 us where the split product with prep inside
+  // takes 10 (1024 -> 2048), 5.5 + 3.5 against 10.9 (2048 -> 3072).
+  const bool norm_apart = T == 1 && (l->has_q_norm || l->has_k_norm) && transposed_twins_wanted() &&
+                          gemvt_takes(T, l->d_model, wide, pre.epilogue, pre.norm);
+  if (ahead && ahead->wt && T == 1) {
+    // One row: the attention launch leaves the memory system idle while it waits on its chain of
+    // dependent loads, and takes along workgroups that read the first rows of the gate | up
+    // weights into the L2s (8 MB: 1134 -> 1120 us per token of the 1B shape; 17 MB and more
+    // slow the attention's own chain down by more than the product gains)
+    static const int ahead_wgs = getenv("SHAINET_HIP_READ_AHEAD_WGS") ? atoi(getenv("SHAINET_HIP_READ_AHEAD_WGS")) : 128;
+    if (ahead_wgs > 0) shainet_attn_read_ahead(l->ctx, ahead->wt, ahead->k, ahead->n, ahead_wgs);
+  }
+  if (!fuse_off && !norm_apart && T <= 16 && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
     // few rows: bias, QK-norm, RoPE and the cache append (256-286, 332-344) happen where the
     // product's head rows are summed up; the attention kernel follows directly
     GemvPrep where;
@@ -158,25 +180,13 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     Fused qkv = pre;
     qkv.epilogue = kGemvQkvPrep;
     qkv.prep = &where;
-    if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm, &where)) {
-      // the copy carries the weights of the norm this product follows (a layer used with another
-      // norm, or with none, gets its copy made again)
-      const float *gamma = qkv.norm ? qkv.gamma : nullptr;
-      if (gamma != l->w_qkv_t_gamma) l->w_qkv_t_stale = true;
-      qkv.w_t = transposed_twin(&l->w_qkv_t, &l->w_qkv_t_stale, l->w_qkv, l->d_model, wide, stream, gamma);
-      l->w_qkv_t_gamma = qkv.w_t ? gamma : nullptr;
-      qkv.w_t_has_gamma = qkv.w_t && gamma;
-    }
+    if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm, &where)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, nullptr, T, l->d_model, wide, stream, qkv))) return rc;
-    // One row: the attention launch leaves the memory system idle while it waits on its chain of
-    // dependent loads, and takes along workgroups that read the first rows of the gate | up
-    // weights into the L2s (8 MB: 1134 -> 1120 us per token of the 1B shape; 17 MB and more
-    // slow the attention's own chain down by more than the product gains)
-    static const int ahead_wgs = getenv("SHAINET_HIP_READ_AHEAD_WGS") ? atoi(getenv("SHAINET_HIP_READ_AHEAD_WGS")) : 128;
-    if (ahead && ahead->wt && ahead_wgs > 0 && T == 1) shainet_attn_read_ahead(l->ctx, ahead->wt, ahead->k, ahead->n, ahead_wgs);
     rc = shainet_attn_finish_prepared(l->ctx, cache, T, l->attn.p);  // 287-296
   } else {
-    if ((rc = l->proj.project(x, l->d_model, l->w_qkv, l->qkv.p, T, l->d_model, wide, stream, pre))) return rc;
+    Fused qkv = pre;
+    if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm)) take_transposed(qkv);
+    if ((rc = l->proj.project(x, l->d_model, l->w_qkv, l->qkv.p, T, l->d_model, wide, stream, qkv))) return rc;
     rc = shainet_attn_forward_strided(l->ctx, cache, nullptr, &T, 1, l->qkv.p, l->qkv.p + l->q_dim,
                                       l->qkv.p + l->q_dim + l->kv_dim, wide, wide, wide, l->attn.p,
                                       SHAINET_HIP_MEM_DEVICE);  // 256-296

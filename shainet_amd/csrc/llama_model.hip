@@ -712,9 +712,12 @@ int shainet_llama_model_repetition_penalty(shainet_llama_model *m, const int *re
     if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("penalty launch: ") + hipGetErrorString(e));
     return SHAINET_HIP_OK;
   }
-  int rc = reserve_ints(&m->d_tokens, &m->d_tokens_cap, (size_t)n);
+  std::vector<int> ids(recent_ids, recent_ids + n);
+  ids.resize((ids.size() + 3) / 4 * 4, -1);
+  int rc = reserve_ints(&m->d_tokens, &m->d_tokens_cap, ids.size());
   if (rc) return rc;
-  if (hipMemcpyAsync(m->d_tokens, recent_ids, (size_t)n * sizeof(int), hipMemcpyHostToDevice, m->stream) != hipSuccess)
+  // (pageable source: the copy has left `ids` when the call returns)
+  if (hipMemcpyAsync(m->d_tokens, ids.data(), ids.size() * sizeof(int), hipMemcpyHostToDevice, m->stream) != hipSuccess)
     return fail(SHAINET_HIP_ERR_RUNTIME, "hipMemcpyAsync(ids) failed");
   hipError_t e = launch_repetition_penalty(m->logits.p, m->vocab, m->d_tokens, n, penalty, m->stream);
   if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("penalty launch: ") + hipGetErrorString(e));

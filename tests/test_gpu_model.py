@@ -851,3 +851,14 @@ def test_generate_greedy_equals_steps(hip, vocab):
     assert got == want
     np.testing.assert_array_equal(row, last)
     m.close()
+
+
+@pytest.mark.parametrize("d,ff,norm", [(260, 516, False), (384, 1020, True), (512, 772, False), (640, 1028, True),
+                                       (1020, 2044, False), (1024, 1536, True), (1536, 2052, True), (3072, 4092, False)])
+def test_one_row_products_of_any_length(hip, d, ff, norm):
+    """Decode steps whose rows fill a wavefront's loads in part: lengths padded to 512, 1024, 2048 and 4096 in the q | k | v
+    product (QK-norm behind it or none), W_o, gate | up and down."""
+    blk, ob, p, r, eps = _block_pair(hip, d, 4, 2, 64, ff, 1e4, seed=d, norm=norm, bias=True, wscale=0.03)
+    for T in (3, 1, 1, 1):
+        x = r.standard_normal((T, d)).astype(np.float32)
+        rm.assert_close(blk.forward_cached(x), _oracle_forward(ob, p, eps, x), ATOL, RTOL, f"T={T}")
