@@ -101,7 +101,7 @@ struct BiasedAttn : Mixer {
     DistanceBias b = bias;
     b.q_stride = w.n_in;
     Fused in = pre;
-    const bool fuse = !from && T <= 16 && dim == vdim && (w.n_in & 3) == 0 && dim >= 2 && dim <= 128 && (dim & (dim - 1)) == 0;
+    const bool fuse = !from && T <= 16 && Projector::few_rows(T, d, w.n_in, d) && dim == vdim && (w.n_in & 3) == 0 && dim >= 2 && dim <= 128 && (dim & (dim - 1)) == 0;
     if (fuse) {
       // few rows: key and value heads go to the cache where the product sums them up
       GemvPrep p = {};

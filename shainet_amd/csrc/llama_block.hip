@@ -172,7 +172,7 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     static const int ahead_wgs = getenv("SHAINET_HIP_READ_AHEAD_WGS") ? atoi(getenv("SHAINET_HIP_READ_AHEAD_WGS")) : 128;
     if (ahead_wgs > 0) shainet_attn_read_ahead(l->ctx, ahead->wt, ahead->k, ahead->n, ahead_wgs);
   }
-  if (!fuse_off && !norm_apart && T <= 16 && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
+  if (!fuse_off && !norm_apart && T <= 16 && Projector::few_rows(T, l->d_model, wide, l->d_model) && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
     // few rows: bias, QK-norm, RoPE and the cache append (256-286, 332-344) happen where the
     // product's head rows are summed up; the attention kernel follows directly
     GemvPrep where;

@@ -117,6 +117,7 @@ struct Fused {
   // the same weights transposed ([N, K]; kGemvSwiglu: [2N, K]) or null: one row of x then takes the
   // product that gives a wavefront whole outputs (launch_gemvt) where its shapes allow
   const float *w_t = nullptr;
+  bool any_few_rows = false;  // up to 16 rows run as the split GEMV, not only the ones it is the faster product for
   bool w_t_has_gamma = false;  // the rows of w_t were made with gamma multiplied in: the norm's factor 1 / rms is all that is left to apply
 };
 
@@ -135,12 +136,17 @@ struct NormWeights {
   }
 };
 
-// y[T,N] = epilogue(norm(x)[T,K] * W), all row-major on the device.  Up to 16 rows
-// (decode) run as one hand-written split GEMV with the norm and the epilogue
+// y[T,N] = epilogue(norm(x)[T,K] * W), all row-major on the device.  A few rows
+// (decode; few_rows) run as one hand-written split GEMV with the norm and the epilogue
 // inside; more rows run as the MFMA product of gemm_kernel.hip (the counterpart of
 // the reference's cuBLAS SGEMM, cuda.cr:237-247) after the separate norm kernel,
 // with the residual add in its epilogue and the SwiGLU activation as a kernel of its own.
 struct Projector {
+  // Whether T rows run as the split GEMV.  Up to 4 do.  It streams the weights once for up to 16, but its multiply-adds
+  // are the vector ALU's, and from 5 rows on the MFMA product is the faster one (a prompt of a 2048 wide model of 4
+  // layers: 4 rows 533 | 600 us, 5 rows 701 | 600, 16 rows 962 | 602); it needs K, N and the row stride of x to be
+  // multiples of 4.
+  static bool few_rows(int T, int K, int N, long long x_stride);
   DevF scratch, normed, wide;
   // split products: a word per partial that says when it is complete (zero between launches)
   unsigned *flags = nullptr;

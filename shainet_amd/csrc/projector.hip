@@ -128,6 +128,10 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
   return SHAINET_HIP_OK;
 }
 
+bool Projector::few_rows(int T, int K, int N, long long x_stride) {
+  return T <= 4 || (T <= 16 && !plan_gemm(T, K, N, x_stride).mfma);
+}
+
 int Projector::project(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
                        hipStream_t stream, const Fused &f) {
   const bool swiglu = f.epilogue == kGemvSwiglu;
@@ -157,7 +161,10 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
       return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("gemv launch: ") + hipGetErrorString(e));
     return SHAINET_HIP_OK;
   }
-  if (T <= 16 && (N & 3) == 0) {
+  // (an epilogue that only it has, or rows of x that the MFMA product cannot load, keep the split GEMV, too)
+  const bool gemv = f.epilogue == kGemvQkvPrep || f.any_few_rows || few_rows(T, K, swiglu ? 2 * N : N, x_stride) ||
+                    (((uintptr_t)x | (uintptr_t)w) & 15);
+  if (T <= 16 && (N & 3) == 0 && gemv) {
     const float *xin = x;
     long long xs = x_stride;
     int norm = f.norm;
@@ -286,6 +293,7 @@ extern "C" int shainet_hip_matmul_f32(const float *x, long long x_stride, const 
   // is said by the next call, which does nothing else then
   if (int rc = check_error_word(p.error)) return rc;
   Fused f;
+  f.any_few_rows = true;
   if (res) {
     f.epilogue = kGemvResidual;
     f.res = res;
