@@ -46,7 +46,7 @@ namespace shainet {
 
 namespace {
 
-constexpr int TK = 16;
+constexpr int TK = 16, kFewStep = 32;
 
 // A partial product is read by a workgroup that may sit on another XCD, whose L2 is not kept
 // coherent with this one's for ordinary accesses: the store is written through to memory.
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
   const int ln = lane & 31, j = lane >> 5, wm = wave / WN, wn = wave % WN;
   const int T = g.T, K = g.K, N = g.N;
 
-  // staging: x: octet tid % 2 of row tid / 2, or half an octet, quarter tid % 4 of row tid / 4; W: octet tid / TN
+  // staging: x: octet tid % 2 of row tid / 2, or half of one, quarter tid % 4 of row tid / 4; W: octet tid / TN
   // of column tid % TN
   const int xrow = NX == 1 ? threadIdx.x >> 2 : threadIdx.x >> 1;
   const int xk = NX == 1 ? 4 * (threadIdx.x & 3) : 8 * (threadIdx.x & 1);
@@ -194,17 +194,11 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       stage[w_unit] = h;
       stage[w_unit + S::kPartW] = m;
       stage[w_unit + 2 * S::kPartW] = l;
-      if (NX == 1) {
+      if constexpr (NX == 1) {
         u32x2 *half = (u32x2 *)(stage + x_unit) + ((xk >> 2) & 1);
         split_quad(rx[0], half[0], half[2 * S::kPartX], half[4 * S::kPartX]);
       } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f32x4 v = rx[i >> 1];
-          unsigned a, b, c;
-          split_pair(i & 1 ? v.z : v.x, i & 1 ? v.w : v.y, a, b, c);
-          h[i] = a, m[i] = b, l[i] = c;
-        }
+        split_octet(rx[0], rx[1], h, m, l);
         stage[x_unit] = h;
         stage[x_unit + S::kPartX] = m;
         stage[x_unit + 2 * S::kPartX] = l;
@@ -362,20 +356,163 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
   }
 }
 
+// Few rows: a wavefront owns the columns of W it multiplies, so they go from memory to its registers and are split
+// there; only x goes through LDS.  A workgroup of four wavefronts owns 32 rows and 128 columns and walks K in steps of 32: wavefronts 0 and 1 take the first half of a step, 2 and 3 the second, 64 columns
+// each, and the two halves' sums meet in LDS at the end.  Lane n of a wavefront loads two neighbouring columns (a
+// row of W 256 bytes at a time) and 8 rows, which are its fragments of two blocks.
+// Against tiles of 64 x 128 with both operands in LDS, which this reads and writes a fifth as much (us): 32 rows of
+// 2048 -> 16384 44 -> 30 (134 MB: 22 at the rate of a read), 2048 -> 3072 19.3 -> 14.4, 45 rows 44 -> 41 and 19.5 -> 15.7,
+// 64 rows of 1024 -> 1024 12.1 -> 9.2.  64 rows by 128 columns this way were slower than 32 (45 rows of
+// 8192 -> 2048 34 against 30.5).  Bound by a launch, the first loads and the kernel that adds the pieces where the
+// weights are small, by reading them where they are not.
+template <bool GUARD>
+__global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
+  constexpr int TM = 32, TN = 128, TS = kFewStep;
+  constexpr int kOct = TM + 4, kPart = 4 * kOct;  // units of 16 bytes: four octets of k, four units apart from a multiple of 16
+  constexpr int kStage = 3 * kPart;
+  constexpr int kMerge = 2 * 2 * 16 * 64 / 4;  // units that two wavefronts' sums take
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kStage > kMerge ? 2 * kStage : kMerge];
+
+  const int group = blockIdx.x & ((1 << g.group_bits) - 1), place = blockIdx.x >> g.group_bits;
+  const int steps = g.steps, pieces = g.pieces ? g.pieces : 1;
+  const int t = place / pieces, s_begin = (place - t * pieces) * g.quota, s_end = min(s_begin + g.quota, steps);
+  if (t >= g.tiles_per_group || s_begin >= s_end) return;
+  const int tile = group * g.tiles_per_group + t;
+  const int m0 = tile % g.tiles_m * TM, n0 = tile / g.tiles_m * TN;
+  const int T = g.T, K = g.K, N = g.N;
+  const int k_begin = s_begin * TS, k_end = min(K, s_end * TS), nk = s_end - s_begin;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 31, j = lane >> 5, wn = wave & 1, kg = wave >> 1;
+  const int col = n0 + 64 * wn + 2 * ln;
+
+  // x: a thread takes four k, piece tid % 8, of row tid / 8 (rows past the last one repeat it)
+  const int xrow = threadIdx.x >> 3, xk = 4 * (threadIdx.x & 7);
+  const unsigned x_off = (unsigned)(((long long)min(m0 + xrow, T - 1) * g.xs + xk) * 4);
+  u32x2 *const x_lds = (u32x2 *)(lds + (xk >> 3) * kOct + xrow) + (xk >> 2 & 1);
+  // W: rows 16 kg + 8 j .. + 7 of a step (columns past the last two repeat them)
+  const int wk = 16 * kg + 8 * j;
+  const unsigned w_off = (unsigned)(((long long)wk * N + min(col, N - 2)) * 4);
+  const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)k_begin * N);
+  const long long row_bytes = 4LL * N;
+
+  // register sets: the tiles of step t travel in set t & 1 and are requested two steps ahead (behind the last step
+  // its tiles are requested again: the loop has no conditions)
+  f32x4 sx[2];
+  f32x2 sw[2][8];
+  int k_next = k_begin, to_load = nk;
+  auto load_tiles = [&](int set) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      sw[set][i] = !GUARD || k_next + wk + i < k_end ? *(const f32x2 *)(w_base + i * row_bytes + w_off) : f32x2{0.f, 0.f};
+    sx[set] = !GUARD || k_next + xk < k_end ? *(const f32x4 *)(x_base + x_off) : f32x4{0.f, 0.f, 0.f, 0.f};
+    if (--to_load > 0) {
+      x_base += TS * 4;
+      w_base += TS * row_bytes;
+      k_next += TS;
+    }
+  };
+  auto park_x = [&](int set, int stage) {
+    u32x2 *at = x_lds + 2 * stage * kStage;
+    split_quad(sx[set], at[0], at[2 * kPart], at[4 * kPart]);
+  };
+
+  f32x16 acc[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+
+  load_tiles(0);
+  load_tiles(1);
+  park_x(0, 0);
+  __syncthreads();
+  auto step = [&](const int kt, const int set) {  // set: holds step kt, the other one step kt + 1
+    const u32x4 *stage = lds + (kt & 1) * kStage + (2 * kg + j) * kOct + ln;
+    u32x4 af[3], bf[3][2];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) af[p] = stage[p * kPart];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        unsigned h, m, l;
+        split_pair(sw[set][2 * i][b], sw[set][2 * i + 1][b], h, m, l);
+        bf[0][b][i] = h, bf[1][b][i] = m, bf[2][b][i] = l;
+      }
+    park_x(set ^ 1, (kt & 1) ^ 1);
+    load_tiles(set);
+#pragma unroll
+    for (int p = 0; p < 6; ++p)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[b] = mfma_bf16(af[kPartA[p]], bf[kPartB[p]][b], acc[b]);
+    __syncthreads();
+  };
+  for (int kt = 0; kt < nk; kt += 2) {
+    step(kt, 0);
+    if (kt + 1 < nk) step(kt + 1, 1);
+  }
+
+  const int row0 = m0 + 4 * j;
+  // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which
+  float probe = 0.f;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) probe = fmaf(acc[b][r], 0.f, probe);
+  if (__any(probe != 0.f)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+#pragma clang loop unroll(disable)
+    for (int k = k_begin + 16 * kg; k < k_end; k += (k & 15) == 15 ? 17 : 1) {
+      const f32x2 wv = *(const f32x2 *)(g.w + (long long)k * N + min(col, N - 2));
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float xv = g.x[(long long)min(row0 + 8 * (r >> 2) + (r & 3), T - 1) * g.xs + k];
+        acc[0][r] = fmaf(xv, wv.x, acc[0][r]);
+        acc[1][r] = fmaf(xv, wv.y, acc[1][r]);
+      }
+    }
+  }
+  // (every wavefront is past the last step's barrier: nobody reads tiles any more)
+  f32x4 *const merge = (f32x4 *)lds + wn * (kMerge / 2) + lane;
+  if (kg == 1) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) merge[64 * r] = f32x4{acc[0][2 * r], acc[1][2 * r], acc[0][2 * r + 1], acc[1][2 * r + 1]};
+  }
+  __syncthreads();
+  if (kg == 1) return;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const f32x4 v = f32x4{acc[0][2 * r], acc[1][2 * r], acc[0][2 * r + 1], acc[1][2 * r + 1]} + merge[64 * r];
+    if (g.pieces) {  // [pair of rows][thread], as the kernel that adds the pieces takes them
+      *(f32x4 *)(g.partials + (long long)blockIdx.x * (TM * TN) + r * 512 + 4 * threadIdx.x) = v;
+    } else if (col < N) {
+      const int row = row0 + 8 * (r >> 1) + 2 * (r & 1);
+      store_pair(g, row, col, f32x2{v.x, v.y});
+      store_pair(g, row + 1, col, f32x2{v.z, v.w});
+    }
+  }
+}
+
 // y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order.  A piece lies in its
 // workgroup's slot as [pair of rows][thread] float4, the layout of the product kernel's accumulators.
-template <int MB, int WN>
-__global__ __launch_bounds__(128 * WN) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
+// A tile's threads are WM x WN wavefronts.
+template <int MB, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
   const int tile = blockIdx.x / (8 * MB), r = blockIdx.x % (8 * MB);  // 8 MB workgroups per tile, a pair of rows of each thread each
   if (tile >= tiles) return;
   const int group = tile / g.tiles_per_group, t = tile - group * g.tiles_per_group;
-  constexpr int TN = 64 * WN;
-  constexpr long long kSlot = 64LL * MB * TN;
-  const float *piece = g.partials + (long long)(((t * g.pieces) << g.group_bits) | group) * kSlot + r * 512 * WN + 4 * threadIdx.x;
+  constexpr int TM = 32 * WM * MB, TN = 64 * WN;
+  constexpr long long kSlot = (long long)TM * TN;
+  const float *piece = g.partials + (long long)(((t * g.pieces) << g.group_bits) | group) * kSlot + r * 256 * WM * WN + 4 * threadIdx.x;
   const long long piece_step = kSlot << g.group_bits;
   const int n = min(g.pieces, (g.steps + g.quota - 1) / g.quota);  // pieces that hold any steps
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = (tile % g.tiles_m) * 64 * MB + (wave / WN) * 32 * MB + 32 * (r >> 3) + 4 * (lane >> 5) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
+  const int row = (tile % g.tiles_m) * TM + (wave / WN) * 32 * MB + 32 * (r >> 3) + 4 * (lane >> 5) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
   const int col = (tile / g.tiles_m) * TN + (wave % WN) * 64 + 2 * (lane & 31);
   if (row >= g.T || col >= g.N) return;
   f32x4 acc = *(const f32x4 *)piece;
@@ -410,25 +547,29 @@ namespace {
 int slots_of(int wn) { return wn == 4 ? 256 : 512; }
 
 // The tile, by what was measured (us, 2048 -> 3072 | 2048 -> 2048 | 2048 -> 16384 | 8192 -> 2048 | 1024 -> 8192):
-//   rows   64 x 128                    128 x 128                  128 x 256                  256 x 256
-//     45   19 | 17 | 42 | 31 | 19      23 | 19 | 59 | 37 | 24
-//    100   22 | 21 | 69 | 41 | 24      23 | 20 | 62 | 39 | 26
-//    256   31 | 25 | 125 | 68 | 40     33 | 28 | 106 | 62 | 37    31 | 27 | 108 | 59 | 37
+//   rows   32 x 128 (few)              128 x 128                  128 x 256                  256 x 256
+//     45   16 | 15 | 41 | 31 | 16      23 | 19 | 59 | 37 | 24
+//     96   19 | 16 | 60 | 35 | 22      22 | 21 | 62 | 37 | 24
+//    128   20 | 19 | 67 | 42 | 24      22 | 20 | 63 | 41 | 24
+//    160   24 | 20 | 88 | 50 | 30      30 | 26 | 102 | 59 | 34
+//    256   33 | 24 | 125 | 72 | 35     31 | 27 | 105 | 61 | 37    31 | 27 | 108 | 59 | 37
 //    512                               47 | 37 | 185 | 106 | 57   45 | 36 | 177 | 102 | 58   52 | 44 | 192 | 100 | 64
 //   1024                               87 | 58 | 360 | 197 | 96   82 | 57 | 342 | 186 | 88   80 | 63 | 315 | 173 | 116
 //   2048                               148 | 100 | 717 | 372 | 187  143 | 99 | 674 | 346 | 181  144 | 100 | 619 | 323 | 164
-// A low tile wastes least on few rows; where the weights are small it is also the faster one in two rounds.
+// A low tile wastes least on few rows, and reads small weights again from the L2 for little: up to 96 rows always, up to
+// 256 where the higher tile would be a fifth padding or the weights are small.
 // The largest needs long runs: at least 36 steps a workgroup, and no tile that two of them share by waiting.
 void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 2;
-  if (T <= 64 || (T <= 128 && (long long)K * N <= 12 << 20)) {
-    p.mb = 1;
-    return;
-  }
+  const long long weights = (long long)K * N, rows1 = (T + 31) / 32 * 32LL, rows2 = (T + 127) / 128 * 128LL;
+  p.few = T <= 96 || (T <= 256 && (weights <= (T <= 128 ? 12 : 5) << 20 || rows2 * 100 >= rows1 * 125));
+  p.few = p.few && (long long)kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows)
+  p.mb = 1;
+  if (p.few) return;
   p.mb = 2;
   if (T <= 256) return;
   p.wn = 4;
-  const long long rows2 = (T + 127) / 128 * 128LL, rows4 = (T + 255) / 256 * 256LL;
+  const long long rows4 = (T + 255) / 256 * 256LL;
   const long long tiles = rows4 / 256 * ((N + 255) / 256), run = tiles * p.steps / slots_of(4);
   if (rows4 * 100 <= rows2 * 115 && run >= 36 && (tiles >= slots_of(4) || 2 * run < p.steps)) p.mb = 4;
 }
@@ -442,8 +583,9 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
            (long long)T * x_stride * 4 < 0xffffffffLL && (long long)TK * N * 4 < 0xffffffffLL;
   p.steps = (K + TK - 1) / TK;
   choose_tile(p, T, K, N);
-  const int TN = 64 * p.wn;
-  p.tiles_m = (T + 64 * p.mb - 1) / (64 * p.mb);
+  const int TN = 64 * p.wn, TM = (p.few ? 32 : 64) * p.mb;
+  if (p.few) p.steps = (K + kFewStep - 1) / kFewStep;
+  p.tiles_m = (T + TM - 1) / TM;
   p.tiles_n = (N + TN - 1) / TN;
   if (!p.mfma) return p;
   const int slots = slots_of(p.wn);
@@ -453,6 +595,18 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
   while (tiles & ((1 << p.group_bits) - 1)) --p.group_bits;
   const int groups = 1 << p.group_bits;
   p.tiles_per_group = tiles / groups;
+  if (p.few) {  // pieces of about twelve steps, more where that leaves compute units without one, of at least four steps each
+    int pieces = p.steps / 12 > 256 / tiles ? p.steps / 12 : 256 / tiles;
+    if (pieces > slots / tiles) pieces = slots / tiles;
+    if (pieces > 16) pieces = 16;
+    if (pieces > p.steps / 4) pieces = p.steps / 4;
+    if (pieces < 1) pieces = 1;
+    p.quota = (p.steps + pieces - 1) / pieces;
+    p.workgroups = tiles * pieces;
+    p.pieces = pieces;
+    if (pieces > 1) p.partial_floats = (size_t)p.workgroups * TM * TN;
+    return p;
+  }
   if (tiles % slots == 0) {  // whole rounds of the chip: a workgroup per tile
     p.quota = p.steps;
     p.workgroups = tiles;
@@ -482,7 +636,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
     p.workgroups = tiles * pieces;
     if (pieces == 1) return p;  // (short K: a workgroup per tile after all)
   }
-  p.partial_floats = (size_t)p.workgroups * 64 * p.mb * TN;
+  p.partial_floats = (size_t)p.workgroups * TM * TN;
   return p;
 }
 
@@ -498,7 +652,20 @@ hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, hipStream_t stream
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || !g.pieces) return e;
   const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL((sgemm_reduce_kernel<MB, WN>), dim3((unsigned)tiles * 8 * MB), dim3(128 * WN), 0, stream, g, tiles);
+  hipLaunchKernelGGL((sgemm_reduce_kernel<MB, 2, WN>), dim3((unsigned)tiles * 8 * MB), dim3(128 * WN), 0, stream, g, tiles);
+  return hipGetLastError();
+}
+
+hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+  const dim3 grid((unsigned)p.workgroups);
+  if (g.K % kFewStep != 0)
+    hipLaunchKernelGGL((sgemm_few_kernel<true>), grid, dim3(256), 0, stream, g);
+  else
+    hipLaunchKernelGGL((sgemm_few_kernel<false>), grid, dim3(256), 0, stream, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !g.pieces) return e;
+  const int tiles = p.tiles_m * p.tiles_n;
+  hipLaunchKernelGGL((sgemm_reduce_kernel<1, 1, 2>), dim3((unsigned)tiles * 8), dim3(128), 0, stream, g, tiles);
   return hipGetLastError();
 }
 
@@ -538,8 +705,9 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   g.tiles_per_group = p.tiles_per_group;
   g.quota = p.quota;
   g.pieces = p.pieces > 1 ? p.pieces : 0;
+  if (p.few) return launch_few(g, p, stream);
   if (p.wn == 4) return p.mb == 4 ? launch_tiles<4, 4>(g, p, stream) : launch_tiles<2, 4>(g, p, stream);
-  return p.mb == 2 ? launch_tiles<2, 2>(g, p, stream) : launch_tiles<1, 2>(g, p, stream);
+  return launch_tiles<2, 2>(g, p, stream);
 }
 
 }  // namespace shainet

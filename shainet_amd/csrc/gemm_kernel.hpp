@@ -8,9 +8,10 @@ namespace shainet {
 
 struct GemmPlan {
   bool mfma;              // false: K, N or the row stride of x is not a multiple of 4 -> the plain kernel
-  int mb, wn;             // tiles of y have 64 mb rows and 64 wn columns
+  bool few;               // tiles of 32 rows and 128 columns, K steps of 32
+  int mb, wn;             // otherwise tiles of 64 mb rows and 64 wn columns, K steps of 16
   int tiles_m, tiles_n;
-  int steps;              // K steps of 16 per tile; a unit of work is one step of one tile
+  int steps;              // K steps per tile; a unit of work is one step of one tile
   int group_bits;         // 2^group_bits groups of workgroups, each with an equal run of the tiles
   int tiles_per_group;
   int quota;              // consecutive units per workgroup (= steps: a workgroup per tile, nothing shared)

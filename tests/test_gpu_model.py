@@ -752,10 +752,11 @@ def test_load_llama_bf16_f16_sharded_qwen_style(hip, tmp_path):
 
 
 @pytest.mark.parametrize("T,K,N", [
-    (17, 4, 4), (64, 16, 132), (65, 20, 124),            # 64 x 128 tiles: one step, ragged columns, the guarded loads
-    (70, 2048, 6400), (129, 36, 128), (256, 528, 260),   # 128 x 128
-    (257, 16, 256), (300, 2052, 1028), (640, 512, 512),  # 128 x 256: whole and ragged, one step, pieces
-    (1024, 2048, 2308), (1000, 1040, 8192),              # 256 x 256: pieces and the kernel that adds them; whole tiles
+    (17, 4, 4), (33, 32, 132), (64, 100, 124), (70, 2048, 6400),  # 32 x 128: ragged rows and columns, guarded loads, whole
+    (96, 8192, 256), (129, 36, 128), (256, 528, 260),             # tiles, pieces
+    (100, 2052, 6400), (256, 2048, 3076),                         # 128 x 128
+    (257, 16, 256), (300, 2052, 1028), (640, 512, 512),           # 128 x 256: whole and ragged, one step, pieces
+    (1024, 2048, 2308), (1000, 1040, 8192),                       # 256 x 256: pieces and the kernel that adds them; whole tiles
 ])
 def test_matmul_split_tiles(hip, T, K, N):
     """Each tile of the product over split operands.  A sum is rounded 6 K / 16 times, each time by at most 2^-24 of
@@ -777,7 +778,7 @@ def test_matmul_split_tiles(hip, T, K, N):
     assert torch.equal(got, binding.matmul(x, w, res))
 
 
-@pytest.mark.parametrize("T", [40, 200, 300, 1100])
+@pytest.mark.parametrize("T", [40, 250, 300, 1100])
 def test_matmul_split_tiles_keep_what_is_not_finite(hip, T):
     """Infinities, NaN and values that a bf16 would round to infinity come out as fp32 arithmetic has them."""
     import torch
