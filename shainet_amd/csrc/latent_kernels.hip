@@ -794,11 +794,17 @@ bool plan_latent_expanded(const LatentShape &sh, int T, int start_row, LatentExp
   if (splits_knob > 0) splits = splits_knob;
   p.splits = splits < 1 ? 1 : splits;
   p.partial_floats = p.splits > 1 ? (size_t)blocks * p.splits * 128 * (p.nt * 32 + 2) : 0;
-  // multiply-adds per (row, key, head): this form's, and its product's share; against the absorbed form's,
-  // whose kernel reaches about half this one's rate
+  // Multiply-adds: per (row, key, head) this form's and the absorbed form's, whose kernel reaches about half
+  // this one's rate; and the products, here of every key row and at twice the rate (the library's), there of the new
+  // rows alone.  A few rows behind many keys are the absorbed form's: 20 rows of 16 heads of 192 and
+  // 128 dimensions behind 500 (3000) keys 614 us (725) a pass of three layers against 671 (918), 40 rows 733 (950)
+  // against 720 (969), 64 rows 872 (1265) against 726 (986); and in front of none, 17 rows 636 against 577, 64
+  // rows 845 against 614.
   const double pairs = (double)T * (sh.window && sh.window < p.key_rows ? sh.window : p.key_rows);
-  const double here = pairs * sh.H * (8 * p.nk + 32 * p.nt) + (double)p.key_rows * sh.kv_rank * sh.H * (sh.dim + sh.vdim);
-  p.pays = T > 16 && here < 2.0 * pairs * sh.H * (sh.row_w + sh.kv_rank);
+  const double product = (double)sh.kv_rank * sh.H * (sh.dim + sh.vdim);
+  const double here = pairs * sh.H * (8 * p.nk + 32 * p.nt) + 0.5 * p.key_rows * product;
+  const double there = 2.0 * pairs * sh.H * (sh.row_w + sh.kv_rank) + T * product;
+  p.pays = T > 16 && (T >= 32 || p.key_rows <= 2 * T) && here < there;
   return true;
 }
 
