@@ -97,10 +97,11 @@ struct DecodePlan {
   SpanTable spans;
   int n_wgs;
   int n_slots;  // partial slots: workgroup index + pair index is unique per segment
+  int align;    // spans end with the pairs: each pair's tiles are rounded up to a multiple of this (1: they do not)
   int cols;     // columns (new rows x heads of a group) per partial: the most any sequence has, at most 16
 };
-// wg_target: 0 = default
-DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target);
+// wg_target: 0 = default; aligned: spans may be made to end with the pairs (more partial slots than without)
+DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligned = true);
 
 // The same plan made on the device, for decode steps whose launches must not change from step to
 // step (a captured graph that is replayed): a step of one new row for each of the first n_seqs
@@ -113,6 +114,7 @@ struct DecodeDevicePlan {
   int tiles_per_wg;
   SpanTable spans;
   int total_tiles;
+  int align;
   int skip;  // a sequence would outgrow the cache or the cos/sin table: the step's kernels do nothing
 };
 constexpr int kDevicePlanWorkgroups = 256;

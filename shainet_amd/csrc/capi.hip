@@ -270,9 +270,11 @@ int run_attention(shainet_attn_ctx *c, const float *q_rot, float *kc, float *vc,
   if (path == Path::kDecodeSplitK) {
     SeqTable att;  // the attention kernel's view: long runs of new rows as two entries
     if (!decode_entries(st, sh, att)) return fail(SHAINET_HIP_ERR_RUNTIME, "decode entries do not fit");
-    const DecodePlan plan = plan_decode(att, sh, c->decode_wgs_override);
+    DecodePlan plan = plan_decode(att, sh, c->decode_wgs_override);
     DecodeArgs d;
     if (ws) {
+      if (decode_partial_floats(sh, plan) > ws->partial_floats || decode_flag_words(plan) > ws->flag_words)
+        plan = plan_decode(att, sh, c->decode_wgs_override, false);  // fewer slots
       if (decode_partial_floats(sh, plan) > ws->partial_floats || decode_flag_words(plan) > ws->flag_words)
         return fail(SHAINET_HIP_ERR_CAPACITY,
                     "this call needs %zu floats of partial results and %zu flag words; the static scratch holds "

@@ -7,8 +7,10 @@
 // Work split.  The key ranges of all (sequence, kv head) pairs are laid end to
 // end in units of 16-key tiles and cut into equal contiguous spans, one per
 // workgroup, so every workgroup streams the same number of bytes whatever the
-// sequence lengths are.  A span that crosses a pair boundary is processed as two
-// segments.  The four wavefronts of a workgroup take the tiles of the span
+// sequence lengths are.  Short launches (spans under 32 tiles) have their pairs rounded up to whole
+// spans instead where that costs no more workgroups, so that every workgroup has one segment:
+// there the second segment, not the bytes, is what a launch waits for (plan_decode).
+// A span that crosses a pair boundary is processed as two segments.  The four wavefronts of a workgroup take the tiles of the span
 // round-robin (across segments), each keeping its own online softmax per segment,
 // and merge through LDS into one partial (max, sum, O) per segment; the workgroup
 // that holds the end of a pair waits, once its own span is done, for the partials
@@ -137,9 +139,15 @@ __device__ __forceinline__ int workgroup_of_tile(int t, int tiles_per_wg, const 
   return 8 * k + r;
 }
 
+// Tiles of a pair in the stream: rounded up to whole spans where spans end with the pairs (align > 1).
+__host__ __device__ inline int padded_tiles(int n_s, int align) {
+  return align > 1 ? (n_s + align - 1) / align * align : n_s;
+}
+
 // One segment of a workgroup's span: tiles [tile0, tile1) of one (sequence, kv head) pair.
 struct Segment {
   int s, kvh, R, L, n_s, tile0, tile1, token;  // R new rows; L keys visible to the last of them
+  int n_p, next;  // the pair's tiles in the stream (n_s, rounded up: plan_decode); where the stream goes on behind the segment
   int rot;  // the segment's tiles are visited from tile0 + rot on, wrapping round to tile0 + rot - 1
   const float *kbase, *vbase;
 };
@@ -157,17 +165,20 @@ __device__ __forceinline__ int segment_rotation(int n_tiles, unsigned rotate) {
 
 // The segment that starts at tile t of the stream; s: a sequence at or before t's, moved up to it.
 __device__ __forceinline__ Segment segment_at(int t, int t_end, int &s, const SeqTable &st, const Shape &sh, int hd,
-                                              int vhd, bool own_v_rows, const float *kc, const float *vc, unsigned rotate) {
+                                              int vhd, bool own_v_rows, const float *kc, const float *vc, unsigned rotate,
+                                              int align) {
   while (s + 1 < st.n_seqs && t >= st.work_off[s + 1]) ++s;
   Segment g;
   g.s = s;
   g.R = st.n_new[s];
   g.L = st.start_pos[s] + g.R;  // visible keys of the last new row
   g.n_s = (g.L + 15) >> 4;    // tiles per kv head of this sequence
+  g.n_p = padded_tiles(g.n_s, align);
   const int rel = t - st.work_off[s];
-  g.kvh = rel / g.n_s;
-  g.tile0 = rel - g.kvh * g.n_s;
-  g.tile1 = g.tile0 + min(g.n_s - g.tile0, t_end - t);
+  g.kvh = rel / g.n_p;
+  g.tile0 = rel - g.kvh * g.n_p;
+  g.next = min(t + g.n_p - g.tile0, t_end);
+  g.tile1 = min(g.n_s, g.tile0 + (g.next - t));  // (never empty: a span starts in front of the pair's last tile)
   g.rot = __builtin_amdgcn_readfirstlane(segment_rotation(g.tile1 - g.tile0, rotate));
   const long long head_base = (long long)st.slot[s] * sh.seq_stride + (long long)g.kvh * sh.cap * hd;
   g.kbase = kc + head_base;
@@ -199,7 +210,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
     const float *__restrict__ q_rot, const float *__restrict__ kc, const float *__restrict__ vc,
     float *__restrict__ out, float *part_o, float *part_ml, unsigned *part_flag, unsigned *flag_set,
     int spin_limit, int *error, SeqTable st_arg, Shape sh, int tiles_per_wg_arg, SpanTable sp_arg, int total_tiles_arg,
-    int n_slots, int pstride, float c, unsigned rotate, const DecodeDevicePlan *__restrict__ dev, ReadAhead ah,
+    int align_arg, int n_slots, int pstride, float c, unsigned rotate, const DecodeDevicePlan *__restrict__ dev, ReadAhead ah,
     DistanceBias db) {
   static_assert(PAD || !BIAS, "sizes of their own come with padding");
   if constexpr (AHEAD) {
@@ -225,6 +236,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   const SpanTable &sp = DEV ? dev->spans : sp_arg;
   const int tiles_per_wg = DEV ? dev->tiles_per_wg : tiles_per_wg_arg;
   const int total_tiles = DEV ? dev->total_tiles : total_tiles_arg;
+  const int align = DEV ? dev->align : align_arg;
   constexpr int NT = C::NT;
   // per wavefront two K tile buffers; after a segment's last tile the wavefront parks its O
   // rows [g][HD] in one while the other already receives the next segment's first tile
@@ -251,7 +263,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   // along them with dependent scalar loads took 2.5 us for a workgroup in the middle of 16
   // sequences).
   int s = (int)__popcll(__ballot(lane + 1 < st.n_seqs && t_begin >= st.work_off[lane + 1 < kMaxSeqs ? lane + 1 : kMaxSeqs]));
-  Segment seg = segment_at(t, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate);
+  Segment seg = segment_at(t, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate, align);
 
   f32x4 v_next[4][C::NVU];
   float qr[HD / 4];
@@ -320,10 +332,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
       bias_row = db.tab + (long long)(seg.kvh * g + cq % g) * db.stride + (db.origin - (Lc - 1));
     }
     // the segment after this one, if the span has one
-    const int t_next = t + (tile1 - seg.tile0);
+    const int t_next = seg.next;
     const bool more = t_next < t_end;
     Segment nseg = seg;
-    if (more) nseg = segment_at(t_next, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate);
+    if (more) nseg = segment_at(t_next, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate, align);
     const int nplace = first_place(t_next);
     const bool nhave = more && nplace < nseg.tile1 - nseg.tile0;
     const int ntile = nhave ? tile_at(nseg, nplace) : 0;
@@ -482,7 +494,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   if (have_merge) {
     // This workgroup holds the end of a pair that others began: they have lower indices, were
     // started before this one and wait for nobody, so waiting for their partials is safe.
-    const int a = st.work_off[mseg.s] + mseg.kvh * mseg.n_s;  // the pair's tiles are [a, a + n_s)
+    const int a = st.work_off[mseg.s] + mseg.kvh * mseg.n_p;  // the pair's tiles are [a, a + n_s)
     const int w_lo = workgroup_of_tile(a, tiles_per_wg, sp);
     const int n_part = (int)blockIdx.x - w_lo + 1;
     const int pair = mseg.s * sh.KV + mseg.kvh;
@@ -607,6 +619,22 @@ __host__ __device__ inline void spans_from_shares(const int (&share)[8], int q, 
   }
 }
 
+// Tiles per span when `total` tiles go to `wgs` workgroups: at least one per wavefront.
+__host__ __device__ inline int least_span(int total, int wgs) {
+  const int q = (total + wgs - 1) / wgs;
+  return q < kDecodeWaves ? kDecodeWaves : q;
+}
+// Spans that end with the pairs (DecodePlan::align): the longest worth having for that, two tiles per
+// wavefront or a quarter more than the least; shorter than the spans of unequal shares.  And the number of spans a
+// pair may have: an odd one, or the pairs' last spans, which wait for the others and merge, meet on one, two or
+// four of the eight XCDs (a call with 32 pairs of 44 tiles of 8 KiB: 18.2 us in 8 spans each, 13.6 laid end
+// to end, 12.0 in 7).
+__host__ __device__ inline int widest_aligned_span(int q) {
+  const int most = q + q / 4 > 2 * kDecodeWaves ? q + q / 4 : 2 * kDecodeWaves;
+  return most < 31 ? most : 31;
+}
+__host__ __device__ inline bool spans_may_end_with(int n_s, int q) { return n_s == 0 || ((n_s + q - 1) / q & 1); }
+
 struct ShareArg {
   int v[8];
 };
@@ -626,20 +654,32 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
       out->st.n_seqs = n_seqs;
       out->tiles_per_wg = 0;
       out->total_tiles = 0;
+      out->align = 1;
       out->skip = 1;
       spans_from_shares(shares.v, 0, out->spans);  // all zero: no workgroup finds tiles
       if (*error == 0) *error = 2;  // a pending 1 (a given-up wait) is the graver report and stays
     }
     return;
   }
-  const int tiles = mine ? sh.KV * ((start + 1 + 15) >> 4) : 0;
-  int incl = tiles;  // inclusive prefix sum over the lanes
+  const int n_s = mine ? (start + 1 + 15) >> 4 : 0;
+  auto prefix = [&](int x) {  // inclusive prefix sum over the lanes
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int up = __shfl_up(incl, o);
-    if (s >= o) incl += up;
-  }
-  const int total = __shfl(incl, 63);
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(x, o);
+      if (s >= o) x += up;
+    }
+    return x;
+  };
+  int tiles = sh.KV * n_s;
+  int incl = prefix(tiles), total = __shfl(incl, 63), q = least_span(total, kDevicePlanWorkgroups), align = 1;
+  for (int a = q; a <= widest_aligned_span(q); ++a)
+    if (__all(spans_may_end_with(n_s, a)) && __shfl(prefix(sh.KV * ((n_s + a - 1) / a)), 63) <= kDevicePlanWorkgroups) {
+      q = align = a;
+      tiles = sh.KV * padded_tiles(n_s, a);
+      incl = prefix(tiles);
+      total = __shfl(incl, 63);
+      break;
+    }
   if (mine) {
     out->st.slot[s] = s;
     out->st.start_pos[s] = start;
@@ -652,9 +692,8 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
     out->st.n_seqs = n_seqs;
     out->st.tok_off[n_seqs] = n_seqs;
     out->st.work_off[n_seqs] = total;
-    int q = (total + kDevicePlanWorkgroups - 1) / kDevicePlanWorkgroups;
-    if (q < kDecodeWaves) q = kDecodeWaves;
     out->tiles_per_wg = q;
+    out->align = align;
     out->total_tiles = total;
     out->skip = 0;
     spans_from_shares(shares.v, q, out->spans);
@@ -663,20 +702,39 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
 
 }  // namespace
 
-DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target) {
+DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligned) {
   DecodePlan p;
-  st.work_off[0] = 0;
-  for (int s = 0; s < st.n_seqs; ++s)
-    st.work_off[s + 1] = st.work_off[s] + sh.KV * ((st.start_pos[s] + st.n_new[s] + 15) / 16);
-  p.total_tiles = st.work_off[st.n_seqs];
+  auto lay_out = [&](int align) {
+    p.align = align;
+    st.work_off[0] = 0;
+    for (int s = 0; s < st.n_seqs; ++s)
+      st.work_off[s + 1] = st.work_off[s] + sh.KV * padded_tiles((st.start_pos[s] + st.n_new[s] + 15) / 16, align);
+    p.total_tiles = st.work_off[st.n_seqs];
+  };
+  lay_out(1);
   // One workgroup on each of the 256 compute units.  Its four wavefronts keep 64 KiB
   // of K and V in flight, 16 MiB over the chip, which saturates HBM; twice as many
   // workgroups only double the partials to merge and the arrivals at each pair's
   // counter (measured: 4 to 10 % slower from batch 1 x 4096 to batch 4 x 32768).
   if (wg_target < 1) wg_target = 256;
-  // at least one tile per wavefront
-  int q = (p.total_tiles + wg_target - 1) / wg_target;
-  if (q < kDecodeWaves) q = kDecodeWaves;
+  int q = least_span(p.total_tiles, wg_target);
+  // Spans that end with the pairs, where that takes no more workgroups: a span that runs from one pair
+  // into the next is two segments behind each other with a merge in between.  Per call with its prep launch, one
+  // sequence, 8 kv heads of 64 (128): 100 keys 13.0 -> 9.1 us (17.4 -> 13.1), whole pairs; 512 keys 13.1 -> 10.4
+  // (17.3 -> 14.3), 1024 keys 13.1 -> 10.5 (18.3 -> 15.5); 16 sequences of 100 keys 16.0 -> 14.6 (20.9 -> 14.4).
+  for (int a = q; aligned && a <= widest_aligned_span(q); ++a) {
+    long long wgs = 0;
+    bool fits = true;
+    for (int s = 0; s < st.n_seqs; ++s) {
+      const int n_s = (st.start_pos[s] + st.n_new[s] + 15) / 16;
+      fits = fits && spans_may_end_with(n_s, a);
+      wgs += (long long)sh.KV * ((n_s + a - 1) / a);
+    }
+    if (!fits || wgs > wg_target) continue;
+    q = a;
+    lay_out(a);
+    break;
+  }
   p.tiles_per_wg = q;
   spans_from_shares(span_shares().v, q, p.spans);
   // the first workgroup count whose spans cover the stream
@@ -759,7 +817,7 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
 #define SHAINET_DECODE_LAUNCH(HD_, DEV_, PAD_)                                                                      \
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, DEV_, PAD_>), grid, block, 0, stream, before,      \
                        after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit,       \
-                       d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.n_slots, p.cols, c, rotate, dev, ah, db)
+                       d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c, rotate, dev, ah, db)
 #define SHAINET_DECODE_LAUNCH_HD(HD_, PAD_) \
   do {                                      \
     if (dev)                                \
@@ -770,7 +828,7 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
 #define SHAINET_DECODE_LAUNCH_BIAS(HD_)                                                                             \
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, false, true, false, true>), grid, block, 0, stream, \
                        before, after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set,           \
-                       spin_limit, d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.n_slots, p.cols, c,   \
+                       spin_limit, d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c,   \
                        rotate, dev, ah, db)
   if (bias && tile_hd == 64)
     SHAINET_DECODE_LAUNCH_BIAS(64);
@@ -781,11 +839,11 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
   else if (ah.w && sh.hd == 64)
     hipLaunchKernelGGL((decode_splitk_kernel<64, kDecodeWaves, false, false, true>), grid, block, 0, stream, d.q_rot, d.kc,
                        d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit, d.error, st, sh, p.tiles_per_wg,
-                       p.spans, p.total_tiles, p.n_slots, p.cols, c, rotate, dev, ah, db);
+                       p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c, rotate, dev, ah, db);
   else if (ah.w)
     hipLaunchKernelGGL((decode_splitk_kernel<128, kDecodeWaves, false, false, true>), grid, block, 0, stream, d.q_rot, d.kc,
                        d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit, d.error, st, sh, p.tiles_per_wg,
-                       p.spans, p.total_tiles, p.n_slots, p.cols, c, rotate, dev, ah, db);
+                       p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c, rotate, dev, ah, db);
   else if (sh.hd == 64)
     SHAINET_DECODE_LAUNCH_HD(64, false);
   else if (sh.hd == 128)

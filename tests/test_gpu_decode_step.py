@@ -68,6 +68,10 @@ CASES = [
     (32, 8, 128, [4095], False, False),                       # batch 1 of the decode workloads
     (32, 8, 128, [0, 1, 15, 16, 17, 300, 2999, 31], True, False),  # empty and tile-edge lengths
     (32, 8, 64, [16000], True, False),                        # one pair over many workgroups
+    (32, 8, 64, [62], False, False),                          # spans that end with the pairs: 4 to 6 tiles, one span each
+    (8, 2, 64, [140, 130, 190], False, True),                 # 9 to 12 tiles: three spans of four
+    (32, 8, 128, [126, 63, 10, 127], True, False),            # whole pairs of unequal lengths, up to 8 tiles
+    (32, 8, 128, [700] * 4, False, False),                    # two tiles per wavefront
     (14, 2, 64, [700, 5, 90], False, True),                   # Qwen2.5-0.5B heads: g = 7, biases
     (8, 8, 128, [int(x) for x in np.random.default_rng(3).integers(1, 1500, 64)], False, False),  # 64 sequences, g = 1
     (32, 2, 128, [513, 64], True, False),                     # g = 16

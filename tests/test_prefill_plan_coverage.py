@@ -67,3 +67,23 @@ def test_decode_and_generic_paths_are_told_apart():
     assert sa.describe_plan(16, 4, 256, [0], [40])["path"] == sa.hip.PATH_GENERIC
     head = sa.describe_plan(32, 8, 128, [5000] * 16, [1] * 16)
     assert head["workgroups"] == 256 and head["units"] * 256 >= 16 * 8 * 313
+
+
+def test_decode_spans_end_with_the_pairs():
+    def split(lens, KV=8, hd=64):
+        p = sa.describe_plan(4 * KV, KV, hd, [n - 1 for n in lens], [1] * len(lens))
+        return p["workgroups"], p["units"]
+
+    apart = 0
+    for tiles in range(1, 250):  # one sequence: an odd number of spans per pair, or spans end to end
+        wgs, q = split([16 * tiles])
+        per = -(-tiles // q)
+        if wgs != 8 * per or per % 2 == 0:
+            apart += 1
+            assert wgs == -(-8 * tiles // q) and q == max(4, -(-8 * tiles // 256)), tiles
+    assert apart < 25  # of 249, the most of them long ones
+    assert split([16 * 5]) == (8, 5) and split([16 * 8]) == (8, 8)      # whole pairs
+    assert split([16 * 12]) == (24, 4) and split([16 * 13]) == (24, 5)
+    assert split([16 * 5] * 16) == (128, 5)
+    assert split([16 * 9] * 16) == (231, 5)  # two spans each would meet on four XCDs: 1152 tiles end to end
+    assert split([64], 300, 256) == (240, 5)  # more pairs than workgroups: end to end

@@ -170,3 +170,22 @@ def test_noalloc_refuses_what_it_cannot_hold(hip):
     with pytest.raises(hip.HipError, match="static scratch"):
         wide.forward_noalloc(c3, q, k, v, [2] * 64)
     assert c3.len(0) == 0
+
+
+def test_noalloc_small_pairs_near_the_scratch_limit(hip):
+    # 248 pairs of one tile: one span per pair would take 496 partial slots of 16 columns x 258 floats,
+    # more than the array holds; spans of four tiles take 310
+    import torch
+
+    H, KV, hd = 496, 31, 132
+    ctxs = [hip.AttnContext(H, KV, hd, max_positions=64) for _ in range(2)]
+    caches = [hip.KVCache(c, 8, 32) for c in ctxs]
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    for step in range(3):
+        q, k, v = _rows(torch, gen, 8, H, KV, hd)
+        want = ctxs[0].forward(caches[0], q, k, v, [1] * 8)
+        got = ctxs[1].forward_noalloc(caches[1], q, k, v, [1] * 8)
+        ctxs[0].sync()
+        ctxs[1].sync()
+        # the same arithmetic on both: one wavefront has a pair's only tile, whatever span it lies in
+        assert torch.equal(got, want), f"step {step}"
