@@ -436,7 +436,7 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvArgs a) {
 // the sums meet in LDS (a wavefront per pair, two rows each, took 0.85 us longer for 3072 rows).
 // DYT: the prologue is Dynamic Tanh instead: x becomes tanh(alpha x) gamma + beta where it is staged.
 // TAIL: rows of a.K values, a multiple of 4 below 256 KV4; the pieces beyond are zeros (one row of 384 -> 1536, in
-// front of which the split product took 7.8 us: 3.9).
+// front of which the split product took 7.7 us: 3.9).
 template <int KV4, int NACC, int SP, bool MULTI, bool PREP = false, bool DYT = false, bool TAIL = false>
 __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   static_assert(!PREP || (NACC == 1 && SP == 1 && !MULTI), "the q | k | v epilogue: one row per wavefront");

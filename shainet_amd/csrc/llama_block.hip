@@ -160,8 +160,8 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     f.w_t_has_gamma = f.w_t && gamma;
   };
   // One row with QK-norm: the sum of squares needs the whole head, which the product over transposed weights does not
-  // hold in one place; it and the prep kernel behind it take 4 + 3.5 us where the split product with prep inside
-  // takes 10 (1024 -> 2048), 5.5 + 3.5 against 10.9 (2048 -> 3072).
+  // hold in one place; it and the prep kernel behind it take 4.8 + 4.3 us where the split product with prep inside
+  // takes 10.2 (1024 -> 2048).
   const bool norm_apart = T == 1 && (l->has_q_norm || l->has_k_norm) && transposed_twins_wanted() &&
                           gemvt_takes(T, l->d_model, wide, pre.epilogue, pre.norm);
   if (ahead && ahead->wt && T == 1) {
