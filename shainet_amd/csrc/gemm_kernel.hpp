@@ -1,4 +1,4 @@
-// Launcher of the fp32 MFMA product y[T,N] = x[T,K] W[K,N] (+ res) for more than 16 rows.
+// Launcher of the product y[T,N] = x[T,K] W[K,N] (+ res) for five rows and more, fp32 on the bf16 matrix cores.
 #pragma once
 #include <hip/hip_runtime.h>
 
