@@ -9,9 +9,10 @@
 // D[m = 4 (l / 16) + r][n = l % 16] for accumulator register r.  The contraction index may be
 // visited in any order as long as A and B agree.
 //
-// Prefill is the expanded form: latent_prefill_kernel, fp32 MFMA 32x32x2 over keys and values that a
+// Prefill is the expanded form: latent_prefill_kernel, split bf16 MFMA 32x32x16 over keys and values that a
 // product made from the cached rows, the rotated key part read from the rows themselves.
 #include "latent_kernels.hpp"
+#include "split_mfma.hpp"
 
 #include <math.h>
 #include <stdint.h>
@@ -20,9 +21,6 @@
 namespace shainet {
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -392,14 +390,19 @@ __global__ __launch_bounds__(1024) void latent_out_kernel(const float *__restric
 // ---- expanded form -----------------------------------------------------------------------------
 //
 // A workgroup owns 128 rows of one head, a wavefront 32 of them; all walk the keys in tiles of 32 that
-// go global memory -> registers -> LDS, the next tile's loads in flight behind the MFMAs of this one
-// (two workgroups share a compute unit, so that one's barriers hide behind the other's MFMAs).
-// S^T = K Q^T, so that the probabilities come out of the accumulator laid out as the B operand of
-// O^T += V^T P^T.  MFMA 32x32x2 layout (lane l): A[m = l % 32][k = l / 32], B[k = l / 32][n = l % 32],
-// D[m = 8 (r / 4) + 4 (l / 32) + r % 4][n = l % 32] for accumulator register r.
-//   scores:  m = key within the tile, n = row; lane half j = l / 32 covers d = 8 i + 4 j + 0..3 of piece i;
+// go global memory -> registers -> split -> LDS (one stage of keys, one of values; the values travel behind the
+// score MFMAs, the next tile's keys behind the others).  Two workgroups share a compute unit, so that one's barriers
+// hide behind the other's MFMAs.  Queries, keys, values and probabilities are exact sums of three bf16 numbers
+// (split_mfma.hpp); queries of more than 128 dimensions have no registers for their parts and are split
+// again for every tile, beside the MFMAs.  S^T = K Q^T, so that the probabilities come out of the accumulator laid out as
+// the B operand of O^T += V^T P^T:
+//   scores:  m = key within the tile, n = row; step i of lane half j covers d = 16 i + 8 j + 0..7;
 //            d runs over the unrotated dimensions, padded to a multiple of 8, then the rotated ones.
-//   output:  tile t, m: d = NT m + t; step r of lane half j is key 8 (r / 4) + 4 j + r % 4.
+//   output:  tile t, m: d = NT m + t; step u of lane half j covers keys 16 u + 4 j + {0..3, 8..11}.
+// LDS in units of 16 bytes: keys [part][octet of d][key], an octet 33 units; values [part][group 2 u + j of eight
+// keys][column], column d at place d / NT of block d % NT, 36 units a block.
+// Bound by registers (256 of them: two wavefronts per SIMD) and the splits beside the MFMAs: 2048 rows of 16 heads of 192 and 128
+// dimensions 268 -> 208 us against v_mfma_f32_32x32x2_f32, whose cycles the vector ALU cannot use.
 // NK: pieces of 8 query / key dimensions at most; NT: tiles of 32 value dimensions.
 struct LatentPrefillArgs {
   const float *q;        // [T, H (dim + rot_dim)], rotated (launch_latent_append)
@@ -417,10 +420,11 @@ struct LatentPrefillArgs {
 
 template <int NK, int NT>
 __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(const LatentPrefillArgs a) {
-  constexpr int KSTR = NK * 8 + 4, VSTR = NT * 32;
-  constexpr int KU = (NK * 2 + 7) / 8, VU = NT;  // float4 of a K (V) tile per thread: 8 threads per row
-  __shared__ __attribute__((aligned(16))) float Ks[32 * KSTR];
-  __shared__ __attribute__((aligned(16))) float Vs[32 * VSTR];
+  constexpr int VSTR = NT * 32, KS = NK / 2;  // columns of the output; MFMA steps of the scores
+  constexpr int KU = (NK + 7) / 8, VU = NT / 2;  // per thread: octets of a tile's keys, eight rows of a column of its values
+  constexpr int kOct = 33, kPartK = NK * kOct, kGroup = NT * 36, kPartV = 4 * kGroup;
+  constexpr bool HELD = NK <= 16 && NK * NT <= 48;  // the parts of the query stay in registers
+  __shared__ __attribute__((aligned(16))) u32x4 lds[3 * kPartK + 3 * kPartV];
   const LatentShape &sh = a.sh;
   // heads fastest: with a multiple of 8 heads an XCD (index % 8) keeps to its own heads' keys and
   // values; the blocks with the most keys start first
@@ -444,60 +448,85 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
   const int per_chunk = (n_tiles + a.splits - 1) / a.splits;
   const int kt0 = kt_all0 + chunk * per_chunk, kt1 = min(kt_all0 + n_tiles, kt0 + per_chunk);
 
-  // staging: 8 threads per key row, 16-byte pieces sub, sub + 8, ...; a thread without a piece of its
-  // own repeats the last one (same source, same place), so no load or store is conditional
-  const int srow = threadIdx.x >> 3, sub = threadIdx.x & 7;
   const unsigned kv_stride = (unsigned)(sh.H * (sh.dim + sh.vdim));
-  const int n_pieces = dn >> 2, r_pieces = dr >> 2;
+  // staging: a thread takes octets sub, sub + 8, ... of one key's row (those behind the last one repeat it) and eight
+  // rows of one or two groups of a column of the values
+  const int k_row = threadIdx.x >> 3, sub = threadIdx.x & 7;
   const float *k_src[KU];
-  unsigned k_step[KU];
-  int k_dst[KU];
+  bool k_rot[KU], k_whole[KU];  // part of the rotated dimensions; the octet's second half lies within the key
 #pragma unroll
   for (int u = 0; u < KU; ++u) {
-    const int p = min(sub + 8 * u, n_pieces + r_pieces - 1);
-    const bool is_rot = p >= n_pieces;
-    k_src[u] = is_rot ? a.key_rot + 4 * (p - n_pieces) : a.kv + h * dn + 4 * p;
-    k_step[u] = is_rot ? (unsigned)sh.row_w : kv_stride;
-    k_dst[u] = srow * KSTR + (is_rot ? dn8 + 4 * (p - n_pieces) : 4 * p);
+    const int d = 8 * min(sub + 8 * u, NK - 1), e = d - dn8;
+    k_rot[u] = e >= 0 && e < dr;  // behind both parts the query is zero, any of the key's values will do
+    k_src[u] = k_rot[u] ? a.key_rot + e : a.kv + h * dn + (d < dn8 ? d : 0);
+    k_whole[u] = k_rot[u] ? e + 4 < dr : d + 4 < dn;
   }
-  // (pieces beyond vdim read what follows: the columns they land in are never stored)
-  const float *v_src = a.kv + sh.H * dn + h * sh.vdim + 4 * sub;
-  f32x4 stage[KU > VU ? KU : VU];
+  const int v_col = threadIdx.x % VSTR, v_group = threadIdx.x / VSTR;
+  const int v_row = 16 * (v_group >> 1) + 4 * (v_group & 1);  // and 16 further on for the second
+  const int v_unit = 3 * kPartK + v_group * kGroup + v_col % NT * 36 + v_col / NT;
+  const unsigned v_off = v_col < sh.vdim ? v_col : 0;  // (columns beyond are never stored)
+  const float *v_src = a.kv + sh.H * dn + h * sh.vdim;
+  f32x4 stage[2 * (KU > VU ? KU : VU)];
   auto load_k = [&](int kt) {
-    const unsigned key = (unsigned)min(kt * 32 + srow, b_hi);
+    const unsigned key = (unsigned)min(kt * 32 + k_row, b_hi);
 #pragma unroll
-    for (int u = 0; u < KU; ++u) stage[u] = *(const f32x4 *)(k_src[u] + (unsigned long long)key * k_step[u]);
+    for (int u = 0; u < KU; ++u) {
+      const float *p = k_src[u] + (unsigned long long)key * (k_rot[u] ? (unsigned)sh.row_w : kv_stride);
+      stage[2 * u] = *(const f32x4 *)p;
+      stage[2 * u + 1] = *(const f32x4 *)(p + (k_whole[u] ? 4 : 0));
+    }
+  };
+  auto load_v = [&](int kt) {
+    if (kt * 32 + 31 <= b_hi) {
+      const float *p = v_src + (unsigned long long)(unsigned)(kt * 32) * kv_stride;
+      const unsigned off = (unsigned)v_row * kv_stride + v_off;
+#pragma unroll
+      for (int u = 0; u < VU; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          stage[2 * u + (i >> 2)][i & 3] = (p + (unsigned long long)(16 * u + (i & 3) + 8 * (i >> 2)) * kv_stride)[off];
+    } else {
+#pragma unroll
+      for (int u = 0; u < VU; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          stage[2 * u + (i >> 2)][i & 3] =
+              v_src[(unsigned long long)(unsigned)min(kt * 32 + v_row + 16 * u + (i & 3) + 8 * (i >> 2), b_hi) * kv_stride + v_off];
+    }
+  };
+  auto park = [&](int u, int unit, int part) {
+    u32x4 hi, mid, lo;
+    split_octet(stage[2 * u], stage[2 * u + 1], hi, mid, lo);
+    lds[unit] = hi;
+    lds[unit + part] = mid;
+    lds[unit + 2 * part] = lo;
   };
   auto park_k = [&]() {
 #pragma unroll
-    for (int u = 0; u < KU; ++u) *(f32x4 *)&Ks[k_dst[u]] = stage[u];
-  };
-  auto load_v = [&](int kt) {
-    const float *p = v_src + (unsigned long long)(unsigned)min(kt * 32 + srow, b_hi) * kv_stride;
-#pragma unroll
-    for (int u = 0; u < VU; ++u) stage[u] = *(const f32x4 *)(p + 32 * u);
+    for (int u = 0; u < KU; ++u) park(u, min(sub + 8 * u, NK - 1) * kOct + k_row, kPartK);
   };
   auto park_v = [&]() {
 #pragma unroll
-    for (int u = 0; u < VU; ++u) *(f32x4 *)&Vs[srow * VSTR + 4 * (sub + 8 * u)] = stage[u];
+    for (int u = 0; u < VU; ++u) park(u, v_unit + 2 * u * kGroup, kPartV);
   };
   if (kt0 < kt1) load_k(kt0);
-  // the padding between and behind the two parts of a key: the query is zero there, so anything finite will do
-  for (int i = threadIdx.x; i < 32 * KSTR; i += 256) Ks[i] = 0.f;
 
-  float qr[NK * 4];
-  {
-    const float *qp = a.q + ((long long)my_row * sh.H + h) * (dn + dr);
+  f32x4 qr[HELD ? 1 : KS][2];
+  u32x4 qf[HELD ? KS : 1][3];
+  const float *q_row = a.q + ((long long)my_row * sh.H + h) * (dn + dr);
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int d = 8 * i + 4 * j, e = d - dn8;
-      f32x4 x = {0.f, 0.f, 0.f, 0.f};
-      if (d < dn || (e >= 0 && e < dr)) x = *(const f32x4 *)(qp + (d < dn ? d : dn + e));
-      qr[4 * i + 0] = x.x * a.c;
-      qr[4 * i + 1] = x.y * a.c;
-      qr[4 * i + 2] = x.z * a.c;
-      qr[4 * i + 3] = x.w * a.c;
+  for (int i = 0; i < KS; ++i) {
+    f32x4 x[2];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const int d = 16 * i + 8 * j + 4 * w, e = d - dn8;
+      x[w] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (d < dn || (e >= 0 && e < dr)) x[w] = *(const f32x4 *)(q_row + (d < dn ? d : dn + e)) * a.c;
     }
+    if constexpr (HELD)
+      split_octet(x[0], x[1], qf[i][0], qf[i][1], qf[i][2]);
+    else
+      qr[i][0] = x[0], qr[i][1] = x[1];
   }
   f32x16 o[NT];
 #pragma unroll
@@ -507,9 +536,8 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
   float m = -INFINITY, l = 0.f;  // reference value of the row's exponentials (log2 units), this lane half's sum
   constexpr float kTau = 8.f;    // scores may exceed it by this much before it moves
 
-  // Per tile: the values travel while the scores are computed, the next tile's keys while the
-  // values are used; each set is parked in LDS behind a barrier that says the stage is free.
-  __syncthreads();
+  // Per tile: the values travel while the scores are computed, the next tile's keys while the values
+  // are used; each set is parked in LDS behind a barrier that says its stage is free.
   if (kt0 < kt1) park_k();
   __syncthreads();
   for (int kt = kt0; kt < kt1; ++kt) {
@@ -520,20 +548,18 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
     if (visible) {
-      const float *kl = &Ks[n * KSTR + 4 * j];
-      constexpr int PF = 2;
-      f32x4 kf[NK];
+      const u32x4 *kl = lds + j * kOct + n;
 #pragma unroll
-      for (int i = 0; i < PF && i < NK; ++i) kf[i] = *(const f32x4 *)(kl + 8 * i);
+      for (int i = 0; i < KS; ++i) {
+        u32x4 kf[3];
 #pragma unroll
-      for (int i = 0; i < NK; ++i) {
-        if (i + PF < NK) kf[i + PF] = *(const f32x4 *)(kl + 8 * (i + PF));
-        __builtin_amdgcn_sched_barrier(0x7);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i].x, qr[4 * i + 0], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i].y, qr[4 * i + 1], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i].z, qr[4 * i + 2], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i].w, qr[4 * i + 3], s, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0x7);
+        for (int w = 0; w < 3; ++w) kf[w] = kl[w * kPartK + 2 * i * kOct];
+        if constexpr (!HELD) {
+          asm volatile("" : "+v"(qr[i][0]), "+v"(qr[i][1]));  // (not moved out of the loop over the tiles)
+          split_octet(qr[i][0], qr[i][1], qf[0][0], qf[0][1], qf[0][2]);
+        }
+#pragma unroll
+        for (int w = 0; w < 6; ++w) s = mfma_bf16(kf[kPartA[w]], qf[HELD ? i : 0][kPartB[w]], s);
       }
       if (k_first < w_lo_max || k_last > w_hi_min) {  // an edge of some row's keys lies in the tile
 #pragma unroll
@@ -570,23 +596,68 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
     __syncthreads();
     if (kt + 1 < kt1) load_k(kt + 1);
     if (visible) {
-      constexpr int PF = 2;
-      typedef float vrow_t __attribute__((ext_vector_type(NT)));
-      const float *vl = &Vs[4 * j * VSTR + NT * n];
-      vrow_t vv[16];
+      const u32x4 *vl = lds + 3 * kPartK + j * kGroup + n;
 #pragma unroll
-      for (int r = 0; r < PF; ++r) vv[r] = *(const vrow_t *)(vl + (8 * (r >> 2) + (r & 3)) * VSTR);
+      for (int u = 0; u < 2; ++u) {
+        u32x4 pf[3];
+        split_octet(f32x4{s[8 * u], s[8 * u + 1], s[8 * u + 2], s[8 * u + 3]},
+                    f32x4{s[8 * u + 4], s[8 * u + 5], s[8 * u + 6], s[8 * u + 7]}, pf[0], pf[1], pf[2]);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        if (r + PF < 16) vv[r + PF] = *(const vrow_t *)(vl + (8 * ((r + PF) >> 2) + ((r + PF) & 3)) * VSTR);
-        __builtin_amdgcn_sched_barrier(0x7);
+        for (int t = 0; t < NT; ++t) {
+          u32x4 vf[3];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[r][t], s[r], o[t], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0x7);
+          for (int w = 0; w < 3; ++w) vf[w] = vl[w * kPartV + 2 * u * kGroup + 36 * t];
+#pragma unroll
+          for (int w = 0; w < 6; ++w) o[t] = mfma_bf16(vf[kPartA[w]], pf[kPartB[w]], o[t]);
+        }
       }
     }
     if (kt + 1 < kt1) park_k();
     __syncthreads();
+  }
+
+  // Results that are not finite come from operands that are not (or from values that round to infinity as bf16): the
+  // wavefront takes its keys again in fp32, which says which.
+  float probe = l * 0.f;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
+  if (wave_active && __any(probe != 0.f)) {
+    m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+    const int last = min(kt1 * 32 - 1, w_hi_max);
+#pragma clang loop unroll(disable)
+    for (int key = max(kt0 * 32, w_lo_min); key <= last; ++key) {
+      if (key < my_lo || key > my_hi) continue;
+      const float *kp = a.kv + (unsigned long long)(unsigned)key * kv_stride, *rp = a.key_rot + (unsigned long long)(unsigned)key * sh.row_w;
+      float sc = 0.f;
+#pragma clang loop unroll(disable)
+      for (int d = 0; d < dn; ++d) sc = fmaf(q_row[d] * a.c, kp[h * dn + d], sc);
+#pragma clang loop unroll(disable)
+      for (int d = 0; d < dr; ++d) sc = fmaf(q_row[dn + d] * a.c, rp[d], sc);
+      if (sc > m) {  // here the reference is the running maximum
+        const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - sc);
+        m = sc;
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+      }
+      const float e = sc == -INFINITY ? 0.f : fast_exp2(sc - m);
+      l += 0.5f * e;  // (both lane halves of a row count every key)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int d = NT * (8 * (r >> 2) + 4 * j + (r & 3)) + t;
+          o[t][r] = fmaf(e, kp[sh.H * dn + h * sh.vdim + (d < sh.vdim ? d : 0)], o[t][r]);
+        }
+    }
   }
 
   l += __shfl_xor(l, 32);
@@ -639,7 +710,8 @@ __global__ __launch_bounds__(256) void latent_prefill_combine_kernel(const Laten
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const float f = s0 + u < a.splits ? fast_exp2(ml[u].x - mm) : 0.f;  // 0 for a chunk in which the row saw no key
+        if (s0 + u >= a.splits) break;
+        const float f = fast_exp2(ml[u].x - mm);  // 0 for a chunk in which the row saw no key
         acc += f * x[u];
         den += f * ml[u].y;
       }

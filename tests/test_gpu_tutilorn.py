@@ -202,6 +202,24 @@ def test_window_edges(hip, tmp_path, monkeypatch, window, rows, path):
             close(np.concatenate(got), want)
 
 
+@pytest.mark.parametrize("name", ["even", "wide", "vast"])
+def test_expanded_keeps_what_is_not_finite_to_the_rows_that_see_it(hip, tmp_path, monkeypatch, name):
+    """A row of NaN makes NaN of itself and of the rows whose window holds it, and of no other: the operands of
+    the expanded form's products are sums of parts, and neighbours in a tile multiply the NaN by zero."""
+    monkeypatch.setenv("SHAINET_HIP_LATENT_PATH", "expanded")
+    p = Pair(hip, tmp_path, geometry(name, mlp=False))
+    rows, bad, window = 200, 100, GEOMETRIES[name]["m"]["window"]
+    x = np.random.default_rng(12).standard_normal((rows, p.cfg["width"])).astype(np.float32)
+    want = p.layer(0, x)
+    x[bad] = np.nan
+    got = p.model.blocks[0].forward_cached(x)
+    sees = np.arange(rows) >= bad
+    if window:
+        sees &= np.arange(rows) < bad + window
+    assert np.isnan(got[sees]).all()
+    close(got[~sees], want[~sees])
+
+
 @pytest.mark.parametrize("path", ["absorbed", "expanded"])
 def test_sink(hip, tmp_path, monkeypatch, path):
     """Sinks that take nearly everything, about half and nothing; the first position sees one key only."""
