@@ -363,9 +363,8 @@ int run_device_tokens(shainet_llama_model *m, const int *d_tokens, int T, bool n
     return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   m->have_logits = false;
   int cur = 0, rc = -1;
-  if (T == 1 && !no_cache && !embedded) {
-    rc = run_step(m, d_tokens);
-    if (rc > 0) return rc;
+  if (T == 1 && !no_cache) {
+    if (!embedded && (rc = run_step(m, d_tokens)) > 0) return rc;
     if (rc < 0 && m->step.mode == SHAINET_HIP_DECODE_PERSISTENT)
       return fail(SHAINET_HIP_ERR_ARGUMENT, "this model's geometry does not fit the one-launch decode step");
   }

@@ -508,6 +508,9 @@ def test_what_belongs_to_other_blocks_is_refused(hip, tmp_path):
     with pytest.raises(hip.ArgumentError):
         p.model.set_decode_mode(p.model.DECODE_PERSISTENT)
         p.model.run([1])
+    p.model.run([1, 2])  # (more rows than one are no decode step)
+    with pytest.raises(hip.ArgumentError):
+        p.model.generate_greedy(3)
     p.model.set_decode_mode(p.model.DECODE_AUTO)
     p.model.clear_cache()
     close(p.model.run([1]), p.logits([1])[0])
