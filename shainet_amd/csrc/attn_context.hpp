@@ -50,9 +50,6 @@ struct shainet_attn_ctx {
   float *d_bq = nullptr, *d_bk = nullptr, *d_bv = nullptr;
   float2 *d_rope = nullptr;
   int rope_positions = 0;
-  // DecodeArgs::ahead_* of the next decode launch (shainet_attn_read_ahead); forgotten after it
-  const float *ahead_w = nullptr;
-  int ahead_k = 0, ahead_n = 0, ahead_wgs = 0;
   hipStream_t stream = nullptr;      // where work is issued
   hipStream_t own_stream = nullptr;  // created with the context, destroyed with it
   shainet::DevBuf q_rot, partials, in_q, in_k, in_v, out;

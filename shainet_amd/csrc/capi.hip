@@ -244,9 +244,10 @@ struct Workspace {
 // QK-norm, RoPE and the append first.  prep == nullptr: q_rot holds rotated
 // queries and the cache already holds the new rows.
 // ws != nullptr: nothing is allocated; the split-K decode path only.
+// ahead (nullable): what a split-K decode launch also reads.
 int run_attention(shainet_attn_ctx *c, const float *q_rot, float *kc, float *vc, float *out, SeqTable &st,
                   const Shape &sh, int total_tokens, float scale, hipStream_t stream, const PrepArgs *prep,
-                  const Workspace *ws = nullptr, const DistanceBias *bias = nullptr) {
+                  const Workspace *ws = nullptr, const DistanceBias *bias = nullptr, const AheadRows *ahead = nullptr) {
   const int v_hd = bias ? bias->v_hd : sh.hd;
   const Path path = choose_path(st, sh, v_hd);
   if (ws && path != Path::kDecodeSplitK)
@@ -297,13 +298,7 @@ int run_attention(shainet_attn_ctx *c, const float *q_rot, float *kc, float *vc,
     d.out = out;
     d.error = c->error;
     d.spin_limit = c->test_lose_marks ? 2000 : 0;
-    if (!ws) {  // (asked for by the caller of this one launch)
-      d.ahead_w = c->ahead_w;
-      d.ahead_k = c->ahead_k;
-      d.ahead_n = c->ahead_n;
-      d.ahead_wgs = c->ahead_wgs;
-    }
-    c->ahead_w = nullptr;
+    if (ahead) d.ahead = *ahead;
     if (prep) {
       e = launch_prep(*prep, st, sh, total_tokens, stream);
       if (e != hipSuccess) return hip_fail(e, "prep launch");
@@ -348,7 +343,8 @@ shainet_attn_ctx *legacy_ctx() {
 
 int shainet_attn_forward_strided(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *seq_ids,
                                  const int *new_tokens, int n_seqs, const float *q, const float *k, const float *v,
-                                 long long q_stride, long long k_stride, long long v_stride, float *out, int mem);
+                                 long long q_stride, long long k_stride, long long v_stride, float *out, int mem,
+                                 const AheadRows *ahead = nullptr);
 
 extern "C" {
 
@@ -790,13 +786,14 @@ int shainet_attn_forward(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *s
 namespace {
 int forward_core(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *seq_ids, const int *new_tokens, int n_seqs,
                  const float *q, const float *k, const float *v, long long q_stride, long long k_stride,
-                 long long v_stride, float *out, int mem, const Workspace *ws);
+                 long long v_stride, float *out, int mem, const Workspace *ws, const AheadRows *ahead = nullptr);
 }
 
 int shainet_attn_forward_strided(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *seq_ids,
                                  const int *new_tokens, int n_seqs, const float *q, const float *k, const float *v,
-                                 long long q_stride, long long k_stride, long long v_stride, float *out, int mem) {
-  return forward_core(c, kc, seq_ids, new_tokens, n_seqs, q, k, v, q_stride, k_stride, v_stride, out, mem, nullptr);
+                                 long long q_stride, long long k_stride, long long v_stride, float *out, int mem,
+                                 const AheadRows *ahead) {
+  return forward_core(c, kc, seq_ids, new_tokens, n_seqs, q, k, v, q_stride, k_stride, v_stride, out, mem, nullptr, ahead);
 }
 
 namespace {
@@ -806,7 +803,7 @@ namespace {
 // large enough or come with ws.
 int forward_core(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *seq_ids, const int *new_tokens, int n_seqs,
                  const float *q, const float *k, const float *v, long long q_stride, long long k_stride,
-                 long long v_stride, float *out, int mem, const Workspace *ws) {
+                 long long v_stride, float *out, int mem, const Workspace *ws, const AheadRows *ahead) {
   if (!c || !kc || kc->ctx != c) return fail(SHAINET_HIP_ERR_ARGUMENT, "context and cache do not belong together");
   if (!kc->v) return fail(SHAINET_HIP_ERR_ARGUMENT, "this cache holds latent rows: there is no V array to attend over");
   if (int rc = refuse_while_lengths_on_device(kc, "shainet_attn_forward")) return rc;
@@ -907,7 +904,7 @@ int forward_core(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *seq_ids, 
   pa.q_rot = q_rot;
   pa.kc = kc->k;
   pa.vc = kc->v;
-  rc = run_attention(c, q_rot, kc->k, kc->v, dout, st, sh, rows, c->scale, c->stream, &pa, ws);
+  rc = run_attention(c, q_rot, kc->k, kc->v, dout, st, sh, rows, c->scale, c->stream, &pa, ws, nullptr, ahead);
   if (rc) {
     // the copies out of the pinned staging buffer may still run: the next call overwrites it
     if (mem == SHAINET_HIP_MEM_HOST) (void)hipStreamSynchronize(c->stream);
@@ -1162,15 +1159,7 @@ void shainet_attn_commit_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int
   c->last_rows = 0;
 }
 
-void shainet_attn_read_ahead(shainet_attn_ctx *c, const float *w, int k, int n, int wgs) {
-  if (!c) return;
-  c->ahead_w = w;
-  c->ahead_k = k;
-  c->ahead_n = n;
-  c->ahead_wgs = wgs;
-}
-
-int shainet_attn_finish_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, float *out) {
+int shainet_attn_finish_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, float *out, const AheadRows *ahead) {
   if (!c || !kc || kc->ctx != c || !out)
     return fail(SHAINET_HIP_ERR_ARGUMENT, "context and cache do not belong together");
   if (new_tokens < 1 || (long long)kc->len[0] + new_tokens > kc->cap)
@@ -1183,7 +1172,8 @@ int shainet_attn_finish_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int 
   st.n_new[0] = new_tokens;
   st.tok_off[1] = new_tokens;
   Shape sh = shape_of(c, kc->cap);
-  const int rc = run_attention(c, c->q_rot.p, kc->k, kc->v, out, st, sh, new_tokens, c->scale, c->stream, nullptr);
+  const int rc =
+      run_attention(c, c->q_rot.p, kc->k, kc->v, out, st, sh, new_tokens, c->scale, c->stream, nullptr, nullptr, nullptr, ahead);
   if (rc) return rc;
   kc->len[0] += new_tokens;
   c->last_rows = new_tokens;

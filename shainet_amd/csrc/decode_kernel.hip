@@ -799,14 +799,14 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
   // time at which the stream reached them: what is between two kernels stays out
   dim3 grid((unsigned)p.n_wgs), block(64 * kDecodeWaves);
   ReadAhead ah = {nullptr, 0, 0, 0};
-  if (d.ahead_w && d.ahead_wgs > 0 && !dev && !bias && !before && !after && (sh.hd == 64 || sh.hd == 128) && d.ahead_k >= 256 &&
-      (d.ahead_k & 255) == 0 && d.ahead_n > 0) {
-    ah.w = d.ahead_w;
-    ah.k = d.ahead_k;
-    ah.n = d.ahead_n;
+  if (d.ahead.w && d.ahead.wgs > 0 && !dev && !bias && !before && !after && (sh.hd == 64 || sh.hd == 128) && d.ahead.k >= 256 &&
+      (d.ahead.k & 255) == 0 && d.ahead.n > 0) {
+    ah.w = d.ahead.w;
+    ah.k = d.ahead.k;
+    ah.n = d.ahead.n;
     ah.first_wg = (p.n_wgs + 7) / 8 * 8;
-    const int most = (d.ahead_n + 3) / 4;
-    grid.x = (unsigned)(ah.first_wg + (d.ahead_wgs < most ? d.ahead_wgs : most));
+    const int most = (d.ahead.n + 3) / 4;
+    grid.x = (unsigned)(ah.first_wg + (d.ahead.wgs < most ? d.ahead.wgs : most));
   }
   // SHAINET_HIP_DECODE_NO_ROTATE: every workgroup walks its segments from their first tile (for
   // comparison); SHAINET_HIP_DECODE_ROTATE=n: starts spread over the first n tiles only

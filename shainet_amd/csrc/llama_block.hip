@@ -121,12 +121,9 @@ void set_vec(std::vector<float> &v, bool &has, const float *src, int n) {
 // no_cache: attention_full_cpu (209-243) instead: the same arithmetic from
 // position 0 over the rows of this call alone; they go through a scratch cache
 // that is empty again afterwards, and the block's own cache is not touched.
-struct AheadRows {  // the transposed gate | up weights ([2 n, k]) the block's next product but one will read
-  const float *wt;
-  int k, n;
-};
 int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out, const Fused &pre = Fused(),
                         const float *residual = nullptr, bool no_cache = false, const AheadRows *ahead = nullptr) {
+  // ahead: the transposed gate | up weights that the block's next product but one will read
   if (!l->w_qkv) return fail(SHAINET_HIP_ERR_ARGUMENT, "weights not set");
   int rc = ensure_context(l);
   if (rc) return rc;
@@ -164,14 +161,6 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
   // takes 10.2 (1024 -> 2048).
   const bool norm_apart = T == 1 && (l->has_q_norm || l->has_k_norm) && transposed_twins_wanted() &&
                           gemvt_takes(T, l->d_model, wide, pre.epilogue, pre.norm);
-  if (ahead && ahead->wt && T == 1) {
-    // One row: the attention launch leaves the memory system idle while it waits on its chain of
-    // dependent loads, and takes along workgroups that read the first rows of the gate | up
-    // weights into the L2s (8 MB: 1134 -> 1120 us per token of the 1B shape; 17 MB and more
-    // slow the attention's own chain down by more than the product gains)
-    static const int ahead_wgs = getenv("SHAINET_HIP_READ_AHEAD_WGS") ? atoi(getenv("SHAINET_HIP_READ_AHEAD_WGS")) : 128;
-    if (ahead_wgs > 0) shainet_attn_read_ahead(l->ctx, ahead->wt, ahead->k, ahead->n, ahead_wgs);
-  }
   if (!fuse_off && !norm_apart && T <= 16 && Projector::few_rows(T, l->d_model, wide, l->d_model) && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
     // few rows: bias, QK-norm, RoPE and the cache append (256-286, 332-344) happen where the
     // product's head rows are summed up; the attention kernel follows directly
@@ -182,14 +171,14 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     qkv.prep = &where;
     if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm, &where)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, nullptr, T, l->d_model, wide, stream, qkv))) return rc;
-    rc = shainet_attn_finish_prepared(l->ctx, cache, T, l->attn.p);  // 287-296
+    rc = shainet_attn_finish_prepared(l->ctx, cache, T, l->attn.p, ahead);  // 287-296
   } else {
     Fused qkv = pre;
     if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, l->qkv.p, T, l->d_model, wide, stream, qkv))) return rc;
     rc = shainet_attn_forward_strided(l->ctx, cache, nullptr, &T, 1, l->qkv.p, l->qkv.p + l->q_dim,
                                       l->qkv.p + l->q_dim + l->kv_dim, wide, wide, wide, l->attn.p,
-                                      SHAINET_HIP_MEM_DEVICE);  // 256-296
+                                      SHAINET_HIP_MEM_DEVICE, ahead);  // 256-296
   }
   if (rc) return rc;
   if (no_cache) {
@@ -513,7 +502,12 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
   if (b->mixer) {
     rc = b->mixer->forward(x, T, h, n1, x, no_cache);
   } else {
-    const AheadRows ahead = {gate.w_t, d, ff};
+    // One row: the attention launch leaves the memory system idle while it waits on its chain of
+    // dependent loads, and takes along workgroups that read the first rows of the gate | up
+    // weights into the L2s (8 MB: 1134 -> 1120 us per token of the 1B shape; 17 MB and more
+    // slow the attention's own chain down by more than the product gains)
+    static const int ahead_wgs = getenv("SHAINET_HIP_READ_AHEAD_WGS") ? atoi(getenv("SHAINET_HIP_READ_AHEAD_WGS")) : 128;
+    const AheadRows ahead = {gate.w_t, d, ff, ahead_wgs};
     rc = attn_forward_device(b->attn, x, T, h, n1, x, no_cache, &ahead);
   }
   if (rc || !ff) return rc;

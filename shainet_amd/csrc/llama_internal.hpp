@@ -8,25 +8,25 @@
 #include "../../include/shainet_hip_attn.h"
 #include "activation.hpp"
 
-// capi.hip: shainet_attn_forward with the rows of q, k and v at given strides
+namespace shainet {
+struct AheadRows;
+struct GemvPrep;
+}
+// capi.hip: shainet_attn_forward with the rows of q, k and v at given strides; ahead (nullable): what a decode
+// launch also reads
 int shainet_attn_forward_strided(shainet_attn_ctx *c, shainet_kv_cache *kc, const int *seq_ids,
                                  const int *new_tokens, int n_seqs, const float *q, const float *k, const float *v,
-                                 long long q_stride, long long k_stride, long long v_stride, float *out, int mem);
+                                 long long q_stride, long long k_stride, long long v_stride, float *out, int mem,
+                                 const shainet::AheadRows *ahead = nullptr);
 
 // capi.hip: the two halves of shainet_attn_forward for one sequence (slot 0 of the
 // cache) when the kernel that produces q | k | v also does the bias / QK-norm / RoPE /
 // append step (the kGemvQkvPrep epilogue).  begin checks the capacity and says where
 // the prepared rows go; finish runs the attention kernel over them and counts the rows
 // into the cache.  Both are asynchronous on the context's stream.
-namespace shainet {
-struct GemvPrep;
-}
 int shainet_attn_begin_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, shainet::GemvPrep *where);
-int shainet_attn_finish_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, float *out);
-// capi.hip: the next decode launch of the context (finish_prepared for a few rows) also reads, in
-// workgroups of its own, what the first `wgs` workgroups of the one-row SwiGLU product over the
-// transposed weights w ([2 n, k]) will read, into the L2s (DecodeArgs::ahead_w)
-void shainet_attn_read_ahead(shainet_attn_ctx *c, const float *w, int k, int n, int wgs);
+int shainet_attn_finish_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, float *out,
+                                 const shainet::AheadRows *ahead = nullptr);
 // capi.hip: instead of finish, when the caller's own kernel appended the rows and attended over them
 void shainet_attn_commit_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens);
 // capi.hip: the pinned host word a context's kernels report a given-up wait into; a block or a

@@ -93,6 +93,22 @@ def _block_calls_match_oracle(hip, d, H, KV, hd, ff, norm, bias, Ts):
     rm.assert_close(blk.forward_cached(x), _oracle_forward(ob, p, eps, x), ATOL, RTOL, "after clear")
 
 
+def test_block_with_new_weights_behind_steps_of_one_row(hip):
+    """A step of one row tells its attention launch which weights to read ahead.  Heads of 6 have no launch that does:
+    nothing of the request is left when the feed-forward gets other weights (and other memory) afterwards."""
+    d, H, KV, hd, ff = 1024, 8, 2, 6, 256
+    blk, ob, p, r, eps = _block_pair(hip, d, H, KV, hd, ff, 1e6, seed=29)
+    for T in (1, 1):
+        x = r.standard_normal((T, d)).astype(np.float32)
+        rm.assert_close(blk.forward_cached(x), _oracle_forward(ob, p, eps, x), ATOL, RTOL, f"T={T}")
+    for name in ("gate", "up", "down"):
+        p[name] = (0.05 * r.standard_normal(p[name].shape)).astype(np.float32)
+    blk.set_ffn(p["gate"], p["up"], p["down"])
+    for T in (3, 1, 2):
+        x = r.standard_normal((T, d)).astype(np.float32)
+        rm.assert_close(blk.forward_cached(x), _oracle_forward(ob, p, eps, x), ATOL, RTOL, f"new weights, T={T}")
+
+
 def test_block_every_small_row_count(hip):
     # 1..16 rows take the fused split GEMV (norm inside for up to 4 rows, a norm kernel first above
     # that), 17 and more the library GEMM: every count around those switches
