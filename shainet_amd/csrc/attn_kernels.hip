@@ -372,46 +372,125 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   }
 
   // Results that are not finite come from operands that are not (or from values that round to infinity as bf16):
-  // the wavefront takes its tiles again in fp32, which says which.
+  // the wavefront takes its tiles again in fp32, which says which.  8192 rows, 32 / 8 heads of 64, NaN in key 5: 4.8 ms a
+  // call against 1.6 without (key by key, one dimension at a time, it was 279).
   {
     float probe = l * 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
-    if (__any(probe != 0.f)) {
+    if (__builtin_expect(__any(probe != 0.f), 0)) {
+      // (what a lane works on is found again from its number: kept for here it would cost the loop above registers)
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const int n = tid & 31, j = (tid & 63) >> 5, my_v = min(v0 + n, VR - 1), row = my_v / g, hg = my_v - row * g, lim = S + row;
+      const long long q_at = BIAS ? (st.tok_off[s] + row) * db.q_stride + (long long)(kvh * g + hg) * hd
+                                  : ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * hd;
+      const float *bias_row = BIAS ? db.tab + (long long)(kvh * g + hg) * db.stride + (db.origin - lim) : nullptr;
       m_ref = 0.f, l = 0.f, thr = -INFINITY;
+      f32x16 sum[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+        for (int r = 0; r < 16; ++r) sum[t][r] = 0.f;
+      // Tile by tile: scores from the fp32 instruction, lane half j with d = 8 i + 4 j .. + 3 of step i, here against
+      // the running maximum; the products with V likewise where every row sees the whole tile, else key by key
+      // (what a row does not see it does not multiply by zero either).
 #pragma clang loop unroll(disable)
-      for (int kt = kt0 + gidx; kt < kt1 && kt * 32 <= wave_hi; kt += G)
-#pragma clang loop unroll(disable)
-        for (int key = kt * 32; key < kt * 32 + 32 && key <= wave_hi; ++key) {
-          if (key > lim) continue;
-          float sc = 0.f;
-#pragma clang loop unroll(disable)
-          for (int d = 0; d < hd; ++d) sc = fmaf(q_rot[q_off + d] * c, kbase[(long long)key * hd + d], sc);
-          if (BIAS && lim - key < db.reach) sc += bias_row[key];
-          if (sc > thr) {  // here the reference is the running maximum
-            const float alpha = thr == -INFINITY ? 0.f : fast_exp2(thr - sc);
-            m_ref = thr = sc;
-            l *= alpha;
+      for (int kt = kt0 + gidx; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
+        const int first = kt * 32;
+        const bool whole = first + 31 <= wave_lo;
+        const float *kr = kbase + (long long)min(first + n, L - 1) * hd + 4 * j, *qr = q_rot + q_at + 4 * j;
+        f32x16 p;
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+        for (int r = 0; r < 16; ++r) p[r] = 0.f;
+#pragma clang loop unroll(disable)
+        for (int d0 = 0; d0 < hd; d0 += 16) {
+          f32x4 kv[2], qv[2];
 #pragma unroll
-              for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+          for (int u = 0; u < 2; ++u) {
+            const int d = d0 + 8 * u;
+            const bool in = !PAD || d + 4 * j < hd;
+            kv[u] = in ? *(const f32x4 *)(kr + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+            qv[u] = in ? *(const f32x4 *)(qr + d) * c : f32x4{0.f, 0.f, 0.f, 0.f};
           }
-          const float e = sc == -INFINITY ? 0.f : fast_exp2(sc - m_ref);
-          l += 0.5f * e;  // (both lane halves of a row count every key)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) p = mfma_f32(kv[i >> 2][i & 3], qv[i >> 2][i & 3], p);
+        }
+        if (BIAS && wave_lo - (first + 31) < db.reach) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = first + 8 * (r >> 2) + 4 * j + (r & 3);
+            if (key <= lim && lim - key < db.reach) p[r] += bias_row[key];
+          }
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          if (!whole && first + 8 * (r >> 2) + 4 * j + (r & 3) > lim) p[r] = -INFINITY;
+          mx = fmaxf(mx, p[r]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        if (mx > thr) {
+          const float alpha = thr == -INFINITY ? 0.f : fast_exp2(thr - mx);
+          m_ref = thr = mx;
+          l *= alpha;
 #pragma unroll
           for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int d = NT * (8 * (r >> 2) + 4 * j + (r & 3)) + t;
-              o[t][r] = fmaf(e, vbase[(long long)key * vhd + (PAD && d >= vhd ? 0 : d)], o[t][r]);
-            }
+            for (int r = 0; r < 16; ++r) sum[t][r] *= alpha;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          p[r] = fast_exp2(p[r] - m_ref);
+          l += p[r];
+        }
+        if (whole) {
+          typedef float vrow_t __attribute__((ext_vector_type(NT)));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = first + 8 * (r >> 2) + 4 * j + (r & 3);
+            const vrow_t v = *(const vrow_t *)(vbase + (long long)key * vhd + (PAD && NT * n >= vhd ? 0 : NT * n));
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sum[t] = mfma_f32(v[t], p[r], sum[t]);
+          }
+          continue;
+        }
+#pragma clang loop unroll(disable)
+        for (int r = 0; r < 16; ++r) {
+          const float own = p[0], other = __shfl_xor(own, 32);
+#pragma unroll
+          for (int i = 0; i < 15; ++i) p[i] = p[i + 1];  // (no register is indexed by a loop counter)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int key = first + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (key > lim) continue;
+            const float e = h == j ? own : other;
+            const float *vr = vbase + (long long)key * vhd;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int w = 0; w < NT; ++w) {  // floats 4 w .. 4 w + 3 of the 4 NT columns that registers 4 q .. 4 q + 3 hold
+                const int d = NT * (8 * q + 4 * j) + 4 * w;
+                const f32x4 v = *(const f32x4 *)(vr + (PAD && d >= vhd ? 0 : d));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  const int at = 4 * w + i;
+                  sum[at % NT][4 * q + at / NT] = fmaf(e, v[i], sum[at % NT][4 * q + at / NT]);
+                }
+              }
+          }
+        }
+      }
+      // (one by one through registers of their own: as whole accumulators the loop above would move them about)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          float x = sum[t][r];
+          asm volatile("" : "+v"(x));
+          o[t][r] = x;
         }
     }
   }

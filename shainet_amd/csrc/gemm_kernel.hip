@@ -249,7 +249,8 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
     }
 
     const int row0 = m0 + wm * 32 * MB + 4 * j, col = n0 + wn * 64 + 2 * ln;
-    // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which
+    // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which (2048 rows
+    // of 2048 -> 16384 with one NaN in x: 1.3 ms against 0.65 without; one k at a time it was 13.9)
     float probe = 0.f;
 #pragma unroll
     for (int a = 0; a < MB; ++a)
@@ -264,18 +265,25 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+      // eight k a turn, four of them a lane half's (K is a multiple of 4: those behind its end are zeros on both sides)
 #pragma clang loop unroll(disable)
-      for (int k = k_begin; k < k_end; ++k) {
-        const float *wr = g.w + (long long)k * N;
-        const float w0 = wr[min(col, N - 1)], w1 = wr[min(col + 1, N - 1)];
+      for (int k0 = k_begin; k0 < k_end; k0 += 8) {
+        const int k = k0 + 4 * j;
+        const bool in = k < k_end;
+        f32x4 xv[MB];
+        f32x2 wv[4];
 #pragma unroll
         for (int a = 0; a < MB; ++a)
+          xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + (wm * MB + a) * 32 + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float xv = g.x[(long long)min(row0 + 32 * a + 8 * (r >> 2) + (r & 3), T - 1) * g.xs + k];
-            acc[a][0][r] = fmaf(xv, w0, acc[a][0][r]);
-            acc[a][1][r] = fmaf(xv, w1, acc[a][1][r]);
-          }
+        for (int i = 0; i < 4; ++i)
+          wv[i] = in ? *(const f32x2 *)(g.w + (long long)(k + i) * N + min(col, N - 2)) : f32x2{0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int a = 0; a < MB; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(xv[a][i], wv[i][b], acc[a][b]);
       }
     }
 
@@ -467,14 +475,18 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
 #pragma clang loop unroll(disable)
-    for (int k = k_begin + 16 * kg; k < k_end; k += (k & 15) == 15 ? 17 : 1) {
-      const f32x2 wv = *(const f32x2 *)(g.w + (long long)k * N + min(col, N - 2));
+    for (int k0 = k_begin + 16 * kg; k0 < k_end; k0 += (k0 & 15) ? 24 : 8) {  // (this wavefront's halves of the steps)
+      const int k = k0 + 4 * j;
+      const bool in = k < k_end;
+      const f32x4 xv = in ? *(const f32x4 *)(g.x + (long long)min(m0 + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x2 wv[4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float xv = g.x[(long long)min(row0 + 8 * (r >> 2) + (r & 3), T - 1) * g.xs + k];
-        acc[0][r] = fmaf(xv, wv.x, acc[0][r]);
-        acc[1][r] = fmaf(xv, wv.y, acc[1][r]);
-      }
+      for (int i = 0; i < 4; ++i)
+        wv[i] = in ? *(const f32x2 *)(g.w + (long long)(k + i) * N + min(col, N - 2)) : f32x2{0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[b] = mfma_f32(xv[i], wv[i][b], acc[b]);
     }
   }
   // (every wavefront is past the last step's barrier: nobody reads tiles any more)

@@ -617,46 +617,107 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
   }
 
   // Results that are not finite come from operands that are not (or from values that round to infinity as bf16): the
-  // wavefront takes its keys again in fp32, which says which.
+  // wavefront takes its keys again in fp32, which says which.  2048 rows of a layer of 16 heads of 192 and 128 dimensions, NaN in
+  // row 5: 5.5 ms with its copies against 3.2 without (key by key, one dimension at a time, it was 89).
   float probe = l * 0.f;
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
   if (wave_active && __any(probe != 0.f)) {
+    f32x16 s;
     m = -INFINITY, l = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+    // Tile by tile: scores from the fp32 instruction, lane half j with four of eight dimensions, here against the
+    // running maximum; the products with V likewise where every row sees the whole tile, else key by key (what a row
+    // does not see it does not multiply by zero either).
     const int last = min(kt1 * 32 - 1, w_hi_max);
 #pragma clang loop unroll(disable)
-    for (int key = max(kt0 * 32, w_lo_min); key <= last; ++key) {
-      if (key < my_lo || key > my_hi) continue;
-      const float *kp = a.kv + (unsigned long long)(unsigned)key * kv_stride, *rp = a.key_rot + (unsigned long long)(unsigned)key * sh.row_w;
-      float sc = 0.f;
+    for (int kt = max(kt0, w_lo_min >> 5); kt * 32 <= last; ++kt) {
+      const int first = kt * 32;
+      const bool whole = first >= w_lo_max && first + 31 <= w_hi_min;
+      const unsigned long long key_row = (unsigned)min(first + n, b_hi);
+      const float *kp = a.kv + key_row * kv_stride + h * dn, *rp = a.key_rot + key_row * sh.row_w;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
+      auto dot = [&](const float *kd, const float *qd, int dims) {
 #pragma clang loop unroll(disable)
-      for (int d = 0; d < dn; ++d) sc = fmaf(q_row[d] * a.c, kp[h * dn + d], sc);
-#pragma clang loop unroll(disable)
-      for (int d = 0; d < dr; ++d) sc = fmaf(q_row[dn + d] * a.c, rp[d], sc);
-      if (sc > m) {  // here the reference is the running maximum
-        const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - sc);
-        m = sc;
+        for (int d0 = 0; d0 < dims; d0 += 16) {
+          f32x4 kv[2], qv[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int d = d0 + 8 * u + 4 * j;
+            kv[u] = d < dims ? *(const f32x4 *)(kd + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+            qv[u] = d < dims ? *(const f32x4 *)(qd + d) * a.c : f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) s = mfma_f32(kv[i >> 2][i & 3], qv[i >> 2][i & 3], s);
+        }
+      };
+      dot(kp, q_row, dn);
+      dot(rp, q_row + dn, dr);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = first + 8 * (r >> 2) + 4 * j + (r & 3);
+        if (!whole && (key < my_lo || key > my_hi)) s[r] = -INFINITY;
+        mx = fmaxf(mx, s[r]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (mx > m) {
+        const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mx);
+        m = mx;
         l *= alpha;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
       }
-      const float e = sc == -INFINITY ? 0.f : fast_exp2(sc - m);
-      l += 0.5f * e;  // (both lane halves of a row count every key)
+      const float mref = m == -INFINITY ? 0.f : m;
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int r = 0; r < 16; ++r) {
+        s[r] = fast_exp2(s[r] - mref);
+        l += s[r];
+      }
+      if (whole) {
+        typedef float vrow_t __attribute__((ext_vector_type(NT)));
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int d = NT * (8 * (r >> 2) + 4 * j + (r & 3)) + t;
-          o[t][r] = fmaf(e, kp[sh.H * dn + h * sh.vdim + (d < sh.vdim ? d : 0)], o[t][r]);
+          const unsigned long long key = (unsigned)(first + 8 * (r >> 2) + 4 * j + (r & 3));
+          const vrow_t v = *(const vrow_t *)(v_src + key * kv_stride + (NT * n < sh.vdim ? NT * n : 0));
+#pragma unroll
+          for (int t = 0; t < NT; ++t) o[t] = mfma_f32(v[t], s[r], o[t]);
         }
+        continue;
+      }
+#pragma clang loop unroll(disable)
+      for (int r = 0; r < 16; ++r) {
+        const float own = s[0], other = __shfl_xor(own, 32);
+#pragma unroll
+        for (int i = 0; i < 15; ++i) s[i] = s[i + 1];  // (no register is indexed by a loop counter)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          const int key = first + 8 * (r >> 2) + 4 * half + (r & 3);
+          if (key < my_lo || key > my_hi) continue;
+          const float e = half == j ? own : other;
+          const float *vr = v_src + (unsigned long long)(unsigned)key * kv_stride;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int w = 0; w < NT; ++w) {  // floats 4 w .. 4 w + 3 of the 4 NT columns that registers 4 q .. 4 q + 3 hold
+              const int d = NT * (8 * q + 4 * j) + 4 * w;
+              const f32x4 v = *(const f32x4 *)(vr + (d < sh.vdim ? d : 0));
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int at = 4 * w + i;
+                o[at % NT][4 * q + at / NT] = fmaf(e, v[i], o[at % NT][4 * q + at / NT]);
+              }
+            }
+        }
+      }
     }
   }
 

@@ -8,7 +8,8 @@
 // 6/16 times per term instead of 1/2: measured against 64 bits the error is 0.8 to 0.95 of the fp32
 // instruction's for sums of 64 to 8192 terms.
 // What is not finite in an operand (or rounds to infinity: above 3.39e38) makes NaN of the sums it enters;
-// callers look for sums that are not finite and take those again in fp32.
+// callers look for sums that are not finite and take those again with the fp32 instruction, its operands straight
+// from memory: the wavefronts that meet such a value cost two to four times what they do otherwise.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -65,6 +66,11 @@ constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
 // D[m = 8 (r / 4) + 4 (l / 32) + r % 4][n = l % 32] in register r.
 __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+}
+
+// The same in fp32 over two k: lane l holds k = l / 32 of row (column) l % 32; the same D.
+__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
 }
 
 }  // namespace shainet

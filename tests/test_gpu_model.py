@@ -815,6 +815,70 @@ def test_matmul_split_tiles_keep_what_is_not_finite(hip, T):
     assert got[10, 0].item() == np.float32(3.4e38) * np.float32(0.5)
 
 
+@pytest.mark.parametrize("T,K,N", [(40, 636, 8200), (70, 20, 132), (250, 2052, 6400), (300, 2052, 1028), (1000, 4100, 4096),
+                                   (2048, 2052, 3076), (1024, 8192, 2308)])
+def test_matmul_not_finite_in_every_tile(hip, T, K, N):
+    """The same for lengths of K that are no whole steps, ragged rows and columns, and the tile of 256 x 256: NaN and
+    infinities where they belong, in the last rows and columns too, and everything else as without them."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    x = torch.randn((T, K), generator=g, device="cuda")
+    w = torch.randn((K, N), generator=g, device="cuda") / K ** 0.5
+    clean = binding.matmul(x, w)
+    x[T - 1, K - 1], x[2, 0] = float("nan"), float("inf")
+    w[K - 3, N - 1] = float("-inf")
+    got = binding.matmul(x, w)
+    want = x.double() @ w.double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(torch.where(got.isinf(), got, 0), torch.where(want.isinf(), want, 0).float())
+    fine = want.isfinite()
+    # (fp32 sums against split ones: both within K roundings of the sum of sizes)
+    assert bool(((got - clean).abs()[fine] <= 2.0 ** -23 * K ** 0.5 * 8).all())
+
+
+def _microseconds(run, wait):
+    import time
+
+    took = []
+    for _ in range(7):
+        wait()
+        t = time.perf_counter()
+        run()
+        wait()
+        took.append(time.perf_counter() - t)
+    return sorted(took[2:])[2] * 1e6
+
+
+def test_a_value_that_is_not_finite_costs_a_few_times_the_product(hip):
+    """Sums that are not finite are taken again: measured two times the product, or five times the attention."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    x, w = torch.randn((2048, 2048), device="cuda"), torch.randn((2048, 16384), device="cuda")
+    clean = _microseconds(lambda: binding.matmul(x, w), torch.cuda.synchronize)
+    x[5, 7] = float("nan")
+    assert _microseconds(lambda: binding.matmul(x, w), torch.cuda.synchronize) < 6 * clean
+    H, KV, hd, T = 32, 8, 64, 8192
+    q, k, v = (torch.randn((T, n * hd), device="cuda") for n in (H, KV, KV))
+    ctx = hip.AttnContext(H, KV, hd, max_positions=T)
+    cache = hip.KVCache(ctx, 1, T)
+
+    def attend():
+        cache.truncate(0, 0)
+        ctx.forward(cache, q, k, v, [T])
+        ctx.sync()
+
+    torch.cuda.synchronize()
+    clean = _microseconds(attend, torch.cuda.synchronize)
+    k[5, 3] = float("nan")
+    torch.cuda.synchronize()
+    assert _microseconds(attend, torch.cuda.synchronize) < 12 * clean
+
+
 @pytest.mark.parametrize("vocab", [31, 2049, 131072])
 def test_device_topk_of_crowded_and_tied_rows(hip, vocab):
     """Rows that a threshold over the threads' largest values does not thin out: all equal, a few allowed among masked
