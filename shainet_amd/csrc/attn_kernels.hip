@@ -220,8 +220,8 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       u32x4 h, m, l;
-      split_octet(f32x4{stage_v[u][0], stage_v[u][1], stage_v[u][2], stage_v[u][3]},
-                  f32x4{stage_v[u][4], stage_v[u][5], stage_v[u][6], stage_v[u][7]}, h, m, l);
+      split_octet(f32x4{stage_v[u][0], stage_v[u][1], stage_v[u][2], stage_v[u][3]} * kLift,
+                  f32x4{stage_v[u][4], stage_v[u][5], stage_v[u][6], stage_v[u][7]} * kLift, h, m, l);
       lds[v_unit[u]] = h;
       lds[v_unit[u] + U::kPartV] = m;
       lds[v_unit[u] + 2 * U::kPartV] = l;
@@ -236,6 +236,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   }
   // the row's query, scaled by scale * log2(e): scores come out in log2 units
   u32x4 qf[KS][3];
+  bool apart;  // some query of the wavefront needs its scores in fp32
   {
     f32x4 t[KS][2];
     const float *qp = q_rot + q_off + 8 * j;
@@ -249,6 +250,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       }
 #pragma unroll
     for (int i = 0; i < KS; ++i) split_octet(t[i][0] * c, t[i][1] * c, qf[i][0], qf[i][1], qf[i][2]);
+    QueryRange range;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) range.add(t[i][0]), range.add(t[i][1]);
+    apart = __any(range.apart(c));
   }
 
   // Online softmax against a reference value per virtual row instead of the running maximum: m_ref is only moved
@@ -371,16 +376,16 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     __syncthreads();  // K(sp + 1) is there, nobody reads V(sp) any more
   }
 
-  // Results that are not finite come from operands that are not (or from values that round to infinity as bf16):
-  // the wavefront takes its tiles again in fp32, which says which.  8192 rows, 32 / 8 heads of 64, NaN in key 5: 4.8 ms a
-  // call against 1.6 without (key by key, one dimension at a time, it was 279).
+  // Results that are not finite come from operands that are not (or are infinite once lifted): the wavefront takes its
+  // tiles again in fp32, which says which.  So does one whose queries ask for it.  8192 rows, 32 / 8 heads of 64, NaN
+  // in key 5: 4.6 ms a call against 1.6 without (key by key, one dimension at a time, it was 279).
   {
     float probe = l * 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
-    if (__builtin_expect(__any(probe != 0.f), 0)) {
+    if (__builtin_expect(apart || __any(probe != 0.f), 0)) {
       // (what a lane works on is found again from its number: kept for here it would cost the loop above registers)
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));
@@ -462,7 +467,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
           const float own = p[0], other = __shfl_xor(own, 32);
 #pragma unroll
           for (int i = 0; i < 15; ++i) p[i] = p[i + 1];  // (no register is indexed by a loop counter)
-#pragma unroll
+#pragma clang loop unroll(disable)
           for (int h = 0; h < 2; ++h) {
             const int key = first + 8 * (r >> 2) + 4 * h + (r & 3);
             if (key > lim) continue;
@@ -492,6 +497,9 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
           asm volatile("" : "+v"(x));
           o[t][r] = x;
         }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) o[t] *= kDropOne;
     }
   }
 

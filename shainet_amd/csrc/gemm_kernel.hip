@@ -188,7 +188,7 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         unsigned a, b, c;
-        split_pair(rw[2 * i], rw[2 * i + 1], a, b, c);
+        split_pair(rw[2 * i] * kLift, rw[2 * i + 1] * kLift, a, b, c);
         h[i] = a, m[i] = b, l[i] = c;
       }
       stage[w_unit] = h;
@@ -196,9 +196,9 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       stage[w_unit + 2 * S::kPartW] = l;
       if constexpr (NX == 1) {
         u32x2 *half = (u32x2 *)(stage + x_unit) + ((xk >> 2) & 1);
-        split_quad(rx[0], half[0], half[2 * S::kPartX], half[4 * S::kPartX]);
+        split_quad(rx[0] * kLift, half[0], half[2 * S::kPartX], half[4 * S::kPartX]);
       } else {
-        split_octet(rx[0], rx[1], h, m, l);
+        split_octet(rx[0] * kLift, rx[1] * kLift, h, m, l);
         stage[x_unit] = h;
         stage[x_unit + S::kPartX] = m;
         stage[x_unit + 2 * S::kPartX] = l;
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
     const int row0 = m0 + wm * 32 * MB + 4 * j, col = n0 + wn * 64 + 2 * ln;
     // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which (2048 rows
     // of 2048 -> 16384 with one NaN in x: 1.3 ms against 0.65 without; one k at a time it was 13.9)
-    float probe = 0.f;
+    float probe = 0.f, down = kDrop;
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
@@ -285,6 +285,7 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
 #pragma unroll
             for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(xv[a][i], wv[i][b], acc[a][b]);
       }
+      down = 1.f;
     }
 
     // A piece travels as [pair of rows][thread] float4: consecutive threads, consecutive 16 bytes.
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
     for (int a = 0; a < MB; ++a)
 #pragma unroll
       for (int r = 0; r < 8; ++r)
-        out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]};
+        out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]} * down;
     // (the thread's offset is taken afresh per tile, or the compiler computes all addresses
     // before the loops and keeps them in scratch memory)
     int in_slot = 4 * threadIdx.x;
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
   };
   auto park_x = [&](int set, int stage) {
     u32x2 *at = x_lds + 2 * stage * kStage;
-    split_quad(sx[set], at[0], at[2 * kPart], at[4 * kPart]);
+    split_quad(sx[set] * kLift, at[0], at[2 * kPart], at[4 * kPart]);
   };
 
   f32x16 acc[2];
@@ -446,7 +447,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         unsigned h, m, l;
-        split_pair(sw[set][2 * i][b], sw[set][2 * i + 1][b], h, m, l);
+        split_pair(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift, h, m, l);
         bf[0][b][i] = h, bf[1][b][i] = m, bf[2][b][i] = l;
       }
     park_x(set ^ 1, (kt & 1) ^ 1);
@@ -488,6 +489,9 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[b] = mfma_f32(xv[i], wv[i][b], acc[b]);
     }
+  } else {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[b] *= kDrop;
   }
   // (every wavefront is past the last step's barrier: nobody reads tiles any more)
   f32x4 *const merge = (f32x4 *)lds + wn * (kMerge / 2) + lane;

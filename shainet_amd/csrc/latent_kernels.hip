@@ -494,26 +494,27 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
               v_src[(unsigned long long)(unsigned)min(kt * 32 + v_row + 16 * u + (i & 3) + 8 * (i >> 2), b_hi) * kv_stride + v_off];
     }
   };
-  auto park = [&](int u, int unit, int part) {
+  auto park = [&](int u, int unit, int part, float lift) {
     u32x4 hi, mid, lo;
-    split_octet(stage[2 * u], stage[2 * u + 1], hi, mid, lo);
+    split_octet(stage[2 * u] * lift, stage[2 * u + 1] * lift, hi, mid, lo);
     lds[unit] = hi;
     lds[unit + part] = mid;
     lds[unit + 2 * part] = lo;
   };
   auto park_k = [&]() {
 #pragma unroll
-    for (int u = 0; u < KU; ++u) park(u, min(sub + 8 * u, NK - 1) * kOct + k_row, kPartK);
+    for (int u = 0; u < KU; ++u) park(u, min(sub + 8 * u, NK - 1) * kOct + k_row, kPartK, 1.f);
   };
   auto park_v = [&]() {
 #pragma unroll
-    for (int u = 0; u < VU; ++u) park(u, v_unit + 2 * u * kGroup, kPartV);
+    for (int u = 0; u < VU; ++u) park(u, v_unit + 2 * u * kGroup, kPartV, kLift);
   };
   if (kt0 < kt1) load_k(kt0);
 
   f32x4 qr[HELD ? 1 : KS][2];
   u32x4 qf[HELD ? KS : 1][3];
   const float *q_row = a.q + ((long long)my_row * sh.H + h) * (dn + dr);
+  QueryRange range;
 #pragma unroll
   for (int i = 0; i < KS; ++i) {
     f32x4 x[2];
@@ -521,13 +522,16 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
     for (int w = 0; w < 2; ++w) {
       const int d = 16 * i + 8 * j + 4 * w, e = d - dn8;
       x[w] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (d < dn || (e >= 0 && e < dr)) x[w] = *(const f32x4 *)(q_row + (d < dn ? d : dn + e)) * a.c;
+      if (d < dn || (e >= 0 && e < dr)) x[w] = *(const f32x4 *)(q_row + (d < dn ? d : dn + e));
+      range.add(x[w]);
+      x[w] *= a.c;
     }
     if constexpr (HELD)
       split_octet(x[0], x[1], qf[i][0], qf[i][1], qf[i][2]);
     else
       qr[i][0] = x[0], qr[i][1] = x[1];
   }
+  const bool apart = __any(range.apart(a.c));  // some query of the wavefront needs its scores in fp32
   f32x16 o[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -616,7 +620,7 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
     __syncthreads();
   }
 
-  // Results that are not finite come from operands that are not (or from values that round to infinity as bf16): the
+  // Results that are not finite come from operands that are not (or are infinite once lifted): the
   // wavefront takes its keys again in fp32, which says which.  2048 rows of a layer of 16 heads of 192 and 128 dimensions, NaN in
   // row 5: 5.5 ms with its copies against 3.2 without (key by key, one dimension at a time, it was 89).
   float probe = l * 0.f;
@@ -624,13 +628,19 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
-  if (wave_active && __any(probe != 0.f)) {
-    f32x16 s;
+  if (__builtin_expect(wave_active && (apart || __any(probe != 0.f)), 0)) {
+    // (what a lane works on is found again from its number: kept for here it would cost the loop above registers)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int n = tid & 31, j = (tid & 63) >> 5, my_row = min(w_row0 + n, a.T - 1);
+    const int my_hi = a.first_key + my_row, my_lo = sh.window ? max(0, my_hi - sh.window + 1) : 0;
+    const float *q_row = a.q + ((long long)my_row * sh.H + h) * (dn + dr), *v_src = a.kv + sh.H * dn + h * sh.vdim;
+    f32x16 s, sum[NT];
     m = -INFINITY, l = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+      for (int r = 0; r < 16; ++r) sum[t][r] = 0.f;
     // Tile by tile: scores from the fp32 instruction, lane half j with four of eight dimensions, here against the
     // running maximum; the products with V likewise where every row sees the whole tile, else key by key (what a row
     // does not see it does not multiply by zero either).
@@ -674,7 +684,7 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+          for (int r = 0; r < 16; ++r) sum[t][r] *= alpha;
       }
       const float mref = m == -INFINITY ? 0.f : m;
 #pragma unroll
@@ -689,7 +699,7 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
           const unsigned long long key = (unsigned)(first + 8 * (r >> 2) + 4 * j + (r & 3));
           const vrow_t v = *(const vrow_t *)(v_src + key * kv_stride + (NT * n < sh.vdim ? NT * n : 0));
 #pragma unroll
-          for (int t = 0; t < NT; ++t) o[t] = mfma_f32(v[t], s[r], o[t]);
+          for (int t = 0; t < NT; ++t) sum[t] = mfma_f32(v[t], s[r], sum[t]);
         }
         continue;
       }
@@ -698,7 +708,7 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
         const float own = s[0], other = __shfl_xor(own, 32);
 #pragma unroll
         for (int i = 0; i < 15; ++i) s[i] = s[i + 1];  // (no register is indexed by a loop counter)
-#pragma unroll
+#pragma clang loop unroll(disable)
         for (int half = 0; half < 2; ++half) {
           const int key = first + 8 * (r >> 2) + 4 * half + (r & 3);
           if (key < my_lo || key > my_hi) continue;
@@ -713,12 +723,24 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
                 const int at = 4 * w + i;
-                o[at % NT][4 * q + at / NT] = fmaf(e, v[i], o[at % NT][4 * q + at / NT]);
+                sum[at % NT][4 * q + at / NT] = fmaf(e, v[i], sum[at % NT][4 * q + at / NT]);
               }
             }
         }
       }
     }
+    // (one by one through registers of their own: as whole accumulators the loop above would move them about)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float x = sum[t][r];
+        asm volatile("" : "+v"(x));
+        o[t][r] = x;
+      }
+  } else {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) o[t] *= kDropOne;
   }
 
   l += __shfl_xor(l, 32);

@@ -493,10 +493,10 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
     u32x2 *at = (u32x2 *)(stage + (k4 >> 3) * kOctX + srow) + (k4 >> 2 & 1);
 #pragma unroll
     for (int u = 0; u < NA; ++u)
-      split_quad(sa[set][u], at[128 * u], at[128 * u + 2 * kPartX], at[128 * u + 4 * kPartX]);
+      split_quad(sa[set][u] * kLift, at[128 * u], at[128 * u + 2 * kPartX], at[128 * u + 4 * kPartX]);
     at = (u32x2 *)(stage + 3 * kPartX + (k4 >> 3) * kOctW + srow) + (k4 >> 2 & 1);
 #pragma unroll
-    for (int u = 0; u < NW; ++u) split_quad(sb[set][u], at[128 * u], at[128 * u + 2 * kPartW], at[128 * u + 4 * kPartW]);
+    for (int u = 0; u < NW; ++u) split_quad(sb[set][u] * kLift, at[128 * u], at[128 * u + 2 * kPartW], at[128 * u + 4 * kPartW]);
   };
   const int n = lane & 31, half = lane >> 5, rw = wave & 1, cw = wave >> 1;
   const int a_unit = half * kOctX + rw * 32 * MB + n, b_unit = 3 * kPartX + half * kOctW + cw * 64 + n;
@@ -576,6 +576,11 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
 #pragma unroll
           for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(xv[a][i], wv[b][i], acc[a][b]);
     }
+  } else {
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] *= kDrop;
   }
 #pragma unroll
   for (int a = 0; a < MB; ++a)

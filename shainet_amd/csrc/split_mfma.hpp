@@ -1,14 +1,18 @@
 // fp32 products on the bf16 matrix cores.  A float is the exact sum of three bf16 numbers, its value
 // rounded to bf16, the rest rounded to bf16, and the rest of that (8 + 8 + 8 mantissa bits with signs of
-// their own; a bf16 has a float's exponents).  Of the nine products of two such sums the six largest make
-// up the product to 2^-26 of itself; the three left out are at most 2^-27 of it each.  Six
+// their own).  A bf16 has a float's exponents and 16 bits less behind them, so the rests of a float below 2^-110
+// would not be whole; operands are lifted by 2^24 first, which makes every part of every float, the smallest
+// subnormal's too, a normal bf16 or zero, and results are brought down again (not the operands of scores, QueryRange,
+// nor probabilities, whose row holds one near 1).  2 to 4 % of a prompt's time; rows of x around 2^-120 had
+// an error of 3.5e-5 without, and 2e-7 with it, as rows around 1 have.  Of the nine products of two such sums
+// the six largest make up the product to 2^-24 of itself: of the three left out two can reach 2^-25 each.  Six
 // v_mfma_f32_32x32x16_bf16 of 32 cycles do what eight v_mfma_f32_32x32x2_f32 of 64 do (192 against 512
 // cycles per 32 x 32 x 16; a loop of nothing else: 1876 TFLOP/s of bf16 = 312 of fp32, against 155), they
 // leave the vector ALU free meanwhile, which the fp32 instruction does not, and round the accumulator
-// 6/16 times per term instead of 1/2: measured against 64 bits the error is 0.8 to 0.95 of the fp32
+// 6/16 times per term instead of 1/2: measured against 64 bits the error is 0.4 to 0.95 of the fp32
 // instruction's for sums of 64 to 8192 terms.
-// What is not finite in an operand (or rounds to infinity: above 3.39e38) makes NaN of the sums it enters;
-// callers look for sums that are not finite and take those again with the fp32 instruction, its operands straight
+// What is not finite in an operand (or infinite once it is lifted: from 2^104 on, and sums of products from 2^80
+// on) makes NaN or infinity of the sums it enters; callers look for sums that are not finite and take those again with the fp32 instruction, its operands straight
 // from memory: the wavefronts that meet such a value cost two to four times what they do otherwise.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -21,6 +25,31 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Operands of a product are lifted before they are split; its result, or that of one lifted operand, comes down.
+constexpr float kLift = 0x1p24f, kDrop = 0x1p-48f, kDropOne = 0x1p-24f;
+
+// Scores of attention are taken of queries and keys as they are: only their size against 1 counts, and what the
+// small ones lose is 2^-134 of the other operand at most.  It can count where a query (scaled, in log2 units) holds
+// numbers of 2^100 and more, and keys numbers below 2^-110, or the query numbers below 2^-109 (other than 0), and keys
+// very large ones: the scores of such queries are taken in fp32.
+struct QueryRange {
+  unsigned least = ~0u, most = 0u;  // of the bits of |q|, doubled; zeros lie above all in `least`
+  __device__ __forceinline__ void add(f32x4 q) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned bits = __builtin_bit_cast(unsigned, q[i]) << 1;
+      least = min(least, bits - 1u);
+      most = max(most, bits);
+    }
+  }
+  // c: what the queries are multiplied by for the scores (the multiplication itself stays with the subtractions of the
+  // split, where it is not rounded)
+  __device__ __forceinline__ bool apart(float c) const {
+    const float lo = __builtin_bit_cast(float, (least + 1u) >> 1), hi = __builtin_bit_cast(float, most >> 1);
+    return (least != ~0u && !(fabsf(lo * c) >= 0x1p-109f)) || !(fabsf(hi * c) < 0x1p100f);
+  }
+};
 
 // two floats rounded to bf16, the first in the low half
 __device__ __forceinline__ unsigned pack_bf16(float a, float b) {

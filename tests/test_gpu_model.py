@@ -839,6 +839,26 @@ def test_matmul_not_finite_in_every_tile(hip, T, K, N):
     assert bool(((got - clean).abs()[fine] <= 2.0 ** -23 * K ** 0.5 * 8).all())
 
 
+@pytest.mark.parametrize("T,K,N", [(40, 640, 1024), (100, 2052, 6400), (300, 2052, 1028), (1000, 4100, 4096), (2048, 2048, 3072)])
+def test_matmul_of_very_small_operands(hip, T, K, N):
+    """Rows of x and columns of W anywhere in a float's range, subnormal numbers among them, lose no bits.  The bound is
+    about twice the error of such sums of numbers around 1 (4.9e-7 of their norm for the longest in one accumulator)."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn((T, K), generator=g, device="cuda")
+    w = torch.randn((K, N), generator=g, device="cuda")
+    for small in (-112, -120, -135, -147):
+        up = min(-small, 100)  # (2^104 and above take another path)
+        for a, b in ((small, up), (up, small)):
+            xs, ws = x * 2.0 ** a, w * 2.0 ** b
+            want = xs.double() @ ws.double()
+            rel = ((binding.matmul(xs, ws).double() - want).norm(dim=1) / want.norm(dim=1)).max()
+            assert float(rel) <= 1.2e-6, (a, b, float(rel))
+
+
 def _microseconds(run, wait):
     import time
 

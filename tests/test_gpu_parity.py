@@ -953,3 +953,39 @@ def test_prefill_keeps_what_is_not_finite(hip, hd, KV, T, cached):
     np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
     fine = np.isfinite(want)
     assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-3 * np.abs(want[fine]))
+
+
+@pytest.mark.parametrize("hd,KV,T,cached", [(64, 2, 300, 0), (128, 2, 70, 100), (96, 4, 40, 33), (128, 8, 700, 0), (64, 8, 2300, 0)])
+@pytest.mark.parametrize("q_by,k_by,v_by,pair", [(1.0, 1.0, 2.0 ** -124, 0), (1.0, 1.0, 2.0 ** -135, 0), (2.0 ** 120, 2.0 ** -120, 1.0, 0),
+                                                 (2.0 ** -124, 2.0 ** 124, 1.0, 0), (1.0, 1.0, 1.0, -122), (1.0, 1.0, 1.0, 122)])
+def test_prefill_of_very_small_operands(hip, hd, KV, T, cached, q_by, k_by, v_by, pair):
+    """Queries, keys and values far below 1 lose no bits: a tenth of the bar of the other tests, relative to the size of the
+    values, and the rounding of results to a subnormal number.  pair: the query's first rotated pair is 2^pair of the
+    others, the keys' the other way round."""
+    import torch
+
+    H, S = 2 * KV, cached + T
+    g = torch.Generator(device="cuda").manual_seed(hd + T)
+    q, k, v = (torch.randn((T, n * hd), generator=g, device="cuda") * by for n, by in ((H, q_by), (KV, k_by), (KV, v_by)))
+    kc, vc = (torch.randn((KV, max(cached, 1), hd), generator=g, device="cuda") * by for by in (k_by, v_by))
+    for d in (0, hd // 2):
+        q.view(T, H, hd)[..., d] *= 2.0 ** pair
+        k.view(T, KV, hd)[..., d] *= 2.0 ** -pair
+        kc[..., d] *= 2.0 ** -pair
+    ctx = hip.AttnContext(H, KV, hd, max_positions=S)
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, S)
+    if cached:
+        cache.fill(0, kc, vc)
+    ctx.sync()
+    got = ctx.forward(cache, q, k, v, [T])
+    ctx.sync()
+    got = got.cpu().numpy().reshape(T, H, hd).astype(np.float64) / v_by
+    qr = ctx.last_q_rot(T).astype(np.float64).reshape(T, H, hd)
+    for h in range(H):
+        kr, vr = (a.astype(np.float64) for a in cache.read(0, h // 2, 0, S))
+        s = qr[:, h] @ kr.T / np.sqrt(hd)
+        s[np.arange(S)[None] > cached + np.arange(T)[:, None]] = -np.inf
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p / p.sum(-1, keepdims=True)) @ (vr / v_by)
+        assert np.abs(got[:, h] - want).max() <= 1e-5 + 2.0 ** -149 / v_by, h

@@ -220,6 +220,41 @@ def test_expanded_keeps_what_is_not_finite_to_the_rows_that_see_it(hip, tmp_path
     close(got[~sees], want[~sees])
 
 
+@pytest.mark.parametrize("name", ["even", "tall", "wide", "vast"])
+def test_expanded_of_very_small_values(hip, tmp_path, monkeypatch, name):
+    """Values around 2^-124 lose no bits; the output matrix brings them back to the size of the rows, 2^-22."""
+    monkeypatch.setenv("SHAINET_HIP_LATENT_PATH", "expanded")
+
+    def edit(w):
+        small = w["l0.mix.uv"] * np.float32(2.0 ** -124)
+        w["l0.mix.uv"] = (small.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)  # (what a bfloat16 holds)
+        w["l0.mix.o"] = w["l0.mix.o"] * np.float32(2.0 ** 101)
+
+    p = Pair(hip, tmp_path, geometry(name, mlp=False), edit=edit)
+    x = (2.0 ** -22 * np.random.default_rng(12).standard_normal((200, p.cfg["width"]))).astype(np.float32)
+    close(p.model.blocks[0].forward_cached(x), p.layer(0, x), 2e-5)
+
+
+@pytest.mark.parametrize("q_by", [-124, 115])
+@pytest.mark.parametrize("name", ["even", "wide", "vast"])
+def test_expanded_of_very_small_and_very_large_queries(hip, tmp_path, monkeypatch, name, q_by):
+    """Queries around 2^q_by and unrotated keys as large as those are small, or the other way round."""
+    monkeypatch.setenv("SHAINET_HIP_LATENT_PATH", "expanded")
+    holds = lambda a: (a.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)  # what a bfloat16 does
+
+    def edit(w):
+        m = GEOMETRIES[name]["m"]
+        q = w["l0.mix.uq"].reshape(m["heads"], m["dim"] + m["rot_dim"], -1).copy()
+        q[:, :m["dim"]] *= np.float32(2.0 ** q_by)
+        q[:, m["dim"]:] *= np.float32(2.0 ** min(q_by, 0))
+        w["l0.mix.uq"] = holds(q.reshape(w["l0.mix.uq"].shape))
+        w["l0.mix.uk"] = holds(w["l0.mix.uk"] * np.float32(2.0 ** -q_by))
+
+    p = Pair(hip, tmp_path, geometry(name, mlp=False), edit=edit)
+    x = np.random.default_rng(12).standard_normal((200, p.cfg["width"])).astype(np.float32)
+    close(p.model.blocks[0].forward_cached(x), p.layer(0, x), 2e-5)
+
+
 @pytest.mark.parametrize("path", ["absorbed", "expanded"])
 def test_sink(hip, tmp_path, monkeypatch, path):
     """Sinks that take nearly everything, about half and nothing; the first position sees one key only."""

@@ -352,6 +352,21 @@ def test_experts_keep_rows_apart(hip, tmp_path, name):
     assert np.isnan(got[384:]).all()
 
 
+def test_experts_of_very_small_hidden_rows(hip, tmp_path):
+    """Hidden rows around 2^-124 between an up matrix that small and a down matrix that large lose no bits."""
+    def edit(w):
+        for n in w:
+            if n.endswith("mlp.shared.up") or ".mlp.e" in n and n.endswith(".up"):
+                w[n] = zm.exact(w[n] * np.float32(2.0 ** -124))
+            if n.endswith("mlp.shared.down") or ".mlp.e" in n and n.endswith(".down"):
+                w[n] = w[n] * np.float32(2.0 ** 98)
+
+    cfg = zm.config([zm.layer(zm.hgrn2(heads=1, dim=4, vdim=4), zm.moe(experts=6, identity=0, top=2, groups=2, keep=1))], eps=1e-25)
+    p = Pair(hip, tmp_path, cfg, seed=5, edit=edit)
+    x = np.random.default_rng(6).standard_normal((150, cfg["width"])).astype(np.float32)
+    close(p.model.blocks[0].forward_cached(x), p.layer(0, x), 2e-5)
+
+
 def test_optional_parts_left_out(hip, tmp_path):
     """No groups, scale, identity or shared expert in the configuration; a layer without a feed-forward."""
     cfg = zm.config([zm.layer(zm.attention(), zm.moe(experts=5, identity=0, top=2, groups=1, keep=1, scale=1.0, shared=0)),
