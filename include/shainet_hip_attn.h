@@ -279,6 +279,12 @@ int shainet_llama_attn_forward_full(shainet_llama_attn *layer, const float *x, i
  * the next call on that stream (SHAINET_HIP_ERR_RUNTIME), which then does nothing else. */
 int shainet_hip_matmul_f32(const float *x, long long x_stride, const float *w, const float *res, float *y, int rows,
                            int k, int n, void *stream);
+/* The MFMA kernel's part of that for dense rows, without launching anything; needs no device.  plan[0] the tiles: 0 = one
+ * thread per element (k or n no multiple of 4), 1 = few rows, 2 = both operands through LDS; plan[1], plan[2] rows and
+ * columns of a tile; plan[3] workgroups; plan[4] pieces a tile's sum is cut into for a second kernel that adds them
+ * (1 = none); plan[5] 1 = workgroups share tiles and the one that ends a tile waits for the others' parts; plan[6] 1 = k
+ * is no whole number of steps.  Lets a test name the kernel instantiation it covers.  No counterpart in the reference. */
+int shainet_hip_describe_matmul(int rows, int k, int n, int plan[7]);
 
 /* ---- the whole block ---------------------------------------------------------
  *

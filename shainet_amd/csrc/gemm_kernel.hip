@@ -592,6 +592,19 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
 
 }  // namespace
 
+static int tile_rows(const GemmPlan &p) { return (p.few ? 32 : 64) * p.mb; }
+static int tile_columns(const GemmPlan &p) { return 64 * p.wn; }
+
+void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
+  plan[0] = !p.mfma ? 0 : p.few ? 1 : 2;
+  plan[1] = p.mfma ? tile_rows(p) : 1;
+  plan[2] = p.mfma ? tile_columns(p) : 1;
+  plan[3] = p.workgroups;
+  plan[4] = p.pieces > 1 ? p.pieces : 1;
+  plan[5] = p.flag_words && p.quota % p.steps != 0;
+  plan[6] = p.mfma && K % (p.few ? kFewStep : TK) != 0;
+}
+
 GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
   GemmPlan p = {};
   // (the kernel addresses the rows of x by 32-bit byte offsets from a base that moves along K)
@@ -599,7 +612,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
            (long long)T * x_stride * 4 < 0xffffffffLL && (long long)TK * N * 4 < 0xffffffffLL;
   p.steps = (K + TK - 1) / TK;
   choose_tile(p, T, K, N);
-  const int TN = 64 * p.wn, TM = (p.few ? 32 : 64) * p.mb;
+  const int TN = tile_columns(p), TM = tile_rows(p);
   if (p.few) p.steps = (K + kFewStep - 1) / kFewStep;
   p.tiles_m = (T + TM - 1) / TM;
   p.tiles_n = (N + TN - 1) / TN;

@@ -21,6 +21,7 @@ struct GemmPlan {
   size_t flag_words;      // words, zero before the first launch (the kernel leaves them zero), that mark pieces complete
 };
 GemmPlan plan_gemm(int T, int K, int N, long long x_stride);
+void describe_gemm(const GemmPlan &p, int K, int plan[7]);  // shainet_hip_describe_matmul
 // Device pointers, 16-byte aligned for the MFMA kernel; rows of x are x_stride floats apart, y and
 // res are dense [T, N]; res nullable (y = res + x W; res == y is allowed);
 // bias [N] nullable (y = act(x W + bias), before res is added).  partials, flags:

@@ -280,6 +280,13 @@ std::mutex g_matmul_lock;
 std::map<hipStream_t, shainet::Projector> g_matmul;
 }  // namespace
 
+extern "C" int shainet_hip_describe_matmul(int rows, int k, int n, int plan[7]) {
+  using namespace shainet;
+  if (!plan || rows < 1 || k < 1 || n < 1) return llama_fail(SHAINET_HIP_ERR_ARGUMENT, "invalid matmul arguments");
+  describe_gemm(plan_gemm(rows, k, n, k), k, plan);
+  return SHAINET_HIP_OK;
+}
+
 extern "C" int shainet_hip_matmul_f32(const float *x, long long x_stride, const float *w, const float *res, float *y,
                                       int rows, int k, int n, void *stream) {
   using namespace shainet;

@@ -147,6 +147,7 @@ _SIGNATURES = {
     "shainet_llama_model_repetition_penalty": (C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.c_double]),
     "shainet_llama_model_topk": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_int), _f32p, C.POINTER(C.c_int)]),
     "shainet_llama_model_sample": (C.c_int, [C.c_void_p, C.c_int, C.c_double, C.c_double, C.POINTER(C.c_int)]),
+    "shainet_hip_describe_matmul": (C.c_int, [C.c_int, C.c_int, C.c_int, _i32p]),
     "shainet_hip_matmul_f32": (C.c_int, [C.c_void_p, C.c_longlong, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int,
                                          C.c_int, C.c_void_p]),
     "shainet_hip_stream_copy_f32": (C.c_int, [C.c_void_p, C.c_void_p, C.c_longlong, C.c_int, C.c_void_p]),
@@ -289,6 +290,15 @@ def describe_plan(num_heads, num_kv_heads, head_dim, start_pos, new_tokens):
     d = dict(zip(PLAN_FIELDS, (int(v) for v in plan)))
     d["padded"] = d["head_dim"] != head_dim   # the tiles are laid out for a larger head_dim than the data's
     return d
+
+
+def describe_matmul(rows, k, n):
+    """What the MFMA product of [rows, k] and [k, n] runs as; nothing is launched and no device is needed."""
+    plan = (C.c_int * 7)()
+    _check(lib().shainet_hip_describe_matmul(rows, k, n, plan))
+    kind, tm, tn, workgroups, pieces, waits, ragged = (int(v) for v in plan)
+    return {"kind": ("plain", "few", "tiles")[kind], "tile": (tm, tn), "workgroups": workgroups, "pieces": pieces,
+            "waits": bool(waits), "ragged_k": bool(ragged)}
 
 
 def matmul(x, w, res=None, out=None, stream=None):

@@ -30,8 +30,7 @@ CASES = [
     ("hd32_prefill_t1024", 32, 8, 32, True, 0, 1024, (64, True, 2, 0, True)),
 ]
 
-# The prefill shapes of the benchmark configurations (BASELINE.json configs[3] and configs[4](a)):
-# (H, KV, head_dim, cached positions, new rows).
+# The prefill shapes of the benchmark configurations: (H, KV, head_dim, cached positions, new rows).
 BASELINE_PREFILL_SHAPES = [
     (32, 8, 64, 0, 2048),
     (32, 8, 64, 0, 8192),
@@ -43,3 +42,34 @@ def instantiation(plan):
     """The kernel instantiation of a plan dict from shainet_amd.describe_plan."""
     inst = (plan["head_dim"], plan["key_chunks"] > 1, plan["groups"], plan["turns"])
     return inst + (True,) if plan.get("padded") else inst
+
+
+# Products, each with what the planner runs it as: rows, k, n, (kind, tile, cut into pieces, tiles shared by waiting, k no
+# whole number of steps).  Ragged rows and columns where an instantiation is reached with them.
+MATMULS = [
+    (40, 96, 132, ("few", (32, 128), False, False, False)),
+    (33, 100, 260, ("few", (32, 128), False, False, True)),
+    (96, 8192, 260, ("few", (32, 128), True, False, False)),
+    (70, 2052, 6400, ("few", (32, 128), True, False, True)),
+    (200, 512, 16384, ("tiles", (128, 128), False, True, False)),
+    (200, 516, 16384, ("tiles", (128, 128), False, True, True)),
+    (100, 4096, 3076, ("tiles", (128, 128), True, False, False)),
+    (100, 2052, 6400, ("tiles", (128, 128), True, False, True)),
+    (1000, 1040, 8192, ("tiles", (128, 256), False, False, False)),
+    (1000, 1044, 8192, ("tiles", (128, 256), False, False, True)),
+    (1100, 640, 8200, ("tiles", (128, 256), False, True, False)),
+    (1100, 644, 8200, ("tiles", (128, 256), False, True, True)),
+    (1000, 2048, 2308, ("tiles", (128, 256), True, False, False)),
+    (300, 2052, 1028, ("tiles", (128, 256), True, False, True)),
+    (2000, 1040, 16384, ("tiles", (256, 256), False, False, False)),
+    (2000, 1044, 16384, ("tiles", (256, 256), False, False, True)),
+    (3000, 1040, 8200, ("tiles", (256, 256), False, True, False)),
+    (3000, 1044, 8200, ("tiles", (256, 256), False, True, True)),
+    (1000, 8192, 2308, ("tiles", (256, 256), True, False, False)),
+    (1000, 4100, 4092, ("tiles", (256, 256), True, False, True)),
+]
+
+
+def matmul_instantiation(plan):
+    """The kernel instantiation of a dict from shainet_amd.hip.describe_matmul."""
+    return plan["kind"], plan["tile"], plan["pieces"] > 1, plan["waits"], plan["ragged_k"]

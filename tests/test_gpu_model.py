@@ -10,6 +10,7 @@ import os
 import numpy as np
 import pytest
 
+import prefill_cases as pc
 import refmath as rm
 import tinyllama
 from oracle import oracle as orc
@@ -772,7 +773,7 @@ def test_load_llama_bf16_f16_sharded_qwen_style(hip, tmp_path):
     (96, 8192, 256), (129, 36, 128), (256, 528, 260),             # tiles, pieces
     (100, 2052, 6400), (256, 2048, 3076),                         # 128 x 128
     (257, 16, 256), (300, 2052, 1028), (640, 512, 512),           # 128 x 256: whole and ragged, one step, pieces
-    (1024, 2048, 2308), (1000, 1040, 8192),                       # 256 x 256: pieces and the kernel that adds them; whole tiles
+    (1024, 2048, 2308), (1000, 1040, 8192),                       # 128 x 256: pieces and the kernel that adds them; whole tiles
 ])
 def test_matmul_split_tiles(hip, T, K, N):
     """Each tile of the product over split operands.  A sum is rounded 6 K / 16 times, each time by at most 2^-24 of
@@ -792,6 +793,28 @@ def test_matmul_split_tiles(hip, T, K, N):
     off = (got.double() - want).abs()
     assert bool((off <= 2.0 ** -24 * (6 * K / 16 + 18) * size).all()), float((off / size).max())
     assert torch.equal(got, binding.matmul(x, w, res))
+
+
+@pytest.mark.parametrize("T,K,N,inst", pc.MATMULS)
+def test_matmul_keeps_every_part(hip, T, K, N, inst):
+    """Every instantiation, rows of x with a single value each: a sum is one product, of which the smallest of the six
+    partial products is up to 2^-17, and every one of them more than the bound.  The parts left out are under 2^-24 of the
+    product; three of the six are as large as that or larger when they are added, which rounds by 2^-24 at most each."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    assert pc.matmul_instantiation(binding.describe_matmul(T, K, N)) == inst
+    g = torch.Generator(device="cuda").manual_seed(T + K + N)
+    at = torch.randint(0, K, (T,), generator=g, device="cuda")
+    at[:2] = torch.tensor([0, K - 1])
+    value = torch.randn((T,), generator=g, device="cuda")
+    x = torch.zeros((T, K), device="cuda")
+    x[torch.arange(T, device="cuda"), at] = value
+    w = torch.randn((K, N), generator=g, device="cuda")
+    want = w[at].double() * value.double()[:, None]
+    off = (binding.matmul(x, w).double() - want).abs()
+    assert bool((off <= 2.0 ** -22 * want.abs()).all()), float((off / want.abs()).nan_to_num().max())
 
 
 @pytest.mark.parametrize("T", [40, 250, 300, 1100])

@@ -87,3 +87,15 @@ def test_decode_spans_end_with_the_pairs():
     assert split([16 * 5] * 16) == (128, 5)
     assert split([16 * 9] * 16) == (231, 5)  # two spans each would meet on four XCDs: 1152 tiles end to end
     assert split([64], 300, 256) == (240, 5)  # more pairs than workgroups: end to end
+
+
+def test_products_run_as_their_cases_say():
+    plan = sa.hip.describe_matmul
+    for T, K, N, inst in pc.MATMULS:
+        assert pc.matmul_instantiation(plan(T, K, N)) == inst, (T, K, N, plan(T, K, N))
+    seen = set()
+    for T, K, N in itertools.product((17, 40, 96, 97, 128, 200, 256, 257, 512, 777, 1024, 1300, 2048, 2304, 3000, 4096),
+                                     (4, 32, 100, 512, 1024, 2048, 2052, 4100, 8192), (4, 132, 1024, 2308, 3072, 8192, 16384)):
+        seen.add(pc.matmul_instantiation(plan(T, K, N)))
+    assert seen <= {inst for *_, inst in pc.MATMULS}, sorted(seen - {inst for *_, inst in pc.MATMULS})
+    assert plan(100, 6, 8)["kind"] == plan(100, 8, 6)["kind"] == "plain"
