@@ -574,7 +574,11 @@ int slots_of(int wn) { return wn == 4 ? 256 : 512; }
 //   2048                               148 | 100 | 717 | 372 | 187  143 | 99 | 674 | 346 | 181  144 | 100 | 619 | 323 | 164
 // A low tile wastes least on few rows, and reads small weights again from the L2 for little: up to 96 rows always, up to
 // 256 where the higher tile would be a fifth padding or the weights are small.
-// The largest needs long runs: at least 36 steps a workgroup, and no tile that two of them share by waiting.
+// The largest needs long runs: at least 36 steps a workgroup.  Less than a round of its tiles is cut into pieces for the
+// second kernel (never one shared by waiting); of more than a round the last one must be empty or at least half
+// full, or the waits for shared tiles cost more than the tile saves (2048 -> 8192, 128 x 256 | 256 x 256, us: 288 tiles
+// of 256 x 256 433 | 503, 320 421 | 474, 352 459 | 502, 384 496 | 468, 448 576 | 548, 544 744 | 785, 576 742 | 757,
+// 640 824 | 759, 704 909 | 846; 4096 -> 8192: 320 802 | 896, 384 973 | 887; 8192 -> 8192: 288 1671 | 1873).
 void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 2;
   const long long weights = (long long)K * N, rows1 = (T + 31) / 32 * 32LL, rows2 = (T + 127) / 128 * 128LL;
@@ -587,7 +591,9 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 4;
   const long long rows4 = (T + 255) / 256 * 256LL;
   const long long tiles = rows4 / 256 * ((N + 255) / 256), run = tiles * p.steps / slots_of(4);
-  if (rows4 * 100 <= rows2 * 115 && run >= 36 && (tiles >= slots_of(4) || 2 * run < p.steps)) p.mb = 4;
+  const long long last = tiles % slots_of(4);
+  const bool fills = tiles < slots_of(4) ? 2 * run < p.steps : last == 0 || 2 * last >= slots_of(4);
+  if (rows4 * 100 <= rows2 * 115 && run >= 36 && fills) p.mb = 4;
 }
 
 }  // namespace

@@ -99,3 +99,12 @@ def test_products_run_as_their_cases_say():
         seen.add(pc.matmul_instantiation(plan(T, K, N)))
     assert seen <= {inst for *_, inst in pc.MATMULS}, sorted(seen - {inst for *_, inst in pc.MATMULS})
     assert plan(100, 6, 8)["kind"] == plan(100, 8, 6)["kind"] == "plain"
+
+
+def test_large_tiles_fill_their_last_round():
+    # more than a round of 256 tiles of 256 x 256: the last round is empty or at least half full
+    for rows in range(2049, 8193, 256):
+        tiles = -(-rows // 256) * 32
+        plan = sa.hip.describe_matmul(rows, 2048, 8192)
+        large = tiles >= 256 and (tiles % 256 == 0 or tiles % 256 >= 128)
+        assert (plan["tile"] == (256, 256)) == (large and -(-rows // 256) * 256 * 100 <= -(-rows // 128) * 128 * 115), (rows, plan)
