@@ -951,15 +951,19 @@ bool plan_latent_expanded(const LatentShape &sh, int T, int start_row, LatentExp
   p.partial_floats = p.splits > 1 ? (size_t)blocks * p.splits * 128 * (p.nt * 32 + 2) : 0;
   // Multiply-adds: per (row, key, head) this form's and the absorbed form's, whose kernel reaches about half
   // this one's rate; and the products, here of every key row and at twice the rate (the library's), there of the new
-  // rows alone.  A few rows behind many keys are the absorbed form's: 20 rows of 16 heads of 192 and
-  // 128 dimensions behind 500 (3000) keys 614 us (725) a pass of three layers against 671 (918), 40 rows 733 (950)
-  // against 720 (969), 64 rows 872 (1265) against 726 (986); and in front of none, 17 rows 636 against 577, 64
-  // rows 845 against 614.
+  // rows alone.  A few rows behind many keys are the absorbed form's, whose tiles of columns hold 32 rows (16 heads) as
+  // cheaply as 17.  A pass of three layers, 16 heads of 96 and 64 | 192 and 128 dimensions, us, absorbed : expanded:
+  //   keys in front   17 rows               32 rows               36 rows               48 rows
+  //        40      387:364 | 605:582     410:371 | 664:602     470:395 | 738:645     474:401 | 785:657
+  //       100      402:389 | 612:620     433:399 | 676:644     474:417 | 747:689     479:423 | 794:691
+  //       200      412:415 | 620:664     436:419 | 677:658     491:433 | 758:697     505:446 | 794:704
+  //       500      430:478 | 635:724     461:480 | 706:738     509:494 | 775:778     519:496 | 826:777
+  //      3000      426:510 | 784:964     488:508 | 893:982     530:526 | 1027:1030   560:530 | 1172:1040
   const double pairs = (double)T * (sh.window && sh.window < p.key_rows ? sh.window : p.key_rows);
   const double product = (double)sh.kv_rank * sh.H * (sh.dim + sh.vdim);
   const double here = pairs * sh.H * (8 * p.nk + 32 * p.nt) + 0.5 * p.key_rows * product;
   const double there = 2.0 * pairs * sh.H * (sh.row_w + sh.kv_rank) + T * product;
-  p.pays = T > 16 && (T >= 32 || p.key_rows <= 2 * T) && here < there;
+  p.pays = T > 16 && (T > 32 || p.key_rows <= 160) && here < there;
   return true;
 }
 
