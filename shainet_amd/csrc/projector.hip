@@ -161,9 +161,11 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
       return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("gemv launch: ") + hipGetErrorString(e));
     return SHAINET_HIP_OK;
   }
-  // (an epilogue that only it has, or rows of x that the MFMA product cannot load, keep the split GEMV, too)
+  // (an epilogue that only it has, or rows that the MFMA product cannot load or store 16 bytes at a time, keep the
+  // split GEMV, too: 8 rows a float off 16 bytes, through a block 2048 wide with a feed-forward of 4096, take 127 us, with
+  // a thread per element 564, on 16 bytes 106)
   const bool gemv = f.epilogue == kGemvQkvPrep || f.any_few_rows || few_rows(T, K, swiglu ? 2 * N : N, x_stride) ||
-                    (((uintptr_t)x | (uintptr_t)w) & 15);
+                    (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)f.res | (uintptr_t)f.bias) & 15);
   if (T <= 16 && (N & 3) == 0 && gemv) {
     const float *xin = x;
     long long xs = x_stride;

@@ -337,6 +337,23 @@ def test_block_device_pointers_match_host_pointers(hip):
     assert blk.cache_len == 5
 
 
+def test_block_device_rows_off_by_a_float(hip):
+    """Device rows that do not lie on 16 bytes (x is the residual of the output projection, too): the same results, by
+    the split GEMV for a few rows, not by a thread per element."""
+    import torch
+
+    d, T = 2048, 8
+    blk, ob, p, r, eps = _block_pair(hip, d, 16, 4, 128, 4096, 1e4, seed=5, wscale=0.02)
+    x = r.standard_normal((T, d)).astype(np.float32)
+    apart = torch.empty(T * d + 1, device="cuda")[1:].view(T, d)
+    apart.copy_(torch.from_numpy(x))
+    whole = torch.from_numpy(x).cuda()
+    rm.assert_close(blk.forward(apart).cpu().numpy(), ob.forward(x, p["norm1"], p["norm2"], eps, p["gate"], p["up"], p["down"], False),
+                    ATOL, RTOL, "off by a float")
+    on = _microseconds(lambda: blk.forward(whole), torch.cuda.synchronize)
+    assert _microseconds(lambda: blk.forward(apart), torch.cuda.synchronize) < 3 * on
+
+
 def test_block_argument_errors(hip):
     blk = hip.LlamaBlock(64, 8, 128)
     with pytest.raises(hip.ArgumentError):
