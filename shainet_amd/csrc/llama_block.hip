@@ -151,7 +151,7 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
   // norm, or with none, gets its copy made again)
   auto take_transposed = [&](Fused &f) {
     const float *gamma = f.norm == kNormRms ? f.gamma : nullptr;
-    if (gamma != l->w_qkv_t_gamma) l->w_qkv_t_stale = true;
+    if (l->w_qkv_t && gamma != l->w_qkv_t_gamma) l->w_qkv_t_stale = true;
     f.w_t = transposed_twin(&l->w_qkv_t, &l->w_qkv_t_stale, l->w_qkv, l->d_model, wide, stream, gamma);
     l->w_qkv_t_gamma = f.w_t ? gamma : nullptr;
     f.w_t_has_gamma = f.w_t && gamma;
@@ -159,8 +159,12 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
   // One row with QK-norm: the sum of squares needs the whole head, which the product over transposed weights does not
   // hold in one place; it and the prep kernel behind it take 4.8 + 4.3 us where the split product with prep inside
   // takes 10.2 (1024 -> 2048).
-  const bool norm_apart = T == 1 && (l->has_q_norm || l->has_k_norm) && transposed_twins_wanted() &&
-                          gemvt_takes(T, l->d_model, wide, pre.epilogue, pre.norm);
+  bool norm_apart = T == 1 && (l->has_q_norm || l->has_k_norm) && gemvt_takes(T, l->d_model, wide, pre.epilogue, pre.norm);
+  if (norm_apart) {
+    Fused qkv = pre;
+    take_transposed(qkv);
+    norm_apart = qkv.w_t != nullptr;
+  }
   if (!fuse_off && !norm_apart && T <= 16 && Projector::few_rows(T, l->d_model, wide, l->d_model) && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
     // few rows: bias, QK-norm, RoPE and the cache append (256-286, 332-344) happen where the
     // product's head rows are summed up; the attention kernel follows directly

@@ -71,18 +71,34 @@ bool transposed_twins_wanted() {
   return wanted;
 }
 
+// Whether a copy of `bytes` leaves enough device memory to what cannot do without (caches that grow, scratch): an eighth
+// of the device's (36 GB), or SHAINET_HIP_TWIN_RESERVE_MB.
+static bool twin_leaves_room(size_t bytes) {
+  size_t free_bytes = 0, total = 0;
+  if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  static const char *const knob = getenv("SHAINET_HIP_TWIN_RESERVE_MB");
+  const size_t reserve = knob ? (size_t)strtoull(knob, nullptr, 10) << 20 : total / 8;
+  return free_bytes >= bytes && free_bytes - bytes >= reserve;
+}
+
 // *twin = src transposed (src: [rows, cols] on the device), allocated on first use.  Returns the
-// twin, or null when there is no memory for it (the caller then goes without).
+// twin, or null when there is no memory for it (the caller then goes without; *stale false without a twin: not asked
+// again until there are new weights).
 const float *transposed_twin(float **twin, bool *stale, const float *src, int rows, int cols, hipStream_t stream,
                              const float *row_scale) {
   if (!transposed_twins_wanted() || !src) return nullptr;
   if (!*twin) {
-    if (hipMalloc((void **)twin, (size_t)rows * cols * sizeof(float)) != hipSuccess) {
+    if (!*stale) return nullptr;
+    const size_t bytes = (size_t)rows * cols * sizeof(float);
+    if (!twin_leaves_room(bytes) || hipMalloc((void **)twin, bytes) != hipSuccess) {
       (void)hipGetLastError();
       *twin = nullptr;
+      *stale = false;
       return nullptr;
     }
-    *stale = true;
   }
   if (*stale) {
     // (waited for, once per set of weights: the copy may next be read on another stream)
