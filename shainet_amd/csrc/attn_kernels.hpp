@@ -115,6 +115,7 @@ struct DecodeDevicePlan {
   SpanTable spans;
   int total_tiles;
   int align;
+  unsigned align_by;  // 2^32 / align, rounded up; 0 where align is 1
   int skip;  // a sequence would outgrow the cache or the cos/sin table: the step's kernels do nothing
 };
 constexpr int kDevicePlanWorkgroups = 256;

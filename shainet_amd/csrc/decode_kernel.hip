@@ -143,6 +143,13 @@ __device__ __forceinline__ int workgroup_of_tile(int t, int tiles_per_wg, const 
 __host__ __device__ inline int padded_tiles(int n_s, int align) {
   return align > 1 ? (n_s + align - 1) / align * align : n_s;
 }
+// The kernel's way to the same: by = 2^32 / align, rounded up (0: spans do not end with the pairs), which gives the
+// quotient of numbers below 2^27 exactly for divisors up to 31; a division in front of the first loads cost a short
+// launch 0.3 us.
+__host__ __device__ inline unsigned align_factor(int align) { return align > 1 ? 0xffffffffu / (unsigned)align + 1u : 0u; }
+__device__ __forceinline__ int padded_tiles_by(int n_s, int align, unsigned by) {
+  return by ? (int)(__umulhi((unsigned)(n_s + align - 1), by) * (unsigned)align) : n_s;
+}
 
 // One segment of a workgroup's span: tiles [tile0, tile1) of one (sequence, kv head) pair.
 struct Segment {
@@ -166,14 +173,14 @@ __device__ __forceinline__ int segment_rotation(int n_tiles, unsigned rotate) {
 // The segment that starts at tile t of the stream; s: a sequence at or before t's, moved up to it.
 __device__ __forceinline__ Segment segment_at(int t, int t_end, int &s, const SeqTable &st, const Shape &sh, int hd,
                                               int vhd, bool own_v_rows, const float *kc, const float *vc, unsigned rotate,
-                                              int align) {
+                                              int align, unsigned align_by) {
   while (s + 1 < st.n_seqs && t >= st.work_off[s + 1]) ++s;
   Segment g;
   g.s = s;
   g.R = st.n_new[s];
   g.L = st.start_pos[s] + g.R;  // visible keys of the last new row
   g.n_s = (g.L + 15) >> 4;    // tiles per kv head of this sequence
-  g.n_p = padded_tiles(g.n_s, align);
+  g.n_p = padded_tiles_by(g.n_s, align, align_by);
   const int rel = t - st.work_off[s];
   g.kvh = rel / g.n_p;
   g.tile0 = rel - g.kvh * g.n_p;
@@ -210,7 +217,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
     const float *__restrict__ q_rot, const float *__restrict__ kc, const float *__restrict__ vc,
     float *__restrict__ out, float *part_o, float *part_ml, unsigned *part_flag, unsigned *flag_set,
     int spin_limit, int *error, SeqTable st_arg, Shape sh, int tiles_per_wg_arg, SpanTable sp_arg, int total_tiles_arg,
-    int align_arg, int n_slots, int pstride, float c, unsigned rotate, const DecodeDevicePlan *__restrict__ dev, ReadAhead ah,
+    int align_arg, unsigned align_by_arg, int n_slots, int pstride, float c, unsigned rotate, const DecodeDevicePlan *__restrict__ dev, ReadAhead ah,
     DistanceBias db) {
   static_assert(PAD || !BIAS, "sizes of their own come with padding");
   if constexpr (AHEAD) {
@@ -237,6 +244,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   const int tiles_per_wg = DEV ? dev->tiles_per_wg : tiles_per_wg_arg;
   const int total_tiles = DEV ? dev->total_tiles : total_tiles_arg;
   const int align = DEV ? dev->align : align_arg;
+  const unsigned align_by = DEV ? dev->align_by : align_by_arg;
   constexpr int NT = C::NT;
   // per wavefront two K tile buffers; after a segment's last tile the wavefront parks its O
   // rows [g][HD] in one while the other already receives the next segment's first tile
@@ -263,7 +271,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   // along them with dependent scalar loads took 2.5 us for a workgroup in the middle of 16
   // sequences).
   int s = (int)__popcll(__ballot(lane + 1 < st.n_seqs && t_begin >= st.work_off[lane + 1 < kMaxSeqs ? lane + 1 : kMaxSeqs]));
-  Segment seg = segment_at(t, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate, align);
+  Segment seg = segment_at(t, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate, align, align_by);
 
   f32x4 v_next[4][C::NVU];
   float qr[HD / 4];
@@ -335,7 +343,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
     const int t_next = seg.next;
     const bool more = t_next < t_end;
     Segment nseg = seg;
-    if (more) nseg = segment_at(t_next, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate, align);
+    if (more) nseg = segment_at(t_next, t_end, s, st, sh, hd, vhd, BIAS, kc, vc, rotate, align, align_by);
     const int nplace = first_place(t_next);
     const bool nhave = more && nplace < nseg.tile1 - nseg.tile0;
     const int ntile = nhave ? tile_at(nseg, nplace) : 0;
@@ -625,15 +633,26 @@ __host__ __device__ inline int least_span(int total, int wgs) {
   return q < kDecodeWaves ? kDecodeWaves : q;
 }
 // Spans that end with the pairs (DecodePlan::align): the longest worth having for that, two tiles per
-// wavefront or a quarter more than the least; shorter than the spans of unequal shares.  And the number of spans a
-// pair may have: an odd one, or the pairs' last spans, which wait for the others and merge, meet on one, two or
-// four of the eight XCDs (a call with 32 pairs of 44 tiles of 8 KiB: 18.2 us in 8 spans each, 13.6 laid end
-// to end, 12.0 in 7).
+// wavefront or a quarter more than the least; shorter than the spans of unequal shares.  And whether pairs of n_s tiles
+// may be cut into spans of q: a pair's last span waits for its others and merges, and with 2, 4 or 8 as a common
+// divisor of the pairs' counts and 8 these meet on four, two or one of the eight XCDs.  Up to four of them on an XCD
+// cost nothing, eight 0.5 to 0.9 us, which spans of one tile per wavefront are worth, 16 and more 1 to 6 us.
+// Attention kernel, us, head_dim 64:   8 pairs of 40 tiles, 4 x 10 spans 8.8, 6 x 7 9.6, 5 x 8 10.6; of 32, 4 x 8 9.8, 5 x 7
+// 9.6; of 160, 5 x 32 12.0, 6 x 27 10.8;   16 of 32, 4 x 8 11.5, 5 x 7 10.2; of 24, 4 x 6 9.3, 5 x 5 9.9, 6 x 4 10.7; of
+// 96, 6 x 16 12.6, 7 x 14 10.6;   32 of 24, 4 x 6 9.9, 5 x 5 10.2; of 16, 4 x 4 11.4, 6 x 3 10.0; of 40, 5 x 8 16.0, 6 x 7 10.4;
+// 64 of 16, 4 x 4 15.2, 6 x 3 10.9.  A pair that is one span waits for nobody.
 __host__ __device__ inline int widest_aligned_span(int q) {
   const int most = q + q / 4 > 2 * kDecodeWaves ? q + q / 4 : 2 * kDecodeWaves;
   return most < 31 ? most : 31;
 }
-__host__ __device__ inline bool spans_may_end_with(int n_s, int q) { return n_s == 0 || ((n_s + q - 1) / q & 1); }
+__host__ __device__ inline bool spans_may_end_with(int n_s, int q, int pairs) {
+  const int count = (n_s + q - 1) / q, shared = count & 7 ? count & -count : 8;  // the common divisor
+  return n_s == 0 || shared == 1 || pairs * shared <= (q == kDecodeWaves ? 64 : 32);
+}
+// The first length to try: whole pairs where they all fit the widest.
+__host__ __device__ inline int first_aligned_span(int q, int longest) {
+  return longest > q && longest <= widest_aligned_span(q) ? longest : q;
+}
 
 struct ShareArg {
   int v[8];
@@ -655,6 +674,7 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
       out->tiles_per_wg = 0;
       out->total_tiles = 0;
       out->align = 1;
+      out->align_by = 0;
       out->skip = 1;
       spans_from_shares(shares.v, 0, out->spans);  // all zero: no workgroup finds tiles
       if (*error == 0) *error = 2;  // a pending 1 (a given-up wait) is the graver report and stays
@@ -672,8 +692,12 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
   };
   int tiles = sh.KV * n_s;
   int incl = prefix(tiles), total = __shfl(incl, 63), q = least_span(total, kDevicePlanWorkgroups), align = 1;
-  for (int a = q; a <= widest_aligned_span(q); ++a)
-    if (__all(spans_may_end_with(n_s, a)) && __shfl(prefix(sh.KV * ((n_s + a - 1) / a)), 63) <= kDevicePlanWorkgroups) {
+  int longest = n_s;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) longest = max(longest, __shfl_xor(longest, o));
+  for (int a = first_aligned_span(q, longest); a <= widest_aligned_span(q); ++a)
+    if (__all(spans_may_end_with(n_s, a, n_seqs * sh.KV)) &&
+        __shfl(prefix(sh.KV * ((n_s + a - 1) / a)), 63) <= kDevicePlanWorkgroups) {
       q = align = a;
       tiles = sh.KV * padded_tiles(n_s, a);
       incl = prefix(tiles);
@@ -694,6 +718,7 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
     out->st.work_off[n_seqs] = total;
     out->tiles_per_wg = q;
     out->align = align;
+    out->align_by = align_factor(align);
     out->total_tiles = total;
     out->skip = 0;
     spans_from_shares(shares.v, q, out->spans);
@@ -719,15 +744,21 @@ DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligne
   if (wg_target < 1) wg_target = 256;
   int q = least_span(p.total_tiles, wg_target);
   // Spans that end with the pairs, where that takes no more workgroups: a span that runs from one pair
-  // into the next is two segments behind each other with a merge in between.  Per call with its prep launch, one
-  // sequence, 8 kv heads of 64 (128): 100 keys 13.0 -> 9.1 us (17.4 -> 13.1), whole pairs; 512 keys 13.1 -> 10.4
-  // (17.3 -> 14.3), 1024 keys 13.1 -> 10.5 (18.3 -> 15.5); 16 sequences of 100 keys 16.0 -> 14.6 (20.9 -> 14.4).
-  for (int a = q; aligned && a <= widest_aligned_span(q); ++a) {
+  // into the next is two segments behind each other with a merge in between.  The attention kernel, 8 kv heads of 64
+  // (128), us, laid end to end : this way: one sequence of 100 keys 10.7 : 7.3 (12.3 : 9.1), whole pairs; of 512 10.1 : 10.2
+  // (11.1 : 11.0), of 528 10.7 : 9.8 (12.7 : 10.8), of 640 9.2 : 9.7 (10.4 : 10.6), of 1040 10.6 : 9.7 (13.7 : 12.4); four
+  // of 640 16.2 : 10.9 (18.1 : 12.6); 16 of 100 13.7 : 7.2 (16.0 : 10.7).
+  int longest = 0;
+  for (int s = 0; s < st.n_seqs; ++s) {
+    const int n_s = (st.start_pos[s] + st.n_new[s] + 15) / 16;
+    longest = n_s > longest ? n_s : longest;
+  }
+  for (int a = first_aligned_span(q, longest); aligned && a <= widest_aligned_span(q); ++a) {
     long long wgs = 0;
     bool fits = true;
     for (int s = 0; s < st.n_seqs; ++s) {
       const int n_s = (st.start_pos[s] + st.n_new[s] + 15) / 16;
-      fits = fits && spans_may_end_with(n_s, a);
+      fits = fits && spans_may_end_with(n_s, a, st.n_seqs * sh.KV);
       wgs += (long long)sh.KV * ((n_s + a - 1) / a);
     }
     if (!fits || wgs > wg_target) continue;
@@ -817,7 +848,7 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
 #define SHAINET_DECODE_LAUNCH(HD_, DEV_, PAD_)                                                                      \
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, DEV_, PAD_>), grid, block, 0, stream, before,      \
                        after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit,       \
-                       d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c, rotate, dev, ah, db)
+                       d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db)
 #define SHAINET_DECODE_LAUNCH_HD(HD_, PAD_) \
   do {                                      \
     if (dev)                                \
@@ -828,7 +859,7 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
 #define SHAINET_DECODE_LAUNCH_BIAS(HD_)                                                                             \
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, false, true, false, true>), grid, block, 0, stream, \
                        before, after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set,           \
-                       spin_limit, d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c,   \
+                       spin_limit, d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c,   \
                        rotate, dev, ah, db)
   if (bias && tile_hd == 64)
     SHAINET_DECODE_LAUNCH_BIAS(64);
@@ -839,11 +870,11 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
   else if (ah.w && sh.hd == 64)
     hipLaunchKernelGGL((decode_splitk_kernel<64, kDecodeWaves, false, false, true>), grid, block, 0, stream, d.q_rot, d.kc,
                        d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit, d.error, st, sh, p.tiles_per_wg,
-                       p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c, rotate, dev, ah, db);
+                       p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db);
   else if (ah.w)
     hipLaunchKernelGGL((decode_splitk_kernel<128, kDecodeWaves, false, false, true>), grid, block, 0, stream, d.q_rot, d.kc,
                        d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit, d.error, st, sh, p.tiles_per_wg,
-                       p.spans, p.total_tiles, p.align, p.n_slots, p.cols, c, rotate, dev, ah, db);
+                       p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db);
   else if (sh.hd == 64)
     SHAINET_DECODE_LAUNCH_HD(64, false);
   else if (sh.hd == 128)

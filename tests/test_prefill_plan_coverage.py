@@ -75,15 +75,21 @@ def test_decode_spans_end_with_the_pairs():
         return p["workgroups"], p["units"]
 
     apart = 0
-    for tiles in range(1, 250):  # one sequence: an odd number of spans per pair, or spans end to end
+    for tiles in range(1, 250):  # one sequence: spans that end with the pairs, or spans end to end
         wgs, q = split([16 * tiles])
         per = -(-tiles // q)
-        if wgs != 8 * per or per % 2 == 0:
+        if wgs != 8 * per:
             apart += 1
             assert wgs == -(-8 * tiles // q) and q == max(4, -(-8 * tiles // 256)), tiles
+        else:  # (all pairs' last spans meet on one XCD only where a span is a tile per wavefront)
+            assert per == 1 or per % 8 or q == 4, tiles
     assert apart < 25  # of 249, the most of them long ones
     assert split([16 * 5]) == (8, 5) and split([16 * 8]) == (8, 8)      # whole pairs
-    assert split([16 * 12]) == (24, 4) and split([16 * 13]) == (24, 5)
+    assert split([16 * 12]) == (24, 4) and split([16 * 13]) == (32, 4)
+    assert split([16 * 40]) == (80, 4) and split([16 * 32]) == (64, 4)
+    assert split([16 * 32] * 2) == (112, 5)   # eight spans each would end on one XCD
+    assert split([16 * 24] * 2) == (96, 4) and split([16 * 24] * 4) == (192, 4)
+    assert split([16 * 40] * 4) == (224, 6) and split([16 * 16] * 4) == (96, 6)
     assert split([16 * 5] * 16) == (128, 5)
     assert split([16 * 9] * 16) == (231, 5)  # two spans each would meet on four XCDs: 1152 tiles end to end
     assert split([64], 300, 256) == (240, 5)  # more pairs than workgroups: end to end
