@@ -348,7 +348,10 @@ def test_block_device_rows_off_by_a_float(hip):
     apart = torch.empty(T * d + 1, device="cuda")[1:].view(T, d)
     apart.copy_(torch.from_numpy(x))
     whole = torch.from_numpy(x).cuda()
-    rm.assert_close(blk.forward(apart).cpu().numpy(), ob.forward(x, p["norm1"], p["norm2"], eps, p["gate"], p["up"], p["down"], False),
+    torch.cuda.synchronize()
+    got = blk.forward(apart)
+    torch.cuda.synchronize()  # the call is asynchronous on the block's stream
+    rm.assert_close(got.cpu().numpy(), ob.forward(x, p["norm1"], p["norm2"], eps, p["gate"], p["up"], p["down"], False),
                     ATOL, RTOL, "off by a float")
     on = _microseconds(lambda: blk.forward(whole), torch.cuda.synchronize)
     assert _microseconds(lambda: blk.forward(apart), torch.cuda.synchronize) < 3 * on
@@ -897,6 +900,23 @@ def test_matmul_of_very_small_operands(hip, T, K, N):
             want = xs.double() @ ws.double()
             rel = ((binding.matmul(xs, ws).double() - want).norm(dim=1) / want.norm(dim=1)).max()
             assert float(rel) <= 1.2e-6, (a, b, float(rel))
+
+
+@pytest.mark.parametrize("K,N", [(256, 1024), (1024, 4096), (2048, 3072), (2048, 16384), (4096, 8192), (8192, 2048), (8192, 28672)])
+def test_few_rows_are_as_exact_as_the_split_gemv(hip, K, N):
+    """Five to sixteen rows of a block run through the few-row tiles, the product by itself as the split GEMV, whose sums are
+    short.  17 rows take the tiles here, too: no larger an error against 64 bits, by more than a tenth."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    assert binding.describe_matmul(17, K, N)["kind"] == "few"
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    x, w = torch.randn((17, K), generator=g, device="cuda"), torch.randn((K, N), generator=g, device="cuda")
+    want = x.double() @ w.double()
+    off = lambda y: float((y.double() - want[:len(y)]).norm() / want[:len(y)].norm())
+    tiles, gemv = off(binding.matmul(x, w)), off(binding.matmul(x[:16].contiguous(), w))
+    assert tiles <= 1.1 * gemv, (tiles, gemv)
 
 
 def _microseconds(run, wait):
