@@ -220,8 +220,8 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       u32x4 h, m, l;
-      split_octet(f32x4{stage_v[u][0], stage_v[u][1], stage_v[u][2], stage_v[u][3]} * kLift,
-                  f32x4{stage_v[u][4], stage_v[u][5], stage_v[u][6], stage_v[u][7]} * kLift, h, m, l);
+      split_octet(f32x4{stage_v[u][0], stage_v[u][1], stage_v[u][2], stage_v[u][3]},
+                  f32x4{stage_v[u][4], stage_v[u][5], stage_v[u][6], stage_v[u][7]}, h, m, l);
       lds[v_unit[u]] = h;
       lds[v_unit[u] + U::kPartV] = m;
       lds[v_unit[u] + 2 * U::kPartV] = l;
@@ -250,10 +250,27 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       }
 #pragma unroll
     for (int i = 0; i < KS; ++i) split_octet(t[i][0] * c, t[i][1] * c, qf[i][0], qf[i][1], qf[i][2]);
-    QueryRange range;
+    float least = INFINITY, most = 0.f;
 #pragma unroll
-    for (int i = 0; i < KS; ++i) range.add(t[i][0]), range.add(t[i][1]);
-    apart = __any(range.apart(c));
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (PAD && 16 * i + 8 * j + 4 * h >= hd) continue;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float size = fabsf(t[i][h][w] * c);
+          least = fminf(least, size);
+          most = fmaxf(most, size);
+        }
+      }
+    apart = false;
+    // (looked at closely only where there is a zero or something out of the ordinary)
+    if (__builtin_expect(__any(!(least >= 0x1p-109f) || !(most < 0x1p100f)), 0)) {
+      QueryRange range;
+#pragma clang loop unroll(disable)
+      for (int d = 4 * j; d < hd; d += 8) range.add(*(const f32x4 *)(q_rot + q_off + d));
+      apart = __any(range.apart(c));
+    }
   }
 
   // Online softmax against a reference value per virtual row instead of the running maximum: m_ref is only moved
@@ -376,16 +393,45 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     __syncthreads();  // K(sp + 1) is there, nobody reads V(sp) any more
   }
 
-  // Results that are not finite come from operands that are not (or are infinite once lifted): the wavefront takes its
-  // tiles again in fp32, which says which.  So does one whose queries ask for it.  8192 rows, 32 / 8 heads of 64, NaN
-  // in key 5: 4.6 ms a call against 1.6 without (key by key, one dimension at a time, it was 279).
+  // Some results are taken again, tile by tile in fp32:
+  //   results that are not finite come from operands that are not, and fp32 says which (8192 rows, 32 / 8 heads of 64, NaN
+  //   in key 5: 4.6 ms a call against 1.6 without; key by key, one dimension at a time, it was 279);
+  //   queries that ask for it (QueryRange);
+  //   values below 2^-110: what they lose by the split, 2^-134 of a key's weight, shows in sums that are themselves small
+  //   (the largest weight of a row is 1 or more, all together under 2^30).  Those may be sums of zeros, too: the
+  //   values are looked at.  Lifted there by 2^24, or sums of subnormal numbers would round to 2^-149.
+  // All values lifted on their way to LDS, and every query looked at closely, cost 8192 rows 5 % (1323 -> 1383 us; this
+  // way 1320) and 2048 rows of 32 / 8 heads of 128 4 % (216 -> 224; 218).
   {
-    float probe = l * 0.f;
+    auto size = [](float x) { return __builtin_bit_cast(unsigned, x) << 1; };  // (in the order of |x|)
+    float probe = l * 0.f, least = INFINITY;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) probe = fmaf(o[t][r], 0.f, probe);
-    if (__builtin_expect(apart || __any(probe != 0.f), 0)) {
+      for (int r = 0; r < 16; ++r) {
+        probe = fmaf(o[t][r], 0.f, probe);
+        least = fminf(least, fabsf(o[t][r]));
+      }
+    bool again = apart || __any(probe != 0.f);
+    float up = 1.f, down = 1.f;
+    if (__builtin_expect(__any(least < 0x1p-80f && thr != -INFINITY), 0) && !again) {
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      unsigned small = ~0u;  // (zeros lie above all)
+#pragma clang loop unroll(disable)
+      for (int kt = kt0 + gidx; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
+        const float *vr = vbase + (long long)min(kt * 32 + (tid & 31), wave_hi) * vhd;
+#pragma clang loop unroll_count(4)
+        for (int d = (tid & 32) >> 3; d < vhd; d += 8) {
+          const f32x4 v = *(const f32x4 *)(vr + d);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) small = min(small, size(v[i]) - 1u);
+        }
+      }
+      again = __any(small < size(0x1p-109f));
+      up = kLift, down = kDropOne;
+    }
+    if (__builtin_expect(again, 0)) {
       // (what a lane works on is found again from its number: kept for here it would cost the loop above registers)
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));
@@ -458,7 +504,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
             const int key = first + 8 * (r >> 2) + 4 * j + (r & 3);
             const vrow_t v = *(const vrow_t *)(vbase + (long long)key * vhd + (PAD && NT * n >= vhd ? 0 : NT * n));
 #pragma unroll
-            for (int t = 0; t < NT; ++t) sum[t] = mfma_f32(v[t], p[r], sum[t]);
+            for (int t = 0; t < NT; ++t) sum[t] = mfma_f32(v[t] * up, p[r], sum[t]);
           }
           continue;
         }
@@ -482,7 +528,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                   const int at = 4 * w + i;
-                  sum[at % NT][4 * q + at / NT] = fmaf(e, v[i], sum[at % NT][4 * q + at / NT]);
+                  sum[at % NT][4 * q + at / NT] = fmaf(e, v[i] * up, sum[at % NT][4 * q + at / NT]);
                 }
               }
           }
@@ -493,13 +539,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          float x = sum[t][r];
+          float x = sum[t][r] * down;
           asm volatile("" : "+v"(x));
           o[t][r] = x;
         }
-    } else {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) o[t] *= kDropOne;
     }
   }
 

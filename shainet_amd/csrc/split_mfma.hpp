@@ -2,9 +2,10 @@
 // rounded to bf16, the rest rounded to bf16, and the rest of that (8 + 8 + 8 mantissa bits with signs of
 // their own).  A bf16 has a float's exponents and 16 bits less behind them, so the rests of a float below 2^-110
 // would not be whole; operands are lifted by 2^24 first, which makes every part of every float, the smallest
-// subnormal's too, a normal bf16 or zero, and results are brought down again (not the operands of scores, QueryRange,
-// nor probabilities, whose row holds one near 1).  2 to 4 % of a prompt's time; rows of x around 2^-120 had
-// an error of 3.5e-5 without, and 2e-7 with it, as rows around 1 have.  Of the nine products of two such sums
+// subnormal's too, a normal bf16 or zero, and results are brought down again.  (Not the operands of scores, see
+// QueryRange, nor probabilities, whose row holds one near 1, nor the values of prefill attention, which looks at its
+// sums instead.)  That is 2 to 4 % of a prompt's products; rows of x around 2^-120 had an error of 3.5e-5 without, and
+// 2e-7 with it, as rows around 1 have.  Of the nine products of two such sums
 // the six largest make up the product to 2^-24 of itself: of the three left out two can reach 2^-25 each.  Six
 // v_mfma_f32_32x32x16_bf16 of 32 cycles do what eight v_mfma_f32_32x32x2_f32 of 64 do (192 against 512
 // cycles per 32 x 32 x 16; a loop of nothing else: 1876 TFLOP/s of bf16 = 312 of fp32, against 155), they
@@ -12,8 +13,9 @@
 // 6/16 times per term instead of 1/2: measured against 64 bits the error is 0.4 to 0.95 of the fp32
 // instruction's for sums of 64 to 8192 terms.
 // What is not finite in an operand (or infinite once it is lifted: from 2^104 on, and sums of products from 2^80
-// on) makes NaN or infinity of the sums it enters; callers look for sums that are not finite and take those again with the fp32 instruction, its operands straight
-// from memory: the wavefronts that meet such a value cost two to four times what they do otherwise.
+// on) makes NaN or infinity of the sums it enters; callers look for sums that are not finite and take those again
+// with the fp32 instruction, its operands straight from memory: the wavefronts that meet such a value cost two to
+// four times what they do otherwise.
 #pragma once
 #include <hip/hip_runtime.h>
 

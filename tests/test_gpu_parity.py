@@ -989,3 +989,34 @@ def test_prefill_of_very_small_operands(hip, hd, KV, T, cached, q_by, k_by, v_by
         p = np.exp(s - s.max(-1, keepdims=True))
         want = (p / p.sum(-1, keepdims=True)) @ (vr / v_by)
         assert np.abs(got[:, h] - want).max() <= 1e-5 + 2.0 ** -149 / v_by, h
+
+
+@pytest.mark.parametrize("hd,KV,T,tiny", [(64, 2, 300, 2.0 ** -124), (128, 2, 300, 2.0 ** -135), (96, 4, 140, 2.0 ** -124), (64, 8, 2300, 0.0)])
+def test_prefill_of_zeros_and_a_tiny_value(hip, hd, KV, T, tiny):
+    """Head 0's values are zeros but for one key's, every third row's queries zeros: sums that are small because values
+    are keep their bits, sums of zeros are zeros."""
+    import torch
+
+    H = 2 * KV
+    g = torch.Generator(device="cuda").manual_seed(hd + T)
+    q, k, v = (torch.randn((T, n * hd), generator=g, device="cuda") for n in (H, KV, KV))
+    q[::3] = 0.0
+    v[:, :hd] = 0.0
+    v[40, :hd] = tiny * torch.randn((hd,), generator=g, device="cuda")
+    ctx = hip.AttnContext(H, KV, hd, max_positions=T)
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, T)
+    got = ctx.forward(cache, q, k, v, [T])
+    ctx.sync()
+    got = got.cpu().numpy().reshape(T, H, hd).astype(np.float64)
+    qr = ctx.last_q_rot(T).astype(np.float64).reshape(T, H, hd)
+    for h in range(H):
+        kr, vr = (a.astype(np.float64) for a in cache.read(0, h // 2, 0, T))
+        s = qr[:, h] @ kr.T / np.sqrt(hd)
+        s[np.arange(T)[None] > np.arange(T)[:, None]] = -np.inf
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p / p.sum(-1, keepdims=True)) @ vr
+        # one key's share; as a subnormal number it is rounded where it is brought down, where groups and chunks of keys
+        # meet, and as the quotient
+        bar = 1e-5 if h > 1 else 1e-5 * np.abs(want) + 2.0 ** -147
+        assert (np.abs(got[:, h] - want) <= bar).all(), h
