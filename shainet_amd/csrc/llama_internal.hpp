@@ -145,7 +145,10 @@ struct Projector {
   // Whether T rows run as the split GEMV.  Up to 4 do.  It streams the weights once for up to 16, but its multiply-adds
   // are the vector ALU's, and from 5 rows on the MFMA product is the faster one (a prompt of a 2048 wide model of 4
   // layers: 4 rows 533 | 600 us, 5 rows 701 | 600, 16 rows 962 | 602); it needs K, N and the row stride of x to be
-  // multiples of 4.
+  // multiples of 4.  Small weights wait for launches alone, and the MFMA product has more of them (norm, head rows,
+  // activation, the sum of pieces): a block of width 64 | 128 | 256 | 512 takes 90 | 88 | 101 | 103 us for 5 rows if all its
+  // products are MFMA's, 68 | 72 | 81 | 93 this way; for 8 rows 84 | 80 | 99 | 98 and 77 | 77 | 93 | 94; from 10 rows on
+  // the MFMA product is the faster one at any size (width 128, 12 rows: 80, and 85 with the smallest as the split GEMV).
   static bool few_rows(int T, int K, int N, long long x_stride);
   DevF scratch, normed, wide;
   // split products: a word per partial that says when it is complete (zero between launches)

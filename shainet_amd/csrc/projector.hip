@@ -145,7 +145,8 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
 }
 
 bool Projector::few_rows(int T, int K, int N, long long x_stride) {
-  return T <= 4 || (T <= 16 && !plan_gemm(T, K, N, x_stride).mfma);
+  const long long weights = (long long)K * N;
+  return T <= 4 || (T <= 6 && weights <= 128 << 10) || (T <= 8 && weights <= 64 << 10) || (T <= 16 && !plan_gemm(T, K, N, x_stride).mfma);
 }
 
 int Projector::project(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,

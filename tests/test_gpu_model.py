@@ -919,6 +919,16 @@ def test_few_rows_are_as_exact_as_the_split_gemv(hip, K, N):
     assert tiles <= 1.1 * gemv, (tiles, gemv)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+def test_a_few_rows_of_a_narrow_block(hip, d):
+    """Up to 6 rows by up to 128 k weights, and 8 by 64 k, run as the split GEMV, more as the MFMA product."""
+    blk, ob, p, r, eps = _block_pair(hip, d, d // 32, 1, 32, 4 * d, 1e4, seed=d)
+    for T in (4, 5, 6, 7, 8, 9, 16):
+        x = r.standard_normal((T, d)).astype(np.float32)
+        rm.assert_close(blk.forward(x), ob.forward(x, p["norm1"], p["norm2"], eps, p["gate"], p["up"], p["down"], False),
+                        ATOL, RTOL, f"T={T}")
+
+
 def _microseconds(run, wait):
     import time
 
