@@ -733,12 +733,21 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
   const int tokens = T <= 4096 ? 4 : 16;
   hipLaunchKernelGGL(moe_select_kernel, dim3((unsigned)((T + tokens - 1) / tokens)), dim3(256), lds, stream, m, w.correction, logits,
                      stride, T, tokens, ids, weights, rank, counts);
-  // rows an expert gets if the router spreads them evenly
-  // (tiles of 64 | 128 rows, us a prompt: width 1024, 145 rows an expert 1347 | 1347, 281: 1904 | 2043, 384: 2310 | 2317;
-  // width 2048, 194: 3249 | 3169, 375: 5196 | 5053, 512: 6139 | 5725; tiles of 32 lose 4 to 23 % everywhere, one row included)
-  const int per_expert = slots / n, best_tm = per_expert > 320 ? 128 : 64;
-  static const int tile_knob = getenv("SHAINET_HIP_MOE_TILE") ? atoi(getenv("SHAINET_HIP_MOE_TILE")) : 0;  // a tuning knob: 64 or 128
-  const int tm = tile_knob == 64 || tile_knob == 128 ? tile_knob : best_tm;
+  // per_expert: rows an expert gets if the router spreads them evenly.  Tiles of 128 rows split each matrix half as often
+  // and fill up worse.  Prompts, 64 | 128, us, rows an expert by width and expert width:
+  //               25           75           125          194          260          375
+  //   1024,  512  949 | 977    1145 | 1194  1264 | 1268  1474 | 1405  1627 | 1654  2060 | 2052   (281: 1890 | 2060)
+  //   1024, 1024  1092 | 1109  1343 | 1331  1504 | 1608  1864 | 1750  2098 | 2037  2706 | 2550
+  //   1536,  768  1158 | 1235  1466 | 1446  1635 | 1533  2163 | 2174  2523 | 2434  3063 | 2963
+  //   2048,  512  1257 | 1298  1473 | 1510  1714 | 1760  2260 | 2089  2730 | 2721  3647 | 3295
+  //   2048,  768  1460 | 1489  1866 | 1827  2278 | 2244  3280 | 3177  4045 | 3926  5520 | 5363
+  //   2048, 1024  1469 | 1451  1895 | 1763  2272 | 2486  3127 | 2866  3766 | 3395  4910 | 4292
+  //   4096,  512  1845 | 2000  2351 | 2472  2817 | 2842  3946 | 3697  5138 | 4781  6469 | 5960
+  // (2048, 768: the last at 425).  Tiles of 32 lose 4 to 23 % everywhere, one row included.
+  const int per_expert = slots / n, best_tm = per_expert > ((long long)m.d * m.ff > 512 << 10 ? 160 : 320) ? 128 : 64;
+  // a tuning knob: 64 or 128 (32, which there once was, is 64)
+  static const int tile_knob = getenv("SHAINET_HIP_MOE_TILE") ? atoi(getenv("SHAINET_HIP_MOE_TILE")) : 0;
+  const int tm = tile_knob == 128 ? 128 : tile_knob == 64 || tile_knob == 32 ? 64 : best_tm;
   hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, stream, m.experts, tm, counts, off, tile_off);
   hipLaunchKernelGGL(moe_scatter_kernel, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, stream, slots, m.top, m.experts,
                      ids, rank, off, rows);

@@ -352,6 +352,17 @@ def test_experts_keep_rows_apart(hip, tmp_path, name):
     assert np.isnan(got[384:]).all()
 
 
+def test_experts_wide_enough_for_tall_tiles(hip, tmp_path):
+    """1040 x 512 weights an expert: 160 rows an expert on average in tiles of 64, 165 in tiles of 128."""
+    cfg = zm.config([zm.layer(zm.hgrn2(heads=1, dim=4, vdim=4), zm.moe(ff=512, experts=2, identity=0, top=1, groups=1, keep=1))], width=1040)
+    p = Pair(hip, tmp_path, cfg, edit=lambda w: w.update({"l0.mix.o": 0 * w["l0.mix.o"]}), seed=3)
+    x = (2 * np.random.default_rng(4).standard_normal((330, 1040))).astype(np.float32)
+    want = p.layer(0, x)
+    close(p.model.blocks[0].forward_cached(x), want)
+    p.model.blocks[0].clear_cache()
+    close(p.model.blocks[0].forward_cached(x[:321]), want[:321])
+
+
 def test_experts_of_very_small_hidden_rows(hip, tmp_path):
     """Hidden rows around 2^-124 between an up matrix that small and a down matrix that large lose no bits."""
     def edit(w):
