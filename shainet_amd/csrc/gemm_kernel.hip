@@ -1,4 +1,4 @@
-// Row-major fp32 product y[T,N] = x[T,K] W[K,N] (+ res) for gfx950, for more than 16 rows: the
+// Row-major fp32 product y[T,N] = x[T,K] W[K,N] (+ res) for gfx950, for five rows and more: the
 // projections of a prefill (llama_block.cr:253-255, 298; swiglu_ff.cr:76-91), where the
 // reference's GPU branch calls cuBLAS SGEMM (llama_block.cr:726-768, cuda.cr:237-247) and its CPU
 // branch SimpleMatrix#* (simple_matrix.cr:61-74).
@@ -366,9 +366,10 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
 }
 
 // Few rows: a wavefront owns the columns of W it multiplies, so they go from memory to its registers and are split
-// there; only x goes through LDS.  A workgroup of four wavefronts owns 32 rows and 128 columns and walks K in steps of 32: wavefronts 0 and 1 take the first half of a step, 2 and 3 the second, 64 columns
-// each, and the two halves' sums meet in LDS at the end.  Lane n of a wavefront loads two neighbouring columns (a
-// row of W 256 bytes at a time) and 8 rows, which are its fragments of two blocks.
+// there; only x goes through LDS.  A workgroup of four wavefronts owns 32 rows and 128 columns and walks K in steps of 32:
+// wavefronts 0 and 1 take the first half of a step, 2 and 3 the second, 64 columns each, and the two halves' sums meet in
+// LDS at the end.  Lane n of a wavefront loads two neighbouring columns (a row of W 256 bytes at a time) and 8 rows, which
+// are its fragments of two blocks.
 // Against tiles of 64 x 128 with both operands in LDS, which this reads and writes a fifth as much (us): 32 rows of
 // 2048 -> 16384 44 -> 30 (134 MB: 22 at the rate of a read), 2048 -> 3072 19.3 -> 14.4, 45 rows 44 -> 41 and 19.5 -> 15.7,
 // 64 rows of 1024 -> 1024 12.1 -> 9.2.  64 rows by 128 columns this way were slower than 32 (45 rows of
