@@ -929,6 +929,18 @@ def test_a_few_rows_of_a_narrow_block(hip, d):
                         ATOL, RTOL, f"T={T}")
 
 
+@pytest.mark.parametrize("T", [5, 16])
+def test_a_few_rows_of_a_block_that_are_not_finite(hip, T):
+    """The same in a block, where the few-row tiles run from five rows on: a last row of NaN stays by itself."""
+    blk, ob, p, r, eps = _block_pair(hip, 1024, 8, 2, 128, 2048, 1e4, seed=T, wscale=0.02)
+    x = r.standard_normal((T, 1024)).astype(np.float32)
+    want = ob.forward(x, p["norm1"], p["norm2"], eps, p["gate"], p["up"], p["down"], False)
+    x[T - 1, 77] = np.nan
+    got = blk.forward(x)
+    rm.assert_close(got[:-1], want[:-1], ATOL, RTOL, "rows in front")
+    assert np.isnan(got[-1]).all()
+
+
 def _microseconds(run, wait):
     import time
 
