@@ -101,6 +101,7 @@ struct BiasedAttn : Mixer {
     DistanceBias b = bias;
     b.q_stride = w.n_in;
     Fused in = pre;
+    in.w_bf16 = w.w_in_bf16;
     const bool fuse = !from && T <= 16 && Projector::few_rows(T, d, w.n_in, d) && dim == vdim && (w.n_in & 3) == 0 && dim >= 2 && dim <= 128 && (dim & (dim - 1)) == 0;
     if (fuse) {
       // few rows: key and value heads go to the cache where the product sums them up
@@ -132,6 +133,7 @@ struct BiasedAttn : Mixer {
       if (kv) kv->len[0] = rows;
     }
     Fused post;
+    post.w_bf16 = w.w_o_bf16;
     if (residual) {
       post.epilogue = kGemvResidual;
       post.res = residual;

@@ -21,6 +21,7 @@ struct BiasedWeights {
   float *w_o = nullptr, *w_o_t = nullptr;    // [H vdim, d]
   int n_in = 0;
   bool w_in_t_stale = true, w_o_t_stale = true;
+  bool w_in_bf16 = false, w_o_bf16 = false;  // every value is a bf16 number: the loader says so
 };
 
 // kv_from != null: keys and values are that mixer's, which has projections of its own, the same kv_heads, dim

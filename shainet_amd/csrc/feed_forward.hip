@@ -27,11 +27,13 @@ struct Dense : FeedForward {
     up.epilogue = kGemvBias;
     up.bias = w.up_bias;
     up.act = w.act;
+    up.w_bf16 = w.up_bf16;
     if (gemvt_takes(T, d, ff, up.epilogue, up.norm)) up.w_t = transposed_twin(&w.up_t, &w.up_t_stale, w.up, d, ff, stream);
     if (int rc = proj.project(h, d, w.up, hidden.p, T, d, ff, stream, up)) return rc;
     Fused down;
     down.epilogue = kGemvBias;
     down.bias = w.down_bias;
+    down.w_bf16 = w.down_bf16;
     if (gemvt_takes(T, ff, d, down.epilogue, down.norm)) down.w_t = transposed_twin(&w.down_t, &w.down_t_stale, w.down, ff, d, stream);
     return proj.project(hidden.p, ff, w.down, y, T, ff, d, stream, down);
   }
@@ -50,7 +52,7 @@ struct Moe : FeedForward {
       if (p) (void)hipFree(p);
   }
   int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream) override {
-    const MoeTensors t = {w.router, w.correction, w.gate_up, w.down, w.shared_gate_up, w.shared_down};
+    const MoeTensors t = {w.router, w.correction, w.gate_up, w.down, w.shared_gate_up, w.shared_down, w.gate_up_bf16, w.down_bf16};
     hipError_t e;
     if (T <= kMoeFewTokens) {
       if (!scratch.reserve(moe_few_floats(m, T))) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
@@ -66,12 +68,17 @@ struct Moe : FeedForward {
         if (!hidden.reserve((size_t)n * m.shared_ff)) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
         Fused gate;
         gate.epilogue = kGemvSwiglu;
+        gate.w_bf16 = w.shared_gate_up_bf16;
         if (int rc = proj.project(hp, m.d, w.shared_gate_up_in, hidden.p, n, m.d, m.shared_ff, stream, gate)) return rc;
-        if (int rc = proj.project(hidden.p, m.shared_ff, w.shared_down_in, yp, n, m.shared_ff, m.d, stream)) return rc;
+        Fused down;
+        down.w_bf16 = w.shared_down_bf16;
+        if (int rc = proj.project(hidden.p, m.shared_ff, w.shared_down_in, yp, n, m.shared_ff, m.d, stream, down)) return rc;
       }
       if (!scratch.reserve(moe_many_floats(m, n)) || !logits.reserve((size_t)n * w.n_router))
         return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-      if (int rc = proj.project(hp, m.d, w.router_in, logits.p, n, m.d, w.n_router, stream)) return rc;
+      Fused router;
+      router.w_bf16 = w.router_bf16;
+      if (int rc = proj.project(hp, m.d, w.router_in, logits.p, n, m.d, w.n_router, stream, router)) return rc;
       e = launch_moe_many(m, t, hp, logits.p, w.n_router, yp, m.shared_ff > 0, n, scratch.p, counts, stream);
       if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("expert launch: ") + hipGetErrorString(e));
     }

@@ -17,6 +17,7 @@ struct DenseWeights {
   float *down = nullptr, *down_t = nullptr, *down_bias = nullptr;  // [ff, d], twin, [d]
   Activation act;
   bool up_t_stale = true, down_t_stale = true;
+  bool up_bf16 = false, down_bf16 = false;  // every value is a bf16 number: the loader says so
 };
 int dense_create(FeedForward **out, int d_model, int ff, DenseWeights **weights);
 
@@ -28,6 +29,8 @@ struct MoeWeights {
   int n_router = 0;
   float *shared_gate_up = nullptr, *shared_down = nullptr;        // [2 ff, d], [d, ff]
   float *shared_gate_up_in = nullptr, *shared_down_in = nullptr;  // [d, 2 ff], [ff, d]
+  // every value is a bf16 number: the loader says so
+  bool router_bf16 = false, gate_up_bf16 = false, down_bf16 = false, shared_gate_up_bf16 = false, shared_down_bf16 = false;
 };
 int moe_create(FeedForward **out, const MoeShape &shape, MoeWeights **weights);
 

@@ -14,7 +14,13 @@
 //      its registers and nothing has to be transposed.  Column c of a wavefront's 64 lies in block c % 2 at
 //      place c / 2: a lane's two blocks are neighbouring columns of y (8-byte stores, 256 bytes a row).
 // Tile loads take a scalar base that moves along K plus a per-thread 32-bit offset.
-// What bounds it: large shapes the power the card may draw.  4096 rows of 2048 -> 16384 run at 232 TFLOP/s
+// W whose values are bf16 numbers (a checkpoint's, most often): the other two of its parts are zeros, and the three
+// products with them add nothing.  They are left out, sum for sum the same bits.  2048 rows of 2048 -> 16384 571 -> 345 us
+// (398 TFLOP/s), 8192 -> 2048 322 -> 194, 512 rows 174 -> 100 and 101 -> 61, 777 rows of 1024 -> 4096 53 -> 35.  What bounds
+// these is issue: the matrix cores are busy 54 % of the time, in which a step's 24 MFMAs share two wavefronts a SIMD with
+// 70 vector instructions each, and everybody meets at a barrier.  Tiles of four by two wavefronts (64 x 128 each) read
+// 10 fragments a step, two by four (128 x 64) 14.
+// What bounds the others: large shapes the power the card may draw.  4096 rows of 2048 -> 16384 run at 232 TFLOP/s
 // with N(0, 1) operands and at 295 with zeros (71 % of the six products' rate); with four wavefronts on
 // 128 x 128 tiles it was 183 and 252, so the large tile, which reads LDS 3/4 as often and splits half as much
 // per product, is worth more than a better schedule (an order forced between MFMAs and splits, three
@@ -57,6 +63,15 @@ __device__ __forceinline__ void coherent_store4(float *p, f32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }
 
+// *base (the same in all lanes) plus a lane's own offset in bytes: one load with a scalar base.  (Of addresses that differ
+// by scalars only the compiler makes 64-bit sums per thread, two instructions each.)
+template <typename V>
+__device__ __forceinline__ V load_at(const V *base, unsigned offset) {
+  uint64_t at = (uint64_t)base;
+  asm("" : "+s"(at), "+v"(offset));
+  return *(const __attribute__((address_space(1))) V *)(at + offset);
+}
+
 struct GemmArgs {
   const float *x;
   long long xs;
@@ -94,23 +109,46 @@ __device__ __forceinline__ void store_pair(const GemmArgs &g, int row, int col, 
   *(f32x2 *)(g.y + o) = v;
 }
 
-// Units of 16 bytes in a stage of LDS.  A part of x: two octets of TM rows, four units apart from a multiple
-// of 16 (a wavefront writes both octets of 32 rows); a part of W: two octets of two wavefronts' two blocks of 32
-// columns, four units of padding behind each (neighbouring columns lie in two blocks).
-template <int MB, int WN>
+// Four registers of a lane's sums, number r of its 4 MB NB: with two blocks beside each other its two columns in two
+// rows, with four its four columns in one row.
+template <int NB>
+__device__ __forceinline__ void store_four(const GemmArgs &g, int row0, int col, int r, f32x4 v) {
+  if constexpr (NB == 2) {
+    const int row = row0 + 32 * (r >> 3) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
+    store_pair(g, row, col, f32x2{v.x, v.y});
+    store_pair(g, row + 1, col, f32x2{v.z, v.w});
+  } else {
+    const int row = row0 + 32 * (r >> 4) + 8 * ((r & 15) >> 2) + (r & 3);
+    if (row >= g.T) return;
+    const long long o = (long long)row * g.N + col;
+    if (g.bias) {
+      const f32x4 b = *(const f32x4 *)(g.bias + col);
+      v = f32x4{activate(g.act, v.x + b.x), activate(g.act, v.y + b.y), activate(g.act, v.z + b.z), activate(g.act, v.w + b.w)};
+    }
+    if (g.res) v = *(const f32x4 *)(g.res + o) + v;
+    *(f32x4 *)(g.y + o) = v;
+  }
+}
+
+// WM x WN wavefronts of MB x NB blocks.  Units of 16 bytes in a stage of LDS.  A part of x: two octets of TM rows, four
+// units apart from a multiple of 16 (a wavefront writes both octets of 32 rows); a part of W: two octets of WN
+// wavefronts' NB blocks of 32 columns, four units of padding behind each (neighbouring columns lie in NB blocks).
+template <int WM, int WN, int MB, int NB, int PARTS>
 struct Stage {
-  static constexpr int kOctX = 64 * MB + 4, kPartX = 2 * kOctX;
-  static constexpr int kOctW = 2 * WN * 36, kPartW = 2 * kOctW;
-  static constexpr int kUnits = 3 * (kPartX + kPartW);
+  static constexpr int kOctX = 32 * WM * MB + 4, kPartX = 2 * kOctX;
+  static constexpr int kOctW = 36 * WN * NB, kPartW = 2 * kOctW;
+  static constexpr int kUnits = 3 * kPartX + PARTS * kPartW;
 };
 
-// GUARD: K need not be a multiple of 16 (pieces beyond its end are zeros).
-template <int MB, int WN, bool GUARD>
-__global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs g) {
-  constexpr int TM = 64 * MB, TN = 64 * WN;
-  constexpr int NX = 2 * MB / WN;  // float4 of the x tile per thread
-  constexpr int kSets = MB == 4 ? 1 : 2;
-  using S = Stage<MB, WN>;
+// PARTS: of W, 3 or (its values are bf16 numbers) 1.  GUARD: K need not be a multiple of 16 (pieces beyond its end are zeros).
+template <int WM, int WN, int MB, int NB, int PARTS, bool GUARD>
+__global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const GemmArgs g) {
+  constexpr int TM = 32 * WM * MB, TN = 32 * WN * NB, NT = 64 * WM * WN;
+  constexpr int NX = 4 * TM / NT;  // float4 of the x tile per thread
+  constexpr int kSets = PARTS == 3 && TM == 256 ? 1 : 2;
+  using S = Stage<WM, WN, MB, NB, PARTS>;
+  static_assert(PARTS == 3 || MB == 2, "six rows of products");
+  static_assert(2 * TN == NT, "a thread stages an octet of W");
   static_assert(NX == 2 || NX == 1, "a thread stages an octet of x, or half of one");
   __shared__ __attribute__((aligned(16))) u32x4 lds[2][S::kUnits];
 
@@ -129,21 +167,9 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
   const int t_first = u0 / steps, t_last = (u1 - 1) / steps;
   const bool leaves_piece = u1 < (t_last + 1) * steps;  // the run ends inside tile t_last
 
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ln = lane & 31, j = lane >> 5, wm = wave / WN, wn = wave % WN;
+  const int wm = wave / WN, wn = wave % WN;
   const int T = g.T, K = g.K, N = g.N;
-
-  // staging: x: octet tid % 2 of row tid / 2, or half of one, quarter tid % 4 of row tid / 4; W: octet tid / TN
-  // of column tid % TN
-  const int xrow = NX == 1 ? threadIdx.x >> 2 : threadIdx.x >> 1;
-  const int xk = NX == 1 ? 4 * (threadIdx.x & 3) : 8 * (threadIdx.x & 1);
-  const int wcol = threadIdx.x & (TN - 1), wk = 8 * (threadIdx.x / TN);
-  const int x_unit = (xk >> 3) * S::kOctX + xrow;
-  const int w_unit = 3 * S::kPartX + (wk >> 3) * S::kOctW + (wcol >> 6) * 72 + (wcol & 1) * 36 + ((wcol & 63) >> 1);
-  // fragments
-  const int a_unit = j * S::kOctX + wm * 32 * MB + ln;
-  const int b_unit = 3 * S::kPartX + j * S::kOctW + wn * 72 + ln;
   const long long w_step = (long long)TK * N * 4;
 
   for (int visit = 0; visit <= t_last - t_first; ++visit) {
@@ -156,6 +182,24 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
     const int m0 = tm * TM, n0 = tn * TN;
     const int k_begin = s_begin * TK, k_end = min(K, s_end * TK);
     const int nk = s_end - s_begin;
+
+    // (what follows from the thread's number is worked out per tile, or the compiler keeps it in scratch memory over the
+    // tile's end and the loads of the first step wait for it)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    const int ln = lane & 31, j = lane >> 5;
+
+    // staging: x: octet tid % 2 of row tid / 2, or half of one, quarter tid % 4 of row tid / 4; W: octet tid / TN
+    // of column tid % TN
+    const int xrow = NX == 1 ? tid >> 2 : tid >> 1;
+    const int xk = NX == 1 ? 4 * (tid & 3) : 8 * (tid & 1);
+    const int wcol = tid & (TN - 1), wk = 8 * (tid / TN);
+    const int x_unit = (xk >> 3) * S::kOctX + xrow;
+    const int w_unit = 3 * S::kPartX + (wk >> 3) * S::kOctW + wcol / (32 * NB) * (36 * NB) + wcol % NB * 36 + wcol % (32 * NB) / NB;
+    // fragments
+    const int a_unit = j * S::kOctX + wm * 32 * MB + ln;
+    const int b_unit = 3 * S::kPartX + j * S::kOctW + wn * 36 * NB + ln;
 
     // (rows past the last one repeat it and columns likewise: their products are never stored)
     const unsigned x_off = (unsigned)(((long long)min(m0 + xrow, T - 1) * g.xs + xk) * 4);
@@ -171,12 +215,15 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
 #pragma unroll
       for (int u = 0; u < NX; ++u) {
         const int kk = k_next + xk + 4 * u;
-        const char *p = x_base + x_off + 16 * u;
-        rx[u] = !GUARD || kk < k_end ? *(const f32x4 *)p : f32x4{0.f, 0.f, 0.f, 0.f};
+        rx[u] = GUARD && kk >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f}
+                : PARTS == 3         ? *(const f32x4 *)(x_base + x_off + 16 * u)
+                                     : load_at((const f32x4 *)(x_base + 16 * u), x_off);
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        rw[i] = !GUARD || k_next + wk + i < k_end ? *(const float *)(w_base + (long long)i * N * 4 + w_off) : 0.f;
+      for (int i = 0; i < 8; ++i) {
+        const float *row = (const float *)(w_base + (long long)i * N * 4);
+        rw[i] = GUARD && k_next + wk + i >= k_end ? 0.f : PARTS == 3 ? *(const float *)((const char *)row + w_off) : load_at(row, w_off);
+      }
       if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
         x_base += TK * 4;
         w_base += w_step;
@@ -187,13 +234,19 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       u32x4 h, m, l;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        unsigned a, b, c;
-        split_pair(rw[2 * i] * kLift, rw[2 * i + 1] * kLift, a, b, c);
-        h[i] = a, m[i] = b, l[i] = c;
+        if constexpr (PARTS == 3) {
+          unsigned a, b, c;
+          split_pair(rw[2 * i] * kLift, rw[2 * i + 1] * kLift, a, b, c);
+          h[i] = a, m[i] = b, l[i] = c;
+        } else {
+          h[i] = pack_high(rw[2 * i] * kLift, rw[2 * i + 1] * kLift);
+        }
       }
       stage[w_unit] = h;
-      stage[w_unit + S::kPartW] = m;
-      stage[w_unit + 2 * S::kPartW] = l;
+      if constexpr (PARTS == 3) {
+        stage[w_unit + S::kPartW] = m;
+        stage[w_unit + 2 * S::kPartW] = l;
+      }
       if constexpr (NX == 1) {
         u32x2 *half = (u32x2 *)(stage + x_unit) + ((xk >> 2) & 1);
         split_quad(rx[0] * kLift, half[0], half[2 * S::kPartX], half[4 * S::kPartX]);
@@ -205,11 +258,11 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       }
     };
 
-    f32x16 acc[MB][2];
+    f32x16 acc[MB][NB];
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
@@ -220,49 +273,115 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
     load_tiles(sx[0], sw[0]);
     __syncthreads();
 
-    // Per step of 16 along K: the fragments are fetched, the next step's tiles are split and go to the other
-    // stage while the MFMAs run, the tiles of a later step are requested into the registers just freed, one barrier.
-    auto step = [&](const int kt, f32x4 (&rx)[NX], float (&rw)[8]) {  // rx, rw: the set that holds step kt + 1
-      const u32x4 *stage = lds[kt & 1];
-      u32x4 af[3][MB], bf[3][2];
+    // (smallest products first; the blocks take turns, no MFMA waits for the one before it)
+    if constexpr (PARTS == 3) {
+      // Per step of 16 along K: the fragments are fetched, the next step's tiles are split and go to the other
+      // stage while the MFMAs run, the tiles of a later step are requested into the registers just freed, one barrier.
+      auto step = [&](const int kt, f32x4 (&rx)[NX], float (&rw)[8]) {  // rx, rw: the set that holds step kt + 1
+        const u32x4 *stage = lds[kt & 1];
+        u32x4 af[3][MB], bf[3][NB];
 #pragma unroll
-      for (int p = 0; p < 3; ++p) {
+        for (int p = 0; p < 3; ++p) {
 #pragma unroll
-        for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * S::kPartX + 32 * a];
+          for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * S::kPartX + 32 * a];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) bf[p][b] = stage[b_unit + p * S::kPartW + 36 * b];
+          for (int b = 0; b < NB; ++b) bf[p][b] = stage[b_unit + p * S::kPartW + 36 * b];
+        }
+        park_tiles(rx, rw, lds[(kt & 1) ^ 1]);
+        load_tiles(rx, rw);
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+#pragma unroll
+          for (int a = 0; a < MB; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p]][b], acc[a][b]);
+        __syncthreads();
+      };
+      for (int kt = 0; kt < nk; kt += 2) {
+        step(kt, sx[kSets - 1], sw[kSets - 1]);
+        if (kt + 1 < nk) step(kt + 1, sx[0], sw[0]);
       }
-      park_tiles(rx, rw, lds[(kt & 1) ^ 1]);
-      load_tiles(rx, rw);
-      // smallest products first; the blocks take turns, no MFMA waits for the one before it
+    } else {
+      // Half the MFMAs leave no time for fragments to arrive within their step: they are fetched a step ahead, from the
+      // stage that is whole since the last barrier, and the tiles of the step behind that one go into the stage whose
+      // fragments everybody has.  Everything else a step does is handed out between its MFMAs, one at a time: left
+      // to itself the compiler puts them after each other (2048 rows of 2048 -> 16384: 385 us, 345 this way).
+      u32x4 af[3][MB], first[2][MB], bf[2][NB];  // (the first parts of x and W of two steps)
+      auto fetch_x = [&](const u32x4 *stage, const int p, u32x4 (&f)[MB]) {
 #pragma unroll
-      for (int p = 0; p < 6; ++p)
+        for (int a = 0; a < MB; ++a) f[a] = stage[a_unit + p * S::kPartX + 32 * a];
+      };
+      auto fetch_w = [&](const u32x4 *stage, u32x4 (&f)[NB]) {
 #pragma unroll
-        for (int a = 0; a < MB; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p]][b], acc[a][b]);
+        for (int b = 0; b < NB; ++b) f[b] = stage[b_unit + 36 * b];
+      };
+      fetch_w(lds[0], bf[0]);
+      fetch_x(lds[0], 2, af[2]);
+      fetch_x(lds[0], 1, af[1]);
+      fetch_x(lds[0], 0, first[0]);
+      park_tiles(sx[1], sw[1], lds[1]);
+      load_tiles(sx[1], sw[1]);
       __syncthreads();
-    };
-    for (int kt = 0; kt < nk; kt += 2) {
-      step(kt, sx[kSets - 1], sw[kSets - 1]);
-      if (kt + 1 < nk) step(kt + 1, sx[0], sw[0]);
+      auto step = [&](const int set) {  // set: of this step's fragments and of the tiles of the step after the next
+        u32x4 *const stage = lds[set];
+        const u32x4 *const next = lds[set ^ 1];
+        u32x4 whole[3], h;
+        constexpr int kSlots = 6 * NB, kPairs = NB, kEvery = NB == 4 ? 2 : 1;  // slots; the first with a pair of x; slots per pair
+        constexpr int kPacks = kPairs + 2 * NX * kEvery, kEnd = kPacks + NB;
+#pragma unroll
+        for (int slot = 0; slot < kSlots; ++slot) {
+          const int run = slot / NB, b = slot % NB, p = 2 - run / 2, a = run % 2;
+          acc[a][b] = mfma_bf16(p ? af[p][a] : first[set][a], bf[set][b], acc[a][b]);
+          if (slot < NB) bf[set ^ 1][slot] = next[b_unit + 36 * slot];
+          if (b == NB - 1 && run == 1) fetch_x(next, 2, af[2]);
+          if (b == NB - 1 && run == 2) fetch_x(next, 0, first[set ^ 1]);
+          if (b == NB - 1 && run == 3) fetch_x(next, 1, af[1]);
+          if (slot >= kPairs && slot < kPacks && (slot - kPairs) % kEvery == 0) {
+            const int i = (slot - kPairs) / kEvery;
+            const f32x4 v = sx[set][i / 2];
+            unsigned q[3];
+            split_pair(v[i % 2 * 2] * kLift, v[i % 2 * 2 + 1] * kLift, q[0], q[1], q[2]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              whole[k][i] = q[k];
+              if (NX == 2 && i == 3) stage[x_unit + k * S::kPartX] = whole[k];
+              if (NX == 1 && i == 1) ((u32x2 *)(stage + x_unit + k * S::kPartX))[(xk >> 2) & 1] = u32x2{whole[k][0], whole[k][1]};
+            }
+          }
+          if (slot >= kPacks && slot < kEnd) {
+#pragma unroll
+            for (int i = (slot - kPacks) * 4 / NB; i < (slot - kPacks + 1) * 4 / NB; ++i)
+              h[i] = pack_high(sw[set][2 * i] * kLift, sw[set][2 * i + 1] * kLift);
+            if (slot == kEnd - 1) stage[w_unit] = h;
+          }
+          if (slot == kEnd) load_tiles(sx[set], sw[set]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+      };
+      // (in pairs: a way out between them has the compiler wait for loads of the step before)
+      for (int kt = 1; kt < nk; kt += 2) {
+        step(0);
+        step(1);
+      }
+      if (nk & 1) step(0);
     }
 
-    const int row0 = m0 + wm * 32 * MB + 4 * j, col = n0 + wn * 64 + 2 * ln;
+    const int row0 = m0 + wm * 32 * MB + 4 * j, col = n0 + wn * 32 * NB + NB * ln;
     // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which (2048 rows
     // of 2048 -> 16384 with one NaN in x: 1.3 ms against 0.65 without; one k at a time it was 13.9)
     float probe = 0.f, down = kDrop;
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = fmaf(acc[a][b][r], 0.f, probe);
     if (__any(probe != 0.f)) {
 #pragma unroll
       for (int a = 0; a < MB; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
       // eight k a turn, four of them a lane half's (K is a multiple of 4: those behind its end are zeros on both sides)
@@ -271,46 +390,49 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
         const int k = k0 + 4 * j;
         const bool in = k < k_end;
         f32x4 xv[MB];
-        f32x2 wv[4];
+        typedef float Columns __attribute__((ext_vector_type(NB)));
+        Columns wv[4];
 #pragma unroll
         for (int a = 0; a < MB; ++a)
           xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + (wm * MB + a) * 32 + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          wv[i] = in ? *(const f32x2 *)(g.w + (long long)(k + i) * N + min(col, N - 2)) : f32x2{0.f, 0.f};
+          wv[i] = in ? *(const Columns *)(g.w + (long long)(k + i) * N + min(col, N - NB)) : Columns(0.f);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int a = 0; a < MB; ++a)
 #pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(xv[a][i], wv[i][b], acc[a][b]);
+            for (int b = 0; b < NB; ++b) acc[a][b] = mfma_f32(xv[a][i], wv[i][b], acc[a][b]);
       }
       down = 1.f;
     }
 
-    // A piece travels as [pair of rows][thread] float4: consecutive threads, consecutive 16 bytes.
+    // A piece travels as [pair of rows, or row][thread] float4: consecutive threads, consecutive 16 bytes.
     constexpr long long kSlot = (long long)TM * TN;
-    f32x4 out[8 * MB];
+    constexpr int kOut = 4 * MB * NB;
+    f32x4 out[kOut];
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int r = 0; r < 8; ++r)
-        out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]} * down;
-    // (the thread's offset is taken afresh per tile, or the compiler computes all addresses
-    // before the loops and keeps them in scratch memory)
-    int in_slot = 4 * threadIdx.x;
-    asm volatile("" : "+v"(in_slot));
+      for (int r = 0; r < 4 * NB; ++r) {
+        if constexpr (NB == 2)
+          out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]} * down;
+        else
+          out[16 * a + r] = f32x4{acc[a][0][r], acc[a][1][r], acc[a][2][r], acc[a][3][r]} * down;
+      }
+    const int in_slot = 4 * tid;
     if (g.pieces) {  // the second kernel adds the pieces
       float *slot = g.partials + blockIdx.x * kSlot + in_slot;
 #pragma unroll
-      for (int r = 0; r < 8 * MB; ++r) *(f32x4 *)(slot + r * 512 * WN) = out[r];
+      for (int r = 0; r < kOut; ++r) *(f32x4 *)(slot + r * 4 * NT) = out[r];
       return;
     }
     if (s_end < steps) {
       float *slot = g.partials + blockIdx.x * kSlot + in_slot;
       __builtin_amdgcn_sched_barrier(0);  // all of out[] is in place before the first store is issued
 #pragma unroll
-      for (int r = 0; r < 8 * MB; ++r) coherent_store4(slot + r * 512 * WN, out[r]);
+      for (int r = 0; r < kOut; ++r) coherent_store4(slot + r * 4 * NT, out[r]);
       // the stores are acknowledged (s_waitcnt vmcnt(0): the barrier alone does not wait for them)
       // before the piece is marked complete
       __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -346,21 +468,20 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
       const float *piece = g.partials + (long long)((p_first << g.group_bits) | group) * kSlot + in_slot;
       const long long piece_step = kSlot << g.group_bits;
       for (int i = 0; i < n_before; ++i) {
-        f32x4 v[8 * MB];
 #pragma unroll
-        for (int r = 0; r < 8 * MB; ++r) v[r] = *(const f32x4 *)(piece + i * piece_step + r * 512 * WN);
-        __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first sum waits
+        for (int r0 = 0; r0 < kOut; r0 += 16) {
+          f32x4 v[16];
 #pragma unroll
-        for (int r = 0; r < 8 * MB; ++r) out[r] += v[r];
+          for (int r = 0; r < 16; ++r) v[r] = *(const f32x4 *)(piece + i * piece_step + (r0 + r) * 4 * NT);
+          __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first sum waits
+#pragma unroll
+          for (int r = 0; r < 16; ++r) out[r0 + r] += v[r];
+        }
       }
     }
-    if (col < N) {  // N is a multiple of 4: a lane's two columns are inside together
+    if (col < N) {  // N is a multiple of 4: a lane's columns are inside together
 #pragma unroll
-      for (int r = 0; r < 8 * MB; ++r) {
-        const int row = row0 + 32 * (r >> 3) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
-        store_pair(g, row, col, f32x2{out[r].x, out[r].y});
-        store_pair(g, row + 1, col, f32x2{out[r].z, out[r].w});
-      }
+      for (int r = 0; r < kOut; ++r) store_four<NB>(g, row0, col, r, out[r]);
     }
   }
 }
@@ -375,7 +496,7 @@ __global__ __launch_bounds__(128 * WN, 2) void sgemm_split_kernel(const GemmArgs
 // 64 rows of 1024 -> 1024 12.1 -> 9.2.  64 rows by 128 columns this way were slower than 32 (45 rows of
 // 8192 -> 2048 34 against 30.5).  Bound by a launch, the first loads and the kernel that adds the pieces where the
 // weights are small, by reading them where they are not.
-template <bool GUARD>
+template <int PARTS, bool GUARD>
 __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
   constexpr int TM = 32, TN = 128, TS = kFewStep;
   constexpr int kOct = TM + 4, kPart = 4 * kOct;  // units of 16 bytes: four octets of k, four units apart from a multiple of 16
@@ -444,23 +565,29 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
   __syncthreads();
   auto step = [&](const int kt, const int set) {  // set: holds step kt, the other one step kt + 1
     const u32x4 *stage = lds + (kt & 1) * kStage + (2 * kg + j) * kOct + ln;
-    u32x4 af[3], bf[3][2];
+    u32x4 af[3], bf[PARTS][2];
 #pragma unroll
     for (int p = 0; p < 3; ++p) af[p] = stage[p * kPart];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        unsigned h, m, l;
-        split_pair(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift, h, m, l);
-        bf[0][b][i] = h, bf[1][b][i] = m, bf[2][b][i] = l;
+        if constexpr (PARTS == 3) {
+          unsigned h, m, l;
+          split_pair(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift, h, m, l);
+          bf[0][b][i] = h, bf[1][b][i] = m, bf[2][b][i] = l;
+        } else {
+          bf[0][b][i] = pack_high(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift);
+        }
       }
     park_x(set ^ 1, (kt & 1) ^ 1);
     load_tiles(set);
 #pragma unroll
-    for (int p = 0; p < 5; ++p)
+    for (int p = 0; p < 5; ++p) {
+      if (kPartB[p] >= PARTS) continue;
 #pragma unroll
-      for (int b = 0; b < 2; ++b) rest[b] = mfma_bf16(af[kPartA[p]], bf[kPartB[p]][b], rest[b]);
+      for (int b = 0; b < 2; ++b) rest[b] = mfma_bf16(af[kPartA[p]], bf[kPartB[p] < PARTS ? kPartB[p] : 0][b], rest[b]);
+    }
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[b] = mfma_bf16(af[0], bf[0][b], acc[b]);
     __syncthreads();
@@ -530,26 +657,25 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 }
 
 // y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order.  A piece lies in its
-// workgroup's slot as [pair of rows][thread] float4, the layout of the product kernel's accumulators.
-// A tile's threads are WM x WN wavefronts.
-template <int MB, int WM, int WN>
+// workgroup's slot as [pair of rows, or row][thread] float4, the layout of the product kernel's accumulators.
+// A tile's threads are WM x WN wavefronts of MB x NB blocks.
+template <int WM, int WN, int MB, int NB>
 __global__ __launch_bounds__(64 * WM * WN) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
-  const int tile = blockIdx.x / (8 * MB), r = blockIdx.x % (8 * MB);  // 8 MB workgroups per tile, a pair of rows of each thread each
+  constexpr int kOut = 4 * MB * NB, TM = 32 * WM * MB, TN = 32 * WN * NB;
+  const int tile = blockIdx.x / kOut, r = blockIdx.x % kOut;  // kOut workgroups per tile, a float4 of each thread each
   if (tile >= tiles) return;
   const int group = tile / g.tiles_per_group, t = tile - group * g.tiles_per_group;
-  constexpr int TM = 32 * WM * MB, TN = 64 * WN;
   constexpr long long kSlot = (long long)TM * TN;
   const float *piece = g.partials + (long long)(((t * g.pieces) << g.group_bits) | group) * kSlot + r * 256 * WM * WN + 4 * threadIdx.x;
   const long long piece_step = kSlot << g.group_bits;
   const int n = min(g.pieces, (g.steps + g.quota - 1) / g.quota);  // pieces that hold any steps
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = (tile % g.tiles_m) * TM + (wave / WN) * 32 * MB + 32 * (r >> 3) + 4 * (lane >> 5) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
-  const int col = (tile / g.tiles_m) * TN + (wave % WN) * 64 + 2 * (lane & 31);
-  if (row >= g.T || col >= g.N) return;
+  const int row0 = (tile % g.tiles_m) * TM + (wave / WN) * 32 * MB + 4 * (lane >> 5);
+  const int col = (tile / g.tiles_m) * TN + (wave % WN) * 32 * NB + NB * (lane & 31);
+  if (col >= g.N) return;
   f32x4 acc = *(const f32x4 *)piece;
   for (int c = 1; c < n; ++c) acc += *(const f32x4 *)(piece + c * piece_step);
-  store_pair(g, row, col, f32x2{acc.x, acc.y});
-  store_pair(g, row + 1, col, f32x2{acc.z, acc.w});
+  store_four<NB>(g, row0, col, r, acc);
 }
 
 // Any shape (K or N not a multiple of 4, unaligned rows): one thread per element of y, W read
@@ -587,6 +713,15 @@ int slots_of(int wn) { return wn == 4 ? 256 : 512; }
 //    512                               47 | 37 | 185 | 106 | 57   45 | 36 | 177 | 102 | 58   52 | 44 | 192 | 100 | 64
 //   1024                               87 | 58 | 360 | 197 | 96   82 | 57 | 342 | 186 | 88   80 | 63 | 315 | 173 | 116
 //   2048                               148 | 100 | 717 | 372 | 187  143 | 99 | 674 | 346 | 181  144 | 100 | 619 | 323 | 164
+// W of one part (us; few | 128 x 128 | 128 x 256 | 256 x 256), the same products:
+//     96   18 22 20 29 | 15 20 20 26 | 59 49 46 65 | 34 33 35 48 | 20 26 24 38
+//    128   18 22 20 29 | 18 19 19 26 | 59 52 48 65 | 40 35 36 48 | 21 28 28 38
+//    200   23 25 24 30 | 20 24 24 26 | 108 71 65 68 | 59 48 42 50 | 28 31 29 39
+//    256   28 26 25 30 | 20 24 24 26 | 112 75 65 70 | 62 50 43 53 | 28 32 35 40
+//    512    - 35 32 41 | - 30 28 38 | - 120 99 112 | - 77 60 69 | - 43 41 49
+//    777    - 49 45 53 | - 40 35 45 | - 219 184 172 | - 115 95 103 | - 67 61 71
+//   2048    - 97 85 90 | - 69 61 68 | - 471 391 349 | - 240 197 193 | - 123 106 96
+// so 128 x 128 is not among its tiles, and 256 x 256 cut into pieces pads less than 8 %.
 // A low tile wastes least on few rows, and reads small weights again from the L2 for little: up to 96 rows always, up to
 // 256 where the higher tile would be a fifth padding or the weights are small.
 // The largest needs long runs: at least 36 steps a workgroup.  Less than a round of its tiles is cut into pieces for the
@@ -598,17 +733,20 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 2;
   const long long weights = (long long)K * N, rows1 = (T + 31) / 32 * 32LL, rows2 = (T + 127) / 128 * 128LL;
   p.few = T <= 96 || (T <= 256 && (weights <= (T <= 128 ? 12 : 5) << 20 || rows2 * 100 >= rows1 * 125));
+  if (p.parts == 1) p.few = T <= 96 || (T <= 256 && weights <= (T <= 128 ? 12 : 9) << 20);
   p.few = p.few && (long long)kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows)
   p.mb = 1;
   if (p.few) return;
   p.mb = 2;
-  if (T <= 256) return;
+  if (T <= 256 && p.parts == 3) return;
   p.wn = 4;
+  if (T <= 256) return;
   const long long rows4 = (T + 255) / 256 * 256LL;
   const long long tiles = rows4 / 256 * ((N + 255) / 256), run = tiles * p.steps / slots_of(4);
   const long long last = tiles % slots_of(4);
   const bool fills = tiles < slots_of(4) ? 2 * run < p.steps : last == 0 || 2 * last >= slots_of(4);
-  if (rows4 * 100 <= rows2 * 115 && run >= 36 && fills) p.mb = 4;
+  const int padding = p.parts == 1 && tiles < slots_of(4) ? 108 : 115;
+  if (rows4 * 100 <= rows2 * padding && run >= 36 && fills) p.mb = 4;
 }
 
 }  // namespace
@@ -626,8 +764,9 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[6] = p.mfma && K % (p.few ? kFewStep : TK) != 0;
 }
 
-GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
+GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
   GemmPlan p = {};
+  p.parts = w_bf16 ? 1 : 3;
   // (the kernel addresses the rows of x by 32-bit byte offsets from a base that moves along K)
   p.mfma = T >= 1 && K >= 4 && N >= 4 && (K & 3) == 0 && (N & 3) == 0 && (x_stride & 3) == 0 &&
            (long long)T * x_stride * 4 < 0xffffffffLL && (long long)TK * N * 4 < 0xffffffffLL;
@@ -692,30 +831,31 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride) {
 
 namespace {
 
-template <int MB, int WN>
+template <int WM, int WN, int MB, int NB, int PARTS>
 hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
-  const dim3 grid((unsigned)p.workgroups);
+  const dim3 grid((unsigned)p.workgroups), block(64 * WM * WN);
   if (g.K % TK != 0)
-    hipLaunchKernelGGL((sgemm_split_kernel<MB, WN, true>), grid, dim3(128 * WN), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true>), grid, block, 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_split_kernel<MB, WN, false>), grid, dim3(128 * WN), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false>), grid, block, 0, stream, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || !g.pieces) return e;
   const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL((sgemm_reduce_kernel<MB, 2, WN>), dim3((unsigned)tiles * 8 * MB), dim3(128 * WN), 0, stream, g, tiles);
+  hipLaunchKernelGGL((sgemm_reduce_kernel<WM, WN, MB, NB>), dim3((unsigned)tiles * 4 * MB * NB), block, 0, stream, g, tiles);
   return hipGetLastError();
 }
 
+template <int PARTS>
 hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
   if (g.K % kFewStep != 0)
-    hipLaunchKernelGGL((sgemm_few_kernel<true>), grid, dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_few_kernel<PARTS, true>), grid, dim3(256), 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_few_kernel<false>), grid, dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_few_kernel<PARTS, false>), grid, dim3(256), 0, stream, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || !g.pieces) return e;
   const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL((sgemm_reduce_kernel<1, 1, 2>), dim3((unsigned)tiles * 8), dim3(128), 0, stream, g, tiles);
+  hipLaunchKernelGGL((sgemm_reduce_kernel<1, 2, 1, 2>), dim3((unsigned)tiles * 8), dim3(128), 0, stream, g, tiles);
   return hipGetLastError();
 }
 
@@ -755,9 +895,13 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   g.tiles_per_group = p.tiles_per_group;
   g.quota = p.quota;
   g.pieces = p.pieces > 1 ? p.pieces : 0;
-  if (p.few) return launch_few(g, p, stream);
-  if (p.wn == 4) return p.mb == 4 ? launch_tiles<4, 4>(g, p, stream) : launch_tiles<2, 4>(g, p, stream);
-  return launch_tiles<2, 2>(g, p, stream);
+  if (p.parts == 1) {
+    if (p.few) return launch_few<1>(g, p, stream);
+    return p.mb == 4 ? launch_tiles<4, 2, 2, 4, 1>(g, p, stream) : launch_tiles<2, 4, 2, 2, 1>(g, p, stream);
+  }
+  if (p.few) return launch_few<3>(g, p, stream);
+  if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4, 2, 3>(g, p, stream) : launch_tiles<2, 4, 2, 2, 3>(g, p, stream);
+  return launch_tiles<2, 2, 2, 2, 3>(g, p, stream);
 }
 
 }  // namespace shainet

@@ -11,6 +11,7 @@ struct GemmPlan {
   bool few;               // tiles of 32 rows and 128 columns, K steps of 32
   int mb, wn;             // otherwise tiles of 64 mb rows and 64 wn columns, K steps of 16
   int tiles_m, tiles_n;
+  int parts;              // bf16 numbers that a weight is the sum of: 3, or 1 where the weights are bf16 numbers
   int steps;              // K steps per tile; a unit of work is one step of one tile
   int group_bits;         // 2^group_bits groups of workgroups, each with an equal run of the tiles
   int tiles_per_group;
@@ -20,7 +21,8 @@ struct GemmPlan {
   size_t partial_floats;  // scratch for the pieces of tiles that two or more workgroups share (0: none)
   size_t flag_words;      // words, zero before the first launch (the kernel leaves them zero), that mark pieces complete
 };
-GemmPlan plan_gemm(int T, int K, int N, long long x_stride);
+// w_bf16: every value of W is a bf16 number
+GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16 = false);
 void describe_gemm(const GemmPlan &p, int K, int plan[7]);  // shainet_hip_describe_matmul
 // Device pointers, 16-byte aligned for the MFMA kernel; rows of x are x_stride floats apart, y and
 // res are dense [T, N]; res nullable (y = res + x W; res == y is allowed);

@@ -120,13 +120,15 @@ int check_matrix(const StTensor &t, long long rows, long long cols, int &dtype) 
   return SHAINET_HIP_OK;
 }
 
-// HF [out, in] tensor -> columns [col0, col0 + out) of the device matrix dst [in, ld]
+// HF [out, in] tensor -> columns [col0, col0 + out) of the device matrix dst [in, ld].  bf16 (nullable): set by the
+// matrix's first tensor, the one at column 0, and kept up by the others: whether all of them are stored as bf16.
 int load_transposed(const shainet_safetensors *st, Stager &stage, const std::string &name, int out_dim, int in_dim,
-                    float *dst, long long ld, long long col0) {
+                    float *dst, long long ld, long long col0, bool *bf16 = nullptr) {
   int rc = SHAINET_HIP_OK, dtype;
   const StTensor *t = need(st, name, rc);
   if (!t) return rc;
   if ((rc = check_matrix(*t, out_dim, in_dim, dtype)) || (rc = stage.put(*t))) return rc;
+  if (bf16) *bf16 = (col0 == 0 || *bf16) && dtype == kBF16;
   dim3 grid((unsigned)((in_dim + 31) / 32), (unsigned)((out_dim + 31) / 32));
   hipLaunchKernelGGL(convert_transpose_kernel, grid, dim3(256), 0, nullptr, stage.dev, dst + col0, out_dim, in_dim, ld,
                      dtype);
@@ -304,16 +306,16 @@ int shainet_hf_load_llama(const char *model_dir, shainet_llama_model **out) {
     if (rc) break;
     const long long wide = bb.q_dim + 2LL * bb.kv_dim;
     // attention weights: HF is [out, in], the products are x * W, so [in, out] (hf_loader.cr:325-329)
-    if ((rc = load_transposed(st, stage, p + ".self_attn.q_proj.weight", bb.q_dim, d, bb.w_qkv, wide, 0))) break;
-    if ((rc = load_transposed(st, stage, p + ".self_attn.k_proj.weight", bb.kv_dim, d, bb.w_qkv, wide, bb.q_dim))) break;
+    if ((rc = load_transposed(st, stage, p + ".self_attn.q_proj.weight", bb.q_dim, d, bb.w_qkv, wide, 0, bb.w_qkv_bf16))) break;
+    if ((rc = load_transposed(st, stage, p + ".self_attn.k_proj.weight", bb.kv_dim, d, bb.w_qkv, wide, bb.q_dim, bb.w_qkv_bf16))) break;
     if ((rc = load_transposed(st, stage, p + ".self_attn.v_proj.weight", bb.kv_dim, d, bb.w_qkv, wide,
-                              bb.q_dim + bb.kv_dim)))
+                              bb.q_dim + bb.kv_dim, bb.w_qkv_bf16)))
       break;
-    if ((rc = load_transposed(st, stage, p + ".self_attn.o_proj.weight", d, bb.q_dim, bb.w_o, d, 0))) break;
+    if ((rc = load_transposed(st, stage, p + ".self_attn.o_proj.weight", d, bb.q_dim, bb.w_o, d, 0, bb.w_o_bf16))) break;
     // dense SwiGLU (333-336)
-    if ((rc = load_transposed(st, stage, p + ".mlp.gate_proj.weight", ff, d, bb.gate_up, 2LL * ff, 0))) break;
-    if ((rc = load_transposed(st, stage, p + ".mlp.up_proj.weight", ff, d, bb.gate_up, 2LL * ff, ff))) break;
-    if ((rc = load_transposed(st, stage, p + ".mlp.down_proj.weight", d, ff, bb.down, d, 0))) break;
+    if ((rc = load_transposed(st, stage, p + ".mlp.gate_proj.weight", ff, d, bb.gate_up, 2LL * ff, 0, bb.gate_up_bf16))) break;
+    if ((rc = load_transposed(st, stage, p + ".mlp.up_proj.weight", ff, d, bb.gate_up, 2LL * ff, ff, bb.gate_up_bf16))) break;
+    if ((rc = load_transposed(st, stage, p + ".mlp.down_proj.weight", d, ff, bb.down, d, 0, bb.down_bf16))) break;
     // RMSNorm (349-350)
     if ((rc = load_plain(st, stage, p + ".input_layernorm.weight", 1, d, bb.norm1->gamma))) break;
     if ((rc = load_plain(st, stage, p + ".post_attention_layernorm.weight", 1, d, bb.norm2->gamma))) break;
@@ -357,8 +359,10 @@ int shainet_hf_load_llama(const char *model_dir, shainet_llama_model **out) {
                          d, (long long)V, (int)kF32);
       if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
         rc = fail(SHAINET_HIP_ERR_RUNTIME, "transposing the tied embedding failed");
+      else
+        *mb.lm_head_bf16 = st->find("model.embed_tokens.weight")->dtype == "BF16";
     } else {
-      rc = load_transposed(st, stage, "lm_head.weight", V, d, mb.lm_head, V, 0);
+      rc = load_transposed(st, stage, "lm_head.weight", V, d, mb.lm_head, V, 0, mb.lm_head_bf16);
     }
   }
   shainet_safetensors_close(st);
@@ -512,19 +516,19 @@ int load_latent_mixer(const shainet_safetensors *st, Stager &stage, const std::s
                       LatentWeights &w) {
   const int qw = c.heads * (c.dim + c.rot_dim), kw = c.heads * c.dim, vw = c.heads * c.vdim;
   int rc;
-  if ((rc = load_transposed(st, stage, p + "dq", c.q_rank, d, w.w_in, w.n_in, 0))) return rc;
-  if ((rc = load_transposed(st, stage, p + "dkv", c.kv_rank + c.rot_dim, d, w.w_in, w.n_in, c.q_rank))) return rc;
-  if ((rc = load_transposed(st, stage, p + "g", c.heads, d, w.w_in, w.n_in, c.q_rank + c.kv_rank + c.rot_dim))) return rc;
+  if ((rc = load_transposed(st, stage, p + "dq", c.q_rank, d, w.w_in, w.n_in, 0, &w.w_in_bf16))) return rc;
+  if ((rc = load_transposed(st, stage, p + "dkv", c.kv_rank + c.rot_dim, d, w.w_in, w.n_in, c.q_rank, &w.w_in_bf16))) return rc;
+  if ((rc = load_transposed(st, stage, p + "g", c.heads, d, w.w_in, w.n_in, c.q_rank + c.kv_rank + c.rot_dim, &w.w_in_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "dq.norm", 1, c.q_rank, w.dq_norm))) return rc;
   if ((rc = load_plain(st, stage, p + "dkv.norm", 1, c.kv_rank, w.dkv_norm))) return rc;
-  if ((rc = load_transposed(st, stage, p + "uq", qw, c.q_rank, w.w_uq, qw, 0))) return rc;
+  if ((rc = load_transposed(st, stage, p + "uq", qw, c.q_rank, w.w_uq, qw, 0, &w.w_uq_bf16))) return rc;
   // W_uk and W_uv twice: a row per output (absorbed), and side by side as a product's matrix (expanded)
   if ((rc = load_plain(st, stage, p + "uk", kw, c.kv_rank, w.u_kv))) return rc;
   if ((rc = load_plain(st, stage, p + "uv", vw, c.kv_rank, w.u_kv + (size_t)kw * c.kv_rank))) return rc;
-  if ((rc = load_transposed(st, stage, p + "uk", kw, c.kv_rank, w.w_ukv, kw + vw, 0))) return rc;
-  if ((rc = load_transposed(st, stage, p + "uv", vw, c.kv_rank, w.w_ukv, kw + vw, kw))) return rc;
+  if ((rc = load_transposed(st, stage, p + "uk", kw, c.kv_rank, w.w_ukv, kw + vw, 0, &w.w_ukv_bf16))) return rc;
+  if ((rc = load_transposed(st, stage, p + "uv", vw, c.kv_rank, w.w_ukv, kw + vw, kw, &w.w_ukv_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "sink", 1, c.heads, w.sink))) return rc;
-  if ((rc = load_transposed(st, stage, p + "o", d, vw, w.w_o, d, 0))) return rc;
+  if ((rc = load_transposed(st, stage, p + "o", d, vw, w.w_o, d, 0, &w.w_o_bf16))) return rc;
   w.w_in_t_stale = w.w_uq_t_stale = w.w_o_t_stale = true;
   return SHAINET_HIP_OK;
 }
@@ -560,9 +564,9 @@ int load_tutilorn(const char *model_dir, const Json &j, shainet_llama_model **ou
     if ((rc = load_latent_mixer(st, stage, p + "mix.", d, lc.mixer, latent_attn_weights(shainet_llama_block_latent_mixer(blocks[i]))))) break;
     if (!lc.ff) continue;
     if ((rc = load_norm(st, stage, p + "norm2", d, *bb.norm2))) break;
-    if ((rc = load_transposed(st, stage, p + "mlp.gate", lc.ff, d, bb.gate_up, 2LL * lc.ff, 0))) break;
-    if ((rc = load_transposed(st, stage, p + "mlp.up", lc.ff, d, bb.gate_up, 2LL * lc.ff, lc.ff))) break;
-    if ((rc = load_transposed(st, stage, p + "mlp.down", d, lc.ff, bb.down, d, 0))) break;
+    if ((rc = load_transposed(st, stage, p + "mlp.gate", lc.ff, d, bb.gate_up, 2LL * lc.ff, 0, bb.gate_up_bf16))) break;
+    if ((rc = load_transposed(st, stage, p + "mlp.up", lc.ff, d, bb.gate_up, 2LL * lc.ff, lc.ff, bb.gate_up_bf16))) break;
+    if ((rc = load_transposed(st, stage, p + "mlp.down", d, lc.ff, bb.down, d, 0, bb.down_bf16))) break;
   }
   // the model owns the blocks from here on, in the order of the layers
   for (int i = 0; i < n; ++i)
@@ -576,7 +580,7 @@ int load_tutilorn(const char *model_dir, const Json &j, shainet_llama_model **ou
   if (!rc) rc = shainet_llama_model_buffers(m, &mb);
   if (!rc) rc = load_plain(st, stage, "embed", cfg.vocab, d, mb.embedding);
   if (!rc) rc = load_norm(st, stage, "final.norm", d, *mb.final_norm);
-  if (!rc) rc = load_transposed(st, stage, "head", cfg.vocab, d, mb.lm_head, cfg.vocab, 0);
+  if (!rc) rc = load_transposed(st, stage, "head", cfg.vocab, d, mb.lm_head, cfg.vocab, 0, mb.lm_head_bf16);
   shainet_safetensors_close(st);
   if (rc) {
     shainet_llama_model_destroy(m);
@@ -722,13 +726,13 @@ int load_centred_norm(const shainet_safetensors *st, Stager &stage, const std::s
 int load_hgrn2(const shainet_safetensors *st, Stager &stage, const std::string &p, int d, const Hgrn2Config &c, Hgrn2Weights &w) {
   const int qw = c.heads * c.dim, vw = c.heads * c.vdim;
   int rc;
-  if ((rc = load_transposed(st, stage, p + "q", qw, d, w.w_in, w.n_in, 0))) return rc;
-  if ((rc = load_transposed(st, stage, p + "f", qw, d, w.w_in, w.n_in, qw))) return rc;
-  if ((rc = load_transposed(st, stage, p + "v", vw, d, w.w_in, w.n_in, 2 * qw))) return rc;
+  if ((rc = load_transposed(st, stage, p + "q", qw, d, w.w_in, w.n_in, 0, &w.w_in_bf16))) return rc;
+  if ((rc = load_transposed(st, stage, p + "f", qw, d, w.w_in, w.n_in, qw, &w.w_in_bf16))) return rc;
+  if ((rc = load_transposed(st, stage, p + "v", vw, d, w.w_in, w.n_in, 2 * qw, &w.w_in_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "f.b", 1, qw, w.f_bias))) return rc;
   if ((rc = load_plain(st, stage, p + "lower", 1, qw, w.lower))) return rc;
   if ((rc = load_plain(st, stage, p + "norm", 1, c.vdim, w.norm))) return rc;
-  return load_transposed(st, stage, p + "o", d, vw, w.w_o, d, 0);
+  return load_transposed(st, stage, p + "o", d, vw, w.w_o, d, 0, &w.w_o_bf16);
 }
 
 int load_biased(const shainet_safetensors *st, Stager &stage, const std::string &p, int d, const ZabutarLayer &l, int max_positions,
@@ -737,10 +741,10 @@ int load_biased(const shainet_safetensors *st, Stager &stage, const std::string 
   BiasedWeights &w = biased_attn_weights(mixer);
   const int qw = c.heads * c.dim, kw = c.kv_heads * c.dim, vw = c.kv_heads * c.vdim;
   int rc;
-  if ((rc = load_transposed(st, stage, p + "q", qw, d, w.w_in, w.n_in, 0))) return rc;
+  if ((rc = load_transposed(st, stage, p + "q", qw, d, w.w_in, w.n_in, 0, &w.w_in_bf16))) return rc;
   if (l.kv_from < 0) {
-    if ((rc = load_transposed(st, stage, p + "k", kw, d, w.w_in, w.n_in, qw))) return rc;
-    if ((rc = load_transposed(st, stage, p + "v", vw, d, w.w_in, w.n_in, qw + kw))) return rc;
+    if ((rc = load_transposed(st, stage, p + "k", kw, d, w.w_in, w.n_in, qw, &w.w_in_bf16))) return rc;
+    if ((rc = load_transposed(st, stage, p + "v", vw, d, w.w_in, w.n_in, qw + kw, &w.w_in_bf16))) return rc;
   }
   const StTensor *t = need(st, p + "rel", rc);
   if (!t) return rc;
@@ -749,14 +753,14 @@ int load_biased(const shainet_safetensors *st, Stager &stage, const std::string 
   std::vector<float> rel;
   if ((rc = read_host_vector(st, p + "rel", rel))) return rc;
   if ((rc = biased_attn_set_table(mixer, rel, (int)t->shape[0], max_positions))) return rc;
-  return load_transposed(st, stage, p + "o", d, c.heads * c.vdim, w.w_o, d, 0);
+  return load_transposed(st, stage, p + "o", d, c.heads * c.vdim, w.w_o, d, 0, &w.w_o_bf16);
 }
 
 int load_xielu(const shainet_safetensors *st, Stager &stage, const std::string &p, int d, int ff, DenseWeights &w) {
   int rc;
-  if ((rc = load_transposed(st, stage, p + "up", ff, d, w.up, ff, 0))) return rc;
+  if ((rc = load_transposed(st, stage, p + "up", ff, d, w.up, ff, 0, &w.up_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "up.b", 1, ff, w.up_bias))) return rc;
-  if ((rc = load_transposed(st, stage, p + "down", d, ff, w.down, d, 0))) return rc;
+  if ((rc = load_transposed(st, stage, p + "down", d, ff, w.down, d, 0, &w.down_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "down.b", 1, d, w.down_bias))) return rc;
   std::vector<float> act;
   if ((rc = read_host_vector(st, p + "act", act))) return rc;
@@ -773,13 +777,16 @@ int load_experts(const shainet_safetensors *st, Stager &stage, const std::string
   const size_t mat = (size_t)m.ff * m.d;
   int rc;
   if ((rc = load_plain(st, stage, p + "router", n, m.d, w.router))) return rc;
-  if ((rc = load_transposed(st, stage, p + "router", n, m.d, w.router_in, w.n_router, 0))) return rc;
+  if ((rc = load_transposed(st, stage, p + "router", n, m.d, w.router_in, w.n_router, 0, &w.router_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "correction", 1, n, w.correction))) return rc;
+  w.gate_up_bf16 = w.down_bf16 = true;
   for (int e = 0; e < m.experts; ++e) {
     const std::string pe = p + "e" + std::to_string(e) + ".";
     if ((rc = load_plain(st, stage, pe + "gate", m.ff, m.d, w.gate_up + 2 * e * mat))) return rc;
     if ((rc = load_plain(st, stage, pe + "up", m.ff, m.d, w.gate_up + (2 * e + 1) * mat))) return rc;
     if ((rc = load_plain(st, stage, pe + "down", m.d, m.ff, w.down + e * mat))) return rc;
+    w.gate_up_bf16 = w.gate_up_bf16 && st->find(pe + "gate")->dtype == "BF16" && st->find(pe + "up")->dtype == "BF16";
+    w.down_bf16 = w.down_bf16 && st->find(pe + "down")->dtype == "BF16";
   }
   if (!m.shared_ff) return SHAINET_HIP_OK;
   const std::string ps = p + "shared.";
@@ -787,9 +794,9 @@ int load_experts(const shainet_safetensors *st, Stager &stage, const std::string
   if ((rc = load_plain(st, stage, ps + "gate", ff, m.d, w.shared_gate_up))) return rc;
   if ((rc = load_plain(st, stage, ps + "up", ff, m.d, w.shared_gate_up + (size_t)ff * m.d))) return rc;
   if ((rc = load_plain(st, stage, ps + "down", m.d, ff, w.shared_down))) return rc;
-  if ((rc = load_transposed(st, stage, ps + "gate", ff, m.d, w.shared_gate_up_in, 2LL * ff, 0))) return rc;
-  if ((rc = load_transposed(st, stage, ps + "up", ff, m.d, w.shared_gate_up_in, 2LL * ff, ff))) return rc;
-  return load_transposed(st, stage, ps + "down", m.d, ff, w.shared_down_in, m.d, 0);
+  if ((rc = load_transposed(st, stage, ps + "gate", ff, m.d, w.shared_gate_up_in, 2LL * ff, 0, &w.shared_gate_up_bf16))) return rc;
+  if ((rc = load_transposed(st, stage, ps + "up", ff, m.d, w.shared_gate_up_in, 2LL * ff, ff, &w.shared_gate_up_bf16))) return rc;
+  return load_transposed(st, stage, ps + "down", m.d, ff, w.shared_down_in, m.d, 0, &w.shared_down_bf16);
 }
 
 // One layer: its parts made and filled.
@@ -850,7 +857,7 @@ int load_zabutar(const char *model_dir, const Json &j, shainet_llama_model **out
   if (!rc) rc = load_plain(st, stage, "embed", cfg.vocab, d, mb.embedding);
   if (!rc) rc = load_plain(st, stage, "pos", cfg.max_positions, d, positions);
   if (!rc) rc = load_centred_norm(st, stage, "final.norm", d, mb.final_norm->gamma);
-  if (!rc) rc = load_transposed(st, stage, "head", cfg.vocab, d, mb.lm_head, cfg.vocab, 0);
+  if (!rc) rc = load_transposed(st, stage, "head", cfg.vocab, d, mb.lm_head, cfg.vocab, 0, mb.lm_head_bf16);
   shainet_safetensors_close(st);
   if (rc) {
     shainet_llama_model_destroy(m);

@@ -82,6 +82,7 @@ struct Hgrn2 : Mixer {
         (no_cache && !other_state.reserve(state_floats())))
       return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     Fused in = pre;
+    in.w_bf16 = w.w_in_bf16;
     if (gemvt_takes(T, d, w.n_in, in.epilogue, in.norm)) in.w_t = transposed_twin(&w.w_in_t, &w.w_in_t_stale, w.w_in, d, w.n_in, cur_stream);
     int rc = proj.project(x, d, w.w_in, raw.p, T, d, w.n_in, cur_stream, in);
     if (rc) return rc;
@@ -103,6 +104,7 @@ struct Hgrn2 : Mixer {
     if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("hgrn2 launch: ") + hipGetErrorString(e));
     if (!no_cache) rows += T;
     Fused post;
+    post.w_bf16 = w.w_o_bf16;
     if (residual) {
       post.epilogue = kGemvResidual;
       post.res = residual;

@@ -15,6 +15,7 @@ struct Hgrn2Weights {
   float *w_o = nullptr, *w_o_t = nullptr;     // [heads vdim, d]
   int n_in = 0;
   bool w_in_t_stale = true, w_o_t_stale = true;
+  bool w_in_bf16 = false, w_o_bf16 = false;  // every value is a bf16 number: the loader says so
 };
 int hgrn2_create(Mixer **out, int d_model, const Hgrn2Config &cfg, double eps);
 Hgrn2Weights &hgrn2_weights(Hgrn2 *l);

@@ -170,6 +170,7 @@ int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const 
 
   // [c_q | c | key part | gates]
   Fused in = pre;
+  in.w_bf16 = w.w_in_bf16;
   if (gemvt_takes(T, d, w.n_in, in.epilogue, in.norm)) in.w_t = transposed_twin(&w.w_in_t, &w.w_in_t_stale, w.w_in, d, w.n_in, stream);
   if ((rc = l->proj.project(x, d, w.w_in, l->raw.p, T, d, w.n_in, stream, in))) return rc;
   // q = RMS(c_q) W_uq
@@ -181,6 +182,7 @@ int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const 
     up.w_t = transposed_twin(&w.w_uq_t, &w.w_uq_t_stale, w.w_uq, q_rank, qw, stream, w.dq_norm);
     up.w_t_has_gamma = up.w_t != nullptr;
   }
+  up.w_bf16 = w.w_uq_bf16;
   if ((rc = l->proj.project(l->raw.p, w.n_in, w.w_uq, l->q.p, T, q_rank, qw, stream, up))) return rc;
 
   LatentRows r = {};
@@ -203,8 +205,10 @@ int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const 
     e = launch_latent_append(r, sh, T, l->q.p, stream);
     if (e == hipSuccess) {
       // keys and values of every position the new rows see
+      Fused expand;
+      expand.w_bf16 = w.w_ukv_bf16;
       if ((rc = l->proj.project(cache->k + (size_t)ex.first_row * sh.row_w, sh.row_w, w.w_ukv, l->kv.p, ex.key_rows,
-                                sh.kv_rank, kvw, stream)))
+                                sh.kv_rank, kvw, stream, expand)))
         return rc;
       e = launch_latent_expanded(l->q.p, l->kv.p, w.sink, r, sh, T, ex, l->partials.p, l->heads.p, stream);
     }
@@ -229,6 +233,7 @@ int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const 
     post.epilogue = kGemvResidual;
     post.res = residual;
   }
+  post.w_bf16 = w.w_o_bf16;
   if (gemvt_takes(T, vw, d, post.epilogue, post.norm)) post.w_t = transposed_twin(&w.w_o_t, &w.w_o_t_stale, w.w_o, vw, d, stream);
   return l->proj.project(l->heads.p, vw, w.w_o, out, T, vw, d, stream, post);
 }

@@ -22,6 +22,7 @@ struct LatentWeights {
   float *sink = nullptr;                     // [H]
   float *w_o = nullptr, *w_o_t = nullptr;    // [H vdim, d_model]
   bool w_in_t_stale = true, w_uq_t_stale = true, w_o_t_stale = true;
+  bool w_in_bf16 = false, w_uq_bf16 = false, w_ukv_bf16 = false, w_o_bf16 = false;  // every value is a bf16 number: the loader says so
   int n_in = 0;
   ~LatentWeights();
 };

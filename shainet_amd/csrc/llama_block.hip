@@ -57,6 +57,7 @@ struct shainet_llama_attn {
   // (and q | k | v, [q_dim + 2 kv_dim, d_model], for layers without QK-norm)
   float *w_o_t = nullptr, *w_qkv_t = nullptr;
   bool w_o_t_stale = true, w_qkv_t_stale = true;
+  bool w_qkv_bf16 = false, w_o_bf16 = false;  // every value is a bf16 number
   // the norm weights multiplied into the rows of w_qkv_t (null: none), and whether any were
   const float *w_qkv_t_gamma = nullptr;
   shainet_attn_ctx *ctx = nullptr;
@@ -161,23 +162,23 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
   // takes 10.2 (1024 -> 2048).
   bool norm_apart = T == 1 && (l->has_q_norm || l->has_k_norm) && gemvt_takes(T, l->d_model, wide, pre.epilogue, pre.norm);
   if (norm_apart) {
-    Fused qkv = pre;
-    take_transposed(qkv);
-    norm_apart = qkv.w_t != nullptr;
+    Fused twin = pre;
+    take_transposed(twin);
+    norm_apart = twin.w_t != nullptr;
   }
+  Fused qkv = pre;
+  qkv.w_bf16 = l->w_qkv_bf16;
   if (!fuse_off && !norm_apart && T <= 16 && Projector::few_rows(T, l->d_model, wide, l->d_model) && (wide & 3) == 0 && hd >= 2 && hd <= 128 && (hd & (hd - 1)) == 0) {
     // few rows: bias, QK-norm, RoPE and the cache append (256-286, 332-344) happen where the
     // product's head rows are summed up; the attention kernel follows directly
     GemvPrep where;
     if ((rc = shainet_attn_begin_prepared(l->ctx, cache, T, &where))) return rc;
-    Fused qkv = pre;
     qkv.epilogue = kGemvQkvPrep;
     qkv.prep = &where;
     if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm, &where)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, nullptr, T, l->d_model, wide, stream, qkv))) return rc;
     rc = shainet_attn_finish_prepared(l->ctx, cache, T, l->attn.p, ahead);  // 287-296
   } else {
-    Fused qkv = pre;
     if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, l->qkv.p, T, l->d_model, wide, stream, qkv))) return rc;
     rc = shainet_attn_forward_strided(l->ctx, cache, nullptr, &T, 1, l->qkv.p, l->qkv.p + l->q_dim,
@@ -191,6 +192,7 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     l->cache_len = total_len;
   }
   Fused post;
+  post.w_bf16 = l->w_o_bf16;
   if (residual) {
     post.epilogue = kGemvResidual;
     post.res = residual;
@@ -279,6 +281,7 @@ int shainet_llama_attn_set_weights(shainet_llama_attn *l, const float *w_q, cons
   int rc = upload_side_by_side(&l->w_qkv, mats, widths, 3, l->d_model);
   if (!rc) rc = upload_floats(&l->w_o, w_o, (size_t)l->q_dim * l->d_model);
   l->w_o_t_stale = l->w_qkv_t_stale = true;
+  l->w_qkv_bf16 = l->w_o_bf16 = false;
   return rc;
 }
 
@@ -335,6 +338,7 @@ struct BlockWeights {
   float *gate_up = nullptr, *down = nullptr;        // device [d_model, 2*ff] (gate | up) and [ff, d_model]
   float *gate_up_t = nullptr, *down_t = nullptr;    // the same transposed ([2*ff, d_model], [d_model, ff]), like w_o_t
   bool gate_up_t_stale = true, down_t_stale = true;
+  bool gate_up_bf16 = false, down_bf16 = false;     // every value is a bf16 number
   // wrapped blocks: norms behind the sublayers [d_model], convolutions in front of them [taps, d_model], and a
   // feed-forward of another kind (null: none)
   float *post1 = nullptr, *post2 = nullptr, *conv1 = nullptr, *conv2 = nullptr;
@@ -497,6 +501,7 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
   Fused gate;
   w.norm2.apply(gate, b->eps);
   gate.epilogue = kGemvSwiglu;
+  gate.w_bf16 = w.gate_up_bf16;
   if (ff && gemvt_takes(T, d, ff, gate.epilogue, gate.norm)) {
     // (the RMSNorm weights ride in the copy; Dynamic Tanh adds beta behind its own, so they stay outside)
     const float *ride = gate.norm == kNormRms ? gate.gamma : nullptr;
@@ -521,6 +526,7 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
   Fused down;
   down.epilogue = kGemvResidual;
   down.res = h;
+  down.w_bf16 = w.down_bf16;
   if (gemvt_takes(T, ff, d, down.epilogue, down.norm)) down.w_t = transposed_twin(&w.down_t, &w.down_t_stale, w.down, ff, d, stream);
   return proj.project(b->hidden.p, ff, w.down, out, T, ff, d, stream, down);
 }
@@ -570,8 +576,11 @@ int shainet_llama_block_buffers(shainet_llama_block *b, LlamaBlockBuffers *out) 
   // (whoever asks for the buffers is about to write the weights: the transposed copies are made again)
   bw.gate_up_t_stale = bw.down_t_stale = true;
   if (l) l->w_o_t_stale = l->w_qkv_t_stale = true;
+  bw.gate_up_bf16 = bw.down_bf16 = false;
+  if (l) l->w_qkv_bf16 = l->w_o_bf16 = false;
   *out = LlamaBlockBuffers{l ? l->w_qkv : nullptr, l ? l->w_o : nullptr, bw.gate_up, bw.down,
-                           &bw.norm1,  &bw.norm2,  b->d_model,  l ? l->q_dim : 0, l ? l->kv_dim : 0, b->ff_hidden};
+                           &bw.norm1,  &bw.norm2,  b->d_model,  l ? l->q_dim : 0, l ? l->kv_dim : 0, b->ff_hidden,
+                           l ? &l->w_qkv_bf16 : nullptr, l ? &l->w_o_bf16 : nullptr, &bw.gate_up_bf16, &bw.down_bf16};
   return SHAINET_HIP_OK;
 }
 
@@ -798,6 +807,7 @@ int shainet_llama_block_set_ffn(shainet_llama_block *b, const float *gate, const
   int rc = upload_side_by_side(&b->w->gate_up, mats, widths, 2, b->d_model);
   if (!rc) rc = upload_floats(&b->w->down, down, (size_t)b->ff_hidden * b->d_model);
   b->w->gate_up_t_stale = b->w->down_t_stale = true;
+  b->w->gate_up_bf16 = b->w->down_bf16 = false;
   return rc;
 }
 

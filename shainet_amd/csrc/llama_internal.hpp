@@ -46,6 +46,8 @@ struct LlamaBlockBuffers {
   float *w_qkv, *w_o, *gate_up, *down;  // w_qkv, w_o: null where the mixer is latent attention; gate_up, down: where there is no feed-forward
   shainet::NormWeights *norm1, *norm2;
   int d_model, q_dim, kv_dim, ff_hidden;
+  // for the loader to say: every value of the matrix is a bf16 number (false until then)
+  bool *w_qkv_bf16, *w_o_bf16, *gate_up_bf16, *down_bf16;
 };
 int shainet_llama_block_buffers(shainet_llama_block *b, LlamaBlockBuffers *out);
 // A block whose mixer is latent attention (latent_attn.hpp), its norms of one kind (kNorm*), with a
@@ -77,6 +79,7 @@ struct LlamaModelBuffers {
   float *embedding;
   shainet::NormWeights *final_norm;
   float *lm_head;
+  bool *lm_head_bf16;  // for the loader to say: every value is a bf16 number (false until then)
 };
 // Position vectors [max_positions, d_model] that are added to the embedding rows: the buffer, allocated on first
 // request, for a loader to fill.  A sequence cannot outgrow them.
@@ -117,6 +120,7 @@ struct Fused {
   // the same weights transposed ([N, K]; kGemvSwiglu: [2N, K]) or null: one row of x then takes the
   // product that gives a wavefront whole outputs (launch_gemvt) where its shapes allow
   const float *w_t = nullptr;
+  bool w_bf16 = false;  // every value of W is a bf16 number: half the MFMAs of many rows have nothing to add
   bool any_few_rows = false;  // up to 16 rows run as the split GEMV, not only the ones it is the faster product for
   bool w_t_has_gamma = false;  // the rows of w_t were made with gamma multiplied in: the norm's factor 1 / rms is all that is left to apply
 };
@@ -168,7 +172,7 @@ struct Projector {
  private:
   int reserve_flags(size_t n_flags, hipStream_t stream);
   // res != nullptr: y = res + x W
-  int gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N, hipStream_t stream,
+  int gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N, hipStream_t stream, bool w_bf16,
            const float *res = nullptr, const float *bias = nullptr, Activation act = Activation());
 };
 

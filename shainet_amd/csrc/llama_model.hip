@@ -82,6 +82,7 @@ struct shainet_llama_model {
   const float *lm_head_t = nullptr;
   float *lm_head_t_own = nullptr;
   bool lm_head_t_stale = true;
+  bool lm_head_bf16 = false;  // every value is a bf16 number
   float *lm_bias = nullptr;     // device [vocab] or null
   hipStream_t stream = nullptr;
   int *error = nullptr;  // pinned host word: set by any kernel of the model that gave up a bounded wait
@@ -122,9 +123,10 @@ int shainet_llama_model_buffers(shainet_llama_model *m, LlamaModelBuffers *out) 
     }
   m->has_final_norm = true;
   m->lm_head_t_stale = true;  // (whoever asks for the buffers is about to write them)
+  m->lm_head_bf16 = false;
   if (m->lm_bias) (void)hipFree(m->lm_bias);  // the loader's output bias is all zeros (hf_loader.cr:404)
   m->lm_bias = nullptr;
-  *out = LlamaModelBuffers{m->embedding, &m->final_norm, m->lm_head};
+  *out = LlamaModelBuffers{m->embedding, &m->final_norm, m->lm_head, &m->lm_head_bf16};
   return SHAINET_HIP_OK;
 }
 
@@ -336,6 +338,7 @@ int head_rows(shainet_llama_model *m, const float *x, int n, float *logits) {
   const int d = m->d_model;
   Fused fin;
   if (m->has_final_norm) m->final_norm.apply(fin, m->eps);
+  fin.w_bf16 = m->lm_head_bf16;
   if (gemvt_takes(n, d, m->vocab, fin.epilogue, fin.norm)) fin.w_t = lm_head_twin(m);
   if (int rc = m->proj.project(x, d, m->lm_head, logits, n, d, m->vocab, m->stream, fin)) return rc;
   for (int i = 0; m->lm_bias && i < n; ++i) {
@@ -494,6 +497,7 @@ int shainet_llama_model_set_lm_head(shainet_llama_model *m, const float *w, cons
   if (!m || !w) return fail(SHAINET_HIP_ERR_ARGUMENT, "null argument");
   if (!shainet_hip_available()) return fail(SHAINET_HIP_ERR_RUNTIME, "no gfx950 device available");
   m->lm_head_t_stale = true;
+  m->lm_head_bf16 = false;
   int rc = upload_floats(&m->lm_head, w, (size_t)m->d_model * m->vocab);
   if (rc) return rc;
   if (bias) return upload_floats(&m->lm_bias, bias, (size_t)m->vocab);

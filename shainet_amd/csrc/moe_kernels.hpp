@@ -25,6 +25,7 @@ struct MoeTensors {
   const float *router, *correction;            // [experts + identity, d], [experts + identity]
   const float *gate_up, *down;                 // [experts][2 ff, d] (gate rows, then up rows), [experts][d, ff]
   const float *shared_gate_up, *shared_down;   // [2 shared_ff, d], [d, shared_ff]
+  bool gate_up_bf16, down_bf16;                // every value is a bf16 number
 };
 bool moe_shape_ok(const MoeShape &m);
 

@@ -133,8 +133,8 @@ int Projector::reserve_flags(size_t n_flags, hipStream_t stream) {
 
 // y = (res +) x W with the library's own MFMA kernel; res == y is allowed.
 int Projector::gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
-                    hipStream_t stream, const float *res, const float *bias, Activation act) {
-  const GemmPlan p = plan_gemm(T, K, N, x_stride);
+                    hipStream_t stream, bool w_bf16, const float *res, const float *bias, Activation act) {
+  const GemmPlan p = plan_gemm(T, K, N, x_stride, w_bf16);
   if (!scratch.reserve(p.partial_floats)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   if (int rc = reserve_flags(p.flag_words, stream)) return rc;
   if (p.flag_words && !error) return llama_fail(SHAINET_HIP_ERR_RUNTIME, "the projector has no error word");
@@ -242,13 +242,13 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
   }
   if (swiglu) {
     if (!wide.reserve((size_t)T * 2 * N)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-    int rc = gemm(xin, xs, w, wide.p, T, K, 2 * N, stream);
+    int rc = gemm(xin, xs, w, wide.p, T, K, 2 * N, stream, f.w_bf16);
     if (rc) return rc;
     e = launch_swiglu_act(wide.p, y, T, N, stream);
     if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("epilogue launch: ") + hipGetErrorString(e));
     return SHAINET_HIP_OK;
   }
-  return gemm(xin, xs, w, y, T, K, N, stream, f.epilogue == kGemvResidual ? f.res : nullptr,
+  return gemm(xin, xs, w, y, T, K, N, stream, f.w_bf16, f.epilogue == kGemvResidual ? f.res : nullptr,
               f.epilogue == kGemvBias ? f.bias : nullptr, f.act);
 }
 

@@ -59,6 +59,11 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
+// two floats that are bf16 numbers, packed the same way
+__device__ __forceinline__ unsigned pack_high(float a, float b) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
+}
+
 // the three parts of two floats, packed
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &high, unsigned &mid, unsigned &low) {
   high = pack_bf16(a, b);
