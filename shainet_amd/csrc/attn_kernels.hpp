@@ -164,7 +164,12 @@ struct DecodeArgs {
 // slots and the columns; everything that depends on the cached lengths is read from *dev.
 hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &sh, const DecodePlan &p, float scale,
                          hipStream_t stream, hipEvent_t before = nullptr, hipEvent_t after = nullptr,
-                         const DecodeDevicePlan *dev = nullptr, const DistanceBias *bias = nullptr);
+                         const DecodeDevicePlan *dev = nullptr, const DistanceBias *bias = nullptr,
+                         const PrepArgs *prep = nullptr);
+// Whether launch_decode takes the rows of a projection as they are (prep), norms, rotates and appends them itself: one
+// new row per sequence without biases, head_dim 64 or 128, spans that end with the pairs, 16-byte pieces, and an
+// output that lies apart from the inputs, which workgroups still read when the first outputs are written.
+bool decode_prepares(const PrepArgs &a, const SeqTable &st, const Shape &sh, const DecodePlan &p, const float *out);
 // Key splits of a prefill launch: 1 when the row blocks alone fill the chip, more
 // when they do not (few new rows on a long cached prefix); each split leaves
 // partial rows in `partials` (prefill_partial_floats) and a second kernel merges.

@@ -299,11 +299,12 @@ int run_attention(shainet_attn_ctx *c, const float *q_rot, float *kc, float *vc,
     d.error = c->error;
     d.spin_limit = c->test_lose_marks ? 2000 : 0;
     if (ahead) d.ahead = *ahead;
-    if (prep) {
+    const bool fused = prep && !bias && decode_prepares(*prep, att, sh, plan, out);
+    if (prep && !fused) {
       e = launch_prep(*prep, st, sh, total_tokens, stream);
       if (e != hipSuccess) return hip_fail(e, "prep launch");
     }
-    e = launch_decode(d, att, sh, plan, scale, stream, ev0, ev1, nullptr, bias);
+    e = launch_decode(d, att, sh, plan, scale, stream, ev0, ev1, nullptr, bias, fused ? prep : nullptr);
   } else {
     if (prep) {
       e = launch_prep(*prep, st, sh, total_tokens, stream);

@@ -207,19 +207,133 @@ struct ReadAhead {
   const float *w;  // [2 n, k]
   int k, n, first_wg;
 };
+
+// The arithmetic of norm_rotate_pair (prep_math.hpp) in the layouts of the kernel below, the same bits: no product fuses
+// into an add.
+#pragma clang fp contract(off)
+__device__ __forceinline__ void norm_rotate_quad(f32x4 &x0, f32x4 &x1, bool has_w, f32x4 w0, f32x4 w1, float inv, f32x4 cs01,
+                                                 f32x4 cs23) {
+#pragma clang fp contract(off)
+  const f32x4 c = {cs01.x, cs01.z, cs23.x, cs23.z}, s = {cs01.y, cs01.w, cs23.y, cs23.w};
+  if (has_w) {
+    x0 = x0 * inv;
+    x0 = x0 * w0;
+    x1 = x1 * inv;
+    x1 = x1 * w1;
+  }
+  const f32x4 p0 = x0 * c, p1 = x1 * s, p2 = x1 * c, p3 = x0 * s;
+  x0 = p0 - p1;
+  x1 = p2 + p3;
+}
+
+// 1 / rms of up to 32 head rows, the squares of a row added up one after the other as the reference does: lane r walks
+// the first half of row r, lane 32 + r goes on with the second.
+template <int HD>
+struct SquareSum {
+  f32x4 x[HD / 8];
+  __device__ __forceinline__ void request(const float *row, int lane) {  // row: lane % 32's
+#pragma unroll
+    for (int i = 0; i < HD / 8; ++i) x[i] = *(const f32x4 *)(row + (lane >> 5) * (HD / 2) + 4 * i);
+  }
+  __device__ __forceinline__ float add_up(float ss) const {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int i = 0; i < HD / 8; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float sq = x[i][e] * x[i][e];
+        ss = ss + sq;
+      }
+    return ss;
+  }
+  __device__ __forceinline__ float factor(double eps, int lane) const {  // in lanes 32 + r
+    const float first = add_up(0.0f);
+    const float mean = add_up(__shfl(first, lane & 31)) / (float)HD;
+    return (float)(1.0 / sqrt((double)mean + eps));
+  }
+};
+
+// Queries as the score MFMAs take them: lane group j holds elements 16 i + 4 j .. + 3 of a head, and so both halves
+// of its pairs.
+template <int HD>
+struct PreparedQueries {
+  static constexpr int NT = HD / 16;
+  f32x4 x[NT], w[NT], cs[NT];
+  __device__ __forceinline__ void request(const float *row, const float *norm, const float2 *table, int j) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      x[i] = *(const f32x4 *)(row + 16 * i + 4 * j);
+      w[i] = norm ? *(const f32x4 *)(norm + 16 * i + 4 * j) : f32x4{1.f, 1.f, 1.f, 1.f};
+      cs[i] = *(const f32x4 *)(table + 16 * (i / 2) + 4 * j + 2 * (i % 2));
+    }
+  }
+  __device__ __forceinline__ void finish(bool has_w, float inv, float (&q)[HD / 4]) {
+#pragma unroll
+    for (int i = 0; i < NT / 2; ++i) {
+      norm_rotate_quad(x[i], x[i + NT / 2], has_w, w[i], w[i + NT / 2], inv, cs[2 * i], cs[2 * i + 1]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q[4 * i + e] = x[i][e], q[4 * (i + NT / 2) + e] = x[i + NT / 2][e];
+    }
+  }
+};
+
+// The new key and value row of a pair, in one wavefront: lane l holds elements 4 l .. + 3 and HD / 2 + 4 l .. + 3 of the
+// key (l < HD / 8, the others as lane l % (HD / 8)), and 4 (l % 16) .. + 3 of every 64 of the value.
+template <int HD>
+struct NewRow {
+  static constexpr int kLanes = HD / 8;
+  f32x4 key[2], w[2], cs[2], value[HD / 64];
+  __device__ __forceinline__ void request(const float *k, const float *v, const float *norm, const float2 *table, int lane) {
+    const int e = 4 * (lane % kLanes);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      key[h] = *(const f32x4 *)(k + h * (HD / 2) + e);
+      w[h] = norm ? *(const f32x4 *)(norm + h * (HD / 2) + e) : f32x4{1.f, 1.f, 1.f, 1.f};
+      cs[h] = *(const f32x4 *)(table + e + 2 * h);
+    }
+#pragma unroll
+    for (int u = 0; u < HD / 64; ++u) value[u] = *(const f32x4 *)(v + 64 * u + 4 * (lane & 15));
+  }
+  __device__ __forceinline__ void finish(bool has_w, float inv) { norm_rotate_quad(key[0], key[1], has_w, w[0], w[1], inv, cs[0], cs[1]); }
+  // into row `row` of a K tile in LDS
+  __device__ __forceinline__ void put_key(char *tile, int row, int lane) const {
+    if (lane >= kLanes) return;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) *(f32x4 *)(tile + row * (HD * 4) + (((lane + h * kLanes) ^ row) << 4)) = key[h];
+  }
+  __device__ __forceinline__ void append(float *k, float *v, int lane) const {
+    if (lane < kLanes) {
+      *(f32x4 *)(k + 4 * lane) = key[0];
+      *(f32x4 *)(k + HD / 2 + 4 * lane) = key[1];
+    }
+#pragma unroll
+    for (int u = 0; u < HD / 64; ++u)
+      if (lane < 16) *(f32x4 *)(v + 64 * u + 4 * lane) = value[u];
+  }
+};
+#pragma clang fp contract(fast)
+
 // AHEAD: workgroups from ah.first_wg on (a multiple of 8) do not attend: workgroup first_wg + j
 // reads the rows 4 j .. 4 j + 3 and n + the same of ah.w with ordinary loads and drops them, so
 // that the launch that needs them next finds them in its XCD's L2 (a decode step of one sequence
 // leaves the memory system idle while it waits on its chain of dependent loads).
+// PREP: q, k and v are a projection's rows, one new row per sequence, and every workgroup has one segment
+// (DecodePlan::align): each wavefront norms and rotates the queries of its group for itself, the one that holds the
+// pair's last tile does the same for the new key, puts it and the new value in the place of the tile's rows
+// from L - 1 on, which are not in memory yet, and appends them behind its last tile.  The launch in front that did all
+// this, and the wait between the two, are gone: one sequence of 1024 positions, 8 kv heads of 64, 10.8 -> 6.7 us a call; a
+// step of a QK-normed model of width 1024 3 us shorter per layer.  The sums of squares are a chain of hd additions (0.2
+// to 0.5 us), which the first tile's way hides.
 // BIAS (with PAD): scores gain a value by distance (DistanceBias), value rows have a width of their own.
-template <int HD, int NW, bool DEV, bool PAD, bool AHEAD = false, bool BIAS = false>
+template <int HD, int NW, bool DEV, bool PAD, bool AHEAD = false, bool BIAS = false, bool PREP = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_splitk_kernel(
     const float *__restrict__ q_rot, const float *__restrict__ kc, const float *__restrict__ vc,
     float *__restrict__ out, float *part_o, float *part_ml, unsigned *part_flag, unsigned *flag_set,
     int spin_limit, int *error, SeqTable st_arg, Shape sh, int tiles_per_wg_arg, SpanTable sp_arg, int total_tiles_arg,
     int align_arg, unsigned align_by_arg, int n_slots, int pstride, float c, unsigned rotate, const DecodeDevicePlan *__restrict__ dev, ReadAhead ah,
-    DistanceBias db) {
+    DistanceBias db, PrepArgs raw) {
   static_assert(PAD || !BIAS, "sizes of their own come with padding");
+  static_assert(!PREP || (!PAD && !DEV && HD <= 128), "preparation of plain host-planned rows");
   if constexpr (AHEAD) {
     if ((int)blockIdx.x >= ah.first_wg) {
       const int row = 4 * ((int)blockIdx.x - ah.first_wg) + (int)(threadIdx.x >> 6);
@@ -310,8 +424,36 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
     issue_k_tile<HD, PAD>(kb_, row, last_row, my_lds + which * C::TILE_BYTES, lane, hd);
     load_v_tile<HD, PAD>(vb_, row, last_row, col, j, v_next, vhd);
   };
-  if (first_place(t) < seg.tile1 - seg.tile0) fetch(0, seg.kbase, seg.vbase, tile_at(seg, first_place(t)) * 16, seg.L - 1);
-  load_q(seg);
+  // PREP: the last row in memory
+  auto last_row = [&](const Segment &sg) { return PREP ? max(sg.L - 2, 0) : sg.L - 1; };
+  NewRow<HD> fresh;
+  bool holds_new = false;  // this wavefront has the pair's last tile
+  if constexpr (PREP) {
+    // (all of it is requested in front of the first tile, and arrives in front of it)
+    const int n = seg.tile1 - seg.tile0, last = seg.n_s - 1 - seg.tile0 - seg.rot;
+    holds_new = seg.tile1 == seg.n_s && ((last < 0 ? last + n : last) & (NW - 1)) == wave;
+    const float *qrow = raw.q + seg.token * raw.q_stride + (long long)seg.kvh * g * HD;
+    const float *krow = raw.k + seg.token * raw.k_stride + (long long)seg.kvh * HD;
+    const float2 *cs = raw.rope_tab + (long long)(seg.L - 1) * (HD / 2);
+    PreparedQueries<HD> pq;
+    pq.request(qrow + (col < g ? col : 0) * HD, raw.q_norm, cs, j);
+    if (holds_new) fresh.request(krow, raw.v + seg.token * raw.v_stride + (long long)seg.kvh * HD, raw.k_norm, cs, lane);
+    float inv = 1.f;
+    if (raw.q_norm || raw.k_norm) {  // row r: head r of the group; row g: the new key
+      const int r = lane & 31;
+      SquareSum<HD> sum;
+      sum.request(r == g ? krow : qrow + (r < g ? r : 0) * HD, lane);
+      if (first_place(t) < n) fetch(0, seg.kbase, seg.vbase, tile_at(seg, first_place(t)) * 16, last_row(seg));
+      inv = sum.factor(raw.eps, lane);
+    } else if (first_place(t) < n) {
+      fetch(0, seg.kbase, seg.vbase, tile_at(seg, first_place(t)) * 16, last_row(seg));
+    }
+    pq.finish(raw.q_norm != nullptr, __shfl(inv, 32 + (col < g ? col : 0)), qr);
+    if (holds_new) fresh.finish(raw.k_norm != nullptr, __shfl(inv, 32 + g));
+  } else {
+    if (first_place(t) < seg.tile1 - seg.tile0) fetch(0, seg.kbase, seg.vbase, tile_at(seg, first_place(t)) * 16, seg.L - 1);
+    load_q(seg);
+  }
 
   // the pair whose last segment this workgroup holds without holding all of it: merged at the
   // end of the span (only a span's first segment can start inside a pair, so there is one at most)
@@ -372,6 +514,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int u = 0; u < C::NVU; ++u) v_cur[r][u] = v_next[r][u];
+      if (PREP && kb + 16 >= L) {  // the pair's last tile: nobody's key L - 1 and no value from there on is in memory
+        fresh.put_key((char *)buf, L - 1 - kb, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int u = 0; u < C::NVU; ++u) v_cur[r][u] = kb + 4 * j + r >= L - 1 ? fresh.value[u] : v_cur[r][u];
+        asm volatile("" ::: "memory");
+      }
       // a tile that lies `reach` or more behind every column's row has no values by distance
       f32x4 near_bias = {0.f, 0.f, 0.f, 0.f};
       if constexpr (BIAS) {
@@ -379,7 +529,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
         if (L - seg.R - (kb + 15) < db.reach) near_bias = ((const Four *)(bias_row + kb + 4 * j))->v;
       }
       if (place + NW < n_here)
-        fetch(par, kbase, vbase, tile_at(seg, place + NW) * 16, L - 1);
+        fetch(par, kbase, vbase, tile_at(seg, place + NW) * 16, last_row(seg));
       else if (nhave)
         fetch(par, nseg.kbase, nseg.vbase, ntile * 16, nseg.L - 1);
 
@@ -422,7 +572,18 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
         }
     }
     // the next segment's query rows (this one's are not needed any more)
-    if (more) load_q(nseg);
+    if (!PREP && more) load_q(nseg);
+    if constexpr (PREP) {  // (behind the last tile: a wait for loads waits for stores, too)
+      if (holds_new) {
+        const long long at = (long long)(L - 1) * HD;
+        fresh.append(const_cast<float *>(kbase) + at, const_cast<float *>(vbase) + at, lane);
+      }
+      if (seg.tile0 == 0 && wave == 0 && col < g) {
+        float *qp = raw.q_rot + ((long long)seg.token * sh.H + seg.kvh * g + col) * HD + 4 * j;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) *(f32x4 *)(qp + 16 * i) = f32x4{qr[4 * i], qr[4 * i + 1], qr[4 * i + 2], qr[4 * i + 3]};
+      }
+    }
 
     // merge the wavefronts through LDS: the wavefront parks its O rows [g][HD] in the one of
     // its two buffers that does not hold (or receive) its next tile
@@ -801,10 +962,27 @@ hipError_t launch_decode_plan(int *lens, int n_seqs, const Shape &sh, int rope_p
   return hipGetLastError();
 }
 
+bool decode_prepares(const PrepArgs &a, const SeqTable &st, const Shape &sh, const DecodePlan &p, const float *out) {
+  static const bool off = getenv("SHAINET_HIP_NO_FUSED_PREP") != nullptr;
+  if (off || (sh.hd != 64 && sh.hd != 128) || p.align <= 1 || a.b_q || a.b_k || a.b_v || !a.rope_tab || !a.q_rot) return false;
+  for (int s = 0; s < st.n_seqs; ++s)  // (two entries of one sequence: the second one's keys include the first one's row)
+    if (st.n_new[s] != 1 || (s && st.slot[s] == st.slot[s - 1])) return false;
+  if (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.q_norm | (uintptr_t)a.k_norm | (uintptr_t)a.rope_tab |
+       (uintptr_t)a.q_rot | (uintptr_t)a.kc | (uintptr_t)a.vc) & 15 || (a.q_stride | a.k_stride | a.v_stride) & 3)
+    return false;
+  auto apart = [&](const float *x, long long stride, int width) {  // x's rows and out's
+    const float *x_end = x + (st.n_seqs - 1) * stride + width, *out_end = out + (long long)st.n_seqs * sh.H * sh.hd;
+    return (uintptr_t)x_end <= (uintptr_t)out || (uintptr_t)out_end <= (uintptr_t)x;
+  };
+  return apart(a.q, a.q_stride, sh.H * sh.hd) && apart(a.k, a.k_stride, sh.KV * sh.hd) && apart(a.v, a.v_stride, sh.KV * sh.hd);
+}
+
 hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &sh, const DecodePlan &p, float scale,
                          hipStream_t stream, hipEvent_t before, hipEvent_t after, const DecodeDevicePlan *dev,
-                         const DistanceBias *bias) {
+                         const DistanceBias *bias, const PrepArgs *prep) {
   const DistanceBias db = bias ? *bias : DistanceBias{};
+  const PrepArgs raw = prep ? *prep : PrepArgs{};
+  if (prep && (dev || bias || !decode_prepares(*prep, st, sh, p, d.out))) return hipErrorInvalidValue;
   if (st.n_seqs < 1 || st.n_seqs > kMaxSeqs || sh.g < 1 || sh.g > 16 || sh.H != sh.KV * sh.g ||
       !decode_tile_head_dim(sh.hd) || p.n_wgs < 1 || !d.partials || !d.part_flag || !d.error)
     return hipErrorInvalidValue;
@@ -848,7 +1026,7 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
 #define SHAINET_DECODE_LAUNCH(HD_, DEV_, PAD_)                                                                      \
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, DEV_, PAD_>), grid, block, 0, stream, before,      \
                        after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit,       \
-                       d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db)
+                       d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db, raw)
 #define SHAINET_DECODE_LAUNCH_HD(HD_, PAD_) \
   do {                                      \
     if (dev)                                \
@@ -860,8 +1038,21 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, false, true, false, true>), grid, block, 0, stream, \
                        before, after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set,           \
                        spin_limit, d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c,   \
-                       rotate, dev, ah, db)
-  if (bias && tile_hd == 64)
+                       rotate, dev, ah, db, raw)
+#define SHAINET_DECODE_LAUNCH_PREP(HD_, AHEAD_)                                                                      \
+  SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, false, false, AHEAD_, false, true>), grid, block, 0,  \
+                       stream, before, after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set,    \
+                       spin_limit, d.error, st, sh, p.tiles_per_wg, p.spans, p.total_tiles, p.align,                 \
+                       align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db, raw)
+  if (prep && sh.hd == 64 && ah.w)
+    SHAINET_DECODE_LAUNCH_PREP(64, true);
+  else if (prep && sh.hd == 64)
+    SHAINET_DECODE_LAUNCH_PREP(64, false);
+  else if (prep && ah.w)
+    SHAINET_DECODE_LAUNCH_PREP(128, true);
+  else if (prep)
+    SHAINET_DECODE_LAUNCH_PREP(128, false);
+  else if (bias && tile_hd == 64)
     SHAINET_DECODE_LAUNCH_BIAS(64);
   else if (bias && tile_hd == 128)
     SHAINET_DECODE_LAUNCH_BIAS(128);
@@ -870,11 +1061,11 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
   else if (ah.w && sh.hd == 64)
     hipLaunchKernelGGL((decode_splitk_kernel<64, kDecodeWaves, false, false, true>), grid, block, 0, stream, d.q_rot, d.kc,
                        d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit, d.error, st, sh, p.tiles_per_wg,
-                       p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db);
+                       p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db, raw);
   else if (ah.w)
     hipLaunchKernelGGL((decode_splitk_kernel<128, kDecodeWaves, false, false, true>), grid, block, 0, stream, d.q_rot, d.kc,
                        d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit, d.error, st, sh, p.tiles_per_wg,
-                       p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db);
+                       p.spans, p.total_tiles, p.align, align_factor(p.align), p.n_slots, p.cols, c, rotate, dev, ah, db, raw);
   else if (sh.hd == 64)
     SHAINET_DECODE_LAUNCH_HD(64, false);
   else if (sh.hd == 128)
@@ -885,6 +1076,7 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
     SHAINET_DECODE_LAUNCH_HD(128, true);
   else
     SHAINET_DECODE_LAUNCH_HD(256, true);
+#undef SHAINET_DECODE_LAUNCH_PREP
 #undef SHAINET_DECODE_LAUNCH_BIAS
 #undef SHAINET_DECODE_LAUNCH_HD
 #undef SHAINET_DECODE_LAUNCH
