@@ -45,6 +45,7 @@
 
 #include "split_mfma.hpp"
 
+#include <math.h>
 #include <stdint.h>
 #include <stdlib.h>
 
@@ -61,15 +62,6 @@ constexpr int TK = 16, kFewStep = 32;
 // until they have waited for the stores.)
 __device__ __forceinline__ void coherent_store4(float *p, f32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
-}
-
-// *base (the same in all lanes) plus a lane's own offset in bytes: one load with a scalar base.  (Of addresses that differ
-// by scalars only the compiler makes 64-bit sums per thread, two instructions each.)
-template <typename V>
-__device__ __forceinline__ V load_at(const V *base, unsigned offset) {
-  uint64_t at = (uint64_t)base;
-  asm("" : "+s"(at), "+v"(offset));
-  return *(const __attribute__((address_space(1))) V *)(at + offset);
 }
 
 struct GemmArgs {
@@ -109,11 +101,21 @@ __device__ __forceinline__ void store_pair(const GemmArgs &g, int row, int col, 
   *(f32x2 *)(g.y + o) = v;
 }
 
-// Four registers of a lane's sums, number r of its 4 MB NB: with two blocks beside each other its two columns in two
-// rows, with four its four columns in one row.
+// Four registers of a lane's sums, number r of its 4 MB NB: with one block its column in four rows, with two blocks beside
+// each other its two columns in two rows, with four its four columns in one row.
 template <int NB>
 __device__ __forceinline__ void store_four(const GemmArgs &g, int row0, int col, int r, f32x4 v) {
-  if constexpr (NB == 2) {
+  if constexpr (NB == 1) {
+    const int row = row0 + 32 * (r >> 2) + 8 * (r & 3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (row + i >= g.T) return;
+      const long long o = (long long)(row + i) * g.N + col;
+      float y = v[i];
+      if (g.bias) y = activate(g.act, y + g.bias[col]);
+      g.y[o] = g.res ? g.res[o] + y : y;
+    }
+  } else if constexpr (NB == 2) {
     const int row = row0 + 32 * (r >> 3) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
     store_pair(g, row, col, f32x2{v.x, v.y});
     store_pair(g, row + 1, col, f32x2{v.z, v.w});
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
 // 64 rows of 1024 -> 1024 12.1 -> 9.2.  64 rows by 128 columns this way were slower than 32 (45 rows of
 // 8192 -> 2048 34 against 30.5).  Bound by a launch, the first loads and the kernel that adds the pieces where the
 // weights are small, by reading them where they are not.
-template <int PARTS, bool GUARD>
+template <bool GUARD>
 __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
   constexpr int TM = 32, TN = 128, TS = kFewStep;
   constexpr int kOct = TM + 4, kPart = 4 * kOct;  // units of 16 bytes: four octets of k, four units apart from a multiple of 16
@@ -565,29 +567,23 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
   __syncthreads();
   auto step = [&](const int kt, const int set) {  // set: holds step kt, the other one step kt + 1
     const u32x4 *stage = lds + (kt & 1) * kStage + (2 * kg + j) * kOct + ln;
-    u32x4 af[3], bf[PARTS][2];
+    u32x4 af[3], bf[3][2];
 #pragma unroll
     for (int p = 0; p < 3; ++p) af[p] = stage[p * kPart];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        if constexpr (PARTS == 3) {
-          unsigned h, m, l;
-          split_pair(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift, h, m, l);
-          bf[0][b][i] = h, bf[1][b][i] = m, bf[2][b][i] = l;
-        } else {
-          bf[0][b][i] = pack_high(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift);
-        }
+        unsigned h, m, l;
+        split_pair(sw[set][2 * i][b] * kLift, sw[set][2 * i + 1][b] * kLift, h, m, l);
+        bf[0][b][i] = h, bf[1][b][i] = m, bf[2][b][i] = l;
       }
     park_x(set ^ 1, (kt & 1) ^ 1);
     load_tiles(set);
 #pragma unroll
-    for (int p = 0; p < 5; ++p) {
-      if (kPartB[p] >= PARTS) continue;
+    for (int p = 0; p < 5; ++p)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) rest[b] = mfma_bf16(af[kPartA[p]], bf[kPartB[p] < PARTS ? kPartB[p] : 0][b], rest[b]);
-    }
+      for (int b = 0; b < 2; ++b) rest[b] = mfma_bf16(af[kPartA[p]], bf[kPartB[p]][b], rest[b]);
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[b] = mfma_bf16(af[0], bf[0][b], acc[b]);
     __syncthreads();
@@ -656,7 +652,180 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
   }
 }
 
-// y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order.  A piece lies in its
+// The same by weights of one part, which leaves registers for more rows: a workgroup of eight wavefronts owns 32 MB
+// rows and 256 / KG columns, 32 of them a wavefront, and walks K in steps of 16 KG, of which each of KG groups of wavefronts
+// takes its own 16.  W goes from memory to registers four steps ahead (64 KB in flight on a compute unit), x through LDS.
+// Sums as in the kernel above, emptied every eight steps, three products instead of six.
+// Against tiles of 32 x 128 that read W once per 32 rows and add 32-row pieces (us, with the kernel that adds the pieces): 45 rows
+// of 2048 -> 16384 40 -> 35, 2048 -> 2048 15.0 -> 12.7, 8192 -> 2048 31 -> 29, 1024 -> 1024 11.6 -> 9.1; 96 rows 59 -> 44,
+// 15.1 -> 14.9, 34 -> 34, 11.7 -> 9.7; and against 128 x 256 in 8 pieces 512 rows of 1024 -> 1024 21 -> 13.  W of 134 MB
+// comes at 4.5 TB/s, smaller ones wait for a launch or two, the first loads and the steps' barriers.
+template <int MB, int KG, bool GUARD>
+__global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) {
+  constexpr int WN = 8 / KG, TM = 32 * MB, TN = 32 * WN, TS = 16 * KG, kSets = 4;
+  constexpr int kOct = TM + 4, kPart = 2 * KG * kOct, kStage = 3 * kPart;  // units of 16 bytes, as above
+  constexpr int kSums = MB * 16 * 64 / 4;                                  // units that a wavefront's sums take
+  constexpr int kRows = 128 / KG, kRounds = (TM + kRows - 1) / kRows;      // rows that all threads stage at once
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kStage > (8 - WN) * kSums ? 2 * kStage : (8 - WN) * kSums];
+
+  const int group = blockIdx.x & ((1 << g.group_bits) - 1), place = blockIdx.x >> g.group_bits;
+  const int steps = g.steps, pieces = g.pieces ? g.pieces : 1;
+  const int t = place / pieces, s_begin = (place - t * pieces) * g.quota, s_end = min(s_begin + g.quota, steps);
+  if (t >= g.tiles_per_group || s_begin >= s_end) return;
+  const int tile = group * g.tiles_per_group + t;
+  const int m0 = tile % g.tiles_m * TM, n0 = tile / g.tiles_m * TN;
+  const int T = g.T, K = g.K, N = g.N;
+  const int k_begin = s_begin * TS, k_end = min(K, s_end * TS), nk = s_end - s_begin;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 31, j = lane >> 5, wn = wave % WN, kg = wave / WN;
+  const int col = n0 + 32 * wn + ln;
+
+  // x: a thread takes four k, piece tid % (4 KG), of row tid / (4 KG) (and kRows on; rows past the last one repeat it)
+  const int xrow = threadIdx.x / (4 * KG), xk = 4 * (threadIdx.x % (4 * KG));
+  unsigned x_off[kRounds];
+#pragma unroll
+  for (int u = 0; u < kRounds; ++u) x_off[u] = (unsigned)(((long long)min(m0 + xrow + kRows * u, T - 1) * g.xs + xk) * 4);
+  u32x2 *const x_lds = (u32x2 *)(lds + (xk >> 3) * kOct + xrow) + (xk >> 2 & 1);
+  // W: rows 16 kg + 8 j .. + 7 of a step (columns past the last one repeat it)
+  const int wk = 16 * kg + 8 * j;
+  const unsigned w_off = (unsigned)(((long long)8 * j * N + min(col, N - 1)) * 4);
+  const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)(k_begin + 16 * kg) * N);
+  const long long row_bytes = 4LL * N;
+
+  // register sets: the tiles of step t travel in set t % 4 and are requested four steps ahead.  Behind the last step its
+  // W is requested again, and its x counts as zeros: the loop has no conditions.
+  f32x4 sx[kSets][kRounds];
+  float sw[kSets][8];
+  int k_next = k_begin, to_load = nk;
+  auto load_tiles = [&](const int set) {
+#pragma unroll
+    for (int u = 0; u < kRounds; ++u) {
+      sx[set][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (to_load > 0 && (!GUARD || k_next + xk < k_end) && (TM % kRows == 0 || xrow + kRows * u < TM)) sx[set][u] = load_at((const f32x4 *)x_base, x_off[u]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      sw[set][i] = GUARD && k_next + wk + i >= k_end ? 0.f : load_at((const float *)(w_base + i * row_bytes), w_off);
+    if (--to_load > 0) {
+      x_base += TS * 4;
+      w_base += TS * row_bytes;
+      k_next += TS;
+    }
+  };
+  auto park_x = [&](const int set, const int stage) {
+#pragma unroll
+    for (int u = 0; u < kRounds; ++u) {
+      if (TM % kRows != 0 && xrow + kRows * u >= TM) continue;
+      u32x2 *at = x_lds + 2 * (stage * kStage + kRows * u);
+      split_quad(sx[set][u] * kLift, at[0], at[2 * kPart], at[4 * kPart]);
+    }
+  };
+
+  f32x16 acc[MB], rest[MB], sum[MB];
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[a][r] = rest[a][r] = sum[a][r] = 0.f;
+
+#pragma unroll
+  for (int set = 0; set < kSets; ++set) load_tiles(set);
+  park_x(0, 0);
+  __syncthreads();
+  auto step = [&](const int set) {  // set: holds this step; its x is in stage set % 2
+    const u32x4 *stage = lds + (set & 1) * kStage + (2 * kg + j) * kOct + ln;
+    u32x4 bf;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bf[i] = pack_high(sw[set][2 * i] * kLift, sw[set][2 * i + 1] * kLift);
+    u32x4 af[3][MB];
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int a = 0; a < MB; ++a) af[p][a] = stage[p * kPart + 32 * a];
+    park_x((set + 1) % kSets, (set & 1) ^ 1);
+    load_tiles(set);
+#pragma unroll
+    for (int p = 2; p > 0; --p)
+#pragma unroll
+      for (int a = 0; a < MB; ++a) rest[a] = mfma_bf16(af[p][a], bf, rest[a]);
+#pragma unroll
+    for (int a = 0; a < MB; ++a) acc[a] = mfma_bf16(af[0][a], bf, acc[a]);
+    __syncthreads();
+  };
+  for (int k0 = 0; k0 < nk; k0 += 8) {
+    for (int kt = k0; kt < min(k0 + 8, nk); kt += 4) {
+      step(0);
+      step(1);
+      step(2);
+      step(3);
+    }
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sum[a][r] += acc[a][r], acc[a][r] = 0.f;
+  }
+
+#pragma unroll
+  for (int a = 0; a < MB; ++a) acc[a] = sum[a] + rest[a];
+  // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which
+  float probe = 0.f;
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) probe = fmaf(acc[a][r], 0.f, probe);
+  if (__any(probe != 0.f)) {
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
+#pragma clang loop unroll(disable)
+    for (int k0 = k_begin + 16 * kg; k0 < k_end; k0 += (k0 & 15) ? TS - 8 : 8) {  // (this wavefront's part of the steps)
+      const int k = k0 + 4 * j;
+      const bool in = k < k_end;
+      f32x4 xv[MB];
+      float wv[4];
+#pragma unroll
+      for (int a = 0; a < MB; ++a)
+        xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + 32 * a + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wv[i] = in ? g.w[(long long)(k + i) * N + min(col, N - 1)] : 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int a = 0; a < MB; ++a) acc[a] = mfma_f32(xv[a][i], wv[i], acc[a]);
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < MB; ++a) acc[a] *= kDrop;
+  }
+  // (every wavefront is past the last step's barrier: nobody reads tiles any more)
+  f32x4 *const merge = (f32x4 *)lds + wn * kSums + lane;
+  if (kg > 0) {
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        merge[(kg - 1) * WN * kSums + 64 * (4 * a + r)] = f32x4{acc[a][4 * r], acc[a][4 * r + 1], acc[a][4 * r + 2], acc[a][4 * r + 3]};
+  }
+  __syncthreads();
+  if (kg > 0) return;
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      f32x4 v = f32x4{acc[a][4 * r], acc[a][4 * r + 1], acc[a][4 * r + 2], acc[a][4 * r + 3]};
+#pragma unroll
+      for (int i = 0; i < KG - 1; ++i) v += merge[i * WN * kSums + 64 * (4 * a + r)];
+      if (g.pieces)  // [four rows][thread], as the kernel that adds the pieces takes them
+        *(f32x4 *)(g.partials + (long long)blockIdx.x * (TM * TN) + (4 * a + r) * (256 * WN) + 4 * threadIdx.x) = v;
+      else if (col < N)
+        store_four<1>(g, m0 + 4 * j, col, 4 * a + r, v);
+    }
+}
+
+// y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order, eight of them in flight (one after the other 16
+// pieces of 45 rows took 3 us more).  A piece lies in its
 // workgroup's slot as [pair of rows, or row][thread] float4, the layout of the product kernel's accumulators.
 // A tile's threads are WM x WN wavefronts of MB x NB blocks.
 template <int WM, int WN, int MB, int NB>
@@ -674,7 +843,14 @@ __global__ __launch_bounds__(64 * WM * WN) void sgemm_reduce_kernel(const GemmAr
   const int col = (tile / g.tiles_m) * TN + (wave % WN) * 32 * NB + NB * (lane & 31);
   if (col >= g.N) return;
   f32x4 acc = *(const f32x4 *)piece;
-  for (int c = 1; c < n; ++c) acc += *(const f32x4 *)(piece + c * piece_step);
+  for (int c0 = 1; c0 < n; c0 += 8) {  // eight loads in flight
+    f32x4 v[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = *(const f32x4 *)(piece + min(c0 + c, n - 1) * piece_step);
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (c0 + c < n) acc += v[c];
+  }
   store_four<NB>(g, row0, col, r, acc);
 }
 
@@ -703,6 +879,41 @@ namespace {
 // workgroups the chip runs at once: two of four wavefronts per compute unit, or one of eight
 int slots_of(int wn) { return wn == 4 ? 256 : 512; }
 
+// Steps per workgroup of sgemm_stream_kernel: as many pieces as leave no compute unit without one, in whole rounds of its
+// four register sets.
+int stream_quota(int tiles, int steps) {
+  int pieces = 256 / tiles;
+  if (pieces > 16) pieces = 16;
+  if (pieces < 1) pieces = 1;
+  return ((steps + pieces - 1) / pieces + 3) / 4 * 4;
+}
+
+// W of one part: the tile of sgemm_stream_kernel by an estimate of its time, and whether that kernel is the one to take.
+// Rounds of workgroups times steps times what a step takes, and for pieces 1.4 us and 0.27 us per MB of them written and
+// read: fitted to 60 products of 5 to 777 rows, 5 % off on average.  It is left from 97 rows on where its loop alone takes
+// 20 us: there the larger tiles, which read W less often, are level or ahead (us, this | 128 x 256): 256 rows of
+// 2048 -> 2048 19.2 | 23.3, 2048 -> 3072 26.9 | 25.5, 8192 -> 2048 52 | 43, 2048 -> 16384 96 | 64; 512 rows of 1024 -> 1024
+// 13.0 | 20.8, 1024 -> 3072 24.3 | 25.0, 2048 -> 2048 28.1 | 28.3, 2048 -> 3072 42 | 33; 777 rows of 1024 -> 1024 19.0 | 24.2,
+// 1024 -> 3072 34 | 32; 96 rows of 2048 -> 16384 43 | 52.
+bool choose_stream(GemmPlan &p, int T, int K, int N) {
+  const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.453f}, {1, 4, 0.534f}, {2, 2, 0.587f}, {3, 2, 0.801f}};
+  float least = INFINITY, loop = 0.f;
+  for (const auto &s : shapes) {
+    const long long tiles = (T + 32 * s.mb - 1) / (32 * s.mb) * (((long long)N * s.kg + 255) / 256);
+    if (tiles > 1 << 20) continue;  // (many rounds: not this kernel's anyway)
+    const int steps = (K + 16 * s.kg - 1) / (16 * s.kg), quota = stream_quota((int)tiles, steps), pieces = (steps + quota - 1) / quota;
+    const long long wgs = tiles * pieces;
+    const float turns = (float)((wgs + 255) / 256) * quota * s.step;
+    const float us = turns + (pieces > 1 ? 1.4f + 0.27e-6f * 8 * 32 * s.mb * (256 / s.kg) * wgs : 0.f);
+    if (us >= least) continue;
+    least = us;
+    loop = turns;
+    p.mb = s.mb;
+    p.kg = s.kg;
+  }
+  return least < INFINITY && (T <= 96 || loop <= 20.f);
+}
+
 // The tile, by what was measured (us, 2048 -> 3072 | 2048 -> 2048 | 2048 -> 16384 | 8192 -> 2048 | 1024 -> 8192):
 //   rows   32 x 128 (few)              128 x 128                  128 x 256                  256 x 256
 //     45   16 | 15 | 41 | 31 | 16      23 | 19 | 59 | 37 | 24
@@ -713,14 +924,11 @@ int slots_of(int wn) { return wn == 4 ? 256 : 512; }
 //    512                               47 | 37 | 185 | 106 | 57   45 | 36 | 177 | 102 | 58   52 | 44 | 192 | 100 | 64
 //   1024                               87 | 58 | 360 | 197 | 96   82 | 57 | 342 | 186 | 88   80 | 63 | 315 | 173 | 116
 //   2048                               148 | 100 | 717 | 372 | 187  143 | 99 | 674 | 346 | 181  144 | 100 | 619 | 323 | 164
-// W of one part (us; few | 128 x 128 | 128 x 256 | 256 x 256), the same products:
-//     96   18 22 20 29 | 15 20 20 26 | 59 49 46 65 | 34 33 35 48 | 20 26 24 38
-//    128   18 22 20 29 | 18 19 19 26 | 59 52 48 65 | 40 35 36 48 | 21 28 28 38
-//    200   23 25 24 30 | 20 24 24 26 | 108 71 65 68 | 59 48 42 50 | 28 31 29 39
-//    256   28 26 25 30 | 20 24 24 26 | 112 75 65 70 | 62 50 43 53 | 28 32 35 40
-//    512    - 35 32 41 | - 30 28 38 | - 120 99 112 | - 77 60 69 | - 43 41 49
-//    777    - 49 45 53 | - 40 35 45 | - 219 184 172 | - 115 95 103 | - 67 61 71
-//   2048    - 97 85 90 | - 69 61 68 | - 471 391 349 | - 240 197 193 | - 123 106 96
+// W of one part (us; 128 x 128 | 128 x 256 | 256 x 256), the same products:
+//    256   26 25 30 | 24 24 26 | 75 65 70 | 50 43 53 | 32 35 40
+//    512   35 32 41 | 30 28 38 | 120 99 112 | 77 60 69 | 43 41 49
+//    777   49 45 53 | 40 35 45 | 219 184 172 | 115 95 103 | 67 61 71
+//   2048   97 85 90 | 69 61 68 | 471 391 349 | 240 197 193 | 123 106 96
 // so 128 x 128 is not among its tiles, and 256 x 256 cut into pieces pads less than 8 %.
 // A low tile wastes least on few rows, and reads small weights again from the L2 for little: up to 96 rows always, up to
 // 256 where the higher tile would be a fifth padding or the weights are small.
@@ -731,10 +939,12 @@ int slots_of(int wn) { return wn == 4 ? 256 : 512; }
 // 640 824 | 759, 704 909 | 846; 4096 -> 8192: 320 802 | 896, 384 973 | 887; 8192 -> 8192: 288 1671 | 1873).
 void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 2;
+  p.kg = 2;
   const long long weights = (long long)K * N, rows1 = (T + 31) / 32 * 32LL, rows2 = (T + 127) / 128 * 128LL;
   p.few = T <= 96 || (T <= 256 && (weights <= (T <= 128 ? 12 : 5) << 20 || rows2 * 100 >= rows1 * 125));
-  if (p.parts == 1) p.few = T <= 96 || (T <= 256 && weights <= (T <= 128 ? 12 : 9) << 20);
+  if (p.parts == 1) p.few = choose_stream(p, T, K, N);
   p.few = p.few && (long long)kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows)
+  if (p.few && p.parts == 1) return;
   p.mb = 1;
   if (p.few) return;
   p.mb = 2;
@@ -752,7 +962,8 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
 }  // namespace
 
 static int tile_rows(const GemmPlan &p) { return (p.few ? 32 : 64) * p.mb; }
-static int tile_columns(const GemmPlan &p) { return 64 * p.wn; }
+static int tile_columns(const GemmPlan &p) { return p.few && p.parts == 1 ? 256 / p.kg : 64 * p.wn; }
+static int step_k(const GemmPlan &p) { return !p.few ? TK : p.parts == 1 ? 16 * p.kg : kFewStep; }
 
 void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[0] = !p.mfma ? 0 : p.few ? 1 : 2;
@@ -761,7 +972,7 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[3] = p.workgroups;
   plan[4] = p.pieces > 1 ? p.pieces : 1;
   plan[5] = p.flag_words && p.quota % p.steps != 0;
-  plan[6] = p.mfma && K % (p.few ? kFewStep : TK) != 0;
+  plan[6] = p.mfma && K % step_k(p) != 0;
 }
 
 GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
@@ -773,7 +984,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
   p.steps = (K + TK - 1) / TK;
   choose_tile(p, T, K, N);
   const int TN = tile_columns(p), TM = tile_rows(p);
-  if (p.few) p.steps = (K + kFewStep - 1) / kFewStep;
+  if (p.few) p.steps = (K + step_k(p) - 1) / step_k(p);
   p.tiles_m = (T + TM - 1) / TM;
   p.tiles_n = (N + TN - 1) / TN;
   if (!p.mfma) return p;
@@ -784,6 +995,13 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
   while (tiles & ((1 << p.group_bits) - 1)) --p.group_bits;
   const int groups = 1 << p.group_bits;
   p.tiles_per_group = tiles / groups;
+  if (p.few && p.parts == 1) {
+    p.quota = stream_quota(tiles, p.steps);
+    p.pieces = (p.steps + p.quota - 1) / p.quota;
+    p.workgroups = tiles * p.pieces;
+    if (p.pieces > 1) p.partial_floats = (size_t)p.workgroups * TM * TN;
+    return p;
+  }
   if (p.few) {  // pieces of about twelve steps, more where that leaves compute units without one, of at least four steps each
     int pieces = p.steps / 12 > 256 / tiles ? p.steps / 12 : 256 / tiles;
     if (pieces > slots / tiles) pieces = slots / tiles;
@@ -845,18 +1063,36 @@ hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, hipStream_t stream
   return hipGetLastError();
 }
 
-template <int PARTS>
 hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
   if (g.K % kFewStep != 0)
-    hipLaunchKernelGGL((sgemm_few_kernel<PARTS, true>), grid, dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_few_kernel<true>), grid, dim3(256), 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_few_kernel<PARTS, false>), grid, dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_few_kernel<false>), grid, dim3(256), 0, stream, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || !g.pieces) return e;
   const int tiles = p.tiles_m * p.tiles_n;
   hipLaunchKernelGGL((sgemm_reduce_kernel<1, 2, 1, 2>), dim3((unsigned)tiles * 8), dim3(128), 0, stream, g, tiles);
   return hipGetLastError();
+}
+
+template <int MB, int KG>
+hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+  const dim3 grid((unsigned)p.workgroups);
+  if (g.K % (16 * KG) != 0)
+    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, true>), grid, dim3(512), 0, stream, g);
+  else
+    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, false>), grid, dim3(512), 0, stream, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !g.pieces) return e;
+  const int tiles = p.tiles_m * p.tiles_n;
+  hipLaunchKernelGGL((sgemm_reduce_kernel<1, 8 / KG, MB, 1>), dim3((unsigned)tiles * 4 * MB), dim3(512 / KG), 0, stream, g, tiles);
+  return hipGetLastError();
+}
+
+template <int MB>
+hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+  return p.kg == 4 ? launch_stream<MB, 4>(g, p, stream) : launch_stream<MB, 2>(g, p, stream);
 }
 
 }  // namespace
@@ -896,10 +1132,10 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   g.quota = p.quota;
   g.pieces = p.pieces > 1 ? p.pieces : 0;
   if (p.parts == 1) {
-    if (p.few) return launch_few<1>(g, p, stream);
+    if (p.few) return p.mb == 1 ? launch_stream<1>(g, p, stream) : p.mb == 2 ? launch_stream<2>(g, p, stream) : launch_stream<3>(g, p, stream);
     return p.mb == 4 ? launch_tiles<4, 2, 2, 4, 1>(g, p, stream) : launch_tiles<2, 4, 2, 2, 1>(g, p, stream);
   }
-  if (p.few) return launch_few<3>(g, p, stream);
+  if (p.few) return launch_few(g, p, stream);
   if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4, 2, 3>(g, p, stream) : launch_tiles<2, 4, 2, 2, 3>(g, p, stream);
   return launch_tiles<2, 2, 2, 2, 3>(g, p, stream);
 }

@@ -8,8 +8,9 @@ namespace shainet {
 
 struct GemmPlan {
   bool mfma;              // false: K, N or the row stride of x is not a multiple of 4 -> the plain kernel
-  bool few;               // tiles of 32 rows and 128 columns, K steps of 32
+  bool few;               // tiles of 32 rows and 128 columns, K steps of 32 (parts 1: see kg)
   int mb, wn;             // otherwise tiles of 64 mb rows and 64 wn columns, K steps of 16
+  int kg;                 // few, parts 1: tiles of 32 mb rows and 256 / kg columns, K steps of 16 kg
   int tiles_m, tiles_n;
   int parts;              // bf16 numbers that a weight is the sum of: 3, or 1 where the weights are bf16 numbers
   int steps;              // K steps per tile; a unit of work is one step of one tile

@@ -48,6 +48,14 @@ __global__ __launch_bounds__(256) void convert_kernel(const void *__restrict__ s
   if (i < n) dst[i] = load_as_f32(src, i, dtype);
 }
 
+// *word = 1 where some element is no bf16 number
+__global__ __launch_bounds__(256) void low_bits_kernel(const void *__restrict__ src, long long n, int dtype, unsigned *word) {
+  unsigned found = 0;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
+    found |= __float_as_uint(load_as_f32(src, i, dtype)) & 0xffffu;
+  if (__any(found != 0) && (threadIdx.x & 63) == 0) atomicOr(word, 1u);
+}
+
 // src [rows, cols] row-major -> dst[c * ld + r] for every (r, c): the transpose, written into a
 // matrix whose rows are ld floats long (dst already points at the first column to fill).
 // 32 x 32 tiles through LDS so that both the reads and the writes are coalesced.
@@ -80,9 +88,11 @@ int dtype_code(const std::string &d) {
 
 struct Stager {
   void *dev = nullptr;
+  unsigned *word = nullptr;
   size_t cap = 0;
   ~Stager() {
     if (dev) (void)hipFree(dev);
+    if (word) (void)hipFree(word);
   }
   int put(const StTensor &t) {
     if ((size_t)t.nbytes > cap) {
@@ -120,15 +130,41 @@ int check_matrix(const StTensor &t, long long rows, long long cols, int &dtype) 
   return SHAINET_HIP_OK;
 }
 
-// HF [out, in] tensor -> columns [col0, col0 + out) of the device matrix dst [in, ld].  bf16 (nullable): set by the
-// matrix's first tensor, the one at column 0, and kept up by the others: whether all of them are stored as bf16.
+// Whether every value of a staged tensor is a bf16 number, whatever type it is stored in.
+int stored_bf16(Stager &stage, const StTensor &t, int dtype, bool *out) {
+  *out = dtype == kBF16;
+  if (*out) return SHAINET_HIP_OK;
+  const long long n = t.nbytes / dtype_size(t.dtype);
+  unsigned found = 0;
+  if (!stage.word && hipMalloc((void **)&stage.word, sizeof found) != hipSuccess) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
+  if (hipMemset(stage.word, 0, sizeof found) != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, "hipMemset failed");
+  const long long blocks = (n + 1023) / 1024;
+  hipLaunchKernelGGL(low_bits_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, nullptr, stage.dev, n, dtype, stage.word);
+  if (hipGetLastError() != hipSuccess || hipMemcpy(&found, stage.word, sizeof found, hipMemcpyDeviceToHost) != hipSuccess)
+    return fail(SHAINET_HIP_ERR_RUNTIME, "looking at tensor '" + t.name + "' failed");
+  *out = !found;
+  return SHAINET_HIP_OK;
+}
+
+// *bf16 (nullable): taken up by a matrix's first tensor, kept up by the others: whether all their values are bf16 numbers
+int note_bf16(Stager &stage, const StTensor &t, int dtype, bool first, bool *bf16) {
+  if (!bf16) return SHAINET_HIP_OK;
+  bool here = false;
+  if (first || *bf16)
+    if (int rc = stored_bf16(stage, t, dtype, &here)) return rc;
+  *bf16 = here;
+  return SHAINET_HIP_OK;
+}
+
+// HF [out, in] tensor -> columns [col0, col0 + out) of the device matrix dst [in, ld].  bf16: note_bf16; the tensor at
+// column 0 comes first
 int load_transposed(const shainet_safetensors *st, Stager &stage, const std::string &name, int out_dim, int in_dim,
                     float *dst, long long ld, long long col0, bool *bf16 = nullptr) {
   int rc = SHAINET_HIP_OK, dtype;
   const StTensor *t = need(st, name, rc);
   if (!t) return rc;
   if ((rc = check_matrix(*t, out_dim, in_dim, dtype)) || (rc = stage.put(*t))) return rc;
-  if (bf16) *bf16 = (col0 == 0 || *bf16) && dtype == kBF16;
+  if ((rc = note_bf16(stage, *t, dtype, col0 == 0, bf16))) return rc;
   dim3 grid((unsigned)((in_dim + 31) / 32), (unsigned)((out_dim + 31) / 32));
   hipLaunchKernelGGL(convert_transpose_kernel, grid, dim3(256), 0, nullptr, stage.dev, dst + col0, out_dim, in_dim, ld,
                      dtype);
@@ -138,11 +174,12 @@ int load_transposed(const shainet_safetensors *st, Stager &stage, const std::str
 }
 
 int load_plain(const shainet_safetensors *st, Stager &stage, const std::string &name, long long rows, long long cols,
-               float *dst) {
+               float *dst, bool *bf16 = nullptr, bool first = true) {
   int rc = SHAINET_HIP_OK, dtype;
   const StTensor *t = need(st, name, rc);
   if (!t) return rc;
   if ((rc = check_matrix(*t, rows, cols, dtype)) || (rc = stage.put(*t))) return rc;
+  if ((rc = note_bf16(stage, *t, dtype, first, bf16))) return rc;
   const long long n = rows * cols;
   hipLaunchKernelGGL(convert_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, stage.dev, dst, n, dtype);
   if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
@@ -294,8 +331,9 @@ int shainet_hf_load_llama(const char *model_dir, shainet_llama_model **out) {
   }
   Stager stage;
   LlamaModelBuffers mb;
+  bool embedding_bf16 = false;
   if (!rc) rc = shainet_llama_model_buffers(m, &mb);
-  if (!rc) rc = load_plain(st, stage, "model.embed_tokens.weight", V, d, mb.embedding);  // [vocab, d]
+  if (!rc) rc = load_plain(st, stage, "model.embed_tokens.weight", V, d, mb.embedding, &embedding_bf16);  // [vocab, d]
   for (int li = 0; li < cfg.num_hidden_layers && !rc; ++li) {
     shainet_llama_block *b = shainet_llama_model_block(m, li);
     shainet_llama_attn *a = shainet_llama_block_attn(b);
@@ -360,7 +398,7 @@ int shainet_hf_load_llama(const char *model_dir, shainet_llama_model **out) {
       if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
         rc = fail(SHAINET_HIP_ERR_RUNTIME, "transposing the tied embedding failed");
       else
-        *mb.lm_head_bf16 = st->find("model.embed_tokens.weight")->dtype == "BF16";
+        *mb.lm_head_bf16 = embedding_bf16;
     } else {
       rc = load_transposed(st, stage, "lm_head.weight", V, d, mb.lm_head, V, 0, mb.lm_head_bf16);
     }
@@ -779,14 +817,11 @@ int load_experts(const shainet_safetensors *st, Stager &stage, const std::string
   if ((rc = load_plain(st, stage, p + "router", n, m.d, w.router))) return rc;
   if ((rc = load_transposed(st, stage, p + "router", n, m.d, w.router_in, w.n_router, 0, &w.router_bf16))) return rc;
   if ((rc = load_plain(st, stage, p + "correction", 1, n, w.correction))) return rc;
-  w.gate_up_bf16 = w.down_bf16 = true;
   for (int e = 0; e < m.experts; ++e) {
     const std::string pe = p + "e" + std::to_string(e) + ".";
-    if ((rc = load_plain(st, stage, pe + "gate", m.ff, m.d, w.gate_up + 2 * e * mat))) return rc;
-    if ((rc = load_plain(st, stage, pe + "up", m.ff, m.d, w.gate_up + (2 * e + 1) * mat))) return rc;
-    if ((rc = load_plain(st, stage, pe + "down", m.d, m.ff, w.down + e * mat))) return rc;
-    w.gate_up_bf16 = w.gate_up_bf16 && st->find(pe + "gate")->dtype == "BF16" && st->find(pe + "up")->dtype == "BF16";
-    w.down_bf16 = w.down_bf16 && st->find(pe + "down")->dtype == "BF16";
+    if ((rc = load_plain(st, stage, pe + "gate", m.ff, m.d, w.gate_up + 2 * e * mat, &w.gate_up_bf16, e == 0))) return rc;
+    if ((rc = load_plain(st, stage, pe + "up", m.ff, m.d, w.gate_up + (2 * e + 1) * mat, &w.gate_up_bf16, false))) return rc;
+    if ((rc = load_plain(st, stage, pe + "down", m.d, m.ff, w.down + e * mat, &w.down_bf16, e == 0))) return rc;
   }
   if (!m.shared_ff) return SHAINET_HIP_OK;
   const std::string ps = p + "shared.";

@@ -282,6 +282,8 @@ int shainet_llama_attn_set_weights(shainet_llama_attn *l, const float *w_q, cons
   if (!rc) rc = upload_floats(&l->w_o, w_o, (size_t)l->q_dim * l->d_model);
   l->w_o_t_stale = l->w_qkv_t_stale = true;
   l->w_qkv_bf16 = l->w_o_bf16 = false;
+  if (!rc) rc = values_are_bf16(l->w_qkv, (size_t)l->d_model * (l->q_dim + 2 * l->kv_dim), &l->w_qkv_bf16);
+  if (!rc) rc = values_are_bf16(l->w_o, (size_t)l->q_dim * l->d_model, &l->w_o_bf16);
   return rc;
 }
 
@@ -808,6 +810,9 @@ int shainet_llama_block_set_ffn(shainet_llama_block *b, const float *gate, const
   if (!rc) rc = upload_floats(&b->w->down, down, (size_t)b->ff_hidden * b->d_model);
   b->w->gate_up_t_stale = b->w->down_t_stale = true;
   b->w->gate_up_bf16 = b->w->down_bf16 = false;
+  const size_t n = (size_t)b->d_model * b->ff_hidden;
+  if (!rc) rc = values_are_bf16(b->w->gate_up, 2 * n, &b->w->gate_up_bf16);
+  if (!rc) rc = values_are_bf16(b->w->down, n, &b->w->down_bf16);
   return rc;
 }
 

@@ -183,6 +183,10 @@ int upload_side_by_side(float **dst, const float *const *mats, const int *widths
 
 int llama_fail(int code, const std::string &msg);
 
+// Whether all n device floats are bf16 numbers (the lower half of their bits is zero), waited for: asked once per set of
+// weights, whatever they came from, so that equal weights take equal products.
+int values_are_bf16(const float *w, size_t n, bool *out);
+
 // Second copies of weight matrices, transposed, for the product of a single row (launch_gemvt).
 // SHAINET_HIP_NO_TRANSPOSED_WEIGHTS turns them off.  transposed_twin: *twin = src ([rows, cols] on
 // the device) transposed, allocated on first use and made again when *stale; returns the twin, or

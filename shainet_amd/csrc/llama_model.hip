@@ -499,6 +499,7 @@ int shainet_llama_model_set_lm_head(shainet_llama_model *m, const float *w, cons
   m->lm_head_t_stale = true;
   m->lm_head_bf16 = false;
   int rc = upload_floats(&m->lm_head, w, (size_t)m->d_model * m->vocab);
+  if (!rc) rc = values_are_bf16(m->lm_head, (size_t)m->d_model * m->vocab, &m->lm_head_bf16);
   if (rc) return rc;
   if (bias) return upload_floats(&m->lm_bias, bias, (size_t)m->vocab);
   if (m->lm_bias) (void)hipFree(m->lm_bias);

@@ -19,6 +19,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <stdint.h>
+
 namespace shainet {
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -107,6 +109,15 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {
 // The same in fp32 over two k: lane l holds k = l / 32 of row (column) l % 32; the same D.
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+}
+
+// *base (the same in all lanes) plus a lane's own offset in bytes: one load with a scalar base.  (Of addresses that differ
+// by scalars only the compiler makes 64-bit sums per thread, two instructions each.)
+template <typename V>
+__device__ __forceinline__ V load_at(const V *base, unsigned offset) {
+  uint64_t at = (uint64_t)base;
+  asm("" : "+s"(at), "+v"(offset));
+  return *(const __attribute__((address_space(1))) V *)(at + offset);
 }
 
 }  // namespace shainet

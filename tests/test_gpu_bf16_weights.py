@@ -1,5 +1,6 @@
-"""Weights a checkpoint stores as bf16 against the same values stored as fp32: the products of the former leave out the
-partial products whose factor is zero, the others take all of them."""
+"""Weights that are all bf16 numbers against the same with one in each matrix that is none, by its last bit: the products of
+the former leave out the partial products whose factor is zero, the others take all of them.  What a checkpoint stores
+them in makes no difference."""
 import json
 
 import numpy as np
@@ -25,13 +26,15 @@ def bf16(a):
     return (np.ascontiguousarray(a, np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
 
 
-def write(folder, cfg, weights, stored_bf16):
+def write(folder, cfg, weights, stored_bf16, nudge=True):
     folder.mkdir()
     (folder / "config.json").write_text(json.dumps(cfg))
     out = {}
     for name, a in weights.items():
-        a = np.ascontiguousarray(a, np.float32)
+        a = np.array(a, np.float32)
         short = stored_bf16(name)
+        if not short and a.ndim == 2 and nudge:
+            a.reshape(-1).view(np.uint32)[a.size // 2] ^= 1
         raw = (a.view(np.uint32) >> 16).astype("<u2") if short else a
         out[name] = ("BF16" if short else "F32", np.shape(weights[name]), raw.tobytes())
     write_safetensors(folder / "model.safetensors", out)
@@ -73,15 +76,18 @@ def assert_alike(got, want):
 # tiles of 32 rows (whole and ragged steps along K), 128 x 256 cut into pieces, shared by waiting and whole, 256 x 256 likewise
 @pytest.mark.parametrize("d,ff,T", [(128, 260, 40), (132, 260, 19), (640, 2052, 100), (1024, 4096, 300), (1028, 2052, 290),
                                     (640, 4100, 1100), (1040, 8192, 2000), (1044, 8196, 2000), (1040, 4100, 3000)])
-def test_bf16_checkpoint_runs_like_its_fp32_copy(hip, tmp_path, d, ff, T):
+def test_bf16_weights_run_like_fp32_ones(hip, tmp_path, d, ff, T):
     cfg, w = llama(d, ff, d + T)
     w["model.norm.weight"] *= np.float32(2.0 ** 20)
     head = w["lm_head.weight"]
     head[5, 3], head[6, d - 1], head[8, 7] = np.nan, np.inf, -np.inf
     head[7] = bf16(head[7] * np.float32(2.0 ** -129))  # bf16 numbers below the normal ones among them
     tokens = np.random.default_rng(1).integers(0, cfg["vocab_size"], T)
-    assert_alike(all_logits(hip, write(tmp_path / "short", cfg, w, lambda n: True), tokens),
-                 all_logits(hip, write(tmp_path / "long", cfg, w, lambda n: False), tokens))
+    got = all_logits(hip, write(tmp_path / "short", cfg, w, lambda n: True), tokens)
+    assert_alike(got, all_logits(hip, write(tmp_path / "long", cfg, w, lambda n: False), tokens))
+    if T < 50:
+        same = all_logits(hip, write(tmp_path / "same", cfg, w, lambda n: "mlp" in n, nudge=False), tokens)
+        assert np.array_equal(got, same, equal_nan=True)
 
 
 @pytest.mark.parametrize("long", ["k_proj", "up_proj", "down_proj", "lm_head"])
