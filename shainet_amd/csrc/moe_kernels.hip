@@ -425,7 +425,8 @@ __global__ __launch_bounds__(256) void moe_scatter_kernel(int n, int top, int ex
 // their partners, so that a lane holds both halves of its outputs.
 // 777 tokens, 145 rows an expert, 1024 -> 512 gate | up with SwiGLU 157 -> 86 us, 512 -> 1024 84 -> 48 us against the
 // fp32 instruction in tiles of 64 rows.  PARTS 1: the matrices' values are bf16 numbers, the products with their other two
-// parts, zeros, are left out: 85 -> 65 and 49 -> 39 us.
+// parts, zeros, are left out, and a step is 32 along K, whole 128-byte lines of a row: 85 -> 51 and 49 -> 34 us (150
+// tokens 61 -> 31 and 34 -> 17), of which loads that hang on no condition are 14 and 5.
 struct GroupedArgs {
   const float *x;
   const int *gather;       // row r of the product is row gather[r] of x; null: row r
@@ -435,14 +436,19 @@ struct GroupedArgs {
   int rows, groups, K, N;
   bool w_bf16;             // every value of w is a bf16 number (PARTS = 1: the other two parts, zeros, are left out)
 };
-template <int MB, bool SWIGLU, bool VEC, int PARTS>
+// LOADS: how pieces of four k are read.  kScalar: any K; kPieces: K a multiple of 4; kSteps: of a step, and no more to it.
+enum { kScalar, kPieces, kSteps };
+template <int MB, bool SWIGLU, int LOADS, int PARTS>
 __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g) {
-  constexpr int TK = 16, TM = 64 * MB, TN = 128;
-  constexpr int NA = TM / 64, NW = TN / 64;  // 16-byte pieces per thread and step
-  constexpr int kOctX = TM + 4, kOctW = TN + 4, kPartX = 2 * kOctX, kPartW = 2 * kOctW;  // units of 16 bytes
+  constexpr int HK = PARTS == 1 ? 2 : 1, TK = 16 * HK, TM = 64 * MB, TN = 128;
+  constexpr int PER = 4 * HK, kRows = 256 / PER;       // threads that share a row's step, rows that all threads read at once
+  constexpr int NA = TM / kRows, NW = TN / kRows;      // 16-byte pieces per thread and step
+  constexpr int kPad = HK == 2 ? 2 : 4;                // (the octets of a row in different banks)
+  constexpr int kOctX = TM + kPad, kOctW = TN + kPad, kPartX = 2 * HK * kOctX, kPartW = 2 * HK * kOctW;  // units of 16 bytes
   __shared__ __attribute__((aligned(16))) u32x4 lds[2][3 * kPartX + PARTS * kPartW];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int grp = 0, tm = blockIdx.x, r0 = 0, r1 = g.rows;
+  const int columns = (g.N + (SWIGLU ? TN / 2 : TN) - 1) / (SWIGLU ? TN / 2 : TN);
+  int grp = 0, tm = blockIdx.x / columns, r0 = 0, r1 = g.rows;
   if (g.tile_off) {
     if (tm >= g.tile_off[g.groups]) return;
     for (int e0 = 0; e0 < g.groups; e0 += 64)
@@ -454,27 +460,32 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
   }
   const int m0 = r0 + tm * TM;
   if (m0 >= r1) return;
-  const int K = g.K, N = g.N, o0 = blockIdx.y * (SWIGLU ? TN / 2 : TN);
+  const int K = g.K, N = g.N, o0 = blockIdx.x % columns * (SWIGLU ? TN / 2 : TN);
   const float *w = g.w + (long long)grp * (SWIGLU ? 2 : 1) * N * K;
   // the matrix row behind row i of the tile
   auto matrix_row = [&](int i) {
     return SWIGLU ? (i >> 5 & 1) * N + min(o0 + (i >> 6) * 32 + (i & 31), N - 1) : min(o0 + i, N - 1);
   };
 
-  // piece u of a thread: quarter tid % 4 of tile row tid / 4 + 64 u
-  const int srow = threadIdx.x >> 2, k4 = 4 * (threadIdx.x & 3);
+  // piece u of a thread: four k, tid % PER, of tile row tid / PER + kRows u
+  const int srow = threadIdx.x / PER, k4 = 4 * (threadIdx.x % PER);
   const float *ap[NA], *bp[NW];
 #pragma unroll
   for (int u = 0; u < NA; ++u) {
-    const int r = min(m0 + srow + 64 * u, r1 - 1);
+    const int r = min(m0 + srow + kRows * u, r1 - 1);
     ap[u] = g.x + (long long)(g.gather ? g.gather[r] : r) * K;
   }
 #pragma unroll
-  for (int u = 0; u < NW; ++u) bp[u] = w + (long long)matrix_row(srow + 64 * u) * K;
+  for (int u = 0; u < NW; ++u) bp[u] = w + (long long)matrix_row(srow + kRows * u) * K;
+  unsigned a_off[NA], b_off[NW];  // kSteps: bytes from a step's first column of row 0 (under 4 GiB: checked at launch)
+#pragma unroll
+  for (int u = 0; u < NA; ++u) a_off[u] = (unsigned)((ap[u] - g.x + k4) * 4);
+#pragma unroll
+  for (int u = 0; u < NW; ++u) b_off[u] = (unsigned)((bp[u] - w + k4) * 4);
   f32x4 sa[2][NA], sb[2][NW];
   auto piece = [&](const float *p, int k) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (VEC) {
+    if constexpr (LOADS != kScalar) {
       if (k < K) v = *(const f32x4 *)(p + k);
     } else {
       if (k < K) v.x = p[k];
@@ -484,26 +495,33 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
     }
     return v;
   };
-  auto load = [&](int set, int k0) {  // (steps behind the last one are zeros, which nobody reads)
+  // (steps behind the last one repeat it, which nobody reads.  No load hangs on a condition: the branches around them had
+  // the loop wait for every load it had just issued)
+  const int last = (K - 1) / TK * TK;
+  auto load = [&](int set, int k0) {
+    k0 = min(k0, last);
+    const int k = k0 + k4, at = min(k, K - 4);
 #pragma unroll
     for (int u = 0; u < NA; ++u)
-      sa[set][u] = piece(ap[u], k0 + k4);
+      sa[set][u] = LOADS == kSteps ? load_at((const f32x4 *)(g.x + k0), a_off[u]) : LOADS == kScalar ? piece(ap[u], k) : *(const f32x4 *)(ap[u] + at);
 #pragma unroll
-    for (int u = 0; u < NW; ++u) sb[set][u] = piece(bp[u], k0 + k4);
+    for (int u = 0; u < NW; ++u)
+      sb[set][u] = LOADS == kSteps ? load_at((const f32x4 *)(w + k0), b_off[u]) : LOADS == kScalar ? piece(bp[u], k) : *(const f32x4 *)(bp[u] + at);
   };
-  auto park = [&](int set, u32x4 *stage) {
+  auto park = [&](int set, int k0, u32x4 *stage) {  // (pieces of k0's step behind the end of K count as zeros)
+    const bool out = LOADS == kPieces && k0 + k4 >= K;
     u32x2 *at = (u32x2 *)(stage + (k4 >> 3) * kOctX + srow) + (k4 >> 2 & 1);
 #pragma unroll
     for (int u = 0; u < NA; ++u)
-      split_quad(sa[set][u] * kLift, at[128 * u], at[128 * u + 2 * kPartX], at[128 * u + 4 * kPartX]);
+      split_quad((out ? f32x4{0.f, 0.f, 0.f, 0.f} : sa[set][u]) * kLift, at[2 * kRows * u], at[2 * (kRows * u + kPartX)], at[2 * (kRows * u + 2 * kPartX)]);
     at = (u32x2 *)(stage + 3 * kPartX + (k4 >> 3) * kOctW + srow) + (k4 >> 2 & 1);
 #pragma unroll
     for (int u = 0; u < NW; ++u) {
-      const f32x4 v = sb[set][u] * kLift;
+      const f32x4 v = (out ? f32x4{0.f, 0.f, 0.f, 0.f} : sb[set][u]) * kLift;
       if constexpr (PARTS == 3)
-        split_quad(v, at[128 * u], at[128 * u + 2 * kPartW], at[128 * u + 4 * kPartW]);
+        split_quad(v, at[2 * kRows * u], at[2 * (kRows * u + kPartW)], at[2 * (kRows * u + 2 * kPartW)]);
       else
-        at[128 * u] = u32x2{pack_high(v.x, v.y), pack_high(v.z, v.w)};
+        at[2 * kRows * u] = u32x2{pack_high(v.x, v.y), pack_high(v.z, v.w)};
     }
   };
   const int n = lane & 31, half = lane >> 5, rw = wave & 1, cw = wave >> 1;
@@ -519,35 +537,41 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
   const int steps = (K + TK - 1) / TK;
   load(0, 0);
   load(1, TK);
-  park(0, lds[0]);
+  __builtin_amdgcn_sched_barrier(0);  // (the loop waits for its loads in the order they have here)
+  park(0, 0, lds[0]);
   load(0, 2 * TK);
   __syncthreads();
   auto step = [&](int kt, int set) {  // set: holds step kt + 1
     const u32x4 *stage = lds[kt & 1];
-    u32x4 af[3][MB], bf[PARTS][2];
+    u32x4 af[HK][3][MB], bf[HK][PARTS][2];
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
+    for (int h = 0; h < HK; ++h)
 #pragma unroll
-      for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * kPartX + 32 * a];
+      for (int p = 0; p < 3; ++p) {
 #pragma unroll
-      for (int b = 0; b < 2 && p < PARTS; ++b) bf[p][b] = stage[b_unit + p * kPartW + 32 * b];
-    }
-    park(set, lds[(kt & 1) ^ 1]);
+        for (int a = 0; a < MB; ++a) af[h][p][a] = stage[a_unit + p * kPartX + 2 * h * kOctX + 32 * a];
+#pragma unroll
+        for (int b = 0; b < 2 && p < PARTS; ++b) bf[h][p][b] = stage[b_unit + p * kPartW + 2 * h * kOctW + 32 * b];
+      }
+    park(set, min((kt + 1) * TK, last), lds[(kt & 1) ^ 1]);
     load(set, (kt + 3) * TK);
 #pragma unroll
-    for (int p = 0; p < 6; ++p) {
-      if (kPartB[p] >= PARTS) continue;
+    for (int h = 0; h < HK; ++h)
 #pragma unroll
-      for (int a = 0; a < MB; ++a)
+      for (int p = 0; p < 6; ++p) {
+        if (kPartB[p] >= PARTS) continue;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p] < PARTS ? kPartB[p] : 0][b], acc[a][b]);
-    }
+        for (int a = 0; a < MB; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[h][kPartA[p]][a], bf[h][kPartB[p] < PARTS ? kPartB[p] : 0][b], acc[a][b]);
+      }
     __syncthreads();
   };
-  for (int kt = 0; kt < steps; kt += 2) {
-    step(kt, 1);
-    if (kt + 1 < steps) step(kt + 1, 0);
+  for (int kt = 1; kt < steps; kt += 2) {  // (in pairs: a way out between them costs waits, too)
+    step(kt - 1, 1);
+    step(kt, 0);
   }
+  if (steps & 1) step(steps - 1, 1);
 
   // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which (777
   // tokens of width 2048, the fifth NaN: 2.8 ms a layer with its copies against 1.6 without; one k at a time it was 73)
@@ -663,17 +687,26 @@ hipError_t launch_product_tm(const GroupedArgs &g, bool swiglu, hipStream_t stre
   constexpr int TM = 64 * MB, TN = 128;
   const long long tiles = g.tile_off ? (long long)g.rows / TM + (g.groups < g.rows ? g.groups : g.rows) : ((long long)g.rows + TM - 1) / TM;
   const int cols = swiglu ? TN / 2 : TN, ny = (g.N + cols - 1) / cols;
-  if (tiles < 1 || tiles > 0x7fffffff || ny > 65535) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)tiles, (unsigned)ny);
+  // (columns fastest: with eight blocks of columns the tiles of an expert's rows meet its matrix in one XCD's L2)
+  if (tiles < 1 || tiles * ny > 0x7fffffff) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(tiles * ny));
   const bool vec = (g.K & 3) == 0 && !(((uintptr_t)g.x | (uintptr_t)g.w) & 15);
-  if (swiglu && vec)
-    hipLaunchKernelGGL((moe_product_kernel<MB, true, true, PARTS>), grid, dim3(256), 0, stream, g);
+  const int loads = !vec ? kScalar : g.K % (PARTS == 1 ? 32 : 16) || (long long)(g.rows > 2 * g.N ? g.rows : 2 * g.N) * g.K >= 1LL << 30 ? kPieces : kSteps;
+#define SHAINET_MOE_PRODUCT(SWIGLU_, LOADS_) \
+  hipLaunchKernelGGL((moe_product_kernel<MB, SWIGLU_, LOADS_, PARTS>), grid, dim3(256), 0, stream, g)
+  if (swiglu && loads == kSteps)
+    SHAINET_MOE_PRODUCT(true, kSteps);
+  else if (swiglu && loads == kPieces)
+    SHAINET_MOE_PRODUCT(true, kPieces);
   else if (swiglu)
-    hipLaunchKernelGGL((moe_product_kernel<MB, true, false, PARTS>), grid, dim3(256), 0, stream, g);
-  else if (vec)
-    hipLaunchKernelGGL((moe_product_kernel<MB, false, true, PARTS>), grid, dim3(256), 0, stream, g);
+    SHAINET_MOE_PRODUCT(true, kScalar);
+  else if (loads == kSteps)
+    SHAINET_MOE_PRODUCT(false, kSteps);
+  else if (loads == kPieces)
+    SHAINET_MOE_PRODUCT(false, kPieces);
   else
-    hipLaunchKernelGGL((moe_product_kernel<MB, false, false, PARTS>), grid, dim3(256), 0, stream, g);
+    SHAINET_MOE_PRODUCT(false, kScalar);
+#undef SHAINET_MOE_PRODUCT
   return hipGetLastError();
 }
 
