@@ -991,6 +991,43 @@ def test_prefill_of_very_small_operands(hip, hd, KV, T, cached, q_by, k_by, v_by
         assert np.abs(got[:, h] - want).max() <= 1e-5 + 2.0 ** -149 / v_by, h
 
 
+@pytest.mark.parametrize("hd,KV,T,cached", [(64, 2, 300, 0), (128, 2, 70, 100), (96, 4, 40, 33), (64, 8, 1500, 0)])
+@pytest.mark.parametrize("pair", [-24, -13, -11, -9, 5, 13, 15, 17, 24])
+def test_prefill_scores_at_the_limits_of_two_fp16_parts(hip, hd, KV, T, cached, pair):
+    """Scores whose queries pass 2^9 in log2 units and whose keys pass 65520, and both well below fp16's normal numbers: one
+    rotated pair is 2^pair of the others in the keys, the other way round in the queries.  Half a key's or a query's last
+    bit of 22, the rounding of each sum over hd in fp32, and the product of the two second parts: at most 2^-20 of the sum of
+    the products' sizes in a score, twice that of the largest value in a result, and 2^-20 of it for the sums behind."""
+    import torch
+
+    H, S = 2 * KV, cached + T
+    g = torch.Generator(device="cuda").manual_seed(hd + T + pair)
+    q, k, v = (torch.randn((T, n * hd), generator=g, device="cuda") for n in (H, KV, KV))
+    kc, vc = (torch.randn((KV, max(cached, 1), hd), generator=g, device="cuda") for _ in range(2))
+    for d in (0, hd // 2):
+        q.view(T, H, hd)[..., d] *= 2.0 ** -pair
+        k.view(T, KV, hd)[..., d] *= 2.0 ** pair
+        kc[..., d] *= 2.0 ** pair
+    ctx = hip.AttnContext(H, KV, hd, max_positions=S)
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, S)
+    if cached:
+        cache.fill(0, kc, vc)
+    ctx.sync()
+    got = ctx.forward(cache, q, k, v, [T])
+    ctx.sync()
+    got = got.cpu().numpy().reshape(T, H, hd).astype(np.float64)
+    qr = ctx.last_q_rot(T).astype(np.float64).reshape(T, H, hd)
+    for h in range(H):
+        kr, vr = (a.astype(np.float64) for a in cache.read(0, h // 2, 0, S))
+        s = qr[:, h] @ kr.T / np.sqrt(hd)
+        sizes = np.abs(qr[:, h]) @ np.abs(kr).T / np.sqrt(hd)
+        s[np.arange(S)[None] > cached + np.arange(T)[:, None]] = -np.inf
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p / p.sum(-1, keepdims=True)) @ vr
+        assert np.abs(got[:, h] - want).max() <= (2 * sizes.max() + 1) * 2.0 ** -20 * np.abs(vr).max(), h
+
+
 @pytest.mark.parametrize("hd,KV,T,tiny", [(64, 2, 300, 2.0 ** -124), (128, 2, 300, 2.0 ** -135), (96, 4, 140, 2.0 ** -124), (64, 8, 2300, 0.0)])
 def test_prefill_of_zeros_and_a_tiny_value(hip, hd, KV, T, tiny):
     """Head 0's values are zeros but for one key's, every third row's queries zeros: sums that are small because values
