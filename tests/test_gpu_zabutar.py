@@ -339,6 +339,19 @@ def test_experts(hip, tmp_path, name):
         close(block_cut(b, x, cuts), want)
 
 
+@pytest.mark.parametrize("top", [1, 8, 9])
+@pytest.mark.parametrize("ff,shared", [(4, 0), (256, 1024), (260, 1028), (512, 36), (516, 4), (768, 0), (772, 1100)])
+def test_experts_down_product_of_few_rows(hip, tmp_path, ff, shared, top):
+    """All rows of an output asked for at once up to 8 slots and 768 values (one, two and three spans of 256, whole and
+    ragged), slot by slot beyond either; shared experts around 1024 values."""
+    cfg = zm.config([zm.layer(zm.hgrn2(heads=1, dim=4, vdim=4), zm.moe(ff=ff, experts=10, identity=2, top=top, groups=1, keep=1,
+                                                                       shared=shared))], width=52)
+    p = Pair(hip, tmp_path, cfg, edit=lambda w: w.update({"l0.mix.o": 0 * w["l0.mix.o"]}), seed=3)
+    x = (2 * np.random.default_rng(4).standard_normal((12, 52))).astype(np.float32)
+    want = p.layer(0, x)
+    close(block_cut(p.model.blocks[0], x, (1, 1, 8, 2)), want)
+
+
 @pytest.mark.parametrize("name", ["plain", "one", "odd"])
 def test_experts_keep_rows_apart(hip, tmp_path, name):
     """A row that is not a number shares tiles of an expert (64 and 128 rows, whole and ragged) with rows before it that are."""
