@@ -255,6 +255,28 @@ def test_expanded_of_very_small_and_very_large_queries(hip, tmp_path, monkeypatc
     close(p.model.blocks[0].forward_cached(x), p.layer(0, x), 2e-5)
 
 
+@pytest.mark.parametrize("q_by", [-24, -17, -14, 6, 9, 11, 24])
+@pytest.mark.parametrize("name", ["even", "wide", "vast"])
+def test_expanded_scores_at_the_limits_of_two_fp16_parts(hip, tmp_path, monkeypatch, name, q_by):
+    """Queries around 2^q_by pass 2^9 in log2 units, unrotated keys around 2^-q_by pass 65520 and lie below fp16's normal
+    numbers.  A score loses 2^-20 of the sum of its products' sizes (22 bits an operand, fp32 sums) wherever it is taken, which
+    the bar of the rows beside it, 2e-5 of the largest result, holds 20 times over."""
+    monkeypatch.setenv("SHAINET_HIP_LATENT_PATH", "expanded")
+    holds = lambda a: (a.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+
+    def edit(w):
+        m = GEOMETRIES[name]["m"]
+        q = w["l0.mix.uq"].reshape(m["heads"], m["dim"] + m["rot_dim"], -1).copy()
+        q[:, :m["dim"]] *= np.float32(2.0 ** q_by)
+        q[:, m["dim"]:] *= np.float32(2.0 ** min(q_by, 0))
+        w["l0.mix.uq"] = holds(q.reshape(w["l0.mix.uq"].shape))
+        w["l0.mix.uk"] = holds(w["l0.mix.uk"] * np.float32(2.0 ** -q_by))
+
+    p = Pair(hip, tmp_path, geometry(name, mlp=False), edit=edit)
+    x = np.random.default_rng(12).standard_normal((200, p.cfg["width"])).astype(np.float32)
+    close(p.model.blocks[0].forward_cached(x), p.layer(0, x), 2e-5)
+
+
 @pytest.mark.parametrize("path", ["absorbed", "expanded"])
 def test_sink(hip, tmp_path, monkeypatch, path):
     """Sinks that take nearly everything, about half and nothing; the first position sees one key only."""
