@@ -402,7 +402,7 @@ __global__ __launch_bounds__(1024) void latent_out_kernel(const float *__restric
 // keys][column], column d at place d / NT of block d % NT, 36 units a block.
 // Bound by registers (256 of them: two wavefronts per SIMD) and the splits beside the MFMAs.  2048 rows of 16 heads of 192 and
 // 128 dimensions: 268 us with v_mfma_f32_32x32x2_f32, whose cycles the vector ALU cannot use, 196 with three bf16 numbers a
-// query and key (too many registers: the queries were split again for every tile), some 170 with two fp16 numbers.
+// query and key (too many registers: the queries were split again for every tile), 133 with two fp16 numbers.
 // NK: pieces of 8 query / key dimensions at most; NT: tiles of 32 value dimensions.
 struct LatentPrefillArgs {
   const float *q;        // [T, H (dim + rot_dim)], rotated (launch_latent_append)
