@@ -392,17 +392,19 @@ __global__ __launch_bounds__(1024) void latent_out_kernel(const float *__restric
 // A workgroup owns 128 rows of one head, a wavefront 32 of them; all walk the keys in tiles of 32 that
 // go global memory -> registers -> split -> LDS (one stage of keys, one of values; the values travel behind the
 // score MFMAs, the next tile's keys behind the others).  Two workgroups share a compute unit, so that one's barriers
-// hide behind the other's MFMAs.  Values and probabilities are exact sums of three bf16 numbers, queries and
-// keys sums of two fp16 numbers (split_mfma.hpp), the queries' parts in registers.  S^T = K Q^T, so that the
-// probabilities come out of the accumulator laid out as the B operand of O^T += V^T P^T:
+// hide behind the other's MFMAs.  Queries, keys, values and probabilities are exact sums of three bf16 numbers
+// (split_mfma.hpp); queries of more than 128 dimensions have no registers for their parts and are split
+// again for every tile, beside the MFMAs.  S^T = K Q^T, so that the probabilities come out of the accumulator laid out as
+// the B operand of O^T += V^T P^T:
 //   scores:  m = key within the tile, n = row; step i of lane half j covers d = 16 i + 8 j + 0..7;
 //            d runs over the unrotated dimensions, padded to a multiple of 8, then the rotated ones.
 //   output:  tile t, m: d = NT m + t; step u of lane half j covers keys 16 u + 4 j + {0..3, 8..11}.
 // LDS in units of 16 bytes: keys [part][octet of d][key], an octet 33 units; values [part][group 2 u + j of eight
 // keys][column], column d at place d / NT of block d % NT, 36 units a block.
-// Bound by registers (256 of them: two wavefronts per SIMD) and the splits beside the MFMAs.  2048 rows of 16 heads of 192 and
-// 128 dimensions: 268 us with v_mfma_f32_32x32x2_f32, whose cycles the vector ALU cannot use, 196 with three bf16 numbers a
-// query and key (too many registers: the queries were split again for every tile), 133 with two fp16 numbers.
+// Bound by registers (256 of them: two wavefronts per SIMD) and the splits beside the MFMAs: 2048 rows of 16 heads of 192 and 128
+// dimensions 268 -> 208 us against v_mfma_f32_32x32x2_f32, whose cycles the vector ALU cannot use.  (Two fp16 numbers a query
+// and key, three products a score and the queries' parts in registers took a third less, but such numbers leave out up to
+// 2^-21 of a product.)
 // NK: pieces of 8 query / key dimensions at most; NT: tiles of 32 value dimensions.
 struct LatentPrefillArgs {
   const float *q;        // [T, H (dim + rot_dim)], rotated (launch_latent_append)
@@ -423,7 +425,8 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
   constexpr int VSTR = NT * 32, KS = NK / 2;  // columns of the output; MFMA steps of the scores
   constexpr int KU = (NK + 7) / 8, VU = NT / 2;  // per thread: octets of a tile's keys, eight rows of a column of its values
   constexpr int kOct = 33, kPartK = NK * kOct, kGroup = NT * 36, kPartV = 4 * kGroup;
-  __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kPartK + 3 * kPartV];
+  constexpr bool HELD = NK <= 16 && NK * NT <= 48;  // the parts of the query stay in registers
+  __shared__ __attribute__((aligned(16))) u32x4 lds[3 * kPartK + 3 * kPartV];
   const LatentShape &sh = a.sh;
   // heads fastest: with a multiple of 8 heads an XCD (index % 8) keeps to its own heads' keys and
   // values; the blocks with the most keys start first
@@ -462,7 +465,7 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
   }
   const int v_col = threadIdx.x % VSTR, v_group = threadIdx.x / VSTR;
   const int v_row = 16 * (v_group >> 1) + 4 * (v_group & 1);  // and 16 further on for the second
-  const int v_unit = 2 * kPartK + v_group * kGroup + v_col % NT * 36 + v_col / NT;
+  const int v_unit = 3 * kPartK + v_group * kGroup + v_col % NT * 36 + v_col / NT;
   const unsigned v_off = v_col < sh.vdim ? v_col : 0;  // (columns beyond are never stored)
   const float *v_src = a.kv + sh.H * dn + h * sh.vdim;
   f32x4 stage[2 * (KU > VU ? KU : VU)];
@@ -493,32 +496,27 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
               v_src[(unsigned long long)(unsigned)min(kt * 32 + v_row + 16 * u + (i & 3) + 8 * (i >> 2), b_hi) * kv_stride + v_off];
     }
   };
+  auto park = [&](int u, int unit, int part, float lift) {
+    u32x4 hi, mid, lo;
+    split_octet(stage[2 * u] * lift, stage[2 * u + 1] * lift, hi, mid, lo);
+    lds[unit] = hi;
+    lds[unit + part] = mid;
+    lds[unit + 2 * part] = lo;
+  };
   auto park_k = [&]() {
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int unit = min(sub + 8 * u, NK - 1) * kOct + k_row;
-      u32x4 hi, lo;
-      split_octet_f16(stage[2 * u], stage[2 * u + 1], hi, lo);
-      lds[unit] = hi;
-      lds[unit + kPartK] = lo;
-    }
+    for (int u = 0; u < KU; ++u) park(u, min(sub + 8 * u, NK - 1) * kOct + k_row, kPartK, 1.f);
   };
   auto park_v = [&]() {
 #pragma unroll
-    for (int u = 0; u < VU; ++u) {
-      const int unit = v_unit + 2 * u * kGroup;
-      u32x4 hi, mid, lo;
-      split_octet(stage[2 * u] * kLift, stage[2 * u + 1] * kLift, hi, mid, lo);
-      lds[unit] = hi;
-      lds[unit + kPartV] = mid;
-      lds[unit + 2 * kPartV] = lo;
-    }
+    for (int u = 0; u < VU; ++u) park(u, v_unit + 2 * u * kGroup, kPartV, kLift);
   };
   if (kt0 < kt1) load_k(kt0);
 
-  u32x4 qf[KS][2];
+  f32x4 qr[HELD ? 1 : KS][2];
+  u32x4 qf[HELD ? KS : 1][3];
   const float *q_row = a.q + ((long long)my_row * sh.H + h) * (dn + dr);
-  float most = 0.f;
+  QueryRange range;
 #pragma unroll
   for (int i = 0; i < KS; ++i) {
     f32x4 x[2];
@@ -527,12 +525,15 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
       const int d = 16 * i + 8 * j + 4 * w, e = d - dn8;
       x[w] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (d < dn || (e >= 0 && e < dr)) x[w] = *(const f32x4 *)(q_row + (d < dn ? d : dn + e));
-#pragma unroll
-      for (int r = 0; r < 4; ++r) most = fmaxf(most, fabsf(x[w][r] * a.c));
+      range.add(x[w]);
+      x[w] *= a.c;
     }
-    split_octet_f16(x[0] * (a.c * kQueryLift), x[1] * (a.c * kQueryLift), qf[i][0], qf[i][1]);
+    if constexpr (HELD)
+      split_octet(x[0], x[1], qf[i][0], qf[i][1], qf[i][2]);
+    else
+      qr[i][0] = x[0], qr[i][1] = x[1];
   }
-  const bool apart = __any(!(most < kMostQuery));  // some query of the wavefront needs its scores in fp32
+  const bool apart = __any(range.apart(a.c));  // some query of the wavefront needs its scores in fp32
   f32x16 o[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -549,20 +550,23 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
     load_v(kt);
     const int k_first = kt * 32, k_last = k_first + 31;
     const bool visible = wave_active && k_first <= w_hi_max && k_last >= w_lo_min;
-    f32x16 s, low;
+    f32x16 s;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = low[r] = 0.f;
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
     if (visible) {
       const u32x4 *kl = lds + j * kOct + n;
 #pragma unroll
       for (int i = 0; i < KS; ++i) {
-        const u32x4 high_part = kl[2 * i * kOct], low_part = kl[kPartK + 2 * i * kOct];
-        low = mfma_f16(low_part, qf[i][0], low);
-        s = mfma_f16(high_part, qf[i][0], s);
-        low = mfma_f16(high_part, qf[i][1], low);
-      }
+        u32x4 kf[3];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = fmaf(low[r], kLowDrop, s[r]) * kScoreDrop;
+        for (int w = 0; w < 3; ++w) kf[w] = kl[w * kPartK + 2 * i * kOct];
+        if constexpr (!HELD) {
+          asm volatile("" : "+v"(qr[i][0]), "+v"(qr[i][1]));  // (not moved out of the loop over the tiles)
+          split_octet(qr[i][0], qr[i][1], qf[0][0], qf[0][1], qf[0][2]);
+        }
+#pragma unroll
+        for (int w = 0; w < 6; ++w) s = mfma_bf16(kf[kPartA[w]], qf[HELD ? i : 0][kPartB[w]], s);
+      }
       if (k_first < w_lo_max || k_last > w_hi_min) {  // an edge of some row's keys lies in the tile
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -598,7 +602,7 @@ __global__ __launch_bounds__(256, NK <= 24 ? 2 : 1) void latent_prefill_kernel(c
     __syncthreads();
     if (kt + 1 < kt1) load_k(kt + 1);
     if (visible) {
-      const u32x4 *vl = lds + 2 * kPartK + j * kGroup + n;
+      const u32x4 *vl = lds + 3 * kPartK + j * kGroup + n;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         u32x4 pf[3];

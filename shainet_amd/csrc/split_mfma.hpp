@@ -2,10 +2,10 @@
 // rounded to bf16, the rest rounded to bf16, and the rest of that (8 + 8 + 8 mantissa bits with signs of
 // their own).  A bf16 has a float's exponents and 16 bits less behind them, so the rests of a float below 2^-110
 // would not be whole; operands are lifted by 2^24 first, which makes every part of every float, the smallest
-// subnormal's too, a normal bf16 or zero, and results are brought down again.  (Not probabilities, whose row holds one
-// near 1, nor the values of prefill attention, which looks at its sums instead.)  That is 2 to 4 % of a prompt's
-// products; rows of x around 2^-120 had an error of 3.5e-5 without, and 2e-7 with it, as rows around 1 have.  Of the nine
-// products of two such sums
+// subnormal's too, a normal bf16 or zero, and results are brought down again.  (Not the operands of scores, see
+// QueryRange and split_pair_f16, nor probabilities, whose row holds one near 1, nor the values of prefill attention, which looks at its
+// sums instead.)  That is 2 to 4 % of a prompt's products; rows of x around 2^-120 had an error of 3.5e-5 without, and
+// 2e-7 with it, as rows around 1 have.  Of the nine products of two such sums
 // the six largest make up the product to 2^-24 of itself: of the three left out two can reach 2^-25 each.  Six
 // v_mfma_f32_32x32x16_bf16 of 32 cycles do what eight v_mfma_f32_32x32x2_f32 of 64 do (192 against 512
 // cycles per 32 x 32 x 16; a loop of nothing else: 1876 TFLOP/s of bf16 = 312 of fp32, against 155), they
@@ -32,6 +32,28 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Operands of a product are lifted before they are split; its result, or that of one lifted operand, comes down.
 constexpr float kLift = 0x1p24f, kDrop = 0x1p-48f, kDropOne = 0x1p-24f;
+
+// Scores of attention (of latent heads; prefill attention's: split_pair_f16) are taken of queries and keys as they are: only their size against 1 counts, and what the
+// small ones lose is 2^-134 of the other operand at most.  It can count where a query (scaled, in log2 units) holds
+// numbers of 2^100 and more, and keys numbers below 2^-110, or the query numbers below 2^-109 (other than 0), and keys
+// very large ones: the scores of such queries are taken in fp32.
+struct QueryRange {
+  unsigned least = ~0u, most = 0u;  // of the bits of |q|, doubled; zeros lie above all in `least`
+  __device__ __forceinline__ void add(f32x4 q) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned bits = __builtin_bit_cast(unsigned, q[i]) << 1;
+      least = min(least, bits - 1u);
+      most = max(most, bits);
+    }
+  }
+  // c: what the queries are multiplied by for the scores (the multiplication itself stays with the subtractions of the
+  // split, where it is not rounded)
+  __device__ __forceinline__ bool apart(float c) const {
+    const float lo = __builtin_bit_cast(float, (least + 1u) >> 1), hi = __builtin_bit_cast(float, most >> 1);
+    return (least != ~0u && !(fabsf(lo * c) >= 0x1p-109f)) || !(fabsf(hi * c) < 0x1p100f);
+  }
+};
 
 // two floats rounded to bf16, the first in the low half
 __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
@@ -84,7 +106,7 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
 }
 
-// Scores of prefill attention, of latent heads too: both operands as sums of two fp16 numbers, the second kept 2^11 times as large so that it
+// Scores of prefill attention: both operands as sums of two fp16 numbers, the second kept 2^11 times as large so that it
 // has the range of the first (22 to 23 bits of a float from 2^-14 up, below that whatever is 2^-36 or more), and three
 // products of the four, those with a second part in an accumulator of their own.  The kernels are bound by the matrix
 // cores, so half the products of the sums of three bf16 numbers show: 2048 rows of 32 / 8 heads of 64 102.9 -> 89.0 us,

@@ -258,9 +258,8 @@ def test_expanded_of_very_small_and_very_large_queries(hip, tmp_path, monkeypatc
 @pytest.mark.parametrize("q_by", [-24, -17, -14, 6, 9, 11, 24])
 @pytest.mark.parametrize("name", ["even", "wide", "vast"])
 def test_expanded_scores_at_the_limits_of_two_fp16_parts(hip, tmp_path, monkeypatch, name, q_by):
-    """Queries around 2^q_by pass 2^9 in log2 units, unrotated keys around 2^-q_by pass 65520 and lie below fp16's normal
-    numbers.  A score loses 2^-20 of the sum of its products' sizes (22 bits an operand, fp32 sums) wherever it is taken, which
-    the bar of the rows beside it, 2e-5 of the largest result, holds 20 times over."""
+    """Queries around 2^q_by in log2 units and unrotated keys around 2^-q_by, the other operand beyond what 16 bits with five
+    of exponent hold or below their normal numbers: the parts of a score are bf16 numbers, to which this makes no difference."""
     monkeypatch.setenv("SHAINET_HIP_LATENT_PATH", "expanded")
     holds = lambda a: (a.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
 
@@ -275,6 +274,48 @@ def test_expanded_scores_at_the_limits_of_two_fp16_parts(hip, tmp_path, monkeypa
     p = Pair(hip, tmp_path, geometry(name, mlp=False), edit=edit)
     x = np.random.default_rng(12).standard_normal((200, p.cfg["width"])).astype(np.float32)
     close(p.model.blocks[0].forward_cached(x), p.layer(0, x), 2e-5)
+
+
+@pytest.mark.parametrize("m", [dict(heads=4, dim=32, rot_dim=16, vdim=40, kv_rank=32), dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=512),
+                               dict(heads=2, dim=224, rot_dim=32, vdim=72, kv_rank=512)])
+def test_expanded_scores_keep_all_24_bits(hip, tmp_path, monkeypatch, m):
+    """Queries of 2^6 (1 + 2^-11 - 2^-14) in log2 units; the even rows' keys hold 1 + 2^-11 - 2^-14 and 1 + 2^-11 + 2^-14 by turns, with
+    signs by turns: a score is 2^-14 of the sum of its products' sizes, and what operands cut to 11 and 11 bits leave out of each, 0.8 x
+    2^-22 of it, adds up.  The odd rows' keys have the same score from one product.  Three bf16 numbers an operand leave out
+    two products of 2^-25 at most; as much again for the sums and the factor of the queries.  Every number in front of the
+    scores is exact: saturated norms, latent rows of two equal values."""
+    monkeypatch.setenv("SHAINET_HIP_LATENT_PATH", "expanded")
+    cfg = tm.config([tm.layer(tm.mixer(q_rank=32, window=0, **m), None)], 64, 160)
+    H, dim, vdim, rank = (m[k] for k in ("heads", "dim", "vdim", "kv_rank"))
+    v, size = (rank / 2) ** 0.5, 2.0 ** (13 - int(np.log2(dim)))  # a latent value behind its norm; a key's size
+    c = cfg["layers"][0]["mixer"]["scale"] * np.log2(np.e)
+    holds = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+
+    def edit(w):
+        for n in w:
+            if n.startswith("l0."):
+                w[n] = np.zeros_like(w[n])
+        for n in ("norm1", "norm1.alpha", "mix.dq.norm", "mix.dkv.norm"):
+            w["l0." + n] = np.ones_like(w["l0." + n])
+        w["l0.mix.sink"] -= 2.0 ** 30
+        w["l0.mix.dkv"][:2, 0] = w["l0.mix.dkv"][2:4, 1] = w["l0.mix.dq"][:2, 2] = 2.0 ** 20  # of even rows, odd rows, all rows
+        q = np.full(1, 2.0 ** 6 * (1 + 2.0 ** -11 - 2.0 ** -14) / c / 4)
+        uq = w["l0.mix.uq"].reshape(H, dim + m["rot_dim"], 32)
+        uq[:, :dim, 0] = holds(q)
+        uq[:, :dim, 1] = holds(q - holds(q))
+        uk = w["l0.mix.uk"].reshape(H, dim, rank)
+        uk[:, 0::2, 0], uk[:, 1::2, 0] = size / v, -size / v
+        uk[:, 0::2, 1], uk[:, 1::2, 1] = size / v * 7 * 2.0 ** -14, -size / v * 9 * 2.0 ** -14
+        uk[:, 1, 2] = -size / v * dim * 2.0 ** -14
+        w["l0.mix.uv"][:, 0], w["l0.mix.uv"][:, 2] = 1 / v, -1 / v
+        w["l0.mix.o"][4:4 + vdim, :vdim] = np.eye(vdim)
+
+    p = Pair(hip, tmp_path, cfg, edit=edit)
+    x = np.zeros((200, 160), np.float32)
+    x[0::2, 0] = x[1::2, 1] = x[:, 2] = 100.0
+    got = np.asarray(p.model.blocks[0].forward_cached(x), np.float64)
+    # gates of one half, and a result moves by ln 2 / 2 of what the difference of the two scores does
+    assert np.abs(got - p.layer(0, x)).max() <= 0.5 * np.log(2) / 2 * 2.0 ** -23 * (2.0 ** 6 * size * dim) + 1e-5
 
 
 @pytest.mark.parametrize("path", ["absorbed", "expanded"])
