@@ -63,7 +63,7 @@ __device__ __forceinline__ void locate_block(const SeqTable &st, int rank, int &
   vb = st.work_off[s] - 1 - level;
 }
 
-// Units of 16 bytes (eight fp16 or bf16, one MFMA operand of a lane) that one key tile takes in LDS.  K: [part][octet of
+// Units of 16 bytes (eight bf16, one MFMA operand of a lane) that one key tile takes in LDS.  K: [part][octet of
 // d][key], an octet's 32 keys one unit apart from a multiple of 16 (a row's octets are written side by side).  V:
 // [part][group of eight keys][column], column d at place d / NT of block d % NT, four units of padding a block; group
 // 2 u + j holds the keys 16 u + 4 j + {0 .. 3, 8 .. 11}, the ones whose probabilities lane half j has in its
@@ -73,7 +73,7 @@ struct TileUnits {
   static constexpr int NT = HD / 32;
   static constexpr int kOctK = 33, kPartK = HD / 8 * kOctK;
   static constexpr int kGroupV = NT * 36, kPartV = 4 * kGroupV;
-  static constexpr int kK = 2 * kPartK, kTile = kK + 3 * kPartV;
+  static constexpr int kK = 3 * kPartK, kTile = kK + 3 * kPartV;
 };
 
 // G = 1: four wavefronts, each with 32 virtual rows, walk the key tiles together.
@@ -89,14 +89,16 @@ struct TileUnits {
 // pieces beyond it repeat the row's first piece (a cache hit, no HBM traffic).
 // BIAS (with PAD): scores gain a value by distance (DistanceBias), value rows have a width of their own.
 //
-// Values and probabilities enter the MFMAs as exact sums of three bf16 numbers, queries and keys as sums of two fp16
-// numbers (split_mfma.hpp): the queries once, a tile by the workgroup on its way to LDS, the probabilities in
-// the registers the scores came in.  A tile costs a wavefront HD / 16 x 3 + HD / 16 x 6 MFMAs of 32 cycles (64:
-// 1152) where the fp32 instruction took HD x 64 (4096), and about as many cycles of vector instructions, which run
-// beside them.  Call times with six MFMAs a step for the scores, too, and now (us): 2048 rows, 32 / 8 heads of 64,
-// 102.9 -> 89.0; 512 rows on 16384 cached, 32 / 4 heads of 128, 671 -> 561.
+// Queries, keys, values and probabilities enter the MFMAs as exact sums of three bf16 numbers
+// (split_mfma.hpp): the queries once, a key tile by the workgroup on its way to LDS, the probabilities in
+// the registers the scores came in.  A tile costs a wavefront HD / 16 x 6 + HD / 16 x 6 MFMAs of 32 cycles (64:
+// 1536) where the fp32 instruction took HD x 64 (4096), and about as many cycles of vector instructions, which run
+// beside them.  Kernel times, the fp32 instruction before (us): 2048 rows, 32 / 8 heads of 64, 99 (146), 8192 rows 1324
+// (2050); 512 rows on 16384 cached, 32 / 4 heads of 128, 684 (1056); 2048 rows, 32 / 8 heads of 128, 186 (279).
 // Bound by the power the card may draw, as the large products are; raising one group's priority changes nothing and
-// parking V between the score MFMAs costs 5 to 16 %.
+// parking V between the score MFMAs costs 5 to 16 %.  (Queries and keys as two fp16 numbers and scores of three products
+// took 14 and 17 % less, but such numbers leave out up to 2^-21 of a product, and where a key's second parts have the signs of the
+// query's that adds up.)
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS>
 __device__ __forceinline__ void prefill_block(const int bid, const float *__restrict__ q_rot,
                                               const float *__restrict__ kc, const float *__restrict__ vc,
@@ -209,10 +211,11 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   auto park_k = [&]() {
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
-      u32x4 h, l;
-      split_octet_f16(stage_k[u][0], stage_k[u][1], h, l);
+      u32x4 h, m, l;
+      split_octet(stage_k[u][0], stage_k[u][1], h, m, l);
       lds[k_unit[u]] = h;
-      lds[k_unit[u] + U::kPartK] = l;
+      lds[k_unit[u] + U::kPartK] = m;
+      lds[k_unit[u] + 2 * U::kPartK] = l;
     }
   };
   auto park_v = [&]() {
@@ -233,8 +236,8 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     load_k(0);
     load_v(0);
   }
-  // the row's query, scaled by scale * log2(e) * 2^6: scores come out 2^6 times as large as in log2 units
-  u32x4 qf[KS][2];
+  // the row's query, scaled by scale * log2(e): scores come out in log2 units
+  u32x4 qf[KS][3];
   bool apart;  // some query of the wavefront needs its scores in fp32
   {
     f32x4 t[KS][2];
@@ -248,28 +251,37 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
         if (!PAD || 16 * i + 8 * j + 4 * h < hd) t[i][h] = *(const f32x4 *)(qp + 16 * i + 4 * h);
       }
 #pragma unroll
-    for (int i = 0; i < KS; ++i) split_octet_f16(t[i][0] * (c * kQueryLift), t[i][1] * (c * kQueryLift), qf[i][0], qf[i][1]);
-    float most = 0.f;
+    for (int i = 0; i < KS; ++i) split_octet(t[i][0] * c, t[i][1] * c, qf[i][0], qf[i][1], qf[i][2]);
+    float least = INFINITY, most = 0.f;
 #pragma unroll
     for (int i = 0; i < KS; ++i)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         if (PAD && 16 * i + 8 * j + 4 * h >= hd) continue;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) most = fmaxf(most, fabsf(t[i][h][w] * c));
+        for (int w = 0; w < 4; ++w) {
+          const float size = fabsf(t[i][h][w] * c);
+          least = fminf(least, size);
+          most = fmaxf(most, size);
+        }
       }
-    apart = __any(!(most < kMostQuery));
+    apart = false;
+    // (looked at closely only where there is a zero or something out of the ordinary)
+    if (__builtin_expect(__any(!(least >= 0x1p-109f) || !(most < 0x1p100f)), 0)) {
+      QueryRange range;
+#pragma clang loop unroll(disable)
+      for (int d = 4 * j; d < hd; d += 8) range.add(*(const f32x4 *)(q_rot + q_off + d));
+      apart = __any(range.apart(c));
+    }
   }
 
   // Online softmax against a reference value per virtual row instead of the running maximum: m_ref is only moved
   // (and l, O rescaled) when a score exceeds it by more than kTau, or for a row's first visible key;
   // probabilities are then at most 2^kTau, no overflow.  A tile on the common path costs a maximum, 16
   // subtractions, exp2 and adds per lane.
-  // The scores are looked at as they come, 2^6 times too large (m_ref, and thr after the loop, are in log2 units); values by
-  // distance, which may be of any size, are added in log2 units.
-  constexpr float kTau = 8.f, kDrop = BIAS ? 1.f : kScoreDrop;
+  constexpr float kTau = 8.f;
   float m_ref = 0.f, l = 0.f;
-  float thr = -INFINITY;  // a row's scores move m_ref when above this: anything finite until its first key, kTau above m_ref after
+  float thr = -INFINITY;  // a row's scores move m_ref when above this: anything finite until its first key, m_ref + kTau after
   f32x16 o[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -299,28 +311,25 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
         for (int r = 0; r < 4; ++r) near_bias[r] = ((const Four *)(bias_row + kt * 32 + 8 * r + 4 * j))->v;
       }
     }
-    f32x16 p, low;
+    f32x16 p;
     if (have) {
       // S^T of the key tile: 32 keys x 32 virtual rows
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = low[r] = 0.f;
+      for (int r = 0; r < 16; ++r) p[r] = 0.f;
       const u32x4 *kl = tile + j * U::kOctK + n;
 #pragma unroll
       for (int i = 0; i < KS; ++i) {
-        const u32x4 kh = kl[2 * i * U::kOctK], kt_low = kl[U::kPartK + 2 * i * U::kOctK];
-        low = mfma_f16(kt_low, qf[i][0], low);
-        p = mfma_f16(kh, qf[i][0], p);
-        low = mfma_f16(kh, qf[i][1], low);
+        u32x4 kf[3];
+#pragma unroll
+        for (int w = 0; w < 3; ++w) kf[w] = kl[w * U::kPartK + 2 * i * U::kOctK];
+#pragma unroll
+        for (int w = 0; w < 6; ++w) p = mfma_bf16(kf[kPartA[w]], qf[i][kPartB[w]], p);
       }
     }
     park_v();
     if (sp + 1 < n_sp) load_v(sp + 1);
     if (have) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = fmaf(low[r], kLowDrop, p[r]);
       if constexpr (BIAS) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) p[r] *= kScoreDrop;
         if (near) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) p[r] += near_bias[r >> 2][r & 3];
@@ -344,9 +353,9 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
         // rare after a row's first tiles: move the reference to this tile's maximum
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         if (mx > thr) {
-          const float alpha = thr != -INFINITY ? fast_exp2(m_ref - mx * kDrop) : 1.f;  // nothing to rescale before a row's first key
-          m_ref = mx * kDrop;
-          thr = mx + kTau / kDrop;
+          const float alpha = thr != -INFINITY ? fast_exp2(m_ref - mx) : 1.f;  // nothing to rescale before a row's first key
+          m_ref = mx;
+          thr = mx + kTau;
           l *= alpha;
 #pragma unroll
           for (int t = 0; t < NT; ++t)
@@ -357,7 +366,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       float psum = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        p[r] = fast_exp2(fmaf(p[r], kDrop, -m_ref));
+        p[r] = fast_exp2(p[r] - m_ref);
         psum += p[r];
       }
       l += psum;
@@ -389,11 +398,12 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   // Some results are taken again, tile by tile in fp32:
   //   results that are not finite come from operands that are not, and fp32 says which (8192 rows, 32 / 8 heads of 64, NaN
   //   in key 5: 4.6 ms a call against 1.6 without; key by key, one dimension at a time, it was 279);
-  //   keys of 65520 and more, NaN in the scores, and queries of 2^9 and more in log2 units;
+  //   queries that ask for it (QueryRange);
   //   values below 2^-110: what they lose by the split, 2^-134 of a key's weight, shows in sums that are themselves small
   //   (the largest weight of a row is 1 or more, all together under 2^30).  Those may be sums of zeros, too: the
   //   values are looked at.  Lifted there by 2^24, or sums of subnormal numbers would round to 2^-149.
-  // (All values lifted on their way to LDS cost 8192 rows of 32 / 8 heads of 64 some 60 us of 1320.)
+  // All values lifted on their way to LDS, and every query looked at closely, cost 8192 rows 5 % (1323 -> 1383 us; this
+  // way 1320) and 2048 rows of 32 / 8 heads of 128 4 % (216 -> 224; 218).
   {
     auto size = [](float x) { return __builtin_bit_cast(unsigned, x) << 1; };  // (in the order of |x|)
     float probe = l * 0.f, least = INFINITY;

@@ -3,7 +3,7 @@
 // their own).  A bf16 has a float's exponents and 16 bits less behind them, so the rests of a float below 2^-110
 // would not be whole; operands are lifted by 2^24 first, which makes every part of every float, the smallest
 // subnormal's too, a normal bf16 or zero, and results are brought down again.  (Not the operands of scores, see
-// QueryRange and split_pair_f16, nor probabilities, whose row holds one near 1, nor the values of prefill attention, which looks at its
+// QueryRange, nor probabilities, whose row holds one near 1, nor the values of prefill attention, which looks at its
 // sums instead.)  That is 2 to 4 % of a prompt's products; rows of x around 2^-120 had an error of 3.5e-5 without, and
 // 2e-7 with it, as rows around 1 have.  Of the nine products of two such sums
 // the six largest make up the product to 2^-24 of itself: of the three left out two can reach 2^-25 each.  Six
@@ -33,7 +33,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // Operands of a product are lifted before they are split; its result, or that of one lifted operand, comes down.
 constexpr float kLift = 0x1p24f, kDrop = 0x1p-48f, kDropOne = 0x1p-24f;
 
-// Scores of attention (of latent heads; prefill attention's: split_pair_f16) are taken of queries and keys as they are: only their size against 1 counts, and what the
+// Scores of attention are taken of queries and keys as they are: only their size against 1 counts, and what the
 // small ones lose is 2^-134 of the other operand at most.  It can count where a query (scaled, in log2 units) holds
 // numbers of 2^100 and more, and keys numbers below 2^-110, or the query numbers below 2^-109 (other than 0), and keys
 // very large ones: the scores of such queries are taken in fp32.
@@ -104,41 +104,6 @@ constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
 // D[m = 8 (r / 4) + 4 (l / 32) + r % 4][n = l % 32] in register r.
 __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
-}
-
-// Scores of prefill attention: both operands as sums of two fp16 numbers, the second kept 2^11 times as large so that it
-// has the range of the first (22 to 23 bits of a float from 2^-14 up, below that whatever is 2^-36 or more), and three
-// products of the four, those with a second part in an accumulator of their own.  The kernels are bound by the matrix
-// cores, so half the products of the sums of three bf16 numbers show: 2048 rows of 32 / 8 heads of 64 102.9 -> 89.0 us,
-// 512 rows of 32 / 4 heads of 128 on 16384 keys 671 -> 561.  And the sums round half as often: the error of the results
-// against 64 bits goes from 2.6e-7 to 2.3e-7 and from 8.3e-7 to 7.9e-7.  Values and probabilities stay three bf16 numbers: a
-// column of values may be of any size.  A score is different, only its size against 1 counts:
-//   queries, in log2 units, are taken 2^6 times as large; where one is 2^9 or more its wavefront takes the fp32 instruction;
-//   a key of 65520 or more becomes an infinity in one part and the opposite one in the other, so its scores are NaN, which
-//   asks for fp32 too;
-//   a small key loses 2^-37 times a query below 2^9, 2^-28 of a score; a small query 2^-43 times a key below 2^16, 2^-27.
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-constexpr float kQueryLift = 0x1p6f, kScoreDrop = 0x1p-6f, kLowDrop = 0x1p-11f, kMostQuery = 0x1p9f;
-
-__device__ __forceinline__ void split_pair_f16(float a, float b, unsigned &high, unsigned &low) {
-  const f16x2 h = __builtin_convertvector((f32x2{a, b}), f16x2);
-  high = __builtin_bit_cast(unsigned, h);
-  a -= (float)h.x;
-  b -= (float)h.y;
-  low = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a * 0x1p11f, b * 0x1p11f}), f16x2));
-}
-__device__ __forceinline__ void split_octet_f16(f32x4 a, f32x4 b, u32x4 &high, u32x4 &low) {
-  unsigned h[4], l[4];
-  split_pair_f16(a.x, a.y, h[0], l[0]);
-  split_pair_f16(a.z, a.w, h[1], l[1]);
-  split_pair_f16(b.x, b.y, h[2], l[2]);
-  split_pair_f16(b.z, b.w, h[3], l[3]);
-  high = u32x4{h[0], h[1], h[2], h[3]};
-  low = u32x4{l[0], l[1], l[2], l[3]};
-}
-__device__ __forceinline__ f32x16 mfma_f16(u32x4 a, u32x4 b, f32x16 acc) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
 }
 
 // The same in fp32 over two k: lane l holds k = l / 32 of row (column) l % 32; the same D.

@@ -994,10 +994,10 @@ def test_prefill_of_very_small_operands(hip, hd, KV, T, cached, q_by, k_by, v_by
 @pytest.mark.parametrize("hd,KV,T,cached", [(64, 2, 300, 0), (128, 2, 70, 100), (96, 4, 40, 33), (64, 8, 1500, 0)])
 @pytest.mark.parametrize("pair", [-24, -13, -11, -9, 5, 13, 15, 17, 24])
 def test_prefill_scores_at_the_limits_of_two_fp16_parts(hip, hd, KV, T, cached, pair):
-    """Scores whose queries pass 2^9 in log2 units and whose keys pass 65520, and both well below fp16's normal numbers: one
-    rotated pair is 2^pair of the others in the keys, the other way round in the queries.  Half a key's or a query's last
-    bit of 22, the rounding of each sum over hd in fp32, and the product of the two second parts: at most 2^-20 of the sum of
-    the products' sizes in a score, twice that of the largest value in a result, and 2^-20 of it for the sums behind."""
+    """Scores whose queries pass 2^9 in log2 units and whose keys pass 65520, and both well below the normal numbers of 16 bits
+    with five of exponent: one rotated pair is 2^pair of the others in the keys, the other way round in the queries.  To the bf16
+    parts of a score this makes no difference: the roundings of sums over hd and the parts left out are at most 2^-20 of the
+    sum of the products' sizes in a score, twice that of the largest value in a result, and 2^-20 of it for the sums behind."""
     import torch
 
     H, S = 2 * KV, cached + T
@@ -1026,6 +1026,46 @@ def test_prefill_scores_at_the_limits_of_two_fp16_parts(hip, hd, KV, T, cached, 
         p = np.exp(s - s.max(-1, keepdims=True))
         want = (p / p.sum(-1, keepdims=True)) @ vr
         assert np.abs(got[:, h] - want).max() <= (2 * sizes.max() + 1) * 2.0 ** -20 * np.abs(vr).max(), h
+
+
+@pytest.mark.parametrize("hd,KV,T,cached", [(16, 2, 300, 0), (64, 2, 300, 0), (64, 8, 1500, 0), (96, 4, 40, 33), (128, 2, 70, 100)])
+def test_prefill_scores_keep_all_24_bits(hip, hd, KV, T, cached):
+    """Every query is 2^6 (1 + 2^-11 - 2^-14) in log2 units, the even keys hold 1 + 2^-11 - 2^-14 and 1 + 2^-11 + 2^-14 by turns,
+    with signs by turns, so that a score is 2^-14 of the sum of its products' sizes, 2^19, and what an operand cut to 11 and 11 bits
+    leaves out of each product, 0.8 x 2^-22 of it, adds up.  The odd keys have the same score from one product.  Three bf16 numbers
+    an operand leave out two products of 2^-25 at most; as much again for the sums and the factor of the queries.  Nothing
+    is rotated."""
+    import torch
+
+    H, S = 2 * KV, cached + T
+    c = float(np.float32(np.log2(np.e)) * np.float32(1 / np.sqrt(hd)))
+    size = 2.0 ** (13 - int(np.log2(hd)))
+    q = torch.full((T, H * hd), float(np.float32(2.0 ** 6 * (1 + 2.0 ** -11 - 2.0 ** -14) / c)), device="cuda")
+    keys = torch.zeros((S, hd), device="cuda")
+    keys[0::2, 0::2] = size * (1 + 2.0 ** -11 - 2.0 ** -14)
+    keys[0::2, 1::2] = -size * (1 + 2.0 ** -11 + 2.0 ** -14)
+    keys[1::2, 1] = -size * hd * 2.0 ** -14
+    values = torch.ones((S, hd), device="cuda")
+    values[1::2] = -1
+    ctx = hip.AttnContext(H, KV, hd, rope_freqs=np.zeros(hd // 2, np.float32), max_positions=S)
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, S)
+    if cached:
+        cache.fill(0, *(a[None, :cached].expand(KV, cached, hd).contiguous() for a in (keys, values)))
+    ctx.sync()
+    got = ctx.forward(cache, q, *(a[cached:].repeat(1, KV) for a in (keys, values)), [T])
+    ctx.sync()
+    got = got.cpu().numpy().reshape(T, H, hd).astype(np.float64)
+    assert np.array_equal(ctx.last_q_rot(T).reshape(T, -1), q.cpu().numpy())
+    kr, vr = (a.astype(np.float64) for a in cache.read(0, KV - 1, 0, S))
+    assert np.array_equal(kr, keys.cpu().numpy())
+    s = kr @ q[0, :hd].cpu().numpy().astype(np.float64) / np.sqrt(hd)  # every row's, every head's
+    sizes = float(np.abs(kr[0]).sum() * q[0, 0].item() / np.sqrt(hd))
+    row = np.where(np.arange(S)[None] > cached + np.arange(T)[:, None], -np.inf, s[None])
+    p = np.exp(row - row.max(-1, keepdims=True))
+    want = ((p / p.sum(-1, keepdims=True)) @ vr)[:, None]
+    # a result moves by half of what the difference of the two scores does
+    assert np.abs(got - want).max() <= 0.5 * 2.0 ** -23 * sizes + 1e-5
 
 
 @pytest.mark.parametrize("hd,KV,T,tiny", [(64, 2, 300, 2.0 ** -124), (128, 2, 300, 2.0 ** -135), (96, 4, 140, 2.0 ** -124), (64, 8, 2300, 0.0)])
