@@ -285,6 +285,11 @@ int shainet_hip_matmul_f32(const float *x, long long x_stride, const float *w, c
  * (1 = none); plan[5] 1 = workgroups share tiles and the one that ends a tile waits for the others' parts; plan[6] 1 = k
  * is no whole number of steps.  Lets a test name the kernel instantiation it covers.  No counterpart in the reference. */
 int shainet_hip_describe_matmul(int rows, int k, int n, int plan[7]);
+/* The same two where every value of W is a bf16 number, for which the caller answers: what a model's projections run as
+ * when its weights are.  (Five to sixteen rows take the MFMA kernel, as they do in a model.)  No counterpart in the reference. */
+int shainet_hip_matmul_bf16_weights_f32(const float *x, long long x_stride, const float *w, const float *res, float *y, int rows,
+                                        int k, int n, void *stream);
+int shainet_hip_describe_matmul_bf16_weights(int rows, int k, int n, int plan[7]);
 
 /* ---- the whole block ---------------------------------------------------------
  *

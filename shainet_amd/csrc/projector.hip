@@ -310,17 +310,16 @@ std::mutex g_matmul_lock;
 // error word their kernels report into), one set per stream: calls on different streams may overlap
 // on the device and must not share partial products.  Never freed, like the reference's class-level scratch.
 std::map<hipStream_t, shainet::Projector> g_matmul;
-}  // namespace
 
-extern "C" int shainet_hip_describe_matmul(int rows, int k, int n, int plan[7]) {
+int describe(int rows, int k, int n, bool w_bf16, int plan[7]) {
   using namespace shainet;
   if (!plan || rows < 1 || k < 1 || n < 1) return llama_fail(SHAINET_HIP_ERR_ARGUMENT, "invalid matmul arguments");
-  describe_gemm(plan_gemm(rows, k, n, k), k, plan);
+  describe_gemm(plan_gemm(rows, k, n, k, w_bf16), k, plan);
   return SHAINET_HIP_OK;
 }
 
-extern "C" int shainet_hip_matmul_f32(const float *x, long long x_stride, const float *w, const float *res, float *y,
-                                      int rows, int k, int n, void *stream) {
+int matmul(const float *x, long long x_stride, const float *w, const float *res, float *y, int rows, int k, int n, void *stream,
+           bool w_bf16) {
   using namespace shainet;
   if (!x || !w || !y || rows < 1 || k < 1 || n < 1 || x_stride < k)
     return llama_fail(SHAINET_HIP_ERR_ARGUMENT, "invalid matmul arguments");
@@ -332,10 +331,28 @@ extern "C" int shainet_hip_matmul_f32(const float *x, long long x_stride, const 
   // is said by the next call, which does nothing else then
   if (int rc = check_error_word(p.error)) return rc;
   Fused f;
-  f.any_few_rows = true;
+  f.any_few_rows = !w_bf16;
+  f.w_bf16 = w_bf16;
   if (res) {
     f.epilogue = kGemvResidual;
     f.res = res;
   }
   return p.project(x, x_stride, w, y, rows, k, n, (hipStream_t)stream, f);
+}
+}  // namespace
+
+extern "C" int shainet_hip_describe_matmul(int rows, int k, int n, int plan[7]) { return describe(rows, k, n, false, plan); }
+
+extern "C" int shainet_hip_describe_matmul_bf16_weights(int rows, int k, int n, int plan[7]) {
+  return describe(rows, k, n, true, plan);
+}
+
+extern "C" int shainet_hip_matmul_f32(const float *x, long long x_stride, const float *w, const float *res, float *y,
+                                      int rows, int k, int n, void *stream) {
+  return matmul(x, x_stride, w, res, y, rows, k, n, stream, false);
+}
+
+extern "C" int shainet_hip_matmul_bf16_weights_f32(const float *x, long long x_stride, const float *w, const float *res, float *y,
+                                                   int rows, int k, int n, void *stream) {
+  return matmul(x, x_stride, w, res, y, rows, k, n, stream, true);
 }

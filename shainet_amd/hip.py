@@ -148,6 +148,9 @@ _SIGNATURES = {
     "shainet_llama_model_topk": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_int), _f32p, C.POINTER(C.c_int)]),
     "shainet_llama_model_sample": (C.c_int, [C.c_void_p, C.c_int, C.c_double, C.c_double, C.POINTER(C.c_int)]),
     "shainet_hip_describe_matmul": (C.c_int, [C.c_int, C.c_int, C.c_int, _i32p]),
+    "shainet_hip_describe_matmul_bf16_weights": (C.c_int, [C.c_int, C.c_int, C.c_int, _i32p]),
+    "shainet_hip_matmul_bf16_weights_f32": (C.c_int, [C.c_void_p, C.c_longlong, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int,
+                                                      C.c_int, C.c_int, C.c_void_p]),
     "shainet_hip_matmul_f32": (C.c_int, [C.c_void_p, C.c_longlong, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int,
                                          C.c_int, C.c_void_p]),
     "shainet_hip_stream_copy_f32": (C.c_int, [C.c_void_p, C.c_void_p, C.c_longlong, C.c_int, C.c_void_p]),
@@ -292,17 +295,19 @@ def describe_plan(num_heads, num_kv_heads, head_dim, start_pos, new_tokens):
     return d
 
 
-def describe_matmul(rows, k, n):
+def describe_matmul(rows, k, n, bf16_weights=False):
     """What the MFMA product of [rows, k] and [k, n] runs as; nothing is launched and no device is needed."""
     plan = (C.c_int * 7)()
-    _check(lib().shainet_hip_describe_matmul(rows, k, n, plan))
+    f = lib().shainet_hip_describe_matmul_bf16_weights if bf16_weights else lib().shainet_hip_describe_matmul
+    _check(f(rows, k, n, plan))
     kind, tm, tn, workgroups, pieces, waits, ragged = (int(v) for v in plan)
     return {"kind": ("plain", "few", "tiles")[kind], "tile": (tm, tn), "workgroups": workgroups, "pieces": pieces,
             "waits": bool(waits), "ragged_k": bool(ragged)}
 
 
-def matmul(x, w, res=None, out=None, stream=None):
-    """y = x @ w (+ res) on torch CUDA float32 tensors: x [T, K] (rows may be strided), w [K, N]."""
+def matmul(x, w, res=None, out=None, stream=None, bf16_weights=False):
+    """y = x @ w (+ res) on torch CUDA float32 tensors: x [T, K] (rows may be strided), w [K, N].  bf16_weights: every value of
+    w is a bf16 number, and the product runs as it does in a model of such weights."""
     import torch
 
     assert x.is_cuda and w.is_cuda and x.dtype == w.dtype == torch.float32 and w.is_contiguous()
@@ -314,8 +319,8 @@ def matmul(x, w, res=None, out=None, stream=None):
     assert out.is_contiguous() and tuple(out.shape) == (T, N)
     if res is not None:
         assert res.is_contiguous() and tuple(res.shape) == (T, N)
-    _check(lib().shainet_hip_matmul_f32(x.data_ptr(), x.stride(0), w.data_ptr(), _ptr(res), out.data_ptr(), T, K, N,
-                                        stream))
+    f = lib().shainet_hip_matmul_bf16_weights_f32 if bf16_weights else lib().shainet_hip_matmul_f32
+    _check(f(x.data_ptr(), x.stride(0), w.data_ptr(), _ptr(res), out.data_ptr(), T, K, N, stream))
     return out
 
 

@@ -69,6 +69,38 @@ MATMULS = [
     (1000, 4100, 4092, ("tiles", (256, 256), True, False, True)),
 ]
 
+# The same of weights that are bf16 numbers: "few" are tiles of 32 to 96 rows whose weights go straight to registers.
+BF16_MATMULS = [
+    (20, 512, 8196, ("few", (32, 64), False, False, False)),
+    (5, 1044, 16380, ("few", (32, 64), False, False, True)),
+    (400, 512, 132, ("few", (32, 64), True, False, False)),
+    (17, 2052, 132, ("few", (32, 64), True, False, True)),
+    (75, 96, 132, ("few", (32, 128), False, False, False)),
+    (40, 100, 132, ("few", (32, 128), False, False, True)),
+    (5, 512, 132, ("few", (32, 128), True, False, False)),
+    (17, 1044, 132, ("few", (32, 128), True, False, True)),
+    (97, 96, 8200, ("few", (64, 128), False, False, False)),
+    (100, 100, 8196, ("few", (64, 128), False, False, True)),
+    (40, 2048, 2308, ("few", (64, 128), True, False, False)),
+    (100, 2052, 2308, ("few", (64, 128), True, False, True)),
+    (200, 96, 8200, ("few", (96, 128), False, False, False)),
+    (257, 100, 8196, ("few", (96, 128), False, False, True)),
+    (96, 2048, 3072, ("few", (96, 128), True, False, False)),
+    (75, 2052, 2308, ("few", (96, 128), True, False, True)),
+    (512, 2048, 16384, ("tiles", (128, 256), False, False, False)),
+    (1300, 36, 16380, ("tiles", (128, 256), False, False, True)),
+    (400, 640, 8200, ("tiles", (128, 256), False, True, False)),
+    (200, 1044, 16384, ("tiles", (128, 256), False, True, True)),
+    (1000, 1040, 1028, ("tiles", (128, 256), True, False, False)),
+    (300, 1044, 4092, ("tiles", (128, 256), True, False, True)),
+    (2000, 640, 8188, ("tiles", (256, 256), False, False, False)),
+    (777, 1044, 16384, ("tiles", (256, 256), False, False, True)),
+    (3000, 512, 8200, ("tiles", (256, 256), False, True, False)),
+    (2000, 2052, 4092, ("tiles", (256, 256), False, True, True)),
+    (2000, 2048, 2308, ("tiles", (256, 256), True, False, False)),
+    (2000, 4100, 1028, ("tiles", (256, 256), True, False, True)),
+]
+
 
 def matmul_instantiation(plan):
     """The kernel instantiation of a dict from shainet_amd.hip.describe_matmul."""

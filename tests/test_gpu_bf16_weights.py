@@ -8,6 +8,7 @@ import pytest
 
 import tutilorn_model as tm
 import zabutar_model as zm
+import zabutar_oracle as zo
 from test_safetensors_host import write_safetensors
 
 pytestmark = pytest.mark.gpu
@@ -115,3 +116,27 @@ def test_other_designs_run_like_their_fp32_copies(hip, tmp_path, T, long):
                 w[n] = w[n] * (1 + r.uniform(0, 2.0 ** -8, np.shape(w[n]))).astype(np.float32)
         assert_alike(all_logits(hip, write(tmp_path / (name + "short"), cfg, w, lambda n: not (long and n.endswith("." + long))), tokens),
                      all_logits(hip, write(tmp_path / (name + "long"), cfg, w, lambda n: False), tokens))
+
+
+@pytest.mark.parametrize("short", [True, False])
+@pytest.mark.parametrize("width,ff,T", [(64, 96, 150), (60, 52, 150), (55, 47, 150), (1040, 512, 330), (1024, 516, 330), (1056, 509, 330)])
+def test_experts_products_keep_every_part(hip, tmp_path, width, ff, T, short):
+    """Tiles of 64 and 128 rows; lengths of K that are whole steps, pieces of four, and neither, by turns of the two products.  A
+    third part of the rows left out of a product is 3.3e-6 of what an expert returns, a part of the weights more; sums of up
+    to 1056 terms, the norms and the activation are off by a tenth of that."""
+    cfg = zm.config([zm.layer(zm.hgrn2(heads=1, dim=4, vdim=4), zm.moe(ff=ff, experts=2, identity=0, top=1, groups=1, keep=1, shared=0))],
+                    width=width)
+    w = zm.make_weights(cfg, 3)
+    w["l0.mix.o"] = 0 * w["l0.mix.o"]
+    if not short:
+        r = np.random.default_rng(7)
+        for n in w:
+            if ".e0." in n or ".e1." in n:
+                w[n] = w[n] * (1 + r.uniform(0, 2.0 ** -8, np.shape(w[n]))).astype(np.float32)
+    x = (2 * np.random.default_rng(4).standard_normal((T, width))).astype(np.float32)
+    model = hip.HFLoader.load_model(write(tmp_path / "m", cfg, w, lambda n: short or ".mlp.e" not in n))
+    got = model.blocks[0].forward_cached(x).astype(np.float64) - x
+    with zm.watch_choices() as gaps:
+        want = zo.layer(cfg, w, 0, x.astype(np.float64), {}) - x
+    assert min(gaps) > 3e-6, "a choice of experts too close to call: another seed"
+    assert np.linalg.norm(got - want) <= 1.2e-6 * np.linalg.norm(want), np.linalg.norm(got - want) / np.linalg.norm(want)

@@ -837,6 +837,42 @@ def test_matmul_keeps_every_part(hip, T, K, N, inst):
     assert bool((off <= 2.0 ** -22 * want.abs()).all()), float((off / want.abs()).nan_to_num().max())
 
 
+@pytest.mark.parametrize("T,K,N,inst", pc.BF16_MATMULS)
+def test_matmul_of_bf16_weights_keeps_every_part(hip, T, K, N, inst):
+    """Every instantiation for weights that are bf16 numbers.  Rows of x with a single value each: a sum is the three products
+    of its parts, exact each, the smallest up to 2^-17 of the whole, and adding them rounds by 2^-24 at most each.  Then sums
+    of all terms: a third part left out is 3.3e-6 of a row's norm, the roundings of 4100 terms in one accumulator under
+    1e-6.  Then what is not finite, where it belongs: fp32 sums beside it round every two terms and where pieces meet."""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    assert pc.matmul_instantiation(binding.describe_matmul(T, K, N, bf16_weights=True)) == inst
+    g = torch.Generator(device="cuda").manual_seed(T + K + N)
+    at = torch.randint(0, K, (T,), generator=g, device="cuda")
+    at[:2] = torch.tensor([0, K - 1])
+    value = torch.randn((T,), generator=g, device="cuda")
+    x = torch.zeros((T, K), device="cuda")
+    x[torch.arange(T, device="cuda"), at] = value
+    w = torch.randn((K, N), generator=g, device="cuda").bfloat16().float()
+    want = w[at].double() * value.double()[:, None]
+    off = (binding.matmul(x, w, bf16_weights=True).double() - want).abs()
+    assert bool((off <= 2.0 ** -22 * want.abs()).all()), float((off / want.abs()).nan_to_num().max())
+
+    x, res = torch.randn((T, K), generator=g, device="cuda"), torch.randn((T, N), generator=g, device="cuda")
+    got = binding.matmul(x, w, res, bf16_weights=True)
+    want = x.double() @ w.double() + res.double()
+    off = ((got.double() - want).norm(dim=1) / want.norm(dim=1)).max()
+    assert float(off) <= 2e-6, float(off)
+    assert torch.equal(got, binding.matmul(x, w, res, bf16_weights=True))
+    size = x.double().abs() @ w.double().abs() + res.double().abs()
+    x[T - 1, K - 1], w[0, N - 1] = float("nan"), float("inf")
+    got, want = binding.matmul(x, w, res, bf16_weights=True), x.double() @ w.double() + res.double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    fine = want.isfinite()
+    assert bool(((got.double() - want).abs() <= 2.0 ** -24 * (K / 2 + 18) * size)[fine].all())
+
+
 @pytest.mark.parametrize("T", [40, 250, 300, 1100])
 def test_matmul_split_tiles_keep_what_is_not_finite(hip, T):
     """Infinities, NaN and values that a bf16 would round to infinity come out as fp32 arithmetic has them."""

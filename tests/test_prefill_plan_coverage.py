@@ -97,14 +97,15 @@ def test_decode_spans_end_with_the_pairs():
 
 def test_products_run_as_their_cases_say():
     plan = sa.hip.describe_matmul
-    for T, K, N, inst in pc.MATMULS:
-        assert pc.matmul_instantiation(plan(T, K, N)) == inst, (T, K, N, plan(T, K, N))
-    seen = set()
-    for T, K, N in itertools.product((17, 40, 96, 97, 128, 200, 256, 257, 512, 777, 1024, 1300, 2048, 2304, 3000, 4096),
-                                     (4, 32, 100, 512, 1024, 2048, 2052, 4100, 8192), (4, 132, 1024, 2308, 3072, 8192, 16384)):
-        seen.add(pc.matmul_instantiation(plan(T, K, N)))
-    assert seen <= {inst for *_, inst in pc.MATMULS}, sorted(seen - {inst for *_, inst in pc.MATMULS})
-    assert plan(100, 6, 8)["kind"] == plan(100, 8, 6)["kind"] == "plain"
+    for cases, bf16 in ((pc.MATMULS, False), (pc.BF16_MATMULS, True)):
+        for T, K, N, inst in cases:
+            assert pc.matmul_instantiation(plan(T, K, N, bf16)) == inst, (T, K, N, plan(T, K, N, bf16))
+        seen = set()
+        for T, K, N in itertools.product((5, 17, 40, 96, 97, 128, 200, 256, 257, 512, 777, 1024, 1300, 2048, 2304, 3000, 4096),
+                                         (4, 32, 100, 512, 1024, 2048, 2052, 4100, 8192), (4, 132, 1024, 2308, 3072, 8192, 16384)):
+            seen.add(pc.matmul_instantiation(plan(T, K, N, bf16)))
+        assert seen <= {inst for *_, inst in cases}, sorted(seen - {inst for *_, inst in cases})
+        assert plan(100, 6, 8, bf16)["kind"] == plan(100, 8, 6, bf16)["kind"] == "plain"
 
 
 def test_large_tiles_fill_their_last_round():
