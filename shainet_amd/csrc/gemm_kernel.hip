@@ -655,7 +655,9 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 // The same by weights of one part, which leaves registers for more rows: a workgroup of eight wavefronts owns 32 MB
 // rows and 256 / KG columns, 32 of them a wavefront, and walks K in steps of 16 KG, of which each of KG groups of wavefronts
 // takes its own 16.  W goes from memory to registers four steps ahead (64 KB in flight on a compute unit), x through LDS.
-// Sums as in the kernel above, emptied every eight steps, three products instead of six.
+// Sums as in the kernel above, emptied every four steps, three products instead of six: no larger an error than
+// that kernel's anywhere (1e-8, 17 rows: 1024 -> 1024 7.5 | 8.0, 2048 -> 16384 8.4 | 10.2, 8192 -> 2048 10.3 | 12.1; emptied every eight
+// steps 96 rows of 768 -> 2304 7.9 | 7.6).
 // Against tiles of 32 x 128 that read W once per 32 rows and add 32-row pieces (us, with the kernel that adds the pieces): 45 rows
 // of 2048 -> 16384 40 -> 35, 2048 -> 2048 15.0 -> 12.7, 8192 -> 2048 31 -> 29, 1024 -> 1024 11.6 -> 9.1; 96 rows 59 -> 44,
 // 15.1 -> 14.9, 34 -> 34, 11.7 -> 9.7; and against 128 x 256 in 8 pieces 512 rows of 1024 -> 1024 21 -> 13.  W of 134 MB
@@ -753,13 +755,11 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
     for (int a = 0; a < MB; ++a) acc[a] = mfma_bf16(af[0][a], bf, acc[a]);
     __syncthreads();
   };
-  for (int k0 = 0; k0 < nk; k0 += 8) {
-    for (int kt = k0; kt < min(k0 + 8, nk); kt += 4) {
-      step(0);
-      step(1);
-      step(2);
-      step(3);
-    }
+  for (int k0 = 0; k0 < nk; k0 += 4) {
+    step(0);
+    step(1);
+    step(2);
+    step(3);
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
@@ -815,8 +815,9 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       f32x4 v = f32x4{acc[a][4 * r], acc[a][4 * r + 1], acc[a][4 * r + 2], acc[a][4 * r + 3]};
-#pragma unroll
-      for (int i = 0; i < KG - 1; ++i) v += merge[i * WN * kSums + 64 * (4 * a + r)];
+      const f32x4 *const other = merge + 64 * (4 * a + r);
+      v += other[0];  // (in pairs: four groups' sums one after the other round a little more)
+      if constexpr (KG == 4) v += other[WN * kSums] + other[2 * WN * kSums];
       if (g.pieces)  // [four rows][thread], as the kernel that adds the pieces takes them
         *(f32x4 *)(g.partials + (long long)blockIdx.x * (TM * TN) + (4 * a + r) * (256 * WN) + 4 * threadIdx.x) = v;
       else if (col < N)
@@ -890,14 +891,16 @@ int stream_quota(int tiles, int steps) {
 
 // W of one part: the tile of sgemm_stream_kernel by an estimate of its time, and whether that kernel is the one to take.
 // Rounds of workgroups times steps times what a step takes, and for pieces 1.4 us and 0.27 us per MB of them written and
-// read: fitted to 60 products of 5 to 777 rows, 5 % off on average.  It is left from 97 rows on where its loop alone takes
-// 20 us: there the larger tiles, which read W less often, are level or ahead (us, this | 128 x 256): 256 rows of
+// read: fitted to 60 products of 5 to 777 rows, 5 % off on average.  Where its loop alone takes more than 20 us,
+// the larger tiles, which read W less often, are level or ahead (us, this | 128 x 256): 256 rows of
 // 2048 -> 2048 19.2 | 23.3, 2048 -> 3072 26.9 | 25.5, 8192 -> 2048 52 | 43, 2048 -> 16384 96 | 64; 512 rows of 1024 -> 1024
 // 13.0 | 20.8, 1024 -> 3072 24.3 | 25.0, 2048 -> 2048 28.1 | 28.3, 2048 -> 3072 42 | 33; 777 rows of 1024 -> 1024 19.0 | 24.2,
 // 1024 -> 3072 34 | 32; 96 rows of 2048 -> 16384 43 | 52.
 bool choose_stream(GemmPlan &p, int T, int K, int N) {
   const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.453f}, {1, 4, 0.534f}, {2, 2, 0.587f}, {3, 2, 0.801f}};
-  float least = INFINITY, loop = 0.f;
+  float least = INFINITY, loop = INFINITY;
+  p.mb = 3;
+  p.kg = 2;
   for (const auto &s : shapes) {
     const long long tiles = (T + 32 * s.mb - 1) / (32 * s.mb) * (((long long)N * s.kg + 255) / 256);
     if (tiles > 1 << 20) continue;  // (many rounds: not this kernel's anyway)
@@ -911,7 +914,7 @@ bool choose_stream(GemmPlan &p, int T, int K, int N) {
     p.mb = s.mb;
     p.kg = s.kg;
   }
-  return least < INFINITY && (T <= 96 || loop <= 20.f);
+  return loop <= 20.f;
 }
 
 // The tile, by what was measured (us, 2048 -> 3072 | 2048 -> 2048 | 2048 -> 16384 | 8192 -> 2048 | 1024 -> 8192):
@@ -929,7 +932,11 @@ bool choose_stream(GemmPlan &p, int T, int K, int N) {
 //    512   35 32 41 | 30 28 38 | 120 99 112 | 77 60 69 | 43 41 49
 //    777   49 45 53 | 40 35 45 | 219 184 172 | 115 95 103 | 67 61 71
 //   2048   97 85 90 | 69 61 68 | 471 391 349 | 240 197 193 | 123 106 96
-// so 128 x 128 is not among its tiles, and 256 x 256 cut into pieces pads less than 8 %.
+// so 128 x 128 is not among its tiles.  Where weights of three parts take tiles of 32 rows, those of one take
+// sgemm_stream_kernel, and 256 x 256 is chosen by the same rule for both, because the sums of 128 x 256 are longer and
+// their error larger (1e-7 of the norm, the three-part product | 128 x 256 | now): 150 rows of 2048 -> 16384 1.02 | 3.42 |
+// 0.96 (62.5 and 60 us), 8192 -> 2048 1.09 | 2.53 | 0.98 (41, 40), 777 rows of 8192 -> 2048 3.49 | 4.94 | 3.49 (100, 107), 1400
+// rows 4.41 | 7.02 | 4.41 (173, 150), of 2048 -> 3072 2.79 | 3.16 | 2.79.
 // A low tile wastes least on few rows, and reads small weights again from the L2 for little: up to 96 rows always, up to
 // 256 where the higher tile would be a fifth padding or the weights are small.
 // The largest needs long runs: at least 36 steps a workgroup.  Less than a round of its tiles is cut into pieces for the
@@ -939,10 +946,9 @@ bool choose_stream(GemmPlan &p, int T, int K, int N) {
 // 640 824 | 759, 704 909 | 846; 4096 -> 8192: 320 802 | 896, 384 973 | 887; 8192 -> 8192: 288 1671 | 1873).
 void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 2;
-  p.kg = 2;
   const long long weights = (long long)K * N, rows1 = (T + 31) / 32 * 32LL, rows2 = (T + 127) / 128 * 128LL;
   p.few = T <= 96 || (T <= 256 && (weights <= (T <= 128 ? 12 : 5) << 20 || rows2 * 100 >= rows1 * 125));
-  if (p.parts == 1) p.few = choose_stream(p, T, K, N);
+  if (p.parts == 1) p.few = choose_stream(p, T, K, N) || p.few;
   p.few = p.few && (long long)kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows)
   if (p.few && p.parts == 1) return;
   p.mb = 1;
@@ -955,8 +961,7 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
   const long long tiles = rows4 / 256 * ((N + 255) / 256), run = tiles * p.steps / slots_of(4);
   const long long last = tiles % slots_of(4);
   const bool fills = tiles < slots_of(4) ? 2 * run < p.steps : last == 0 || 2 * last >= slots_of(4);
-  const int padding = p.parts == 1 && tiles < slots_of(4) ? 108 : 115;
-  if (rows4 * 100 <= rows2 * padding && run >= 36 && fills) p.mb = 4;
+  if (rows4 * 100 <= rows2 * 115 && run >= 36 && fills) p.mb = 4;
 }
 
 }  // namespace

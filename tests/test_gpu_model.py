@@ -873,6 +873,23 @@ def test_matmul_of_bf16_weights_keeps_every_part(hip, T, K, N, inst):
     assert bool(((got.double() - want).abs() <= 2.0 ** -24 * (K / 2 + 18) * size)[fine].all())
 
 
+@pytest.mark.parametrize("T,K,N", [(17, 1024, 1024), (17, 2048, 16384), (96, 768, 2304), (97, 8192, 2048), (150, 512, 2048), (150, 2048, 16384),
+                                   (150, 8192, 2048), (192, 4096, 4096), (200, 2048, 16384), (777, 8192, 2048), (777, 4096, 4096),
+                                   (1400, 2048, 3072), (1400, 8192, 2048)])
+def test_bf16_weights_are_no_less_exact(hip, T, K, N):
+    """Against 64 bits, the product that knows its weights to be bf16 numbers and the one that does not: the order of sums may
+    differ, what it costs may not grow.  (17408 sums and more: the two are compared to a hundredth.)"""
+    import torch
+
+    from shainet_amd import hip as binding
+
+    g = torch.Generator(device="cuda").manual_seed(T + K + N)
+    x, w = torch.randn((T, K), generator=g, device="cuda"), torch.randn((K, N), generator=g, device="cuda").bfloat16().float()
+    want = x.double() @ w.double()
+    off = [float((binding.matmul(x, w, bf16_weights=known).double() - want).norm() / want.norm()) for known in (False, True)]
+    assert off[1] <= 1.01 * off[0], off
+
+
 @pytest.mark.parametrize("T", [40, 250, 300, 1100])
 def test_matmul_split_tiles_keep_what_is_not_finite(hip, T):
     """Infinities, NaN and values that a bf16 would round to infinity come out as fp32 arithmetic has them."""
