@@ -67,12 +67,6 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ 
   }
 }
 
-__global__ __launch_bounds__(256) void low_bits_kernel(const float *__restrict__ w, size_t n, unsigned *word) {
-  unsigned found = 0;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) found |= __float_as_uint(w[i]) & 0xffffu;
-  if (__any(found != 0) && (threadIdx.x & 63) == 0) atomicOr(word, 1u);
-}
-
 __global__ __launch_bounds__(256) void add_kernel(const float *__restrict__ a, const float *__restrict__ b,
                                                   float *__restrict__ out, long long n) {
   const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
@@ -489,13 +483,6 @@ hipError_t launch_gather_rows(const float *x, const int *rows, float *out, int n
   // (a row gather is what the embedding lookup is)
   hipLaunchKernelGGL(embed_kernel, dim3((unsigned)n), dim3(256), 0, stream, x, rows, out, cols, 1.f,
                      (const float *)nullptr);
-  return hipGetLastError();
-}
-
-hipError_t launch_low_bits(const float *w, size_t n, unsigned *word, hipStream_t stream) {
-  if (!w || !n || !word) return hipErrorInvalidValue;
-  const size_t blocks = (n + 1023) / 1024;
-  hipLaunchKernelGGL(low_bits_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream, w, n, word);
   return hipGetLastError();
 }
 

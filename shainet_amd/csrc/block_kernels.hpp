@@ -67,7 +67,4 @@ hipError_t launch_topk(const float *logits, int vocab, int k, bool finite_only, 
 hipError_t launch_greedy_embed(const float *logits, int vocab, void *scratch, int *id, const float *table, float *out, int d_model,
                                float scale, const float *position, hipStream_t stream);
 
-// *word |= the lower 16 bits of the n floats at w
-hipError_t launch_low_bits(const float *w, size_t n, unsigned *word, hipStream_t stream);
-
 }  // namespace shainet

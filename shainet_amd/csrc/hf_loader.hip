@@ -86,13 +86,41 @@ int dtype_code(const std::string &d) {
   return -1;
 }
 
+// Whether all n elements are bf16 numbers, waited for.  The word the device answers in is kept from call to call; without
+// memory for one the answer is no, which is always right.
+struct Bf16Look {
+  unsigned *word = nullptr;
+  ~Bf16Look() {
+    if (word) (void)hipFree(word);
+  }
+  int operator()(const void *src, long long n, int dtype, bool *out) {
+    *out = dtype == kBF16;
+    if (*out) return SHAINET_HIP_OK;
+    unsigned found = 0;
+    if (!word && hipMalloc((void **)&word, sizeof found) != hipSuccess) {
+      (void)hipGetLastError();
+      word = nullptr;
+      return SHAINET_HIP_OK;
+    }
+    hipError_t e = hipMemset(word, 0, sizeof found);
+    if (e == hipSuccess) {
+      const long long blocks = (n + 1023) / 1024;
+      hipLaunchKernelGGL(low_bits_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, nullptr, src, n, dtype, word);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(&found, word, sizeof found, hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("looking at weights: ") + hipGetErrorString(e));
+    *out = !found;
+    return SHAINET_HIP_OK;
+  }
+};
+
 struct Stager {
   void *dev = nullptr;
-  unsigned *word = nullptr;
+  Bf16Look look;
   size_t cap = 0;
   ~Stager() {
     if (dev) (void)hipFree(dev);
-    if (word) (void)hipFree(word);
   }
   int put(const StTensor &t) {
     if ((size_t)t.nbytes > cap) {
@@ -130,28 +158,12 @@ int check_matrix(const StTensor &t, long long rows, long long cols, int &dtype) 
   return SHAINET_HIP_OK;
 }
 
-// Whether every value of a staged tensor is a bf16 number, whatever type it is stored in.
-int stored_bf16(Stager &stage, const StTensor &t, int dtype, bool *out) {
-  *out = dtype == kBF16;
-  if (*out) return SHAINET_HIP_OK;
-  const long long n = t.nbytes / dtype_size(t.dtype);
-  unsigned found = 0;
-  if (!stage.word && hipMalloc((void **)&stage.word, sizeof found) != hipSuccess) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-  if (hipMemset(stage.word, 0, sizeof found) != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, "hipMemset failed");
-  const long long blocks = (n + 1023) / 1024;
-  hipLaunchKernelGGL(low_bits_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, nullptr, stage.dev, n, dtype, stage.word);
-  if (hipGetLastError() != hipSuccess || hipMemcpy(&found, stage.word, sizeof found, hipMemcpyDeviceToHost) != hipSuccess)
-    return fail(SHAINET_HIP_ERR_RUNTIME, "looking at tensor '" + t.name + "' failed");
-  *out = !found;
-  return SHAINET_HIP_OK;
-}
-
 // *bf16 (nullable): taken up by a matrix's first tensor, kept up by the others: whether all their values are bf16 numbers
 int note_bf16(Stager &stage, const StTensor &t, int dtype, bool first, bool *bf16) {
   if (!bf16) return SHAINET_HIP_OK;
   bool here = false;
   if (first || *bf16)
-    if (int rc = stored_bf16(stage, t, dtype, &here)) return rc;
+    if (int rc = stage.look(stage.dev, t.nbytes / dtype_size(t.dtype), dtype, &here)) return rc;
   *bf16 = here;
   return SHAINET_HIP_OK;
 }
@@ -228,6 +240,11 @@ int read_text(const std::string &path, std::string &out) {
 }
 
 }  // namespace
+
+int shainet::values_are_bf16(const float *w, size_t n, bool *out) {
+  Bf16Look look;
+  return look(w, (long long)n, kF32, out);
+}
 
 extern "C" {
 

@@ -270,19 +270,6 @@ int upload_floats(float **dst, const float *src, size_t n) {
   return SHAINET_HIP_OK;
 }
 
-int values_are_bf16(const float *w, size_t n, bool *out) {
-  *out = false;
-  unsigned *word = nullptr, found = 0;
-  if (hipMalloc((void **)&word, sizeof *word) != hipSuccess) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-  hipError_t e = hipMemset(word, 0, sizeof *word);
-  if (e == hipSuccess) e = launch_low_bits(w, n, word, nullptr);
-  if (e == hipSuccess) e = hipMemcpy(&found, word, sizeof found, hipMemcpyDeviceToHost);
-  (void)hipFree(word);
-  if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("looking at weights: ") + hipGetErrorString(e));
-  *out = !found;
-  return SHAINET_HIP_OK;
-}
-
 int upload_side_by_side(float **dst, const float *const *mats, const int *widths, int count, int rows) {
   if (*dst) (void)hipFree(*dst);
   *dst = nullptr;
