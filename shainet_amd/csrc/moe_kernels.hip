@@ -347,64 +347,70 @@ __global__ __launch_bounds__(256) void moe_down_kernel(MoeShape m, MoeTensors w,
   if (lane == 0) y[(long long)t * m.d + j] = s + same * h[(long long)t * m.d + j];
 }
 
-// The same for at most eight slots and experts of at most 256 U values, a multiple of 4: all rows, the shared expert's first
+// The same for at most G slots and experts of at most 256 U values, a multiple of 4: all rows, the shared expert's first
 // 1024 values too, are requested before the first is looked at, where the kernel above goes to memory once per four slots and
 // once for the shared expert (a launch is a wavefront per SIMD, and so these round trips; the same sums in the same
-// order).  6 of 24 experts of 512 -> 1024 beside a shared one of 1024: 10.5 -> 6.5 us.
-template <int U>
+// order).  No load hangs on a condition: a slot without an expert's row has a buffer without records, whose loads come
+// back as zeros and go nowhere.  (With branches around them the compiler had U = 1 wait for one load after the other, in 424
+// registers: 18.6 us where it is 5.2 now.)  Two, four and eight slots, because such loads take their turn, too: 8 rows with 2
+// slots of 768 10 us, in eight slots 19.  U = 3 holds 224 registers of rows in eight slots; a fourth span would not leave two
+// wavefronts a SIMD, which several rows live on.
+// One row | 8 rows, the kernel above -> this (us; 24 experts; slots x values -> outputs, shared values):
+//   6 x 512 -> 1024, 1024  11.4 -> 5.3 | 30 -> 18.5      8 x 256 -> 1024, 512  9.2 -> 4.5 | 24 -> 12
+//   8 x 768 -> 2048, 2048  19.9 -> 13.8 | 109 -> 77      8 x 256 -> 2048, none 9.0 -> 5.2 | 42 -> 21
+//   8 x 512 -> 2048, 1024  14.7 -> 8.1 | 76 -> 43        4 x 768 -> 2048, none 10.1 -> 6.3 | 49 -> 31
+//   2 x 768 -> 1024, none  6.4 -> 3.8 | 15.5 -> 9.8      1 x 256 -> 1024, none 3.9 -> 3.4 | 7.6 -> 5.9
+template <int U, int G>
 __global__ __launch_bounds__(256) void moe_down_once_kernel(MoeShape m, MoeTensors w, const float *__restrict__ h,
                                                             const float *__restrict__ hidden, int width,
                                                             const int *__restrict__ ids, const float *__restrict__ weights,
                                                             float *__restrict__ y) {
-  constexpr int G = 8, S = 4;
+  constexpr int S = 4;
   const int j = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.y, lane = threadIdx.x & 63;
   if (j >= m.d) return;
   const float *hid = hidden + (long long)t * (m.top + 1) * width;
   const int n4 = m.ff >> 2, s4 = m.shared_ff >> 2;
-  const f32x4 *sa = (const f32x4 *)(w.shared_down + (long long)j * m.shared_ff), *sb = (const f32x4 *)(hid + (long long)m.top * width);
-  float wk[G], same = 0.f;
-  bool real[G];
-  int e[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    e[g] = g < m.top ? ids[t * m.top + g] : m.experts;
-    wk[g] = g < m.top ? weights[t * m.top + g] : 0.f;
-  }
+  // piece i of a row of n (nothing is read beyond the row)
+  auto row = [](const float *p, int n) { return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, n * 4, 0x00027000); };
+  auto piece = [](__amdgpu_buffer_rsrc_t r, int i) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 16 * i, 0, 0)); };
+  auto piece_once = [](__amdgpu_buffer_rsrc_t r, int i) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 16 * i, 0, 2)); };
+  const float *sa = w.shared_down + (long long)j * m.shared_ff, *sb = hid + (long long)m.top * width;
+  // (the slots' experts and weights in lanes: as scalars they came one after the other, too)
+  const int slot = t * m.top + min(lane, m.top - 1);
+  const int id = lane < m.top ? ids[slot] : m.experts;
+  const float weight = lane < m.top ? weights[slot] : 0.f;
   f32x4 x[G][U], v[G][U], sx[S], sv[S];
+  const auto shared_w = row(sa, min(m.shared_ff, 256 * S)), shared_h = row(sb, min(m.shared_ff, 256 * S));
 #pragma unroll
-  for (int k = 0; k < S; ++k)
-    if (64 * k < s4) {
-      const int i = min(64 * k + lane, s4 - 1);
-      sx[k] = __builtin_nontemporal_load(sa + i);
-      sv[k] = sb[i];
-    }
+  for (int k = 0; k < S; ++k) {
+    sx[k] = piece_once(shared_w, 64 * k + lane);
+    sv[k] = piece(shared_h, 64 * k + lane);
+  }
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    real[g] = e[g] < m.experts;
-    if (!real[g]) {
-      same += wk[g];
-      continue;
-    }
-    const f32x4 *a = (const f32x4 *)(w.down + ((long long)e[g] * m.d + j) * m.ff), *b = (const f32x4 *)(hid + (long long)g * width);
+    const int e = __builtin_amdgcn_readlane(id, g);
+    const bool real = e < m.experts;
+    const auto down = row(w.down + ((long long)(real ? e : 0) * m.d + j) * m.ff, real ? m.ff : 0), of = row(hid + (long long)g * width, real ? m.ff : 0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = min(64 * u + lane, n4 - 1);
-      x[g][u] = __builtin_nontemporal_load(a + i);
-      v[g][u] = b[i];
+      x[g][u] = piece_once(down, 64 * u + lane);
+      v[g][u] = piece(of, 64 * u + lane);
     }
   }
+  __builtin_amdgcn_sched_barrier(0);  // (no sum starts, and waits, in front of the last load)
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int k = 0; k < S; ++k)
-    if (64 * k + lane < s4) acc += sx[k] * sv[k];
-  for (int i = 64 * S + lane; i < s4; i += 64) acc += __builtin_nontemporal_load(sa + i) * sb[i];
+  for (int k = 0; k < S; ++k) acc += sx[k] * sv[k];
+  for (int i = 64 * S + lane; i < s4; i += 64) acc += __builtin_nontemporal_load((const f32x4 *)sa + i) * ((const f32x4 *)sb)[i];
+  float same = 0.f;
 #pragma unroll
-  for (int g = 0; g < G; ++g)
-    if (real[g]) {
+  for (int g = 0; g < G; ++g) {
+    const bool real = __builtin_amdgcn_readlane(id, g) < m.experts;
+    const float wk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), g));
+    same += real ? 0.f : wk;
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (64 * u + lane < n4) acc += wk[g] * (x[g][u] * v[g][u]);
-    }
+    for (int u = 0; u < U; ++u) acc += (real && 64 * u + lane < n4 ? wk : 0.f) * (x[g][u] * v[g][u]);
+  }
   const float s = wave_sum((acc.x + acc.y) + (acc.z + acc.w));
   if (lane == 0) y[(long long)t * m.d + j] = s + same * h[(long long)t * m.d + j];
 }
@@ -815,18 +821,28 @@ hipError_t launch_moe_few(const MoeShape &m, const MoeTensors &w, const float *h
                        ids, weights);
   }
   const int spans = (m.ff + 255) / 256;
-#define SHAINET_MOE_DOWN(U_) \
-  hipLaunchKernelGGL(moe_down_once_kernel<U_>, g3, dim3(256), 0, stream, m, w, h, hidden, width, ids, weights, y)
+#define SHAINET_MOE_DOWN(U_, G_) \
+  hipLaunchKernelGGL((moe_down_once_kernel<U_, G_>), g3, dim3(256), 0, stream, m, w, h, hidden, width, ids, weights, y)
+#define SHAINET_MOE_DOWN_SLOTS(U_) \
+  do {                             \
+    if (m.top <= 2)                \
+      SHAINET_MOE_DOWN(U_, 2);     \
+    else if (m.top <= 4)           \
+      SHAINET_MOE_DOWN(U_, 4);     \
+    else                           \
+      SHAINET_MOE_DOWN(U_, 8);     \
+  } while (0)
   if (vec_ff && m.top <= 8 && spans == 1)
-    SHAINET_MOE_DOWN(1);
+    SHAINET_MOE_DOWN_SLOTS(1);
   else if (vec_ff && m.top <= 8 && spans == 2)
-    SHAINET_MOE_DOWN(2);
+    SHAINET_MOE_DOWN_SLOTS(2);
   else if (vec_ff && m.top <= 8 && spans == 3)
-    SHAINET_MOE_DOWN(3);
+    SHAINET_MOE_DOWN_SLOTS(3);
   else if (vec_ff)
     hipLaunchKernelGGL(moe_down_kernel<true>, g3, dim3(256), 0, stream, m, w, h, hidden, width, ids, weights, y);
   else
     hipLaunchKernelGGL(moe_down_kernel<false>, g3, dim3(256), 0, stream, m, w, h, hidden, width, ids, weights, y);
+#undef SHAINET_MOE_DOWN_SLOTS
 #undef SHAINET_MOE_DOWN
   return hipGetLastError();
 }
