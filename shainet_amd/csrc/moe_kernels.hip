@@ -552,40 +552,36 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
   for (int u = 0; u < NW; ++u) b_off[u] = (unsigned)((bp[u] - w + k4) * 4);
   f32x4 sa[2][NA], sb[2][NW];
   auto piece = [&](const float *p, int k) {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (LOADS != kScalar) {
-      if (k < K) v = *(const f32x4 *)(p + k);
-    } else {
-      if (k < K) v.x = p[k];
-      if (k + 1 < K) v.y = p[k + 1];
-      if (k + 2 < K) v.z = p[k + 2];
-      if (k + 3 < K) v.w = p[k + 3];
-    }
-    return v;
+    if constexpr (LOADS == kScalar) return f32x4{p[min(k, K - 1)], p[min(k + 1, K - 1)], p[min(k + 2, K - 1)], p[min(k + 3, K - 1)]};
+    return *(const f32x4 *)(p + min(k, K - 4));
+  };
+  // what lies behind the end of K counts as zeros
+  auto inside = [&](f32x4 v, int k) {
+    if constexpr (LOADS == kScalar) return f32x4{k < K ? v.x : 0.f, k + 1 < K ? v.y : 0.f, k + 2 < K ? v.z : 0.f, k + 3 < K ? v.w : 0.f};
+    return LOADS == kPieces && k >= K ? f32x4{0.f, 0.f, 0.f, 0.f} : v;
   };
   // (steps behind the last one repeat it, which nobody reads.  No load hangs on a condition: the branches around them had
-  // the loop wait for every load it had just issued)
+  // the loop wait for every load it had just issued: 75 rows of 1023 -> 511 by weights of three parts 92 -> 75 us)
   const int last = (K - 1) / TK * TK;
   auto load = [&](int set, int k0) {
     k0 = min(k0, last);
-    const int k = k0 + k4, at = min(k, K - 4);
+    const int k = k0 + k4;
 #pragma unroll
     for (int u = 0; u < NA; ++u)
-      sa[set][u] = LOADS == kSteps ? load_at((const f32x4 *)(g.x + k0), a_off[u]) : LOADS == kScalar ? piece(ap[u], k) : *(const f32x4 *)(ap[u] + at);
+      sa[set][u] = LOADS == kSteps ? load_at((const f32x4 *)(g.x + k0), a_off[u]) : piece(ap[u], k);
 #pragma unroll
     for (int u = 0; u < NW; ++u)
-      sb[set][u] = LOADS == kSteps ? load_at((const f32x4 *)(w + k0), b_off[u]) : LOADS == kScalar ? piece(bp[u], k) : *(const f32x4 *)(bp[u] + at);
+      sb[set][u] = LOADS == kSteps ? load_at((const f32x4 *)(w + k0), b_off[u]) : piece(bp[u], k);
   };
-  auto park = [&](int set, int k0, u32x4 *stage) {  // (pieces of k0's step behind the end of K count as zeros)
-    const bool out = LOADS == kPieces && k0 + k4 >= K;
+  auto park = [&](int set, int k0, u32x4 *stage) {  // k0: the step's
     u32x2 *at = (u32x2 *)(stage + (k4 >> 3) * kOctX + srow) + (k4 >> 2 & 1);
 #pragma unroll
     for (int u = 0; u < NA; ++u)
-      split_quad((out ? f32x4{0.f, 0.f, 0.f, 0.f} : sa[set][u]) * kLift, at[2 * kRows * u], at[2 * (kRows * u + kPartX)], at[2 * (kRows * u + 2 * kPartX)]);
+      split_quad(inside(sa[set][u], k0 + k4) * kLift, at[2 * kRows * u], at[2 * (kRows * u + kPartX)], at[2 * (kRows * u + 2 * kPartX)]);
     at = (u32x2 *)(stage + 3 * kPartX + (k4 >> 3) * kOctW + srow) + (k4 >> 2 & 1);
 #pragma unroll
     for (int u = 0; u < NW; ++u) {
-      const f32x4 v = (out ? f32x4{0.f, 0.f, 0.f, 0.f} : sb[set][u]) * kLift;
+      const f32x4 v = inside(sb[set][u], k0 + k4) * kLift;
       if constexpr (PARTS == 3)
         split_quad(v, at[2 * kRows * u], at[2 * (kRows * u + kPartW)], at[2 * (kRows * u + 2 * kPartW)]);
       else
@@ -667,10 +663,11 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
 #pragma clang loop unroll(disable)
     for (int k0 = 0; k0 < K; k0 += 8) {  // four of eight k a lane half's
       f32x4 xv[MB], wv[2];
+      const int k = k0 + 4 * half;
 #pragma unroll
-      for (int a = 0; a < MB; ++a) xv[a] = piece(xr[a], k0 + 4 * half);
+      for (int a = 0; a < MB; ++a) xv[a] = inside(piece(xr[a], k), k);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) wv[b] = piece(wr[b], k0 + 4 * half);
+      for (int b = 0; b < 2; ++b) wv[b] = inside(piece(wr[b], k), k);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
