@@ -102,11 +102,15 @@ __device__ __forceinline__ void store_pair(const GemmArgs &g, int row, int col, 
 }
 
 // Four registers of a lane's sums, number r of its 4 MB NB: with one block its column in four rows, with two blocks beside
-// each other its two columns in two rows, with four its four columns in one row.
+// each other its two columns in two rows, with four its four columns in one row.  row_of: the first of these rows.
+template <int NB>
+__device__ __forceinline__ int row_of(int r) {
+  return NB == 1 ? 32 * (r >> 2) + 8 * (r & 3) : NB == 2 ? 32 * (r >> 3) + 8 * ((r & 7) >> 1) + 2 * (r & 1) : 32 * (r >> 4) + 8 * ((r & 15) >> 2) + (r & 3);
+}
 template <int NB>
 __device__ __forceinline__ void store_four(const GemmArgs &g, int row0, int col, int r, f32x4 v) {
+  const int row = row0 + row_of<NB>(r);
   if constexpr (NB == 1) {
-    const int row = row0 + 32 * (r >> 2) + 8 * (r & 3);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (row + i >= g.T) return;
@@ -116,11 +120,9 @@ __device__ __forceinline__ void store_four(const GemmArgs &g, int row0, int col,
       g.y[o] = g.res ? g.res[o] + y : y;
     }
   } else if constexpr (NB == 2) {
-    const int row = row0 + 32 * (r >> 3) + 8 * ((r & 7) >> 1) + 2 * (r & 1);
     store_pair(g, row, col, f32x2{v.x, v.y});
     store_pair(g, row + 1, col, f32x2{v.z, v.w});
   } else {
-    const int row = row0 + 32 * (r >> 4) + 8 * ((r & 15) >> 2) + (r & 3);
     if (row >= g.T) return;
     const long long o = (long long)row * g.N + col;
     if (g.bias) {
@@ -186,9 +188,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     const int nk = s_end - s_begin;
 
     // (what follows from the thread's number is worked out per tile, or the compiler keeps it in scratch memory over the
-    // tile's end and the loads of the first step wait for it)
+    // tile's end and the loads of the first step wait for it.  128 x 128 has the registers, and without them puts all of a step's
+    // splits in front of its MFMAs: 200 rows of 8192 -> 1024, a workgroup a compute unit, 30 -> 35 us)
     int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
+    if constexpr (PARTS == 1 || WN == 4) asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const int ln = lane & 31, j = lane >> 5;
 
@@ -825,10 +828,24 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
     }
 }
 
-// y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order, eight of them in flight (one after the other 16
-// pieces of 45 rows took 3 us more).  A piece lies in its
-// workgroup's slot as [pair of rows, or row][thread] float4, the layout of the product kernel's accumulators.
-// A tile's threads are WM x WN wavefronts of MB x NB blocks.
+// acc + piece 0 + piece 1 + ..., all C in flight
+template <int C>
+__device__ __forceinline__ f32x4 add_pieces(f32x4 acc, const float *piece, long long step) {
+  f32x4 v[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) v[c] = *(const f32x4 *)(piece + c * step);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < C; ++c) acc += v[c];
+  return acc;
+}
+
+// y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order, four of them in flight: 16 pieces of 17 rows of 132
+// columns 5.4 us one after the other, 4.1 two at a time, 3.6 so, 3.1 eight at a time; launches that fill the chip take the
+// same time each way.  Only what is needed is requested, or those take 10 to 30 % longer: pieces that are not there, and
+// rows that pad a tile (777 rows of 8192 -> 4092, four pieces of tiles of 256 x 256: 11.4 us, with them 14.4).
+// A piece lies in its workgroup's slot as [pair of rows, or row][thread] float4, the layout of the product kernel's
+// accumulators.  A tile's threads are WM x WN wavefronts of MB x NB blocks.
 template <int WM, int WN, int MB, int NB>
 __global__ __launch_bounds__(64 * WM * WN) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
   constexpr int kOut = 4 * MB * NB, TM = 32 * WM * MB, TN = 32 * WN * NB;
@@ -842,16 +859,16 @@ __global__ __launch_bounds__(64 * WM * WN) void sgemm_reduce_kernel(const GemmAr
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row0 = (tile % g.tiles_m) * TM + (wave / WN) * 32 * MB + 4 * (lane >> 5);
   const int col = (tile / g.tiles_m) * TN + (wave % WN) * 32 * NB + NB * (lane & 31);
-  if (col >= g.N) return;
-  f32x4 acc = *(const f32x4 *)piece;
-  for (int c0 = 1; c0 < n; c0 += 8) {  // eight loads in flight
-    f32x4 v[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = *(const f32x4 *)(piece + min(c0 + c, n - 1) * piece_step);
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      if (c0 + c < n) acc += v[c];
-  }
+  if (row0 + row_of<NB>(r) >= g.T || col >= g.N) return;  // (nothing is read for rows that pad a tile)
+  f32x4 acc = {-0.f, -0.f, -0.f, -0.f};  // (which adds nothing to anything)
+  int left = n;
+  for (; left >= 4; left -= 4, piece += 4 * piece_step) acc = add_pieces<4>(acc, piece, piece_step);
+  if (left == 3)
+    acc = add_pieces<3>(acc, piece, piece_step);
+  else if (left == 2)
+    acc = add_pieces<2>(acc, piece, piece_step);
+  else if (left == 1)
+    acc = add_pieces<1>(acc, piece, piece_step);
   store_four<NB>(g, row0, col, r, acc);
 }
 
