@@ -188,9 +188,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     const int nk = s_end - s_begin;
 
     // (what follows from the thread's number is worked out per tile, or the compiler keeps it in scratch memory over the
-    // tile's end and the loads of the first step wait for it)
+    // tile's end and the loads of the first step wait for it.  128 x 128 has the registers, and without them puts all of a step's
+    // splits in front of its MFMAs: 200 rows of 8192 -> 1024, a workgroup a compute unit, 30 -> 35 us)
     int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
+    if constexpr (PARTS == 1 || WN == 4) asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const int ln = lane & 31, j = lane >> 5;
 
