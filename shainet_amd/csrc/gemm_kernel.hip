@@ -908,14 +908,18 @@ int stream_quota(int tiles, int steps) {
 
 // W of one part: the tile of sgemm_stream_kernel by an estimate of its time, and whether that kernel is the one to take.
 // Rounds of workgroups times steps times what a step takes, and for pieces 1.4 us and 0.27 us per MB of them written and
-// read: fitted to 60 products of 5 to 777 rows, 5 % off on average.  Where its loop alone takes more than 20 us,
-// the larger tiles, which read W less often, are level or ahead (us, this | 128 x 256): 256 rows of
+// read: fitted to 60 products of 5 to 777 rows, 5 % off on average.  Where its loop alone takes more than 20 us or one
+// round of workgroups does not do, the larger tiles, which read W less often, are level or ahead, and so they are of a loop of
+// four steps in tiles of 96 rows (over 408 products of 97 to 4000 rows, K 32 to 2048, N 256 to 32000, this rule loses 0.5 % to
+// the better of the two, without the second and third 12 %; us, this | 128 x 256): 256 rows of
 // 2048 -> 2048 19.2 | 23.3, 2048 -> 3072 26.9 | 25.5, 8192 -> 2048 52 | 43, 2048 -> 16384 96 | 64; 512 rows of 1024 -> 1024
 // 13.0 | 20.8, 1024 -> 3072 24.3 | 25.0, 2048 -> 2048 28.1 | 28.3, 2048 -> 3072 42 | 33; 777 rows of 1024 -> 1024 19.0 | 24.2,
-// 1024 -> 3072 34 | 32; 96 rows of 2048 -> 16384 43 | 52.
-bool choose_stream(GemmPlan &p, int T, int K, int N) {
+// 1024 -> 3072 34 | 32; 96 rows of 2048 -> 16384 43 | 52; rounds: 512 rows of 128 -> 16384 30 | 15, 2048 rows of 128 -> 4096 31 | 17.
+// short_rounds: its loop is of four steps, and in several rounds.
+bool choose_stream(GemmPlan &p, int T, int K, int N, bool &short_rounds) {
   const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.453f}, {1, 4, 0.534f}, {2, 2, 0.587f}, {3, 2, 0.801f}};
-  float least = INFINITY, loop = INFINITY;
+  float least = INFINITY;
+  bool fits = false;
   p.mb = 3;
   p.kg = 2;
   for (const auto &s : shapes) {
@@ -927,11 +931,12 @@ bool choose_stream(GemmPlan &p, int T, int K, int N) {
     const float us = turns + (pieces > 1 ? 1.4f + 0.27e-6f * 8 * 32 * s.mb * (256 / s.kg) * wgs : 0.f);
     if (us >= least) continue;
     least = us;
-    loop = turns;
+    fits = wgs <= 256 && turns <= 20.f && !(s.mb == 3 && quota == 4);
+    short_rounds = wgs > 256 && quota == 4;
     p.mb = s.mb;
     p.kg = s.kg;
   }
-  return loop <= 20.f;
+  return fits;
 }
 
 // The tile, by what was measured (us, 2048 -> 3072 | 2048 -> 2048 | 2048 -> 16384 | 8192 -> 2048 | 1024 -> 8192):
@@ -965,7 +970,15 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
   p.wn = 2;
   const long long weights = (long long)K * N, rows1 = (T + 31) / 32 * 32LL, rows2 = (T + 127) / 128 * 128LL;
   p.few = T <= 96 || (T <= 256 && (weights <= (T <= 128 ? 12 : 5) << 20 || rows2 * 100 >= rows1 * 125));
-  if (p.parts == 1) p.few = choose_stream(p, T, K, N) || p.few;
+  if (p.parts == 1) {
+    const bool low = p.few;
+    bool short_rounds = false;
+    p.few = choose_stream(p, T, K, N, short_rounds) || low;
+    // (its loop goes by four steps: of up to 64 long rows most are empty, and many rounds of four do not pay, either; as many
+    // sums in tiles of 32 rows, us, this | three parts: 48 rows of 32 -> 32000 8.7 | 7.2, 200 rows 29 | 20, 97 rows of 64 -> 32000
+    // 15.8 | 14.2, of 128 18.7 | 17.5, but of 128 -> 16384 9.4 | 10.7)
+    if (low && (K <= 64 || short_rounds)) p.parts = 3;
+  }
   p.few = p.few && (long long)kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows)
   if (p.few && p.parts == 1) return;
   p.mb = 1;

@@ -84,7 +84,7 @@ BF16_MATMULS = [
     (40, 2048, 2308, ("few", (64, 128), True, False, False)),
     (100, 2052, 2308, ("few", (64, 128), True, False, True)),
     (200, 96, 8200, ("few", (96, 128), False, False, False)),
-    (257, 100, 8196, ("few", (96, 128), False, False, True)),
+    (200, 100, 8196, ("few", (96, 128), False, False, True)),
     (96, 2048, 3072, ("few", (96, 128), True, False, False)),
     (75, 2052, 2308, ("few", (96, 128), True, False, True)),
     (512, 2048, 16384, ("tiles", (128, 256), False, False, False)),

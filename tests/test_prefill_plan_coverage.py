@@ -115,3 +115,12 @@ def test_large_tiles_fill_their_last_round():
         plan = sa.hip.describe_matmul(rows, 2048, 8192)
         large = tiles >= 256 and (tiles % 256 == 0 or tiles % 256 >= 128)
         assert (plan["tile"] == (256, 256)) == (large and -(-rows // 256) * 256 * 100 <= -(-rows // 128) * 128 * 115), (rows, plan)
+
+
+def test_low_tiles_of_bf16_weights_stay_within_a_round():
+    # more than a workgroup a compute unit, each with a start of its own, takes up to three times as long as the large tiles
+    for T, K, N in ((4000, 32, 4096), (512, 64, 32000), (777, 128, 16384), (2048, 128, 4096), (512, 256, 16384), (1100, 192, 4096)):
+        assert sa.hip.describe_matmul(T, K, N, bf16_weights=True)["kind"] == "tiles", (T, K, N)
+    for T, K, N in itertools.product((257, 300, 512, 777, 1100, 2048, 4000), (32, 100, 256, 512, 1024, 2048), (132, 1024, 4092, 16384)):
+        plan = sa.hip.describe_matmul(T, K, N, bf16_weights=True)
+        assert plan["kind"] == "tiles" or plan["workgroups"] <= 256, (T, K, N, plan)
