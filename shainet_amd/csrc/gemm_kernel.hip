@@ -15,7 +15,7 @@
 //      place c / 2: a lane's two blocks are neighbouring columns of y (8-byte stores, 256 bytes a row).
 // Tile loads take a scalar base that moves along K plus a per-thread 32-bit offset.
 // W whose values are bf16 numbers (a checkpoint's, most often): the other two of its parts are zeros, and the three
-// products with them add nothing.  They are left out, sum for sum the same bits.  2048 rows of 2048 -> 16384 571 -> 345 us
+// products with them add nothing.  They are left out, in the same tiles with the same bits.  2048 rows of 2048 -> 16384 571 -> 345 us
 // (398 TFLOP/s), 8192 -> 2048 322 -> 194, 512 rows 174 -> 100 and 101 -> 61, 777 rows of 1024 -> 4096 53 -> 35.  What bounds
 // these is issue: the matrix cores are busy 54 % of the time, in which a step's 24 MFMAs share two wavefronts a SIMD with
 // 70 vector instructions each, and everybody meets at a barrier.  Tiles of four by two wavefronts (64 x 128 each) read
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 // rows and 256 / KG columns, 32 of them a wavefront, and walks K in steps of 16 KG, of which each of KG groups of wavefronts
 // takes its own 16.  W goes from memory to registers four steps ahead (64 KB in flight on a compute unit), x through LDS.
 // Sums as in the kernel above, emptied every four steps, three products instead of six: no larger an error than
-// that kernel's anywhere (1e-8, 17 rows: 1024 -> 1024 7.5 | 8.0, 2048 -> 16384 8.4 | 10.2, 8192 -> 2048 10.3 | 12.1; emptied every eight
+// that kernel's anywhere (1e-8, 17 rows: 1024 -> 1024 7.9 | 7.9, 2048 -> 16384 8.4 | 10.2, 8192 -> 2048 10.3 | 12.1; emptied every eight
 // steps 96 rows of 768 -> 2304 7.9 | 7.6).
 // Against tiles of 32 x 128 that read W once per 32 rows and add 32-row pieces (us, with the kernel that adds the pieces): 45 rows
 // of 2048 -> 16384 40 -> 35, 2048 -> 2048 15.0 -> 12.7, 8192 -> 2048 31 -> 29, 1024 -> 1024 11.6 -> 9.1; 96 rows 59 -> 44,
