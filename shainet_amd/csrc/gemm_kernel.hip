@@ -661,12 +661,18 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 // Sums as in the kernel above, emptied every four steps, three products instead of six: no larger an error than
 // that kernel's anywhere (1e-8, 17 rows: 1024 -> 1024 7.9 | 7.9, 2048 -> 16384 8.4 | 10.2, 8192 -> 2048 10.3 | 12.1; emptied every eight
 // steps 96 rows of 768 -> 2304 7.9 | 7.6).
-// Against tiles of 32 x 128 that read W once per 32 rows and add 32-row pieces (us, with the kernel that adds the pieces): 45 rows
-// of 2048 -> 16384 40 -> 35, 2048 -> 2048 15.0 -> 12.7, 8192 -> 2048 31 -> 29, 1024 -> 1024 11.6 -> 9.1; 96 rows 59 -> 44,
-// 15.1 -> 14.9, 34 -> 34, 11.7 -> 9.7; and against 128 x 256 in 8 pieces 512 rows of 1024 -> 1024 21 -> 13.  W of 134 MB
-// comes at 4.5 TB/s, smaller ones wait for a launch or two, the first loads and the steps' barriers.
+// Bound by reading W where it is large: nothing but these loads takes 24.9 us for 2048 -> 16384 and 17.9 for 8192 -> 2048, a launch
+// of 4 included.  Loads of x that hung on a condition had the compiler wait for every load in flight once in four steps,
+// and twice in front of the loop; and wavefronts that fetch fragments, split, multiply and meet, one after the other, all
+// at the same time, leave each of these idle while the others last.  Us without the kernel that adds pieces, such loops | now: 45
+// rows of 2048 -> 16384 30.7 | 27.0, 8192 -> 2048 24.1 | 21.9, 2048 -> 3072 12.5 | 10.6, 17 rows of 2048 -> 16384 30.1 | 26.4, 777 rows of
+// 1024 -> 2048 24.8 | 21.8, 1024 -> 1024 15.1 | 13.6.  (Fragments a step ahead serve the 64-row tiles only: tiles of 32 rows have
+// three MFMAs to put the rest between and are level or slower, 96 rows have no registers for them.  Tried and not kept:
+// non-temporal loads of W, 30.7 | 32.7; eight wavefronts that take 64 columns and every eighth step by themselves, without a barrier:
+// 32.9; tiles of 64 x 64: level at best.)
 template <int MB, int KG, bool GUARD>
 __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) {
+  constexpr bool AHEAD = MB == 2;  // whether fragments are fetched a step ahead
   constexpr int WN = 8 / KG, TM = 32 * MB, TN = 32 * WN, TS = 16 * KG, kSets = 4;
   constexpr int kOct = TM + 4, kPart = 2 * KG * kOct, kStage = 3 * kPart;  // units of 16 bytes, as above
   constexpr int kSums = MB * 16 * 64 / 4;                                  // units that a wavefront's sums take
@@ -695,36 +701,51 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
   u32x2 *const x_lds = (u32x2 *)(lds + (xk >> 3) * kOct + xrow) + (xk >> 2 & 1);
   // W: rows 16 kg + 8 j .. + 7 of a step (columns past the last one repeat it)
   const int wk = 16 * kg + 8 * j;
-  const unsigned w_off = (unsigned)(((long long)8 * j * N + min(col, N - 1)) * 4);
-  const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)(k_begin + 16 * kg) * N);
+  const unsigned w_off = (unsigned)(((long long)(GUARD ? 0 : 8 * j) * N + min(col, N - 1)) * 4);
+  const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)(k_begin + (GUARD ? 0 : 16 * kg)) * N);
   const long long row_bytes = 4LL * N;
 
-  // register sets: the tiles of step t travel in set t % 4 and are requested four steps ahead.  Behind the last step its
-  // W is requested again, and its x counts as zeros: the loop has no conditions.
+  // Register sets: what step t takes of W travels in set t % 4 and is requested four or five steps ahead, its x likewise.  Behind
+  // the end the last step's is requested again, x counts as zeros, and so it does where K ends within a step (GUARD): no load
+  // hangs on a condition, in front of which the compiler would wait for all those in flight.
   f32x4 sx[kSets][kRounds];
   float sw[kSets][8];
-  int k_next = k_begin, to_load = nk;
-  auto load_tiles = [&](const int set) {
+  int x_step = 0, w_step = 0;  // to be requested next
+  auto load_x = [&](const int set) {
 #pragma unroll
-    for (int u = 0; u < kRounds; ++u) {
-      sx[set][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (to_load > 0 && (!GUARD || k_next + xk < k_end) && (TM % kRows == 0 || xrow + kRows * u < TM)) sx[set][u] = load_at((const f32x4 *)x_base, x_off[u]);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      sw[set][i] = GUARD && k_next + wk + i >= k_end ? 0.f : load_at((const float *)(w_base + i * row_bytes), w_off);
-    if (--to_load > 0) {
+    for (int u = 0; u < kRounds; ++u)
+      sx[set][u] = load_at((const f32x4 *)x_base, GUARD && k_begin + x_step * TS + xk >= k_end ? x_off[u] - 4 * xk : x_off[u]);
+    if (x_step + 1 < nk) {
+      ++x_step;
       x_base += TS * 4;
-      w_base += TS * row_bytes;
-      k_next += TS;
     }
   };
-  auto park_x = [&](const int set, const int stage) {
+  auto load_w = [&](const int set) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      sw[set][i] = GUARD ? load_at((const float *)w_base, (unsigned)(min(wk + i, k_end - k_begin - w_step * TS - 1) * row_bytes) + w_off)
+                         : load_at((const float *)(w_base + i * row_bytes), w_off);
+    if (w_step + 1 < nk) {
+      ++w_step;
+      w_base += TS * row_bytes;
+    }
+  };
+  unsigned parts[kRounds][3][2];  // of x of step t
+  auto split_x = [&](const int t, const int set) {
+    const float lift = (GUARD ? k_begin + t * TS + xk < k_end : t < nk) ? kLift : 0.f;
+#pragma unroll
+    for (int u = 0; u < kRounds; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        split_pair(sx[set][u][2 * h] * lift, sx[set][u][2 * h + 1] * lift, parts[u][0][h], parts[u][1][h], parts[u][2][h]);
+  };
+  auto park_x = [&](const int stage) {
 #pragma unroll
     for (int u = 0; u < kRounds; ++u) {
       if (TM % kRows != 0 && xrow + kRows * u >= TM) continue;
       u32x2 *at = x_lds + 2 * (stage * kStage + kRows * u);
-      split_quad(sx[set][u] * kLift, at[0], at[2 * kPart], at[4 * kPart]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) at[2 * p * kPart] = u32x2{parts[u][p][0], parts[u][p][1]};
     }
   };
 
@@ -734,39 +755,96 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[a][r] = rest[a][r] = sum[a][r] = 0.f;
 
-#pragma unroll
-  for (int set = 0; set < kSets; ++set) load_tiles(set);
-  park_x(0, 0);
-  __syncthreads();
-  auto step = [&](const int set) {  // set: holds this step; its x is in stage set % 2
-    const u32x4 *stage = lds + (set & 1) * kStage + (2 * kg + j) * kOct + ln;
-    u32x4 bf;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) bf[i] = pack_high(sw[set][2 * i] * kLift, sw[set][2 * i + 1] * kLift);
-    u32x4 af[3][MB];
-#pragma unroll
-    for (int p = 0; p < 3; ++p)
-#pragma unroll
-      for (int a = 0; a < MB; ++a) af[p][a] = stage[p * kPart + 32 * a];
-    park_x((set + 1) % kSets, (set & 1) ^ 1);
-    load_tiles(set);
-#pragma unroll
-    for (int p = 2; p > 0; --p)
-#pragma unroll
-      for (int a = 0; a < MB; ++a) rest[a] = mfma_bf16(af[p][a], bf, rest[a]);
-#pragma unroll
-    for (int a = 0; a < MB; ++a) acc[a] = mfma_bf16(af[0][a], bf, acc[a]);
-    __syncthreads();
-  };
-  for (int k0 = 0; k0 < nk; k0 += 4) {
-    step(0);
-    step(1);
-    step(2);
-    step(3);
+  auto empty = [&]() {
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
       for (int r = 0; r < 16; ++r) sum[a][r] += acc[a][r], acc[a][r] = 0.f;
+  };
+  u32x4 af[AHEAD ? 2 : 1][3][MB], bf[AHEAD ? 2 : 1];
+  auto fetch_x = [&](const int set, const int stage, const int p, const int a) {
+    af[set][p][a] = lds[stage * kStage + (2 * kg + j) * kOct + ln + p * kPart + 32 * a];
+  };
+  auto pack_w = [&](const int set, const int from, const int i) { bf[set][i] = pack_high(sw[from][2 * i] * kLift, sw[from][2 * i + 1] * kLift); };
+  auto multiply = [&](const int set, const int p, const int a) {  // smallest products first
+    f32x16 &to = p ? rest[a] : acc[a];
+    to = mfma_bf16(af[set][p][a], bf[set], to);
+  };
+
+  // (what is needed first is requested first)
+  load_w(0);
+  load_x(0);
+  load_x(1);
+#pragma unroll
+  for (int set = 1; set < kSets; ++set) load_w(set);
+  load_x(2);
+  load_x(3);
+  split_x(0, 0);
+  park_x(0);
+  load_x(0);
+  if constexpr (!AHEAD) {
+    __syncthreads();
+    auto step = [&](const int t, const int at) {  // at: t % 4
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pack_w(0, at, i);
+#pragma unroll
+      for (int i = 0; i < 3 * MB; ++i) fetch_x(0, at & 1, i / MB, i % MB);
+      split_x(t + 1, (at + 1) % kSets);
+      park_x((at & 1) ^ 1);
+      load_x((at + 1) % kSets);
+      load_w(at);
+#pragma unroll
+      for (int i = 0; i < 3 * MB; ++i) multiply(0, 2 - i / MB, i % MB);
+      __syncthreads();
+    };
+    for (int t = 0; t < nk; t += 4) {
+      step(t, 0);
+      step(t + 1, 1);
+      step(t + 2, 2);
+      step(t + 3, 3);
+      empty();
+    }
+  } else {
+    // Fragments are fetched a step ahead, from the stage that is whole since the last barrier, and the x of the step behind that
+    // one goes into the stage whose fragments everybody has.  What else a step does stands between its MFMAs: left to itself the
+    // compiler puts it behind them, and all wavefronts are at the same of the two at the same time.
+    split_x(1, 1);
+    park_x(1);
+    load_x(1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pack_w(0, 0, i);
+    load_w(0);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 3 * MB; ++i) fetch_x(0, 0, i / MB, i % MB);
+    __syncthreads();
+    auto step = [&](const int t, const int at) {  // at: t % 4
+      const int cur = at & 1, next = cur ^ 1;
+#pragma unroll
+      for (int slot = 0; slot < 3 * MB; ++slot) {
+        multiply(cur, 2 - slot / MB, slot % MB);
+#pragma unroll
+        for (int i = 2 * slot; i < 2 * slot + 2 && i < 3 * MB; ++i) fetch_x(next, next, 2 - i / MB, i % MB);
+        if (slot < 2) {
+          pack_w(next, (at + 1) % kSets, 2 * slot);
+          pack_w(next, (at + 1) % kSets, 2 * slot + 1);
+          if (slot == 1) load_w((at + 1) % kSets);
+        } else if (slot == 2) {
+          split_x(t + 2, (at + 2) % kSets);
+          park_x(cur);
+          load_x((at + 2) % kSets);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+    };
+    for (int t = 0; t < nk; t += 4) {
+      step(t, 0);
+      step(t + 1, 1);
+      step(t + 2, 2);
+      step(t + 3, 3);
+      empty();
+    }
   }
 
 #pragma unroll
@@ -907,17 +985,16 @@ int stream_quota(int tiles, int steps) {
 }
 
 // W of one part: the tile of sgemm_stream_kernel by an estimate of its time, and whether that kernel is the one to take.
-// Rounds of workgroups times steps times what a step takes, and for pieces 1.4 us and 0.27 us per MB of them written and
-// read: fitted to 60 products of 5 to 777 rows, 5 % off on average.  Where its loop alone takes more than 20 us or one
-// round of workgroups does not do, the larger tiles, which read W less often, are level or ahead, and so they are of a loop of
-// four steps in tiles of 96 rows (over 408 products of 97 to 4000 rows, K 32 to 2048, N 256 to 32000, this rule loses 0.5 % to
-// the better of the two, without the second and third 12 %; us, this | 128 x 256): 256 rows of
-// 2048 -> 2048 19.2 | 23.3, 2048 -> 3072 26.9 | 25.5, 8192 -> 2048 52 | 43, 2048 -> 16384 96 | 64; 512 rows of 1024 -> 1024
-// 13.0 | 20.8, 1024 -> 3072 24.3 | 25.0, 2048 -> 2048 28.1 | 28.3, 2048 -> 3072 42 | 33; 777 rows of 1024 -> 1024 19.0 | 24.2,
-// 1024 -> 3072 34 | 32; 96 rows of 2048 -> 16384 43 | 52; rounds: 512 rows of 128 -> 16384 30 | 15, 2048 rows of 128 -> 4096 31 | 17.
+// Rounds of workgroups times steps times what a step takes, and for pieces 2.95 us and 0.416 us per MB of them written and
+// read: fitted to what each of the four tiles and 128 x 256 take for 80 products of 8 to 1400 rows, K 32 to 8192, N 32 to 16384, of which
+// the choice loses 0.9 % to the best of the five.  Where its loop alone takes more than 17 us or one round of workgroups does
+// not do, the larger tiles, which read W less often, are level or ahead, and so they are of a loop of four steps in tiles of 96 rows (us,
+// this | 128 x 256): 256 rows of 2048 -> 2048 19.0 | 23.1, 2048 -> 3072 25.6 | 25.5, 2048 -> 4608 35 | 30; 400 rows of 2048 -> 1536 21.4 |
+// 23.8; 512 rows of 1024 -> 1024 12.6 | 21, 1024 -> 3072 20.8 | 25.2; 777 rows of 1024 -> 1024 16.6 | 24.3, 1024 -> 2048 22.1 | 26.0,
+// 1024 -> 3072 35 | 30; 1400 rows of 2048 -> 1024 34 | 31; rounds: 512 rows of 128 -> 16384 30 | 15, 2048 rows of 128 -> 4096 31 | 17.
 // short_rounds: its loop is of four steps, and in several rounds.
 bool choose_stream(GemmPlan &p, int T, int K, int N, bool &short_rounds) {
-  const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.453f}, {1, 4, 0.534f}, {2, 2, 0.587f}, {3, 2, 0.801f}};
+  const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.483f}, {1, 4, 0.563f}, {2, 2, 0.506f}, {3, 2, 0.643f}};
   float least = INFINITY;
   bool fits = false;
   p.mb = 3;
@@ -928,10 +1005,10 @@ bool choose_stream(GemmPlan &p, int T, int K, int N, bool &short_rounds) {
     const int steps = (K + 16 * s.kg - 1) / (16 * s.kg), quota = stream_quota((int)tiles, steps), pieces = (steps + quota - 1) / quota;
     const long long wgs = tiles * pieces;
     const float turns = (float)((wgs + 255) / 256) * quota * s.step;
-    const float us = turns + (pieces > 1 ? 1.4f + 0.27e-6f * 8 * 32 * s.mb * (256 / s.kg) * wgs : 0.f);
+    const float us = turns + (pieces > 1 ? 2.95f + 0.416e-6f * 8 * 32 * s.mb * (256 / s.kg) * wgs : 0.f);
     if (us >= least) continue;
     least = us;
-    fits = wgs <= 256 && turns <= 20.f && !(s.mb == 3 && quota == 4);
+    fits = wgs <= 256 && turns <= 17.f && !(s.mb == 3 && quota == 4);
     short_rounds = wgs > 256 && quota == 4;
     p.mb = s.mb;
     p.kg = s.kg;
@@ -979,7 +1056,7 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
     // 15.8 | 14.2, of 128 18.7 | 17.5, but of 128 -> 16384 9.4 | 10.7)
     if (low && (K <= 64 || short_rounds)) p.parts = 3;
   }
-  p.few = p.few && (long long)kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows)
+  p.few = p.few && 2LL * kFewStep * N * 4 < 0xffffffffLL;  // (32-bit offsets into a step's rows, 64 at most)
   if (p.few && p.parts == 1) return;
   p.mb = 1;
   if (p.few) return;
@@ -1125,11 +1202,6 @@ hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, hipStream_t strea
   return hipGetLastError();
 }
 
-template <int MB>
-hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
-  return p.kg == 4 ? launch_stream<MB, 4>(g, p, stream) : launch_stream<MB, 2>(g, p, stream);
-}
-
 }  // namespace
 
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
@@ -1167,7 +1239,8 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   g.quota = p.quota;
   g.pieces = p.pieces > 1 ? p.pieces : 0;
   if (p.parts == 1) {
-    if (p.few) return p.mb == 1 ? launch_stream<1>(g, p, stream) : p.mb == 2 ? launch_stream<2>(g, p, stream) : launch_stream<3>(g, p, stream);
+    if (p.few && p.kg == 4) return launch_stream<1, 4>(g, p, stream);
+    if (p.few) return p.mb == 1 ? launch_stream<1, 2>(g, p, stream) : p.mb == 2 ? launch_stream<2, 2>(g, p, stream) : launch_stream<3, 2>(g, p, stream);
     return p.mb == 4 ? launch_tiles<4, 2, 2, 4, 1>(g, p, stream) : launch_tiles<2, 4, 2, 2, 1>(g, p, stream);
   }
   if (p.few) return launch_few(g, p, stream);
