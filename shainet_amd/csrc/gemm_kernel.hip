@@ -216,24 +216,40 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     f32x4 sx[kSets][NX];
     float sw[kSets][8];
     int k_next = k_begin, to_load = nk;
-    auto load_tiles = [&](f32x4 (&rx)[NX], float (&rw)[8]) {
+    unsigned w_row[8];  // (PARTS 1) a row of W each: one base serves all of a step's loads
 #pragma unroll
-      for (int u = 0; u < NX; ++u) {
-        const int kk = k_next + xk + 4 * u;
-        rx[u] = GUARD && kk >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f}
-                : PARTS == 3         ? *(const f32x4 *)(x_base + x_off + 16 * u)
-                                     : load_at((const f32x4 *)(x_base + 16 * u), x_off);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float *row = (const float *)(w_base + (long long)i * N * 4);
-        rw[i] = GUARD && k_next + wk + i >= k_end ? 0.f : PARTS == 3 ? *(const float *)((const char *)row + w_off) : load_at(row, w_off);
-      }
+    for (int i = 0; i < 8; ++i) w_row[i] = w_off + 4u * i * (unsigned)N;
+    constexpr int kLoads = NX + 8;
+    auto load_one = [&](f32x4 (&rx)[NX], float (&rw)[8], const int l) {
+      if (l < NX)
+        rx[l] = GUARD && k_next + xk + 4 * l >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : load_at((const f32x4 *)(x_base + 16 * l), x_off);
+      else
+        rw[l - NX] = GUARD && k_next + wk + l - NX >= k_end ? 0.f : load_at((const float *)w_base, w_row[l - NX]);
+    };
+    auto advance = [&]() {
       if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
         x_base += TK * 4;
         w_base += w_step;
         k_next += TK;
       }
+    };
+    auto load_tiles = [&](f32x4 (&rx)[NX], float (&rw)[8]) {
+      if constexpr (PARTS == 1) {
+#pragma unroll
+        for (int l = 0; l < kLoads; ++l) load_one(rx, rw, l);
+      } else {
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+          const int kk = k_next + xk + 4 * u;
+          rx[u] = GUARD && kk >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4 *)(x_base + x_off + 16 * u);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float *row = (const float *)(w_base + (long long)i * N * 4);
+          rw[i] = GUARD && k_next + wk + i >= k_end ? 0.f : *(const float *)((const char *)row + w_off);
+        }
+      }
+      advance();
     };
     auto park_tiles = [&](const f32x4 (&rx)[NX], const float (&rw)[8], u32x4 *stage) {
       u32x4 h, m, l;
@@ -310,7 +326,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
       // Half the MFMAs leave no time for fragments to arrive within their step: they are fetched a step ahead, from the
       // stage that is whole since the last barrier, and the tiles of the step behind that one go into the stage whose
       // fragments everybody has.  Everything else a step does is handed out between its MFMAs, one at a time: left
-      // to itself the compiler puts them after each other (2048 rows of 2048 -> 16384: 385 us, 345 this way).
+      // to itself the compiler puts them after each other (2048 rows of 2048 -> 16384: 385 us, 345 this way).  So do the loads:
+      // all in one slot, each row of W with a base of its own, stood in the way of both wavefronts of a SIMD at once (us, so |
+      // handed out: 2048 rows of 2048 -> 16384 358 | 345, 8192 -> 2048 188 | 182, 1024 rows of 2048 -> 16384 188 | 183, 777 rows of
+      // 1024 -> 4096 29.3 | 28.0, 512 rows of 2048 -> 3072 27.0 | 25.9).  Two steps to a barrier, with three stages of LDS: 0 to 5 % slower.
       u32x4 af[3][MB], first[2][MB], bf[2][NB];  // (the first parts of x and W of two steps)
       auto fetch_x = [&](const u32x4 *stage, const int p, u32x4 (&f)[MB]) {
 #pragma unroll
@@ -359,7 +378,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
               h[i] = pack_high(sw[set][2 * i] * kLift, sw[set][2 * i + 1] * kLift);
             if (slot == kEnd - 1) stage[w_unit] = h;
           }
-          if (slot == kEnd) load_tiles(sx[set], sw[set]);
+          if (slot >= kEnd) {
+            constexpr int kLeft = kSlots - kEnd;
+#pragma unroll
+            for (int l = (slot - kEnd) * kLoads / kLeft; l < (slot - kEnd + 1) * kLoads / kLeft; ++l) load_one(sx[set], sw[set], l);
+            if (slot == kSlots - 1) advance();
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
