@@ -84,7 +84,7 @@ struct BiasedAttn : Mixer {
   shainet_kv_cache *cache() override { return kv ? kv : from->kv; }
   BiasedAttn *biased() override { return this; }
 
-  int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache) override {
+  int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache, Handover *next = nullptr) override {
     const int H = cfg.heads, KV = cfg.kv_heads, dim = cfg.dim, vdim = cfg.vdim, d = d_model, qw = H * dim;
     if (!table) return fail(SHAINET_HIP_ERR_ARGUMENT, "weights not set");
     hipStream_t s = ctx->stream;
@@ -133,6 +133,7 @@ struct BiasedAttn : Mixer {
       if (kv) kv->len[0] = rows;
     }
     Fused post;
+    post.next = next;
     post.w_bf16 = w.w_o_bf16;
     if (residual) {
       post.epilogue = kGemvResidual;

@@ -43,6 +43,7 @@
 // kernel, with the whole chip, adds the pieces in a fixed order (and the residual).
 #include "gemm_kernel.hpp"
 
+#include "attn_kernels.hpp"
 #include "split_mfma.hpp"
 
 #include <math.h>
@@ -923,10 +924,13 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
       const f32x4 *const other = merge + 64 * (4 * a + r);
       v += other[0];  // (in pairs: four groups' sums one after the other round a little more)
       if constexpr (KG == 4) v += other[WN * kSums] + other[2 * WN * kSums];
-      if (g.pieces)  // [four rows][thread], as the kernel that adds the pieces takes them
-        *(f32x4 *)(g.partials + (long long)blockIdx.x * (TM * TN) + (4 * a + r) * (256 * WN) + 4 * threadIdx.x) = v;
-      else if (col < N)
+      if (g.pieces) {  // row by row
+        float *const piece = g.partials + (long long)blockIdx.x * (TM * TN) + (32 * a + 8 * r + 4 * j) * TN + 32 * wn + ln;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) piece[i * TN] = v[i];
+      } else if (col < N) {
         store_four<1>(g, m0 + 4 * j, col, 4 * a + r, v);
+      }
     }
 }
 
@@ -942,36 +946,148 @@ __device__ __forceinline__ f32x4 add_pieces(f32x4 acc, const float *piece, long 
   return acc;
 }
 
-// y tile = (res +) piece 0 + piece 1 + ... of the tile, in that order, four of them in flight: 16 pieces of 17 rows of 132
-// columns 5.4 us one after the other, 4.1 two at a time, 3.6 so, 3.1 eight at a time; launches that fill the chip take the
-// same time each way.  Only what is needed is requested, or those take 10 to 30 % longer: pieces that are not there, and
-// rows that pad a tile (777 rows of 8192 -> 4092, four pieces of tiles of 256 x 256: 11.4 us, with them 14.4).
-// A piece lies in its workgroup's slot as [pair of rows, or row][thread] float4, the layout of the product kernel's
-// accumulators.  A tile's threads are WM x WN wavefronts of MB x NB blocks.
-template <int WM, int WN, int MB, int NB>
-__global__ __launch_bounds__(64 * WM * WN) void sgemm_reduce_kernel(const GemmArgs g, int tiles) {
-  constexpr int kOut = 4 * MB * NB, TM = 32 * WM * MB, TN = 32 * WN * NB;
-  const int tile = blockIdx.x / kOut, r = blockIdx.x % kOut;  // kOut workgroups per tile, a float4 of each thread each
-  if (tile >= tiles) return;
-  const int group = tile / g.tiles_per_group, t = tile - group * g.tiles_per_group;
-  constexpr long long kSlot = (long long)TM * TN;
-  const float *piece = g.partials + (long long)(((t * g.pieces) << g.group_bits) | group) * kSlot + r * 256 * WM * WN + 4 * threadIdx.x;
-  const long long piece_step = kSlot << g.group_bits;
-  const int n = min(g.pieces, (g.steps + g.quota - 1) / g.quota);  // pieces that hold any steps
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = (tile % g.tiles_m) * TM + (wave / WN) * 32 * MB + 4 * (lane >> 5);
-  const int col = (tile / g.tiles_m) * TN + (wave % WN) * 32 * NB + NB * (lane & 31);
-  if (row0 + row_of<NB>(r) >= g.T || col >= g.N) return;  // (nothing is read for rows that pad a tile)
+// How a product's tiles lie in its workgroups' slots.  `columns` of a lane: 1: row by row; 2: [pair of rows][thread] float4, two
+// neighbouring columns of two rows; 4: [row][thread] float4, four columns of one.
+struct PieceShape {
+  int tm, tn;      // rows and columns of a tile
+  int rows, wn;    // rows of a wavefront, wavefronts along the columns
+  int threads;     // of the workgroup
+};
+
+// Where the first piece of (row, col) lies: four columns of a row, or (COLUMNS 2) two columns of two rows.
+template <int COLUMNS>
+__device__ __forceinline__ const float *first_piece(const GemmArgs &g, const PieceShape &s, int row, int col) {
+  const int tm = row / s.tm, tn = col / s.tn, r = row - tm * s.tm, c = col - tn * s.tn;
+  const int tile = tn * g.tiles_m + tm, group = tile / g.tiles_per_group, t = tile - group * g.tiles_per_group;
+  const float *slot = g.partials + (((long long)t * g.pieces << g.group_bits) | group) * s.tm * s.tn;
+  if constexpr (COLUMNS == 1) return slot + r * s.tn + c;
+  const int wm = r / s.rows, q = r - wm * s.rows, in = q & 31, at = 4 * (in >> 3) + (in & 3);  // (of the 16 registers of a block)
+  const int out = COLUMNS == 2 ? 8 * (q >> 5) + at / 2 : 16 * (q >> 5) + at;
+  const int thread = (wm * s.wn + c / (32 * COLUMNS)) * 64 + 32 * (in >> 2 & 1) + c % (32 * COLUMNS) / COLUMNS;
+  return slot + 4 * ((long long)out * s.threads + thread);
+}
+
+// piece 0 + piece 1 + ... in that order, four of them in flight: 16 pieces of 17 rows of 132 columns 5.4 us one after the other, 4.1
+// two at a time, 3.6 so, 3.1 eight at a time; launches that fill the chip take the same time each way.  Only pieces
+// that are there are requested, and nothing for rows that pad a tile: with them 777 rows of 8192 -> 4092 took 14.4 us, not 11.4.
+__device__ __forceinline__ f32x4 sum_of_pieces(const GemmArgs &g, const PieceShape &s, const float *piece) {
+  const long long step = (long long)s.tm * s.tn << g.group_bits;
   f32x4 acc = {-0.f, -0.f, -0.f, -0.f};  // (which adds nothing to anything)
-  int left = n;
-  for (; left >= 4; left -= 4, piece += 4 * piece_step) acc = add_pieces<4>(acc, piece, piece_step);
+  int left = min(g.pieces, (g.steps + g.quota - 1) / g.quota);  // pieces that hold any steps
+  for (; left >= 4; left -= 4, piece += 4 * step) acc = add_pieces<4>(acc, piece, step);
   if (left == 3)
-    acc = add_pieces<3>(acc, piece, piece_step);
+    acc = add_pieces<3>(acc, piece, step);
   else if (left == 2)
-    acc = add_pieces<2>(acc, piece, piece_step);
+    acc = add_pieces<2>(acc, piece, step);
   else if (left == 1)
-    acc = add_pieces<1>(acc, piece, piece_step);
-  store_four<NB>(g, row0, col, r, acc);
+    acc = add_pieces<1>(acc, piece, step);
+  return acc;
+}
+
+__device__ __forceinline__ float swiglu(float gate, float up) {  // (swiglu_ff.cr:84-89)
+  const double g = (double)gate;
+  return (float)((g / (1.0 + exp(-g))) * (double)up);
+}
+
+// y = (res +) the sum of a product's pieces, or (SWIGLU) silu(gate) * up of its columns gate | up.  A thread takes what a lane of
+// the product held in one register of four: grid (columns, rows).
+template <int COLUMNS, bool SWIGLU>
+__global__ __launch_bounds__(256) void sgemm_sum_kernel(const GemmArgs g, const PieceShape s) {
+  constexpr int R = COLUMNS == 2 ? 2 : 1, C = 4 / R;
+  const int row = R * blockIdx.y, col = C * (blockIdx.x * blockDim.x + threadIdx.x), N = SWIGLU ? g.N / 2 : g.N;
+  if (col >= N) return;
+  const f32x4 v = sum_of_pieces(g, s, first_piece<COLUMNS>(g, s, row, col));
+  if constexpr (SWIGLU) {
+    const f32x4 u = sum_of_pieces(g, s, first_piece<COLUMNS>(g, s, row, N + col));
+    const f32x4 h = {swiglu(v.x, u.x), swiglu(v.y, u.y), swiglu(v.z, u.z), swiglu(v.w, u.w)};
+    float *y = g.y + (long long)row * N + col;
+    if constexpr (R == 1) {
+      *(f32x4 *)y = h;
+    } else {
+      *(f32x2 *)y = f32x2{h.x, h.y};
+      if (row + 1 < g.T) *(f32x2 *)(y + N) = f32x2{h.z, h.w};
+    }
+  } else {
+    store_four<R == 1 ? 4 : 2>(g, row, col, 0, v);
+  }
+}
+
+// The same, and the norm of the whole rows, which the next product reads, in one launch: a workgroup takes a row (COLUMNS 2: two rows), a
+// thread up to two registers of four.  The sums of squares are fp64, as rms_norm.cr has them.  Bound by a launch and two round trips; us, a
+// sum and a norm | this: 45 rows of 8192 -> 2048, 16 pieces, 4.9 + 3.9 | 5.0, of 2048 -> 2048 3.9 + 4.2 | 4.3; 512 rows of 8192 -> 2048, 8
+// pieces, 8.3 + 5.1 | 11.0, 2048 rows, 4 pieces, with Dynamic Tanh 18.6 + 7.2 | 24.5.
+template <int COLUMNS>
+__global__ __launch_bounds__(1024) void sgemm_sum_norm_kernel(const GemmArgs g, const PieceShape s, const NextNorm norm) {
+  constexpr int R = COLUMNS == 2 ? 2 : 1, C = 4 / R, kMost = 2;
+  __shared__ double red[R][16];
+  const int row = R * blockIdx.x, N = g.N;
+  const bool second = R == 2 && row + 1 < g.T;
+  f32x4 v[kMost], res[kMost];
+  double sq[R] = {};
+#pragma unroll
+  for (int u = 0; u < kMost; ++u) {  // (the residual is requested in front of the pieces, whose sums wait for theirs)
+    const int col = C * (threadIdx.x + u * blockDim.x);
+    res[u] = f32x4{-0.f, -0.f, -0.f, -0.f};
+    if (!g.res || col >= N) continue;
+    const float *at = g.res + (long long)row * N + col;
+    if constexpr (R == 1) {
+      res[u] = *(const f32x4 *)at;
+    } else {
+      const f32x2 a = *(const f32x2 *)at, b = *(const f32x2 *)(at + (second ? N : 0));
+      res[u] = f32x4{a.x, a.y, b.x, b.y};
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kMost; ++u) {
+    const int col = C * (threadIdx.x + u * blockDim.x);
+    v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (col >= N) continue;
+    v[u] = res[u] + sum_of_pieces(g, s, first_piece<COLUMNS>(g, s, row, col));
+    float *at = g.y + (long long)row * N + col;
+    if constexpr (R == 1) {
+      *(f32x4 *)at = v[u];
+    } else {
+      *(f32x2 *)at = f32x2{v[u].x, v[u].y};
+      if (second) *(f32x2 *)(at + N) = f32x2{v[u].z, v[u].w};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sq[i / C] += (double)v[u][i] * (double)v[u][i];
+  }
+  double rms[R];
+  if (norm.kind == kNormRms) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) sq[r] += __shfl_xor(sq[r], o);
+      if ((threadIdx.x & 63) == 0) red[r][threadIdx.x >> 6] = sq[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      double total = 0.0;
+      for (int w = 0; w < (int)blockDim.x >> 6; ++w) total += red[r][w];
+      rms[r] = sqrt(total / (double)N + norm.eps);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kMost; ++u) {
+    const int col = C * (threadIdx.x + u * blockDim.x);
+    if (col >= N) continue;
+    f32x4 n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float gamma = norm.gamma ? norm.gamma[col + i % C] : 1.f;
+      n[i] = norm.kind == kNormRms ? (float)(((double)v[u][i] / rms[i / C]) * (double)gamma)
+                                   : __fadd_rn(__fmul_rn(tanhf(__fmul_rn(norm.alpha, v[u][i])), gamma), norm.beta[col + i % C]);
+    }
+    float *out = norm.rows + (long long)row * N + col;
+    if constexpr (R == 1) {
+      *(f32x4 *)out = n;
+    } else {
+      *(f32x2 *)out = f32x2{n.x, n.y};
+      if (second) *(f32x2 *)(out + N) = f32x2{n.z, n.w};
+    }
+  }
 }
 
 // Any shape (K or N not a multiple of 4, unaligned rows): one thread per element of y, W read
@@ -1111,6 +1227,15 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[6] = p.mfma && K % step_k(p) != 0;
 }
 
+// (the norm of a row takes a workgroup of up to 1024 threads, two registers of four each; rows and their pairs along the grid's second
+// dimension, which ends at 65535)
+bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
+  if (!p.mfma || p.pieces <= 1) return false;
+  const bool pairs = !(p.few && p.parts == 1) && !(p.parts == 1 && p.mb == 4);
+  if (next.swiglu) return !next.norm.rows && N % 8 == 0 && T <= 65535;
+  return N % 4 == 0 && N / (pairs ? 2 : 4) <= 2048;
+}
+
 GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
   GemmPlan p = {};
   p.parts = w_bf16 ? 1 : 3;
@@ -1185,54 +1310,66 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
 
 namespace {
 
+// The kernel that adds the pieces; a lane of the product holds COLUMNS neighbouring columns.
+template <int COLUMNS>
+hipError_t launch_sum(const GemmArgs &g, const PieceShape &s, const GemmNext &next, hipStream_t stream) {
+  constexpr int R = COLUMNS == 2 ? 2 : 1, C = 4 / R;
+  const int N = next.swiglu ? g.N / 2 : g.N, quads = (N + C - 1) / C, rows = (g.T + R - 1) / R;
+  if (next.norm.rows) {
+    const int threads = quads < 1024 ? (quads + 63) / 64 * 64 : 1024;
+    hipLaunchKernelGGL((sgemm_sum_norm_kernel<COLUMNS>), dim3((unsigned)rows), dim3(threads), 0, stream, g, s, next.norm);
+    return hipGetLastError();
+  }
+  const int threads = quads < 256 ? (quads + 63) / 64 * 64 : 256;
+  const dim3 grid((unsigned)((quads + threads - 1) / threads), (unsigned)rows);
+  if (next.swiglu)
+    hipLaunchKernelGGL((sgemm_sum_kernel<COLUMNS, true>), grid, dim3(threads), 0, stream, g, s);
+  else
+    hipLaunchKernelGGL((sgemm_sum_kernel<COLUMNS, false>), grid, dim3(threads), 0, stream, g, s);
+  return hipGetLastError();
+}
+
 template <int WM, int WN, int MB, int NB, int PARTS>
-hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups), block(64 * WM * WN);
   if (g.K % TK != 0)
     hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true>), grid, block, 0, stream, g);
   else
     hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false>), grid, block, 0, stream, g);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !g.pieces) return e;
-  const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL((sgemm_reduce_kernel<WM, WN, MB, NB>), dim3((unsigned)tiles * 4 * MB * NB), block, 0, stream, g, tiles);
-  return hipGetLastError();
+  return e != hipSuccess || !g.pieces ? e : launch_sum<NB>(g, PieceShape{32 * WM * MB, 32 * WN * NB, 32 * MB, WN, 64 * WM * WN}, next, stream);
 }
 
-hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
   if (g.K % kFewStep != 0)
     hipLaunchKernelGGL((sgemm_few_kernel<true>), grid, dim3(256), 0, stream, g);
   else
     hipLaunchKernelGGL((sgemm_few_kernel<false>), grid, dim3(256), 0, stream, g);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !g.pieces) return e;
-  const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL((sgemm_reduce_kernel<1, 2, 1, 2>), dim3((unsigned)tiles * 8), dim3(128), 0, stream, g, tiles);
-  return hipGetLastError();
+  return e != hipSuccess || !g.pieces ? e : launch_sum<2>(g, PieceShape{32, 128, 32, 2, 128}, next, stream);
 }
 
 template <int MB, int KG>
-hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, hipStream_t stream) {
+hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
   if (g.K % (16 * KG) != 0)
     hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, true>), grid, dim3(512), 0, stream, g);
   else
     hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, false>), grid, dim3(512), 0, stream, g);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !g.pieces) return e;
-  const int tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL((sgemm_reduce_kernel<1, 8 / KG, MB, 1>), dim3((unsigned)tiles * 4 * MB), dim3(512 / KG), 0, stream, g, tiles);
-  return hipGetLastError();
+  return e != hipSuccess || !g.pieces ? e : launch_sum<1>(g, PieceShape{32 * MB, 256 / KG, 0, 0, 0}, next, stream);
 }
 
 }  // namespace
 
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
                        unsigned *flags, int *error, int T, int K, int N, const GemmPlan &p, hipStream_t stream,
-                       unsigned *flag_set, int spin_limit, const float *bias, Activation act) {
+                       unsigned *flag_set, int spin_limit, const float *bias, Activation act, const GemmNext &next) {
+  if ((next.swiglu || next.norm.rows) && !gemm_takes_next(p, T, N, next)) return hipErrorInvalidValue;
   if (!x || !w || !y || T < 1 || K < 1 || N < 1 || x_stride < K) return hipErrorInvalidValue;
-  const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias) & 15);
+  const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias | (uintptr_t)next.norm.rows) & 15);
+  if (!aligned && (next.swiglu || next.norm.rows)) return hipErrorInvalidValue;
   if (!p.mfma || !aligned) {
     hipLaunchKernelGGL(sgemm_plain_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)(T < 65535 ? T : 65535)), dim3(256), 0, stream, x,
                        x_stride, w, y, res, T, K, N, bias, act);
@@ -1263,13 +1400,13 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   g.quota = p.quota;
   g.pieces = p.pieces > 1 ? p.pieces : 0;
   if (p.parts == 1) {
-    if (p.few && p.kg == 4) return launch_stream<1, 4>(g, p, stream);
-    if (p.few) return p.mb == 1 ? launch_stream<1, 2>(g, p, stream) : p.mb == 2 ? launch_stream<2, 2>(g, p, stream) : launch_stream<3, 2>(g, p, stream);
-    return p.mb == 4 ? launch_tiles<4, 2, 2, 4, 1>(g, p, stream) : launch_tiles<2, 4, 2, 2, 1>(g, p, stream);
+    if (p.few && p.kg == 4) return launch_stream<1, 4>(g, p, next, stream);
+    if (p.few) return p.mb == 1 ? launch_stream<1, 2>(g, p, next, stream) : p.mb == 2 ? launch_stream<2, 2>(g, p, next, stream) : launch_stream<3, 2>(g, p, next, stream);
+    return p.mb == 4 ? launch_tiles<4, 2, 2, 4, 1>(g, p, next, stream) : launch_tiles<2, 4, 2, 2, 1>(g, p, next, stream);
   }
-  if (p.few) return launch_few(g, p, stream);
-  if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4, 2, 3>(g, p, stream) : launch_tiles<2, 4, 2, 2, 3>(g, p, stream);
-  return launch_tiles<2, 2, 2, 2, 3>(g, p, stream);
+  if (p.few) return launch_few(g, p, next, stream);
+  if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4, 2, 3>(g, p, next, stream) : launch_tiles<2, 4, 2, 2, 3>(g, p, next, stream);
+  return launch_tiles<2, 2, 2, 2, 3>(g, p, next, stream);
 }
 
 }  // namespace shainet

@@ -6,6 +6,19 @@
 
 namespace shainet {
 
+// What happens to y next, where a kernel of its own adds the pieces of a product's tiles (GemmPlan::pieces > 1).
+struct NextNorm {
+  int kind = 0;          // kNorm*
+  const float *gamma = nullptr, *beta = nullptr;
+  float alpha = 0.f;
+  double eps = 0.0;
+  float *rows = nullptr;  // [T, N]: the norm of y's rows goes there (null: none)
+};
+struct GemmNext {
+  NextNorm norm;
+  bool swiglu = false;  // N = gate | up, and y is [T, N / 2]: silu(gate) * up
+};
+
 struct GemmPlan {
   bool mfma;              // false: K, N or the row stride of x is not a multiple of 4 -> the plain kernel
   bool few;               // tiles of 32 rows and 128 columns, K steps of 32 (parts 1: see kg)
@@ -34,6 +47,9 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]);  // shainet_hip_descr
 // words of their own, instead of flags, and a wait ends after spin_limit polls); null / 0 otherwise.
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
                        unsigned *flags, int *error, int T, int K, int N, const GemmPlan &p, hipStream_t stream,
-                       unsigned *flag_set = nullptr, int spin_limit = 0, const float *bias = nullptr, Activation act = Activation());
+                       unsigned *flag_set = nullptr, int spin_limit = 0, const float *bias = nullptr, Activation act = Activation(),
+                       const GemmNext &next = GemmNext());
+// Whether the product's last launch does that, too.
+bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next);
 
 }  // namespace shainet

@@ -74,7 +74,7 @@ struct Hgrn2 : Mixer {
   }
   Hgrn2 *hgrn2() override { return this; }
 
-  int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache) override {
+  int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache, Handover *next = nullptr) override {
     const int d = d_model, vw = cfg.heads * cfg.vdim;
     Hgrn2Plan plan;
     if (!plan_hgrn2(T, cfg.heads, cfg.dim, cfg.vdim, plan)) return fail(SHAINET_HIP_ERR_ARGUMENT, "too many rows in one call");
@@ -104,6 +104,7 @@ struct Hgrn2 : Mixer {
     if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("hgrn2 launch: ") + hipGetErrorString(e));
     if (!no_cache) rows += T;
     Fused post;
+    post.next = next;
     post.w_bf16 = w.w_o_bf16;
     if (residual) {
       post.epilogue = kGemvResidual;

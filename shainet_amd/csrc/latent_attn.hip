@@ -148,7 +148,7 @@ void latent_attn_share_error_word(LatentAttn *l, int *word) {
 }
 
 int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const Fused &pre, const float *residual,
-                        bool no_cache) {
+                        bool no_cache, Handover *next) {
   const LatentShape &sh = l->sh;
   LatentWeights &w = *l->w;
   shainet_attn_ctx *ctx = l->ctx;
@@ -229,6 +229,7 @@ int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const 
     cache->len[0] += T;
   }
   Fused post;
+  post.next = next;
   if (residual) {
     post.epilogue = kGemvResidual;
     post.res = residual;

@@ -42,6 +42,6 @@ void latent_attn_share_error_word(LatentAttn *l, int *word);
 // out = (residual +) mixer(pre(x)), T rows on the device, appended behind the cached ones; no_cache:
 // the rows attend among themselves from position 0 and the cache stays as it is
 int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const Fused &pre, const float *residual,
-                        bool no_cache);
+                        bool no_cache, Handover *next = nullptr);
 
 }  // namespace shainet

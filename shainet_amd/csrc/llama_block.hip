@@ -123,7 +123,8 @@ void set_vec(std::vector<float> &v, bool &has, const float *src, int n) {
 // position 0 over the rows of this call alone; they go through a scratch cache
 // that is empty again afterwards, and the block's own cache is not touched.
 int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out, const Fused &pre = Fused(),
-                        const float *residual = nullptr, bool no_cache = false, const AheadRows *ahead = nullptr) {
+                        const float *residual = nullptr, bool no_cache = false, const AheadRows *ahead = nullptr,
+                        Handover *next = nullptr) {
   // ahead: the transposed gate | up weights that the block's next product but one will read
   if (!l->w_qkv) return fail(SHAINET_HIP_ERR_ARGUMENT, "weights not set");
   int rc = ensure_context(l);
@@ -192,6 +193,7 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     l->cache_len = total_len;
   }
   Fused post;
+  post.next = next;
   post.w_bf16 = l->w_o_bf16;
   if (residual) {
     post.epilogue = kGemvResidual;
@@ -362,8 +364,8 @@ struct LatentMixer : Mixer {
   int *error_word() override { return shainet_attn_error_word(latent_attn_context(l)); }
   void share_error_word(int *word) override { latent_attn_share_error_word(l, word); }
   Projector &projector() override { return latent_attn_projector(l); }
-  int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache) override {
-    return latent_attn_forward(l, x, T, out, pre, residual, no_cache);
+  int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache, Handover *next = nullptr) override {
+    return latent_attn_forward(l, x, T, out, pre, residual, no_cache, next);
   }
   int reserve(int positions) override { return latent_attn_reserve(l, positions); }
   int clear() override { return shainet_kv_cache_clear(cache(), -1); }
@@ -500,6 +502,16 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
   // h = x + attention_cached_cpu(@norm1.forward(x))
   Fused n1;
   w.norm1.apply(n1, b->eps);
+  // The norms between products ride in the launch that adds a product's pieces, where there is one: this block's second in the
+  // mixer's last, the next block's first in the last of this one.
+  Handover *const behind = carry && carry->next.norm ? &carry->next : nullptr;
+  Handover second;
+  second.norm = &w.norm2;
+  second.eps = b->eps;
+  if (carry) {
+    n1.normed = carry->normed;
+    carry->normed = nullptr;
+  }
   Fused gate;
   w.norm2.apply(gate, b->eps);
   gate.epilogue = kGemvSwiglu;
@@ -511,7 +523,7 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
     gate.w_t_has_gamma = gate.w_t && ride;
   }
   if (b->mixer) {
-    rc = b->mixer->forward(x, T, h, n1, x, no_cache);
+    rc = b->mixer->forward(x, T, h, n1, x, no_cache, ff ? &second : behind);
   } else {
     // One row: the attention launch leaves the memory system idle while it waits on its chain of
     // dependent loads, and takes along workgroups that read the first rows of the gate | up
@@ -519,25 +531,34 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
     // slow the attention's own chain down by more than the product gains)
     static const int ahead_wgs = getenv("SHAINET_HIP_READ_AHEAD_WGS") ? atoi(getenv("SHAINET_HIP_READ_AHEAD_WGS")) : 128;
     const AheadRows ahead = {gate.w_t, d, ff, ahead_wgs};
-    rc = attn_forward_device(b->attn, x, T, h, n1, x, no_cache, &ahead);
+    rc = attn_forward_device(b->attn, x, T, h, n1, x, no_cache, &ahead, ff ? &second : behind);
   }
+  if (!ff && behind) carry->normed = behind->rows;
   if (rc || !ff) return rc;
+  gate.normed = second.rows;
   // hidden = silu(normed2 * gate_proj) * (normed2 * up_proj), normed2 = @norm2.forward(h)
   if ((rc = proj.project(h, d, w.gate_up, b->hidden.p, T, d, ff, stream, gate))) return rc;
   // out = h + hidden * down_proj
   Fused down;
   down.epilogue = kGemvResidual;
   down.res = h;
+  down.next = behind;
   down.w_bf16 = w.down_bf16;
   if (gemvt_takes(T, ff, d, down.epilogue, down.norm)) down.w_t = transposed_twin(&w.down_t, &w.down_t_stale, w.down, ff, d, stream);
-  return proj.project(b->hidden.p, ff, w.down, out, T, ff, d, stream, down);
+  rc = proj.project(b->hidden.p, ff, w.down, out, T, ff, d, stream, down);
+  if (behind) carry->normed = behind->rows;
+  return rc;
 }
 
 }  // namespace
 
 // used by the model (llama_model.hip)
 int shainet_llama_block_forward_device(shainet_llama_block *b, const float *x, int T, float *out, bool no_cache, BlockCarry *carry) {
-  return block_forward_device(b, x, T, out, no_cache, b->wrapped ? carry : nullptr);
+  return block_forward_device(b, x, T, out, no_cache, carry);
+}
+const NormWeights *shainet_llama_block_first_norm(const shainet_llama_block *b, double *eps) {
+  *eps = b->eps;
+  return b->wrapped ? nullptr : &b->w->norm1;
 }
 int shainet_llama_block_join_carry(shainet_llama_block *b, const BlockCarry &carry, float *x, int T) {
   return join(b, x, carry.y, carry.post, x, nullptr, nullptr, nullptr, nullptr, T, true, b->mixer->stream());

@@ -65,10 +65,22 @@ struct WrappedBlockBuffers {
 };
 WrappedBlockBuffers shainet_llama_block_wrapped_buffers(shainet_llama_block *b);
 shainet::Mixer *shainet_llama_block_mixer_of(shainet_llama_block *b);  // null: the grouped-query attention of a LLaMA block
+namespace shainet {
+// The norm of what reads a product's result next, for the product to take along where its last launch holds whole rows.
+struct Handover {
+  const NormWeights *norm = nullptr;
+  double eps = 0.0;
+  const float *rows = nullptr;  // set by the product: the result's rows behind the norm, dense; null: the norm is still to be taken
+};
+
+}
 // The result of such a block's last sublayer that has not joined the residual yet: the next block's first launch
 // does it (shainet_llama_block_forward_device), or shainet_llama_block_join_carry behind the last block.
 struct BlockCarry {
   const float *y = nullptr, *post = nullptr;
+  // other blocks: the rows behind the block's first norm, if the block before has taken it; and the next block's first norm
+  const float *normed = nullptr;
+  shainet::Handover next;
 };
 // A model without blocks yet, and one more block for it (which it then owns), for loaders of designs
 // whose layers are not all alike.
@@ -122,6 +134,8 @@ struct Fused {
   const float *w_t = nullptr;
   bool w_bf16 = false;  // every value of W is a bf16 number: half the MFMAs of many rows have nothing to add
   bool any_few_rows = false;  // up to 16 rows run as the split GEMV, not only the ones it is the faster product for
+  const float *normed = nullptr;  // [T, K]: the rows of x behind the norm, where an earlier product handed them over (more than a few rows only)
+  Handover *next = nullptr;       // nullable; for kGemvPlain and kGemvResidual
   bool w_t_has_gamma = false;  // the rows of w_t were made with gamma multiplied in: the norm's factor 1 / rms is all that is left to apply
 };
 
@@ -144,7 +158,8 @@ struct NormWeights {
 // (decode; few_rows) run as one hand-written split GEMV with the norm and the epilogue
 // inside; more rows run as the MFMA product of gemm_kernel.hip (the counterpart of
 // the reference's cuBLAS SGEMM, cuda.cr:237-247) after the separate norm kernel,
-// with the residual add in its epilogue and the SwiGLU activation as a kernel of its own.
+// with the residual add in its epilogue.  The SwiGLU activation and the norm of what comes next ride in the kernel that adds
+// the pieces of the product's tiles where there is one, and are kernels of their own elsewhere.
 struct Projector {
   // Whether T rows run as the split GEMV.  Up to 4 do.  It streams the weights once for up to 16, but its multiply-adds
   // are the vector ALU's, and from 5 rows on the MFMA product is the faster one (a prompt of a 2048 wide model of 4
@@ -154,7 +169,7 @@ struct Projector {
   // products are MFMA's, 68 | 72 | 81 | 93 this way; for 8 rows 84 | 80 | 99 | 98 and 77 | 77 | 93 | 94; from 10 rows on
   // the MFMA product is the faster one at any size (width 128, 12 rows: 80, and 85 with the smallest as the split GEMV).
   static bool few_rows(int T, int K, int N, long long x_stride);
-  DevF scratch, normed, wide;
+  DevF scratch, normed, wide, handed;
   // split products: a word per partial that says when it is complete (zero between launches)
   unsigned *flags = nullptr;
   size_t flags_cap = 0;
@@ -173,7 +188,7 @@ struct Projector {
   int reserve_flags(size_t n_flags, hipStream_t stream);
   // res != nullptr: y = res + x W
   int gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N, hipStream_t stream, bool w_bf16,
-           const float *res = nullptr, const float *bias = nullptr, Activation act = Activation());
+           const float *res = nullptr, const float *bias = nullptr, Activation act = Activation(), bool swiglu = false, Handover *next = nullptr);
 };
 
 // Replace *dst (device, hipMalloc'ed or null) by a copy of n host floats.

@@ -25,6 +25,7 @@ using namespace shainet;
 
 // llama_block.hip
 int shainet_llama_block_forward_device(shainet_llama_block *b, const float *x, int T, float *out, bool no_cache, BlockCarry *carry);
+const shainet::NormWeights *shainet_llama_block_first_norm(const shainet_llama_block *b, double *eps);  // null: taken by the block itself
 int shainet_llama_block_join_carry(shainet_llama_block *b, const BlockCarry &carry, float *x, int T);
 bool shainet_llama_block_keeps_state(const shainet_llama_block *b);
 int shainet_llama_block_save_state(shainet_llama_block *b);
@@ -380,8 +381,11 @@ int run_device_tokens(shainet_llama_model *m, const int *d_tokens, int T, bool n
                                   : launch_embed(m->embedding, d_tokens, m->act[0].p, T, d, m->stream, m->embedding_scale, positions);
     if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("embedding launch: ") + hipGetErrorString(e));
     BlockCarry carry;
-    for (shainet_llama_block *b : m->blocks) {
+    for (size_t i = 0; i < m->blocks.size(); ++i) {
+      shainet_llama_block *b = m->blocks[i];
       if ((rc = shainet_llama_block_set_stream(b, m->stream))) return rc;
+      carry.next = Handover();
+      if (i + 1 < m->blocks.size()) carry.next.norm = shainet_llama_block_first_norm(m->blocks[i + 1], &carry.next.eps);
       if ((rc = shainet_llama_block_forward_device(b, m->act[cur].p, T, m->act[cur ^ 1].p, no_cache, &carry))) return rc;
       cur ^= 1;
     }

@@ -21,7 +21,8 @@ struct Mixer {
   virtual Projector &projector() = 0;
   // out = (residual +) mixer(pre(x)), T rows on the device behind the ones before; no_cache: the rows see
   // each other from position 0 and nothing of what is kept changes.  Asynchronous on the stream.
-  virtual int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache) = 0;
+  // next (nullable): the norm that follows, for the mixer's last product.
+  virtual int forward(const float *x, int T, float *out, const Fused &pre, const float *residual, bool no_cache, Handover *next = nullptr) = 0;
   virtual int reserve(int positions) = 0;
   virtual int clear() = 0;
   virtual int len() = 0;

@@ -132,14 +132,35 @@ int Projector::reserve_flags(size_t n_flags, hipStream_t stream) {
 }
 
 // y = (res +) x W with the library's own MFMA kernel; res == y is allowed.
+// swiglu: W is gate | up and y [T, N / 2].
 int Projector::gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
-                    hipStream_t stream, bool w_bf16, const float *res, const float *bias, Activation act) {
+                    hipStream_t stream, bool w_bf16, const float *res, const float *bias, Activation act, bool swiglu, Handover *next) {
   const GemmPlan p = plan_gemm(T, K, N, x_stride, w_bf16);
+  const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias) & 15);
+  GemmNext also;
+  also.swiglu = swiglu;
+  float *result = y;
+  if (swiglu && !(aligned && gemm_takes_next(p, T, N, also))) {
+    if (!wide.reserve((size_t)T * N)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
+    result = wide.p;
+    also.swiglu = false;
+  }
+  // (without the memory for them the rows are normed in front of the next product, as after one that adds no pieces)
+  if (next && next->norm->kind != kNormNone && !bias && aligned && gemm_takes_next(p, T, N, also) && handed.reserve((size_t)T * N)) {
+    also.norm.kind = next->norm->kind;
+    also.norm.gamma = next->norm->gamma;
+    also.norm.beta = next->norm->beta;
+    also.norm.alpha = next->norm->alpha;
+    also.norm.eps = next->eps;
+    also.norm.rows = handed.p;
+    next->rows = handed.p;
+  }
   if (!scratch.reserve(p.partial_floats)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   if (int rc = reserve_flags(p.flag_words, stream)) return rc;
   if (p.flag_words && !error) return llama_fail(SHAINET_HIP_ERR_RUNTIME, "the projector has no error word");
-  hipError_t e = launch_gemm(x, x_stride, w, y, res, scratch.p, flags, error, T, K, N, p, stream,
-                             lose_marks ? flags + flags_cap : nullptr, lose_marks ? 2000 : 0, bias, act);
+  hipError_t e = launch_gemm(x, x_stride, w, result, res, scratch.p, flags, error, T, K, N, p, stream,
+                             lose_marks ? flags + flags_cap : nullptr, lose_marks ? 2000 : 0, bias, act, also);
+  if (e == hipSuccess && swiglu && !also.swiglu) e = launch_swiglu_act(wide.p, y, T, N / 2, stream);
   if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("gemm launch: ") + hipGetErrorString(e));
   return SHAINET_HIP_OK;
 }
@@ -152,6 +173,7 @@ bool Projector::few_rows(int T, int K, int N, long long x_stride) {
 int Projector::project(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
                        hipStream_t stream, const Fused &f) {
   const bool swiglu = f.epilogue == kGemvSwiglu;
+  if (f.next) f.next->rows = nullptr;
   if (f.epilogue == kGemvQkvPrep && (!f.prep || T > 16 || (N & 3)))
     return llama_fail(SHAINET_HIP_ERR_ARGUMENT, "the fused q | k | v epilogue takes at most 16 rows");
   if (f.w_t && gemvt_takes(T, K, N, f.epilogue, f.norm, f.prep) && !(((uintptr_t)x | (uintptr_t)f.gamma | (uintptr_t)f.beta) & 15)) {
@@ -228,11 +250,15 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
       return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("gemv launch: ") + hipGetErrorString(e));
     return SHAINET_HIP_OK;
   }
-  // many rows: norm kernel, MFMA product (the residual rides in its epilogue), activation kernel
+  // many rows: norm kernel, MFMA product (the residual rides in its epilogue), activation kernel; the latter and the next norm
+  // where the pieces of the product's tiles are added, if they are
   const float *xin = x;
   long long xs = x_stride;
   hipError_t e = hipSuccess;
-  if (f.norm) {
+  if (f.norm && f.normed) {
+    xin = f.normed;
+    xs = K;
+  } else if (f.norm) {
     if (!normed.reserve((size_t)T * K)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     e = f.norm == kNormDynTanh ? launch_dyn_tanh(x, x_stride, f.gamma, f.beta, f.alpha, normed.p, T, K, stream)
                                : launch_rmsnorm(x, x_stride, f.gamma, normed.p, T, K, f.eps, stream);
@@ -240,22 +266,16 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
     xin = normed.p;
     xs = K;
   }
-  if (swiglu) {
-    if (!wide.reserve((size_t)T * 2 * N)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-    int rc = gemm(xin, xs, w, wide.p, T, K, 2 * N, stream, f.w_bf16);
-    if (rc) return rc;
-    e = launch_swiglu_act(wide.p, y, T, N, stream);
-    if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("epilogue launch: ") + hipGetErrorString(e));
-    return SHAINET_HIP_OK;
-  }
+  if (swiglu) return gemm(xin, xs, w, y, T, K, 2 * N, stream, f.w_bf16, nullptr, nullptr, Activation(), true);
   return gemm(xin, xs, w, y, T, K, N, stream, f.w_bf16, f.epilogue == kGemvResidual ? f.res : nullptr,
-              f.epilogue == kGemvBias ? f.bias : nullptr, f.act);
+              f.epilogue == kGemvBias ? f.bias : nullptr, f.act, false, f.next);
 }
 
 void Projector::release() {
   scratch.release();
   normed.release();
   wide.release();
+  handed.release();
   if (flags) (void)hipFree(flags);
   flags = nullptr;
   flags_cap = 0;

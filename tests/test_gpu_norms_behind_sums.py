@@ -1,0 +1,102 @@
+"""Norms and SwiGLU in the launch that adds the pieces of a product's tiles, against 64 bits: two blocks, so that the norm between
+them is handed over, too."""
+import numpy as np
+import pytest
+
+import tutilorn_model as tm
+from test_gpu_bf16_weights import bf16, write
+from test_gpu_tutilorn import Pair, close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import shainet_amd as sa
+
+    assert sa.HIP.fully_available(), "no gfx950 device or libshainet_hip_kernels.so missing"
+    return sa
+
+
+H, KV, HD, EPS, THETA = 16, 8, 64, 1e-5, 1e4
+
+
+def llama(d, ff, vocab, seed):
+    cfg = {"model_type": "llama", "vocab_size": vocab, "hidden_size": d, "num_attention_heads": H, "num_hidden_layers": 2,
+           "intermediate_size": ff, "num_key_value_heads": KV, "head_dim": HD, "tie_word_embeddings": False, "rms_norm_eps": EPS,
+           "rope_theta": THETA}
+    r = np.random.default_rng(seed)
+
+    def matrix(o, i):
+        return bf16(r.standard_normal((o, i), np.float32) * np.float32(i ** -0.5))
+
+    w = {"model.embed_tokens.weight": bf16(r.standard_normal((vocab, d), np.float32)), "lm_head.weight": matrix(vocab, d)}
+    for p in ("model.layers.0.", "model.layers.1."):
+        for name, o, i in (("self_attn.q_proj", H * HD, d), ("self_attn.k_proj", KV * HD, d), ("self_attn.v_proj", KV * HD, d),
+                           ("self_attn.o_proj", d, H * HD), ("mlp.gate_proj", ff, d), ("mlp.up_proj", ff, d), ("mlp.down_proj", d, ff)):
+            w[p + name + ".weight"] = matrix(o, i)
+        for name in ("input_layernorm", "post_attention_layernorm"):
+            w[p + name + ".weight"] = bf16(1 + 0.3 * r.standard_normal(d, np.float32))
+    w["model.norm.weight"] = bf16(1 + 0.3 * r.standard_normal(d, np.float32))
+    return cfg, w
+
+
+def logits_in_64_bits(w, tokens):
+    import torch
+
+    w = {n: torch.from_numpy(np.ascontiguousarray(a)).cuda().double() for n, a in w.items()}
+    T = len(tokens)
+    norm = lambda x, g: x / (x * x).mean(-1, keepdim=True).add(EPS).sqrt() * g  # noqa: E731
+    freq = torch.tensor([1.0 / THETA ** (2.0 * i / HD) for i in range(HD // 2)], dtype=torch.float64, device="cuda").float()
+    a = (torch.arange(T, device="cuda").float()[:, None] * freq).double()[:, None]
+
+    def turn(x):
+        u, v = x[..., :HD // 2], x[..., HD // 2:]
+        return torch.cat([u * a.cos() - v * a.sin(), v * a.cos() + u * a.sin()], -1)
+
+    hidden = torch.ones(T, T, dtype=torch.bool, device="cuda").triu(1)
+    x = w["model.embed_tokens.weight"][torch.from_numpy(tokens).cuda()]
+    for p in ("model.layers.0.", "model.layers.1."):
+        g = lambda n: w[p + n + ".weight"]  # noqa: E731
+        h = norm(x, g("input_layernorm"))
+        q, k, v = ((h @ g("self_attn.%s_proj" % n).T).view(T, -1, HD) for n in "qkv")
+        q, k = turn(q), turn(k)
+        heads = [torch.softmax((q[:, i] @ k[:, i * KV // H].T / HD ** 0.5).masked_fill(hidden, -np.inf), -1) @ v[:, i * KV // H] for i in range(H)]
+        x = x + torch.cat(heads, 1) @ g("self_attn.o_proj").T
+        h = norm(x, g("post_attention_layernorm"))
+        x = x + (torch.nn.functional.silu(h @ g("mlp.gate_proj").T) * (h @ g("mlp.up_proj").T)) @ g("mlp.down_proj").T
+    return (norm(x, w["model.norm.weight"]) @ w["lm_head.weight"].T).cpu().numpy()
+
+
+# tiles of a row at a time; of pairs of rows, the last one alone; of 256 x 256; more columns than a workgroup holds; no whole
+# registers of gate | up
+@pytest.mark.parametrize("d,ff,T,short,tile", [
+    (1024, 4096, 45, True, (32, 64)), (1024, 4096, 33, False, (32, 128)), (1024, 4096, 777, True, (128, 256)),
+    (2052, 4096, 245, False, (128, 128)), (1028, 8200, 1999, True, (256, 256)), (2308, 8192, 999, False, (256, 256)),
+    (4100, 2048, 40, False, (32, 128)), (1024, 2050, 45, True, None)])
+def test_norms_and_swiglu_behind_sums(hip, tmp_path, d, ff, T, short, tile):
+    """Against 64 bits: sums of up to 8200 terms round a row by 8200^0.5 times 2^-24 at random, and what they hand on as much
+    again; a row normed by another's factor, or not at all, is off by itself."""
+    if tile:
+        plan = hip.hip.describe_matmul(T, ff, d, bf16_weights=short)
+        assert plan["pieces"] > 1 and plan["tile"] == tile, plan
+    cfg, w = llama(d, ff, 260, d + T)
+    if not short:
+        for n in w:
+            if w[n].ndim == 2:
+                w[n] = w[n] * np.float32(1 + 2.0 ** -12)
+    tokens = np.random.default_rng(1).integers(0, 260, T)
+    model = hip.HFLoader.load_model(write(tmp_path / "m", cfg, w, lambda n: short, nudge=False))
+    got, want = model.run_rows(tokens, range(T)).astype(np.float64), logits_in_64_bits(w, tokens)
+    off = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert off.max() <= 2 * 8200 ** 0.5 * 2.0 ** -24, off.max()
+
+
+@pytest.mark.parametrize("T", [60, 301])
+def test_dynamic_tanh_behind_sums(hip, tmp_path, T):
+    cfg = tm.config([tm.layer(tm.mixer(heads=8, dim=64, rot_dim=32, vdim=64, kv_rank=128, q_rank=128, window=50), 2048) for _ in range(2)],
+                    vocab=260, width=512)
+    assert hip.hip.describe_matmul(T, 2048, 512, bf16_weights=True)["pieces"] > 1
+    p = Pair(hip, tmp_path, cfg)
+    ids = [int(t) for t in np.random.default_rng(2).integers(0, 260, T)]
+    close(p.model.run_rows(ids, range(T)), p.logits(ids), 2e-5)
