@@ -5,6 +5,7 @@
 #include <hip/hip_ext.h>
 
 #include "activation.hpp"
+#include "residual_kernels.hpp"
 
 // A kernel launch that hands the kernel's own first and last clock reading to two events when
 // there are any (hipExtLaunchKernel), and is a plain launch, as a caller's stream capture may
@@ -241,6 +242,7 @@ struct GemvArgs {
   int epilogue;
   int rows_per_wave;     // filled in by launch_gemv
   GemvPrep prep;         // kGemvQkvPrep only (y is not written then)
+  ResidualArgs join;     // launch_gemvt, join.x not null: x is the row that this makes (join.h, which is not written); no norm
 };
 struct GemvPlan {
   int rows_per_instr;     // 1: 256-column tiles; 4: 64-column tiles, four rows of W per load instruction
@@ -258,6 +260,8 @@ hipError_t launch_gemv(const GemvArgs &a, const GemvPlan &p, hipStream_t stream)
 // kGemvQkvPrep epilogue, a.w: [(H + 2 KV) hd, K], where *prep asks for no QK-norm).
 bool gemvt_takes(int T, int K, int N, int epilogue, int norm, const GemvPrep *prep = nullptr);
 hipError_t launch_gemvt(const GemvArgs &a, hipStream_t stream);
+// Whether launch_gemvt takes a.join along (row_join_fits beside).
+bool gemvt_takes_join(int K, int N, int epilogue, int norm);
 
 // A pinned host int per context (block, model) that its kernels set when they give up a
 // bounded wait for other workgroups (null when it cannot be allocated); check_error_word,

@@ -21,9 +21,10 @@ struct Dense : FeedForward {
     for (float *p : {w.up, w.up_t, w.up_bias, w.down, w.down_t, w.down_bias})
       if (p) (void)hipFree(p);
   }
-  int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream) override {
+  int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream, const ResidualArgs *join) override {
     if (!hidden.reserve((size_t)T * ff)) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     Fused up;
+    up.join = join;
     up.epilogue = kGemvBias;
     up.bias = w.up_bias;
     up.act = w.act;
@@ -51,14 +52,15 @@ struct Moe : FeedForward {
                      w.shared_down_in})
       if (p) (void)hipFree(p);
   }
-  int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream) override {
+  int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream, const ResidualArgs *join) override {
     const MoeTensors t = {w.router, w.correction, w.gate_up, w.down, w.shared_gate_up, w.shared_down, w.gate_up_bf16, w.down_bf16};
     hipError_t e;
     if (T <= kMoeFewTokens) {
       if (!scratch.reserve(moe_few_floats(m, T))) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-      e = launch_moe_few(m, t, h, y, T, scratch.p, stream);
+      e = launch_moe_few(m, t, h, y, T, scratch.p, stream, join);
       return e == hipSuccess ? SHAINET_HIP_OK : fail(SHAINET_HIP_ERR_RUNTIME, std::string("expert launch: ") + hipGetErrorString(e));
     }
+    if (join) return fail(SHAINET_HIP_ERR_ARGUMENT, "one row only");
     constexpr int kAtOnce = 8192;  // tokens whose experts' rows are in memory together
     for (int t0 = 0; t0 < T; t0 += kAtOnce) {
       const int n = T - t0 < kAtOnce ? T - t0 : kAtOnce;

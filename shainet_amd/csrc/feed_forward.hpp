@@ -7,8 +7,9 @@ namespace shainet {
 
 struct FeedForward {
   virtual ~FeedForward() {}
-  // y = f(h), T rows of d_model, not the same buffer; proj: the block's
-  virtual int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream) = 0;
+  // y = f(h), T rows of d_model, not the same buffer; proj: the block's.  join (nullable; one row): h is still to be made by it,
+  // in the first launch where that takes it along.
+  virtual int forward(Projector &proj, const float *h, int T, float *y, hipStream_t stream, const ResidualArgs *join) = 0;
 };
 
 // y = act(h W_up + b_up) W_down + b_down

@@ -19,6 +19,7 @@
 //     (llama_block.cr:256-286, 332-344) on each head row where it is summed up.
 #include "attn_kernels.hpp"
 #include "prep_math.hpp"
+#include "row_join.hpp"
 
 #include <math.h>
 #include <stdint.h>
@@ -437,11 +438,15 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvArgs a) {
 // DYT: the prologue is Dynamic Tanh instead: x becomes tanh(alpha x) gamma + beta where it is staged.
 // TAIL: rows of a.K values, a multiple of 4 below 256 KV4; the pieces beyond are zeros (one row of 384 -> 1536, in
 // front of which the split product took 7.7 us: 3.9).
-template <int KV4, int NACC, int SP, bool MULTI, bool PREP = false, bool DYT = false, bool TAIL = false>
+// JOIN: x is the row between two sublayers of a block with norms around them, which each workgroup works out while its weights are on
+// their way (row_join.hpp).  As a launch of its own that row took 3.9 us of a decode step and the gap behind it 0.8, in
+// eight of 33 launches a token of four such layers; here 6.8 us for 4.5 + 3.9 (1024 -> 3072), 8.1 for 5.4 + 3.9 (1024 -> 4096).
+template <int KV4, int NACC, int SP, bool MULTI, bool PREP = false, bool DYT = false, bool TAIL = false, bool JOIN = false>
 __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   static_assert(!PREP || (NACC == 1 && SP == 1 && !MULTI), "the q | k | v epilogue: one row per wavefront");
   static_assert(!DYT || (SP == 1 && !PREP), "rows shared by two wavefronts come without a norm");
   static_assert(!TAIL || (SP == 1 && !PREP && !DYT), "odd row lengths: no norm or RMSNorm");
+  static_assert(!JOIN || (SP == 1 && !MULTI && !DYT && !TAIL && NACC == 1 && KV4 >= 4), "a whole row per workgroup");
   const bool rms_norm = !DYT && a.norm;
   // x: up to 2048 values stay in registers.  Longer (half) rows: a wavefront with one output reads
   // them again from memory (the L2), eight 16-byte pieces at a time, where they are used; one with
@@ -455,7 +460,7 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   constexpr bool XSH = !MULTI, XREG = !XSH && KV4 <= 8, XLDS = !XSH && !XREG;
   __shared__ __align__(16) float xs[XLDS ? 4 * 256 * KV4 : 4];
   __shared__ __align__(16) float xsh[XSH ? 256 * KV4 * SP : 4];
-  __shared__ float half_s[4], sq_s[4];
+  __shared__ float half_s[4], sq_s[4], join_s[JOIN ? 8 : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rpw = a.rows_per_wave;
   const int N = a.N;
@@ -492,7 +497,10 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   constexpr bool NORMS = SP == 1;  // (rows shared by two wavefronts come without the norm: gemvt_takes)
   f32x4 b_own[XSH && DYT ? XO : 1];  // its share of beta
   f32x4 x_own[XSH ? XO : 1], g_own[XSH && NORMS ? XO : 1];  // this thread's share of x (and gamma) on its way to LDS
-  if constexpr (XSH) {
+  JoinRow<JOIN ? XO : 1> row;
+  if constexpr (JOIN) {
+    row.request(a.join);
+  } else if constexpr (XSH) {
 #pragma unroll
     for (int i = 0; i < XO; ++i)
       x_own[i] = within(4 * threadIdx.x + 1024 * i) ? *(const f32x4 *)(a.x + 4 * threadIdx.x + 1024 * i) : kZero;
@@ -508,6 +516,11 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
   }
   if (live || PREP) load_row(wa, n0);
   if constexpr (XSH) {
+    if constexpr (JOIN) {
+      row.finish(a.join, join_s, blockIdx.x == 0);
+#pragma unroll
+      for (int i = 0; i < XO; ++i) x_own[i] = row.x[i];
+    }
     if constexpr (DYT) {
 #pragma unroll
       for (int i = 0; i < XO; ++i) x_own[i] = dyn_tanh4(x_own[i], a.alpha, g_own[i], b_own[i]);
@@ -793,8 +806,15 @@ bool gemvt_takes(int T, int K, int N, int epilogue, int norm, const GemvPrep *pr
   return epilogue == kGemvPlain || epilogue == kGemvResidual || epilogue == kGemvSwiglu || epilogue == kGemvBias;
 }
 
+bool gemvt_takes_join(int K, int N, int epilogue, int norm) {
+  return (K == 1024 || K == 2048) && N <= 32768 && !norm && (epilogue == kGemvPlain || epilogue == kGemvBias || epilogue == kGemvQkvPrep);
+}
+
 hipError_t launch_gemvt(const GemvArgs &args, hipStream_t stream) {
   GemvArgs a = args;
+  const bool join = a.join.x != nullptr;
+  if (join && (!gemvt_takes_join(a.K, a.N, a.epilogue, a.norm) || !row_join_fits(a.join) || a.join.d != a.K)) return hipErrorInvalidValue;
+  if (join) a.join.h = nullptr;
   const bool prep = a.epilogue == kGemvQkvPrep;
   if (!gemvt_takes(a.T, a.K, a.N, a.epilogue, a.norm, &a.prep) || !a.x || !a.w || (!a.y && !prep)) return hipErrorInvalidValue;
   if ((a.epilogue == kGemvResidual && !a.res) || (a.epilogue == kGemvBias && !a.bias)) return hipErrorInvalidValue;
@@ -808,11 +828,27 @@ hipError_t launch_gemvt(const GemvArgs &args, hipStream_t stream) {
     a.N = a.N / 2;  // pairs, two per workgroup
     a.rows_per_wave = 1;
     const dim3 pgrid((unsigned)((a.N + 1) / 2));
+    if (join) {
+      if (a.K == 1024)
+        hipLaunchKernelGGL((gemvt_kernel<4, 1, 1, false, true, false, false, true>), pgrid, dim3(256), 0, stream, a);
+      else
+        hipLaunchKernelGGL((gemvt_kernel<8, 1, 1, false, true, false, false, true>), pgrid, dim3(256), 0, stream, a);
+      return hipGetLastError();
+    }
     switch (a.K) {
       case 1024: hipLaunchKernelGGL((gemvt_kernel<4, 1, 1, false, true>), pgrid, dim3(256), 0, stream, a); break;
       case 2048: hipLaunchKernelGGL((gemvt_kernel<8, 1, 1, false, true>), pgrid, dim3(256), 0, stream, a); break;
       default: hipLaunchKernelGGL((gemvt_kernel<16, 1, 1, false, true>), pgrid, dim3(256), 0, stream, a); break;
     }
+    return hipGetLastError();
+  }
+  if (join) {
+    a.rows_per_wave = 1;
+    const dim3 jgrid((unsigned)((a.N + 3) / 4));
+    if (a.K == 1024)
+      hipLaunchKernelGGL((gemvt_kernel<4, 1, 1, false, false, false, false, true>), jgrid, dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL((gemvt_kernel<8, 1, 1, false, false, false, false, true>), jgrid, dim3(256), 0, stream, a);
     return hipGetLastError();
   }
   const bool two = a.epilogue == kGemvSwiglu;

@@ -427,10 +427,10 @@ int grouped_only(const shainet_llama_block *b, const char *what) {
 
 namespace {
 
-// One residual_kernels.hpp launch: (with y) the result y of a sublayer joins x; (with pre) what the next sublayer
-// reads, from conv's state if there is a convolution.
-int join(shainet_llama_block *b, const float *x, const float *y, const float *post, float *x_out, const float *pre,
-         const float *conv_w, ConvState *conv, float *h, int T, bool no_cache, hipStream_t stream) {
+// (with y) The result y of a sublayer joins x; (with pre) what the next sublayer reads, from conv's state if there is a
+// convolution.
+ResidualArgs joining(shainet_llama_block *b, const float *x, const float *y, const float *post, float *x_out, const float *pre,
+                     const float *conv_w, ConvState *conv, float *h, int T, bool no_cache) {
   ResidualArgs a = {};
   a.x = x;
   a.y = y;
@@ -451,13 +451,16 @@ int join(shainet_llama_block *b, const float *x, const float *y, const float *po
       conv->cur ^= 1;
     }
   }
+  return a;
+}
+int join(const ResidualArgs &a, hipStream_t stream) {
   const hipError_t e = launch_residual(a, stream);
   return e == hipSuccess ? SHAINET_HIP_OK : fail(SHAINET_HIP_ERR_RUNTIME, std::string("residual launch: ") + hipGetErrorString(e));
 }
 
 // x <- x + norm1b(mixer(conv1(norm1(x)))), then x <- x + norm2b(ff(conv2(norm2(x)))), where conv(h) = h + the
-// convolution.  Each arrow and what the next sublayer reads are one launch; carry takes the last one over
-// to the next block (BlockCarry).
+// convolution.  Each arrow and what the next sublayer reads are one launch, or for one row part of that sublayer's first
+// where it takes them along; carry takes the last one over to the next block (BlockCarry).
 int wrapped_forward_device(shainet_llama_block *b, const float *x, int T, float *out, bool no_cache, BlockCarry *carry) {
   BlockWeights &w = *b->w;
   const size_t n = (size_t)T * b->d_model;
@@ -465,20 +468,27 @@ int wrapped_forward_device(shainet_llama_block *b, const float *x, int T, float 
   if (!w.norm1.gamma || !w.post1) return fail(SHAINET_HIP_ERR_ARGUMENT, "weights not set");
   if (!b->h.reserve(n) || !b->y.reserve(n) || !b->joined.reserve(n) || !b->factors.reserve((size_t)T)) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   const bool carried = carry && carry->y;
-  int rc = join(b, x, carried ? carry->y : nullptr, carried ? carry->post : nullptr, b->joined.p, w.norm1.gamma, w.conv1, &b->conv[0],
-                b->h.p, T, no_cache, stream);
+  const ResidualArgs first = joining(b, x, carried ? carry->y : nullptr, carried ? carry->post : nullptr, b->joined.p, w.norm1.gamma, w.conv1,
+                                     &b->conv[0], b->h.p, T, no_cache);
   if (carry) carry->y = nullptr;
   const float *res = carried ? b->joined.p : x;
-  if (!rc) rc = b->mixer->forward(b->h.p, T, b->y.p, Fused(), nullptr, no_cache);
-  if (!rc && !w.ff) rc = join(b, res, b->y.p, w.post1, out, nullptr, nullptr, nullptr, nullptr, T, no_cache, stream);
+  Fused pre;
+  if (T == 1) pre.join = &first;
+  int rc = pre.join ? SHAINET_HIP_OK : join(first, stream);
+  if (!rc) rc = b->mixer->forward(b->h.p, T, b->y.p, pre, nullptr, no_cache);
+  if (!rc && !w.ff) rc = join(joining(b, res, b->y.p, w.post1, out, nullptr, nullptr, nullptr, nullptr, T, no_cache), stream);
   if (!rc && w.ff) {
-    rc = join(b, res, b->y.p, w.post1, out, w.norm2.gamma, w.conv2, &b->conv[1], b->h.p, T, no_cache, stream);
-    if (!rc) rc = w.ff->forward(b->mixer->projector(), b->h.p, T, b->y.p, stream);
+    // (a sublayer's result is read by the join behind it, and the feed-forward's last product writes the buffer again behind its
+    // first launch)
+    const ResidualArgs second = joining(b, res, b->y.p, w.post1, out, w.norm2.gamma, w.conv2, &b->conv[1], b->h.p, T, no_cache);
+    const ResidualArgs *const taken = T == 1 ? &second : nullptr;
+    if (!taken) rc = join(second, stream);
+    if (!rc) rc = w.ff->forward(b->mixer->projector(), b->h.p, T, b->y.p, stream, taken);
     if (!rc && carry) {
       carry->y = b->y.p;
       carry->post = w.post2;
     } else if (!rc) {
-      rc = join(b, out, b->y.p, w.post2, out, nullptr, nullptr, nullptr, nullptr, T, no_cache, stream);
+      rc = join(joining(b, out, b->y.p, w.post2, out, nullptr, nullptr, nullptr, nullptr, T, no_cache), stream);
     }
   }
   if (!rc && !no_cache) b->pos += T;
@@ -561,7 +571,7 @@ const NormWeights *shainet_llama_block_first_norm(const shainet_llama_block *b, 
   return b->wrapped ? nullptr : &b->w->norm1;
 }
 int shainet_llama_block_join_carry(shainet_llama_block *b, const BlockCarry &carry, float *x, int T) {
-  return join(b, x, carry.y, carry.post, x, nullptr, nullptr, nullptr, nullptr, T, true, b->mixer->stream());
+  return join(joining(b, x, carry.y, carry.post, x, nullptr, nullptr, nullptr, nullptr, T, true), b->mixer->stream());
 }
 bool shainet_llama_block_keeps_state(const shainet_llama_block *b) { return b->wrapped; }
 int shainet_llama_block_save_state(shainet_llama_block *b) {

@@ -11,6 +11,7 @@
 namespace shainet {
 struct AheadRows;
 struct GemvPrep;
+struct ResidualArgs;
 }
 // capi.hip: shainet_attn_forward with the rows of q, k and v at given strides; ahead (nullable): what a decode
 // launch also reads
@@ -136,6 +137,7 @@ struct Fused {
   bool any_few_rows = false;  // up to 16 rows run as the split GEMV, not only the ones it is the faster product for
   const float *normed = nullptr;  // [T, K]: the rows of x behind the norm, where an earlier product handed them over (more than a few rows only)
   Handover *next = nullptr;       // nullable; for kGemvPlain and kGemvResidual
+  const ResidualArgs *join = nullptr;  // x is this row's h, still to be made: in the product's launch where that takes it along (x may stay unwritten then)
   bool w_t_has_gamma = false;  // the rows of w_t were made with gamma multiplied in: the norm's factor 1 / rms is all that is left to apply
 };
 

@@ -15,6 +15,8 @@
 
 namespace shainet {
 
+struct ResidualArgs;
+
 constexpr int kMaxRouterOutputs = 1024;
 
 struct MoeShape {
@@ -30,10 +32,11 @@ struct MoeTensors {
 bool moe_shape_ok(const MoeShape &m);
 
 constexpr int kMoeFewTokens = 8;
+// join (nullable): h, one row, is still to be made by it.
 // y [T, d] for T <= kMoeFewTokens rows h [T, d]; scratch: moe_few_floats(m, T) floats
 size_t moe_few_floats(const MoeShape &m, int T);
 hipError_t launch_moe_few(const MoeShape &m, const MoeTensors &w, const float *h, float *y, int T, float *scratch,
-                          hipStream_t stream);
+                          hipStream_t stream, const ResidualArgs *join = nullptr);
 
 // Any number of rows.  logits: the router's product with h, rows of `stride` floats; y [T, d] holds the shared
 // expert's rows already (add_to_y) or nothing.

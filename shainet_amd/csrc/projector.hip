@@ -176,8 +176,15 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
   if (f.next) f.next->rows = nullptr;
   if (f.epilogue == kGemvQkvPrep && (!f.prep || T > 16 || (N & 3)))
     return llama_fail(SHAINET_HIP_ERR_ARGUMENT, "the fused q | k | v epilogue takes at most 16 rows");
-  if (f.w_t && gemvt_takes(T, K, N, f.epilogue, f.norm, f.prep) && !(((uintptr_t)x | (uintptr_t)f.gamma | (uintptr_t)f.beta) & 15)) {
+  const bool one_row = f.w_t && gemvt_takes(T, K, N, f.epilogue, f.norm, f.prep) && !(((uintptr_t)x | (uintptr_t)f.gamma | (uintptr_t)f.beta) & 15);
+  const bool joins = one_row && f.join && f.join->d == K && row_join_fits(*f.join) && gemvt_takes_join(K, N, f.epilogue, f.norm);
+  if (f.join && !joins) {
+    const hipError_t e = launch_residual(*f.join, stream);
+    if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("residual launch: ") + hipGetErrorString(e));
+  }
+  if (one_row) {
     GemvArgs a = {};
+    if (joins) a.join = *f.join;
     a.x = x;
     a.x_stride = x_stride;
     a.norm = f.norm;

@@ -284,6 +284,15 @@ hipError_t launch_residual(const ResidualArgs &args, hipStream_t stream) {
   return hipGetLastError();
 }
 
+bool row_join_fits(const ResidualArgs &a) {
+  // (workgroups read x, y and hist_in while one of them writes)
+  return a.T == 1 && (a.d == 1024 || a.d == 2048) && a.x && a.pre && (!a.y || (a.post && a.x_out && a.x_out != a.x && a.x_out != a.y)) &&
+         (!a.conv || (a.taps >= 1 && a.taps <= 4)) && (!a.hist_out || a.hist_out != a.hist_in) &&
+         !(((uintptr_t)a.x | (uintptr_t)a.y | (uintptr_t)a.post | (uintptr_t)a.x_out | (uintptr_t)a.pre | (uintptr_t)a.conv | (uintptr_t)a.hist_in |
+            (uintptr_t)a.hist_out | (uintptr_t)a.h) &
+           15);
+}
+
 hipError_t launch_add_one(float *x, long long n, hipStream_t stream) {
   if (!x || n < 1 || (n + 255) / 256 > 0x7fffffffLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL(add_one_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x, n);

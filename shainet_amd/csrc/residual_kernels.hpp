@@ -28,6 +28,8 @@ struct ResidualArgs {
   float eps;
 };
 hipError_t launch_residual(const ResidualArgs &a, hipStream_t stream);
+// Whether a row of it may be worked out inside the launch that reads h (row_join.hpp).
+bool row_join_fits(const ResidualArgs &a);
 
 // x[i] += 1, n floats: weights stored as the distance from 1
 hipError_t launch_add_one(float *x, long long n, hipStream_t stream);
