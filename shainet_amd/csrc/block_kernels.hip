@@ -9,6 +9,7 @@
 //   Sampler                text/sampler.cr:38-120   greedy, repetition penalty, top-k
 // All of them are bound by HBM (or by latency at decode sizes); fp64 arithmetic is
 // free at these intensities on this part.
+#include "activation.hpp"
 #include "block_kernels.hpp"
 
 #include <math.h>
@@ -81,11 +82,6 @@ __global__ __launch_bounds__(256) void add_kernel(const float *__restrict__ a, c
   } else {
     for (long long j = i; j < n; ++j) out[j] = (float)((double)a[j] + (double)b[j]);
   }
-}
-
-__device__ __forceinline__ float swiglu(float gate, float up) {
-  const double g = (double)gate;
-  return (float)((g / (1.0 + exp(-g))) * (double)up);
 }
 
 __global__ __launch_bounds__(256) void swiglu_act_kernel(const float *__restrict__ gate_up, float *__restrict__ hidden,

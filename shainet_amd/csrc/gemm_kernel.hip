@@ -145,8 +145,29 @@ struct Stage {
   static constexpr int kUnits = 3 * kPartX + PARTS * kPartW;
 };
 
+// SWIGLU: W is gate | up, y is [T, N / 2], silu(gate) * up.  A lane then holds both halves of its NB / 2 columns of y: hidden column h of
+// the tile's TN / 2.
+__device__ __forceinline__ int gate_up_place(int NB, int h, int up) { return NB == 2 ? 2 * h + up : 4 * (h >> 1) + (h & 1) + 2 * up; }
+template <int NB>
+__device__ __forceinline__ void store_swiglu(const GemmArgs &g, int row0, int h, int r, f32x4 v) {
+  const int row = row0 + row_of<NB>(r), N = g.N / 2;
+  if (row >= g.T) return;
+  float *const y = g.y + (long long)row * N + h;
+  if constexpr (NB == 2) {
+    y[0] = swiglu(v.x, v.y);
+    const float second = swiglu(v.z, v.w);
+    if (row + 1 < g.T) y[N] = second;
+  } else {
+    *(f32x2 *)y = f32x2{swiglu(v.x, v.z), swiglu(v.y, v.w)};
+  }
+}
+
 // PARTS: of W, 3 or (its values are bf16 numbers) 1.  GUARD: K need not be a multiple of 16 (pieces beyond its end are zeros).
-template <int WM, int WN, int MB, int NB, int PARTS, bool GUARD>
+// SWIGLU (no pieces): the activation, a launch of 10.6 us behind 512 rows of 2048 -> 2 x 8192 and of 32.5 behind 2048 rows, between which the
+// wide rows were written and read again, happens where the sums are.  Us, both launches | this: 512 rows 113.8 | 99.4, 2048 rows
+// 408 | 358, 777 rows of 1024 -> 2 x 1024 in tiles of sgemm_stream_kernel 29.5 | 22.8; weights of three parts: a block of width 2048 401 | 392 at 384
+// rows, 461 | 451 at 512, level at 2048, of width 1024 264 | 255 at 777.
+template <int WM, int WN, int MB, int NB, int PARTS, bool GUARD, bool SWIGLU>
 __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const GemmArgs g) {
   constexpr int TM = 32 * WM * MB, TN = 32 * WN * NB, NT = 64 * WM * WN;
   constexpr int NX = 4 * TM / NT;  // float4 of the x tile per thread
@@ -200,7 +221,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     // of column tid % TN
     const int xrow = NX == 1 ? tid >> 2 : tid >> 1;
     const int xk = NX == 1 ? 4 * (tid & 3) : 8 * (tid & 1);
-    const int wcol = tid & (TN - 1), wk = 8 * (tid / TN);
+    int wcol = tid & (TN - 1), w_from = min(n0 + wcol, N - 1);
+    const int wk = 8 * (tid / TN);
+    if constexpr (SWIGLU) {  // (32 columns of gate, the same of up, and so on: 128 bytes of a row together)
+      const int up = wcol >> 5 & 1, h = (wcol >> 6) * 32 + (wcol & 31);
+      w_from = up * (N / 2) + min(n0 / 2 + h, N / 2 - 1);
+      wcol = gate_up_place(NB, h, up);
+    }
     const int x_unit = (xk >> 3) * S::kOctX + xrow;
     const int w_unit = 3 * S::kPartX + (wk >> 3) * S::kOctW + wcol / (32 * NB) * (36 * NB) + wcol % NB * 36 + wcol % (32 * NB) / NB;
     // fragments
@@ -209,7 +236,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
 
     // (rows past the last one repeat it and columns likewise: their products are never stored)
     const unsigned x_off = (unsigned)(((long long)min(m0 + xrow, T - 1) * g.xs + xk) * 4);
-    const unsigned w_off = (unsigned)(((long long)wk * N + min(n0 + wcol, N - 1)) * 4);
+    const unsigned w_off = (unsigned)(((long long)wk * N + w_from) * 4);
     const char *x_base = (const char *)(g.x + k_begin);
     const char *w_base = (const char *)(g.w + (long long)k_begin * N);
 
@@ -426,8 +453,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
         for (int a = 0; a < MB; ++a)
           xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + (wm * MB + a) * 32 + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          wv[i] = in ? *(const Columns *)(g.w + (long long)(k + i) * N + min(col, N - NB)) : Columns(0.f);
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (SWIGLU) {
+            const float *gate = g.w + (long long)(k + i) * N + min(col / 2, N / 2 - NB / 2);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) wv[i][b] = in ? gate[b / (NB / 2) * (N / 2) + b % (NB / 2)] : 0.f;
+          } else {
+            wv[i] = in ? *(const Columns *)(g.w + (long long)(k + i) * N + min(col, N - NB)) : Columns(0.f);
+          }
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -511,7 +545,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     }
     if (col < N) {  // N is a multiple of 4: a lane's columns are inside together
 #pragma unroll
-      for (int r = 0; r < kOut; ++r) store_four<NB>(g, row0, col, r, out[r]);
+      for (int r = 0; r < kOut; ++r) {
+        if constexpr (SWIGLU)
+          store_swiglu<NB>(g, row0, col / 2, r, out[r]);
+        else
+          store_four<NB>(g, row0, col, r, out[r]);
+      }
     }
   }
 }
@@ -695,7 +734,8 @@ __global__ __launch_bounds__(256, 2) void sgemm_few_kernel(const GemmArgs g) {
 // three MFMAs to put the rest between and are level or slower, 96 rows have no registers for them.  Tried and not kept:
 // non-temporal loads of W, 30.7 | 32.7; eight wavefronts that take 64 columns and every eighth step by themselves, without a barrier:
 // 32.9; tiles of 64 x 64: level at best.)
-template <int MB, int KG, bool GUARD>
+// SWIGLU (no pieces): wavefronts take 32 columns of gate and 32 of up in turn, and hand over by LDS.
+template <int MB, int KG, bool GUARD, bool SWIGLU>
 __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) {
   constexpr bool AHEAD = MB == 2;  // whether fragments are fetched a step ahead
   constexpr int WN = 8 / KG, TM = 32 * MB, TN = 32 * WN, TS = 16 * KG, kSets = 4;
@@ -716,7 +756,8 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, j = lane >> 5, wn = wave % WN, kg = wave / WN;
-  const int col = n0 + 32 * wn + ln;
+  const int col = SWIGLU ? n0 / 2 + 32 * (wn / 2) + ln : n0 + 32 * wn + ln, columns = SWIGLU ? N / 2 : N;
+  const int w_from = min(col, columns - 1) + (SWIGLU ? wn % 2 * columns : 0);
 
   // x: a thread takes four k, piece tid % (4 KG), of row tid / (4 KG) (and kRows on; rows past the last one repeat it)
   const int xrow = threadIdx.x / (4 * KG), xk = 4 * (threadIdx.x % (4 * KG));
@@ -726,7 +767,7 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
   u32x2 *const x_lds = (u32x2 *)(lds + (xk >> 3) * kOct + xrow) + (xk >> 2 & 1);
   // W: rows 16 kg + 8 j .. + 7 of a step (columns past the last one repeat it)
   const int wk = 16 * kg + 8 * j;
-  const unsigned w_off = (unsigned)(((long long)(GUARD ? 0 : 8 * j) * N + min(col, N - 1)) * 4);
+  const unsigned w_off = (unsigned)(((long long)(GUARD ? 0 : 8 * j) * N + w_from) * 4);
   const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)(k_begin + (GUARD ? 0 : 16 * kg)) * N);
   const long long row_bytes = 4LL * N;
 
@@ -895,7 +936,7 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
       for (int a = 0; a < MB; ++a)
         xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + 32 * a + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) wv[i] = in ? g.w[(long long)(k + i) * N + min(col, N - 1)] : 0.f;
+      for (int i = 0; i < 4; ++i) wv[i] = in ? g.w[(long long)(k + i) * N + w_from] : 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -915,16 +956,19 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
         merge[(kg - 1) * WN * kSums + 64 * (4 * a + r)] = f32x4{acc[a][4 * r], acc[a][4 * r + 1], acc[a][4 * r + 2], acc[a][4 * r + 3]};
   }
   __syncthreads();
-  if (kg > 0) return;
+  if (!SWIGLU && kg > 0) return;
 #pragma unroll
   for (int a = 0; a < MB; ++a)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      if (SWIGLU && kg > 0) continue;
       f32x4 v = f32x4{acc[a][4 * r], acc[a][4 * r + 1], acc[a][4 * r + 2], acc[a][4 * r + 3]};
       const f32x4 *const other = merge + 64 * (4 * a + r);
       v += other[0];  // (in pairs: four groups' sums one after the other round a little more)
       if constexpr (KG == 4) v += other[WN * kSums] + other[2 * WN * kSums];
-      if (g.pieces) {  // row by row
+      if constexpr (SWIGLU) {  // (each lane puts what it has where it found the first other sum)
+        merge[64 * (4 * a + r)] = v;
+      } else if (g.pieces) {  // row by row
         float *const piece = g.partials + (long long)blockIdx.x * (TM * TN) + (32 * a + 8 * r + 4 * j) * TN + 32 * wn + ln;
 #pragma unroll
         for (int i = 0; i < 4; ++i) piece[i * TN] = v[i];
@@ -932,6 +976,25 @@ __global__ __launch_bounds__(512, 1) void sgemm_stream_kernel(const GemmArgs g) 
         store_four<1>(g, m0 + 4 * j, col, 4 * a + r, v);
       }
     }
+  if constexpr (SWIGLU) {
+    __syncthreads();
+    // (all wavefronts: those of a pair of gate and up take its registers of four in turn)
+    constexpr int kShare = 2 * KG;  // wavefronts that share a pair of the sums
+    const int share = kg * 2 + wn % 2;
+    const f32x4 *const gate = (const f32x4 *)lds + wn / 2 * 2 * kSums + lane, *const up = gate + kSums;
+#pragma unroll
+    for (int i = 0; i < (4 * MB + kShare - 1) / kShare; ++i) {
+      const int at = share + kShare * i;
+      if (at >= 4 * MB || col >= columns) continue;
+      const f32x4 a = gate[64 * at], b = up[64 * at];
+      const int row = m0 + 4 * j + row_of<1>(at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = swiglu(a[e], b[e]);
+        if (row + e < T) g.y[(long long)(row + e) * columns + col] = v;
+      }
+    }
+  }
 }
 
 // acc + piece 0 + piece 1 + ..., all C in flight
@@ -982,11 +1045,6 @@ __device__ __forceinline__ f32x4 sum_of_pieces(const GemmArgs &g, const PieceSha
   else if (left == 1)
     acc = add_pieces<1>(acc, piece, step);
   return acc;
-}
-
-__device__ __forceinline__ float swiglu(float gate, float up) {  // (swiglu_ff.cr:84-89)
-  const double g = (double)gate;
-  return (float)((g / (1.0 + exp(-g))) * (double)up);
 }
 
 // y = (res +) the sum of a product's pieces, or (SWIGLU) silu(gate) * up of its columns gate | up.  A thread takes what a lane of
@@ -1230,9 +1288,11 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
 // (the norm of a row takes a workgroup of up to 1024 threads, two registers of four each; rows and their pairs along the grid's second
 // dimension, which ends at 65535)
 bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
-  if (!p.mfma || p.pieces <= 1) return false;
+  if (!p.mfma) return false;
+  // (by the kernel that adds the pieces, or by the product itself, but for three-part weights in tiles of 32 rows)
+  if (next.swiglu) return !next.norm.rows && N % 8 == 0 && (p.pieces > 1 ? T <= 65535 : !(p.few && p.parts == 3));
+  if (p.pieces <= 1) return false;
   const bool pairs = !(p.few && p.parts == 1) && !(p.parts == 1 && p.mb == 4);
-  if (next.swiglu) return !next.norm.rows && N % 8 == 0 && T <= 65535;
   return N % 4 == 0 && N / (pairs ? 2 : 4) <= 2048;
 }
 
@@ -1332,10 +1392,15 @@ hipError_t launch_sum(const GemmArgs &g, const PieceShape &s, const GemmNext &ne
 template <int WM, int WN, int MB, int NB, int PARTS>
 hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups), block(64 * WM * WN);
-  if (g.K % TK != 0)
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true>), grid, block, 0, stream, g);
+  const bool swiglu = next.swiglu && !g.pieces;
+  if (swiglu && g.K % TK != 0)
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, true>), grid, block, 0, stream, g);
+  else if (swiglu)
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false, true>), grid, block, 0, stream, g);
+  else if (g.K % TK != 0)
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, false>), grid, block, 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false, false>), grid, block, 0, stream, g);
   const hipError_t e = hipGetLastError();
   return e != hipSuccess || !g.pieces ? e : launch_sum<NB>(g, PieceShape{32 * WM * MB, 32 * WN * NB, 32 * MB, WN, 64 * WM * WN}, next, stream);
 }
@@ -1353,10 +1418,15 @@ hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, const GemmNext &next
 template <int MB, int KG>
 hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
-  if (g.K % (16 * KG) != 0)
-    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, true>), grid, dim3(512), 0, stream, g);
+  const bool guard = g.K % (16 * KG) != 0, swiglu = next.swiglu && !g.pieces;
+  if (swiglu && guard)
+    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, true, true>), grid, dim3(512), 0, stream, g);
+  else if (swiglu)
+    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, false, true>), grid, dim3(512), 0, stream, g);
+  else if (guard)
+    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, true, false>), grid, dim3(512), 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, false>), grid, dim3(512), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_stream_kernel<MB, KG, false, false>), grid, dim3(512), 0, stream, g);
   const hipError_t e = hipGetLastError();
   return e != hipSuccess || !g.pieces ? e : launch_sum<1>(g, PieceShape{32 * MB, 256 / KG, 0, 0, 0}, next, stream);
 }

@@ -43,15 +43,10 @@ __device__ __forceinline__ f32x4 dyn_tanh4(f32x4 x, float alpha, f32x4 g, f32x4 
                tanhf(alpha * x.w) * g.w + b.w};
 }
 
-__device__ __forceinline__ float swiglu1(float gate, float up) {
-  const double g = (double)gate;
-  return (float)((g / (1.0 + exp(-g))) * (double)up);
-}
-
 // row, col: the place of a.x in y
 __device__ __forceinline__ f32x4 apply_epilogue(const GemvArgs &g, f32x4 a, f32x4 b, int row, int col) {
   const int epi = g.epilogue;
-  if (epi == kGemvSwiglu) return f32x4{swiglu1(a.x, b.x), swiglu1(a.y, b.y), swiglu1(a.z, b.z), swiglu1(a.w, b.w)};
+  if (epi == kGemvSwiglu) return f32x4{swiglu(a.x, b.x), swiglu(a.y, b.y), swiglu(a.z, b.z), swiglu(a.w, b.w)};
   if (epi == kGemvResidual) {
     const f32x4 r = *(const f32x4 *)(g.res + (long long)row * g.N + col);
     return f32x4{(float)((double)r.x + (double)a.x), (float)((double)r.y + (double)a.y),
@@ -676,7 +671,7 @@ __global__ __launch_bounds__(256) void gemvt_kernel(GemvArgs a) {
       if (wave < 2 && lane == 0 && live) prep_pair_end(a.prep, target, half_s[wave], half_s[wave + 2]);
     } else if (lane == 0) {
       float v = s[0];
-      if (a.epilogue == kGemvSwiglu) v = swiglu1(s[0], s[NACC - 1]);
+      if (a.epilogue == kGemvSwiglu) v = swiglu(s[0], s[NACC - 1]);
       if (residual) v = (float)((double)res_v + (double)s[0]);
       if (biased) v = activate(a.act, s[0] + res_v);
       a.y[n] = v;

@@ -21,6 +21,7 @@
 // 16, the group's last arrival at a counter of the groups, and the last of those releases
 // everybody through one word per group (bounded polls: a give-up sets the error word and the
 // launch still ends).  Nothing is reset between launches: the numbers keep counting up.
+#include "activation.hpp"
 #include "step_kernel.hpp"
 
 #include <math.h>
@@ -49,11 +50,6 @@ __device__ __forceinline__ void coherent_store(float *p, float v) {
 // was measured too: slower.)
 __device__ __forceinline__ float part_load(const float *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ float swiglu1(float gate, float up) {  // swiglu_ff.cr:84-89
-  const double g = (double)gate;
-  return (float)((g / (1.0 + exp(-g))) * (double)up);
 }
 
 #define STEP_TRACE(slot)                                                                          \
@@ -384,7 +380,7 @@ __device__ __forceinline__ void hidden_slice(const View &v, const float *part, i
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int t = t0 + e * NT + v.tid;
-      if (t < nrows) xs[t] = swiglu1(gate[e], up[e]);
+      if (t < nrows) xs[t] = swiglu(gate[e], up[e]);
     }
   }
   __syncthreads();
