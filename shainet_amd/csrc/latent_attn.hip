@@ -212,6 +212,8 @@ int latent_attn_forward(LatentAttn *l, const float *x, int T, float *out, const 
         return rc;
       e = launch_latent_expanded(l->q.p, l->kv.p, w.sink, r, sh, T, ex, l->partials.p, l->heads.p, stream);
     }
+  } else if (T == 1 && latent_row_fits(sh, start_row)) {
+    e = launch_latent_row(l->q.p, w.u_kv, w.u_kv + (size_t)sh.H * sh.dim * sh.kv_rank, w.sink, r, sh, l->heads.p, stream);
   } else {
     LatentPlan plan;
     if (!plan_latent_absorbed(sh, T, start_row, plan)) return fail(SHAINET_HIP_ERR_ARGUMENT, "too many rows in one call");

@@ -387,6 +387,295 @@ __global__ __launch_bounds__(1024) void latent_out_kernel(const float *__restric
   }
 }
 
+// One new row that sees few keys: the append, the queries' way to the latent space, the attention and the way back in one
+// launch, a workgroup of 512 threads per head.  A row (of the cache, W_uk or W_uv) is read by 16 lanes, P pieces of 16 bytes each,
+// so that the 32 quarters of the wavefronts take 32 keys a round, G rounds in registers, of which a score needs a sum over
+// 16 lanes and the weighted sum nothing more: keys are read once.  Each quarter keeps its own online softmax; quarters meet in
+// registers, wavefronts in LDS.  Everything that the first rounds need is requested before anything is waited for.
+// Bound by what a compute unit gets from its L2 (64 bytes a clock: 422 KB of 16 heads' share at 180 keys), whose way is kept
+// for what is needed next: keys are requested behind W_uk, and W_uv behind the keys (all at once in front: 10.4 us), and by
+// the meetings.  16 heads of 64 + 32 and 64 dimensions, latents of 256: us, three launches and the gaps between them | this:
+// 30 keys 18.0 | 7.5, 110 keys 17.8 | 7.6, 190 keys 18.8 | 8.7, 410 keys 18.8 | 12.5, 810 keys 18.9 | 16.8; of 128 + 64 and 128,
+// latents of 512: 30 keys 21.0 | 12.0, 190 keys 21.5 | 16.3, 410 keys 21.6 | 20.5.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false)); }
+template <int CTRL>
+__device__ __forceinline__ double dpp(double x) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, false));
+}
+// the sum over 16 neighbouring lanes, in each of them (rotations by 8, 4, 2 and 1)
+template <class V>
+__device__ __forceinline__ V sum16(V x) {
+  x += dpp<0x128>(x);
+  x += dpp<0x124>(x);
+  x += dpp<0x122>(x);
+  return x + dpp<0x121>(x);
+}
+// lane l's value and that of the same lane of the other quarter of its half (WIDE: of the other half)
+template <bool WIDE>
+__device__ __forceinline__ float2 both(float x) {
+  const unsigned b = __float_as_uint(x);
+  typedef unsigned pair_t __attribute__((ext_vector_type(2)));
+  pair_t r;
+  if constexpr (WIDE)
+    r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  else
+    r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return float2{__uint_as_float(r.x), __uint_as_float(r.y)};
+}
+__device__ __forceinline__ float sum_quarters(float x) {
+  float2 v = both<false>(x);
+  v = both<true>(v.x + v.y);
+  return v.x + v.y;
+}
+__device__ __forceinline__ float max_quarters(float x) {
+  float2 v = both<false>(x);
+  v = both<true>(fmaxf(v.x, v.y));
+  return fmaxf(v.x, v.y);
+}
+
+template <int P>
+struct RowPieces {
+  f32x4 x[P];
+  // a row of a base that all threads share; at: where the lane's pieces lie in a row
+  __device__ __forceinline__ void request(const float *base, unsigned row, const unsigned (&at)[P]) {
+#pragma unroll
+    for (int u = 0; u < P; ++u) x[u] = *(const f32x4 *)((const char *)base + (row + at[u]));
+  }
+  __device__ __forceinline__ float dot(const f32x4 (&y)[P]) const {  // in all 16 lanes
+    float s = 0.f, t = 0.f;
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      s = fmaf(x[u].x, y[u].x, fmaf(x[u].y, y[u].y, s));
+      t = fmaf(x[u].z, y[u].z, fmaf(x[u].w, y[u].w, t));
+    }
+    return sum16(s + t);
+  }
+};
+
+template <int P, int G, int RK, int RV>
+__global__ __launch_bounds__(512) void latent_row_kernel(const float *__restrict__ q, const float *__restrict__ uk,
+                                                         const float *__restrict__ uv, const float *__restrict__ sink, LatentRows r,
+                                                         LatentShape sh, float qscale, float *__restrict__ out) {
+  constexpr int W4 = 16 * P, kOwn = (64 * P + 511) / 512;
+  __shared__ f32x4 part[8][W4], qa[128 * kOwn], fresh[128 * kOwn];
+  __shared__ float top[8], sums[8];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, l = tid & 15, quarter = tid >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w4 = sh.row_w >> 2, k4 = sh.kv_rank >> 2, dim = sh.dim, vdim = sh.vdim, half = sh.rot_dims >> 1;
+  const int lo = sh.window ? max(0, r.start_row - sh.window + 1) : 0, n_old = r.start_row - lo;
+  const float *const qh = q + (long long)h * (dim + sh.rot_dim);
+  const float *const ukh = uk + (long long)h * dim * sh.kv_rank, *const uvh = uv + (long long)h * vdim * sh.kv_rank;
+  const float *const raw = r.raw + r.kv_off, *const keys = r.rows + (long long)lo * sh.row_w;
+  const unsigned k_bytes = 4u * sh.kv_rank, row_bytes = 4u * sh.row_w;
+  unsigned at_k[P], at_row[P];  // (past the end: the last piece again)
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    at_k[u] = 16u * min(l + 16 * u, k4 - 1);
+    at_row[u] = 16u * min(l + 16 * u, w4 - 1);
+  }
+
+  // what the new row and the rotated queries are made of: elements tid, tid + 512, ...
+  float squares[P], from[kOwn], beside[kOwn], q_from[kOwn], q_beside[kOwn], gamma[kOwn];
+  float2 turn[kOwn];
+#pragma unroll
+  for (int u = 0; u < P; ++u) squares[u] = raw[min(lane + 64 * u, sh.kv_rank - 1)];
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) {
+    const int i = min(tid + 512 * u, sh.kv_rank + sh.rot_dim - 1), e = i - sh.kv_rank;
+    const bool turns = e >= 0 && e < sh.rot_dims;
+    from[u] = raw[i];
+    beside[u] = raw[turns ? sh.kv_rank + (e ^ 1) : i];
+    q_from[u] = qh[e >= 0 ? dim + e : 0];
+    q_beside[u] = qh[turns ? dim + (e ^ 1) : 0];
+    gamma[u] = r.kv_norm[min(i, sh.kv_rank - 1)];
+    turn[u] = float2{1.f, 0.f};
+    if (half) turn[u] = r.rope_tab[(long long)r.start_pos * half + (turns ? e >> 1 : 0)];
+  }
+  const float gate = r.raw[r.gate_off + h], sk = sink[h] * kLog2e;
+
+  RowPieces<P> w[RK];
+  float qd[RK];
+  auto load_uk = [&](int i, int d) {
+    w[i].request(ukh, min(d, dim - 1) * k_bytes, at_k);
+    qd[i] = qh[min(d, dim - 1)];
+  };
+#pragma unroll
+  for (int i = 0; i < RK; ++i) load_uk(i, quarter + 32 * i);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // the new row
+  double sq = 0.0;
+#pragma unroll
+  for (int u = 0; u < P; ++u) sq += lane + 64 * u < sh.kv_rank ? (double)squares[u] * (double)squares[u] : 0.0;
+  sq = sum16(sq);
+  sq += __shfl_xor(sq, 16);
+  sq += __shfl_xor(sq, 32);
+  const double rms = sqrt(sq / (double)sh.kv_rank + r.eps);
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) {
+    const int i = tid + 512 * u, e = i - sh.kv_rank;
+    const bool turns = e < sh.rot_dims, inside = e < sh.rot_dim;
+    const float c = turns ? turn[u].x : 1.f, s = !turns ? 0.f : (e & 1) ? turn[u].y : -turn[u].y;
+    const float normed = (float)(((double)from[u] / rms) * (double)gamma[u]);
+    const float v = e < 0 ? normed : !inside ? 0.f : turns ? from[u] * c + beside[u] * s : from[u];
+    ((float *)fresh)[i] = v;
+    if (h == 0 && i < sh.row_w) r.rows[(long long)r.start_row * sh.row_w + i] = v;
+    ((float *)qa)[i] = !inside ? 0.f : (turns ? q_from[u] * c + q_beside[u] * s : q_from[u]) * qscale;
+  }
+
+  // the queries' way to the latent space
+  f32x4 acc[P];
+#pragma unroll
+  for (int u = 0; u < P; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto take_uk = [&](int d) {
+#pragma unroll
+    for (int i = 0; i < RK; ++i) {
+      const float x = d + 32 * i < dim ? qd[i] : 0.f;
+#pragma unroll
+      for (int u = 0; u < P; ++u) acc[u] += x * w[i].x[u];
+    }
+  };
+  take_uk(quarter);  // (what is in flight for later is not waited for here, as it would be in the loop)
+  for (int d = quarter + 32 * RK; d - quarter < dim; d += 32 * RK) {
+#pragma unroll
+    for (int i = 0; i < RK; ++i) load_uk(i, d + 32 * i);
+    take_uk(d);
+  }
+  // keys k0 .. k0 + 32 G - 1, those that there are (a wavefront without any asks for none: a compute unit's way to its L2 is what
+  // the launch waits for)
+  RowPieces<P> kv[G];
+  auto load_keys = [&](int k0) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (k0 + 32 * g + 4 * wave < n_old) {
+        kv[g].request(keys, min(k0 + 32 * g + quarter, n_old - 1) * row_bytes, at_row);
+      } else {
+#pragma unroll
+        for (int u = 0; u < P; ++u) kv[g].x[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  __builtin_amdgcn_sched_barrier(0);
+  load_keys(0);
+  __builtin_amdgcn_sched_barrier(0);
+  auto meet = [&]() {  // acc of the quarters of a wavefront
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      f32x4 t;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) t[e] = sum_quarters(acc[u][e]);
+      if (lane < 16) part[wave][l + 16 * u] = t;
+    }
+  };
+  meet();
+  __syncthreads();
+  if (tid < k4) {
+    f32x4 t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = part[i][tid];
+    qa[tid] = (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) * qscale;
+  }
+  __syncthreads();
+
+  // quarter 0 begins with the new row, the others with none
+  RowPieces<P> own;
+  f32x4 qv[P];
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    qv[u] = qa[l + 16 * u];
+    own.x[u] = fresh[l + 16 * u];
+  }
+  float m = own.dot(qv), den = 1.f;
+  if (quarter > 0) m = -INFINITY, den = 0.f;
+#pragma unroll
+  for (int u = 0; u < P; ++u) acc[u] = quarter > 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : own.x[u];
+  auto attend = [&](int k0) {
+    float s[G], most = m;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int u = 0; u < P; ++u)
+        if (16 * u + 15 >= w4) kv[g].x[u] = l + 16 * u < w4 ? kv[g].x[u] : f32x4{0.f, 0.f, 0.f, 0.f};
+      s[g] = kv[g].dot(qv);
+      if (k0 + 32 * g + quarter >= n_old) s[g] = -INFINITY;
+      most = fmaxf(most, s[g]);
+    }
+    const float ref = most == -INFINITY ? 0.f : most;  // no key seen so far
+    const float alpha = fast_exp2(m - ref);
+    m = most;
+    den *= alpha;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      s[g] = fast_exp2(s[g] - ref);
+      den += s[g];
+    }
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      acc[u] *= alpha;
+#pragma unroll
+      for (int g = 0; g < G; ++g) acc[u] += s[g] * kv[g].x[u];
+    }
+  };
+  attend(0);
+  for (int k0 = 32 * G; k0 < n_old; k0 += 32 * G) {
+    load_keys(k0);
+    attend(k0);
+  }
+  // (W_uv behind the keys: what else is on its way holds them up)
+  RowPieces<P> v[RV];
+  auto load_uv = [&](int i, int j) { v[i].request(uvh, min(j, vdim - 1) * k_bytes, at_k); };
+#pragma unroll
+  for (int i = 0; i < RV; ++i) load_uv(i, quarter + 32 * i);
+  __builtin_amdgcn_sched_barrier(0);
+
+  const float wave_top = max_quarters(m), scale = fast_exp2(m - (wave_top == -INFINITY ? 0.f : wave_top));
+#pragma unroll
+  for (int u = 0; u < P; ++u) acc[u] *= scale;
+  meet();
+  den = sum_quarters(den * scale);
+  if (lane == 0) {
+    top[wave] = wave_top;
+    sums[wave] = den;
+  }
+  __syncthreads();
+  float mm = sk, all = 0.f, f[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) mm = fmaxf(mm, top[i]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    f[i] = fast_exp2(top[i] - mm);
+    all += f[i] * sums[i];
+  }
+  const float factor = sigmoid1(gate) / (all + fast_exp2(sk - mm));
+  if (tid < k4) {
+    f32x4 t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = part[i][tid] * f[i];
+    qa[tid] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    qv[u] = qa[l + 16 * u];
+    if (16 * u + 15 >= k4) qv[u] = l + 16 * u < k4 ? qv[u] : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto give = [&](int j) {
+#pragma unroll
+    for (int i = 0; i < RV; ++i) {
+      const float s = v[i].dot(qv);
+      if (l == 0 && j + 32 * i < vdim) out[(long long)h * vdim + j + 32 * i] = s * factor;
+    }
+  };
+  give(quarter);
+  for (int j = quarter + 32 * RV; j - quarter < vdim; j += 32 * RV) {
+#pragma unroll
+    for (int i = 0; i < RV; ++i) load_uv(i, j + 32 * i);
+    give(j);
+  }
+}
+
 // ---- expanded form -----------------------------------------------------------------------------
 //
 // A workgroup owns 128 rows of one head, a wavefront 32 of them; all walk the keys in tiles of 32 that
@@ -925,6 +1214,30 @@ hipError_t launch_latent_out(const float *partials, const float *uv, const float
   else
     hipLaunchKernelGGL(latent_out_kernel<4>, grid, dim3(1024), lds, stream, partials, part_ml, uv, sink, r, sh, T, p.splits,
                        p.v_w, out);
+  return hipGetLastError();
+}
+
+bool latent_row_fits(const LatentShape &sh, int start_row) {
+  // (the times above, less 5.4 us for a launch and its meetings: 0.047 us per 1000 floats of a head's weights, 0.04 of the keys'.  The
+  // three launches take 18 us and more)
+  const long long keys = sh.window && start_row >= sh.window ? sh.window : (long long)start_row + 1;
+  return shape_ok(sh) && start_row >= 0 && (sh.kv_rank & 3) == 0 && sh.row_w <= 576 && sh.H <= 256 &&
+         47LL * (sh.dim + sh.vdim) * sh.kv_rank + 40 * keys * sh.row_w <= 12600000;
+}
+
+hipError_t launch_latent_row(const float *q, const float *uk, const float *uv, const float *sink, const LatentRows &r,
+                             const LatentShape &sh, float *out, hipStream_t stream) {
+  if (!rows_ok(r, sh, 1) || !latent_row_fits(sh, r.start_row) || !q || !uk || !uv || !sink || !out ||
+      (((uintptr_t)uk | (uintptr_t)uv | (uintptr_t)r.rows) & 15))
+    return hipErrorInvalidValue;
+  const float qscale = sh.scale * kLog2e;
+#define SHAINET_LAUNCH_LATENT_ROW(P_, G_, RK_, RV_)                                                                          \
+  hipLaunchKernelGGL((latent_row_kernel<P_, G_, RK_, RV_>), dim3((unsigned)sh.H), dim3(512), 0, stream, q, uk, uv, sink, r, sh, qscale, out)
+  if (sh.row_w <= 320)
+    SHAINET_LAUNCH_LATENT_ROW(5, 4, 2, 2);
+  else
+    SHAINET_LAUNCH_LATENT_ROW(9, 2, 2, 1);
+#undef SHAINET_LAUNCH_LATENT_ROW
   return hipGetLastError();
 }
 

@@ -67,6 +67,11 @@ hipError_t launch_latent_absorbed(const float *q_abs, const float *rows, float *
 hipError_t launch_latent_out(const float *partials, const float *uv, const float *sink, const LatentRows &r,
                              const LatentShape &sh, int T, const LatentPlan &p, float *out, hipStream_t stream);
 
+// One row (q, out as above): the append and the three launches above in one, where latent_row_fits.
+bool latent_row_fits(const LatentShape &sh, int start_row);
+hipError_t launch_latent_row(const float *q, const float *uk, const float *uv, const float *sink, const LatentRows &r,
+                             const LatentShape &sh, float *out, hipStream_t stream);
+
 // Attention of T rows over expanded keys and values (q as launch_latent_append leaves it): kv [key_rows, H dim + H vdim] = the latents of cached rows
 // first_row .. first_row + key_rows - 1 (the ones any of the T rows sees) times [W_uk | W_uv].  False: sizes
 // that are no multiple of 4, dim + rot_dim above 256 or vdim above 128 (the absorbed form takes those).
