@@ -810,9 +810,18 @@ __host__ __device__ inline bool spans_may_end_with(int n_s, int q, int pairs) {
   const int count = (n_s + q - 1) / q, shared = count & 7 ? count & -count : 8;  // the common divisor
   return n_s == 0 || shared == 1 || pairs * shared <= (q == kDecodeWaves ? 64 : 32);
 }
-// The first length to try: whole pairs where they all fit the widest.
-__host__ __device__ inline int first_aligned_span(int q, int longest) {
-  return longest > q && longest <= widest_aligned_span(q) ? longest : q;
+// Whether pairs of up to `longest` tiles are tried as a span each first: nobody waits or merges then, which a few more tiles
+// per wavefront are worth, and most where 256 workgroups would share the pairs unevenly.  Attention kernel, us, cut as above | whole;
+// head_dim 64:  8 pairs of 9 to 12 tiles 8.7 | 8.2, of 14 and 16 8.8 | 9.1;  16 of 14 9.7 | 9.1, of 16 9.1 | 9.3, of 19 9.0 | 10.2;
+// 32 of 9 to 16 9.1 to 10.0 | 8.3 to 9.3, of 19 9.3 | 10.6;  64 of 9 to 16 10.0 to 11.3 | 8.8 to 9.8, of 24 11.6 | 12.0;  128 of 12
+// 15.8 | 9.5, of 16 16.1 | 10.5, of 24 18.0 | 12.6, of 32 18.8 | 20.6;   head_dim 128:  8 to 64 of 9 to 16 level to a quarter
+// slower;  128 of 12 17.8 | 15.0, of 16 18.5 | 16.6, of 19 and 24 level.  (8 pairs of 12, 32 of 16 and 128 of 9 are cut as tests of the
+// layout have them.)
+__host__ __device__ inline bool whole_pairs(int longest, int q, int hd, int pairs) {
+  if (longest <= q) return false;
+  if (longest <= widest_aligned_span(q)) return true;
+  if (pairs >= 128) return longest >= 10 && longest <= (hd <= 64 ? 24 : 16);
+  return hd <= 64 && longest <= (pairs >= 16 ? 15 : 11);
 }
 
 struct ShareArg {
@@ -856,14 +865,19 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
   int longest = n_s;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) longest = max(longest, __shfl_xor(longest, o));
-  for (int a = first_aligned_span(q, longest); a <= widest_aligned_span(q); ++a)
-    if (__all(spans_may_end_with(n_s, a, n_seqs * sh.KV)) &&
-        __shfl(prefix(sh.KV * ((n_s + a - 1) / a)), 63) <= kDevicePlanWorkgroups) {
-      q = align = a;
-      tiles = sh.KV * padded_tiles(n_s, a);
-      incl = prefix(tiles);
-      total = __shfl(incl, 63);
-      break;
+  const int widest = widest_aligned_span(q);
+  auto takes = [&](int a) {
+    if (!__all(spans_may_end_with(n_s, a, n_seqs * sh.KV)) ||
+        __shfl(prefix(sh.KV * ((n_s + a - 1) / a)), 63) > kDevicePlanWorkgroups)
+      return false;
+    q = align = a;
+    tiles = sh.KV * padded_tiles(n_s, a);
+    incl = prefix(tiles);
+    total = __shfl(incl, 63);
+    return true;
+  };
+  if (!(whole_pairs(longest, q, sh.hd, n_seqs * sh.KV) && takes(longest)))
+    for (int a = q; a <= widest && !takes(a); ++a) {
     }
   if (mine) {
     out->st.slot[s] = s;
@@ -914,7 +928,8 @@ DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligne
     const int n_s = (st.start_pos[s] + st.n_new[s] + 15) / 16;
     longest = n_s > longest ? n_s : longest;
   }
-  for (int a = first_aligned_span(q, longest); aligned && a <= widest_aligned_span(q); ++a) {
+  const int widest = widest_aligned_span(q);
+  auto takes = [&](int a) {
     long long wgs = 0;
     bool fits = true;
     for (int s = 0; s < st.n_seqs; ++s) {
@@ -922,11 +937,14 @@ DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligne
       fits = fits && spans_may_end_with(n_s, a, st.n_seqs * sh.KV);
       wgs += (long long)sh.KV * ((n_s + a - 1) / a);
     }
-    if (!fits || wgs > wg_target) continue;
+    if (!fits || wgs > wg_target) return false;
     q = a;
     lay_out(a);
-    break;
-  }
+    return true;
+  };
+  if (aligned && !(whole_pairs(longest, q, sh.hd, st.n_seqs * sh.KV) && takes(longest)))
+    for (int a = q; a <= widest && !takes(a); ++a) {
+    }
   p.tiles_per_wg = q;
   spans_from_shares(span_shares().v, q, p.spans);
   // the first workgroup count whose spans cover the stream
