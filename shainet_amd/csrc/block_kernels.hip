@@ -204,6 +204,7 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long v) {
 
 constexpr int kTopkChunk = 2048;   // logits per workgroup in the first pass; 8 keys per thread
 constexpr int kTopkThreads = 256;  // >= kMaxTopK
+constexpr int kTopkHeld = 4;       // candidates that a thread of the merge holds: 1024 of them, 40 of a vocabulary of 51000
 
 struct TopkLds {
   unsigned long long best[kTopkThreads];   // every thread's largest key
@@ -225,53 +226,92 @@ __device__ __forceinline__ void topk_threshold(TopkLds &s, unsigned long long mi
       mine = other > mine ? other : mine;
     }
   }
-  const int groups = few ? kTopkThreads / 4 : kTopkThreads;
   if (!few || (threadIdx.x & 3) == 0) s.best[few ? threadIdx.x >> 2 : threadIdx.x] = mine;
   if (threadIdx.x == 0) s.threshold = 0ull, s.pooled = 0;
   __syncthreads();
   int above = 0;
-#pragma unroll 8
-  for (int j = 0; j < groups; ++j) above += s.best[j] > mine;
+  if (few) {  // (the four threads that hold a key share the comparisons)
+    unsigned long long other[kTopkThreads / 16];
+#pragma unroll
+    for (int u = 0; u < kTopkThreads / 16; ++u) other[u] = s.best[(threadIdx.x & 3) + 4 * u];
+#pragma unroll
+    for (int u = 0; u < kTopkThreads / 16; ++u) above += other[u] > mine;
+    above += __shfl_xor(above, 1);
+    above += __shfl_xor(above, 2);
+  } else {
+#pragma unroll 16
+    for (int j = 0; j < kTopkThreads; ++j) above += s.best[j] > mine;
+  }
   if (above == k - 1) s.threshold = mine;  // (of several threads only where they hold the same)
   __syncthreads();
 }
-__device__ __forceinline__ void topk_pool(TopkLds &s, unsigned long long key) {
-  if (key != 0ull && key >= s.threshold) {
-    const int at = atomicAdd(&s.pooled, 1);
-    if (at < kTopkChunk) s.pool[at] = key;
+// (a wavefront asks for the places of all its keys at once)
+template <int N>
+__device__ __forceinline__ void topk_pool(TopkLds &s, const unsigned long long (&keys)[N]) {
+  const unsigned long long least = s.threshold > 1ull ? s.threshold : 1ull, here = __ballot(true);
+  const int lane = threadIdx.x & 63;
+  int place[N], n = 0;
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const unsigned long long taken = __ballot(keys[u] >= least);
+    place[u] = n + __popcll(taken & ((1ull << lane) - 1));
+    n += __popcll(taken);
+  }
+  if (n == 0) return;
+  int at = 0;
+  if (lane == __ffsll(here) - 1) at = atomicAdd(&s.pooled, n);
+  at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    if (keys[u] >= least && at + place[u] < kTopkChunk) s.pool[at + place[u]] = keys[u];
+}
+// win = the k largest of the pool in order (0 behind the last one).  Up to 128 of them: four, or two, threads compare a key.
+template <int P>
+__device__ __forceinline__ void topk_rank_by(TopkLds &s, int k, int n) {
+  const int part = threadIdx.x % P;
+  for (int i = threadIdx.x / P; i < n; i += kTopkThreads / P) {
+    const unsigned long long key = s.pool[i];
+    int above = 0;
+#pragma unroll 8
+    for (int j = part; j < n; j += P) above += s.pool[j] > key;
+#pragma unroll
+    for (int o = 1; o < P; o <<= 1) above += __shfl_xor(above, o);
+    if (part == 0 && above < k) s.win[above] = key;
   }
 }
-// win = the k largest of the pool in order (0 behind the last one)
 __device__ __forceinline__ void topk_rank(TopkLds &s, int k) {
   __syncthreads();
   const int n = s.pooled;
-  for (int i = threadIdx.x; i < n; i += kTopkThreads) {
-    const unsigned long long key = s.pool[i];
-    int above = 0;
-    for (int j = 0; j < n; ++j) above += s.pool[j] > key;
-    if (above < k) s.win[above] = key;
-  }
+  if (n <= kTopkThreads / 4)
+    topk_rank_by<4>(s, k, n);
+  else if (n <= kTopkThreads / 2)
+    topk_rank_by<2>(s, k, n);
+  else
+    topk_rank_by<1>(s, k, n);
   for (int r = n + (int)threadIdx.x; r < k; r += kTopkThreads) s.win[r] = 0ull;
   __syncthreads();
 }
 
 // cand[r * chunks + c]: the r-th largest key of chunk c.  Rounds of "take the largest key" took 32 us for
 // k = 40 (two barriers a round); a threshold and ranks 8 us, nearly whatever k is; the merge with the draw behind
-// it 34 + 8 us and now 7.5.
+// it 34 + 8 us and 8.  Bound by their chains: logits asked for one after the other behind a condition, a place in the pool at a time,
+// a thread per key that compares it with all others; all at once, a place per wavefront, and up to four threads a key: 5.4 and 5.7.
 __global__ __launch_bounds__(kTopkThreads) void topk_chunk_kernel(const float *__restrict__ logits, int vocab, int k,
                                                                   int finite_only, unsigned long long *__restrict__ cand) {
   __shared__ TopkLds s;
   unsigned long long keys[8], mine = 0ull;
   const int base = blockIdx.x * kTopkChunk;
+  float v[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = logits[min(base + u * kTopkThreads + (int)threadIdx.x, vocab - 1)];
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
     const int idx = base + u * kTopkThreads + threadIdx.x;
-    keys[u] = idx < vocab ? make_key(logits[idx], idx, finite_only != 0) : 0ull;
+    keys[u] = idx < vocab ? make_key(v[u], idx, finite_only != 0) : 0ull;
     mine = keys[u] > mine ? keys[u] : mine;
   }
   topk_threshold(s, mine, k);
-#pragma unroll
-  for (int u = 0; u < 8; ++u) topk_pool(s, keys[u]);
+  topk_pool(s, keys);
   topk_rank(s, k);
   if ((int)threadIdx.x < k) cand[(long long)threadIdx.x * gridDim.x + blockIdx.x] = s.win[threadIdx.x];
 }
@@ -286,10 +326,24 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const float *_
                                                                   int *__restrict__ pick, double temperature, double r) {
   __shared__ TopkLds s;
   __shared__ double weight[kMaxTopK];
-  unsigned long long mine = 0ull;
-  for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) mine = cand[i] > mine ? cand[i] : mine;
+  unsigned long long keys[kTopkHeld], mine = 0ull;
+#pragma unroll
+  for (int u = 0; u < kTopkHeld; ++u) keys[u] = cand[min(u * kTopkThreads + (int)threadIdx.x, n_cand - 1)];
+#pragma unroll
+  for (int u = 0; u < kTopkHeld; ++u) {
+    if (u * kTopkThreads + (int)threadIdx.x >= n_cand) keys[u] = 0ull;
+    mine = keys[u] > mine ? keys[u] : mine;
+  }
+  for (int i = kTopkHeld * kTopkThreads + threadIdx.x; i < n_cand; i += kTopkThreads) mine = cand[i] > mine ? cand[i] : mine;
   topk_threshold(s, mine, k);
-  for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) topk_pool(s, cand[i]);
+  auto pool = [&]() {
+    topk_pool(s, keys);
+    for (int i = kTopkHeld * kTopkThreads + threadIdx.x; i < n_cand; i += kTopkThreads) {
+      const unsigned long long key[1] = {cand[i]};
+      topk_pool(s, key);
+    }
+  };
+  pool();
   __syncthreads();
   if (s.pooled > kTopkChunk) {  // too many for the pool: the threshold is raised to the k-th largest key, a bit at a time
     unsigned long long low = 0ull;
@@ -307,7 +361,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const float *_
     __syncthreads();
     if (threadIdx.x == 0) s.threshold = low, s.pooled = 0;
     __syncthreads();
-    for (int i = threadIdx.x; i < n_cand; i += kTopkThreads) topk_pool(s, cand[i]);
+    pool();
   }
   topk_rank(s, k);
   const int n = s.pooled < k ? s.pooled : k, t = threadIdx.x;
@@ -344,8 +398,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const float *_
 
 // Sampler.greedy and the next step's embedding lookup in one launch of one workgroup: *id = the largest finite
 // logit's place (0: none), out = its row of the table.  cand null: the logits themselves are read here, 128 KB of
-// them (vocabulary of 32000): 6.7 us, where two top-k launches and the lookup took 11; from 65536 on the
-// chunks' largest keys are (n of them).
+// them (vocabulary of 32000): 4.7 us (6.7 with a 64-bit key for each of them and conditional loads), where two top-k launches and the
+// lookup took 11; from 65536 on the chunks' largest keys are (n of them).
 __global__ __launch_bounds__(1024) void greedy_embed_kernel(const float *__restrict__ logits, int vocab,
                                                             const unsigned long long *__restrict__ cand, int n,
                                                             int *__restrict__ id, const float *__restrict__ table,
@@ -357,21 +411,24 @@ __global__ __launch_bounds__(1024) void greedy_embed_kernel(const float *__restr
     for (int i = threadIdx.x; i < n; i += 1024) best = cand[i] > best ? cand[i] : best;
   } else {
     const int whole = vocab & ~3;
+    float most = -INFINITY;  // (a thread comes by its logits in their order: the first of equals stays)
+    int place = 0;
     for (int i0 = 0; i0 < whole; i0 += 8 * 4096) {
       f32x4 v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int i = i0 + u * 4096 + 4 * (int)threadIdx.x;
-        v[u] = i < whole ? *(const f32x4 *)(logits + i) : f32x4{NAN, NAN, NAN, NAN};
-      }
+      for (int u = 0; u < 8; ++u) v[u] = *(const f32x4 *)(logits + min(i0 + u * 4096 + 4 * (int)threadIdx.x, whole - 4));
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
+      for (int u = 0; u < 8; ++u) {
+        const int i = min(i0 + u * 4096 + 4 * (int)threadIdx.x, whole - 4);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const unsigned long long key = make_key(v[u][c], i0 + u * 4096 + 4 * (int)threadIdx.x + c, true);
-          best = key > best ? key : best;
+          const bool more = v[u][c] > most && v[u][c] < INFINITY;
+          most = more ? v[u][c] : most;
+          place = more ? i + c : place;
         }
+      }
     }
+    best = make_key(most, place, true);
     if (whole + (int)threadIdx.x < vocab) {
       const unsigned long long key = make_key(logits[whole + threadIdx.x], whole + threadIdx.x, true);
       best = key > best ? key : best;
