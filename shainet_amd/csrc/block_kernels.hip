@@ -84,6 +84,15 @@ __global__ __launch_bounds__(256) void add_kernel(const float *__restrict__ a, c
   }
 }
 
+__global__ __launch_bounds__(256) void copy_floats_kernel(const float *__restrict__ x, float *__restrict__ out, long long n) {
+  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i + 3 < n && !(((uintptr_t)x | (uintptr_t)out) & 15)) {
+    *(f32x4 *)(out + i) = *(const f32x4 *)(x + i);
+  } else {
+    for (long long j = i; j < n && j < i + 4; ++j) out[j] = x[j];
+  }
+}
+
 __global__ __launch_bounds__(256) void swiglu_act_kernel(const float *__restrict__ gate_up, float *__restrict__ hidden,
                                                          int ff) {
   const int r = blockIdx.y;
@@ -544,6 +553,12 @@ hipError_t launch_add(const float *a, const float *b, float *out, long long n, h
   const long long blocks = (n + 1023) / 1024;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL(add_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a, b, out, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_floats(const float *x, float *out, long long n, hipStream_t stream) {
+  if (!x || !out || n < 1 || (n + 1023) / 1024 > 0x7fffffffLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(copy_floats_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, stream, x, out, n);
   return hipGetLastError();
 }
 

@@ -89,6 +89,7 @@ struct shainet_llama_model {
   int *error = nullptr;  // pinned host word: set by any kernel of the model that gave up a bounded wait
   Projector proj;
   DevF act[2], logits;
+  PinnedF logits_pin;        // one row on its way to the host
   DevF row_act, row_logits;  // shainet_llama_model_run_rows: the wanted rows and their logits
   int *d_tokens = nullptr;
   size_t d_tokens_cap = 0;
@@ -454,6 +455,7 @@ int shainet_llama_model_destroy(shainet_llama_model *m) {
   if (m->d_ids) (void)hipFree(m->d_ids);
   if (m->d_gen) (void)hipFree(m->d_gen);
   if (m->h_pick) (void)hipHostFree(m->h_pick);
+  m->logits_pin.release();
   if (m->topk_scratch) (void)hipFree(m->topk_scratch);
   m->proj.release();
   m->step.release();
@@ -558,7 +560,16 @@ static int run_host_tokens(shainet_llama_model *m, const int *tokens, int n_toke
   return run_device_tokens(m, m->d_tokens, n_tokens, no_cache, last_block);
 }
 
+// One row goes through pinned memory, which a launch behind the last one writes: a copy to pageable memory is begun by the host once
+// the stream has come to its end (a prompt of 45 tokens 508 us, this way 475).
 static int copy_logits_back(shainet_llama_model *m, const float *from, size_t n, float *to) {
+  if (n <= (size_t)m->vocab && m->logits_pin.reserve((size_t)m->vocab)) {
+    const hipError_t e = launch_copy_floats(from, m->logits_pin.p, (long long)n, m->stream);
+    if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("logits launch: ") + hipGetErrorString(e));
+    if (hipStreamSynchronize(m->stream) != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, "copying the logits back failed");
+    memcpy(to, m->logits_pin.p, n * sizeof(float));
+    return check_error_word(m->error);
+  }
   if (hipMemcpyAsync(to, from, n * sizeof(float), hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
       hipStreamSynchronize(m->stream) != hipSuccess)
     return fail(SHAINET_HIP_ERR_RUNTIME, "copying the logits back failed");
@@ -781,11 +792,7 @@ int shainet_llama_model_write_logits(shainet_llama_model *m, const float *logits
 int shainet_llama_model_read_logits(shainet_llama_model *m, float *logits) {
   if (!m || !logits) return fail(SHAINET_HIP_ERR_ARGUMENT, "null argument");
   if (!m->have_logits) return fail(SHAINET_HIP_ERR_ARGUMENT, "no logits: call shainet_llama_model_run first");
-  if (hipMemcpyAsync(logits, m->logits.p, (size_t)m->vocab * sizeof(float), hipMemcpyDeviceToHost, m->stream) !=
-          hipSuccess ||
-      hipStreamSynchronize(m->stream) != hipSuccess)
-    return fail(SHAINET_HIP_ERR_RUNTIME, "copying the logits back failed");
-  return check_error_word(m->error);
+  return copy_logits_back(m, m->logits.p, (size_t)m->vocab, logits);
 }
 
 }  // extern "C"
