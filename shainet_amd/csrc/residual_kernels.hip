@@ -201,6 +201,78 @@ __global__ __launch_bounds__(256) void residual_conv_kernel(const ResidualArgs a
   }
 }
 
+// Both launches in one, where nothing is written in place: a wavefront makes a row, the taps - 1 rows in front of the workgroup's
+// 9 - taps among them, and the rows meet in LDS.  PL: 16-byte pieces per lane.  Bound by a launch, two round trips and fetching its own
+// instructions (with a thread's columns of all rows in registers, three times as many of them, 8.5 us at 777 rows).  Us, two launches
+// and the gap between them | this: 40 rows of 1024 9.4 | 5.6, 777 rows 11.1 | 6.7, 2000 rows 14.7 | 10.6; 300 rows of 2048 11.1 | 8.7.
+constexpr int kJoined = 8;
+template <int PL>
+__global__ __launch_bounds__(64 * kJoined) void residual_rows_kernel(const ResidualArgs a) {
+  __shared__ f32x4 hs[kJoined][64 * PL];
+  const int d4 = a.d >> 2, back = a.taps - 1, rows = kJoined - back, first = blockIdx.x * rows;
+  const int lane = threadIdx.x & 63, k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = first - back + k;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 x[PL], w[PL / 4][4];
+#pragma unroll
+  for (int q = 0; q < PL / 4; ++q)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[q][j] = ((const f32x4 *)a.conv + (long long)min(j, back) * d4)[min((int)(threadIdx.x & 255) + 256 * q, d4 - 1)];
+  if (t >= 0) {
+    const long long row = (long long)min(t, a.T - 1) * d4;
+    f32x4 y[PL], post[PL], pre[PL];
+#pragma unroll
+    for (int p = 0; p < PL; ++p) {
+      const int i = min(lane + 64 * p, d4 - 1);
+      x[p] = ((const f32x4 *)a.x + row)[i];
+      y[p] = ((const f32x4 *)(a.y ? a.y : a.x) + row)[i];
+      post[p] = ((const f32x4 *)(a.y ? a.post : a.pre))[i];
+      pre[p] = ((const f32x4 *)a.pre)[i];
+    }
+    auto factor = [&](const f32x4 (&v)[PL]) {
+      float sq = 0.f;
+#pragma unroll
+      for (int p = 0; p < PL; ++p) sq += sum4(lane + 64 * p < d4 ? v[p] * v[p] : zero);
+      return inv_rms(wave_sum(sq), a.d, a.eps);
+    };
+    if (a.y) {
+      const float f = factor(y);
+#pragma unroll
+      for (int p = 0; p < PL; ++p) {
+        x[p] += y[p] * f * post[p];
+        if (k >= back && t < a.T && lane + 64 * p < d4) ((f32x4 *)a.x_out + row)[lane + 64 * p] = x[p];
+      }
+    }
+    const float f = factor(x);
+#pragma unroll
+    for (int p = 0; p < PL; ++p) x[p] = x[p] * f * pre[p];
+  } else {
+#pragma unroll
+    for (int p = 0; p < PL; ++p)
+      x[p] = a.hist_in ? ((const f32x4 *)a.hist_in + (long long)(back + t) * d4)[min(lane + 64 * p, d4 - 1)] : zero;
+  }
+  // the last rows of [what came in | this call's]
+  const int slot = t - (a.T - back);
+  const bool kept = a.hist_out && t < a.T && (k >= back || (t < 0 && blockIdx.x == 0)) && slot >= 0;
+#pragma unroll
+  for (int p = 0; p < PL; ++p) {
+    hs[k][lane + 64 * p] = x[p];
+    if (kept && lane + 64 * p < d4) ((f32x4 *)a.hist_out + (long long)slot * d4)[lane + 64 * p] = x[p];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PL / 4; ++q) {
+    const int i = (threadIdx.x & 255) + 256 * q;
+    if (i >= d4) continue;
+    for (int r = threadIdx.x >> 8; r < rows && first + r < a.T; r += 2) {
+      f32x4 c = zero;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j <= back) c += hs[r + j][i] * w[q][j];
+      ((f32x4 *)a.h + (long long)(first + r) * d4)[i] = hs[r + back][i] + c;
+    }
+  }
+}
+
 // Any width and number of taps: an element per thread.
 __global__ __launch_bounds__(256) void residual_conv_any_kernel(const ResidualArgs a, const float *__restrict__ x) {
   const int back = a.taps - 1, i = blockIdx.y * 256 + threadIdx.x;
@@ -254,6 +326,15 @@ hipError_t launch_residual(const ResidualArgs &args, hipStream_t stream) {
     return hipGetLastError();
   }
   if (a.conv && !a.factors) return hipErrorInvalidValue;
+  const bool apart = a.h != a.x && a.h != a.y && (!a.y || (a.x_out != a.x && a.x_out != a.y));
+  if (vec && a.conv && a.taps >= 2 && a.taps <= 4 && d4 <= 512 && apart) {
+    const dim3 grid((unsigned)((a.T + kJoined - a.taps) / (kJoined + 1 - a.taps)));
+    if (d4 <= 256)
+      hipLaunchKernelGGL(residual_rows_kernel<4>, grid, dim3(64 * kJoined), 0, stream, a);
+    else
+      hipLaunchKernelGGL(residual_rows_kernel<8>, grid, dim3(64 * kJoined), 0, stream, a);
+    return hipGetLastError();
+  }
   const dim3 rows((unsigned)a.T);
   const int pieces = vec ? (d4 + 255) / 256 : 99;
   {

@@ -27,3 +27,18 @@ def test_rows_joined_where_they_are_read(hip, tmp_path, width, taps):  # noqa: F
     p.model.clear_cache()
     close(p.model.run_full(ids[:1]), want[0], TOL)  # a row that leaves no state behind
     close(run_cut(p.model, ids, (1,)), want, TOL)
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("width", [8, 1024, 1028, 2048, 2052])
+def test_rows_joined_many_at_a_time(hip, tmp_path, width, taps):  # noqa: F811
+    """Whole workgroups of rows, one more and one less, the first of them behind a short call's: widths of one and two pieces and the
+    next one, which takes two launches."""
+    cfg = zm.config([zm.layer(zm.hgrn2(heads=2, dim=16, vdim=32), zm.dense(64)), zm.layer(zm.hgrn2(heads=2, dim=16, vdim=32), zm.dense(64))],
+                    60, width, taps=taps, max_positions=40)
+    p = Pair(hip, tmp_path, cfg)
+    rows = 9 - taps
+    ids = tokens(4 * rows + 4, cfg["vocab"])
+    want = p.logits(ids)
+    for cuts in ((4 * rows + 4,), (2, rows + 1, 2 * rows - 1, 2), (rows, 3 * rows, 4)):
+        close(run_cut(p.model, ids, cuts), want, TOL)
