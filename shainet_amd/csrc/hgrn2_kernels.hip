@@ -592,7 +592,13 @@ bool plan_hgrn2(int T, int H, int dim, int vdim, Hgrn2Plan &p) {
   p.chunks = 0;
   p.scratch_floats = 0;
   if (T <= 16) return true;
+  // Short chunks while a round of workgroups takes them all: each is a chain that gets shorter with it, the states in between
+  // are more.  Us, the three launches with chunks of 64 | 32 | 16 rows: 8 heads of 128 x 128, 75 rows 39 | 29 | 27, 200 rows 39 | 30.4 | 29.7
+  // (104 workgroups of the shortest), 400 rows 40 | 32.6 | 33.4 (200), 777 rows 42 | 38 | 54, 1500 rows 48 | 61 | 80;  16 heads, 300 rows 41 |
+  // 34 | 50, 777 rows 49 | 61 | 97.
   for (int c : {64, 32, 16}) {
+    const int shorter = c / 2;
+    if (c > 16 && ((long long)T + shorter - 1) / shorter * H <= (c == 64 ? 256 : 128)) continue;
     if (output_lds(c, dim) > (size_t)(kMaxLds - 8192) || (vdim + 31) / 32 > (c == 64 ? 16 : 32)) continue;
     const long long all = ((long long)T + c - 1) / c;
     p.chunk = c;
