@@ -588,8 +588,14 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
   // (steps behind the last one repeat it, which nobody reads.  No load hangs on a condition: the branches around them had
   // the loop wait for every load it had just issued: 75 rows of 1023 -> 511 by weights of three parts 92 -> 75 us)
   const int last = (K - 1) / TK * TK;
+  // Rows of K floats lie a power of two apart, most often, and tiles that all begin at their first column ask the same few memory
+  // channels for all of their rows at once: they begin apart (by column tile alone: the order of a row's sums does not depend on other
+  // rows).  75 rows of 1024 -> 2 x 512 29.4 -> 25.5 us, 777 rows 50.9 -> 49.6; tiles of 128 rows, which read W half as often, are level
+  // or slower.
+  const int start = MB == 1 && LOADS == kSteps ? (int)((unsigned)(blockIdx.x % columns) * 5u % (unsigned)(K / TK)) * TK : 0;
   auto load = [&](int set, int k0) {
     k0 = min(k0, last);
+    if constexpr (MB == 1 && LOADS == kSteps) k0 = k0 + start > last ? k0 + start - K : k0 + start;
     const int k = k0 + k4;
 #pragma unroll
     for (int u = 0; u < NA; ++u)
@@ -654,6 +660,20 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
 #pragma unroll
           for (int b = 0; b < 2; ++b) acc[a][b] = mfma_bf16(af[h][kPartA[p]][a], bf[h][kPartB[p] < PARTS ? kPartB[p] : 0][b], acc[a][b]);
       }
+    if constexpr (PARTS == 1 && LOADS == kSteps) {
+      // fragments, and then splits, stores and loads handed out between the MFMAs, the loads behind the half of them (masks: 0x100
+      // reads of LDS, 2 vector instructions, 8 MFMAs, 0x200 stores to LDS, 0x20 loads).  777 rows of 2048 -> 2 x 768 165 -> 149 us, 768 ->
+      // 2048 103 -> 92; of 1024 -> 2 x 512 51.8 -> 50.9; the loads left where they fell: 158 and 97
+      __builtin_amdgcn_sched_group_barrier(0x100, HK * (3 * MB + 2), 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, 16, 0);
+#pragma unroll
+      for (int i = 0; i < 12 * MB; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        if (i >= 6) __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+      }
+    }
     __syncthreads();
   };
   for (int kt = 1; kt < steps; kt += 2) {  // (in pairs: a way out between them costs waits, too)
