@@ -476,37 +476,37 @@ __global__ __launch_bounds__(256) void moe_select_kernel(MoeShape m, const float
   }
 }
 
-// Where the experts' rows and tiles begin; clears the counters for the next call.
-__global__ __launch_bounds__(1024) void moe_offsets_kernel(int experts, int tile, int *counts, int *__restrict__ off,
-                                                           int *__restrict__ tile_off) {
-  __shared__ int a[1024], b[1024];
-  const int e = threadIdx.x;
-  const int c = e < experts ? counts[e] : 0;
-  a[e] = c;
-  b[e] = (c + tile - 1) / tile;
+// Where the experts' rows and tiles begin, which every workgroup works out for itself (the first leaves it), and the rows' tokens in
+// the experts' order.  Bound by a launch and two round trips.  In two launches, one workgroup of them with ten steps of a scan through
+// LDS, 3.9 + 0.8 + 2.9 us (777 tokens of six); this 4.7
+__global__ __launch_bounds__(1024) void moe_rows_kernel(int n, int top, int experts, int tile, const int *__restrict__ counts,
+                                                        const int *__restrict__ ids, const int *__restrict__ rank, int *__restrict__ off,
+                                                        int *__restrict__ tile_off, int *__restrict__ rows) {
+  __shared__ int begins[1024], waves[2][16];
+  const int e = threadIdx.x, lane = e & 63, wave = e >> 6, i = blockIdx.x * 1024 + e, at = min(i, n - 1);
+  const int mine = ids[at], place = rank[at];
+  const int c = counts[min(e, experts - 1)], own = e < experts ? c : 0, tiles = (own + tile - 1) / tile;
+  int a = own, b = tiles;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(a, o), y = __shfl_up(b, o);
+    a += lane >= o ? x : 0;
+    b += lane >= o ? y : 0;
+  }
+  if (lane == 63) waves[0][wave] = a, waves[1][wave] = b;
   __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const int x = e >= o ? a[e - o] : 0, y = e >= o ? b[e - o] : 0;
-    __syncthreads();
-    a[e] += x;
-    b[e] += y;
-    __syncthreads();
+  for (int w = 0; w < wave; ++w) {
+    a += waves[0][w];
+    b += waves[1][w];
   }
-  if (e < experts) {
-    off[e + 1] = a[e];
-    tile_off[e + 1] = b[e];
-    counts[e] = 0;
+  begins[e] = a - own;
+  if (blockIdx.x == 0 && e < experts) {
+    off[e + 1] = a;
+    tile_off[e + 1] = b;
+    if (e == 0) off[0] = tile_off[0] = 0;
   }
-  if (e == 0) off[0] = tile_off[0] = 0;
-}
-
-__global__ __launch_bounds__(256) void moe_scatter_kernel(int n, int top, int experts, const int *__restrict__ ids,
-                                                          const int *__restrict__ rank, const int *__restrict__ off,
-                                                          int *__restrict__ rows) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const int e = ids[i];
-  if (e < experts) rows[off[e] + rank[i]] = i / top;
+  __syncthreads();
+  if (i < n && mine < experts) rows[begins[mine] + place] = i / top;
 }
 
 // Rows of x (gathered, or as they lie) times the matrices of their groups, [N, K] (SWIGLU: [2N, K], gate
@@ -746,14 +746,18 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
     }
 }
 
-// y[t] (+)= sum over the slots of weight * the expert's row, in the slots' order
+// y[t] (+)= sum over the slots of weight * the expert's row, in the slots' order.  The first workgroup clears the
+// counters for the next call.
 template <int W>
 __global__ __launch_bounds__(256) void moe_combine_kernel(MoeShape m, const float *__restrict__ h,
                                                           const float *__restrict__ rows_y, const int *__restrict__ ids,
                                                           const float *__restrict__ weights, const int *__restrict__ rank,
-                                                          const int *__restrict__ off, int add, float *__restrict__ y) {
+                                                          const int *__restrict__ off, int add, float *__restrict__ y,
+                                                          int *__restrict__ counts) {
   typedef float vec_t __attribute__((ext_vector_type(W)));
   const int t = blockIdx.x, n = m.d / W;
+  if (t == 0 && blockIdx.y == 0)
+    for (int e = threadIdx.x; e < m.experts; e += 256) counts[e] = 0;
   for (int i = blockIdx.y * 256 + threadIdx.x; i < n; i += gridDim.y * 256) {
     vec_t s = add ? ((const vec_t *)(y + (long long)t * m.d))[i] : (vec_t)(0.f);
     for (int k = 0; k < m.top; ++k) {
@@ -933,9 +937,8 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
   // a tuning knob: 64 or 128 (32, which there once was, is 64)
   static const int tile_knob = getenv("SHAINET_HIP_MOE_TILE") ? atoi(getenv("SHAINET_HIP_MOE_TILE")) : 0;
   const int tm = tile_knob == 128 ? 128 : tile_knob == 64 || tile_knob == 32 ? 64 : best_tm;
-  hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, stream, m.experts, tm, counts, off, tile_off);
-  hipLaunchKernelGGL(moe_scatter_kernel, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, stream, slots, m.top, m.experts,
-                     ids, rank, off, rows);
+  hipLaunchKernelGGL(moe_rows_kernel, dim3((unsigned)((slots + 1023) / 1024)), dim3(1024), 0, stream, slots, m.top, m.experts, tm,
+                     counts, ids, rank, off, tile_off, rows);
   GroupedArgs g = {};
   g.x = h;
   g.gather = rows;
@@ -961,9 +964,9 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
   const int per = vec ? 1024 : 256;
   const dim3 grid((unsigned)T, (unsigned)((m.d + per - 1) / per));
   if (vec)
-    hipLaunchKernelGGL(moe_combine_kernel<4>, grid, dim3(256), 0, stream, m, h, rows_y, ids, weights, rank, off, add_to_y ? 1 : 0, y);
+    hipLaunchKernelGGL(moe_combine_kernel<4>, grid, dim3(256), 0, stream, m, h, rows_y, ids, weights, rank, off, add_to_y ? 1 : 0, y, counts);
   else
-    hipLaunchKernelGGL(moe_combine_kernel<1>, grid, dim3(256), 0, stream, m, h, rows_y, ids, weights, rank, off, add_to_y ? 1 : 0, y);
+    hipLaunchKernelGGL(moe_combine_kernel<1>, grid, dim3(256), 0, stream, m, h, rows_y, ids, weights, rank, off, add_to_y ? 1 : 0, y, counts);
   return hipGetLastError();
 }
 
