@@ -1070,6 +1070,49 @@ __global__ __launch_bounds__(256) void sgemm_sum_kernel(const GemmArgs g, const 
   }
 }
 
+// The sum is q | k | v heads: queries and keys are rotated (prep_math.hpp's arithmetic) and, with the values, put where the attention
+// reads them.  A thread takes the same place of a head's two halves.  Bound by a launch and its round trips; us, a sum and the launch that
+// rotates | this: 45 rows of 2048 -> 3072 4.1 + 3.3 | 4.6, 512 rows 7.5 + 5.3 | 8.1.
+template <int COLUMNS>
+__global__ __launch_bounds__(256) void sgemm_sum_prep_kernel(const GemmArgs g, const PieceShape s, const GemvPrep p) {
+  constexpr int R = COLUMNS == 2 ? 2 : 1, C = 4 / R;
+  const int half = p.hd / 2, per = half / C, heads = p.H + 2 * p.KV, item = blockIdx.x * 256 + threadIdx.x;
+  if (item >= heads * per) return;
+  const int head = item / per, i = C * (item - head * per), row = R * blockIdx.y, col = head * p.hd + i;
+  const bool second = R == 2 && row + 1 < g.T;
+  float2 cs[R][C];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < C; ++c) cs[r][c] = p.rope_tab[(long long)(p.start_pos + min(row + r, g.T - 1)) * half + i + c];
+  f32x4 a = sum_of_pieces(g, s, first_piece<COLUMNS>(g, s, row, col)), b = sum_of_pieces(g, s, first_piece<COLUMNS>(g, s, row, col + half));
+  if (head < p.H + p.KV) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma clang fp contract(off)
+      const float2 t = cs[e / C][e % C];
+      const float p0 = a[e] * t.x, p1 = b[e] * t.y, p2 = b[e] * t.x, p3 = a[e] * t.y;
+      a[e] = p0 - p1;
+      b[e] = p2 + p3;
+    }
+  }
+  const int kv = head < p.H + p.KV ? head - p.H : head - p.H - p.KV;
+  float *const to = head < p.H ? p.q_rot + ((long long)row * p.H + head) * p.hd + i
+                               : (head < p.H + p.KV ? p.kc : p.vc) + ((long long)kv * p.cap + p.start_pos + row) * p.hd + i;
+  const long long next = head < p.H ? (long long)p.H * p.hd : p.hd;  // floats to the same place of the next row
+  if constexpr (R == 1) {
+    *(f32x4 *)to = a;
+    *(f32x4 *)(to + half) = b;
+  } else {
+    *(f32x2 *)to = f32x2{a.x, a.y};
+    *(f32x2 *)(to + half) = f32x2{b.x, b.y};
+    if (second) {
+      *(f32x2 *)(to + next) = f32x2{a.z, a.w};
+      *(f32x2 *)(to + next + half) = f32x2{b.z, b.w};
+    }
+  }
+}
+
 // The same, and the norm of the whole rows, which the next product reads, in one launch: a workgroup takes a row (COLUMNS 2: two rows), a
 // thread up to two registers of four.  The sums of squares are fp64, as rms_norm.cr has them.  Bound by a launch and two round trips; us, a
 // sum and a norm | this: 45 rows of 8192 -> 2048, 16 pieces, 4.9 + 3.9 | 5.0, of 2048 -> 2048 3.9 + 4.2 | 4.3; 512 rows of 8192 -> 2048, 8
@@ -1292,6 +1335,10 @@ bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
   // (by the kernel that adds the pieces, or by the product itself, but for three-part weights in tiles of 32 rows)
   if (next.swiglu) return !next.norm.rows && N % 8 == 0 && (p.pieces > 1 ? T <= 65535 : !(p.few && p.parts == 3));
   if (p.pieces <= 1) return false;
+  if (const GemvPrep *q = next.prep)
+    return !next.norm.rows && !q->q_norm && !q->k_norm && !q->b_q && !q->b_k && !q->b_v && q->rope_tab && q->hd % 8 == 0 &&
+           (long long)(q->H + 2 * q->KV) * q->hd == N && T <= 65535 && q->start_pos >= 0 && q->start_pos + T <= q->cap &&
+           !(((uintptr_t)q->q_rot | (uintptr_t)q->kc | (uintptr_t)q->vc) & 15);
   const bool pairs = !(p.few && p.parts == 1) && !(p.parts == 1 && p.mb == 4);
   return N % 4 == 0 && N / (pairs ? 2 : 4) <= 2048;
 }
@@ -1375,6 +1422,11 @@ template <int COLUMNS>
 hipError_t launch_sum(const GemmArgs &g, const PieceShape &s, const GemmNext &next, hipStream_t stream) {
   constexpr int R = COLUMNS == 2 ? 2 : 1, C = 4 / R;
   const int N = next.swiglu ? g.N / 2 : g.N, quads = (N + C - 1) / C, rows = (g.T + R - 1) / R;
+  if (next.prep) {
+    hipLaunchKernelGGL((sgemm_sum_prep_kernel<COLUMNS>), dim3((unsigned)((quads / 2 + 255) / 256), (unsigned)rows), dim3(256), 0, stream, g, s,
+                       *next.prep);
+    return hipGetLastError();
+  }
   if (next.norm.rows) {
     const int threads = quads < 1024 ? (quads + 63) / 64 * 64 : 1024;
     hipLaunchKernelGGL((sgemm_sum_norm_kernel<COLUMNS>), dim3((unsigned)rows), dim3(threads), 0, stream, g, s, next.norm);
@@ -1436,10 +1488,11 @@ hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, const GemmNext &n
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
                        unsigned *flags, int *error, int T, int K, int N, const GemmPlan &p, hipStream_t stream,
                        unsigned *flag_set, int spin_limit, const float *bias, Activation act, const GemmNext &next) {
-  if ((next.swiglu || next.norm.rows) && !gemm_takes_next(p, T, N, next)) return hipErrorInvalidValue;
+  const bool more = next.swiglu || next.norm.rows || next.prep;
+  if (more && !gemm_takes_next(p, T, N, next)) return hipErrorInvalidValue;
   if (!x || !w || !y || T < 1 || K < 1 || N < 1 || x_stride < K) return hipErrorInvalidValue;
   const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias | (uintptr_t)next.norm.rows) & 15);
-  if (!aligned && (next.swiglu || next.norm.rows)) return hipErrorInvalidValue;
+  if (!aligned && more) return hipErrorInvalidValue;
   if (!p.mfma || !aligned) {
     hipLaunchKernelGGL(sgemm_plain_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)(T < 65535 ? T : 65535)), dim3(256), 0, stream, x,
                        x_stride, w, y, res, T, K, N, bias, act);

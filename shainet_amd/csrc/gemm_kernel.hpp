@@ -14,8 +14,10 @@ struct NextNorm {
   double eps = 0.0;
   float *rows = nullptr;  // [T, N]: the norm of y's rows goes there (null: none)
 };
+struct GemvPrep;  // attn_kernels.hpp
 struct GemmNext {
   NextNorm norm;
+  const GemvPrep *prep = nullptr;  // N = q | k | v heads, without norms and biases: rotated and put where it says (y is not written)
   bool swiglu = false;  // N = gate | up, and y is [T, N / 2]: silu(gate) * up
 };
 

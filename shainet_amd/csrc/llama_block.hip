@@ -179,7 +179,15 @@ int attn_forward_device(shainet_llama_attn *l, const float *x, int T, float *out
     if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm, &where)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, nullptr, T, l->d_model, wide, stream, qkv))) return rc;
     rc = shainet_attn_finish_prepared(l->ctx, cache, T, l->attn.p, ahead);  // 287-296
+  } else if (GemvPrep where; !fuse_off && T > 1 && !l->has_q_norm && !l->has_k_norm && !l->has_bq && !l->has_bk && !l->has_bv &&
+             !(rc = shainet_attn_begin_prepared(l->ctx, cache, T, &where)) &&
+             Projector::spreads(x, l->w_qkv, l->qkv.p, T, l->d_model, wide, l->w_qkv_bf16, where)) {
+    // many rows: RoPE and the append where the pieces of the product's tiles are added
+    qkv.spread = &where;
+    if ((rc = l->proj.project(x, l->d_model, l->w_qkv, l->qkv.p, T, l->d_model, wide, stream, qkv))) return rc;
+    rc = shainet_attn_finish_prepared(l->ctx, cache, T, l->attn.p, ahead);
   } else {
+    if (rc) return rc;
     if (gemvt_takes(T, l->d_model, wide, qkv.epilogue, qkv.norm)) take_transposed(qkv);
     if ((rc = l->proj.project(x, l->d_model, l->w_qkv, l->qkv.p, T, l->d_model, wide, stream, qkv))) return rc;
     rc = shainet_attn_forward_strided(l->ctx, cache, nullptr, &T, 1, l->qkv.p, l->qkv.p + l->q_dim,

@@ -133,6 +133,7 @@ struct Fused {
   // the same weights transposed ([N, K]; kGemvSwiglu: [2N, K]) or null: one row of x then takes the
   // product that gives a wavefront whole outputs (launch_gemvt) where its shapes allow
   const float *w_t = nullptr;
+  const GemvPrep *spread = nullptr;  // many rows, Projector::spreads: y is q | k | v, whose heads go where it says (y is scratch)
   bool w_bf16 = false;  // every value of W is a bf16 number: half the MFMAs of many rows have nothing to add
   bool any_few_rows = false;  // up to 16 rows run as the split GEMV, not only the ones it is the faster product for
   const float *normed = nullptr;  // [T, K]: the rows of x behind the norm, where an earlier product handed them over (more than a few rows only)
@@ -171,6 +172,8 @@ struct Projector {
   // products are MFMA's, 68 | 72 | 81 | 93 this way; for 8 rows 84 | 80 | 99 | 98 and 77 | 77 | 93 | 94; from 10 rows on
   // the MFMA product is the faster one at any size (width 128, 12 rows: 80, and 85 with the smallest as the split GEMV).
   static bool few_rows(int T, int K, int N, long long x_stride);
+  // Whether the product of many rows [T, K] without gaps puts q | k | v heads where `where` says (Fused::spread).
+  static bool spreads(const float *x, const float *w, const float *y, int T, int K, int N, bool w_bf16, const GemvPrep &where);
   DevF scratch, normed, wide, handed;
   // split products: a word per partial that says when it is complete (zero between launches)
   unsigned *flags = nullptr;
@@ -190,7 +193,8 @@ struct Projector {
   int reserve_flags(size_t n_flags, hipStream_t stream);
   // res != nullptr: y = res + x W
   int gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N, hipStream_t stream, bool w_bf16,
-           const float *res = nullptr, const float *bias = nullptr, Activation act = Activation(), bool swiglu = false, Handover *next = nullptr);
+           const float *res = nullptr, const float *bias = nullptr, Activation act = Activation(), bool swiglu = false, Handover *next = nullptr,
+           const GemvPrep *spread = nullptr);
 };
 
 // Replace *dst (device, hipMalloc'ed or null) by a copy of n host floats.

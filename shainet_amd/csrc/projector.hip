@@ -134,12 +134,15 @@ int Projector::reserve_flags(size_t n_flags, hipStream_t stream) {
 // y = (res +) x W with the library's own MFMA kernel; res == y is allowed.
 // swiglu: W is gate | up and y [T, N / 2].
 int Projector::gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
-                    hipStream_t stream, bool w_bf16, const float *res, const float *bias, Activation act, bool swiglu, Handover *next) {
+                    hipStream_t stream, bool w_bf16, const float *res, const float *bias, Activation act, bool swiglu, Handover *next,
+                    const GemvPrep *spread) {
   const GemmPlan p = plan_gemm(T, K, N, x_stride, w_bf16);
   const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias) & 15);
   GemmNext also;
   also.swiglu = swiglu;
+  also.prep = spread;
   float *result = y;
+  if (spread && !(aligned && gemm_takes_next(p, T, N, also))) return llama_fail(SHAINET_HIP_ERR_ARGUMENT, "this product does not spread heads");
   if (swiglu && !(aligned && gemm_takes_next(p, T, N, also))) {
     if (!wide.reserve((size_t)T * N)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     result = wide.p;
@@ -163,6 +166,12 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
   if (e == hipSuccess && swiglu && !also.swiglu) e = launch_swiglu_act(wide.p, y, T, N / 2, stream);
   if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("gemm launch: ") + hipGetErrorString(e));
   return SHAINET_HIP_OK;
+}
+
+bool Projector::spreads(const float *x, const float *w, const float *y, int T, int K, int N, bool w_bf16, const GemvPrep &where) {
+  GemmNext next;
+  next.prep = &where;
+  return !few_rows(T, K, N, K) && !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) && gemm_takes_next(plan_gemm(T, K, N, K, w_bf16), T, N, next);
 }
 
 bool Projector::few_rows(int T, int K, int N, long long x_stride) {
@@ -275,7 +284,7 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
   }
   if (swiglu) return gemm(xin, xs, w, y, T, K, 2 * N, stream, f.w_bf16, nullptr, nullptr, Activation(), true);
   return gemm(xin, xs, w, y, T, K, N, stream, f.w_bf16, f.epilogue == kGemvResidual ? f.res : nullptr,
-              f.epilogue == kGemvBias ? f.bias : nullptr, f.act, false, f.next);
+              f.epilogue == kGemvBias ? f.bias : nullptr, f.act, false, f.next, f.spread);
 }
 
 void Projector::release() {
