@@ -2,7 +2,7 @@
 //
 // Decode is the absorbed form: per layer one launch that takes the queries to the latent space and
 // appends the new rows, one that attends over key ranges in parallel, one that merges the ranges and
-// takes the result back through W_uv.  All heads share a cached row, so 16 (row, head) pairs are the
+// takes the result back through W_uv; one row over few keys is a single launch (latent_row_kernel).  All heads share a cached row, so 16 (row, head) pairs are the
 // columns of one MFMA tile and a row is read once per 16 of them.
 //
 // MFMA 16x16x4 layout (lane l): A[m = l % 16][k = l / 16], B[k = l / 16][n = l % 16],

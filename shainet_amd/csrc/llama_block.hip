@@ -476,6 +476,7 @@ int wrapped_forward_device(shainet_llama_block *b, const float *x, int T, float 
   if (!w.norm1.gamma || !w.post1) return fail(SHAINET_HIP_ERR_ARGUMENT, "weights not set");
   if (!b->h.reserve(n) || !b->y.reserve(n) || !b->joined.reserve(n) || !b->factors.reserve((size_t)T)) return fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
   const bool carried = carry && carry->y;
+  const int before[2] = {b->conv[0].cur, b->conv[1].cur};
   const ResidualArgs first = joining(b, x, carried ? carry->y : nullptr, carried ? carry->post : nullptr, b->joined.p, w.norm1.gamma, w.conv1,
                                      &b->conv[0], b->h.p, T, no_cache);
   if (carry) carry->y = nullptr;
@@ -499,6 +500,9 @@ int wrapped_forward_device(shainet_llama_block *b, const float *x, int T, float 
       rc = join(joining(b, out, b->y.p, w.post2, out, nullptr, nullptr, nullptr, nullptr, T, no_cache), stream);
     }
   }
+  // (a call that ends early leaves the convolutions' rows as it found them: the buffer that was read is not written)
+  if (rc)
+    for (int i = 0; i < 2; ++i) b->conv[i].cur = before[i];
   if (!rc && !no_cache) b->pos += T;
   return rc;
 }

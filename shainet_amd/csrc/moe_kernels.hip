@@ -746,6 +746,11 @@ __global__ __launch_bounds__(256, 2) void moe_product_kernel(const GroupedArgs g
     }
 }
 
+// (where a call ends early)
+__global__ __launch_bounds__(256) void moe_clear_kernel(int experts, int *counts) {
+  for (int e = threadIdx.x; e < experts; e += 256) counts[e] = 0;
+}
+
 // y[t] (+)= sum over the slots of weight * the expert's row, in the slots' order.  The first workgroup clears the
 // counters for the next call.
 template <int W>
@@ -951,7 +956,11 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
   g.groups = m.experts;
   g.K = m.d;
   g.N = m.ff;
-  if ((e = launch_product(g, tm, true, stream)) != hipSuccess) return e;
+  auto ended = [&]() {
+    hipLaunchKernelGGL(moe_clear_kernel, dim3(1), dim3(256), 0, stream, m.experts, counts);
+    return e;
+  };
+  if ((e = launch_product(g, tm, true, stream)) != hipSuccess) return ended();
   g.x = hidden;
   g.gather = nullptr;
   g.w = w.down;
@@ -959,7 +968,7 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
   g.y = rows_y;
   g.K = m.ff;
   g.N = m.d;
-  if ((e = launch_product(g, tm, false, stream)) != hipSuccess) return e;
+  if ((e = launch_product(g, tm, false, stream)) != hipSuccess) return ended();
   const bool vec = (m.d & 3) == 0;
   const int per = vec ? 1024 : 256;
   const dim3 grid((unsigned)T, (unsigned)((m.d + per - 1) / per));

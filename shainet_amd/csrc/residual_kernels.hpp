@@ -3,8 +3,9 @@
 //   x' = x + y / rms(y) * post           the sublayer's result y joins the residual
 //   h  = x' / rms(x') * pre              what the next sublayer reads, before
 //   h' = h + conv(h)                     and after a causal convolution over time on each channel
-// A single row is one launch.  More rows are two: the first joins y and takes the norms' factors, the second
-// walks the rows of a column for the convolution.  Every part but x can be left out.
+// A single row is one launch, and so are more where nothing is written in place (two to four taps, up to 2048 columns).  Otherwise
+// they are two: the first joins y and takes the norms' factors, the second walks the rows of a column for the convolution.  Every
+// part but x can be left out.
 #pragma once
 #include <hip/hip_runtime.h>
 
