@@ -802,7 +802,9 @@ bool gemvt_takes(int T, int K, int N, int epilogue, int norm, const GemvPrep *pr
 }
 
 bool gemvt_takes_join(int K, int N, int epilogue, int norm) {
-  return (K == 1024 || K == 2048) && N <= 32768 && !norm && (epilogue == kGemvPlain || epilogue == kGemvBias || epilogue == kGemvQkvPrep);
+  // Every workgroup reads what the row is made of, 44 KB per 1024 columns: us, the row's launch, a gap of 0.8 and the product | this:  K 1024,
+  // N 2048 8.9 | 6.1, 3072 9.3 | 6.8, 4096 10.2 | 8.2;  K 2048, N 3072 11.3 | 9.7, 6144 15.0 | 15.4, 8192 18.4 | 20.1.
+  return (K == 1024 || K == 2048) && (long long)N * (K / 1024) <= 6144 && !norm && (epilogue == kGemvPlain || epilogue == kGemvBias || epilogue == kGemvQkvPrep);
 }
 
 hipError_t launch_gemvt(const GemvArgs &args, hipStream_t stream) {
