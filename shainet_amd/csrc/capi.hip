@@ -1128,6 +1128,7 @@ int *shainet_attn_error_word(shainet_attn_ctx *c) { return c ? c->error : nullpt
 int shainet_attn_begin_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, GemvPrep *where) {
   if (!c || !kc || kc->ctx != c || !where)
     return fail(SHAINET_HIP_ERR_ARGUMENT, "context and cache do not belong together");
+  if (int rc = refuse_while_lengths_on_device(kc, "shainet_attn_forward")) return rc;
   if (new_tokens < 1) return fail(SHAINET_HIP_ERR_ARGUMENT, "new_tokens must be positive");
   if ((long long)kc->len[0] + new_tokens > kc->cap)
     return fail(SHAINET_HIP_ERR_CAPACITY, "sequence 0: %d cached + %d new rows exceed capacity %d", kc->len[0],
@@ -1163,6 +1164,7 @@ void shainet_attn_commit_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int
 int shainet_attn_finish_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, float *out, const AheadRows *ahead) {
   if (!c || !kc || kc->ctx != c || !out)
     return fail(SHAINET_HIP_ERR_ARGUMENT, "context and cache do not belong together");
+  if (int rc = refuse_while_lengths_on_device(kc, "shainet_attn_forward")) return rc;
   if (new_tokens < 1 || (long long)kc->len[0] + new_tokens > kc->cap)
     return fail(SHAINET_HIP_ERR_CAPACITY, "sequence 0: %d cached + %d new rows exceed capacity %d", kc->len[0],
                 new_tokens, kc->cap);

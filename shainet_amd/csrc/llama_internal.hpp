@@ -22,7 +22,7 @@ int shainet_attn_forward_strided(shainet_attn_ctx *c, shainet_kv_cache *kc, cons
 
 // capi.hip: the two halves of shainet_attn_forward for one sequence (slot 0 of the
 // cache) when the kernel that produces q | k | v also does the bias / QK-norm / RoPE /
-// append step (the kGemvQkvPrep epilogue).  begin checks the capacity and says where
+// append step (the kGemvQkvPrep epilogue).  Both refuse a cache whose lengths are on the device; begin checks the capacity and says where
 // the prepared rows go; finish runs the attention kernel over them and counts the rows
 // into the cache.  Both are asynchronous on the context's stream.
 int shainet_attn_begin_prepared(shainet_attn_ctx *c, shainet_kv_cache *kc, int new_tokens, shainet::GemvPrep *where);
