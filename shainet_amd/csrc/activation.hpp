@@ -16,28 +16,10 @@ __device__ __forceinline__ float activate(const Activation &a, float z) {
   return z;
 }
 
-// silu(gate) up in fp64 (swiglu_ff.cr:84-89).  2^n times a series for the rest, up to 2^-47 of its value, and a reciprocal refined once to
-// 2^-45: rounded to fp32 the same as the library's exp and a division, in a third of their instructions, which were most of what a
-// launch of them took (512 rows of 2 x 8192 10.6 us).  Infinities and NaN as there.
+// silu(gate) up in fp64 (swiglu_ff.cr:84-89)
 __device__ __forceinline__ float swiglu(float gate, float up) {
-  const double g = (double)gate, z = g * -1.4426950408889634;
-  const double t = fmin(fmax(z, -1100.0), 1000.0), n = rint(t), r = (t - n) * 0.6931471805599453;
-  double p = 1.0 / 39916800;
-  p = fma(p, r, 1.0 / 3628800);
-  p = fma(p, r, 1.0 / 362880);
-  p = fma(p, r, 1.0 / 40320);
-  p = fma(p, r, 1.0 / 5040);
-  p = fma(p, r, 1.0 / 720);
-  p = fma(p, r, 1.0 / 120);
-  p = fma(p, r, 1.0 / 24);
-  p = fma(p, r, 1.0 / 6);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
-  const double d = 1.0 + ldexp(p, (int)n);
-  double q = __builtin_amdgcn_rcp(d);
-  q = fma(fma(-d, q, 1.0), q, q);
-  return (float)((z >= 1024.0 ? g * 0.0 : g * q) * (double)up);
+  const double g = (double)gate;
+  return (float)((g / (1.0 + exp(-g))) * (double)up);
 }
 
 }  // namespace shainet
