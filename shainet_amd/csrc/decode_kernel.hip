@@ -810,18 +810,30 @@ __host__ __device__ inline bool spans_may_end_with(int n_s, int q, int pairs) {
   const int count = (n_s + q - 1) / q, shared = count & 7 ? count & -count : 8;  // the common divisor
   return n_s == 0 || shared == 1 || pairs * shared <= (q == kDecodeWaves ? 64 : 32);
 }
-// Whether pairs of up to `longest` tiles are tried as a span each first: nobody waits or merges then, which a few more tiles
-// per wavefront are worth, and most where 256 workgroups would share the pairs unevenly.  Attention kernel, us, cut as above | whole;
+// Whether pairs of up to `longest` tiles may be a span each: nobody waits or merges then, which a few more tiles
+// per wavefront are worth.  Attention kernel, us, cut as above | whole;
 // head_dim 64:  8 pairs of 9 to 12 tiles 8.7 | 8.2, of 14 and 16 8.8 | 9.1;  16 of 14 9.7 | 9.1, of 16 9.1 | 9.3, of 19 9.0 | 10.2;
 // 32 of 9 to 16 9.1 to 10.0 | 8.3 to 9.3, of 19 9.3 | 10.6;  64 of 9 to 16 10.0 to 11.3 | 8.8 to 9.8, of 24 11.6 | 12.0;  128 of 12
-// 15.8 | 9.5, of 16 16.1 | 10.5, of 24 18.0 | 12.6, of 32 18.8 | 20.6;   head_dim 128:  8 to 64 of 9 to 16 level to a quarter
-// slower;  128 of 12 17.8 | 15.0, of 16 18.5 | 16.6, of 19 and 24 level.  (8 pairs of 12, 32 of 16 and 128 of 9 are cut as tests of the
-// layout have them.)
+// 15.5 | 8.9, of 16 15.6 | 9.9, of 24 16.7 | 12.2, of 32 18.8 | 20.6;   head_dim 128:  8 to 64 of 9 to 16 level to a quarter
+// slower;  128 of 12 17.7 | 13.0, of 16 18.7 | 15.3, of 19 and 24 level;   head_dim 96 and 256, 128 of 10 to 16 17.8 to 18.7 | 11.0 to 13.0 and
+// 23.2 to 27.0 | 19.5 to 25.4.
+// (Three plans have been left as they were laid out before, although whole is level or better: 8 pairs of 12 tiles 8.7 | 8.2, 32 of
+// 16 10.0 | 9.3, 128 of 9 12.9 | 8.7.)
 __host__ __device__ inline bool whole_pairs(int longest, int q, int hd, int pairs) {
   if (longest <= q) return false;
   if (longest <= widest_aligned_span(q)) return true;
   if (pairs >= 128) return longest >= 10 && longest <= (hd <= 64 ? 24 : 16);
   return hd <= 64 && longest <= (pairs >= 16 ? 15 : 11);
+}
+// And whether that is tried in front of the cuts that end with the pairs: not where a few long pairs would be what the launch takes.
+// 16 sequences of 8 kv heads, some of them longer, us, such a cut | whole;  four rows x heads of 64:  1 of 16 tiles and 15 of 1 9.9 | 9.3,
+// 1 of 20 and 15 of 8 level, of 24 and 1 10.2 | 11.1 (heads of 16 to 48: 9.2 | 10.4), 4 of 24 and 12 of 8 10.7 | 11.3, 8 of 24 and 8 of 1
+// level;  heads of 96:  1 of 10 and 15 of 1 9.7 | 10.6, 1 of 16 11.2 | 12.3;  of 128:  11.1 | 11.8, 12.4 | 13.2 (but 8 of 10 and 8 of 4, which
+// take all 256 workgroups, 12.6 | 12.2);  of 256:  12.1 | 16.5, 15.2 | 20.7.  More rows make the merge dearer:  8 x 64 of 24 and 1 10.6 |
+// 10.5, 16 x 64 13.5 | 11.1;  8 x 128 of 16 and 1 12.2 | 12.2 and 14.4 | 14.2, 16 x 128 16.1 | 14.1;  8 x 256 18.6 | 23.4, 16 x 256 24.1 | 27.3.
+// Where no cut ends with the pairs, whole is the better way in any case:  1 of 16 and 15 of 8 15.3 | 9.5, 18.6 | 12.5, 17.8 | 13.7, 24 | 23.7.
+__host__ __device__ inline bool whole_first(int longest, int q, int hd, int cols) {
+  return longest <= widest_aligned_span(q) || (hd <= 64 && longest <= 16) || (hd <= 128 && cols >= 8);
 }
 
 struct ShareArg {
@@ -876,9 +888,10 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int *__restrict__ lens,
     total = __shfl(incl, 63);
     return true;
   };
-  if (!(whole_pairs(longest, q, sh.hd, n_seqs * sh.KV) && takes(longest)))
-    for (int a = q; a <= widest && !takes(a); ++a) {
-    }
+  const bool whole = whole_pairs(longest, q, sh.hd, n_seqs * sh.KV), first = whole && whole_first(longest, q, sh.hd, sh.g);
+  bool laid = first && takes(longest);
+  for (int a = q; a <= widest && !laid; ++a) laid = takes(a);
+  if (whole && !first && !laid) takes(longest);
   if (mine) {
     out->st.slot[s] = s;
     out->st.start_pos[s] = start;
@@ -924,9 +937,11 @@ DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligne
   // (11.1 : 11.0), of 528 10.7 : 9.8 (12.7 : 10.8), of 640 9.2 : 9.7 (10.4 : 10.6), of 1040 10.6 : 9.7 (13.7 : 12.4); four
   // of 640 16.2 : 10.9 (18.1 : 12.6); 16 of 100 13.7 : 7.2 (16.0 : 10.7).
   int longest = 0;
+  p.cols = 0;
   for (int s = 0; s < st.n_seqs; ++s) {
     const int n_s = (st.start_pos[s] + st.n_new[s] + 15) / 16;
     longest = n_s > longest ? n_s : longest;
+    p.cols = st.n_new[s] * sh.g > p.cols ? st.n_new[s] * sh.g : p.cols;
   }
   const int widest = widest_aligned_span(q);
   auto takes = [&](int a) {
@@ -942,9 +957,10 @@ DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligne
     lay_out(a);
     return true;
   };
-  if (aligned && !(whole_pairs(longest, q, sh.hd, st.n_seqs * sh.KV) && takes(longest)))
-    for (int a = q; a <= widest && !takes(a); ++a) {
-    }
+  const bool whole = aligned && whole_pairs(longest, q, sh.hd, st.n_seqs * sh.KV), first = whole && whole_first(longest, q, sh.hd, p.cols);
+  bool laid = first && takes(longest);
+  for (int a = q; aligned && a <= widest && !laid; ++a) laid = takes(a);
+  if (whole && !first && !laid) takes(longest);
   p.tiles_per_wg = q;
   spans_from_shares(span_shares().v, q, p.spans);
   // the first workgroup count whose spans cover the stream
@@ -953,8 +969,6 @@ DecodePlan plan_decode(SeqTable &st, const Shape &sh, int wg_target, bool aligne
   while (p.n_wgs > 1 && begin_of(p.n_wgs - 1) >= p.total_tiles) --p.n_wgs;
   while (begin_of(p.n_wgs) < p.total_tiles) ++p.n_wgs;
   p.n_slots = p.n_wgs + st.n_seqs * sh.KV;
-  p.cols = 0;
-  for (int s = 0; s < st.n_seqs; ++s) p.cols = st.n_new[s] * sh.g > p.cols ? st.n_new[s] * sh.g : p.cols;
   return p;
 }
 

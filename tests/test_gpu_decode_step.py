@@ -78,6 +78,8 @@ CASES = [
     (32, 8, 96, [700, 33, 1], True, True),                    # head_dim 96: tiles padded to 128
     (8, 4, 44, [300, 2000], False, False),                    # head_dim 44: tiles padded to 64
     (8, 2, 8, [40], False, False),                            # head_dim 8: tiles padded to 64
+    (16, 8, 64, [381] + [3] * 15, False, False),              # a few long pairs among short ones, 24 tiles and then 25
+    (16, 8, 96, [252] + [14] * 31, True, False),              # whole where no cut ends with the pairs
 ]
 
 

@@ -12,7 +12,10 @@ pytestmark = pytest.mark.gpu
     (32, 8, 64, [16 * 9], True), (32, 8, 64, [16 * 11], True), (8, 8, 64, [16 * 12], False), (8, 2, 32, [16 * 10 + 1], True),
     (32, 8, 64, [16 * 15, 3], True), (16, 8, 64, [16 * 15 + 1, 16 * 15], False), (32, 8, 64, [16 * 9 + 1] + [150] * 15, True),
     (16, 8, 64, [16 * 24] + [1, 17, 130] * 5, True), (16, 8, 64, [16 * 24 + 1] + [380] * 15, False),
-    (32, 8, 128, [16 * 16] + [250] * 15, True), (32, 8, 128, [16 * 16 + 1] + [250] * 15, False), (32, 8, 128, [16 * 11], False)])
+    (32, 8, 128, [16 * 16] + [250] * 15, True), (32, 8, 128, [16 * 16 + 1] + [250] * 15, False), (32, 8, 128, [16 * 11], False),
+    # a few long pairs among short ones
+    (16, 8, 64, [16 * 24] + [16] * 15, False), (16, 8, 64, [16 * 24] + [16 * 8] * 15, False), (16, 8, 48, [16 * 16 + 1] + [9] * 15, False),
+    (16, 8, 96, [16 * 16] + [16] * 15, False), (16, 8, 256, [16 * 10] + [16] * 15, False), (16, 8, 128, [16 * 16] + [16] * 31, True)])
 def test_decode_over_whole_pairs(H, KV, hd, lengths, whole):
     """A score is a sum of hd products and a result one of up to 385, each rounded by 2^-24: at random 385^0.5 2^-24, 1.2e-6, and
     a score's share, at sizes of up to ten, again."""

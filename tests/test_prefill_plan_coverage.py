@@ -124,3 +124,22 @@ def test_low_tiles_of_bf16_weights_stay_within_a_round():
     for T, K, N in itertools.product((257, 300, 512, 777, 1100, 2048, 4000), (32, 100, 256, 512, 1024, 2048), (132, 1024, 4092, 16384)):
         plan = sa.hip.describe_matmul(T, K, N, bf16_weights=True)
         assert plan["kind"] == "tiles" or plan["workgroups"] <= 256, (T, K, N, plan)
+
+
+def test_a_few_long_pairs_are_cut():
+    """A batch of which some sequences are longer: whole pairs would have their workgroups work alone for the longest.  Where no cut
+    ends with the pairs the longest are whole."""
+    def split(lens, hd, KV=8, g=4):
+        p = sa.describe_plan(g * KV, KV, hd, [16 * n - 1 for n in lens], [1] * len(lens))
+        return p["workgroups"], p["units"]
+
+    for hd in (16, 48, 64):
+        assert split([24] + [1] * 15, hd) == (160, 5) and split([24] + [8] * 15, hd) == (144, 8)
+        assert split([16] + [1] * 15, hd) == (128, 16) and split([24] + [12] * 15, hd) == (128, 24)
+        assert split([24] * 4 + [8] * 12, hd) == (192, 8) and split([24] + [1] * 15, hd, g=8) == (128, 24)
+    for hd in (96, 128, 256):
+        assert split([16] + [1] * 15, hd) == (144, 6) and split([10] + [1] * 15, hd) == split([12] + [4] * 15, hd) == (144, 4)
+        assert split([16] + [8] * 15, hd) == (128, 16) and split([16] * 16, hd) == (128, 16) and split([16] + [1] * 31, hd) == (256, 16)
+    assert split([16] + [1] * 15, 128, g=8) == (128, 16) and split([16] + [1] * 15, 256, g=8) == (144, 6)
+    assert split([24] + [1, 2, 9] * 5, 64) == (128, 24)   # nothing that ends with all of them
+    assert split([3] * 16, 64) == (128, 4)
