@@ -976,7 +976,8 @@ hipError_t launch_moe_many(const MoeShape &m, const MoeTensors &w, const float *
     hipLaunchKernelGGL(moe_combine_kernel<4>, grid, dim3(256), 0, stream, m, h, rows_y, ids, weights, rank, off, add_to_y ? 1 : 0, y, counts);
   else
     hipLaunchKernelGGL(moe_combine_kernel<1>, grid, dim3(256), 0, stream, m, h, rows_y, ids, weights, rank, off, add_to_y ? 1 : 0, y, counts);
-  return hipGetLastError();
+  e = hipGetLastError();
+  return e == hipSuccess ? e : ended();
 }
 
 }  // namespace shainet
