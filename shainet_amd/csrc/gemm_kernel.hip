@@ -1227,17 +1227,20 @@ int stream_quota(int tiles, int steps) {
 
 // W of one part: the tile of sgemm_stream_kernel by an estimate of its time, and whether that kernel is the one to take.
 // Rounds of workgroups times steps times what a step takes, and for pieces 2.95 us and 0.416 us per MB of them written and
-// read: fitted to what each of the four tiles and 128 x 256 take for 80 products of 8 to 1400 rows, K 32 to 8192, N 32 to 16384, of which
-// the choice loses 0.9 % to the best of the five.  Where its loop alone takes more than 17 us or one round of workgroups does
+// read: fitted to what each of the four tiles and 128 x 256 take for 80 products of 8 to 1400 rows, K 32 to 8192, N 32 to 16384 (tiles of
+// 32 x 128 0.475 a step, not 0.483, by 31 products that are nearly level: 65 to 96 rows of 2048 -> 2048, 32 x 128 | 32 x 64, 14.0 | 15.0, 4096 ->
+// 1024 14.5 | 15.3, 768 -> 2048 10.2 | 10.7); of 342 products of 9 to 777 rows the choice loses 1.9 % to the best of the five.  Where its loop alone takes more than 17 us or one round of workgroups does
 // not do, the larger tiles, which read W less often, are level or ahead, and so they are of a loop of four steps in tiles of 96 rows (us,
 // this | 128 x 256): 256 rows of 2048 -> 2048 19.0 | 23.1, 2048 -> 3072 25.6 | 25.5, 2048 -> 4608 35 | 30; 400 rows of 2048 -> 1536 21.4 |
 // 23.8; 512 rows of 1024 -> 1024 12.6 | 21, 1024 -> 3072 20.8 | 25.2; 777 rows of 1024 -> 1024 16.6 | 24.3, 1024 -> 2048 22.1 | 26.0,
-// 1024 -> 3072 35 | 30; 1400 rows of 2048 -> 1024 34 | 31; rounds: 512 rows of 128 -> 16384 30 | 15, 2048 rows of 128 -> 4096 31 | 17.
-// short_rounds: its loop is of four steps, and in several rounds.
-bool choose_stream(GemmPlan &p, int T, int K, int N, bool &short_rounds) {
-  const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.483f}, {1, 4, 0.563f}, {2, 2, 0.506f}, {3, 2, 0.643f}};
-  float least = INFINITY;
-  bool fits = false;
+// 1024 -> 3072 35 | 30; 1400 rows of 2048 -> 1024 34 | 31; rounds: 512 rows of 128 -> 16384 30 | 15, 2048 rows of 128 -> 4096 31 | 17.  The
+// tile that is within these bounds may be the second best, by the 5 % that the estimate is good to: 512 rows of 2048 -> 1024, for which the
+// best one's loop takes 18 us, 19.2 | 24.0, 1024 rows of 2048 -> 512 19.4 | 23.1;  777 rows of 1536 -> 1536, a fifth behind the best, 30.2 | 25.5.
+// few: rows that this kernel takes in any case.  short_rounds: its loop is of four steps, and in several rounds.
+bool choose_stream(GemmPlan &p, int T, int K, int N, bool few, bool &short_rounds) {
+  const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.475f}, {1, 4, 0.563f}, {2, 2, 0.506f}, {3, 2, 0.643f}};
+  float least = INFINITY, least_fitting = INFINITY;
+  int fitting_mb = 0, fitting_kg = 0;
   p.mb = 3;
   p.kg = 2;
   for (const auto &s : shapes) {
@@ -1247,12 +1250,21 @@ bool choose_stream(GemmPlan &p, int T, int K, int N, bool &short_rounds) {
     const long long wgs = tiles * pieces;
     const float turns = (float)((wgs + 255) / 256) * quota * s.step;
     const float us = turns + (pieces > 1 ? 2.95f + 0.416e-6f * 8 * 32 * s.mb * (256 / s.kg) * wgs : 0.f);
+    if (us < least_fitting && wgs <= 256 && turns <= 17.f && !(s.mb == 3 && quota == 4)) {
+      least_fitting = us;
+      fitting_mb = s.mb;
+      fitting_kg = s.kg;
+    }
     if (us >= least) continue;
     least = us;
-    fits = wgs <= 256 && turns <= 17.f && !(s.mb == 3 && quota == 4);
     short_rounds = wgs > 256 && quota == 4;
     p.mb = s.mb;
     p.kg = s.kg;
+  }
+  const bool fits = least_fitting <= 1.05f * least;
+  if (fits && !few) {
+    p.mb = fitting_mb;
+    p.kg = fitting_kg;
   }
   return fits;
 }
@@ -1291,7 +1303,7 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
   if (p.parts == 1) {
     const bool low = p.few;
     bool short_rounds = false;
-    p.few = choose_stream(p, T, K, N, short_rounds) || low;
+    p.few = choose_stream(p, T, K, N, low, short_rounds) || low;
     // (its loop goes by four steps: of up to 64 long rows most are empty, and many rounds of four do not pay, either; as many
     // sums in tiles of 32 rows, us, this | three parts: 48 rows of 32 -> 32000 8.7 | 7.2, 200 rows 29 | 20, 97 rows of 64 -> 32000
     // 15.8 | 14.2, of 128 18.7 | 17.5, but of 128 -> 16384 9.4 | 10.7)

@@ -143,3 +143,16 @@ def test_a_few_long_pairs_are_cut():
     assert split([16] + [1] * 15, 128, g=8) == (128, 16) and split([16] + [1] * 15, 256, g=8) == (144, 6)
     assert split([24] + [1, 2, 9] * 5, 64) == (128, 24)   # nothing that ends with all of them
     assert split([3] * 16, 64) == (128, 4)
+
+
+def test_the_second_best_tile_where_the_best_does_not_fit():
+    """Rows whose best tile by the estimate takes a loop longer than the larger tiles': one hardly behind it is taken instead of those."""
+    def tile(*shape):
+        p = sa.hip.describe_matmul(*shape, bf16_weights=True)
+        return p["kind"], p["tile"], p["pieces"]
+
+    for T, K, N in ((512, 2048, 1024), (480, 2048, 1024), (1024, 2048, 512), (1000, 2048, 512)):
+        assert tile(T, K, N) == ("few", (64, 128), 4)
+    assert tile(777, 1536, 1536)[0] == tile(512, 2048, 2052)[0] == "tiles"   # a fifth behind, or none that fits
+    for T in (65, 80, 96):
+        assert tile(T, 2048, 2048) == ("few", (32, 128), 4)
