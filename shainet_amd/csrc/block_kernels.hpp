@@ -21,9 +21,9 @@ hipError_t launch_transpose(const float *src, float *dst, int rows, int cols, hi
 hipError_t launch_transposed_differ(const float *a, const float *b, int rows, int cols, int *differ, hipStream_t stream);
 // out = a + b, n floats
 hipError_t launch_add(const float *a, const float *b, float *out, long long n, hipStream_t stream);
-// hidden[r, j] = silu(gate_up[r, j]) * gate_up[r, ff + j];  gate_up is [rows, 2*ff]
 // out = x, n floats; either may be pinned host memory
 hipError_t launch_copy_floats(const float *x, float *out, long long n, hipStream_t stream);
+// hidden[r, j] = silu(gate_up[r, j]) * gate_up[r, ff + j];  gate_up is [rows, 2*ff]
 hipError_t launch_swiglu_act(const float *gate_up, float *hidden, int rows, int ff, hipStream_t stream);
 // out[t, :] = table[tokens[t], :] * scale (+ positions[t, :]);  the caller has checked 0 <= tokens[t] < vocab
 hipError_t launch_embed(const float *table, const int *tokens, float *out, int n_tokens, int d_model,

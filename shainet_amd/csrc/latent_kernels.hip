@@ -1218,11 +1218,13 @@ hipError_t launch_latent_out(const float *partials, const float *uv, const float
 }
 
 bool latent_row_fits(const LatentShape &sh, int start_row) {
-  // (the times above, less 5.4 us for a launch and its meetings: 0.047 us per 1000 floats of a head's weights, 0.04 of the keys'.  The
-  // three launches take 18 us and more)
-  const long long keys = sh.window && start_row >= sh.window ? sh.window : (long long)start_row + 1;
+  // (the times above, less 5.4 us for a launch and its meetings: 0.047 us per 1000 floats of a head's weights, 0.04 of the keys', in rows
+  // as wide as the form's lanes take them: 1100 keys of 80 floats 17.6 us, of 144 17.7;  600 keys of 352 22.1, of 416 20.6.  The three launches
+  // take 18 us and more, of more than 64 heads 24 and more: a step of a layer, the launches beside these included, three | this, 128
+  // heads of 64 + 32 and 64, latents of 256, 800 keys 44.7 | 38.0, 1100 47.4 | 43.9;  of 128 + 64 and 128, latents of 512, 480 keys 73 | 60)
+  const long long keys = sh.window && start_row >= sh.window ? sh.window : (long long)start_row + 1, row = sh.row_w <= 320 ? 288 : 576;
   return shape_ok(sh) && start_row >= 0 && (sh.kv_rank & 3) == 0 && sh.row_w <= 576 && sh.H <= 256 &&
-         47LL * (sh.dim + sh.vdim) * sh.kv_rank + 40 * keys * sh.row_w <= 12600000;
+         47LL * (sh.dim + sh.vdim) * (row == 288 ? 256 : 512) + 40 * keys * row <= (sh.H <= 64 ? 12600000 : row == 288 ? 17600000 : 19000000);
 }
 
 hipError_t launch_latent_row(const float *q, const float *uk, const float *uv, const float *sink, const LatentRows &r,

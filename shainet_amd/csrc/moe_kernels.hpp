@@ -32,9 +32,9 @@ struct MoeTensors {
 bool moe_shape_ok(const MoeShape &m);
 
 constexpr int kMoeFewTokens = 8;
-// join (nullable): h, one row, is still to be made by it.
-// y [T, d] for T <= kMoeFewTokens rows h [T, d]; scratch: moe_few_floats(m, T) floats
 size_t moe_few_floats(const MoeShape &m, int T);
+// y [T, d] for T <= kMoeFewTokens rows h [T, d]; scratch: moe_few_floats(m, T) floats.  join (nullable): h, one row, is still to
+// be made by it.
 hipError_t launch_moe_few(const MoeShape &m, const MoeTensors &w, const float *h, float *y, int T, float *scratch,
                           hipStream_t stream, const ResidualArgs *join = nullptr);
 
