@@ -1261,7 +1261,7 @@ bool choose_stream(GemmPlan &p, int T, int K, int N, bool few, bool &short_round
     p.mb = s.mb;
     p.kg = s.kg;
   }
-  const bool fits = least_fitting <= 1.05f * least;
+  const bool fits = fitting_mb > 0 && least_fitting <= 1.05f * least;  // (none: more tiles than this kernel is asked for)
   if (fits && !few) {
     p.mb = fitting_mb;
     p.kg = fitting_kg;

@@ -156,3 +156,10 @@ def test_the_second_best_tile_where_the_best_does_not_fit():
     assert tile(777, 1536, 1536)[0] == tile(512, 2048, 2052)[0] == "tiles"   # a fifth behind, or none that fits
     for T in (65, 80, 96):
         assert tile(T, 2048, 2048) == ("few", (32, 128), 4)
+
+
+def test_no_more_rows_than_a_grid_has_are_cut_into_pieces():
+    """The kernel that adds the pieces has a row per workgroup of its grid's second dimension, which ends at 65535."""
+    for T, K, N, bf16 in itertools.product((65536, 65537, 100000, 131072, 500000, 1 << 21), (4, 64, 100, 1024, 8192, 32768),
+                                           (4, 32, 100, 132, 512, 1024, 3072, 16384), (False, True)):
+        assert sa.hip.describe_matmul(T, K, N, bf16_weights=bf16)["pieces"] == 1, (T, K, N, bf16)
