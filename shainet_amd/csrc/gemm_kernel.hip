@@ -166,7 +166,7 @@ __device__ __forceinline__ void store_swiglu(const GemmArgs &g, int row0, int h,
 // SWIGLU (no pieces): the activation, a launch of 10.6 us behind 512 rows of 2048 -> 2 x 8192 and of 32.5 behind 2048 rows, between which the
 // wide rows were written and read again, happens where the sums are.  Us, both launches | this: 512 rows 113.8 | 99.4, 2048 rows
 // 408 | 358, 777 rows of 1024 -> 2 x 1024 in tiles of sgemm_stream_kernel 29.5 | 22.8; weights of three parts: a block of width 2048 401 | 392 at 384
-// rows, 461 | 451 at 512, level at 2048, of width 1024 264 | 255 at 777.
+// rows, 461 | 451 at 512, of width 1024 264 | 255 at 777; none in tiles of 256 x 256 (gemm_takes_next).
 template <int WM, int WN, int MB, int NB, int PARTS, bool GUARD, bool SWIGLU>
 __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const GemmArgs g) {
   constexpr int TM = 32 * WM * MB, TN = 32 * WN * NB, NT = 64 * WM * WN;
@@ -1340,16 +1340,17 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[6] = p.mfma && K % step_k(p) != 0;
 }
 
-// (the norm of a row takes a workgroup of up to 1024 threads, two registers of four each; rows and their pairs along the grid's second
-// dimension, which ends at 65535)
+// (the norm of a row takes a workgroup of up to 1024 threads, two registers of four each)
 bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
   if (!p.mfma) return false;
-  // (by the kernel that adds the pieces, or by the product itself, but for three-part weights in tiles of 32 rows)
-  if (next.swiglu) return !next.norm.rows && N % 8 == 0 && (p.pieces > 1 ? T <= 65535 : !(p.few && p.parts == 3));
+  // (by the kernel that adds the pieces, or by the product itself, but for three-part weights in tiles of 32 rows, and of 256 x 256, whose
+  // activations nothing else of a compute unit runs beside: us, a launch of its own behind it | in it, 777 rows of 2048 -> 2 x 8192 360 | 380,
+  // 1024 rows 373 | 390, 2048 rows of 1024 -> 2 x 4096 194 | 207; a block of 24 shapes 1 % slower on average)
+  if (next.swiglu) return !next.norm.rows && N % 8 == 0 && (p.pieces > 1 || !(p.parts == 3 && (p.few || p.mb == 4)));
   if (p.pieces <= 1) return false;
   if (const GemvPrep *q = next.prep)
     return !next.norm.rows && !q->q_norm && !q->k_norm && !q->b_q && !q->b_k && !q->b_v && q->rope_tab && q->hd % 8 == 0 &&
-           (long long)(q->H + 2 * q->KV) * q->hd == N && T <= 65535 && q->start_pos >= 0 && q->start_pos + T <= q->cap &&
+           (long long)(q->H + 2 * q->KV) * q->hd == N && q->start_pos >= 0 && q->start_pos + T <= q->cap &&
            !(((uintptr_t)q->q_rot | (uintptr_t)q->kc | (uintptr_t)q->vc) & 15);
   const bool pairs = !(p.few && p.parts == 1) && !(p.parts == 1 && p.mb == 4);
   return N % 4 == 0 && N / (pairs ? 2 : 4) <= 2048;
@@ -1429,7 +1430,8 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
 
 namespace {
 
-// The kernel that adds the pieces; a lane of the product holds COLUMNS neighbouring columns.
+// The kernel that adds the pieces; a lane of the product holds COLUMNS neighbouring columns.  (Rows go along the grid's second dimension,
+// which ends at 65535: no product of as many is cut into pieces.)
 template <int COLUMNS>
 hipError_t launch_sum(const GemmArgs &g, const PieceShape &s, const GemmNext &next, hipStream_t stream) {
   constexpr int R = COLUMNS == 2 ? 2 : 1, C = 4 / R;
@@ -1456,11 +1458,13 @@ hipError_t launch_sum(const GemmArgs &g, const PieceShape &s, const GemmNext &ne
 template <int WM, int WN, int MB, int NB, int PARTS>
 hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups), block(64 * WM * WN);
+  constexpr bool kSwiglu = PARTS == 1 || MB < 4;  // (the others leave it to a launch of its own)
   const bool swiglu = next.swiglu && !g.pieces;
+  if (swiglu && !kSwiglu) return hipErrorInvalidValue;
   if (swiglu && g.K % TK != 0)
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, true>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, kSwiglu>), grid, block, 0, stream, g);
   else if (swiglu)
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false, true>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false, kSwiglu>), grid, block, 0, stream, g);
   else if (g.K % TK != 0)
     hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, false>), grid, block, 0, stream, g);
   else

@@ -1,4 +1,5 @@
-"""SwiGLU where a product's sums are, without pieces, against 64 bits: every tile that does it, columns that do not fill one, K that
+"""SwiGLU where a product's sums are, without pieces, against 64 bits: every tile that does it (and those of 256 x 256 and three parts,
+which leave it to a launch of its own), columns that do not fill one, K that
 does not fill a step, tiles that two workgroups share, and a tile computed again because a value in it is not finite; and the activation by
 itself, in its last bit and far out."""
 import numpy as np
