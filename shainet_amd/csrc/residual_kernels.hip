@@ -366,7 +366,8 @@ hipError_t launch_residual(const ResidualArgs &args, hipStream_t stream) {
 }
 
 bool row_join_fits(const ResidualArgs &a) {
-  // (workgroups read x, y and hist_in while one of them writes)
+  // (workgroups read x, y and hist_in while one of them writes.  JoinRow has no pieces of 1024 columns that are only partly there: rows of
+  // other widths keep the launch of their own)
   return a.T == 1 && (a.d == 1024 || a.d == 2048) && a.x && a.pre && (!a.y || (a.post && a.x_out && a.x_out != a.x && a.x_out != a.y)) &&
          (!a.conv || (a.taps >= 1 && a.taps <= 4)) && (!a.hist_out || a.hist_out != a.hist_in) &&
          !(((uintptr_t)a.x | (uintptr_t)a.y | (uintptr_t)a.post | (uintptr_t)a.x_out | (uintptr_t)a.pre | (uintptr_t)a.conv | (uintptr_t)a.hist_in |
