@@ -1227,18 +1227,20 @@ int stream_quota(int tiles, int steps) {
 
 // W of one part: the tile of sgemm_stream_kernel by an estimate of its time, and whether that kernel is the one to take.
 // Rounds of workgroups times steps times what a step takes, and for pieces 2.95 us and 0.416 us per MB of them written and
-// read: fitted to what each of the four tiles and 128 x 256 take for 80 products of 8 to 1400 rows, K 32 to 8192, N 32 to 16384 (tiles of
-// 32 x 128 0.475 a step, not 0.483, by 31 products that are nearly level: 65 to 96 rows of 2048 -> 2048, 32 x 128 | 32 x 64, 14.0 | 15.0, 4096 ->
-// 1024 14.5 | 15.3, 768 -> 2048 10.2 | 10.7); of 342 products of 9 to 777 rows the choice loses 1.9 % to the best of the five.  Where its loop alone takes more than 17 us or one round of workgroups does
+// read: fitted to what each of the four tiles and 128 x 256 take for 80 products of 8 to 1400 rows, K 32 to 8192, N 32 to 16384, of which
+// the choice loses 0.9 % to the best of the five, and 1.9 % of 342 others of 9 to 777 rows.  (Tiles of 32 x 128 at 0.475 us a step would take 14.0 us
+// where those of 32 x 64 take 15.0 for 65 to 96 rows of 2048 -> 2048, but their errors are larger: 8.05 against 7.96e-8 there, 10.4 against 9.3 for
+// 17 rows of 8192 -> 1536.)  Where a workgroup has more steps than `most`, 15 to 21 us of them, or one round of workgroups does
 // not do, the larger tiles, which read W less often, are level or ahead, and so they are of a loop of four steps in tiles of 96 rows (us,
 // this | 128 x 256): 256 rows of 2048 -> 2048 19.0 | 23.1, 2048 -> 3072 25.6 | 25.5, 2048 -> 4608 35 | 30; 400 rows of 2048 -> 1536 21.4 |
 // 23.8; 512 rows of 1024 -> 1024 12.6 | 21, 1024 -> 3072 20.8 | 25.2; 777 rows of 1024 -> 1024 16.6 | 24.3, 1024 -> 2048 22.1 | 26.0,
 // 1024 -> 3072 35 | 30; 1400 rows of 2048 -> 1024 34 | 31; rounds: 512 rows of 128 -> 16384 30 | 15, 2048 rows of 128 -> 4096 31 | 17.  The
-// tile that is within these bounds may be the second best, by the 5 % that the estimate is good to: 512 rows of 2048 -> 1024, for which the
-// best one's loop takes 18 us, 19.2 | 24.0, 1024 rows of 2048 -> 512 19.4 | 23.1;  777 rows of 1536 -> 1536, a fifth behind the best, 30.2 | 25.5.
+// tile that is within these bounds may be the second best, up to a quarter behind: the sums of 128 x 256 are longer, and their errors twice as large
+// (us and 1e-8 of the norm, this | 128 x 256: 512 rows of 2048 -> 1024 18.2 and 8.1 | 23.4 and 14.0, 777 rows of 1536 -> 1536 28.9 and 8.0 | 25.1 and 17.3,
+// 257 rows of 1280 -> 4608 28.3 and 7.7 | 26.7 and 19.0, 1700 rows of 8192 -> 64 21.9 and 9.4 | 29.0 and 25.3).
 // few: rows that this kernel takes in any case.  short_rounds: its loop is of four steps, and in several rounds.
 bool choose_stream(GemmPlan &p, int T, int K, int N, bool few, bool &short_rounds) {
-  const struct { int mb, kg; float step; } shapes[] = {{1, 2, 0.475f}, {1, 4, 0.563f}, {2, 2, 0.506f}, {3, 2, 0.643f}};
+  const struct { int mb, kg; float step; int most; } shapes[] = {{1, 2, 0.483f, 44}, {1, 4, 0.563f, 36}, {2, 2, 0.506f, 32}, {3, 2, 0.643f, 24}};
   float least = INFINITY, least_fitting = INFINITY;
   int fitting_mb = 0, fitting_kg = 0;
   p.mb = 3;
@@ -1250,8 +1252,9 @@ bool choose_stream(GemmPlan &p, int T, int K, int N, bool few, bool &short_round
     const long long wgs = tiles * pieces;
     const float turns = (float)((wgs + 255) / 256) * quota * s.step;
     const float us = turns + (pieces > 1 ? 2.95f + 0.416e-6f * 8 * 32 * s.mb * (256 / s.kg) * wgs : 0.f);
-    if (us < least_fitting && wgs <= 256 && turns <= 17.f && !(s.mb == 3 && quota == 4)) {
-      least_fitting = us;
+    const float fitting = turns > 17.f ? 1.05f * us : us;  // (long loops are the estimate's weak side: 512 rows of 2048 -> 1024, 32 x 64 21.7 | 64 x 128 19.7)
+    if (fitting < least_fitting && wgs <= 256 && quota <= s.most && !(s.mb == 3 && quota == 4)) {
+      least_fitting = fitting;
       fitting_mb = s.mb;
       fitting_kg = s.kg;
     }
@@ -1261,7 +1264,7 @@ bool choose_stream(GemmPlan &p, int T, int K, int N, bool few, bool &short_round
     p.mb = s.mb;
     p.kg = s.kg;
   }
-  const bool fits = fitting_mb > 0 && least_fitting <= 1.05f * least;  // (none: more tiles than this kernel is asked for)
+  const bool fits = fitting_mb > 0 && least_fitting <= 1.24f * least;  // (none: more tiles than this kernel is asked for)
   if (fits && !few) {
     p.mb = fitting_mb;
     p.kg = fitting_kg;

@@ -875,7 +875,8 @@ def test_matmul_of_bf16_weights_keeps_every_part(hip, T, K, N, inst):
 
 @pytest.mark.parametrize("T,K,N", [(17, 1024, 1024), (17, 2048, 16384), (96, 768, 2304), (97, 8192, 2048), (150, 512, 2048), (150, 2048, 16384),
                                    (150, 8192, 2048), (192, 4096, 4096), (200, 2048, 16384), (777, 8192, 2048), (777, 4096, 4096),
-                                   (1400, 2048, 3072), (1400, 8192, 2048), (80, 2048, 2048), (512, 2048, 1024), (1000, 2048, 512)])
+                                   (1400, 2048, 3072), (1400, 8192, 2048), (512, 2048, 1024), (1000, 2048, 512), (777, 1536, 1536),
+                                   (257, 1280, 4608), (1400, 2048, 260), (1700, 8192, 64)])
 def test_bf16_weights_are_no_less_exact(hip, T, K, N):
     """Against 64 bits, the product that knows its weights to be bf16 numbers and the one that does not: the order of sums may
     differ, what it costs may not grow.  (17408 sums and more: the two are compared to a hundredth.)"""

@@ -145,17 +145,22 @@ def test_a_few_long_pairs_are_cut():
     assert split([3] * 16, 64) == (128, 4)
 
 
-def test_the_second_best_tile_where_the_best_does_not_fit():
-    """Rows whose best tile by the estimate takes a loop longer than the larger tiles': one hardly behind it is taken instead of those."""
+def test_products_of_few_long_sums_stay_in_small_tiles():
+    """The larger tiles' sums are longer, and their errors twice as large: a tile of the small ones that is within its bounds is taken
+    where the best one by the estimate is not, up to a quarter behind it."""
     def tile(*shape):
         p = sa.hip.describe_matmul(*shape, bf16_weights=True)
         return p["kind"], p["tile"], p["pieces"]
 
     for T, K, N in ((512, 2048, 1024), (480, 2048, 1024), (1024, 2048, 512), (1000, 2048, 512)):
         assert tile(T, K, N) == ("few", (64, 128), 4)
-    assert tile(777, 1536, 1536)[0] == tile(512, 2048, 2052)[0] == "tiles"   # a fifth behind, or none that fits
-    for T in (65, 80, 96):
-        assert tile(T, 2048, 2048) == ("few", (32, 128), 4)
+    for T, K, N in ((777, 1536, 1536), (512, 1536, 2304), (257, 1280, 4608), (3000, 1536, 512)):
+        assert tile(T, K, N) == ("few", (96, 128), 2)
+    for T, K, N in ((1400, 2048, 260), (257, 2048, 1616), (1700, 8192, 64), (3000, 4096, 64)):
+        assert tile(T, K, N)[:2] == ("few", (32, 64))
+    for T, K, N in ((600, 1280, 1616), (224, 1280, 4608)):
+        assert tile(T, K, N) == ("few", (32, 128), 1)
+    assert tile(1000, 1280, 2304)[0] == tile(512, 2048, 2052)[0] == "tiles"   # none that fits
 
 
 def test_no_more_rows_than_a_grid_has_are_cut_into_pieces():
