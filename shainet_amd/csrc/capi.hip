@@ -68,6 +68,7 @@ namespace {
 int scratch_on_current_device(unsigned char **out);  // below, with the static scratch of the entry point that allocates nothing
 
 int hip_fail(hipError_t e, const char *what) {
+  (void)hipGetLastError();  // (said here: the next call's first launch would report it as its own)
   return fail(e == hipErrorOutOfMemory ? SHAINET_HIP_ERR_ALLOC : SHAINET_HIP_ERR_RUNTIME, "%s: %s", what,
               hipGetErrorString(e));
 }

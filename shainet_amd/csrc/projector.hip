@@ -28,7 +28,10 @@ bool DevF::reserve(size_t n) {
   float *np = nullptr;
   if (hipMalloc((void **)&np, want * sizeof(float)) != hipSuccess) {
     (void)hipGetLastError();
-    if (hipMalloc((void **)&np, n * sizeof(float)) != hipSuccess) return false;
+    if (hipMalloc((void **)&np, n * sizeof(float)) != hipSuccess) {
+      (void)hipGetLastError();  // (a launch behind this would report it as its own)
+      return false;
+    }
     want = n;
   }
   if (p) (void)hipFree(p);
@@ -148,7 +151,10 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
     result = wide.p;
     also.swiglu = false;
   }
-  // (without the memory for them the rows are normed in front of the next product, as after one that adds no pieces)
+  if (!scratch.reserve(p.partial_floats)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
+  if (int rc = reserve_flags(p.flag_words, stream)) return rc;
+  // (what the product itself needs comes first: without the memory for these rows they are normed in front of the next product, as
+  // after one that adds no pieces)
   if (next && next->norm->kind != kNormNone && !bias && aligned && gemm_takes_next(p, T, N, also) && handed.reserve((size_t)T * N)) {
     also.norm.kind = next->norm->kind;
     also.norm.gamma = next->norm->gamma;
@@ -158,8 +164,6 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
     also.norm.rows = handed.p;
     next->rows = handed.p;
   }
-  if (!scratch.reserve(p.partial_floats)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-  if (int rc = reserve_flags(p.flag_words, stream)) return rc;
   if (p.flag_words && !error) return llama_fail(SHAINET_HIP_ERR_RUNTIME, "the projector has no error word");
   hipError_t e = launch_gemm(x, x_stride, w, result, res, scratch.p, flags, error, T, K, N, p, stream,
                              lose_marks ? flags + flags_cap : nullptr, lose_marks ? 2000 : 0, bias, act, also);

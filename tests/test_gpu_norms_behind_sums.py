@@ -3,8 +3,10 @@ them is handed over, too."""
 import numpy as np
 import pytest
 
+import refmath as rm
 import tutilorn_model as tm
 from test_gpu_bf16_weights import bf16, write
+from test_gpu_model import ATOL, RTOL, _block_pair, _oracle_forward
 from test_gpu_tutilorn import Pair, close
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +102,13 @@ def test_dynamic_tanh_behind_sums(hip, tmp_path, T):
     p = Pair(hip, tmp_path, cfg)
     ids = [int(t) for t in np.random.default_rng(2).integers(0, 260, T)]
     close(p.model.run_rows(ids, range(T)), p.logits(ids), 2e-5)
+
+
+def test_a_call_without_memory_leaves_no_error_behind(hip):
+    """512 GB of hidden rows are not to be had, as rows handed over may not be: the next launch does not report that as its own."""
+    d, ff = 4, 1 << 17
+    blk, ob, p, r, eps = _block_pair(hip, d, 1, 1, 4, ff, 1e6, seed=3, wscale=0.002)
+    with pytest.raises(hip.HipError, match="hipMalloc failed"):
+        blk.forward(np.ones((1 << 20, d), np.float32))
+    x = r.standard_normal((40, d)).astype(np.float32)
+    rm.assert_close(blk.forward_cached(x), _oracle_forward(ob, p, eps, x), ATOL, RTOL, "behind it")
