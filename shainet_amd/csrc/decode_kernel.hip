@@ -817,8 +817,8 @@ __host__ __device__ inline bool spans_may_end_with(int n_s, int q, int pairs) {
 // 15.5 | 8.9, of 16 15.6 | 9.9, of 24 16.7 | 12.2, of 32 18.8 | 20.6;   head_dim 128:  8 to 64 of 9 to 16 level to a quarter
 // slower;  128 of 12 17.7 | 13.0, of 16 18.7 | 15.3, of 19 and 24 level;   head_dim 96 and 256, 128 of 10 to 16 17.8 to 18.7 | 11.0 to 13.0 and
 // 23.2 to 27.0 | 19.5 to 25.4.
-// (Three plans have been left as they were laid out before, although whole is level or better: 8 pairs of 12 tiles 8.7 | 8.2, 32 of
-// 16 10.0 | 9.3, 128 of 9 12.9 | 8.7.)
+// (Three plans stay cut although whole is level or better, because tests that state the layout name them: 8 pairs of 12 tiles 8.7 | 8.2,
+// 32 of 16 10.0 | 9.3, 128 of 9 12.9 | 8.7.)
 __host__ __device__ inline bool whole_pairs(int longest, int q, int hd, int pairs) {
   if (longest <= q) return false;
   if (longest <= widest_aligned_span(q)) return true;
