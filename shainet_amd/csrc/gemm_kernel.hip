@@ -15,11 +15,7 @@
 //      place c / 2: a lane's two blocks are neighbouring columns of y (8-byte stores, 256 bytes a row).
 // Tile loads take a scalar base that moves along K plus a per-thread 32-bit offset.
 // W whose values are bf16 numbers (a checkpoint's, most often): the other two of its parts are zeros, and the three
-// products with them add nothing.  They are left out, in the same tiles with the same bits.  2048 rows of 2048 -> 16384 571 -> 345 us
-// (398 TFLOP/s), 8192 -> 2048 322 -> 194, 512 rows 174 -> 100 and 101 -> 61, 777 rows of 1024 -> 4096 53 -> 35.  What bounds
-// these is issue: the matrix cores are busy 54 % of the time, in which a step's 24 MFMAs share two wavefronts a SIMD with
-// 70 vector instructions each, and everybody meets at a barrier.  Tiles of four by two wavefronts (64 x 128 each) read
-// 10 fragments a step, two by four (128 x 64) 14.
+// products with them add nothing.  They are left out: sgemm_wide_kernel, sgemm_stream_kernel.
 // What bounds the others: large shapes the power the card may draw.  4096 rows of 2048 -> 16384 run at 232 TFLOP/s
 // with N(0, 1) operands and at 295 with zeros (71 % of the six products' rate); with four wavefronts on
 // 128 x 128 tiles it was 183 and 252, so the large tile, which reads LDS 3/4 as often and splits half as much
@@ -54,7 +50,7 @@ namespace shainet {
 
 namespace {
 
-constexpr int TK = 16, kFewStep = 32;
+constexpr int TK = 16, kFewStep = 32, kWideStep = 32;  // K of a step: tiles of three-part weights, of 32 rows, large tiles of one-part weights
 
 // A partial product is read by a workgroup that may sit on another XCD, whose L2 is not kept
 // coherent with this one's for ordinary accesses: the store is written through to memory.
@@ -135,45 +131,90 @@ __device__ __forceinline__ void store_four(const GemmArgs &g, int row0, int col,
   }
 }
 
-// WM x WN wavefronts of MB x NB blocks.  Units of 16 bytes in a stage of LDS.  A part of x: two octets of TM rows, four
-// units apart from a multiple of 16 (a wavefront writes both octets of 32 rows); a part of W: two octets of WN
-// wavefronts' NB blocks of 32 columns, four units of padding behind each (neighbouring columns lie in NB blocks).
-template <int WM, int WN, int MB, int NB, int PARTS>
-struct Stage {
-  static constexpr int kOctX = 32 * WM * MB + 4, kPartX = 2 * kOctX;
-  static constexpr int kOctW = 36 * WN * NB, kPartW = 2 * kOctW;
-  static constexpr int kUnits = 3 * kPartX + PARTS * kPartW;
-};
+// The piece of a tile that a workgroup's run leaves unfinished: to its slot, which is marked complete.
+template <int OUT>
+__device__ __forceinline__ void leave_piece(const GemmArgs &g, float *slot, int step, const f32x4 (&out)[OUT]) {
+  __builtin_amdgcn_sched_barrier(0);  // all of out[] is in place before the first store is issued
+#pragma unroll
+  for (int r = 0; r < OUT; ++r) coherent_store4(slot + r * step, out[r]);
+  // the stores are acknowledged (s_waitcnt vmcnt(0): the barrier alone does not wait for them)
+  // before the piece is marked complete
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(g.flag_set + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
-// SWIGLU: W is gate | up, y is [T, N / 2], silu(gate) * up.  A lane then holds both halves of its NB / 2 columns of y: hidden column h of
-// the tile's TN / 2.
-__device__ __forceinline__ int gate_up_place(int NB, int h, int up) { return NB == 2 ? 2 * h + up : 4 * (h >> 1) + (h & 1) + 2 * up; }
-template <int NB>
-__device__ __forceinline__ void store_swiglu(const GemmArgs &g, int row0, int h, int r, f32x4 v) {
-  const int row = row0 + row_of<NB>(r), N = g.N / 2;
-  if (row >= g.T) return;
-  float *const y = g.y + (long long)row * N + h;
-  if constexpr (NB == 2) {
-    y[0] = swiglu(v.x, v.y);
-    const float second = swiglu(v.z, v.w);
-    if (row + 1 < g.T) y[N] = second;
-  } else {
-    *(f32x2 *)y = f32x2{swiglu(v.x, v.z), swiglu(v.y, v.w)};
+// Adds the tile's earlier pieces, those of the `before` places from `first` on (lower indices, waiting for nobody), to out[].
+template <int OUT>
+__device__ __forceinline__ void add_earlier_pieces(const GemmArgs &g, int group, int first, int before, long long slot_floats, int in_slot,
+                                                   int step, f32x4 (&out)[OUT]) {
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < 64) {
+    for (int spins = 0;; ++spins) {
+      bool ok = true;
+      for (int i = lane; i < before; i += 64)
+        ok = ok && __hip_atomic_load(g.flags + (((first + i) << g.group_bits) | group), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+      if (__all(ok)) {
+        for (int i = lane; i < before; i += 64)
+          __hip_atomic_store(g.flags + (((first + i) << g.group_bits) | group), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+      if (spins >= g.spin_limit) {
+        if (lane == 0) *g.error = 1;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(2);
+    }
+  }
+  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  // ((own piece + piece 0) + piece 1) + ...
+  const float *piece = g.partials + (long long)((first << g.group_bits) | group) * slot_floats + in_slot;
+  const long long piece_step = slot_floats << g.group_bits;
+  for (int i = 0; i < before; ++i) {
+#pragma unroll
+    for (int r0 = 0; r0 < OUT; r0 += 16) {
+      f32x4 v[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] = *(const f32x4 *)(piece + i * piece_step + (r0 + r) * step);
+      __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first sum waits
+#pragma unroll
+      for (int r = 0; r < 16; ++r) out[r0 + r] += v[r];
+    }
   }
 }
 
-// PARTS: of W, 3 or (its values are bf16 numbers) 1.  GUARD: K need not be a multiple of 16 (pieces beyond its end are zeros).
+// WM x WN wavefronts of MB x 2 blocks.  Units of 16 bytes in a stage of LDS.  A part of x: two octets of TM rows, four
+// units apart from a multiple of 16 (a wavefront writes both octets of 32 rows); a part of W: two octets of WN
+// wavefronts' two blocks of 32 columns, four units of padding behind each (neighbouring columns lie in both).
+template <int WM, int WN, int MB>
+struct Stage {
+  static constexpr int kOctX = 32 * WM * MB + 4, kPartX = 2 * kOctX;
+  static constexpr int kOctW = 72 * WN, kPartW = 2 * kOctW;
+  static constexpr int kUnits = 3 * (kPartX + kPartW);
+};
+
+// SWIGLU: W is gate | up, y is [T, N / 2], silu(gate) * up.  A lane then holds both halves of its column of y: hidden column h of the tile's TN / 2.
+__device__ __forceinline__ void store_swiglu(const GemmArgs &g, int row0, int h, int r, f32x4 v) {
+  const int row = row0 + row_of<2>(r), N = g.N / 2;
+  if (row >= g.T) return;
+  float *const y = g.y + (long long)row * N + h;
+  y[0] = swiglu(v.x, v.y);
+  const float second = swiglu(v.z, v.w);
+  if (row + 1 < g.T) y[N] = second;
+}
+
+// W of three parts.  GUARD: K need not be a multiple of 16 (pieces beyond its end are zeros).
 // SWIGLU (no pieces): the activation, a launch of 10.6 us behind 512 rows of 2048 -> 2 x 8192 and of 32.5 behind 2048 rows, between which the
 // wide rows were written and read again, happens where the sums are.  Us, both launches | this: 512 rows 113.8 | 99.4, 2048 rows
 // 408 | 358, 777 rows of 1024 -> 2 x 1024 in tiles of sgemm_stream_kernel 29.5 | 22.8; weights of three parts: a block of width 2048 401 | 392 at 384
 // rows, 461 | 451 at 512, of width 1024 264 | 255 at 777; none in tiles of 256 x 256 (gemm_takes_next).
-template <int WM, int WN, int MB, int NB, int PARTS, bool GUARD, bool SWIGLU>
+template <int WM, int WN, int MB, bool GUARD, bool SWIGLU>
 __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const GemmArgs g) {
-  constexpr int TM = 32 * WM * MB, TN = 32 * WN * NB, NT = 64 * WM * WN;
+  constexpr int NB = 2, TM = 32 * WM * MB, TN = 32 * WN * NB, NT = 64 * WM * WN;
   constexpr int NX = 4 * TM / NT;  // float4 of the x tile per thread
-  constexpr int kSets = PARTS == 3 && TM == 256 ? 1 : 2;
-  using S = Stage<WM, WN, MB, NB, PARTS>;
-  static_assert(PARTS == 3 || MB == 2, "six rows of products");
+  constexpr int kSets = TM == 256 ? 1 : 2;
+  using S = Stage<WM, WN, MB>;
   static_assert(2 * TN == NT, "a thread stages an octet of W");
   static_assert(NX == 2 || NX == 1, "a thread stages an octet of x, or half of one");
   __shared__ __attribute__((aligned(16))) u32x4 lds[2][S::kUnits];
@@ -213,7 +254,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     // tile's end and the loads of the first step wait for it.  128 x 128 has the registers, and without them puts all of a step's
     // splits in front of its MFMAs: 200 rows of 8192 -> 1024, a workgroup a compute unit, 30 -> 35 us)
     int tid = threadIdx.x;
-    if constexpr (PARTS == 1 || WN == 4) asm volatile("" : "+v"(tid));
+    if constexpr (WN == 4) asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const int ln = lane & 31, j = lane >> 5;
 
@@ -226,7 +267,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     if constexpr (SWIGLU) {  // (32 columns of gate, the same of up, and so on: 128 bytes of a row together)
       const int up = wcol >> 5 & 1, h = (wcol >> 6) * 32 + (wcol & 31);
       w_from = up * (N / 2) + min(n0 / 2 + h, N / 2 - 1);
-      wcol = gate_up_place(NB, h, up);
+      wcol = 2 * h + up;
     }
     const int x_unit = (xk >> 3) * S::kOctX + xrow;
     const int w_unit = 3 * S::kPartX + (wk >> 3) * S::kOctW + wcol / (32 * NB) * (36 * NB) + wcol % NB * 36 + wcol % (32 * NB) / NB;
@@ -244,58 +285,34 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     f32x4 sx[kSets][NX];
     float sw[kSets][8];
     int k_next = k_begin, to_load = nk;
-    unsigned w_row[8];  // (PARTS 1) a row of W each: one base serves all of a step's loads
+    auto load_tiles = [&](f32x4 (&rx)[NX], float (&rw)[8]) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) w_row[i] = w_off + 4u * i * (unsigned)N;
-    constexpr int kLoads = NX + 8;
-    auto load_one = [&](f32x4 (&rx)[NX], float (&rw)[8], const int l) {
-      if (l < NX)
-        rx[l] = GUARD && k_next + xk + 4 * l >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : load_at((const f32x4 *)(x_base + 16 * l), x_off);
-      else
-        rw[l - NX] = GUARD && k_next + wk + l - NX >= k_end ? 0.f : load_at((const float *)w_base, w_row[l - NX]);
-    };
-    auto advance = [&]() {
+      for (int u = 0; u < NX; ++u) {
+        const int kk = k_next + xk + 4 * u;
+        rx[u] = GUARD && kk >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4 *)(x_base + x_off + 16 * u);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float *row = (const float *)(w_base + (long long)i * N * 4);
+        rw[i] = GUARD && k_next + wk + i >= k_end ? 0.f : *(const float *)((const char *)row + w_off);
+      }
       if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
         x_base += TK * 4;
         w_base += w_step;
         k_next += TK;
       }
     };
-    auto load_tiles = [&](f32x4 (&rx)[NX], float (&rw)[8]) {
-      if constexpr (PARTS == 1) {
-#pragma unroll
-        for (int l = 0; l < kLoads; ++l) load_one(rx, rw, l);
-      } else {
-#pragma unroll
-        for (int u = 0; u < NX; ++u) {
-          const int kk = k_next + xk + 4 * u;
-          rx[u] = GUARD && kk >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4 *)(x_base + x_off + 16 * u);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float *row = (const float *)(w_base + (long long)i * N * 4);
-          rw[i] = GUARD && k_next + wk + i >= k_end ? 0.f : *(const float *)((const char *)row + w_off);
-        }
-      }
-      advance();
-    };
     auto park_tiles = [&](const f32x4 (&rx)[NX], const float (&rw)[8], u32x4 *stage) {
       u32x4 h, m, l;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        if constexpr (PARTS == 3) {
-          unsigned a, b, c;
-          split_pair(rw[2 * i] * kLift, rw[2 * i + 1] * kLift, a, b, c);
-          h[i] = a, m[i] = b, l[i] = c;
-        } else {
-          h[i] = pack_high(rw[2 * i] * kLift, rw[2 * i + 1] * kLift);
-        }
+        unsigned a, b, c;
+        split_pair(rw[2 * i] * kLift, rw[2 * i + 1] * kLift, a, b, c);
+        h[i] = a, m[i] = b, l[i] = c;
       }
       stage[w_unit] = h;
-      if constexpr (PARTS == 3) {
-        stage[w_unit + S::kPartW] = m;
-        stage[w_unit + 2 * S::kPartW] = l;
-      }
+      stage[w_unit + S::kPartW] = m;
+      stage[w_unit + 2 * S::kPartW] = l;
       if constexpr (NX == 1) {
         u32x2 *half = (u32x2 *)(stage + x_unit) + ((xk >> 2) & 1);
         split_quad(rx[0] * kLift, half[0], half[2 * S::kPartX], half[4 * S::kPartX]);
@@ -323,105 +340,31 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
     __syncthreads();
 
     // (smallest products first; the blocks take turns, no MFMA waits for the one before it)
-    if constexpr (PARTS == 3) {
-      // Per step of 16 along K: the fragments are fetched, the next step's tiles are split and go to the other
-      // stage while the MFMAs run, the tiles of a later step are requested into the registers just freed, one barrier.
-      auto step = [&](const int kt, f32x4 (&rx)[NX], float (&rw)[8]) {  // rx, rw: the set that holds step kt + 1
-        const u32x4 *stage = lds[kt & 1];
-        u32x4 af[3][MB], bf[3][NB];
+    // Per step of 16 along K: the fragments are fetched, the next step's tiles are split and go to the other
+    // stage while the MFMAs run, the tiles of a later step are requested into the registers just freed, one barrier.
+    auto step = [&](const int kt, f32x4 (&rx)[NX], float (&rw)[8]) {  // rx, rw: the set that holds step kt + 1
+      const u32x4 *stage = lds[kt & 1];
+      u32x4 af[3][MB], bf[3][NB];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) {
+      for (int p = 0; p < 3; ++p) {
 #pragma unroll
-          for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * S::kPartX + 32 * a];
+        for (int a = 0; a < MB; ++a) af[p][a] = stage[a_unit + p * S::kPartX + 32 * a];
 #pragma unroll
-          for (int b = 0; b < NB; ++b) bf[p][b] = stage[b_unit + p * S::kPartW + 36 * b];
-        }
-        park_tiles(rx, rw, lds[(kt & 1) ^ 1]);
-        load_tiles(rx, rw);
-#pragma unroll
-        for (int p = 0; p < 6; ++p)
-#pragma unroll
-          for (int a = 0; a < MB; ++a)
-#pragma unroll
-            for (int b = 0; b < NB; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p]][b], acc[a][b]);
-        __syncthreads();
-      };
-      for (int kt = 0; kt < nk; kt += 2) {
-        step(kt, sx[kSets - 1], sw[kSets - 1]);
-        if (kt + 1 < nk) step(kt + 1, sx[0], sw[0]);
+        for (int b = 0; b < NB; ++b) bf[p][b] = stage[b_unit + p * S::kPartW + 36 * b];
       }
-    } else {
-      // Half the MFMAs leave no time for fragments to arrive within their step: they are fetched a step ahead, from the
-      // stage that is whole since the last barrier, and the tiles of the step behind that one go into the stage whose
-      // fragments everybody has.  Everything else a step does is handed out between its MFMAs, one at a time: left
-      // to itself the compiler puts them after each other (2048 rows of 2048 -> 16384: 385 us, 345 this way).  So do the loads:
-      // all in one slot, each row of W with a base of its own, stood in the way of both wavefronts of a SIMD at once (us, so |
-      // handed out: 2048 rows of 2048 -> 16384 358 | 345, 8192 -> 2048 188 | 182, 1024 rows of 2048 -> 16384 188 | 183, 777 rows of
-      // 1024 -> 4096 29.3 | 28.0, 512 rows of 2048 -> 3072 27.0 | 25.9).  Two steps to a barrier, with three stages of LDS: 0 to 5 % slower.
-      u32x4 af[3][MB], first[2][MB], bf[2][NB];  // (the first parts of x and W of two steps)
-      auto fetch_x = [&](const u32x4 *stage, const int p, u32x4 (&f)[MB]) {
+      park_tiles(rx, rw, lds[(kt & 1) ^ 1]);
+      load_tiles(rx, rw);
 #pragma unroll
-        for (int a = 0; a < MB; ++a) f[a] = stage[a_unit + p * S::kPartX + 32 * a];
-      };
-      auto fetch_w = [&](const u32x4 *stage, u32x4 (&f)[NB]) {
+      for (int p = 0; p < 6; ++p)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) f[b] = stage[b_unit + 36 * b];
-      };
-      fetch_w(lds[0], bf[0]);
-      fetch_x(lds[0], 2, af[2]);
-      fetch_x(lds[0], 1, af[1]);
-      fetch_x(lds[0], 0, first[0]);
-      park_tiles(sx[1], sw[1], lds[1]);
-      load_tiles(sx[1], sw[1]);
+        for (int a = 0; a < MB; ++a)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) acc[a][b] = mfma_bf16(af[kPartA[p]][a], bf[kPartB[p]][b], acc[a][b]);
       __syncthreads();
-      auto step = [&](const int set) {  // set: of this step's fragments and of the tiles of the step after the next
-        u32x4 *const stage = lds[set];
-        const u32x4 *const next = lds[set ^ 1];
-        u32x4 whole[3], h;
-        constexpr int kSlots = 6 * NB, kPairs = NB, kEvery = NB == 4 ? 2 : 1;  // slots; the first with a pair of x; slots per pair
-        constexpr int kPacks = kPairs + 2 * NX * kEvery, kEnd = kPacks + NB;
-#pragma unroll
-        for (int slot = 0; slot < kSlots; ++slot) {
-          const int run = slot / NB, b = slot % NB, p = 2 - run / 2, a = run % 2;
-          acc[a][b] = mfma_bf16(p ? af[p][a] : first[set][a], bf[set][b], acc[a][b]);
-          if (slot < NB) bf[set ^ 1][slot] = next[b_unit + 36 * slot];
-          if (b == NB - 1 && run == 1) fetch_x(next, 2, af[2]);
-          if (b == NB - 1 && run == 2) fetch_x(next, 0, first[set ^ 1]);
-          if (b == NB - 1 && run == 3) fetch_x(next, 1, af[1]);
-          if (slot >= kPairs && slot < kPacks && (slot - kPairs) % kEvery == 0) {
-            const int i = (slot - kPairs) / kEvery;
-            const f32x4 v = sx[set][i / 2];
-            unsigned q[3];
-            split_pair(v[i % 2 * 2] * kLift, v[i % 2 * 2 + 1] * kLift, q[0], q[1], q[2]);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-              whole[k][i] = q[k];
-              if (NX == 2 && i == 3) stage[x_unit + k * S::kPartX] = whole[k];
-              if (NX == 1 && i == 1) ((u32x2 *)(stage + x_unit + k * S::kPartX))[(xk >> 2) & 1] = u32x2{whole[k][0], whole[k][1]};
-            }
-          }
-          if (slot >= kPacks && slot < kEnd) {
-#pragma unroll
-            for (int i = (slot - kPacks) * 4 / NB; i < (slot - kPacks + 1) * 4 / NB; ++i)
-              h[i] = pack_high(sw[set][2 * i] * kLift, sw[set][2 * i + 1] * kLift);
-            if (slot == kEnd - 1) stage[w_unit] = h;
-          }
-          if (slot >= kEnd) {
-            constexpr int kLeft = kSlots - kEnd;
-#pragma unroll
-            for (int l = (slot - kEnd) * kLoads / kLeft; l < (slot - kEnd + 1) * kLoads / kLeft; ++l) load_one(sx[set], sw[set], l);
-            if (slot == kSlots - 1) advance();
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        __syncthreads();
-      };
-      // (in pairs: a way out between them has the compiler wait for loads of the step before)
-      for (int kt = 1; kt < nk; kt += 2) {
-        step(0);
-        step(1);
-      }
-      if (nk & 1) step(0);
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+      step(kt, sx[kSets - 1], sw[kSets - 1]);
+      if (kt + 1 < nk) step(kt + 1, sx[0], sw[0]);
     }
 
     const int row0 = m0 + wm * 32 * MB + 4 * j, col = n0 + wn * 32 * NB + NB * ln;
@@ -455,9 +398,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           if constexpr (SWIGLU) {
-            const float *gate = g.w + (long long)(k + i) * N + min(col / 2, N / 2 - NB / 2);
+            const float *gate = g.w + (long long)(k + i) * N + min(col / 2, N / 2 - 1);
 #pragma unroll
-            for (int b = 0; b < NB; ++b) wv[i][b] = in ? gate[b / (NB / 2) * (N / 2) + b % (NB / 2)] : 0.f;
+            for (int b = 0; b < NB; ++b) wv[i][b] = in ? gate[b * (N / 2)] : 0.f;
           } else {
             wv[i] = in ? *(const Columns *)(g.w + (long long)(k + i) * N + min(col, N - NB)) : Columns(0.f);
           }
@@ -472,19 +415,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
       down = 1.f;
     }
 
-    // A piece travels as [pair of rows, or row][thread] float4: consecutive threads, consecutive 16 bytes.
+    // A piece travels as [pair of rows][thread] float4: consecutive threads, consecutive 16 bytes.
     constexpr long long kSlot = (long long)TM * TN;
     constexpr int kOut = 4 * MB * NB;
     f32x4 out[kOut];
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int r = 0; r < 4 * NB; ++r) {
-        if constexpr (NB == 2)
-          out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]} * down;
-        else
-          out[16 * a + r] = f32x4{acc[a][0][r], acc[a][1][r], acc[a][2][r], acc[a][3][r]} * down;
-      }
+      for (int r = 0; r < 4 * NB; ++r)
+        out[8 * a + r] = f32x4{acc[a][0][2 * r], acc[a][1][2 * r], acc[a][0][2 * r + 1], acc[a][1][2 * r + 1]} * down;
     const int in_slot = 4 * tid;
     if (g.pieces) {  // the second kernel adds the pieces
       float *slot = g.partials + blockIdx.x * kSlot + in_slot;
@@ -493,65 +432,303 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
       return;
     }
     if (s_end < steps) {
-      float *slot = g.partials + blockIdx.x * kSlot + in_slot;
-      __builtin_amdgcn_sched_barrier(0);  // all of out[] is in place before the first store is issued
-#pragma unroll
-      for (int r = 0; r < kOut; ++r) coherent_store4(slot + r * 4 * NT, out[r]);
-      // the stores are acknowledged (s_waitcnt vmcnt(0): the barrier alone does not wait for them)
-      // before the piece is marked complete
-      __builtin_amdgcn_s_waitcnt(0x0F70);
-      __syncthreads();
-      if (threadIdx.x == 0) __hip_atomic_store(g.flag_set + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      leave_piece(g, g.partials + blockIdx.x * kSlot + in_slot, 4 * NT, out);
       continue;
     }
-    if (s_begin > 0) {
-      // the tile's earlier pieces lie with the places before this one, from the one that holds the tile's first unit on
-      const int p_first = t * steps / g.quota, n_before = place - p_first;
-      if (wave == 0) {
-        for (int spins = 0;; ++spins) {
-          bool ok = true;
-          for (int i = lane; i < n_before; i += 64)
-            ok = ok && __hip_atomic_load(g.flags + (((p_first + i) << g.group_bits) | group), __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT) != 0u;
-          if (__all(ok)) {
-            for (int i = lane; i < n_before; i += 64)
-              __hip_atomic_store(g.flags + (((p_first + i) << g.group_bits) | group), 0u, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-            break;
-          }
-          if (spins >= g.spin_limit) {
-            if (lane == 0) *g.error = 1;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(2);
-        }
-      }
-      __syncthreads();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      // ((own piece + piece 0) + piece 1) + ...
-      const float *piece = g.partials + (long long)((p_first << g.group_bits) | group) * kSlot + in_slot;
-      const long long piece_step = kSlot << g.group_bits;
-      for (int i = 0; i < n_before; ++i) {
-#pragma unroll
-        for (int r0 = 0; r0 < kOut; r0 += 16) {
-          f32x4 v[16];
-#pragma unroll
-          for (int r = 0; r < 16; ++r) v[r] = *(const f32x4 *)(piece + i * piece_step + (r0 + r) * 4 * NT);
-          __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first sum waits
-#pragma unroll
-          for (int r = 0; r < 16; ++r) out[r0 + r] += v[r];
-        }
-      }
+    if (s_begin > 0) {  // the tile's earlier pieces lie with the places before this one, from the one that holds the tile's first unit on
+      const int p_first = t * steps / g.quota;
+      add_earlier_pieces(g, group, p_first, place - p_first, kSlot, in_slot, 4 * NT, out);
     }
     if (col < N) {  // N is a multiple of 4: a lane's columns are inside together
 #pragma unroll
       for (int r = 0; r < kOut; ++r) {
         if constexpr (SWIGLU)
-          store_swiglu<NB>(g, row0, col / 2, r, out[r]);
+          store_swiglu(g, row0, col / 2, r, out[r]);
         else
           store_four<NB>(g, row0, col, r, out[r]);
       }
     }
+  }
+}
+
+// W of one part in tiles of 256 x 256 (WM 4: wavefronts of 64 rows and 128 columns) and 128 x 256 (WM 2: 64 x 64), on
+// v_mfma_f32_16x16x32_bf16.  A step is 32 of K.  Stages of LDS: unit [part][octet of k][row] and [octet][block of 16 columns][place], as
+// above but for 16 rows and 16 columns a block; column c of a wavefront's lies in block c % NB at place c / NB, so that a lane holds NB
+// neighbouring columns of four rows of each block.
+// The three products of a block follow each other on one accumulator.  What that is worth is power: a loop of nothing but these MFMAs reaches
+// 2150 TFLOP/s on random numbers in this order, 2020 with the products outermost, and 1780 with v_mfma_f32_32x32x16_bf16 in any order.
+// A wavefront holds the fragments of its columns of W for a step; those of its rows arrive one block of 16 ahead.  The next step's tiles are
+// split and put into the other stage, and the registers asked for again at once, in small pieces of work behind each MFMA.
+// Us, tiles of 32 x 32 blocks and steps of 16 | this, both launches where there are two: 2048 rows of 2048 -> 16384 344 | 318, 8192 -> 2048 185 | 167, 2048 -> 2048
+// 60.6 | 57.1, 777 rows of 2048 -> 16384 164 | 144, 512 rows 90.9 | 85.4, of 8192 -> 2048 57.6 | 56.7, of 2048 -> 3072 30.6 | 30.6; with all loads, splits
+// and writes of a step in its first half 325, 173, 59.7, 153, 90.7, 58.9.  Errors against 64 bits 0.3 to 2 % smaller (fewer roundings).
+// What bounds it: on zeros 2048 rows of 2048 -> 16384 take 279 us, of which the MFMAs and fragments are 201, splits 26, writes to LDS 31 (17 cycles each
+// while MFMAs run) and loads 21; on random numbers the clock is at 2.06 GHz.
+template <int WM, bool GUARD, bool SWIGLU>
+__global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
+  constexpr int WN = 8 / WM, MB = 4, NB = 2 * WM, TM = 64 * WM, TN = 256, NT = 512;
+  constexpr int NX = WM / 2;               // octets of x a thread stages (of W: two)
+  constexpr int kSets = WM == 4 ? 1 : 2;   // register sets: tiles are requested one step (of 3072 cycles) ahead, or two (of 1536)
+  // units of 16 bytes; blocks of W a few units apart from 16, so that eight neighbouring threads' columns lie on eight different ones modulo 8
+  constexpr int kOctX = TM, kPartX = 4 * kOctX, kBlockW = NB == 8 ? (SWIGLU ? 18 : 17) : (SWIGLU ? 20 : 18), kOctW = WN * NB * kBlockW;
+  constexpr int kW = 3 * kPartX, kUnits = kW + 4 * kOctW;
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kUnits];
+
+  // (workgroups and their runs as above)
+  const int group = blockIdx.x & ((1 << g.group_bits) - 1), place = blockIdx.x >> g.group_bits;
+  const int steps = g.steps;
+  int u0 = place * g.quota, u1 = min(u0 + g.quota, g.tiles_per_group * steps);
+  if (g.pieces) {
+    const int t = place / g.pieces;
+    u0 = t * steps + (place - t * g.pieces) * g.quota;
+    u1 = t < g.tiles_per_group ? min(u0 + g.quota, (t + 1) * steps) : u0;
+  }
+  if (u0 >= u1) return;
+  const int t_first = u0 / steps, t_last = (u1 - 1) / steps;
+  const bool leaves_piece = u1 < (t_last + 1) * steps;
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int T = g.T, K = g.K, N = g.N;
+
+  for (int visit = 0; visit <= t_last - t_first; ++visit) {
+    const int t = leaves_piece ? (visit == 0 ? t_last : t_first + visit - 1) : t_first + visit;
+    const int s_begin = t == t_first ? u0 - t_first * steps : 0;
+    const int s_end = t == t_last ? u1 - t_last * steps : steps;
+    const int tile = group * g.tiles_per_group + t;
+    const int tm = tile % g.tiles_m, tn = tile / g.tiles_m;
+    const int m0 = tm * TM, n0 = tn * TN;
+    const int k_begin = s_begin * kWideStep, k_end = min(K, s_end * kWideStep);
+    const int nk = s_end - s_begin;
+
+    int tid = threadIdx.x;  // (worked out again per tile, as above)
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, ln = lane & 15, j = lane >> 4;
+
+    // staging: x: octet tid / 8 % 4 of row tid % 8 + 8 (tid / 32) (and 128 on); W: octets tid / 256 and two on of column tid % 256
+    const int xrow = (tid & 7) + 8 * (tid >> 5), xk = 8 * (tid >> 3 & 3);
+    const int wk = 8 * (tid >> 8);
+    int wcol = tid & 255, w_from = min(n0 + wcol, N - 1);
+    if constexpr (SWIGLU) {  // (32 columns of gate, the same of up, and so on: 128 bytes of a row together; a lane holds both of a hidden column)
+      const int up = wcol >> 5 & 1, h = (wcol >> 6) * 32 + (wcol & 31);
+      w_from = up * (N / 2) + min(n0 / 2 + h, N / 2 - 1);
+      wcol = NB * (h / (NB / 2)) + h % (NB / 2) + NB / 2 * up;
+    }
+    const int x_unit = (xk >> 3) * kOctX + xrow;
+    const int w_unit = kW + (wk >> 3) * kOctW + wcol / (16 * NB) * (NB * kBlockW) + wcol % NB * kBlockW + wcol % (16 * NB) / NB;
+    // fragments
+    const int a_unit = j * kOctX + wm * 64 + ln, b_unit = kW + j * kOctW + wn * (NB * kBlockW) + ln;
+
+    // (rows past the last one repeat it and columns likewise: their products are never stored)
+    unsigned x_off[NX], w_row[8];
+#pragma unroll
+    for (int u = 0; u < NX; ++u) x_off[u] = (unsigned)(((long long)min(m0 + xrow + 128 * u, T - 1) * g.xs + xk) * 4);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w_row[i] = (unsigned)(((long long)(wk + i) * N + w_from) * 4);
+    const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)k_begin * N);
+
+    f32x4 sx[kSets][NX][2];
+    float sw[kSets][2][8];
+    int k_next = k_begin, to_load = nk;
+    auto load_x = [&](const int set, const int u, const int h) {
+      sx[set][u][h] = GUARD && k_next + xk + 4 * h >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : load_from((const f32x4 *)(x_base + 16 * h), x_off[u]);
+    };
+    auto load_w = [&](const int set, const int o, const int i) {
+      sw[set][o][i] = GUARD && k_next + wk + 16 * o + i >= k_end ? 0.f : load_from((const float *)(w_base + o * (64LL * N)), w_row[i]);
+    };
+    auto advance = [&]() {
+      if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
+        x_base += kWideStep * 4;
+        w_base += (long long)kWideStep * N * 4;
+        k_next += kWideStep;
+      }
+    };
+
+    // The work beside the MFMAs, in pieces of at most four vector instructions (a SIMD issues two of them during an MFMA for nothing) or a write, of
+    // which four wavefronts' take 70 cycles.  Per octet of x: four pairs split in four pieces each, three writes, two loads of the next; per octet of W: four
+    // pairs, a write, eight loads.
+    constexpr int kItemsX = 21 * NX, kItems = kItemsX + 26;
+    u32x4 whole[3];
+    float pa, pb;
+    auto item = [&](const int it, const int set, u32x4 *stage) {
+      if (it < kItemsX) {
+        const int u = it / 21, m = it % 21, i = m / 4;
+        if (m >= 19) {
+          load_x(set, u, m - 19);
+        } else if (m >= 16) {
+          stage[x_unit + 128 * u + (m - 16) * kPartX] = whole[m - 16];
+        } else if (m % 4 == 0) {
+          pa = sx[set][u][i / 2][i % 2 * 2] * kLift;
+          pb = sx[set][u][i / 2][i % 2 * 2 + 1] * kLift;
+          whole[0][i] = pack_bf16(pa, pb);
+        } else if (m % 4 == 1) {
+          pa -= __builtin_bit_cast(float, whole[0][i] << 16);
+          pb -= __builtin_bit_cast(float, whole[0][i] & 0xffff0000u);
+        } else if (m % 4 == 2) {
+          whole[1][i] = pack_bf16(pa, pb);
+          pa -= __builtin_bit_cast(float, whole[1][i] << 16);
+        } else {
+          pb -= __builtin_bit_cast(float, whole[1][i] & 0xffff0000u);
+          whole[2][i] = pack_bf16(pa, pb);
+        }
+      } else {
+        const int o = (it - kItemsX) / 13, m = (it - kItemsX) % 13;
+        if (m >= 5)
+          load_w(set, o, m - 5);
+        else if (m == 4)
+          stage[w_unit + 2 * o * kOctW] = whole[0];
+        else
+          whole[0][m] = pack_high(sw[set][o][2 * m] * kLift, sw[set][o][2 * m + 1] * kLift);
+      }
+      if (it == kItems - 1) advance();
+    };
+    auto load_all = [&](const int set) {
+#pragma unroll
+      for (int u = 0; u < NX; ++u) load_x(set, u, 0), load_x(set, u, 1);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) load_w(set, i / 8, i % 8);
+      advance();
+    };
+
+    f32x4 acc[MB][NB];
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 af[2][3], bf[NB];
+    auto fetch_x = [&](const u32x4 *stage, const int a, const int p) { af[a & 1][p] = stage[a_unit + 16 * a + p * kPartX]; };
+    auto fetch_w = [&](const u32x4 *stage, const int b) { bf[b] = stage[b_unit + b * kBlockW]; };
+    auto multiply = [&](const int a, const int b, const int p) { acc[a][b] = mfma_bf16_16(af[a & 1][p], bf[b], acc[a][b]); };
+
+    // (after the last barrier of the tile before this one nobody reads what he uses any more)
+    load_all(0);
+    if constexpr (kSets == 2) load_all(1);
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) item(it, 0, lds);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) bf[b] = u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) af[(MB - 1) & 1][p] = u32x4{0, 0, 0, 0};
+    __syncthreads();
+
+    // A turn of the loop is the last blocks of rows of the step before (of zeros in front of the first), in which the fragments of W and of the
+    // first block of rows arrive, and all others of step kt.  (So the barrier stands where a turn ends: there the compiler waits for all of LDS anyway.)
+    auto step = [&](const int kt, const int set) {  // set: holds the tiles of step kt + 1
+      const u32x4 *const stage = lds + (kt & 1) * kUnits;
+      u32x4 *const next = lds + ((kt & 1) ^ 1) * kUnits;
+      constexpr int kSlots = 3 * MB * NB;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const int a = (i + MB - 1) % MB;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int p = 2; p >= 0; --p) {  // smallest products first
+            multiply(a, b, p);
+            if (i == 0 && p == 0) fetch_w(stage, b);
+            if (p == 1 && b < 3) fetch_x(stage, (a + 1) % MB, 2 - b);
+            const int slot = 3 * (i * NB + b) + 2 - p;
+#pragma unroll
+            for (int it = slot * kItems / kSlots; it < (slot + 1) * kItems / kSlots; ++it) item(it, set, next);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      __syncthreads();
+    };
+    if constexpr (kSets == 1) {
+      for (int kt = 0; kt < nk; ++kt) step(kt, 0);
+    } else {
+      // (in pairs: a way out between them has the compiler wait for loads of the step before)
+      for (int kt = 1; kt < nk; kt += 2) {
+        step(kt - 1, 1);
+        step(kt, 0);
+      }
+      if (nk & 1) step(nk - 1, 1);
+    }
+#pragma unroll
+    for (int slot = 0; slot < 3 * NB; ++slot) multiply(MB - 1, slot / 3, 2 - slot % 3);
+
+    const int row0 = m0 + wm * 64 + 4 * j, col = n0 + wn * 16 * NB + NB * ln;
+    // sums that are not finite come from operands that are not (or overflow): again in fp32, which says which
+    float probe = 0.f, down = kDrop;
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) probe = fmaf(acc[a][b][r], 0.f, probe);
+    if (__any(probe != 0.f)) {
+#pragma unroll
+      for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // 16 k a turn, four of them a quarter's (K is a multiple of 4: those behind its end are zeros on both sides)
+#pragma clang loop unroll(disable)
+      for (int k0 = k_begin; k0 < k_end; k0 += 16) {
+        const int k = k0 + 4 * j;
+        const bool in = k < k_end;
+        f32x4 xv[MB];
+#pragma unroll
+        for (int a = 0; a < MB; ++a)
+          xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + wm * 64 + 16 * a + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            const int from = SWIGLU ? b / (NB / 2) * (N / 2) + min(col / 2 + b % (NB / 2), N / 2 - 1) : min(col + b, N - 1);
+            const float wv = in ? g.w[(long long)(k + i) * N + from] : 0.f;
+#pragma unroll
+            for (int a = 0; a < MB; ++a) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[a][i], wv, acc[a][b], 0, 0, 0);
+          }
+      }
+      down = 1.f;
+    }
+
+    // A piece travels as [row of a block, four columns][thread] float4: consecutive threads, consecutive 16 bytes.
+    constexpr long long kSlot = (long long)TM * TN;
+    constexpr int Q = NB / 4, kOut = 4 * MB * Q;
+    f32x4 out[kOut];
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+          out[(4 * a + r) * Q + q] = f32x4{acc[a][4 * q][r], acc[a][4 * q + 1][r], acc[a][4 * q + 2][r], acc[a][4 * q + 3][r]} * down;
+    const int in_slot = 4 * tid;
+    if (g.pieces) {  // the second kernel adds the pieces
+      float *slot = g.partials + blockIdx.x * kSlot + in_slot;
+#pragma unroll
+      for (int r = 0; r < kOut; ++r) *(f32x4 *)(slot + r * 4 * NT) = out[r];
+      return;
+    }
+    if (s_end < steps) {
+      leave_piece(g, g.partials + blockIdx.x * kSlot + in_slot, 4 * NT, out);
+      continue;
+    }
+    if (s_begin > 0) {
+      const int p_first = t * steps / g.quota;
+      add_earlier_pieces(g, group, p_first, place - p_first, kSlot, in_slot, 4 * NT, out);
+    }
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const f32x4 *const v = out + (4 * a + r) * Q;
+        const int row = row0 + 16 * a + r;
+        if constexpr (SWIGLU) {  // (N / 2 is a multiple of 4: a lane's hidden columns are inside together)
+          if (row >= T || col >= N) continue;
+          float *const y = g.y + (long long)row * (N / 2) + col / 2;
+          if constexpr (Q == 1)
+            *(f32x2 *)y = f32x2{swiglu(v[0].x, v[0].z), swiglu(v[0].y, v[0].w)};
+          else
+            *(f32x4 *)y = f32x4{swiglu(v[0].x, v[1].x), swiglu(v[0].y, v[1].y), swiglu(v[0].z, v[1].z), swiglu(v[0].w, v[1].w)};
+        } else {
+#pragma unroll
+          for (int q = 0; q < Q; ++q)  // (N is a multiple of 4, not of a lane's columns)
+            if (col + 4 * q < N) store_four<4>(g, row, col + 4 * q, 0, v[q]);
+        }
+      }
   }
 }
 
@@ -1010,7 +1187,7 @@ __device__ __forceinline__ f32x4 add_pieces(f32x4 acc, const float *piece, long 
 }
 
 // How a product's tiles lie in its workgroups' slots.  `columns` of a lane: 1: row by row; 2: [pair of rows][thread] float4, two
-// neighbouring columns of two rows; 4: [row][thread] float4, four columns of one.
+// neighbouring columns of two rows of blocks of 32; 4 and 8: [row, four columns][thread] float4, of blocks of 16 rows.
 struct PieceShape {
   int tm, tn;      // rows and columns of a tile
   int rows, wn;    // rows of a wavefront, wavefronts along the columns
@@ -1024,9 +1201,16 @@ __device__ __forceinline__ const float *first_piece(const GemmArgs &g, const Pie
   const int tile = tn * g.tiles_m + tm, group = tile / g.tiles_per_group, t = tile - group * g.tiles_per_group;
   const float *slot = g.partials + (((long long)t * g.pieces << g.group_bits) | group) * s.tm * s.tn;
   if constexpr (COLUMNS == 1) return slot + r * s.tn + c;
-  const int wm = r / s.rows, q = r - wm * s.rows, in = q & 31, at = 4 * (in >> 3) + (in & 3);  // (of the 16 registers of a block)
-  const int out = COLUMNS == 2 ? 8 * (q >> 5) + at / 2 : 16 * (q >> 5) + at;
-  const int thread = (wm * s.wn + c / (32 * COLUMNS)) * 64 + 32 * (in >> 2 & 1) + c % (32 * COLUMNS) / COLUMNS;
+  const int wm = r / s.rows, q = r - wm * s.rows;
+  int out, thread;
+  if constexpr (COLUMNS == 2) {
+    const int in = q & 31, at = 4 * (in >> 3) + (in & 3);  // (of the 16 registers of a block)
+    out = 8 * (q >> 5) + at / 2;
+    thread = (wm * s.wn + c / 64) * 64 + 32 * (in >> 2 & 1) + c % 64 / 2;
+  } else {
+    out = (4 * (q >> 4) + (q & 3)) * (COLUMNS / 4) + c % COLUMNS / 4;
+    thread = (wm * s.wn + c / (16 * COLUMNS)) * 64 + 16 * (q >> 2 & 3) + c % (16 * COLUMNS) / COLUMNS;
+  }
   return slot + 4 * ((long long)out * s.threads + thread);
 }
 
@@ -1331,7 +1515,7 @@ void choose_tile(GemmPlan &p, int T, int K, int N) {
 
 static int tile_rows(const GemmPlan &p) { return (p.few ? 32 : 64) * p.mb; }
 static int tile_columns(const GemmPlan &p) { return p.few && p.parts == 1 ? 256 / p.kg : 64 * p.wn; }
-static int step_k(const GemmPlan &p) { return !p.few ? TK : p.parts == 1 ? 16 * p.kg : kFewStep; }
+static int step_k(const GemmPlan &p) { return !p.few ? p.parts == 1 ? kWideStep : TK : p.parts == 1 ? 16 * p.kg : kFewStep; }
 
 void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[0] = !p.mfma ? 0 : p.few ? 1 : 2;
@@ -1340,7 +1524,7 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[3] = p.workgroups;
   plan[4] = p.pieces > 1 ? p.pieces : 1;
   plan[5] = p.flag_words && p.quota % p.steps != 0;
-  plan[6] = p.mfma && K % step_k(p) != 0;
+  plan[6] = p.mfma && K % (p.few ? step_k(p) : TK) != 0;
 }
 
 // (the norm of a row takes a workgroup of up to 1024 threads, two registers of four each)
@@ -1355,8 +1539,7 @@ bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
     return !next.norm.rows && !q->q_norm && !q->k_norm && !q->b_q && !q->b_k && !q->b_v && q->rope_tab && q->hd % 8 == 0 &&
            (long long)(q->H + 2 * q->KV) * q->hd == N && q->start_pos >= 0 && q->start_pos + T <= q->cap &&
            !(((uintptr_t)q->q_rot | (uintptr_t)q->kc | (uintptr_t)q->vc) & 15);
-  const bool pairs = !(p.few && p.parts == 1) && !(p.parts == 1 && p.mb == 4);
-  return N % 4 == 0 && N / (pairs ? 2 : 4) <= 2048;
+  return N % 4 == 0 && N / (p.parts == 1 ? 4 : 2) <= 2048;
 }
 
 GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
@@ -1368,7 +1551,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
   p.steps = (K + TK - 1) / TK;
   choose_tile(p, T, K, N);
   const int TN = tile_columns(p), TM = tile_rows(p);
-  if (p.few) p.steps = (K + step_k(p) - 1) / step_k(p);
+  p.steps = (K + step_k(p) - 1) / step_k(p);
   p.tiles_m = (T + TM - 1) / TM;
   p.tiles_n = (N + TN - 1) / TN;
   if (!p.mfma) return p;
@@ -1405,7 +1588,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
   }
   // Otherwise one round of workgroups shares the K steps of all tiles evenly.
   const long long units = (long long)p.tiles_per_group * p.steps;
-  const int least = 16;  // steps of 16: a workgroup's start and end must not outweigh its loop
+  const int sixteen = step_k(p) / TK, least = 16 / sixteen;  // (16 steps of 16: a workgroup's start and end must not outweigh its loop)
   int places = slots / groups;
   int quota = (int)((units + places - 1) / places);
   if (quota < least) quota = p.steps < least ? p.steps : least;
@@ -1420,7 +1603,7 @@ GemmPlan plan_gemm(int T, int K, int N, long long x_stride, bool w_bf16) {
     static const int pieces_knob = getenv("SHAINET_HIP_GEMM_PIECES") ? atoi(getenv("SHAINET_HIP_GEMM_PIECES")) : 0;
     if (pieces > 16) pieces = 16;  // (45 rows of 8192 -> 2048: 32 pieces 35.2 us, 16 pieces 30.7 us)
     if (pieces_knob > 0) pieces = pieces_knob;  // SHAINET_HIP_GEMM_PIECES: a tuning knob
-    if (pieces > p.steps / 8) pieces = p.steps / 8;
+    if (pieces > p.steps * sixteen / 8) pieces = p.steps * sixteen / 8;
     if (pieces < 1) pieces = 1;
     p.quota = (p.steps + pieces - 1) / pieces;
     p.pieces = pieces;
@@ -1458,22 +1641,38 @@ hipError_t launch_sum(const GemmArgs &g, const PieceShape &s, const GemmNext &ne
   return hipGetLastError();
 }
 
-template <int WM, int WN, int MB, int NB, int PARTS>
+template <int WM, int WN, int MB>
 hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups), block(64 * WM * WN);
-  constexpr bool kSwiglu = PARTS == 1 || MB < 4;  // (the others leave it to a launch of its own)
+  constexpr bool kSwiglu = MB < 4;  // (the others leave it to a launch of its own)
   const bool swiglu = next.swiglu && !g.pieces;
   if (swiglu && !kSwiglu) return hipErrorInvalidValue;
   if (swiglu && g.K % TK != 0)
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, kSwiglu>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, true, kSwiglu>), grid, block, 0, stream, g);
   else if (swiglu)
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false, kSwiglu>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, false, kSwiglu>), grid, block, 0, stream, g);
   else if (g.K % TK != 0)
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, true, false>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, true, false>), grid, block, 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, NB, PARTS, false, false>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((sgemm_split_kernel<WM, WN, MB, false, false>), grid, block, 0, stream, g);
   const hipError_t e = hipGetLastError();
-  return e != hipSuccess || !g.pieces ? e : launch_sum<NB>(g, PieceShape{32 * WM * MB, 32 * WN * NB, 32 * MB, WN, 64 * WM * WN}, next, stream);
+  return e != hipSuccess || !g.pieces ? e : launch_sum<2>(g, PieceShape{32 * WM * MB, 64 * WN, 32 * MB, WN, 64 * WM * WN}, next, stream);
+}
+
+template <int WM>
+hipError_t launch_wide(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
+  const dim3 grid((unsigned)p.workgroups);
+  const bool guard = g.K % kWideStep != 0, swiglu = next.swiglu && !g.pieces;
+  if (swiglu && guard)
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, true, true>), grid, dim3(512), 0, stream, g);
+  else if (swiglu)
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, true>), grid, dim3(512), 0, stream, g);
+  else if (guard)
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, true, false>), grid, dim3(512), 0, stream, g);
+  else
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, false>), grid, dim3(512), 0, stream, g);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || !g.pieces ? e : launch_sum<2 * WM>(g, PieceShape{64 * WM, 256, 64, 8 / WM, 512}, next, stream);
 }
 
 hipError_t launch_few(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
@@ -1544,11 +1743,11 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   if (p.parts == 1) {
     if (p.few && p.kg == 4) return launch_stream<1, 4>(g, p, next, stream);
     if (p.few) return p.mb == 1 ? launch_stream<1, 2>(g, p, next, stream) : p.mb == 2 ? launch_stream<2, 2>(g, p, next, stream) : launch_stream<3, 2>(g, p, next, stream);
-    return p.mb == 4 ? launch_tiles<4, 2, 2, 4, 1>(g, p, next, stream) : launch_tiles<2, 4, 2, 2, 1>(g, p, next, stream);
+    return p.mb == 4 ? launch_wide<4>(g, p, next, stream) : launch_wide<2>(g, p, next, stream);
   }
   if (p.few) return launch_few(g, p, next, stream);
-  if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4, 2, 3>(g, p, next, stream) : launch_tiles<2, 4, 2, 2, 3>(g, p, next, stream);
-  return launch_tiles<2, 2, 2, 2, 3>(g, p, next, stream);
+  if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4>(g, p, next, stream) : launch_tiles<2, 4, 2>(g, p, next, stream);
+  return launch_tiles<2, 2, 2>(g, p, next, stream);
 }
 
 }  // namespace shainet

@@ -106,6 +106,12 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
 }
 
+// The same of 16 x 16 over 32 k: lane l holds k = 8 (l / 16) .. + 7 of row (column) l % 16.
+// D[m = 4 (l / 16) + r][n = l % 16] in register r.
+__device__ __forceinline__ f32x4 mfma_bf16_16(u32x4 a, u32x4 b, f32x4 acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+}
+
 // The same in fp32 over two k: lane l holds k = l / 32 of row (column) l % 32; the same D.
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
@@ -115,6 +121,14 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 acc) {
 // by scalars only the compiler makes 64-bit sums per thread, two instructions each.)
 template <typename V>
 __device__ __forceinline__ V load_at(const V *base, unsigned offset) {
+  uint64_t at = (uint64_t)base;
+  asm("" : "+s"(at), "+v"(offset));
+  return *(const __attribute__((address_space(1))) V *)(at + offset);
+}
+
+// The same with an offset that keeps its register over a loop.
+template <typename V>
+__device__ __forceinline__ V load_from(const V *base, unsigned &offset) {
   uint64_t at = (uint64_t)base;
   asm("" : "+s"(at), "+v"(offset));
   return *(const __attribute__((address_space(1))) V *)(at + offset);
