@@ -208,6 +208,23 @@ struct ReadAhead {
   int k, n, first_wg;
 };
 
+// Workgroup ah.first_wg + j reads the rows 4 j .. 4 j + 3 and n + the same of ah.w and drops them.
+__device__ __forceinline__ void read_ahead(const ReadAhead &ah) {
+  const int row = 4 * ((int)blockIdx.x - ah.first_wg) + (int)(threadIdx.x >> 6);
+  if (row >= ah.n) return;
+  const int pieces = ah.k >> 8;  // 16-byte pieces per lane and row
+  for (int half = 0; half < 2; ++half) {
+    const float *p = ah.w + ((long long)half * ah.n + row) * ah.k + 4 * (threadIdx.x & 63);
+    for (int i0 = 0; i0 < pieces; i0 += 8) {
+      f32x4 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = *(const f32x4 *)(p + 256 * min(i0 + u, pieces - 1));
+#pragma unroll
+      for (int u = 0; u < 8; ++u) asm volatile("" : : "v"(v[u]));
+    }
+  }
+}
+
 // The arithmetic of norm_rotate_pair (prep_math.hpp) in the layouts of the kernel below, the same bits: no product fuses
 // into an add.
 #pragma clang fp contract(off)
@@ -336,19 +353,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   static_assert(!PREP || (!PAD && !DEV && HD <= 128), "preparation of plain host-planned rows");
   if constexpr (AHEAD) {
     if ((int)blockIdx.x >= ah.first_wg) {
-      const int row = 4 * ((int)blockIdx.x - ah.first_wg) + (int)(threadIdx.x >> 6);
-      if (row >= ah.n) return;
-      const int pieces = ah.k >> 8;  // 16-byte pieces per lane and row
-      for (int half = 0; half < 2; ++half) {
-        const float *p = ah.w + ((long long)half * ah.n + row) * ah.k + 4 * (threadIdx.x & 63);
-        for (int i0 = 0; i0 < pieces; i0 += 8) {
-          f32x4 v[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) v[u] = *(const f32x4 *)(p + 256 * min(i0 + u, pieces - 1));
-#pragma unroll
-          for (int u = 0; u < 8; ++u) asm volatile("" : : "v"(v[u]));
-        }
-      }
+      read_ahead(ah);
       return;
     }
   }
@@ -749,6 +754,260 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 128 ? 2 : 1) void decode_
   }
 }
 
+// Pairs of up to 12 tiles (heads of 128: 8), a workgroup each, one new row per sequence: the arithmetic of the kernel above in its order, the
+// same bits, with everything requested at once.  T: tiles per wavefront, those of the longest pair; a wavefront without a T-th one
+// requests its pair's last again, so that no load hangs on a condition.  The queries (and the new key and value) are made once, in pieces of
+// a few threads, and read from LDS: by every wavefront for itself, as above, they were 25 of a wavefront's 33 loads, and a compute unit takes 16
+// cycles for each.  K goes to LDS by instructions that the compiler does not count: those it knows have it wait for everything in flight in front
+// of any exchange between lanes.  Grid: kv heads (and workgroups that read ahead), sequences.
+// Us of the launch, the kernel above | this, one sequence, 8 kv heads of 64: 61 keys 6.3 | 4.3, 125 7.2 | 5.2, 171 7.9 | 6.3; with QK-norm 31 keys
+// 6.8 | 4.7, 81 7.6 | 5.7, 171 8.4 | 6.8; heads of 128, 101 keys 9.8 | 7.2, with QK-norm 11.4 | 7.8; 16 sequences of 101 keys 8.0 | 5.6, of 181 9.2 | 7.1, of
+// heads of 128 with QK-norm 12.4 | 8.9.  (Every wavefront its queries, K straight to registers 5.2, 6.6, 7.8; by LDS 5.2, 6.4, 7.3.)  What bounds it, in cycles
+// of 6400 for 61 keys: arguments 1200, loads requested and there 1700, queries 500, a tile's MFMAs and softmax 1900, merge and stores 1500.
+struct RowSeqs {
+  int start[kMaxSeqs], slot[kMaxSeqs];
+};
+constexpr int kRowsPlain = 0, kRowsPrep = 1, kRowsBias = 2;  // queries and new rows are prepared; are a projection's; scores gain a value by distance
+template <int HD>
+constexpr int kRowTiles = HD == 64 ? 3 : 2;
+
+// the larger of a lane's value and that of the lane 16 (32) away
+__device__ __forceinline__ float max_across_quarters(float x) {
+  auto larger = [](unsigned a, unsigned b) { return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)); };
+  unsigned bits = __builtin_bit_cast(unsigned, x);
+  auto p = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+  bits = __builtin_bit_cast(unsigned, larger(p[0], p[1]));
+  p = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+  return larger(p[0], p[1]);
+}
+
+template <int HD, int T, int MODE>
+__global__ __launch_bounds__(256, 1) void decode_rows_kernel(const float *__restrict__ q_rot, const float *__restrict__ kc,
+                                                             const float *__restrict__ vc, float *__restrict__ out, const RowSeqs seqs,
+                                                             Shape sh, float c, unsigned rotate, ReadAhead ah, DistanceBias db, PrepArgs raw) {
+  using C = DecodeCfg<HD>;
+  constexpr int NT = C::NT, NW = 4;
+  constexpr bool PREP = MODE == kRowsPrep, BIAS = MODE == kRowsBias;
+  const int kvh = blockIdx.x, s = blockIdx.y;
+  const int start = seqs.start[s], seq_slot = seqs.slot[s];
+  // (all arguments together, or those behind a condition are asked for behind it, a round trip later)
+  asm volatile("" : : "s"(start), "s"(seq_slot), "s"(kc), "s"(vc), "s"(out), "s"(sh.KV), "s"(sh.g), "s"(sh.cap), "s"(sh.seq_stride), "s"(rotate));
+  if constexpr (PREP)
+    asm volatile("" : : "s"(raw.q), "s"(raw.k), "s"(raw.v), "s"(raw.q_stride), "s"(raw.k_stride), "s"(raw.v_stride), "s"(raw.q_norm), "s"(raw.k_norm),
+                 "s"(raw.rope_tab), "s"(raw.q_rot));
+  if (ah.w && kvh >= ah.first_wg) {
+    read_ahead(ah);
+    return;
+  }
+  if (kvh >= sh.KV) return;  // (between the last pair and the first that reads ahead)
+  constexpr int kRow = HD + 4;  // floats from a query to the next in LDS
+  __shared__ __attribute__((aligned(1024))) char k_lds[NW][T][C::TILE_BYTES];
+  __shared__ __attribute__((aligned(16))) float sm_o[NW][16 * HD], sm_q[17 * kRow], sm_v[HD];
+  __shared__ float sm_m[NW][16], sm_l[NW][16];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, j = lane >> 4;
+  const int g = sh.g;
+  const int L = start + 1, n = (L + 15) >> 4;
+  const long long head_base = (long long)seq_slot * sh.seq_stride + (long long)kvh * sh.cap * HD;
+  const float *kbase = kc + head_base;
+  const float *vbase = vc + (BIAS ? ((long long)seq_slot * sh.KV + kvh) * sh.cap * HD : head_base);
+  const float ce = BIAS ? 1.f : c;
+  const int cq = col < g ? col : 0;  // columns beyond the last repeat column 0: their results are never stored
+
+  // a thread's piece of the queries, and of the new key (row g): four elements and, to prepare, the four a half further
+  constexpr int kPieces = PREP ? HD / 8 : HD / 4, kRounds = (17 * kPieces + 255) / 256;
+  const int items = (PREP ? g + 1 : g) * kPieces;
+  const float *qrow = PREP ? raw.q + s * raw.q_stride + (long long)kvh * g * HD
+                           : q_rot + (BIAS ? s * db.q_stride + (long long)kvh * g * HD : ((long long)s * sh.H + kvh * g) * HD);
+  const float *krow = PREP ? raw.k + s * raw.k_stride + (long long)kvh * HD : nullptr;
+  f32x4 x[kRounds][2], w[kRounds][2], cs[kRounds][2], fresh;
+  SquareSum<HD> sum;
+  const bool norms = PREP && (raw.q_norm || raw.k_norm), has_items = 64 * wave < items;
+  const int vi = (int)threadIdx.x - (256 - HD / 4);  // the last threads: the new value
+#pragma unroll
+  for (int u = 0; u < kRounds; ++u) {
+    const int at = threadIdx.x + 256 * u, row = at / kPieces, e = 4 * (at % kPieces);
+    if (at < items) {
+      const float *src = PREP && row == g ? krow : qrow + row * HD;
+      x[u][0] = *(const f32x4 *)(src + e);
+      if constexpr (PREP) {
+        const float *norm = row == g ? raw.k_norm : raw.q_norm;
+        const float2 *table = raw.rope_tab + (long long)(L - 1) * (HD / 2) + e;
+        x[u][1] = *(const f32x4 *)(src + HD / 2 + e);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          w[u][h] = f32x4{1.f, 1.f, 1.f, 1.f};
+          if (norm) w[u][h] = *(const f32x4 *)(norm + h * (HD / 2) + e);
+          cs[u][h] = *(const f32x4 *)(table + 2 * h);
+        }
+      }
+    }
+  }
+  if constexpr (PREP) {
+    if (norms && has_items) {  // row r: head r of the group; row g: the new key
+      const int r = lane & 31;
+      sum.request(r == g ? krow : qrow + (r < g ? r : 0) * HD, lane);
+    }
+    if (vi >= 0) fresh = *(const f32x4 *)(raw.v + s * raw.v_stride + (long long)kvh * HD + 4 * vi);
+  }
+
+  // the wavefront's tiles, in the order of the kernel above
+  const int last_row = PREP ? max(L - 2, 0) : L - 1;  // (in memory)
+  const int rot = rotate && n > 1 ? (int)((((unsigned)(s * sh.KV + kvh)) * 2654435761u >> 12) % min((unsigned)n, rotate)) : 0;
+  int kb[T];
+  f32x4 vf[T][4][C::NVU];
+#pragma unroll
+  for (int u = 0; u < T; ++u) {
+    const int k = min(wave + NW * u, n - 1) + rot;
+    kb[u] = 16 * (k < n ? k : k - n);
+#pragma unroll
+    for (int i = 0; i < C::NKI; ++i) {  // (as issue_k_tile)
+      const int slot = i * 64 + lane, row = slot / C::PPR, piece = slot % C::PPR ^ row;
+      const unsigned off = (unsigned)(min(kb[u] + row, last_row) * C::ROW_BYTES + 16 * piece);
+      const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)LDS_PTR(&k_lds[wave][u][i * 1024]));
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(to), "v"(off), "s"(kbase) : "memory");
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < T; ++u)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const unsigned off = (unsigned)(min(kb[u] + 4 * j + r, last_row) * C::ROW_BYTES + 16 * col);
+#pragma unroll
+      for (int w2 = 0; w2 < C::NVU; ++w2)
+        vf[u][r][w2] = __builtin_nontemporal_load((const __attribute__((address_space(1))) f32x4 *)((uintptr_t)vbase + off + 256 * w2));
+    }
+  f32x4 near_bias[T];
+  if constexpr (BIAS) {
+    struct __attribute__((packed, aligned(4))) Four { f32x4 v; };
+    const float *bias_row = db.tab + (long long)(kvh * g + cq) * db.stride + (db.origin - (L - 1));
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      near_bias[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (L - 1 - (kb[u] + 15) < db.reach) near_bias[u] = ((const Four *)(bias_row + kb[u] + 4 * j))->v;
+    }
+  }
+
+  if (has_items) {
+    const float inv = norms ? sum.factor(raw.eps, lane) : 1.f;
+#pragma unroll
+    for (int u = 0; u < kRounds; ++u) {
+      const int at = threadIdx.x + 256 * u, row = at / kPieces, e = 4 * (at % kPieces);
+      const float inv_row = norms ? __shfl(inv, 32 + (row < 17 ? row : 0)) : 1.f;
+      if (at >= items) continue;
+      if constexpr (PREP) {
+        norm_rotate_quad(x[u][0], x[u][1], (row == g ? raw.k_norm : raw.q_norm) != nullptr, w[u][0], w[u][1], inv_row, cs[u][0], cs[u][1]);
+        float *to = row == g ? const_cast<float *>(kbase) + (long long)(L - 1) * HD : raw.q_rot + ((long long)s * sh.H + kvh * g + row) * HD;
+        *(f32x4 *)(to + e) = x[u][0];
+        *(f32x4 *)(to + HD / 2 + e) = x[u][1];
+        *(f32x4 *)&sm_q[row * kRow + HD / 2 + e] = x[u][1];
+      }
+      *(f32x4 *)&sm_q[row * kRow + e] = x[u][0];
+    }
+  }
+  if (PREP && vi >= 0) {
+    *(f32x4 *)(const_cast<float *>(vbase) + (long long)(L - 1) * HD + 4 * vi) = fresh;
+    *(f32x4 *)&sm_v[4 * vi] = fresh;
+  }
+  __syncthreads();
+  float qr[HD / 4];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const f32x4 v = *(const f32x4 *)&sm_q[cq * kRow + 16 * i + 4 * j];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qr[4 * i + e] = v[e];
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // the tiles are there
+  asm volatile("" ::: "memory");
+
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < T; ++u) {
+    if (wave + NW * u >= n) continue;
+    const bool last = PREP && kb[u] + 16 >= L;  // the pair's last tile: nobody's key L - 1 and no value from there on is in memory
+    const char *tile = k_lds[wave][u] + col * C::ROW_BYTES, *fresh_key = (const char *)&sm_q[g * kRow];
+    const bool mine = last && kb[u] + col == L - 1;
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const f32x4 kk = *(const f32x4 *)(mine ? fresh_key + 64 * i + 16 * j : tile + (((4 * i + j) ^ col) << 4));
+      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.x, qr[4 * i + 0], s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.y, qr[4 * i + 1], s1, 0, 0, 0);
+      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.z, qr[4 * i + 2], s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.w, qr[4 * i + 3], s1, 0, 0, 0);
+    }
+    if (last) {
+#pragma unroll
+      for (int w2 = 0; w2 < C::NVU; ++w2) {
+        const f32x4 v = *(const f32x4 *)&sm_v[64 * w2 + 4 * col];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vf[u][r][w2] = kb[u] + 4 * j + r >= L - 1 ? v : vf[u][r][w2];
+      }
+    }
+    float sv[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      sv[r] = (kb[u] + 4 * j + r < L) ? (BIAS ? (s0[r] + s1[r]) * c + near_bias[u][r] : s0[r] + s1[r]) : -INFINITY;
+    const float mnew = fmaxf(m, max_across_quarters(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]))));
+    const float mref = mnew == -INFINITY ? 0.f : mnew;  // (a tile of nothing but -inf)
+    const float alpha = fast_exp2((m - mref) * ce);
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = fast_exp2((sv[r] - mref) * ce);
+    l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+    m = mnew;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) o[i] *= alpha;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int w2 = 0; w2 < C::NVU; ++w2) {
+        o[4 * w2 + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][r][w2].x, p[r], o[4 * w2 + 0], 0, 0, 0);
+        o[4 * w2 + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][r][w2].y, p[r], o[4 * w2 + 1], 0, 0, 0);
+        o[4 * w2 + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][r][w2].z, p[r], o[4 * w2 + 2], 0, 0, 0);
+        o[4 * w2 + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][r][w2].w, p[r], o[4 * w2 + 3], 0, 0, 0);
+      }
+  }
+
+  // the wavefronts' shares meet in LDS, in their order
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (col < g) {
+#pragma unroll
+    for (int w2 = 0; w2 < C::NVU; ++w2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *(f32x4 *)&sm_o[wave][col * HD + 64 * w2 + 4 * (4 * j + r)] = f32x4{o[4 * w2][r], o[4 * w2 + 1][r], o[4 * w2 + 2][r], o[4 * w2 + 3][r]};
+    if (j == 0) {
+      sm_m[wave][col] = m;
+      sm_l[wave][col] = l;
+    }
+  }
+  __syncthreads();
+  float *const to = out + ((long long)s * sh.H + kvh * g) * HD;
+  for (int idx = threadIdx.x; idx < g * (HD / 4); idx += 64 * NW) {
+    const int cc = idx / (HD / 4);
+    float mm = sm_m[0][cc];
+#pragma unroll
+    for (int w2 = 1; w2 < NW; ++w2) mm = fmaxf(mm, sm_m[w2][cc]);
+    const float mref = mm == -INFINITY ? 0.f : mm;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float ls = 0.f;
+#pragma unroll
+    for (int w2 = 0; w2 < NW; ++w2) {
+      const float f = fast_exp2((sm_m[w2][cc] - mref) * ce);  // 0 for a wavefront without a tile
+      acc += f * *(const f32x4 *)&sm_o[w2][4 * idx];
+      ls += f * sm_l[w2][cc];
+    }
+    *(f32x4 *)(to + 4 * idx) = f32x4{acc.x / ls, acc.y / ls, acc.z / ls, acc.w / ls};
+  }
+}
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kDecodeWaves = 4;  // wavefronts per workgroup (eight measured 4 % slower)
 
@@ -834,6 +1093,20 @@ __host__ __device__ inline bool whole_pairs(int longest, int q, int hd, int pair
 // Where no cut ends with the pairs, whole is the better way in any case:  1 of 16 and 15 of 8 15.3 | 9.5, 18.6 | 12.5, 17.8 | 13.7, 24 | 23.7.
 __host__ __device__ inline bool whole_first(int longest, int q, int hd, int cols) {
   return longest <= widest_aligned_span(q) || (hd <= 64 && longest <= 16) || (hd <= 128 && cols >= 8);
+}
+
+// Tiles per wavefront of decode_rows_kernel, or 0: not a call for it.  (Longer pairs would take more rounds of a wavefront's tiles, 1 us each, which the
+// kernel above overlaps with their loads; heads of 128 take twice the registers.)
+int row_tiles(const SeqTable &st, const Shape &sh, const DecodePlan &p, const DistanceBias *bias) {
+  if ((sh.hd != 64 && sh.hd != 128) || p.align <= 1 || (bias && bias->v_hd != sh.hd)) return 0;
+  int most = 0;
+  for (int s = 0; s < st.n_seqs; ++s) {
+    const int n = (st.start_pos[s] + 16) / 16;
+    if (st.n_new[s] != 1 || st.tok_off[s] != s || n > p.align || (s && st.slot[s] == st.slot[s - 1])) return 0;
+    most = n > most ? n : most;
+  }
+  const int tiles = (most + kDecodeWaves - 1) / kDecodeWaves;
+  return tiles <= (sh.hd == 64 ? kRowTiles<64> : kRowTiles<128>) ? tiles : 0;
 }
 
 struct ShareArg {
@@ -1055,6 +1328,40 @@ hipError_t launch_decode(const DecodeArgs &d, const SeqTable &st, const Shape &s
                                  : getenv("SHAINET_HIP_DECODE_ROTATE")
                                      ? (unsigned)atoi(getenv("SHAINET_HIP_DECODE_ROTATE"))
                                      : 0x7fffffffu;
+  if (const int tiles = dev ? 0 : row_tiles(st, sh, p, bias)) {
+    RowSeqs seqs = {};
+    for (int s = 0; s < st.n_seqs; ++s) {
+      seqs.start[s] = st.start_pos[s];
+      seqs.slot[s] = st.slot[s];
+    }
+    if (st.n_seqs > 1) ah.w = nullptr;
+    grid = dim3(ah.w ? grid.x : (unsigned)sh.KV, (unsigned)st.n_seqs);
+#define SHAINET_ROWS_LAUNCH(HD_, T_, MODE_)                                                                                          \
+  SHAINET_LAUNCH_TIMED((decode_rows_kernel<HD_, T_, MODE_>), grid, block, 0, stream, before, after, d.q_rot, d.kc, d.vc, d.out, seqs, \
+                       sh, c, rotate, ah, db, raw)
+#define SHAINET_ROWS_LAUNCH_T(HD_, T_)           \
+  do {                                           \
+    if (prep)                                    \
+      SHAINET_ROWS_LAUNCH(HD_, T_, kRowsPrep);   \
+    else if (bias)                               \
+      SHAINET_ROWS_LAUNCH(HD_, T_, kRowsBias);   \
+    else                                         \
+      SHAINET_ROWS_LAUNCH(HD_, T_, kRowsPlain);  \
+  } while (0)
+    if (sh.hd == 64 && tiles == 1)
+      SHAINET_ROWS_LAUNCH_T(64, 1);
+    else if (sh.hd == 64 && tiles == 2)
+      SHAINET_ROWS_LAUNCH_T(64, 2);
+    else if (sh.hd == 64)
+      SHAINET_ROWS_LAUNCH_T(64, 3);
+    else if (tiles == 1)
+      SHAINET_ROWS_LAUNCH_T(128, 1);
+    else
+      SHAINET_ROWS_LAUNCH_T(128, 2);
+#undef SHAINET_ROWS_LAUNCH_T
+#undef SHAINET_ROWS_LAUNCH
+    return hipGetLastError();
+  }
 #define SHAINET_DECODE_LAUNCH(HD_, DEV_, PAD_)                                                                      \
   SHAINET_LAUNCH_TIMED((decode_splitk_kernel<HD_, kDecodeWaves, DEV_, PAD_>), grid, block, 0, stream, before,      \
                        after, d.q_rot, d.kc, d.vc, d.out, part_o, part_ml, d.part_flag, flag_set, spin_limit,       \
