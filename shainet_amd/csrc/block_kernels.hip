@@ -11,6 +11,7 @@
 // free at these intensities on this part.
 #include "activation.hpp"
 #include "block_kernels.hpp"
+#include "split_mfma.hpp"
 
 #include <math.h>
 #include <stdint.h>
@@ -18,8 +19,6 @@
 namespace shainet {
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -30,7 +29,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 // One workgroup per row.
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ x, long long x_stride,
                                                       const float *__restrict__ gamma, float *__restrict__ out,
-                                                      int cols, double eps) {
+                                                      int cols, double eps, bool planes) {
   __shared__ double red[4];
   const float *xr = x + (long long)blockIdx.x * x_stride;
   float *orow = out + (long long)blockIdx.x * cols;
@@ -60,7 +59,10 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ 
       y.y = (float)(((double)v.y / rms) * (double)gm.y);
       y.z = (float)(((double)v.z / rms) * (double)gm.z);
       y.w = (float)(((double)v.w / rms) * (double)gm.w);
-      *(f32x4 *)(orow + j) = y;
+      if (planes)
+        store_planes(out, blockIdx.x, gridDim.x, j, cols, y);
+      else
+        *(f32x4 *)(orow + j) = y;
     }
   } else {
     for (int j = threadIdx.x; j < cols; j += 256)
@@ -129,14 +131,18 @@ __global__ __launch_bounds__(256) void embed_list_kernel(const float *__restrict
 // Dynamic Tanh: no statistics over the row, so a workgroup takes 1024 columns of one row.
 __global__ __launch_bounds__(256) void dyn_tanh_kernel(const float *__restrict__ x, long long x_stride,
                                                        const float *__restrict__ gamma, const float *__restrict__ beta,
-                                                       float alpha, float *__restrict__ out, int cols) {
+                                                       float alpha, float *__restrict__ out, int cols, bool planes) {
   const float *xr = x + (long long)blockIdx.x * x_stride;
   float *orow = out + (long long)blockIdx.x * cols;
   const int j = (blockIdx.y * 256 + threadIdx.x) * 4;
   if (j + 3 < cols && ((cols | x_stride) & 3) == 0) {
     const f32x4 v = *(const f32x4 *)(xr + j), g = *(const f32x4 *)(gamma + j), b = *(const f32x4 *)(beta + j);
-    *(f32x4 *)(orow + j) = f32x4{tanhf(alpha * v.x) * g.x + b.x, tanhf(alpha * v.y) * g.y + b.y,
-                                 tanhf(alpha * v.z) * g.z + b.z, tanhf(alpha * v.w) * g.w + b.w};
+    const f32x4 y = {tanhf(alpha * v.x) * g.x + b.x, tanhf(alpha * v.y) * g.y + b.y, tanhf(alpha * v.z) * g.z + b.z,
+                     tanhf(alpha * v.w) * g.w + b.w};
+    if (planes)
+      store_planes(out, blockIdx.x, gridDim.x, j, cols, y);
+    else
+      *(f32x4 *)(orow + j) = y;
   } else {
     for (int k = j; k < cols && k < j + 4; ++k) orow[k] = tanhf(alpha * xr[k]) * gamma[k] + beta[k];
   }
@@ -525,18 +531,19 @@ hipError_t launch_transpose(const float *src, float *dst, int rows, int cols, hi
 }
 
 hipError_t launch_rmsnorm(const float *x, long long x_stride, const float *gamma, float *out, int rows, int cols,
-                          double eps, hipStream_t stream) {
-  if (rows < 1 || cols < 1 || x_stride < cols) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)rows), dim3(256), 0, stream, x, x_stride, gamma, out, cols, eps);
+                          double eps, hipStream_t stream, bool planes) {
+  if (rows < 1 || cols < 1 || x_stride < cols || (planes && (cols % 32 || x_stride % 4))) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)rows), dim3(256), 0, stream, x, x_stride, gamma, out, cols, eps, planes);
   return hipGetLastError();
 }
 
 hipError_t launch_dyn_tanh(const float *x, long long x_stride, const float *gamma, const float *beta, float alpha,
-                           float *out, int rows, int cols, hipStream_t stream) {
-  if (!x || !gamma || !beta || !out || rows < 1 || cols < 1 || x_stride < cols || (cols + 1023) / 1024 > 65535)
+                           float *out, int rows, int cols, hipStream_t stream, bool planes) {
+  if (!x || !gamma || !beta || !out || rows < 1 || cols < 1 || x_stride < cols || (cols + 1023) / 1024 > 65535 ||
+      (planes && (cols % 32 || x_stride % 4)))
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(dyn_tanh_kernel, dim3((unsigned)rows, (unsigned)((cols + 1023) / 1024)), dim3(256), 0, stream, x,
-                     x_stride, gamma, beta, alpha, out, cols);
+                     x_stride, gamma, beta, alpha, out, cols, planes);
   return hipGetLastError();
 }
 

@@ -9,10 +9,11 @@ namespace shainet {
 // out[r, :] = x[r, :] / sqrt(mean(x[r, :]^2) + eps) * gamma   (gamma == nullptr: ones);
 // the rows of x are x_stride floats apart, those of out are dense
 hipError_t launch_rmsnorm(const float *x, long long x_stride, const float *gamma, float *out, int rows, int cols,
-                          double eps, hipStream_t stream);
+                          double eps, hipStream_t stream, bool planes = false);
+// planes: out is the parts of the rows (split_mfma.hpp, store_planes; cols a multiple of 32)
 // out[r, j] = tanh(alpha x[r, j]) * gamma[j] + beta[j], fp32; rows as for launch_rmsnorm
 hipError_t launch_dyn_tanh(const float *x, long long x_stride, const float *gamma, const float *beta, float alpha,
-                           float *out, int rows, int cols, hipStream_t stream);
+                           float *out, int rows, int cols, hipStream_t stream, bool planes = false);
 // dst[c, r] = src[r, c]: src is [rows, cols], dst [cols, rows], both dense
 hipError_t launch_transpose(const float *src, float *dst, int rows, int cols, hipStream_t stream,
                             const float *row_scale = nullptr);

@@ -64,6 +64,7 @@ __device__ __forceinline__ void coherent_store4(float *p, f32x4 v) {
 struct GemmArgs {
   const float *x;
   long long xs;
+  const unsigned short *planes;  // instead of x: its parts, lifted, [3][K / 32][T][32] (split_mfma.hpp)
   const float *w;
   float *y;
   const float *res;  // nullable: y = res + x W
@@ -462,12 +463,18 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
 // Us, tiles of 32 x 32 blocks and steps of 16 | this, both launches where there are two: 2048 rows of 2048 -> 16384 344 | 318, 8192 -> 2048 185 | 167, 2048 -> 2048
 // 60.6 | 57.1, 777 rows of 2048 -> 16384 164 | 144, 512 rows 90.9 | 85.4, of 8192 -> 2048 57.6 | 56.7, of 2048 -> 3072 30.6 | 30.6; with all loads, splits
 // and writes of a step in its first half 325, 173, 59.7, 153, 90.7, 58.9.  Errors against 64 bits 0.3 to 2 % smaller (fewer roundings).
-// What bounds it: on zeros 2048 rows of 2048 -> 16384 take 279 us, of which the MFMAs and fragments are 201, splits 26, writes to LDS 31 (17 cycles each
-// while MFMAs run) and loads 21; on random numbers the clock is at 2.06 GHz.
-template <int WM, bool GUARD, bool SWIGLU>
+// PLANES: x comes as its parts, which go from memory to LDS by themselves (a row's 64 bytes of a step, the four octets of row r at places o ^ (r / 2 % 4),
+// so that eight rows of an octet lie on eight banks' widths): no splits, a quarter of the writes.  The same bits.  Us, x | its parts: 2048 rows of
+// 2048 -> 16384 320 | 298, 777 rows 149 | 131, 512 rows 93 | 83, 300 rows 82 | 76, 512 rows of 2048 -> 3072 32.4 | 30.6, 2048 rows of 2048 -> 2048 58 | 55,
+// 8192 -> 2048 173 | 160, 512 rows 57 | 58.  The copies are not counted by the compiler: a step ends with a wait for all but its loads of W,
+// which are requested behind them.
+// What bounds it: on zeros 2048 rows of 2048 -> 16384 (x itself) take 279 us, of which the MFMAs and fragments are 201, splits 26, writes to LDS 31 (17
+// cycles each while MFMAs run) and loads 21; on random numbers the clock is at 2.06 GHz.
+template <int WM, bool GUARD, bool SWIGLU, bool PLANES>
 __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
   constexpr int WN = 8 / WM, MB = 4, NB = 2 * WM, TM = 64 * WM, TN = 256, NT = 512;
-  constexpr int NX = WM / 2;               // octets of x a thread stages (of W: two)
+  static_assert(!(GUARD && PLANES), "planes hold whole steps");
+  constexpr int NX = WM / 2;               // octets of x a thread stages (of W: two); PLANES: 16 rows of a part that a wavefront copies
   constexpr int kSets = WM == 4 ? 1 : 2;   // register sets: tiles are requested one step (of 3072 cycles) ahead, or two (of 1536)
   // units of 16 bytes; blocks of W a few units apart from 16, so that eight neighbouring threads' columns lie on eight different ones modulo 8
   constexpr int kOctX = TM, kPartX = 4 * kOctX, kBlockW = NB == 8 ? (SWIGLU ? 18 : 17) : (SWIGLU ? 20 : 18), kOctW = WN * NB * kBlockW;
@@ -517,28 +524,34 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     const int x_unit = (xk >> 3) * kOctX + xrow;
     const int w_unit = kW + (wk >> 3) * kOctW + wcol / (16 * NB) * (NB * kBlockW) + wcol % NB * kBlockW + wcol % (16 * NB) / NB;
     // fragments
-    const int a_unit = j * kOctX + wm * 64 + ln, b_unit = kW + j * kOctW + wn * (NB * kBlockW) + ln;
+    const int a_unit = PLANES ? (wm * 64 + ln) * 4 + (j ^ (ln >> 1 & 3)) : j * kOctX + wm * 64 + ln, b_unit = kW + j * kOctW + wn * (NB * kBlockW) + ln;
 
     // (rows past the last one repeat it and columns likewise: their products are never stored)
     unsigned x_off[NX], w_row[8];
 #pragma unroll
-    for (int u = 0; u < NX; ++u) x_off[u] = (unsigned)(((long long)min(m0 + xrow + 128 * u, T - 1) * g.xs + xk) * 4);
+    for (int u = 0; u < NX; ++u) {
+      if constexpr (PLANES)
+        x_off[u] = 64u * (unsigned)min(m0 + 16 * (wave + 8 * u) + (lane >> 2), T - 1) + 16u * ((lane & 3) ^ (lane >> 3 & 3));
+      else
+        x_off[u] = (unsigned)(((long long)min(m0 + xrow + 128 * u, T - 1) * g.xs + xk) * 4);
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) w_row[i] = (unsigned)(((long long)(wk + i) * N + w_from) * 4);
-    const char *x_base = (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)k_begin * N);
+    const char *x_base = PLANES ? (const char *)(g.planes + (long long)k_begin * T) : (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)k_begin * N);
+    const long long plane = 2LL * T * K;
 
     f32x4 sx[kSets][NX][2];
     float sw[kSets][2][8];
-    int k_next = k_begin, to_load = nk;
+    int k_next = k_begin, to_load = nk, to_copy = nk;
     auto load_x = [&](const int set, const int u, const int h) {
-      sx[set][u][h] = GUARD && k_next + xk + 4 * h >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : load_from((const f32x4 *)(x_base + 16 * h), x_off[u]);
+      if constexpr (!PLANES) sx[set][u][h] = GUARD && k_next + xk + 4 * h >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : load_from((const f32x4 *)(x_base + 16 * h), x_off[u]);
     };
     auto load_w = [&](const int set, const int o, const int i) {
       sw[set][o][i] = GUARD && k_next + wk + 16 * o + i >= k_end ? 0.f : load_from((const float *)(w_base + o * (64LL * N)), w_row[i]);
     };
     auto advance = [&]() {
       if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
-        x_base += kWideStep * 4;
+        if constexpr (!PLANES) x_base += kWideStep * 4;
         w_base += (long long)kWideStep * N * 4;
         k_next += kWideStep;
       }
@@ -547,11 +560,16 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     // The work beside the MFMAs, in pieces of at most four vector instructions (a SIMD issues two of them during an MFMA for nothing) or a write, of
     // which four wavefronts' take 70 cycles.  Per octet of x: four pairs split in four pieces each, three writes, two loads of the next; per octet of W: four
     // pairs, a write, eight loads.
-    constexpr int kItemsX = 21 * NX, kItems = kItemsX + 26;
+    constexpr int kItemsX = PLANES ? 3 * NX : 21 * NX, kItems = kItemsX + 26;
     u32x4 whole[3];
     float pa, pb;
     auto item = [&](const int it, const int set, u32x4 *stage) {
-      if (it < kItemsX) {
+      if (PLANES && it < kItemsX) {
+        const int u = it / 3, p = it % 3;
+        const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)(stage + p * kPartX + 64 * (wave + 8 * u)));
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(to), "v"(x_off[u]), "s"(x_base + p * plane) : "memory");
+        if (it == kItemsX - 1 && --to_copy > 0) x_base += 64LL * T;
+      } else if (it < kItemsX) {
         const int u = it / 21, m = it % 21, i = m / 4;
         if (m >= 19) {
           load_x(set, u, m - 19);
@@ -584,7 +602,7 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     };
     auto load_all = [&](const int set) {
 #pragma unroll
-      for (int u = 0; u < NX; ++u) load_x(set, u, 0), load_x(set, u, 1);
+      for (int u = 0; u < (PLANES ? 0 : NX); ++u) load_x(set, u, 0), load_x(set, u, 1);
 #pragma unroll
       for (int i = 0; i < 16; ++i) load_w(set, i / 8, i % 8);
       advance();
@@ -596,7 +614,7 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
 #pragma unroll
       for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     u32x4 af[2][3], bf[NB];
-    auto fetch_x = [&](const u32x4 *stage, const int a, const int p) { af[a & 1][p] = stage[a_unit + 16 * a + p * kPartX]; };
+    auto fetch_x = [&](const u32x4 *stage, const int a, const int p) { af[a & 1][p] = stage[a_unit + (PLANES ? 64 : 16) * a + p * kPartX]; };
     auto fetch_w = [&](const u32x4 *stage, const int b) { bf[b] = stage[b_unit + b * kBlockW]; };
     auto multiply = [&](const int a, const int b, const int p) { acc[a][b] = mfma_bf16_16(af[a & 1][p], bf[b], acc[a][b]); };
 
@@ -609,6 +627,7 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     for (int b = 0; b < NB; ++b) bf[b] = u32x4{0, 0, 0, 0};
 #pragma unroll
     for (int p = 0; p < 3; ++p) af[(MB - 1) & 1][p] = u32x4{0, 0, 0, 0};
+    if constexpr (PLANES) __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
 
     // A turn of the loop is the last blocks of rows of the step before (of zeros in front of the first), in which the fragments of W and of the
@@ -633,6 +652,7 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
             __builtin_amdgcn_sched_barrier(0);
           }
       }
+      if constexpr (PLANES) __builtin_amdgcn_s_waitcnt(0x4F70);  // vmcnt(16): all but this step's loads of W, which were requested behind its copies
       __syncthreads();
     };
     if constexpr (kSets == 1) {
@@ -670,7 +690,9 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
         f32x4 xv[MB];
 #pragma unroll
         for (int a = 0; a < MB; ++a)
-          xv[a] = in ? *(const f32x4 *)(g.x + (long long)min(m0 + wm * 64 + 16 * a + ln, T - 1) * g.xs + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+          xv[a] = !in      ? f32x4{0.f, 0.f, 0.f, 0.f}
+                  : PLANES ? join_planes(g.planes + ((long long)(k / 32) * T + min(m0 + wm * 64 + 16 * a + ln, T - 1)) * 32 + k % 32, (long long)T * K)
+                           : *(const f32x4 *)(g.x + (long long)min(m0 + wm * 64 + 16 * a + ln, T - 1) * g.xs + k);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1367,7 +1389,10 @@ __global__ __launch_bounds__(1024) void sgemm_sum_norm_kernel(const GemmArgs g, 
     }
     float *out = norm.rows + (long long)row * N + col;
     if constexpr (R == 1) {
-      *(f32x4 *)out = n;
+      if (norm.planes)
+        store_planes(norm.rows, row, g.T, col, N, n);
+      else
+        *(f32x4 *)out = n;
     } else {
       *(f32x2 *)out = f32x2{n.x, n.y};
       if (second) *(f32x2 *)(out + N) = f32x2{n.z, n.w};
@@ -1527,6 +1552,8 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[6] = p.mfma && K % (p.few ? step_k(p) : TK) != 0;
 }
 
+bool gemm_takes_planes(const GemmPlan &p, int K) { return p.mfma && p.parts == 1 && !p.few && K % kWideStep == 0; }
+
 // (the norm of a row takes a workgroup of up to 1024 threads, two registers of four each)
 bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
   if (!p.mfma) return false;
@@ -1534,7 +1561,7 @@ bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next) {
   // activations nothing else of a compute unit runs beside: us, a launch of its own behind it | in it, 777 rows of 2048 -> 2 x 8192 360 | 380,
   // 1024 rows 373 | 390, 2048 rows of 1024 -> 2 x 4096 194 | 207; a block of 24 shapes 1 % slower on average)
   if (next.swiglu) return !next.norm.rows && N % 8 == 0 && (p.pieces > 1 || !(p.parts == 3 && (p.few || p.mb == 4)));
-  if (p.pieces <= 1) return false;
+  if (p.pieces <= 1 || (next.norm.planes && (p.parts != 1 || N % 32 != 0))) return false;
   if (const GemvPrep *q = next.prep)
     return !next.norm.rows && !q->q_norm && !q->k_norm && !q->b_q && !q->b_k && !q->b_v && q->rope_tab && q->hd % 8 == 0 &&
            (long long)(q->H + 2 * q->KV) * q->hd == N && q->start_pos >= 0 && q->start_pos + T <= q->cap &&
@@ -1659,18 +1686,19 @@ hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, const GemmNext &ne
   return e != hipSuccess || !g.pieces ? e : launch_sum<2>(g, PieceShape{32 * WM * MB, 64 * WN, 32 * MB, WN, 64 * WM * WN}, next, stream);
 }
 
-template <int WM>
+template <int WM, bool PLANES>
 hipError_t launch_wide(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
   const bool guard = g.K % kWideStep != 0, swiglu = next.swiglu && !g.pieces;
+  if (guard && PLANES) return hipErrorInvalidValue;
   if (swiglu && guard)
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, true, true>), grid, dim3(512), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, !PLANES, true, PLANES>), grid, dim3(512), 0, stream, g);
   else if (swiglu)
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, true>), grid, dim3(512), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, true, PLANES>), grid, dim3(512), 0, stream, g);
   else if (guard)
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, true, false>), grid, dim3(512), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, !PLANES, false, PLANES>), grid, dim3(512), 0, stream, g);
   else
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, false>), grid, dim3(512), 0, stream, g);
+    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, false, PLANES>), grid, dim3(512), 0, stream, g);
   const hipError_t e = hipGetLastError();
   return e != hipSuccess || !g.pieces ? e : launch_sum<2 * WM>(g, PieceShape{64 * WM, 256, 64, 8 / WM, 512}, next, stream);
 }
@@ -1705,12 +1733,13 @@ hipError_t launch_stream(const GemmArgs &g, const GemmPlan &p, const GemmNext &n
 
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
                        unsigned *flags, int *error, int T, int K, int N, const GemmPlan &p, hipStream_t stream,
-                       unsigned *flag_set, int spin_limit, const float *bias, Activation act, const GemmNext &next) {
+                       unsigned *flag_set, int spin_limit, const float *bias, Activation act, const GemmNext &next, bool planes) {
+  if (planes && !gemm_takes_planes(p, K)) return hipErrorInvalidValue;
   const bool more = next.swiglu || next.norm.rows || next.prep;
   if (more && !gemm_takes_next(p, T, N, next)) return hipErrorInvalidValue;
   if (!x || !w || !y || T < 1 || K < 1 || N < 1 || x_stride < K) return hipErrorInvalidValue;
   const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias | (uintptr_t)next.norm.rows) & 15);
-  if (!aligned && more) return hipErrorInvalidValue;
+  if (!aligned && (more || planes)) return hipErrorInvalidValue;
   if (!p.mfma || !aligned) {
     hipLaunchKernelGGL(sgemm_plain_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)(T < 65535 ? T : 65535)), dim3(256), 0, stream, x,
                        x_stride, w, y, res, T, K, N, bias, act);
@@ -1719,8 +1748,9 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   if (p.partial_floats && !partials) return hipErrorInvalidValue;
   if (p.flag_words && (!flags || !error)) return hipErrorInvalidValue;
   GemmArgs g = {};
-  g.x = x;
+  g.x = planes ? nullptr : x;
   g.xs = x_stride;
+  g.planes = planes ? (const unsigned short *)x : nullptr;
   g.w = w;
   g.y = y;
   g.res = res;
@@ -1743,7 +1773,8 @@ hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float
   if (p.parts == 1) {
     if (p.few && p.kg == 4) return launch_stream<1, 4>(g, p, next, stream);
     if (p.few) return p.mb == 1 ? launch_stream<1, 2>(g, p, next, stream) : p.mb == 2 ? launch_stream<2, 2>(g, p, next, stream) : launch_stream<3, 2>(g, p, next, stream);
-    return p.mb == 4 ? launch_wide<4>(g, p, next, stream) : launch_wide<2>(g, p, next, stream);
+    if (planes) return p.mb == 4 ? launch_wide<4, true>(g, p, next, stream) : launch_wide<2, true>(g, p, next, stream);
+    return p.mb == 4 ? launch_wide<4, false>(g, p, next, stream) : launch_wide<2, false>(g, p, next, stream);
   }
   if (p.few) return launch_few(g, p, next, stream);
   if (p.wn == 4) return p.mb == 4 ? launch_tiles<2, 4, 4>(g, p, next, stream) : launch_tiles<2, 4, 2>(g, p, next, stream);

@@ -13,6 +13,7 @@ struct NextNorm {
   float alpha = 0.f;
   double eps = 0.0;
   float *rows = nullptr;  // [T, N]: the norm of y's rows goes there (null: none)
+  bool planes = false;    // as their parts (split_mfma.hpp, store_planes); W of one part
 };
 struct GemvPrep;  // attn_kernels.hpp
 struct GemmNext {
@@ -50,7 +51,9 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]);  // shainet_hip_descr
 hipError_t launch_gemm(const float *x, long long x_stride, const float *w, float *y, const float *res, float *partials,
                        unsigned *flags, int *error, int T, int K, int N, const GemmPlan &p, hipStream_t stream,
                        unsigned *flag_set = nullptr, int spin_limit = 0, const float *bias = nullptr, Activation act = Activation(),
-                       const GemmNext &next = GemmNext());
+                       const GemmNext &next = GemmNext(), bool planes = false);
+// planes: x is [3][T][K] of bf16, the parts of its lifted values (split_mfma.hpp, split_planes), in a product that takes it so.
+bool gemm_takes_planes(const GemmPlan &p, int K);
 // Whether the product's last launch does that, too.
 bool gemm_takes_next(const GemmPlan &p, int T, int N, const GemmNext &next);
 

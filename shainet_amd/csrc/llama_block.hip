@@ -530,6 +530,8 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
   Handover second;
   second.norm = &w.norm2;
   second.eps = b->eps;
+  second.n = 2 * ff;
+  second.w_bf16 = w.gate_up_bf16;
   if (carry) {
     n1.normed = carry->normed;
     carry->normed = nullptr;
@@ -558,6 +560,7 @@ int block_forward_device(shainet_llama_block *b, const float *x, int T, float *o
   if (!ff && behind) carry->normed = behind->rows;
   if (rc || !ff) return rc;
   gate.normed = second.rows;
+  gate.normed_planes = second.planes;
   // hidden = silu(normed2 * gate_proj) * (normed2 * up_proj), normed2 = @norm2.forward(h)
   if ((rc = proj.project(h, d, w.gate_up, b->hidden.p, T, d, ff, stream, gate))) return rc;
   // out = h + hidden * down_proj

@@ -71,7 +71,10 @@ namespace shainet {
 struct Handover {
   const NormWeights *norm = nullptr;
   double eps = 0.0;
+  int n = 0;             // columns of the product that reads these rows, and whether its weights are bf16 numbers (0: it takes the rows as they are)
+  bool w_bf16 = false;
   const float *rows = nullptr;  // set by the product: the result's rows behind the norm, dense; null: the norm is still to be taken
+  bool planes = false;          // set by the product: as their parts, which that product takes so (gemm_takes_planes)
 };
 
 }
@@ -137,6 +140,7 @@ struct Fused {
   bool w_bf16 = false;  // every value of W is a bf16 number: half the MFMAs of many rows have nothing to add
   bool any_few_rows = false;  // up to 16 rows run as the split GEMV, not only the ones it is the faster product for
   const float *normed = nullptr;  // [T, K]: the rows of x behind the norm, where an earlier product handed them over (more than a few rows only)
+  bool normed_planes = false;     // as their parts (Handover::planes)
   Handover *next = nullptr;       // nullable; for kGemvPlain and kGemvResidual
   const ResidualArgs *join = nullptr;  // x is this row's h, still to be made: in the product's launch where that takes it along (x may stay unwritten then)
   bool w_t_has_gamma = false;  // the rows of w_t were made with gamma multiplied in: the norm's factor 1 / rms is all that is left to apply
@@ -194,7 +198,7 @@ struct Projector {
   // res != nullptr: y = res + x W
   int gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N, hipStream_t stream, bool w_bf16,
            const float *res = nullptr, const float *bias = nullptr, Activation act = Activation(), bool swiglu = false, Handover *next = nullptr,
-           const GemvPrep *spread = nullptr);
+           const GemvPrep *spread = nullptr, bool planes = false);
 };
 
 // Replace *dst (device, hipMalloc'ed or null) by a copy of n host floats.

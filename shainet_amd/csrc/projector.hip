@@ -138,7 +138,7 @@ int Projector::reserve_flags(size_t n_flags, hipStream_t stream) {
 // swiglu: W is gate | up and y [T, N / 2].
 int Projector::gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
                     hipStream_t stream, bool w_bf16, const float *res, const float *bias, Activation act, bool swiglu, Handover *next,
-                    const GemvPrep *spread) {
+                    const GemvPrep *spread, bool planes) {
   const GemmPlan p = plan_gemm(T, K, N, x_stride, w_bf16);
   const bool aligned = !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)res | (uintptr_t)bias) & 15);
   GemmNext also;
@@ -155,18 +155,21 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
   if (int rc = reserve_flags(p.flag_words, stream)) return rc;
   // (what the product itself needs comes first: without the memory for these rows they are normed in front of the next product, as
   // after one that adds no pieces)
-  if (next && next->norm->kind != kNormNone && !bias && aligned && gemm_takes_next(p, T, N, also) && handed.reserve((size_t)T * N)) {
+  const bool as_planes = next && p.parts == 1 && next->n && gemm_takes_planes(plan_gemm(T, N, next->n, N, next->w_bf16), N);
+  if (next && next->norm->kind != kNormNone && !bias && aligned && gemm_takes_next(p, T, N, also) &&
+      handed.reserve((size_t)T * N / 2 * (as_planes ? 3 : 2))) {
     also.norm.kind = next->norm->kind;
     also.norm.gamma = next->norm->gamma;
     also.norm.beta = next->norm->beta;
     also.norm.alpha = next->norm->alpha;
     also.norm.eps = next->eps;
     also.norm.rows = handed.p;
+    also.norm.planes = next->planes = as_planes;
     next->rows = handed.p;
   }
   if (p.flag_words && !error) return llama_fail(SHAINET_HIP_ERR_RUNTIME, "the projector has no error word");
   hipError_t e = launch_gemm(x, x_stride, w, result, res, scratch.p, flags, error, T, K, N, p, stream,
-                             lose_marks ? flags + flags_cap : nullptr, lose_marks ? 2000 : 0, bias, act, also);
+                             lose_marks ? flags + flags_cap : nullptr, lose_marks ? 2000 : 0, bias, act, also, planes);
   if (e == hipSuccess && swiglu && !also.swiglu) e = launch_swiglu_act(wide.p, y, T, N / 2, stream);
   if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("gemm launch: ") + hipGetErrorString(e));
   return SHAINET_HIP_OK;
@@ -275,20 +278,26 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
   const float *xin = x;
   long long xs = x_stride;
   hipError_t e = hipSuccess;
+  bool planes = false;
   if (f.norm && f.normed) {
     xin = f.normed;
     xs = K;
+    planes = f.normed_planes;
   } else if (f.norm) {
-    if (!normed.reserve((size_t)T * K)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
-    e = f.norm == kNormDynTanh ? launch_dyn_tanh(x, x_stride, f.gamma, f.beta, f.alpha, normed.p, T, K, stream)
-                               : launch_rmsnorm(x, x_stride, f.gamma, normed.p, T, K, f.eps, stream);
+    // (rows that the product copies as their parts are written so: 2048 rows of 2048 -> 16384 319 us and 298, 512 rows 94 and 83, 777 rows
+    // 151 and 131, 512 rows of 2048 -> 3072 32.8 and 30.6; a launch of its own for the parts would take 5 to 8 of these)
+    planes = (x_stride & 3) == 0 && !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)f.res | (uintptr_t)f.bias) & 15) &&
+             gemm_takes_planes(plan_gemm(T, K, swiglu ? 2 * N : N, K, f.w_bf16), K);
+    if (!normed.reserve((size_t)T * K / 2 * (planes ? 3 : 2) + 1)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
+    e = f.norm == kNormDynTanh ? launch_dyn_tanh(x, x_stride, f.gamma, f.beta, f.alpha, normed.p, T, K, stream, planes)
+                               : launch_rmsnorm(x, x_stride, f.gamma, normed.p, T, K, f.eps, stream, planes);
     if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("norm launch: ") + hipGetErrorString(e));
     xin = normed.p;
     xs = K;
   }
-  if (swiglu) return gemm(xin, xs, w, y, T, K, 2 * N, stream, f.w_bf16, nullptr, nullptr, Activation(), true);
+  if (swiglu) return gemm(xin, xs, w, y, T, K, 2 * N, stream, f.w_bf16, nullptr, nullptr, Activation(), true, nullptr, nullptr, planes);
   return gemm(xin, xs, w, y, T, K, N, stream, f.w_bf16, f.epilogue == kGemvResidual ? f.res : nullptr,
-              f.epilogue == kGemvBias ? f.bias : nullptr, f.act, false, f.next, f.spread);
+              f.epilogue == kGemvBias ? f.bias : nullptr, f.act, false, f.next, f.spread, planes);
 }
 
 void Projector::release() {

@@ -97,6 +97,48 @@ __device__ __forceinline__ void split_octet(f32x4 a, f32x4 b, u32x4 &high, u32x4
   low = u32x4{l[0].x, l[0].y, l[1].x, l[1].y};
 }
 
+// The parts of four lifted floats as a product takes them from memory, in three planes.  What a bf16 cannot hold lifted (not finite, or from
+// 2^104 on) is NaN in the first plane, so that its sums are taken again, and stands as it is in the two others.
+__device__ __forceinline__ void split_planes(f32x4 v, u32x2 (&part)[3]) {
+  split_quad(v * kLift, part[0], part[1], part[2]);
+  const unsigned any = 0x7f807f80u;  // exponents of all ones
+  const unsigned a = part[0].x & any, b = part[0].y & any;
+  if ((a & 0xffffu) == 0x7f80u || (a >> 16) == 0x7f80u || (b & 0xffffu) == 0x7f80u || (b >> 16) == 0x7f80u) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = 16 * (i & 1);
+      const unsigned bits = __builtin_bit_cast(unsigned, (float)v[i]);
+      if ((part[0][i >> 1] >> at & 0x7f80u) != 0x7f80u) continue;
+      part[0][i >> 1] = (part[0][i >> 1] & ~(0xffffu << at)) | 0x7fc0u << at;
+      part[1][i >> 1] = (part[1][i >> 1] & ~(0xffffu << at)) | (bits >> 16) << at;
+      part[2][i >> 1] = (part[2][i >> 1] & ~(0xffffu << at)) | (bits & 0xffffu) << at;
+    }
+  }
+}
+// ... and into planes [3][cols / 32][rows][32]: four neighbouring columns of a row (of 64 bytes in a plane, so that what a product copies
+// for a step of 32 along K lies together: rows of whole planes, K apart by a power of two, took 2048 rows of 8192 -> 2048 from 160 to 248 us)
+__device__ __forceinline__ void store_planes(void *planes, int row, int rows, int col, int cols, f32x4 v) {
+  u32x2 part[3];
+  split_planes(v, part);
+  unsigned short *at = (unsigned short *)planes + ((long long)(col / 32) * rows + row) * 32 + col % 32;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) *(u32x2 *)(at + p * (long long)rows * cols) = part[p];
+}
+// four neighbouring floats, whole again; plane: numbers from a part to the next
+__device__ __forceinline__ f32x4 join_planes(const unsigned short *at, long long plane) {
+  const u32x2 h = *(const u32x2 *)at, m = *(const u32x2 *)(at + plane), l = *(const u32x2 *)(at + 2 * plane);
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    auto part = [&](const u32x2 &p) { return (i & 1 ? p[i >> 1] >> 16 : p[i >> 1] & 0xffffu) << 16; };
+    const unsigned a = part(h), b = part(m), c = part(l);
+    v[i] = (a & 0x7f800000u) == 0x7f800000u
+               ? __builtin_bit_cast(float, b | c >> 16)
+               : ((__builtin_bit_cast(float, a) + __builtin_bit_cast(float, b)) + __builtin_bit_cast(float, c)) * kDropOne;
+  }
+  return v;
+}
+
 // The parts of the two factors in the six products that are taken, smallest first.
 constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
 
