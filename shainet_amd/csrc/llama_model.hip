@@ -377,7 +377,11 @@ int run_device_tokens(shainet_llama_model *m, const int *d_tokens, int T, bool n
     const int start = no_cache ? 0 : shainet_llama_model_cache_len(m);
     if ((rc = check_positions(m, start, T))) return rc;
     const float *positions = m->positions ? m->positions + (size_t)start * d : nullptr;
-    const hipError_t e = embedded ? hipSuccess
+    // (one id that the host knows, whose row of the table is its embedding as it stands: nobody has to copy it)
+    const float *in_table = list && T == 1 && !embedded && !positions && m->embedding_scale == 1.f && (d & 3) == 0 && !m->blocks.empty()
+                                ? m->embedding + (size_t)list->id[0] * d
+                                : nullptr;
+    const hipError_t e = embedded || in_table ? hipSuccess
                          : list   ? launch_embed_list(m->embedding, *list, m->act[0].p, T, d, m->stream, m->embedding_scale, positions)
                                   : launch_embed(m->embedding, d_tokens, m->act[0].p, T, d, m->stream, m->embedding_scale, positions);
     if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("embedding launch: ") + hipGetErrorString(e));
@@ -387,7 +391,8 @@ int run_device_tokens(shainet_llama_model *m, const int *d_tokens, int T, bool n
       if ((rc = shainet_llama_block_set_stream(b, m->stream))) return rc;
       carry.next = Handover();
       if (i + 1 < m->blocks.size()) carry.next.norm = shainet_llama_block_first_norm(m->blocks[i + 1], &carry.next.eps);
-      if ((rc = shainet_llama_block_forward_device(b, m->act[cur].p, T, m->act[cur ^ 1].p, no_cache, &carry))) return rc;
+      const float *from = i == 0 && in_table ? in_table : m->act[cur].p;
+      if ((rc = shainet_llama_block_forward_device(b, from, T, m->act[cur ^ 1].p, no_cache, &carry))) return rc;
       cur ^= 1;
     }
     if (carry.y && (rc = shainet_llama_block_join_carry(m->blocks.back(), carry, m->act[cur].p, T))) return rc;
