@@ -392,8 +392,10 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const float *_
   if (t < n) weight[t] = exp((double)v / temperature - (double)key_value(s.win[0], logits) / temperature);
   __syncthreads();
   if (t != 0) return;
+  // (the host may be looking at the word)
+  auto say = [&](int id) { __hip_atomic_store(pick, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
   if (n <= 0) {  // all-NaN row: nothing to sample (sampler.cr:121)
-    *pick = 0;
+    say(0);
     return;
   }
   double sum = 0.0;
@@ -408,7 +410,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const float *_
       break;
     }
   }
-  *pick = (int)(~(unsigned)(s.win[best] & 0xffffffffu));
+  say((int)(~(unsigned)(s.win[best] & 0xffffffffu)));
 }
 
 // Sampler.greedy and the next step's embedding lookup in one launch of one workgroup: *id = the largest finite

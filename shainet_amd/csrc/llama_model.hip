@@ -753,6 +753,18 @@ int shainet_llama_model_topk(shainet_llama_model *m, int k, int *ids, float *val
   return run_topk(m, k, false, ids, vals, count);
 }
 
+// The id is there when the host sees it: the word is written by the last launch on the stream, behind everything else, and a wait for the stream
+// would be a packet and a signal more (a token of a chat 4 us).  A stream that has come to its end, or to an error, without it ends the wait.
+static constexpr int kNoPick = -1;  // (ids are not negative)
+static bool wait_for_pick(const int *word, hipStream_t stream) {
+  while (*(const volatile int *)word == kNoPick) {
+    for (int i = 0; i < 4096 && *(const volatile int *)word == kNoPick; ++i) __builtin_ia32_pause();
+    if (*(const volatile int *)word == kNoPick && hipStreamQuery(stream) != hipErrorNotReady)
+      return hipStreamSynchronize(stream) == hipSuccess && *(const volatile int *)word != kNoPick;
+  }
+  return true;
+}
+
 int shainet_llama_model_sample(shainet_llama_model *m, int k, double temperature, double r, int *token) {
   if (!m || !token) return fail(SHAINET_HIP_ERR_ARGUMENT, "null argument");
   if (!m->have_logits) return fail(SHAINET_HIP_ERR_ARGUMENT, "no logits: call shainet_llama_model_run first");
@@ -770,11 +782,11 @@ int shainet_llama_model_sample(shainet_llama_model *m, int k, double temperature
     return fail(SHAINET_HIP_ERR_ALLOC, "hipHostMalloc failed");
   // dividing by a positive temperature keeps the order of the logits: the selection over v / t
   // (sampler.cr:100-115) is the selection over v
+  *(volatile int *)m->h_pick = kNoPick;
   const hipError_t e = launch_topk(m->logits.p, m->vocab, k, false, m->topk_scratch, nullptr, nullptr, nullptr, m->stream, -1, m->h_pick,
                                    temperature, r);
   if (e != hipSuccess) return fail(SHAINET_HIP_ERR_RUNTIME, std::string("sample launch: ") + hipGetErrorString(e));
-  if (hipStreamSynchronize(m->stream) != hipSuccess)
-    return fail(SHAINET_HIP_ERR_RUNTIME, "waiting for the sampled id failed");
+  if (!wait_for_pick(m->h_pick, m->stream)) return fail(SHAINET_HIP_ERR_RUNTIME, "waiting for the sampled id failed");
   if (int rc = check_error_word(m->error)) return rc;
   *token = *(volatile int *)m->h_pick;
   return SHAINET_HIP_OK;
