@@ -5,9 +5,9 @@
 // attention_kv_kernel (cuda_kernels.cu:734-806):
 //
 //   prefill_mfma_kernel   many new rows.  Query rows and the heads of a group
-//       are flattened into "virtual rows"; a wavefront owns 32 of them, a
-//       workgroup 128.  K/V tiles of 32 keys are split into bf16 parts on their way
-//       to LDS and consumed by v_mfma_f32_32x32x16_bf16.
+//       are flattened into "virtual rows"; a wavefront owns 32 of them.
+//       K/V tiles of 32 keys are split into bf16 parts on their way
+//       to LDS and consumed by v_mfma_f32_16x16x32_bf16.
 //   generic_attn_kernel   any head_dim; one wavefront per (row, head).  Used for
 //       head dims other than 64 and 128.
 //
@@ -35,24 +35,28 @@ __device__ __forceinline__ int find_seq(const SeqTable &st, int item, const int 
 }
 
 // ---------------------------------------------------------------------------
-// Prefill: MFMA 32x32x16, K/V tiles staged through LDS.
+// Prefill: MFMA 16x16x32, K/V tiles staged through LDS.
 //
 // Virtual row v of a (sequence, kv head): query row v / g, head kvh*g + v % g.
-// MFMA layout (lane l, j = l/32): A[m = l%32][k = 8j .. 8j+7], B[k = 8j .. 8j+7][n = l%32],
-// D[m = 8*(r/4) + 4*j + r%4][n = l%32] for accumulator register r = 0..15.
-//   scores:  m = key within the tile, n = virtual row, k = d.
-//   output:  tile t, m = d index (d = NT*m + t), contraction over the tile's keys in
-//            the order the score accumulator holds them.
+// MFMA layout (lane l, j = l/16): A[m = l%16][k = 8j .. 8j+7], B[k = 8j .. 8j+7][n = l%16],
+// D[m = 4j + r][n = l%16] for accumulator register r = 0..3.  A wavefront's 32 keys x 32 virtual rows are
+// two blocks by two:
+//   scores:  m = key within the block, n = virtual row, k = d.
+//   output:  block t, m = d index (d = NT*m + t), contraction over the tile's 32 keys in
+//            the order the score accumulators hold them.
 // Row block number `rank` in dispatch order -> (sequence, block).  Level 0 is every
 // sequence's last block (the longest key range), level 1 the one before, and so
 // on.  st.work_off[s] = row blocks of sequence s, st.ord = sequences by descending
 // block count.
+// PER: blocks that are handed out together, those of one sequence from PER vb on.
+template <int PER = 1>
 __device__ __forceinline__ void locate_block(const SeqTable &st, int rank, int &s, int &vb) {
+  auto count = [&](int i) { return (st.work_off[i] + PER - 1) / PER; };
   s = 0;
   int level = 0;
   for (int b = st.n_seqs - 1; b >= 0; --b) {  // levels [n_{b+1}, n_b) have b+1 active sequences
-    const int lo = b + 1 < st.n_seqs ? st.work_off[st.ord[b + 1]] : 0;
-    const int cnt = (st.work_off[st.ord[b]] - lo) * (b + 1);
+    const int lo = b + 1 < st.n_seqs ? count(st.ord[b + 1]) : 0;
+    const int cnt = (count(st.ord[b]) - lo) * (b + 1);
     if (rank < cnt) {
       level = lo + rank / (b + 1);
       s = st.ord[rank % (b + 1)];
@@ -60,29 +64,42 @@ __device__ __forceinline__ void locate_block(const SeqTable &st, int rank, int &
     }
     rank -= cnt;
   }
-  vb = st.work_off[s] - 1 - level;
+  vb = count(s) - 1 - level;
+}
+
+// The number of a block (PER = 1) in that order: all blocks of lower levels and those of its own level in front of it.
+__device__ __forceinline__ int block_rank(const SeqTable &st, int s, int vb) {
+  const int level = st.work_off[s] - 1 - vb;
+  int rank = 0;
+  bool before = true;
+  for (int b = 0; b < st.n_seqs; ++b) {
+    before = before && st.ord[b] != s;
+    rank += min(st.work_off[st.ord[b]], level) + (before && st.work_off[st.ord[b]] > level ? 1 : 0);
+  }
+  return rank;
 }
 
 // Units of 16 bytes (eight bf16, one MFMA operand of a lane) that one key tile takes in LDS.  K: [part][octet of
-// d][key], an octet's 32 keys one unit apart from a multiple of 16 (a row's octets are written side by side).  V:
-// [part][group of eight keys][column], column d at place d / NT of block d % NT, four units of padding a block; group
-// 2 u + j holds the keys 16 u + 4 j + {0 .. 3, 8 .. 11}, the ones whose probabilities lane half j has in its
-// registers 8 u .. 8 u + 7.
+// d][key], key r of octet o at place r ^ o % 8.  V: [part][group of eight keys][column], column d at place d / NT of block d % NT; group
+// j holds the keys 4 j + {0 .. 3, 16 .. 19}, the ones whose probabilities the lanes of quarter j have.
+// LDS serves a read in four turns of 16 lanes (0 .. 3, 12 .. 15, 20 .. 23 and 24 .. 27 are the first), whose units have to differ modulo 16: octets
+// and groups are multiples of 16 apart, and only the lowest bits of a place depend on the octet of a quarter.  (33 units an octet, 72 or 136 a group: a third
+// to half of all cycles of LDS were conflicts.)  So have 16 neighbouring threads' writes: eight octets of two keys eight apart, 16 columns.
 template <int HD>
 struct TileUnits {
-  static constexpr int NT = HD / 32;
-  static constexpr int kOctK = 33, kPartK = HD / 8 * kOctK;
-  static constexpr int kGroupV = NT * 36, kPartV = 4 * kGroupV;
+  static constexpr int NT = HD / 16;
+  static constexpr int kPartK = HD / 8 * 32;
+  static constexpr int kBlockV = NT == 8 ? 18 : 20, kGroupV = NT * kBlockV, kPartV = 4 * kGroupV;
   static constexpr int kK = 3 * kPartK, kTile = kK + 3 * kPartV;
+  static __device__ __forceinline__ int key_unit(int oct, int r) { return oct * 32 + (r ^ (oct & 7)); }
 };
 
-// G = 1: four wavefronts, each with 32 virtual rows, walk the key tiles together.
-// G = 2: eight wavefronts; wavefronts 4..7 own the same rows as 0..3 and take every
-// second key tile, so that each SIMD holds two wavefronts of one workgroup and the
-// waits and vector instructions of one hide behind the MFMAs of the other
-// even when a launch puts a single workgroup on a compute unit.  The two
+// Eight wavefronts, two groups of four, one of each on a SIMD and half a step apart: while one group has MFMAs, the
+// other has softmax, splits and staging.
+// G = 2: wavefronts 4..7 own the same 128 virtual rows as 0..3 and take every second key tile; the two
 // halves merge through LDS.
-// One workgroup's work: the row block (and key chunk) number `bid` of the launch.
+// G = 1: two row blocks of a sequence; both groups walk the same key tiles, which are staged and split once for 256 rows.
+// One workgroup's work: the row block, or pair of them (and key chunk) number `bid` of the launch.
 // PAD: the head dimension of the data (sh.hd, a multiple of 4) is smaller than HD, the one the
 // tiles are laid out for: query elements beyond it are zeros (whatever stands in for the keys'
 // there does not reach the scores), output elements beyond it are not stored, and a tile's
@@ -91,14 +108,26 @@ struct TileUnits {
 //
 // Queries, keys, values and probabilities enter the MFMAs as exact sums of three bf16 numbers
 // (split_mfma.hpp): the queries once, a key tile by the workgroup on its way to LDS, the probabilities in
-// the registers the scores came in.  A tile costs a wavefront HD / 16 x 6 + HD / 16 x 6 MFMAs of 32 cycles (64:
-// 1536) where the fp32 instruction took HD x 64 (4096), and about as many cycles of vector instructions, which run
-// beside them.  Kernel times, the fp32 instruction before (us): 2048 rows, 32 / 8 heads of 64, 99 (146), 8192 rows 1324
-// (2050); 512 rows on 16384 cached, 32 / 4 heads of 128, 684 (1056); 2048 rows, 32 / 8 heads of 128, 186 (279).
-// Bound by the power the card may draw, as the large products are; raising one group's priority changes nothing and
-// parking V between the score MFMAs costs 5 to 16 %.  (Queries and keys as two fp16 numbers and scores of three products
+// the registers the scores came in.  A tile costs a wavefront HD / 16 x 12 + HD / 16 x 12 MFMAs of 16 cycles (64:
+// 1536) where the fp32 instruction took HD x 64 (4096).
+// Us, v_mfma_f32_32x32x16_bf16 with both wavefronts of a SIMD in step | this: 2048 rows, 32 / 8 heads of 64, 106.7 | 96.4, 4096 rows 370 | 303, 512 rows on
+// 16384 366 | 304; 512 rows on 16384, 32 / 4 heads of 128, 690 | 551, 2048 rows, 32 / 8 heads of 128, 221 | 199, 4096 rows 743 | 596; 2048 rows of 32 heads of 96
+// 214 | 178.  Errors against 64 bits 0 to 13 % smaller.
+// What each part of it gave: half a step apart 104 | 100 and fragments a block ahead of their MFMAs 98; the layout of LDS without conflicts 96 | 92.6; a block's
+// products on one accumulator rather than two in turn 1 %; the reference value of the softmax as where the scores' sums begin 1 to 2.6 %; two row blocks a
+// workgroup and the queries' third parts in LDS, which ended spills, 656 | 568 (512 rows on 16384, heads of 128).  In step
+// again (no group waits half a step at the start) short ranges take 2 to 10 % longer.
+// What bounds it: heads of 128 the power the card may draw (matrix cores busy 78 % at 1.9 GHz); heads of 64 vector instructions: 281 and 16
+// exponentials a tile and wavefront, of which a SIMD issues two during an MFMA of 16 cycles.  (Queries and keys as two fp16 numbers and scores of three products
 // took 14 and 17 % less, but such numbers leave out up to 2^-21 of a product, and where a key's second parts have the signs of the
 // query's that adds up.)
+// Heads of 128 have no registers for the queries' third parts, or those of 24 of 32 octets: these lie in LDS, too.  (G = 2: both groups have the same.)
+template <int HD, int G>
+constexpr int kThirds = HD == 128 ? (G == 2 ? 4 : 3) : 0;
+template <int HD, int G>
+constexpr int kLdsUnits = 2 * TileUnits<HD>::kTile + (G == 2 ? 4 : 8) * kThirds<HD, G> * 128;
+static_assert(kLdsUnits<128, 1> * 16 <= 160 * 1024 && kLdsUnits<128, 2> * 16 <= 160 * 1024, "LDS of a compute unit");
+
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS>
 __device__ __forceinline__ void prefill_block(const int bid, const float *__restrict__ q_rot,
                                               const float *__restrict__ kc, const float *__restrict__ vc,
@@ -107,11 +136,13 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
                                               int ns, float c, const DistanceBias &db) {
   static_assert(PAD || !BIAS, "sizes of their own come with padding");
   using U = TileUnits<HD>;
-  constexpr int KS = HD / 16;   // MFMA steps along d of the scores
-  constexpr int NT = HD / 32;   // d tiles of the output
-  constexpr int NI = HD / 64;   // items per thread to stage the G K (or V) tiles of one step
-  constexpr int NTHREADS = 256 * G;
-  __shared__ __attribute__((aligned(16))) u32x4 lds[G * U::kTile];
+  constexpr int KS = HD / 32;   // MFMA steps along d of the scores
+  constexpr int NT = HD / 16;   // d blocks of the output
+  // items per thread to stage a tile of K (or V): G = 2, the tile of its group; G = 1, the one that all share, heads of 64: K is the first
+  // group's, V the second's
+  constexpr int NI = G == 2 ? HD / 64 : 1;
+  constexpr bool kOneOfTwo = G == 1 && HD == 64;
+  __shared__ __attribute__((aligned(16))) u32x4 lds[kLdsUnits<HD, G>];
 
   // Workgroups are numbered so that the hardware dispatcher, which hands them out in
   // index order, starts the row blocks with the longest key ranges first; the kv
@@ -123,7 +154,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int chunk = SPLIT ? (bid / sh.KV) % ns : 0;
   const int item = SPLIT ? bid / sh.KV / ns : bid / sh.KV;
   int s, vb;
-  locate_block(st, item, s, vb);
+  locate_block<3 - G>(st, item, s, vb);
   // These are the same for all lanes of a wavefront, which the compiler cannot see: said so,
   // tile counts, loop conditions and address bases live in scalar registers
   auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
@@ -133,18 +164,15 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int L = S + T, VR = T * g;
   const int lane = threadIdx.x & 63;
   const int wave = uniform((threadIdx.x >> 6) & 3);  // which 32 virtual rows of the block
-  const int gidx = uniform(threadIdx.x >> 8);        // which share of the key tiles (always 0 for G = 1)
-  const int n = lane & 31, j = lane >> 5;
+  const int gidx = uniform(threadIdx.x >> 8);        // which group of wavefronts
+  const int wg_hi = st.start_pos[s] + min((vb + 1) * 128 * (3 - G) - 1, st.n_new[s] * sh.g - 1) / sh.g;
+  if (G == 1) vb = 2 * vb + gidx;
+  const int first_tile = G == 2 ? gidx : 0;  // a group's first key tile
+  const int n = lane & 15, j = lane >> 4;
   const int v0 = vb * 128 + wave * 32;
   const bool wave_active = v0 < VR;
-  const int my_v = v0 + n;
-  const bool valid = my_v < VR;
-  const int row = valid ? my_v / g : T - 1;
-  const int hg = valid ? my_v - row * g : 0;
-  const int lim = S + row;                                            // last visible key of this lane's row
   const int wave_lo = S + (wave_active ? v0 / g : 0);                 // smallest lim in the wavefront
   const int wave_hi = wave_active ? S + min(v0 + 31, VR - 1) / g : -1;  // largest
-  const int wg_hi = S + min(vb * 128 + 127, VR - 1) / g;
   const int n_tiles = wg_hi / 32 + 1;
   const int tiles_per_chunk = SPLIT ? (n_tiles + ns - 1) / ns : n_tiles;
   const int kt0 = chunk * tiles_per_chunk, kt1 = min(n_tiles, kt0 + tiles_per_chunk);
@@ -153,27 +181,37 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const float *kbase = kc + head_base;
   const int vhd = BIAS ? uniform(db.v_hd) : hd;
   const float *vbase = vc + (BIAS ? ((long long)st.slot[s] * sh.KV + kvh) * sh.cap * vhd : head_base);
-  const long long qo_off = ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * vhd;  // of the row's result
-  const long long q_off = BIAS ? (st.tok_off[s] + row) * db.q_stride + (long long)(kvh * g + hg) * hd : qo_off;
-  // entry of key row k: bias_row[k]
-  const float *bias_row = BIAS ? db.tab + (long long)(kvh * g + hg) * db.stride + (db.origin - lim) : nullptr;
+  // a lane's two virtual rows, v0 + n and 16 on
+  int lim[2];  // last visible key of the row
+  long long q_off[2];        // of the row's query
+  const float *bias_row[2];  // entry of key row k: bias_row[k]
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int my_v = v0 + 16 * b + n;
+    const int row = my_v < VR ? my_v / g : T - 1, hg = my_v < VR ? my_v - row * g : 0;
+    lim[b] = S + row;
+    q_off[b] = BIAS ? (st.tok_off[s] + row) * db.q_stride + (long long)(kvh * g + hg) * hd
+                    : ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * hd;
+    bias_row[b] = BIAS ? db.tab + (long long)(kvh * g + hg) * db.stride + (db.origin - lim[b]) : nullptr;
+  }
 
-  // what a thread stages of a step's G tiles: K, an octet of d of a row; V, eight rows of a column
+  // what a thread stages of its group's tile: K, an octet of d of a row; V, eight rows of a column
   unsigned k_off[NI], v_off[NI];
   int k_row[NI], v_row[NI], k_unit[NI], v_unit[NI];
   bool k_second[NI];  // the octet's second half lies within the row
 #pragma unroll
   for (int u = 0; u < NI; ++u) {
-    const int idx = threadIdx.x + NTHREADS * u;
-    const int oct = idx % (HD / 8), r = idx / (HD / 8);
+    const int idx = (G == 2 || kOneOfTwo ? threadIdx.x & 255 : threadIdx.x) + 256 * u;
+    const int pair = HD == 128 ? idx >> 5 : idx >> 4;  // (of keys eight apart)
+    const int oct = (idx & 7) | (HD == 128 ? idx >> 1 & 8 : 0), r = (idx & 8) | (pair & 7) | (pair & 8) << 1;
     k_row[u] = r;
     k_off[u] = PAD && 8 * oct >= hd ? 0u : 32u * oct;
     k_second[u] = !PAD || 8 * oct + 4 < hd;
-    k_unit[u] = (r >> 5) * U::kTile + oct * U::kOctK + (r & 31);
-    const int d = idx % HD, group = idx / HD & 3, ts = idx / (4 * HD);
-    v_row[u] = 32 * ts + 16 * (group >> 1) + 4 * (group & 1);
+    k_unit[u] = (G == 2 ? gidx * U::kTile : 0) + U::key_unit(oct, r);
+    const int d = idx % HD, group = idx / HD;
+    v_row[u] = 4 * group;
     v_off[u] = PAD && d >= vhd ? 0u : 4u * d;
-    v_unit[u] = ts * U::kTile + U::kK + group * U::kGroupV + d % NT * 36 + d / NT;
+    v_unit[u] = (G == 2 ? gidx * U::kTile : 0) + U::kK + group * U::kGroupV + d % NT * U::kBlockV + d / NT;
   }
   const unsigned k_stride = (unsigned)hd * 4, v_stride = (unsigned)vhd * 4;
   f32x4 stage_k[NI][2];
@@ -181,7 +219,8 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   // a scalar base and a 32-bit byte offset per lane (a head's rows span less than 4 GiB: checked
   // at launch); rows past the last one repeat it
   auto load_k = [&](int sp) {
-    const int first = (kt0 + G * sp) * 32;
+    if (kOneOfTwo && gidx) return;
+    const int first = (kt0 + G * sp + first_tile) * 32;
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       const char *p = (const char *)kbase + ((unsigned)min(first + k_row[u], L - 1) * k_stride + k_off[u]);
@@ -190,14 +229,15 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     }
   };
   auto load_v = [&](int sp) {
-    const int first = (kt0 + G * sp) * 32;
-    if (first + 32 * G <= L) {
+    if (kOneOfTwo && !gidx) return;
+    const int first = (kt0 + G * sp + first_tile) * 32;
+    if (first + 32 <= L) {
       const char *base = (const char *)vbase + (unsigned long long)first * v_stride;
 #pragma unroll
       for (int u = 0; u < NI; ++u) {
         const unsigned off = (unsigned)v_row[u] * v_stride + v_off[u];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) stage_v[u][i] = *(const float *)(base + (unsigned long long)((i & 3) + 8 * (i >> 2)) * v_stride + off);
+        for (int i = 0; i < 8; ++i) stage_v[u][i] = *(const float *)(base + (unsigned long long)((i & 3) + 16 * (i >> 2)) * v_stride + off);
       }
     } else {
 #pragma unroll
@@ -205,195 +245,287 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           stage_v[u][i] = *(const float *)((const char *)vbase +
-                                           ((unsigned)min(first + v_row[u] + (i & 3) + 8 * (i >> 2), L - 1) * v_stride + v_off[u]));
+                                           ((unsigned)min(first + v_row[u] + (i & 3) + 16 * (i >> 2), L - 1) * v_stride + v_off[u]));
     }
   };
-  auto park_k = [&]() {
+  auto park_k = [&](int sp) {
+    if (kOneOfTwo && gidx) return;
+    u32x4 *const to = lds + (G == 1 && sp & 1 ? U::kTile : 0);
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       u32x4 h, m, l;
       split_octet(stage_k[u][0], stage_k[u][1], h, m, l);
-      lds[k_unit[u]] = h;
-      lds[k_unit[u] + U::kPartK] = m;
-      lds[k_unit[u] + 2 * U::kPartK] = l;
+      to[k_unit[u]] = h;
+      to[k_unit[u] + U::kPartK] = m;
+      to[k_unit[u] + 2 * U::kPartK] = l;
     }
   };
-  auto park_v = [&]() {
+  auto park_v = [&](int sp) {
+    if (kOneOfTwo && !gidx) return;
+    u32x4 *const to = lds + (G == 1 && sp & 1 ? U::kTile : 0);
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       u32x4 h, m, l;
       split_octet(f32x4{stage_v[u][0], stage_v[u][1], stage_v[u][2], stage_v[u][3]},
                   f32x4{stage_v[u][4], stage_v[u][5], stage_v[u][6], stage_v[u][7]}, h, m, l);
-      lds[v_unit[u]] = h;
-      lds[v_unit[u] + U::kPartV] = m;
-      lds[v_unit[u] + 2 * U::kPartV] = l;
+      to[v_unit[u]] = h;
+      to[v_unit[u] + U::kPartV] = m;
+      to[v_unit[u] + 2 * U::kPartV] = l;
     }
   };
 
-  // steps of G tiles, one per group of wavefronts; below "tile sp" is this group's tile of step sp
+  // steps of a tile, or (G = 2) of one per group; below "tile sp" is a group's tile of step sp (in the last step the second group
+  // may have none left: it stages its last rows again)
   const int n_sp = kt0 < kt1 ? (kt1 - kt0 + G - 1) / G : 0;
   if (n_sp > 0) {
     load_k(0);
     load_v(0);
   }
   // the row's query, scaled by scale * log2(e): scores come out in log2 units
-  u32x4 qf[KS][3];
+  u32x4 qf[KS][2][3];
+  u32x4 *const third = lds + 2 * U::kTile + (G == 2 ? wave : 4 * gidx + wave) * (kThirds<HD, G> * 128) + lane;
   bool apart;  // some query of the wavefront needs its scores in fp32
   {
-    f32x4 t[KS][2];
-    const float *qp = q_rot + q_off + 8 * j;
-#pragma unroll
-    for (int i = 0; i < KS; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        // (lanes past the last virtual row repeat the last row: their results are never used)
-        t[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (!PAD || 16 * i + 8 * j + 4 * h < hd) t[i][h] = *(const f32x4 *)(qp + 16 * i + 4 * h);
-      }
-#pragma unroll
-    for (int i = 0; i < KS; ++i) split_octet(t[i][0] * c, t[i][1] * c, qf[i][0], qf[i][1], qf[i][2]);
     float least = INFINITY, most = 0.f;
 #pragma unroll
-    for (int i = 0; i < KS; ++i)
+    for (int b = 0; b < 2; ++b) {
+      f32x4 t[KS][2];
+      const float *qp = q_rot + q_off[b] + 8 * j;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (PAD && 16 * i + 8 * j + 4 * h >= hd) continue;
+      for (int i = 0; i < KS; ++i)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float size = fabsf(t[i][h][w] * c);
-          least = fminf(least, size);
-          most = fmaxf(most, size);
+        for (int h = 0; h < 2; ++h) {
+          // (lanes past the last virtual row repeat the last row: their results are never used)
+          t[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (!PAD || 32 * i + 8 * j + 4 * h < hd) t[i][h] = *(const f32x4 *)(qp + 32 * i + 4 * h);
+        }
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        split_octet(t[i][0] * c, t[i][1] * c, qf[i][b][0], qf[i][b][1], qf[i][b][2]);
+        if (i < kThirds<HD, G> && (G == 1 || gidx == 0)) third[(2 * i + b) * 64] = qf[i][b][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (PAD && 32 * i + 8 * j + 4 * h >= hd) continue;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const float size = fabsf(t[i][h][w] * c);
+            least = fminf(least, size);
+            most = fmaxf(most, size);
+          }
         }
       }
+    }
     apart = false;
     // (looked at closely only where there is a zero or something out of the ordinary)
     if (__builtin_expect(__any(!(least >= 0x1p-109f) || !(most < 0x1p100f)), 0)) {
       QueryRange range;
 #pragma clang loop unroll(disable)
-      for (int d = 4 * j; d < hd; d += 8) range.add(*(const f32x4 *)(q_rot + q_off + d));
+      for (int d = 4 * j; d < hd; d += 16) {
+        range.add(*(const f32x4 *)(q_rot + q_off[0] + d));
+        range.add(*(const f32x4 *)(q_rot + q_off[1] + d));
+      }
       apart = __any(range.apart(c));
     }
   }
 
   // Online softmax against a reference value per virtual row instead of the running maximum: m_ref is only moved
   // (and l, O rescaled) when a score exceeds it by more than kTau, or for a row's first visible key;
-  // probabilities are then at most 2^kTau, no overflow.  A tile on the common path costs a maximum, 16
-  // subtractions, exp2 and adds per lane.
+  // probabilities are then at most 2^kTau, no overflow.  The sums of the scores begin at -m_ref.  A tile on the common path costs a
+  // maximum, 16 exp2 and adds per lane.
   constexpr float kTau = 8.f;
-  float m_ref = 0.f, l = 0.f;
-  float thr = -INFINITY;  // a row's scores move m_ref when above this: anything finite until its first key, m_ref + kTau after
-  f32x16 o[NT];
+  float m_ref[2] = {0.f, 0.f}, l[2] = {0.f, 0.f};
+  float thr[2] = {-INFINITY, -INFINITY};  // scores less m_ref move it when above this: anything finite until the row's first key, kTau after
+  f32x4 o[NT][2];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
-
-  // One stage of LDS for K and one for V.  Step sp: scores and softmax of tile sp from K(sp), V(sp) is parked
-  // meanwhile; a barrier; O^T += V^T(sp) P^T(sp), K(sp + 1) is parked meanwhile; a barrier.  What is parked was
-  // requested a step before.
-  const u32x4 *tile = lds + gidx * U::kTile;
-  if (n_sp > 0) {
-    park_k();
-    if (n_sp > 1) load_k(1);
-  }
-  __syncthreads();
-  for (int sp = 0; sp < n_sp; ++sp) {
-    const int kt = kt0 + G * sp + gidx;  // this group's tile
-    const bool have = kt < kt1 && kt * 32 <= wave_hi;
+    for (int b = 0; b < 2; ++b) o[t][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // A step of a group has two halves: MFMAs (O^T += V^T(sp - 1) P^T(sp - 1), scores of tile sp) and everything else (softmax of tile sp, P
+  // split, V(sp) and K(sp + 1) parked, the next requested), a barrier behind each.  The second group is half a step behind: while a SIMD's
+  // one wavefront has MFMAs only, its other one has none.  G = 2: each group stages its own tiles, one of K and one of V.  G = 1: both stage
+  // half of each, into two stages in turn; the second group does so a step ahead, for the first needs them half a step later.
+  // (heads of 128, G = 2, have no registers for a tile of K during the MFMAs: it is requested and parked within the other half)
+  constexpr bool kLate = HD == 128 && G == 2;
+  const int k_at[2] = {U::key_unit(j, n) + (G == 2 ? gidx * U::kTile : 0), (U::key_unit(j, n) ^ 4) + (G == 2 ? gidx * U::kTile : 0)}, v_at = U::kK + j * U::kGroupV + n + (G == 2 ? gidx * U::kTile : 0);
+  // tiles that some row of the wavefront sees
+  const int n_mine = max(0, (min(kt1, wave_hi / 32 + 1) - kt0 - first_tile + G - 1) / G) * (wave_hi >= 0);
+  auto stage_v_tile = [&](int sp) {
+    park_v(sp);
+    if constexpr (!kLate)
+      load_v(sp + 1);
+    else if (sp + 1 < n_sp)
+      load_k(sp + 1);
+  };
+  auto stage_k_tile = [&](int sp) {
+    if (sp + 1 < n_sp) {
+      park_k(sp + 1);
+      if constexpr (kLate) load_v(sp + 1);
+    }
+    if (!kLate) load_k(sp + 2);
+  };
+  f32x4 p[2][2];   // [virtual rows][keys]: scores, then probabilities
+  u32x4 pf[2][3];  // their parts
+  f32x4 near_bias[BIAS ? 2 : 1][2];
+  bool near = false;
+  auto scores = [&](int sp) {
+    const int kt = kt0 + G * sp + first_tile;
+    auto key = [&](int k, int w) { return lds[k_at[k / 2 & 1] + (G == 1 && sp & 1 ? U::kTile : 0) + w * U::kPartK + k / 2 * 128 + k % 2 * 16]; };
     // the tile's values by distance are asked for in front of its MFMAs; a tile that lies
     // `reach` or more behind all rows of the wavefront has none
-    f32x4 near_bias[BIAS ? 4 : 1];
-    const bool near = BIAS && have && wave_lo - (kt * 32 + 31) < db.reach;
     if constexpr (BIAS) {
+      near = wave_lo - (kt * 32 + 31) < db.reach;
       if (near) {
         struct __attribute__((packed, aligned(4))) Four { f32x4 v; };
 #pragma unroll
-        for (int r = 0; r < 4; ++r) near_bias[r] = ((const Four *)(bias_row + kt * 32 + 8 * r + 4 * j))->v;
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int a = 0; a < 2; ++a) near_bias[b][a] = ((const Four *)(bias_row[b] + kt * 32 + 16 * a + 4 * j))->v;
       }
     }
-    f32x16 p;
-    if (have) {
-      // S^T of the key tile: 32 keys x 32 virtual rows
+    // S^T of the key tile: 32 keys x 32 virtual rows; fragments arrive a block ahead of the MFMAs that take them
+    u32x4 fr[2][3], qt[2];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = 0.f;
-      const u32x4 *kl = tile + j * U::kOctK + n;
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int i = 0; i < KS; ++i) {
-        u32x4 kf[3];
+      for (int b = 0; b < 2; ++b) p[b][a] = f32x4{-m_ref[b], -m_ref[b], -m_ref[b], -m_ref[b]};
 #pragma unroll
-        for (int w = 0; w < 3; ++w) kf[w] = kl[w * U::kPartK + 2 * i * U::kOctK];
+    for (int w = 0; w < 3; ++w) fr[0][w] = key(0, w);
 #pragma unroll
-        for (int w = 0; w < 6; ++w) p = mfma_bf16(kf[kPartA[w]], qf[i][kPartB[w]], p);
+    for (int k = 0; k < 2 * KS; ++k) {
+      const int i = k / 2, a = k % 2;
+      if (i < kThirds<HD, G> && a == 0) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) qt[b] = third[(2 * i + b) * 64];
+      }
+      if (k + 1 < 2 * KS) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w) fr[k + 1 & 1][w] = key(k + 1, w);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int w = 0; w < 6; ++w)
+          p[b][a] = mfma_bf16_16(fr[k & 1][kPartA[w]], kPartB[w] == 2 && i < kThirds<HD, G> ? qt[b] : qf[i][b][kPartB[w]], p[b][a]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto softmax = [&](int sp) {
+    const int kt = kt0 + G * sp + first_tile;
+    if constexpr (BIAS) {
+      if (near) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int a = 0; a < 2; ++a) p[b][a] += near_bias[b][a];
       }
     }
-    park_v();
-    if (sp + 1 < n_sp) load_v(sp + 1);
-    if (have) {
-      if constexpr (BIAS) {
-        if (near) {
+    if (kt * 32 + 31 > wave_lo) {  // tile crosses the diagonal for some row of this wavefront
 #pragma unroll
-          for (int r = 0; r < 16; ++r) p[r] += near_bias[r >> 2][r & 3];
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (kt * 32 + 16 * a + 4 * j + r > lim[b]) p[b][a][r] = -INFINITY;
+    }
+    float mx[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+      mx[b] = fmaxf(fmaxf(fmaxf(fmaxf(p[b][0][0], p[b][0][1]), p[b][0][2]), fmaxf(fmaxf(p[b][0][3], p[b][1][0]), p[b][1][1])),
+                    fmaxf(p[b][1][2], p[b][1][3]));
+    // mx covers this lane's quarter of the row's keys in the tile; the row's maximum is above thr
+    // exactly when one of the four quarters' is (never for a row without a visible key here:
+    // -inf), so the quarters only exchange their maxima once a move is certain
+    if (__builtin_amdgcn_ballot_w64(mx[0] > thr[0] || mx[1] > thr[1]) != 0) {
+      // rare after a row's first tiles: move the reference to this tile's maximum
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        mx[b] = fmaxf(mx[b], __shfl_xor(mx[b], 16));
+        mx[b] = fmaxf(mx[b], __shfl_xor(mx[b], 32));
+        if (mx[b] > thr[b]) {
+          const float moved = m_ref[b] + mx[b], by = moved - m_ref[b];
+          const float alpha = thr[b] != -INFINITY ? fast_exp2(-by) : 1.f;  // nothing to rescale before a row's first key
+          m_ref[b] = moved;
+          thr[b] = kTau;
+          p[b][0] -= by;
+          p[b][1] -= by;
+          l[b] *= alpha;
+#pragma unroll
+          for (int t = 0; t < NT; ++t) o[t][b] *= alpha;
         }
       }
-      if (kt * 32 + 31 > wave_lo) {  // tile crosses the diagonal for some row of this wavefront
+    }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kt * 32 + 8 * (r >> 2) + 4 * j + (r & 3);
-          if (key > lim) p[r] = -INFINITY;
-        }
-      }
-      float mx = fmaxf(fmaxf(p[0], p[1]), p[2]);
-#pragma unroll
-      for (int r = 3; r < 15; r += 2) mx = fmaxf(fmaxf(mx, p[r]), p[r + 1]);
-      mx = fmaxf(mx, p[15]);
-      // mx covers this lane's half of the row's keys in the tile; the row's maximum is above thr
-      // exactly when one of the two halves' is (never for a row without a visible key here:
-      // -inf), so the halves only exchange their maxima once a move is certain
-      if (__builtin_amdgcn_ballot_w64(mx > thr) != 0) {
-        // rare after a row's first tiles: move the reference to this tile's maximum
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (mx > thr) {
-          const float alpha = thr != -INFINITY ? fast_exp2(m_ref - mx) : 1.f;  // nothing to rescale before a row's first key
-          m_ref = mx;
-          thr = mx + kTau;
-          l *= alpha;
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
-        }
-      }
+    for (int b = 0; b < 2; ++b) {
       float psum = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p[r] = fast_exp2(p[r] - m_ref);
-        psum += p[r];
-      }
-      l += psum;
-    }
-    __syncthreads();  // V(sp) is there, nobody reads K(sp) any more
-    if (have) {
-      // O^T += V^T P^T; the probabilities are where the scores were
-      const u32x4 *vl = tile + U::kK + j * U::kGroupV + n;
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        u32x4 pf[3];
-        split_octet(f32x4{p[8 * u], p[8 * u + 1], p[8 * u + 2], p[8 * u + 3]},
-                    f32x4{p[8 * u + 4], p[8 * u + 5], p[8 * u + 6], p[8 * u + 7]}, pf[0], pf[1], pf[2]);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          u32x4 vf[3];
-#pragma unroll
-          for (int w = 0; w < 3; ++w) vf[w] = vl[w * U::kPartV + 2 * u * U::kGroupV + 36 * t];
-#pragma unroll
-          for (int w = 0; w < 6; ++w) o[t] = mfma_bf16(vf[kPartA[w]], pf[kPartB[w]], o[t]);
+        for (int r = 0; r < 4; ++r) {
+          p[b][a][r] = fast_exp2(p[b][a][r]);
+          psum += p[b][a][r];
         }
-      }
+      l[b] += psum;
+      split_octet(p[b][0], p[b][1], pf[b][0], pf[b][1], pf[b][2]);
     }
-    if (sp + 1 < n_sp) park_k();
-    if (sp + 2 < n_sp) load_k(sp + 2);
-    __syncthreads();  // K(sp + 1) is there, nobody reads V(sp) any more
+  };
+  auto outputs = [&](int sp) {  // O^T += V^T P^T
+    const u32x4 *const vl = lds + v_at + (G == 1 && sp & 1 ? U::kTile : 0);
+    u32x4 fr[2][3];
+#pragma unroll
+    for (int w = 0; w < 3; ++w) fr[0][w] = vl[w * U::kPartV];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (t + 1 < NT) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w) fr[t + 1 & 1][w] = vl[w * U::kPartV + (t + 1) * U::kBlockV];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int w = 0; w < 6; ++w) o[t][b] = mfma_bf16_16(fr[t & 1][kPartA[w]], pf[b][kPartB[w]], o[t][b]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (n_sp > 0) {
+    park_k(0);
+    if (!kLate) load_k(1);
   }
+  __syncthreads();
+  if (gidx == 1) {
+    if (G == 1 && n_sp > 0) {
+      stage_v_tile(0);
+      stage_k_tile(0);
+    }
+    __syncthreads();
+  }
+  const int ahead = G == 1 ? gidx : 0;
+  // (what is requested and parked behind the last tile is nobody's: its rows are the last one again, its stage is free)
+  int sp = 0;
+  for (; sp < n_mine; ++sp) {
+    if constexpr (HD == 128) __builtin_amdgcn_s_setprio(1);
+    scores(sp);
+    if constexpr (HD == 128) __builtin_amdgcn_s_setprio(0);
+    __syncthreads();  // nobody of the group reads V(sp - 1) and K(sp) any more
+    if constexpr (HD == 128) __builtin_amdgcn_sched_barrier(0);  // (V is split in this half; heads of 64 have fewer MFMAs than this half has work)
+    stage_v_tile(sp + ahead);
+    softmax(sp);
+    if constexpr (kLate) __builtin_amdgcn_sched_barrier(0);  // (K is on its way meanwhile)
+    stage_k_tile(sp + ahead);
+    __syncthreads();  // V(sp) and K(sp + 1) are there
+    if constexpr (HD == 128) __builtin_amdgcn_s_setprio(1);
+    outputs(sp);
+  }
+  if constexpr (HD == 128) __builtin_amdgcn_s_setprio(0);
+  for (; sp < n_sp; ++sp) {  // tiles that only others see
+    __syncthreads();
+    if (sp + ahead < n_sp) stage_v_tile(sp + ahead);
+    if (sp + ahead + 1 < n_sp) stage_k_tile(sp + ahead);
+    __syncthreads();
+  }
+  if (gidx == 0) __syncthreads();
 
   // Some results are taken again, tile by tile in fp32:
   //   results that are not finite come from operands that are not, and fp32 says which (8192 rows, 32 / 8 heads of 64, NaN
@@ -406,22 +538,22 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   // way 1320) and 2048 rows of 32 / 8 heads of 128 4 % (216 -> 224; 218).
   {
     auto size = [](float x) { return __builtin_bit_cast(unsigned, x) << 1; };  // (in the order of |x|)
-    float probe = l * 0.f, least = INFINITY;
+    float probe = l[0] * 0.f + l[1] * 0.f, least = INFINITY;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        probe = fmaf(o[t][r], 0.f, probe);
-        least = fminf(least, fabsf(o[t][r]));
+      for (int r = 0; r < 8; ++r) {
+        probe = fmaf(o[t][r >> 2][r & 3], 0.f, probe);
+        least = fminf(least, fabsf(o[t][r >> 2][r & 3]));
       }
     bool again = apart || __any(probe != 0.f);
     float up = 1.f, down = 1.f;
-    if (__builtin_expect(__any(least < 0x1p-80f && thr != -INFINITY), 0) && !again) {
+    if (__builtin_expect(__any(least < 0x1p-80f && (thr[0] != -INFINITY || thr[1] != -INFINITY)), 0) && !again) {
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));
       unsigned small = ~0u;  // (zeros lie above all)
 #pragma clang loop unroll(disable)
-      for (int kt = kt0 + gidx; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
+      for (int kt = kt0 + first_tile; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
         const float *vr = vbase + (long long)min(kt * 32 + (tid & 31), wave_hi) * vhd;
 #pragma clang loop unroll_count(4)
         for (int d = (tid & 32) >> 3; d < vhd; d += 8) {
@@ -437,102 +569,129 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       // (what a lane works on is found again from its number: kept for here it would cost the loop above registers)
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));
-      const int n = tid & 31, j = (tid & 63) >> 5, my_v = min(v0 + n, VR - 1), row = my_v / g, hg = my_v - row * g, lim = S + row;
-      const long long q_at = BIAS ? (st.tok_off[s] + row) * db.q_stride + (long long)(kvh * g + hg) * hd
-                                  : ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * hd;
-      const float *bias_row = BIAS ? db.tab + (long long)(kvh * g + hg) * db.stride + (db.origin - lim) : nullptr;
-      m_ref = 0.f, l = 0.f, thr = -INFINITY;
-      f32x16 sum[NT];
+      const int n = tid & 15, j = (tid & 63) >> 4;
+      int lim[2];
+      const float *bias_row[2], *qr[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int my_v = min(v0 + 16 * b + n, VR - 1), row = my_v / g, hg = my_v - row * g;
+        lim[b] = S + row;
+        qr[b] = q_rot + 4 * j + (BIAS ? (st.tok_off[s] + row) * db.q_stride + (long long)(kvh * g + hg) * hd
+                                      : ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * hd);
+        bias_row[b] = BIAS ? db.tab + (long long)(kvh * g + hg) * db.stride + (db.origin - lim[b]) : nullptr;
+        m_ref[b] = 0.f, l[b] = 0.f, thr[b] = -INFINITY;
+      }
+      f32x4 sum[NT][2];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sum[t][r] = 0.f;
-      // Tile by tile: scores from the fp32 instruction, lane half j with d = 8 i + 4 j .. + 3 of step i, here against
+        for (int b = 0; b < 2; ++b) sum[t][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // Tile by tile: scores from the fp32 instruction, lane quarter j with d = 16 i + 4 j .. + 3 of step i, here against
       // the running maximum; the products with V likewise where every row sees the whole tile, else key by key
       // (what a row does not see it does not multiply by zero either).
 #pragma clang loop unroll(disable)
-      for (int kt = kt0 + gidx; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
+      for (int kt = kt0 + first_tile; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
         const int first = kt * 32;
         const bool whole = first + 31 <= wave_lo;
-        const float *kr = kbase + (long long)min(first + n, L - 1) * hd + 4 * j, *qr = q_rot + q_at + 4 * j;
-        f32x16 p;
+        const float *kr[2] = {kbase + (long long)min(first + n, L - 1) * hd + 4 * j, kbase + (long long)min(first + 16 + n, L - 1) * hd + 4 * j};
+        float p[2][8];  // [virtual rows][16 (i / 4) + 4 j + i % 4 of the keys]
+        {
+          f32x4 sc[2][2];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) p[r] = 0.f;
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) sc[b][a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma clang loop unroll(disable)
-        for (int d0 = 0; d0 < hd; d0 += 16) {
-          f32x4 kv[2], qv[2];
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int d = d0 + 8 * u;
+          for (int d = 0; d < hd; d += 16) {
             const bool in = !PAD || d + 4 * j < hd;
-            kv[u] = in ? *(const f32x4 *)(kr + d) : f32x4{0.f, 0.f, 0.f, 0.f};
-            qv[u] = in ? *(const f32x4 *)(qr + d) * c : f32x4{0.f, 0.f, 0.f, 0.f};
+            f32x4 kv[2], qv[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+              kv[a] = in ? *(const f32x4 *)(kr[a] + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+              qv[a] = in ? *(const f32x4 *)(qr[a] + d) * c : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+              for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[b][a] = mfma_f32_16(kv[a][i], qv[b][i], sc[b][a]);
           }
 #pragma unroll
-          for (int i = 0; i < 8; ++i) p = mfma_f32(kv[i >> 2][i & 3], qv[i >> 2][i & 3], p);
-        }
-        if (BIAS && wave_lo - (first + 31) < db.reach) {
+          for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = first + 8 * (r >> 2) + 4 * j + (r & 3);
-            if (key <= lim && lim - key < db.reach) p[r] += bias_row[key];
+            for (int i = 0; i < 8; ++i) p[b][i] = sc[b][i >> 2][i & 3];
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          if (BIAS && wave_lo - (first + 31) < db.reach) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const int key = first + 16 * (i >> 2) + 4 * j + (i & 3);
+              if (key <= lim[b] && lim[b] - key < db.reach) p[b][i] += bias_row[b][key];
+            }
           }
-        }
-        float mx = -INFINITY;
+          float mx = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          if (!whole && first + 8 * (r >> 2) + 4 * j + (r & 3) > lim) p[r] = -INFINITY;
-          mx = fmaxf(mx, p[r]);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (mx > thr) {
-          const float alpha = thr == -INFINITY ? 0.f : fast_exp2(thr - mx);
-          m_ref = thr = mx;
-          l *= alpha;
+          for (int i = 0; i < 8; ++i) {
+            if (!whole && first + 16 * (i >> 2) + 4 * j + (i & 3) > lim[b]) p[b][i] = -INFINITY;
+            mx = fmaxf(mx, p[b][i]);
+          }
+          mx = fmaxf(mx, __shfl_xor(mx, 16));
+          mx = fmaxf(mx, __shfl_xor(mx, 32));
+          if (mx > thr[b]) {
+            const float alpha = thr[b] == -INFINITY ? 0.f : fast_exp2(thr[b] - mx);
+            m_ref[b] = thr[b] = mx;
+            l[b] *= alpha;
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < NT; ++t) sum[t][b] *= alpha;
+          }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sum[t][r] *= alpha;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          p[r] = fast_exp2(p[r] - m_ref);
-          l += p[r];
+          for (int i = 0; i < 8; ++i) {
+            p[b][i] = fast_exp2(p[b][i] - m_ref[b]);
+            l[b] += p[b][i];
+          }
         }
         if (whole) {
-          typedef float vrow_t __attribute__((ext_vector_type(NT)));
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = first + 8 * (r >> 2) + 4 * j + (r & 3);
-            const vrow_t v = *(const vrow_t *)(vbase + (long long)key * vhd + (PAD && NT * n >= vhd ? 0 : NT * n));
+          for (int i = 0; i < 8; ++i) {
+            const float *vr = vbase + (long long)(first + 16 * (i >> 2) + 4 * j + (i & 3)) * vhd;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) sum[t] = mfma_f32(v[t] * up, p[r], sum[t]);
+            for (int w = 0; w < NT / 4; ++w) {
+              const int d = NT * n + 4 * w;
+              const f32x4 v = *(const f32x4 *)(vr + (PAD && d >= vhd ? 0 : d)) * up;
+#pragma unroll
+              for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) sum[4 * w + t][b] = mfma_f32_16(v[t], p[b][i], sum[4 * w + t][b]);
+            }
           }
           continue;
         }
 #pragma clang loop unroll(disable)
-        for (int r = 0; r < 16; ++r) {
-          const float own = p[0], other = __shfl_xor(own, 32);
+        for (int i = 0; i < 8; ++i) {
+          const float own[2] = {p[0][0], p[1][0]};
 #pragma unroll
-          for (int i = 0; i < 15; ++i) p[i] = p[i + 1];  // (no register is indexed by a loop counter)
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int k = 0; k < 7; ++k) p[b][k] = p[b][k + 1];  // (no register is indexed by a loop counter)
 #pragma clang loop unroll(disable)
-          for (int h = 0; h < 2; ++h) {
-            const int key = first + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (key > lim) continue;
-            const float e = h == j ? own : other;
+          for (int h = 0; h < 4; ++h) {
+            const int key = first + 16 * (i >> 2) + 4 * h + (i & 3);
+            const float e[2] = {__shfl(own[0], n + 16 * h), __shfl(own[1], n + 16 * h)};
+            if (key > max(lim[0], lim[1])) continue;
             const float *vr = vbase + (long long)key * vhd;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int w = 0; w < NT; ++w) {  // floats 4 w .. 4 w + 3 of the 4 NT columns that a lane holds
+              const int d = NT * 4 * j + 4 * w;
+              const f32x4 v = *(const f32x4 *)(vr + (PAD && d >= vhd ? 0 : d)) * up;
 #pragma unroll
-              for (int w = 0; w < NT; ++w) {  // floats 4 w .. 4 w + 3 of the 4 NT columns that registers 4 q .. 4 q + 3 hold
-                const int d = NT * (8 * q + 4 * j) + 4 * w;
-                const f32x4 v = *(const f32x4 *)(vr + (PAD && d >= vhd ? 0 : d));
+              for (int b = 0; b < 2; ++b) {
+                if (key > lim[b]) continue;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  const int at = 4 * w + i;
-                  sum[at % NT][4 * q + at / NT] = fmaf(e, v[i] * up, sum[at % NT][4 * q + at / NT]);
-                }
+                for (int k = 0; k < 4; ++k) sum[(4 * w + k) % NT][b][(4 * w + k) / NT] = fmaf(e[b], v[k], sum[(4 * w + k) % NT][b][(4 * w + k) / NT]);
               }
+            }
           }
         }
       }
@@ -540,79 +699,86 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float x = sum[t][r] * down;
+        for (int r = 0; r < 8; ++r) {
+          float x = sum[t][r >> 2][r & 3] * down;
           asm volatile("" : "+v"(x));
-          o[t][r] = x;
+          o[t][r >> 2][r & 3] = x;
         }
     }
   }
 
-  l += __shfl_xor(l, 32);
+  // (what a lane works on is found again from its number: kept for here it would cost the loop above registers)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
   // what the merges below call the maximum: the reference the sums are relative to, in log2
   // units, or -inf for a row that saw no key (its l and O are 0)
-  float m = thr == -INFINITY ? -INFINITY : m_ref;
+  float m[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    l[b] += __shfl_xor(l[b], 16);
+    l[b] += __shfl_xor(l[b], 32);
+    m[b] = thr[b] == -INFINITY ? -INFINITY : m_ref[b];
+  }
   if constexpr (G == 2) {
+    const int lane = tid & 63;
     // the second group hands its (max, sum, O) to the first through the tile stages
-    // (every wavefront is past the last step's barrier: nobody reads tiles any more)
-    float *xo = (float *)lds;                   // [4 row chunks][16 * NT registers][64 lanes]
-    float *xm = (float *)lds + 4 * 16 * NT * 64;  // [4][64] max, then [4][64] sum
-    static_assert(sizeof lds >= (4 * 16 * NT * 64 + 512) * sizeof(float), "the merge fits the tiles");
+    f32x4 *xo = (f32x4 *)lds;                       // [4 row chunks][2 NT registers of four][64 lanes]
+    float *xm = (float *)lds + 4 * 8 * NT * 64;     // [4][2][64] max, then the same of sums
+    static_assert(sizeof lds >= (4 * 8 * NT * 64 + 1024) * sizeof(float), "the merge fits the tiles");
+    __syncthreads();  // nobody reads tiles any more
     if (gidx == 1) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int b = 0; b < 2; ++b) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) xo[((wave * NT + t) * 16 + r) * 64 + lane] = o[t][r];
-      xm[wave * 64 + lane] = m;
-      xm[256 + wave * 64 + lane] = l;
+        for (int t = 0; t < NT; ++t) xo[((wave * NT + t) * 2 + b) * 64 + lane] = o[t][b];
+        xm[(wave * 2 + b) * 64 + lane] = m[b];
+        xm[512 + (wave * 2 + b) * 64 + lane] = l[b];
+      }
     }
     __syncthreads();
     if (gidx == 1) return;
-    const float m1 = xm[wave * 64 + lane], l1 = xm[256 + wave * 64 + lane];
-    const float mnew = fmaxf(m, m1);
-    // a side that saw no visible key has max -inf: its factor is 0 (and both may be, in a key chunk)
-    const float a0 = m == -INFINITY ? 0.f : fast_exp2(m - mnew);
-    const float a1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mnew);
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int b = 0; b < 2; ++b) {
+      const float m1 = xm[(wave * 2 + b) * 64 + lane], l1 = xm[512 + (wave * 2 + b) * 64 + lane];
+      const float mnew = fmaxf(m[b], m1);
+      // a side that saw no visible key has max -inf: its factor is 0 (and both may be, in a key chunk)
+      const float a0 = m[b] == -INFINITY ? 0.f : fast_exp2(m[b] - mnew);
+      const float a1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mnew);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[t][r] = o[t][r] * a0 + xo[((wave * NT + t) * 16 + r) * 64 + lane] * a1;
-    l = l * a0 + l1 * a1;
-    m = mnew;
-  }
-  if (SPLIT) {  // unnormalised partial of this key chunk: [128 virtual rows][HD], (max, sum) per row
-    const long long pbase = (((long long)item * sh.KV + kvh) * ns + chunk) * 128 + wave * 32 + n;
-    float *op = part_o + pbase * HD;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = NT * (8 * (r >> 2) + 4 * j + (r & 3));
-      if constexpr (NT == 2) {
-        *(float2 *)(op + d) = float2{o[0][r], o[1][r]};
-      } else {
-        *(f32x4 *)(op + d) = f32x4{o[0][r], o[1][r], o[2][r], o[3][r]};
-      }
+      for (int t = 0; t < NT; ++t) o[t][b] = o[t][b] * a0 + xo[((wave * NT + t) * 2 + b) * 64 + lane] * a1;
+      l[b] = l[b] * a0 + l1 * a1;
+      m[b] = mnew;
     }
-    if (j == 0) *(float2 *)(part_ml + 2 * pbase) = float2{m, l};
-  } else if (valid) {
-    const float inv = 1.0f / l;
-    float *op = out + qo_off;
+  }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = NT * (8 * (r >> 2) + 4 * j + (r & 3));
-      if (PAD && d >= vhd) continue;  // (the width is a multiple of 4 and d of NT = 2 or 4: a store lies inside or outside as a whole)
-      if constexpr (NT == 2) {
-        *(float2 *)(op + d) = float2{o[0][r] * inv, o[1][r] * inv};
-      } else {
-        *(f32x4 *)(op + d) = f32x4{o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
-      }
+  for (int b = 0; b < 2; ++b) {
+    const int n = tid & 15, j = (tid & 63) >> 4, my_v = v0 + 16 * b + n;
+    if (my_v >= VR) continue;
+    if (SPLIT) {  // unnormalised partial of this key chunk: [128 virtual rows][HD], (max, sum) per row
+      const long long pbase = (((long long)(G == 1 ? uniform(block_rank(st, s, vb)) : item) * sh.KV + kvh) * ns + chunk) * 128 + wave * 32 + 16 * b + n;
+      float *op = part_o + pbase * HD + NT * 4 * j;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int w = 0; w < NT; w += 4) *(f32x4 *)(op + NT * r + w) = f32x4{o[w][b][r], o[w + 1][b][r], o[w + 2][b][r], o[w + 3][b][r]};
+      if (j == 0) *(float2 *)(part_ml + 2 * pbase) = float2{m[b], l[b]};
+    } else {
+      const int row = my_v / g, hg = my_v - row * g;
+      const float inv = 1.0f / l[b];
+      float *op = out + ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * vhd + NT * 4 * j;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int w = 0; w < NT; w += 4) {
+          if (PAD && NT * (4 * j + r) + w >= vhd) continue;  // (the width is a multiple of 4)
+          *(f32x4 *)(op + NT * r + w) = f32x4{o[w][b][r] * inv, o[w + 1][b][r] * inv, o[w + 2][b][r] * inv, o[w + 3][b][r] * inv};
+        }
     }
   }
 }
 
-// (three workgroups of four wavefronts on a compute unit where the registers allow: 8192 rows, 32 / 8 heads of 64,
-// 1377 -> 1324 us)
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS = false>
-__global__ __launch_bounds__(256 * G, G == 1 ? (HD == 64 && !PAD ? 3 : 2) : 1) void prefill_mfma_kernel(const float *__restrict__ q_rot,
+__global__ __launch_bounds__(512, 2) void prefill_mfma_kernel(const float *__restrict__ q_rot,
                                                               const float *__restrict__ kc,
                                                               const float *__restrict__ vc,
                                                               float *__restrict__ out,
@@ -628,7 +794,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? (HD == 64 && !PAD ? 3 : 2) : 1) v
 // every workgroup, instead of the dispatcher starting another workgroup where one has ended
 // (3.5 us later, measured).
 template <int HD, int G, bool PAD, bool BIAS = false>
-__global__ __launch_bounds__(256 * G, 1) void prefill_turns_kernel(const float *__restrict__ q_rot,
+__global__ __launch_bounds__(512, 2) void prefill_turns_kernel(const float *__restrict__ q_rot,
                                                                    const float *__restrict__ kc,
                                                                    const float *__restrict__ vc,
                                                                    float *__restrict__ out, SeqTable st, Shape sh,
@@ -865,13 +1031,11 @@ size_t prefill_partial_floats(const Shape &sh, int items, int ns, int v_hd) {
 PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_per_cu, int groups, int v_hd) {
   PrefillLaunch p;
   p.n_wgs = (long long)items * sh.KV * ns;
-  // With fewer workgroups than three per compute unit everything is resident at
-  // once: run one workgroup per compute unit (below) and give it eight wavefronts,
-  // two per SIMD (G = 2).  Larger launches already have several workgroups per unit.
+  // A launch of up to three row blocks a compute unit has each in a workgroup of its own, whose groups share its keys; in larger ones a workgroup takes
+  // two, whose groups share the tiles.
   p.groups = groups == 1 || groups == 2 ? groups : (p.n_wgs <= 768 ? 2 : 1);
-  // static LDS of the kernel: `groups` K tiles and V tiles
   const int tile_hd = prefill_tile_head_dim(widest(sh, v_hd));
-  const size_t static_lds = (size_t)16 * p.groups * (tile_hd == 64 ? TileUnits<64>::kTile : TileUnits<128>::kTile);
+  const size_t static_lds = (size_t)16 * (tile_hd == 64 ? kLdsUnits<64, 1> : p.groups == 2 ? kLdsUnits<128, 2> : kLdsUnits<128, 1>);
   p.pad = 0;
   // With fewer workgroups than three per compute unit everything is resident at
   // once and the dispatcher cannot balance the triangular work: one workgroup per
@@ -894,6 +1058,16 @@ PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_pe
   return p;
 }
 
+long long prefill_workgroups(const SeqTable &st, const Shape &sh, const PrefillLaunch &p, int items, int ns) {
+  if (p.turns) return (p.n_wgs + p.turns - 1) / p.turns;
+  int units = items;
+  if (p.groups == 1) {
+    units = 0;
+    for (int s = 0; s < st.n_seqs; ++s) units += (st.work_off[s] + 1) / 2;
+  }
+  return (long long)units * sh.KV * ns;
+}
+
 hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, float *out, float *partials,
                           const SeqTable &st, const Shape &sh, int items, int ns, float scale,
                           hipStream_t stream, int wgs_per_cu, int groups_wanted, hipEvent_t before, hipEvent_t after,
@@ -910,16 +1084,14 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
   // the kernels address a row of a (sequence, kv head) by a 32-bit byte offset from its first row
   if ((long long)sh.cap * sh.hd * 4 > 0xffffffffLL) return hipErrorInvalidValue;
   const float c = scale * kLog2e;
-  dim3 grid((unsigned)n_wgs);
+  dim3 grid((unsigned)prefill_workgroups(st, sh, plan, items, ns));
   float *part_o = partials;
   float *part_ml = partials ? partials + (size_t)items * sh.KV * ns * 128 * tile_hd : nullptr;
   const int groups = plan.groups;
   const size_t lds_pad = plan.pad;
   if (plan.turns) {
-    const int turns = plan.turns;
-    dim3 fewer((unsigned)((n_wgs + turns - 1) / turns));
 #define SHAINET_LAUNCH_TURNS(HD_, ...)                                                                          \
-  SHAINET_LAUNCH_TIMED((prefill_turns_kernel<HD_, 2, __VA_ARGS__>), fewer, dim3(512), 0, stream, before, after, q_rot, kc, \
+  SHAINET_LAUNCH_TIMED((prefill_turns_kernel<HD_, 2, __VA_ARGS__>), grid, dim3(512), 0, stream, before, after, q_rot, kc, \
                        vc, out, st, sh, (int)n_wgs, c, db)
     if (tile_hd == 64) {
       if (bias)
@@ -946,7 +1118,7 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
       SHAINET_LAUNCH_TIMED((prefill_mfma_kernel<HD_, SPLIT_, 2, __VA_ARGS__>), grid, dim3(512), lds_pad, stream, before, \
                            main_after, q_rot, kc, vc, out, part_o, part_ml, st, sh, ns, c, db);                     \
     else                                                                                                        \
-      SHAINET_LAUNCH_TIMED((prefill_mfma_kernel<HD_, SPLIT_, 1, __VA_ARGS__>), grid, dim3(256), lds_pad, stream, before, \
+      SHAINET_LAUNCH_TIMED((prefill_mfma_kernel<HD_, SPLIT_, 1, __VA_ARGS__>), grid, dim3(512), lds_pad, stream, before, \
                            main_after, q_rot, kc, vc, out, part_o, part_ml, st, sh, ns, c, db);                     \
   } while (0)
 #define SHAINET_LAUNCH_PREFILL_HD(HD_, ...)             \

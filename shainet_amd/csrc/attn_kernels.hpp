@@ -189,11 +189,13 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
 // Which instantiation a prefill launch uses and how it is laid out; launch_prefill follows it.
 struct PrefillLaunch {
   long long n_wgs;   // row blocks x kv heads x key chunks
-  int groups;        // 1: four wavefronts per workgroup; 2: eight
+  int groups;        // of wavefronts that share a row block's keys.  1: a workgroup takes two row blocks of a sequence, a group of wavefronts each
   int turns;         // 0: one workgroup per row block and chunk; 2 or 3: prefill_turns_kernel with that many blocks per workgroup
   int wgs_per_cu;    // 0: as the kernel's registers and LDS allow; 1..3: LDS padded to that occupancy
   size_t pad;        // bytes of dynamic LDS that enforce wgs_per_cu
 };
+// Workgroups of such a launch; st as plan_work left it.
+long long prefill_workgroups(const SeqTable &st, const Shape &sh, const PrefillLaunch &p, int items, int ns);
 PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_per_cu, int groups, int v_hd = 0);
 hipError_t launch_generic(const float *q_rot, const float *kc, const float *vc, float *out,
                           const SeqTable &st, const Shape &sh, int total_tokens, float scale,

@@ -1259,7 +1259,7 @@ int shainet_attn_describe_plan(int num_heads, int num_kv_heads, int head_dim, in
     plan[2] = ns;
     plan[3] = p.groups;
     plan[4] = p.turns;
-    plan[5] = (int)(p.turns ? (p.n_wgs + p.turns - 1) / p.turns : p.n_wgs);
+    plan[5] = (int)prefill_workgroups(st, sh, p, items, ns);
     plan[6] = items;
     plan[7] = p.wgs_per_cu;
   } else {

@@ -158,6 +158,8 @@ __device__ __forceinline__ f32x4 mfma_bf16_16(u32x4 a, u32x4 b, f32x4 acc) {
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
 }
+// ... and of 16 x 16 over four k: lane l holds k = l / 16 of row (column) l % 16; D as of mfma_bf16_16
+__device__ __forceinline__ f32x4 mfma_f32_16(float a, float b, f32x4 acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
 
 // *base (the same in all lanes) plus a lane's own offset in bytes: one load with a scalar base.  (Of addresses that differ
 // by scalars only the compiler makes 64-bit sums per thread, two instructions each.)
