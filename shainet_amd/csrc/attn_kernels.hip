@@ -1010,18 +1010,30 @@ int prefill_key_splits(const SeqTable &st, const Shape &sh, int items) {
     const int t = (st.start_pos[s] + st.n_new[s] + 31) / 32;
     longest = t > longest ? t : longest;
   }
-  int ns = (int)((512 + wgs - 1) / wgs);
-  // With long key ranges, about 1024 workgroups: four-wavefront workgroups that share the
-  // compute units two or more at a time and drift apart then do better than 512 of eight
-  // wavefronts, one per unit, whose two wavefronts per SIMD move in step (512 rows on 16384
-  // cached, 128 row blocks: 1078 -> 1053 us); chunks under 32 tiles lose more to their set-up
-  // (1024 rows into an empty cache: 109 -> 115 us).
+  // With long key ranges, about 1024 row blocks and chunks: two blocks share a workgroup and its tiles then.
   const int ns_1024 = (int)((1024 + wgs - 1) / wgs);
-  if (longest / ns_1024 >= 32) ns = ns_1024;
+  if (longest / ns_1024 >= 32) return ns_1024 < 16 ? ns_1024 : 16;
+  // Otherwise what is estimated to end first, in times of a key tile: a compute unit has one workgroup at a time, which costs five tiles beside
+  // its own, and the launch that merges costs four more and one for each chunk.  Us, chunks by a target of 512 workgroups | these: 32 / 8 heads of 64, 800 rows 49 | 41, 200 on
+  // 2000 46 | 37, 400 on 4000 113 | 89; heads of 128, 800 rows 86 | 73, 32 / 4 heads, 512 on 4096 214 | 188; heads of 96, 777 rows 70 | 59.
+  double blocks = 0, tiles = 0;
+  for (int s = 0; s < st.n_seqs; ++s) {
+    const double n = (st.n_new[s] * (double)sh.g + 127) / 128;
+    blocks += n;
+    tiles += n * ((st.start_pos[s] + st.n_new[s] * 0.5) / 32 + 1);
+  }
   const int cap = longest / 8;  // at least eight key tiles per chunk
-  if (ns > cap) ns = cap;
-  if (ns > 16) ns = 16;
-  return ns < 1 ? 1 : ns;
+  int best = 1;
+  double least = 0;
+  for (int ns = 1; ns == 1 || (ns <= cap && ns <= 16); ++ns) {
+    const double rounds = (double)((wgs * ns + 255) / 256), one = (longest + ns - 1) / ns + 5, all = rounds * (tiles / blocks / ns + 5);
+    const double ends = (one > all ? one : all) + (ns > 1 ? 4 + ns : 0);
+    if (ns == 1 || ends < least) {
+      least = ends;
+      best = ns;
+    }
+  }
+  return best;
 }
 
 size_t prefill_partial_floats(const Shape &sh, int items, int ns, int v_hd) {
