@@ -114,8 +114,7 @@ struct TileUnits {
 // 16384 366 | 304; 512 rows on 16384, 32 / 4 heads of 128, 690 | 551, 2048 rows, 32 / 8 heads of 128, 221 | 199, 4096 rows 743 | 596; 2048 rows of 32 heads of 96
 // 214 | 178.  Errors against 64 bits 0 to 13 % smaller.
 // What each part of it gave: half a step apart 104 | 100 and fragments a block ahead of their MFMAs 98; the layout of LDS without conflicts 96 | 92.6; a block's
-// products on one accumulator rather than two in turn 1 %; the reference value of the softmax as where the scores' sums begin 1 to 2.6 %; two row blocks a
-// workgroup and the queries' third parts in LDS, which ended spills, 656 | 568 (512 rows on 16384, heads of 128).  In step
+// products on one accumulator rather than two in turn 1 %; two row blocks a workgroup and the queries' third parts in LDS, which ended spills, 656 | 568 (512 rows on 16384, heads of 128).  In step
 // again (no group waits half a step at the start) short ranges take 2 to 10 % longer.
 // What bounds it: heads of 128 the power the card may draw (matrix cores busy 78 % at 1.9 GHz); heads of 64 vector instructions: 281 and 16
 // exponentials a tile and wavefront, of which a SIMD issues two during an MFMA of 16 cycles.  (Queries and keys as two fp16 numbers and scores of three products
@@ -330,11 +329,12 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 
   // Online softmax against a reference value per virtual row instead of the running maximum: m_ref is only moved
   // (and l, O rescaled) when a score exceeds it by more than kTau, or for a row's first visible key;
-  // probabilities are then at most 2^kTau, no overflow.  The sums of the scores begin at -m_ref.  A tile on the common path costs a
-  // maximum, 16 exp2 and adds per lane.
+  // probabilities are then at most 2^kTau, no overflow.  A tile on the common path costs a maximum, 16
+  // subtractions, exp2 and adds per lane.  (Sums of scores that begin at -m_ref save the subtractions, 1 to 2.6 %, but round more often where a
+  // score is small beside m_ref: errors against 64 bits grew by 3 to 16 %.)
   constexpr float kTau = 8.f;
   float m_ref[2] = {0.f, 0.f}, l[2] = {0.f, 0.f};
-  float thr[2] = {-INFINITY, -INFINITY};  // scores less m_ref move it when above this: anything finite until the row's first key, kTau after
+  float thr[2] = {-INFINITY, -INFINITY};  // a row's scores move m_ref when above this: anything finite until its first key, m_ref + kTau after
   f32x4 o[NT][2];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -387,7 +387,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) p[b][a] = f32x4{-m_ref[b], -m_ref[b], -m_ref[b], -m_ref[b]};
+      for (int b = 0; b < 2; ++b) p[b][a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 3; ++w) fr[0][w] = key(0, w);
 #pragma unroll
@@ -444,12 +444,9 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
         mx[b] = fmaxf(mx[b], __shfl_xor(mx[b], 16));
         mx[b] = fmaxf(mx[b], __shfl_xor(mx[b], 32));
         if (mx[b] > thr[b]) {
-          const float moved = m_ref[b] + mx[b], by = moved - m_ref[b];
-          const float alpha = thr[b] != -INFINITY ? fast_exp2(-by) : 1.f;  // nothing to rescale before a row's first key
-          m_ref[b] = moved;
-          thr[b] = kTau;
-          p[b][0] -= by;
-          p[b][1] -= by;
+          const float alpha = thr[b] != -INFINITY ? fast_exp2(m_ref[b] - mx[b]) : 1.f;  // nothing to rescale before a row's first key
+          m_ref[b] = mx[b];
+          thr[b] = mx[b] + kTau;
           l[b] *= alpha;
 #pragma unroll
           for (int t = 0; t < NT; ++t) o[t][b] *= alpha;
@@ -463,7 +460,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p[b][a][r] = fast_exp2(p[b][a][r]);
+          p[b][a][r] = fast_exp2(p[b][a][r] - m_ref[b]);
           psum += p[b][a][r];
         }
       l[b] += psum;
