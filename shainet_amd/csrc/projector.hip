@@ -288,7 +288,8 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
     // 151 and 131, 512 rows of 2048 -> 3072 32.8 and 30.6; a launch of its own for the parts would take 5 to 8 of these)
     planes = (x_stride & 3) == 0 && !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)f.res | (uintptr_t)f.bias) & 15) &&
              gemm_takes_planes(plan_gemm(T, K, swiglu ? 2 * N : N, K, f.w_bf16), K);
-    if (!normed.reserve((size_t)T * K / 2 * (planes ? 3 : 2) + 1)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
+    planes = planes && normed.reserve((size_t)T * K / 2 * 3);  // (without the memory for them they stay floats)
+    if (!planes && !normed.reserve((size_t)T * K)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     e = f.norm == kNormDynTanh ? launch_dyn_tanh(x, x_stride, f.gamma, f.beta, f.alpha, normed.p, T, K, stream, planes)
                                : launch_rmsnorm(x, x_stride, f.gamma, normed.p, T, K, f.eps, stream, planes);
     if (e != hipSuccess) return llama_fail(SHAINET_HIP_ERR_RUNTIME, std::string("norm launch: ") + hipGetErrorString(e));
