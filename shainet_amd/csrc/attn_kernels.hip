@@ -357,7 +357,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       load_k(sp + 1);
   };
   auto stage_k_tile = [&](int sp) {
-    if (sp + 1 < n_sp) {
+    if (HD == 64 || sp + 1 < n_sp) {
       park_k(sp + 1);
       if constexpr (kLate) load_v(sp + 1);
     }
@@ -501,26 +501,41 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int ahead = G == 1 ? gidx : 0;
   // (what is requested and parked behind the last tile is nobody's: its rows are the last one again, its stage is free)
   int sp = 0;
-  for (; sp < n_mine; ++sp) {
-    if constexpr (HD == 128) __builtin_amdgcn_s_setprio(1);
-    scores(sp);
-    if constexpr (HD == 128) __builtin_amdgcn_s_setprio(0);
-    __syncthreads();  // nobody of the group reads V(sp - 1) and K(sp) any more
-    if constexpr (HD == 128) __builtin_amdgcn_sched_barrier(0);  // (V is split in this half; heads of 64 have fewer MFMAs than this half has work)
-    stage_v_tile(sp + ahead);
-    softmax(sp);
-    if constexpr (kLate) __builtin_amdgcn_sched_barrier(0);  // (K is on its way meanwhile)
-    stage_k_tile(sp + ahead);
-    __syncthreads();  // V(sp) and K(sp + 1) are there
-    if constexpr (HD == 128) __builtin_amdgcn_s_setprio(1);
-    outputs(sp);
+  if constexpr (HD == 64) {
+    if (n_mine > 0) scores(0);
+    for (; sp < n_mine - 1; ++sp) {
+      __syncthreads();  // nobody of the group reads V(sp - 1) and K(sp) any more
+      stage_v_tile(sp + ahead);
+      softmax(sp);
+      stage_k_tile(sp + ahead);
+      __syncthreads();  // V(sp) and K(sp + 1) are there
+      outputs(sp);
+      scores(sp + 1);
+    }
+  } else {  // (a loop that begins with the scores has no spills here; heads of 64 take 2 % longer so)
+    for (; sp < n_mine; ++sp) {
+      __builtin_amdgcn_s_setprio(1);
+      scores(sp);
+      __builtin_amdgcn_s_setprio(0);
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);  // (V is split in this half; heads of 64 have fewer MFMAs than this half has work)
+      stage_v_tile(sp + ahead);
+      softmax(sp);
+      if constexpr (kLate) __builtin_amdgcn_sched_barrier(0);  // (K is on its way meanwhile)
+      stage_k_tile(sp + ahead);
+      __syncthreads();
+      __builtin_amdgcn_s_setprio(1);
+      outputs(sp);
+    }
+    __builtin_amdgcn_s_setprio(0);
   }
-  if constexpr (HD == 128) __builtin_amdgcn_s_setprio(0);
-  for (; sp < n_sp; ++sp) {  // tiles that only others see
+  for (; sp < n_sp; ++sp) {  // the wavefront's last tile (heads of 64), and those that only others see
     __syncthreads();
     if (sp + ahead < n_sp) stage_v_tile(sp + ahead);
+    if (HD == 64 && sp < n_mine) softmax(sp);
     if (sp + ahead + 1 < n_sp) stage_k_tile(sp + ahead);
     __syncthreads();
+    if (HD == 64 && sp < n_mine) outputs(sp);
   }
   if (gidx == 0) __syncthreads();
 
