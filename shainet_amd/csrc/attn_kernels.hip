@@ -110,9 +110,9 @@ struct TileUnits {
 // (split_mfma.hpp): the queries once, a key tile by the workgroup on its way to LDS, the probabilities in
 // the registers the scores came in.  A tile costs a wavefront HD / 16 x 12 + HD / 16 x 12 MFMAs of 16 cycles (64:
 // 1536) where the fp32 instruction took HD x 64 (4096).
-// Us, v_mfma_f32_32x32x16_bf16 with both wavefronts of a SIMD in step | this: 2048 rows, 32 / 8 heads of 64, 106.7 | 96.4, 4096 rows 370 | 303, 512 rows on
-// 16384 366 | 304; 512 rows on 16384, 32 / 4 heads of 128, 690 | 551, 2048 rows, 32 / 8 heads of 128, 221 | 199, 4096 rows 743 | 596; 2048 rows of 32 heads of 96
-// 214 | 178.  Errors against 64 bits 0 to 13 % smaller.
+// Us, v_mfma_f32_32x32x16_bf16 with both wavefronts of a SIMD in step | this: 2048 rows, 32 / 8 heads of 64, 111 | 100, 4096 rows 380 | 317, 512 rows on
+// 16384 376 | 319; 512 rows on 16384, 32 / 4 heads of 128, 715 | 580, 2048 rows, 32 / 8 heads of 128, 225 | 204, 4096 rows 763 | 616; 2048 rows of 32 heads of 96
+// 219 | 186; 600 and 700 rows, 32 / 8 heads of 64, 33.0 | 33.8 and 35.9 | 36.4.  Errors against 64 bits 2 to 15 % smaller.
 // What each part of it gave: half a step apart 104 | 100 and fragments a block ahead of their MFMAs 98; the layout of LDS without conflicts 96 | 92.6; a block's
 // products on one accumulator rather than two in turn 1 %; two row blocks a workgroup and the queries' third parts in LDS, which ended spills, 656 | 568 (512 rows on 16384, heads of 128).  In step
 // again (no group waits half a step at the start) short ranges take 2 to 10 % longer.
@@ -1025,9 +1025,11 @@ int prefill_key_splits(const SeqTable &st, const Shape &sh, int items) {
   // With long key ranges, about 1024 row blocks and chunks: two blocks share a workgroup and its tiles then.
   const int ns_1024 = (int)((1024 + wgs - 1) / wgs);
   if (longest / ns_1024 >= 32) return ns_1024 < 16 ? ns_1024 : 16;
-  // Otherwise what is estimated to end first, in times of a key tile: a compute unit has one workgroup at a time, which costs five tiles beside
-  // its own, and the launch that merges costs four more and one for each chunk.  Us, chunks by a target of 512 workgroups | these: 32 / 8 heads of 64, 800 rows 49 | 41, 200 on
-  // 2000 46 | 37, 400 on 4000 113 | 89; heads of 128, 800 rows 86 | 73, 32 / 4 heads, 512 on 4096 214 | 188; heads of 96, 777 rows 70 | 59.
+  // Otherwise what is estimated to end first, in times of a key tile: a compute unit has one workgroup at a time, which costs three tiles beside
+  // its own; the launch that merges costs six for two chunks and one and a half for each further one (heads over 64, whose tiles take longer: four and a
+  // half, one and a quarter).
+  // Us, chunks by a target of 512 workgroups | these: 32 / 8 heads of 64, 800 rows 49 | 41, 200 on 2000 46 | 37, 400 on 4000 113 | 89; heads of 128, 800 rows 86 | 73,
+  // 32 / 4 heads, 512 on 4096 214 | 181; heads of 96, 777 rows 70 | 59.
   double blocks = 0, tiles = 0;
   for (int s = 0; s < st.n_seqs; ++s) {
     const double n = (st.n_new[s] * (double)sh.g + 127) / 128;
@@ -1038,8 +1040,8 @@ int prefill_key_splits(const SeqTable &st, const Shape &sh, int items) {
   int best = 1;
   double least = 0;
   for (int ns = 1; ns == 1 || (ns <= cap && ns <= 16); ++ns) {
-    const double rounds = (double)((wgs * ns + 255) / 256), one = (longest + ns - 1) / ns + 5, all = rounds * (tiles / blocks / ns + 5);
-    const double ends = (one > all ? one : all) + (ns > 1 ? 4 + ns : 0);
+    const double rounds = (double)((wgs * ns + 255) / 256), one = (longest + ns - 1) / ns + 3, all = rounds * (tiles / blocks / ns + 3);
+    const double ends = (one > all ? one : all) + (ns == 1 ? 0 : sh.hd <= 64 ? 3 + 1.5 * ns : 2 + 1.25 * ns);
     if (ns == 1 || ends < least) {
       least = ends;
       best = ns;
