@@ -112,7 +112,8 @@ struct TileUnits {
 // 1536) where the fp32 instruction took HD x 64 (4096).
 // Us, v_mfma_f32_32x32x16_bf16 with both wavefronts of a SIMD in step | this: 2048 rows, 32 / 8 heads of 64, 111 | 100, 4096 rows 380 | 317, 512 rows on
 // 16384 376 | 319; 512 rows on 16384, 32 / 4 heads of 128, 715 | 580, 2048 rows, 32 / 8 heads of 128, 225 | 204, 4096 rows 763 | 616; 2048 rows of 32 heads of 96
-// 219 | 186; 600 and 700 rows, 32 / 8 heads of 64, 33.0 | 33.8 and 35.9 | 36.4.  Errors against 64 bits 2 to 15 % smaller.
+// 219 | 186; 32 / 8 heads of 64, 45 rows 11.9 | 12.3, 600 and
+// 700 33.0 | 33.8 and 35.9 | 36.4 (start and end of a workgroup).  Errors against 64 bits 2 to 15 % smaller.
 // What each part of it gave: half a step apart 104 | 100 and fragments a block ahead of their MFMAs 98; the layout of LDS without conflicts 96 | 92.6; a block's
 // products on one accumulator rather than two in turn 1 %; two row blocks a workgroup and the queries' third parts in LDS, which ended spills, 656 | 568 (512 rows on 16384, heads of 128).  In step
 // again (no group waits half a step at the start) short ranges take 2 to 10 % longer.
@@ -491,7 +492,8 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     if (!kLate) load_k(1);
   }
   __syncthreads();
-  if (gidx == 1) {
+  const bool half_apart = G == 1 || n_sp > 1;  // (a tile each: 64 rows, 32 / 8 heads of 64, 14.0 | 13.4 us with both groups in step)
+  if (gidx == 1 && half_apart) {
     if (G == 1 && n_sp > 0) {
       stage_v_tile(0);
       stage_k_tile(0);
@@ -537,7 +539,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     __syncthreads();
     if (HD == 64 && sp < n_mine) outputs(sp);
   }
-  if (gidx == 0) __syncthreads();
+  if (gidx == 0 && half_apart) __syncthreads();
 
   // Some results are taken again, tile by tile in fp32:
   //   results that are not finite come from operands that are not, and fp32 says which (8192 rows, 32 / 8 heads of 64, NaN
