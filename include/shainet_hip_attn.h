@@ -216,8 +216,8 @@ int shainet_attn_last_q_rot(shainet_attn_ctx *ctx, float *out, int rows);
  * plan[0] path: 0 = split-K decode kernel, 1 = MFMA prefill kernel, 2 = generic kernel;
  * plan[1] the head_dim the kernel's tiles are laid out for (64, 128 or 256: the first that holds
  * head_dim; head_dim itself on the generic path); plan[2] key chunks per row block (1 = none, > 1 adds the combine kernel);
- * plan[3] groups of four wavefronts that share a prefill row block's keys (1 = a workgroup takes two row blocks, a group
- * each, 2 = both groups take one; decode: 1); plan[4] row blocks a
+ * plan[3] groups of four wavefronts of a prefill workgroup (1 = two, which take a row block each, 2 = two, which share a
+ * row block's keys, 3 = one, which takes a row block; decode: 1); plan[4] row blocks a
  * workgroup takes in turn (0 = one workgroup per block and chunk); plan[5] workgroups;
  * plan[6] decode: 16-key tiles per workgroup, prefill: row blocks; plan[7] workgroups per
  * compute unit the launch is held to (0 = no limit).  Lets a test name the kernel instantiation

@@ -16,6 +16,7 @@
 // no LDS round trip for P.  The contraction index of an MFMA may be visited in
 // any order as long as A and B agree.
 #include "attn_kernels.hpp"
+#include "lane_quarters.hpp"
 #include "split_mfma.hpp"
 
 #include <math.h>
@@ -99,6 +100,7 @@ struct TileUnits {
 // G = 2: wavefronts 4..7 own the same 128 virtual rows as 0..3 and take every second key tile; the two
 // halves merge through LDS.
 // G = 1: two row blocks of a sequence; both groups walk the same key tiles, which are staged and split once for 256 rows.
+// G = 3: one group, one row block; two or three such workgroups share a compute unit.
 // One workgroup's work: the row block, or pair of them (and key chunk) number `bid` of the launch.
 // PAD: the head dimension of the data (sh.hd, a multiple of 4) is smaller than HD, the one the
 // tiles are laid out for: query elements beyond it are zeros (whatever stands in for the keys'
@@ -122,11 +124,13 @@ struct TileUnits {
 // took 14 and 17 % less, but such numbers leave out up to 2^-21 of a product, and where a key's second parts have the signs of the
 // query's that adds up.)
 // Heads of 128 have no registers for the queries' third parts, or those of 24 of 32 octets: these lie in LDS, too.  (G = 2: both groups have the same.)
+// G = 3: heads of 64 keep within 168 registers so (three wavefronts on a SIMD); heads of 128 those of 24, or two workgroups would not fit.
 template <int HD, int G>
-constexpr int kThirds = HD == 128 ? (G == 2 ? 4 : 3) : 0;
+constexpr int kThirds = HD == 128 ? (G == 2 ? 4 : 3) : G == 3 ? 2 : 0;
 template <int HD, int G>
-constexpr int kLdsUnits = 2 * TileUnits<HD>::kTile + (G == 2 ? 4 : 8) * kThirds<HD, G> * 128;
+constexpr int kLdsUnits = (G == 3 ? 1 : 2) * TileUnits<HD>::kTile + (G == 1 ? 8 : 4) * kThirds<HD, G> * 128;
 static_assert(kLdsUnits<128, 1> * 16 <= 160 * 1024 && kLdsUnits<128, 2> * 16 <= 160 * 1024, "LDS of a compute unit");
+static_assert(2 * kLdsUnits<128, 3> * 16 <= 160 * 1024, "two workgroups of one group share a compute unit");
 
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS>
 __device__ __forceinline__ void prefill_block(const int bid, const float *__restrict__ q_rot,
@@ -140,7 +144,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   constexpr int NT = HD / 16;   // d blocks of the output
   // items per thread to stage a tile of K (or V): G = 2, the tile of its group; G = 1, the one that all share, heads of 64: K is the first
   // group's, V the second's
-  constexpr int NI = G == 2 ? HD / 64 : 1;
+  constexpr int NI = G == 1 ? 1 : HD / 64;
   constexpr bool kOneOfTwo = G == 1 && HD == 64;
   __shared__ __attribute__((aligned(16))) u32x4 lds[kLdsUnits<HD, G>];
 
@@ -154,7 +158,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int chunk = SPLIT ? (bid / sh.KV) % ns : 0;
   const int item = SPLIT ? bid / sh.KV / ns : bid / sh.KV;
   int s, vb;
-  locate_block<3 - G>(st, item, s, vb);
+  locate_block<G == 1 ? 2 : 1>(st, item, s, vb);
   // These are the same for all lanes of a wavefront, which the compiler cannot see: said so,
   // tile counts, loop conditions and address bases live in scalar registers
   auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
@@ -164,9 +168,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int L = S + T, VR = T * g;
   const int lane = threadIdx.x & 63;
   const int wave = uniform((threadIdx.x >> 6) & 3);  // which 32 virtual rows of the block
-  const int gidx = uniform(threadIdx.x >> 8);        // which group of wavefronts
-  const int wg_hi = st.start_pos[s] + min((vb + 1) * 128 * (3 - G) - 1, st.n_new[s] * sh.g - 1) / sh.g;
+  const int gidx = G == 3 ? 0 : uniform(threadIdx.x >> 8);  // which group of wavefronts
+  const int wg_hi = st.start_pos[s] + min((vb + 1) * (G == 1 ? 256 : 128) - 1, st.n_new[s] * sh.g - 1) / sh.g;
   if (G == 1) vb = 2 * vb + gidx;
+  constexpr int kStep = G == 2 ? 2 : 1;      // key tiles of a step
   const int first_tile = G == 2 ? gidx : 0;  // a group's first key tile
   const int n = lane & 15, j = lane >> 4;
   const int v0 = vb * 128 + wave * 32;
@@ -175,7 +180,9 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int wave_hi = wave_active ? S + min(v0 + 31, VR - 1) / g : -1;  // largest
   const int n_tiles = wg_hi / 32 + 1;
   const int tiles_per_chunk = SPLIT ? (n_tiles + ns - 1) / ns : n_tiles;
-  const int kt0 = chunk * tiles_per_chunk, kt1 = min(n_tiles, kt0 + tiles_per_chunk);
+  int kt0 = chunk * tiles_per_chunk;
+  if constexpr (G == 3) asm volatile("" : "+s"(kt0));  // (of a range that begins at 0 it keeps addresses per thread: 28 spills in padded tiles, 159 | 114 us at 64 sequences of 100 rows)
+  const int kt1 = min(n_tiles, kt0 + tiles_per_chunk);
   const int hd = PAD ? uniform(sh.hd) : HD;  // floats between two rows of q, K, V and the output
   const long long head_base = (long long)st.slot[s] * sh.seq_stride + (long long)kvh * sh.cap * hd;
   const float *kbase = kc + head_base;
@@ -201,7 +208,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   bool k_second[NI];  // the octet's second half lies within the row
 #pragma unroll
   for (int u = 0; u < NI; ++u) {
-    const int idx = (G == 2 || kOneOfTwo ? threadIdx.x & 255 : threadIdx.x) + 256 * u;
+    const int idx = (G != 1 || kOneOfTwo ? threadIdx.x & 255 : threadIdx.x) + 256 * u;
     const int pair = HD == 128 ? idx >> 5 : idx >> 4;  // (of keys eight apart)
     const int oct = (idx & 7) | (HD == 128 ? idx >> 1 & 8 : 0), r = (idx & 8) | (pair & 7) | (pair & 8) << 1;
     k_row[u] = r;
@@ -220,7 +227,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   // at launch); rows past the last one repeat it
   auto load_k = [&](int sp) {
     if (kOneOfTwo && gidx) return;
-    const int first = (kt0 + G * sp + first_tile) * 32;
+    const int first = (kt0 + kStep * sp + first_tile) * 32;
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       const char *p = (const char *)kbase + ((unsigned)min(first + k_row[u], L - 1) * k_stride + k_off[u]);
@@ -230,7 +237,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   };
   auto load_v = [&](int sp) {
     if (kOneOfTwo && !gidx) return;
-    const int first = (kt0 + G * sp + first_tile) * 32;
+    const int first = (kt0 + kStep * sp + first_tile) * 32;
     if (first + 32 <= L) {
       const char *base = (const char *)vbase + (unsigned long long)first * v_stride;
 #pragma unroll
@@ -276,14 +283,14 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 
   // steps of a tile, or (G = 2) of one per group; below "tile sp" is a group's tile of step sp (in the last step the second group
   // may have none left: it stages its last rows again)
-  const int n_sp = kt0 < kt1 ? (kt1 - kt0 + G - 1) / G : 0;
+  const int n_sp = kt0 < kt1 ? (kt1 - kt0 + kStep - 1) / kStep : 0;
   if (n_sp > 0) {
     load_k(0);
     load_v(0);
   }
   // the row's query, scaled by scale * log2(e): scores come out in log2 units
   u32x4 qf[KS][2][3];
-  u32x4 *const third = lds + 2 * U::kTile + (G == 2 ? wave : 4 * gidx + wave) * (kThirds<HD, G> * 128) + lane;
+  u32x4 *const third = lds + 2 * U::kTile + (G == 1 ? 4 * gidx + wave : wave) * (kThirds<HD, G> * 128) + lane;
   bool apart;  // some query of the wavefront needs its scores in fp32
   {
     float least = INFINITY, most = 0.f;
@@ -302,7 +309,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
 #pragma unroll
       for (int i = 0; i < KS; ++i) {
         split_octet(t[i][0] * c, t[i][1] * c, qf[i][b][0], qf[i][b][1], qf[i][b][2]);
-        if (i < kThirds<HD, G> && (G == 1 || gidx == 0)) third[(2 * i + b) * 64] = qf[i][b][2];
+        if (i < kThirds<HD, G> && (G != 2 || gidx == 0)) third[(2 * i + b) * 64] = qf[i][b][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           if (PAD && 32 * i + 8 * j + 4 * h >= hd) continue;
@@ -346,30 +353,33 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   // one wavefront has MFMAs only, its other one has none.  G = 2: each group stages its own tiles, one of K and one of V.  G = 1: both stage
   // half of each, into two stages in turn; the second group does so a step ahead, for the first needs them half a step later.
   // (heads of 128, G = 2, have no registers for a tile of K during the MFMAs: it is requested and parked within the other half)
-  constexpr bool kLate = HD == 128 && G == 2;
+  constexpr bool kLate = HD == 128 && G != 1;
   const int k_at[2] = {U::key_unit(j, n) + (G == 2 ? gidx * U::kTile : 0), (U::key_unit(j, n) ^ 4) + (G == 2 ? gidx * U::kTile : 0)}, v_at = U::kK + j * U::kGroupV + n + (G == 2 ? gidx * U::kTile : 0);
   // tiles that some row of the wavefront sees
-  const int n_mine = max(0, (min(kt1, wave_hi / 32 + 1) - kt0 - first_tile + G - 1) / G) * (wave_hi >= 0);
+  const int n_mine = max(0, (min(kt1, wave_hi / 32 + 1) - kt0 - first_tile + kStep - 1) / kStep) * (wave_hi >= 0);
+  constexpr bool kExact = G == 3;                 // nothing is requested for nobody: ranges are short
+  constexpr bool kScoresFirst = HD == 128 || G == 3;  // in the loop below
   auto stage_v_tile = [&](int sp) {
     park_v(sp);
-    if constexpr (!kLate)
-      load_v(sp + 1);
-    else if (sp + 1 < n_sp)
+    if constexpr (!kLate) {
+      if (!kExact || sp + 1 < n_sp) load_v(sp + 1);
+    } else if (sp + 1 < n_sp) {
       load_k(sp + 1);
+    }
   };
   auto stage_k_tile = [&](int sp) {
-    if (HD == 64 || sp + 1 < n_sp) {
+    if ((HD == 64 && !kExact) || sp + 1 < n_sp) {
       park_k(sp + 1);
       if constexpr (kLate) load_v(sp + 1);
     }
-    if (!kLate) load_k(sp + 2);
+    if (!kLate && (!kExact || sp + 2 < n_sp)) load_k(sp + 2);
   };
   f32x4 p[2][2];   // [virtual rows][keys]: scores, then probabilities
   u32x4 pf[2][3];  // their parts
   f32x4 near_bias[BIAS ? 2 : 1][2];
   bool near = false;
   auto scores = [&](int sp) {
-    const int kt = kt0 + G * sp + first_tile;
+    const int kt = kt0 + kStep * sp + first_tile;
     auto key = [&](int k, int w) { return lds[k_at[k / 2 & 1] + (G == 1 && sp & 1 ? U::kTile : 0) + w * U::kPartK + k / 2 * 128 + k % 2 * 16]; };
     // the tile's values by distance are asked for in front of its MFMAs; a tile that lies
     // `reach` or more behind all rows of the wavefront has none
@@ -412,7 +422,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     }
   };
   auto softmax = [&](int sp) {
-    const int kt = kt0 + G * sp + first_tile;
+    const int kt = kt0 + kStep * sp + first_tile;
     if constexpr (BIAS) {
       if (near) {
 #pragma unroll
@@ -442,8 +452,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       // rare after a row's first tiles: move the reference to this tile's maximum
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        mx[b] = fmaxf(mx[b], __shfl_xor(mx[b], 16));
-        mx[b] = fmaxf(mx[b], __shfl_xor(mx[b], 32));
+        mx[b] = max_across_quarters(mx[b]);
         if (mx[b] > thr[b]) {
           const float alpha = thr[b] != -INFINITY ? fast_exp2(m_ref[b] - mx[b]) : 1.f;  // nothing to rescale before a row's first key
           m_ref[b] = mx[b];
@@ -489,10 +498,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   };
   if (n_sp > 0) {
     park_k(0);
-    if (!kLate) load_k(1);
+    if (!kLate && (!kExact || n_sp > 1)) load_k(1);
   }
   __syncthreads();
-  const bool half_apart = G == 1 || n_sp > 1;  // (a tile each: 64 rows, 32 / 8 heads of 64, 14.0 | 13.4 us with both groups in step)
+  const bool half_apart = G == 1 || (G == 2 && n_sp > 1);  // (a tile each: 64 rows, 32 / 8 heads of 64, 14.0 | 13.4 us with both groups in step)
   if (gidx == 1 && half_apart) {
     if (G == 1 && n_sp > 0) {
       stage_v_tile(0);
@@ -503,7 +512,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   const int ahead = G == 1 ? gidx : 0;
   // (what is requested and parked behind the last tile is nobody's: its rows are the last one again, its stage is free)
   int sp = 0;
-  if constexpr (HD == 64) {
+  if constexpr (!kScoresFirst) {
     if (n_mine > 0) scores(0);
     for (; sp < n_mine - 1; ++sp) {
       __syncthreads();  // nobody of the group reads V(sp - 1) and K(sp) any more
@@ -534,10 +543,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   for (; sp < n_sp; ++sp) {  // the wavefront's last tile (heads of 64), and those that only others see
     __syncthreads();
     if (sp + ahead < n_sp) stage_v_tile(sp + ahead);
-    if (HD == 64 && sp < n_mine) softmax(sp);
+    if (!kScoresFirst && sp < n_mine) softmax(sp);
     if (sp + ahead + 1 < n_sp) stage_k_tile(sp + ahead);
     __syncthreads();
-    if (HD == 64 && sp < n_mine) outputs(sp);
+    if (!kScoresFirst && sp < n_mine) outputs(sp);
   }
   if (gidx == 0 && half_apart) __syncthreads();
 
@@ -567,7 +576,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       asm volatile("" : "+v"(tid));
       unsigned small = ~0u;  // (zeros lie above all)
 #pragma clang loop unroll(disable)
-      for (int kt = kt0 + first_tile; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
+      for (int kt = kt0 + first_tile; kt < kt1 && kt * 32 <= wave_hi; kt += kStep) {
         const float *vr = vbase + (long long)min(kt * 32 + (tid & 31), wave_hi) * vhd;
 #pragma clang loop unroll_count(4)
         for (int d = (tid & 32) >> 3; d < vhd; d += 8) {
@@ -604,7 +613,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       // the running maximum; the products with V likewise where every row sees the whole tile, else key by key
       // (what a row does not see it does not multiply by zero either).
 #pragma clang loop unroll(disable)
-      for (int kt = kt0 + first_tile; kt < kt1 && kt * 32 <= wave_hi; kt += G) {
+      for (int kt = kt0 + first_tile; kt < kt1 && kt * 32 <= wave_hi; kt += kStep) {
         const int first = kt * 32;
         const bool whole = first + 31 <= wave_lo;
         const float *kr[2] = {kbase + (long long)min(first + n, L - 1) * hd + 4 * j, kbase + (long long)min(first + 16 + n, L - 1) * hd + 4 * j};
@@ -729,8 +738,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   float m[2];
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    l[b] += __shfl_xor(l[b], 16);
-    l[b] += __shfl_xor(l[b], 32);
+    l[b] = sum_across_quarters(l[b]);
     m[b] = thr[b] == -INFINITY ? -INFINITY : m_ref[b];
   }
   if constexpr (G == 2) {
@@ -764,35 +772,48 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       m[b] = mnew;
     }
   }
+  // A lane has 4 NT neighbouring columns of a row: stored as they are, an instruction would write 16 bytes into each of 64 lines.  Traded among the
+  // quarters, four lanes write 64 bytes together (us, as they are | traded: 64 sequences of 64 rows, 32 / 8 heads of 64, 33.2 | 27.0, of 100 rows, 32 heads of
+  // 128, 121 | 113, 64 sequences of 96 rows, two blocks a workgroup 58.2 | 52.7).
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const int n = tid & 15, j = (tid & 63) >> 4, my_v = v0 + 16 * b + n;
+    f32x4 line[NT / 4][4];  // [..][i]: the piece of four columns at NT i + 4 h + j
+#pragma unroll
+    for (int h = 0; h < NT / 4; ++h) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = (4 * h + q) / (NT / 4), w = 4 * ((4 * h + q) % (NT / 4));
+        line[h][q] = f32x4{o[w][b][r], o[w + 1][b][r], o[w + 2][b][r], o[w + 3][b][r]};
+      }
+      transpose_quarters(line[h]);
+    }
     if (my_v >= VR) continue;
     if (SPLIT) {  // unnormalised partial of this key chunk: [128 virtual rows][HD], (max, sum) per row
       const long long pbase = (((long long)(G == 1 ? uniform(block_rank(st, s, vb)) : item) * sh.KV + kvh) * ns + chunk) * 128 + wave * 32 + 16 * b + n;
-      float *op = part_o + pbase * HD + NT * 4 * j;
+      float *op = part_o + pbase * HD + 4 * j;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int h = 0; h < NT / 4; ++h)
 #pragma unroll
-        for (int w = 0; w < NT; w += 4) *(f32x4 *)(op + NT * r + w) = f32x4{o[w][b][r], o[w + 1][b][r], o[w + 2][b][r], o[w + 3][b][r]};
+        for (int i = 0; i < 4; ++i) *(f32x4 *)(op + 4 * (NT * i + 4 * h)) = line[h][i];
       if (j == 0) *(float2 *)(part_ml + 2 * pbase) = float2{m[b], l[b]};
     } else {
       const int row = my_v / g, hg = my_v - row * g;
       const float inv = 1.0f / l[b];
-      float *op = out + ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * vhd + NT * 4 * j;
+      float *op = out + ((long long)(st.tok_off[s] + row) * sh.H + kvh * g + hg) * vhd + 4 * j;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int h = 0; h < NT / 4; ++h)
 #pragma unroll
-        for (int w = 0; w < NT; w += 4) {
-          if (PAD && NT * (4 * j + r) + w >= vhd) continue;  // (the width is a multiple of 4)
-          *(f32x4 *)(op + NT * r + w) = f32x4{o[w][b][r] * inv, o[w + 1][b][r] * inv, o[w + 2][b][r] * inv, o[w + 3][b][r] * inv};
+        for (int i = 0; i < 4; ++i) {
+          if (PAD && 4 * (NT * i + 4 * h + j) >= vhd) continue;  // (the width is a multiple of 4)
+          *(f32x4 *)(op + 4 * (NT * i + 4 * h)) = line[h][i] * inv;
         }
     }
   }
 }
 
 template <int HD, bool SPLIT, int G, bool PAD, bool BIAS = false>
-__global__ __launch_bounds__(512, 2) void prefill_mfma_kernel(const float *__restrict__ q_rot,
+__global__ __launch_bounds__(G == 3 ? 256 : 512, G == 3 && HD == 64 && !BIAS ? 3 : 2) void prefill_mfma_kernel(const float *__restrict__ q_rot,
                                                               const float *__restrict__ kc,
                                                               const float *__restrict__ vc,
                                                               float *__restrict__ out,
@@ -1056,23 +1077,51 @@ size_t prefill_partial_floats(const Shape &sh, int items, int ns, int v_hd) {
   return ns > 1 ? (size_t)items * sh.KV * ns * 128 * (prefill_tile_head_dim(widest(sh, v_hd)) + 2) : 0;
 }
 
-PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_per_cu, int groups, int v_hd) {
+// How many key tiles a row block of a sequence walks through on average (per: blocks that walk together), all chunks of them.
+static double mean_tiles(const SeqTable &st, const Shape &sh, int s, int per) {
+  return (st.start_pos[s] + 0.5 * st.n_new[s] + 64.0 * per / sh.g) / 32 + 0.5;
+}
+
+static long long block_pairs(const SeqTable &st) {
+  long long pairs = 0;
+  for (int s = 0; s < st.n_seqs; ++s) pairs += (st.work_off[s] + 1) / 2;
+  return pairs;
+}
+
+PrefillLaunch plan_prefill_launch(const SeqTable &st, const Shape &sh, int items, int ns, int wgs_per_cu, int groups, int v_hd) {
   PrefillLaunch p;
   p.n_wgs = (long long)items * sh.KV * ns;
-  // A launch of up to three row blocks a compute unit has each in a workgroup of its own, whose groups share its keys; in larger ones a workgroup takes
-  // two, whose groups share the tiles.
-  p.groups = groups == 1 || groups == 2 ? groups : (p.n_wgs <= 768 ? 2 : 1);
   const int tile_hd = prefill_tile_head_dim(widest(sh, v_hd));
-  const size_t static_lds = (size_t)16 * (tile_hd == 64 ? kLdsUnits<64, 1> : p.groups == 2 ? kLdsUnits<128, 2> : kLdsUnits<128, 1>);
+  p.groups = groups >= 1 && groups <= 3 ? groups : 2;
+  if (p.groups != groups) {
+    double tiles = 0, pair_tiles = 0, rows = 0;
+    const long long pairs = block_pairs(st);
+    for (int s = 0; s < st.n_seqs; ++s) {
+      tiles += st.work_off[s] * mean_tiles(st, sh, s, 1);
+      pair_tiles += (st.work_off[s] + 1) / 2 * mean_tiles(st, sh, s, 2);
+      rows += (double)st.n_new[s] * sh.g;
+    }
+    if (p.n_wgs > 768) {
+      // More than three row blocks a compute unit: two blocks a workgroup, which share a tile's splits and of whose groups one has MFMAs while the other has none, or a workgroup a block,
+      // two or three on a compute unit, which start and end beside each other and leave no half empty where a sequence has an odd block.  What is
+      // estimated to end first, in us: 256 pairs take 7 and, a key tile, 1.1 to 2.6 by how full they are (heads over 64: 12.5, 1.6 to 4.6), 256 blocks
+      // 3.2 and 1.1 a tile, longer ranges 1.43 (5.5 and 2.45).
+      // Us, two blocks | one: 64 sequences, 32 / 8 heads of 64, of 40 rows 25.5 | 22.2, 100 rows 59.6 | 44.3, 200 rows 135 | 96, 400 rows 330 | 282, 40 on 500 82 | 96,
+      // 100 on 2000 634 | 733; one of 4096 rows 343 | 351; heads of 128, of 40 rows 39 | 36, 200 rows 228 | 198, 100 on 500 357 | 410; 32 heads of 96, of 100 rows
+      // (a block each) 157 | 110, 40 on 500 397 | 320, 400 rows 671 | 700.
+      const double walk = tiles / items / ns, pair_walk = pair_tiles / pairs / ns, full = rows / (256.0 * pairs);
+      const double two = pairs * sh.KV * ns / 256.0 * (tile_hd == 64 ? 7 + (1.1 + 1.5 * full) * pair_walk : 12.5 + (1.6 + 3 * full) * pair_walk);
+      const double one = p.n_wgs / 256.0 * (tile_hd > 64 ? 5.5 + 2.45 * walk : walk < 13 ? 3.2 + 1.1 * walk : 1.43 * walk - 1.1);
+      p.groups = one < two ? 3 : 1;
+    }
+  }
   p.pad = 0;
-  // With fewer workgroups than three per compute unit everything is resident at
-  // once and the dispatcher cannot balance the triangular work: one workgroup per
-  // compute unit lets it hand the short row blocks to whichever unit finishes first.
-  if (wgs_per_cu == 0 && p.n_wgs <= 768) wgs_per_cu = 1;
-  p.wgs_per_cu = wgs_per_cu >= 1 && wgs_per_cu <= 3 ? wgs_per_cu : 0;
-  if (p.wgs_per_cu) {
-    const size_t want = (size_t)160 * 1024 / wgs_per_cu;  // one more workgroup would not fit
-    const size_t floor_ = (size_t)160 * 1024 / (wgs_per_cu + 1) + 256;
+  // Eight wavefronts fill a compute unit's registers.  Of the workgroups of four, up to 256 have one each to themselves, more as many as fit.
+  p.wgs_per_cu = p.groups != 3 ? 1 : wgs_per_cu >= 1 && wgs_per_cu <= 3 ? wgs_per_cu : p.n_wgs <= 256 ? 1 : 0;
+  if (p.groups == 3 && p.wgs_per_cu) {
+    const size_t static_lds = (size_t)16 * (tile_hd == 64 ? kLdsUnits<64, 3> : kLdsUnits<128, 3>);
+    const size_t want = (size_t)160 * 1024 / p.wgs_per_cu;  // one more workgroup would not fit
+    const size_t floor_ = (size_t)160 * 1024 / (p.wgs_per_cu + 1) + 256;
     if (static_lds < floor_ && floor_ <= want) p.pad = floor_ - static_lds;
   }
   static const bool turns_off = getenv("SHAINET_HIP_PREFILL_NO_TURNS") != nullptr;
@@ -1088,12 +1137,7 @@ PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_pe
 
 long long prefill_workgroups(const SeqTable &st, const Shape &sh, const PrefillLaunch &p, int items, int ns) {
   if (p.turns) return (p.n_wgs + p.turns - 1) / p.turns;
-  int units = items;
-  if (p.groups == 1) {
-    units = 0;
-    for (int s = 0; s < st.n_seqs; ++s) units += (st.work_off[s] + 1) / 2;
-  }
-  return (long long)units * sh.KV * ns;
+  return (p.groups == 1 ? block_pairs(st) : items) * sh.KV * ns;
 }
 
 hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, float *out, float *partials,
@@ -1106,7 +1150,7 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
   if (bias && (!db.tab || (v_hd & 3) || (db.q_stride & 3) || v_hd < 4 || (long long)sh.cap * v_hd * 4 > 0xffffffffLL)) return hipErrorInvalidValue;
   if (!table_ok(st, sh) || !tile_hd || !prefill_tile_head_dim(sh.hd) || items < 1 || ns < 1 || (ns > 1 && !partials)) return hipErrorInvalidValue;
   const bool pad = tile_hd != sh.hd;
-  const PrefillLaunch plan = plan_prefill_launch(sh, items, ns, wgs_per_cu, groups_wanted, v_hd);
+  const PrefillLaunch plan = plan_prefill_launch(st, sh, items, ns, wgs_per_cu, groups_wanted, v_hd);
   const long long n_wgs = plan.n_wgs;
   if (n_wgs > 0x7fffffffLL) return hipErrorInvalidValue;
   // the kernels address a row of a (sequence, kv head) by a 32-bit byte offset from its first row
@@ -1142,7 +1186,10 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
   hipEvent_t main_after = ns == 1 ? after : nullptr;  // with key chunks the combine kernel ends the timed stretch
 #define SHAINET_LAUNCH_PREFILL(HD_, SPLIT_, ...)                                                               \
   do {                                                                                                          \
-    if (groups == 2)                                                                                            \
+    if (groups == 3)                                                                                            \
+      SHAINET_LAUNCH_TIMED((prefill_mfma_kernel<HD_, SPLIT_, 3, __VA_ARGS__>), grid, dim3(256), lds_pad, stream, before, \
+                           main_after, q_rot, kc, vc, out, part_o, part_ml, st, sh, ns, c, db);                     \
+    else if (groups == 2)                                                                                       \
       SHAINET_LAUNCH_TIMED((prefill_mfma_kernel<HD_, SPLIT_, 2, __VA_ARGS__>), grid, dim3(512), lds_pad, stream, before, \
                            main_after, q_rot, kc, vc, out, part_o, part_ml, st, sh, ns, c, db);                     \
     else                                                                                                        \

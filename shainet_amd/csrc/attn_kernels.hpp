@@ -179,9 +179,9 @@ size_t prefill_partial_floats(const Shape &sh, int items, int ns, int v_hd = 0);
 // The head dimension the MFMA prefill kernel lays its tiles out for when the data's is hd: 64 or
 // 128, the first that holds hd (a multiple of 4); 0 when neither does.
 int prefill_tile_head_dim(int hd);
-// wgs_per_cu: 0 = default; 1..3 pads the kernel's LDS so that at most that many
-// workgroups share a compute unit (a tuning knob).
-// groups: 0 = default; 1 or 2 forces the number of wavefront groups per workgroup (a tuning knob).
+// wgs_per_cu: 0 = default; 1..3 pads the LDS of workgroups of one group so that at most that many
+// share a compute unit (a tuning knob; of two groups there is one).
+// groups: 0 = default; 1 to 3 forces that layout (PrefillLaunch; a tuning knob).
 hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, float *out, float *partials,
                           const SeqTable &st, const Shape &sh, int items, int ns, float scale,
                           hipStream_t stream, int wgs_per_cu = 0, int groups = 0, hipEvent_t before = nullptr,
@@ -189,14 +189,14 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
 // Which instantiation a prefill launch uses and how it is laid out; launch_prefill follows it.
 struct PrefillLaunch {
   long long n_wgs;   // row blocks x kv heads x key chunks
-  int groups;        // of wavefronts that share a row block's keys.  1: a workgroup takes two row blocks of a sequence, a group of wavefronts each
+  int groups;        // 1: a workgroup takes two row blocks of a sequence, a group of four wavefronts each; 2: two groups share a row block's keys; 3: one group, one row block
   int turns;         // 0: one workgroup per row block and chunk; 2 or 3: prefill_turns_kernel with that many blocks per workgroup
-  int wgs_per_cu;    // 0: as the kernel's registers and LDS allow; 1..3: LDS padded to that occupancy
+  int wgs_per_cu;    // 0: as the kernel's registers and LDS allow (of one group: two or three); 1..3: of one group, LDS padded to that occupancy
   size_t pad;        // bytes of dynamic LDS that enforce wgs_per_cu
 };
 // Workgroups of such a launch; st as plan_work left it.
 long long prefill_workgroups(const SeqTable &st, const Shape &sh, const PrefillLaunch &p, int items, int ns);
-PrefillLaunch plan_prefill_launch(const Shape &sh, int items, int ns, int wgs_per_cu, int groups, int v_hd = 0);
+PrefillLaunch plan_prefill_launch(const SeqTable &st, const Shape &sh, int items, int ns, int wgs_per_cu, int groups, int v_hd = 0);
 hipError_t launch_generic(const float *q_rot, const float *kc, const float *vc, float *out,
                           const SeqTable &st, const Shape &sh, int total_tokens, float scale,
                           hipStream_t stream, const DistanceBias *bias = nullptr);

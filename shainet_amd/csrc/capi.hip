@@ -1253,7 +1253,7 @@ int shainet_attn_describe_plan(int num_heads, int num_kv_heads, int head_dim, in
   } else if (path == Path::kPrefillMfma) {
     const int items = plan_work(st, sh, path);
     const int ns = prefill_key_splits(st, sh, items);
-    const PrefillLaunch p = plan_prefill_launch(sh, items, ns, 0, 0);
+    const PrefillLaunch p = plan_prefill_launch(st, sh, items, ns, 0, 0);
     plan[0] = 1;
     plan[1] = prefill_tile_head_dim(head_dim);
     plan[2] = ns;

@@ -41,6 +41,7 @@
 //   output: tile t, row m is d = 64*(t/4) + 4*m + t%4; k-step r of lane group j is
 //           key 4*j + r of the tile, where accumulator register r of S^T lives.
 #include "attn_kernels.hpp"
+#include "lane_quarters.hpp"
 
 #include <math.h>
 #include <stdint.h>
@@ -770,16 +771,6 @@ struct RowSeqs {
 constexpr int kRowsPlain = 0, kRowsPrep = 1, kRowsBias = 2;  // queries and new rows are prepared; are a projection's; scores gain a value by distance
 template <int HD>
 constexpr int kRowTiles = HD == 64 ? 3 : 2;
-
-// the larger of a lane's value and that of the lane 16 (32) away
-__device__ __forceinline__ float max_across_quarters(float x) {
-  auto larger = [](unsigned a, unsigned b) { return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)); };
-  unsigned bits = __builtin_bit_cast(unsigned, x);
-  auto p = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
-  bits = __builtin_bit_cast(unsigned, larger(p[0], p[1]));
-  p = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-  return larger(p[0], p[1]);
-}
 
 template <int HD, int T, int MODE>
 __global__ __launch_bounds__(256, 1) void decode_rows_kernel(const float *__restrict__ q_rot, const float *__restrict__ kc,

@@ -52,6 +52,19 @@ def test_every_reachable_instantiation_is_covered():
     assert seen == covered, sorted(covered - seen)  # and nothing in the table is unreachable
 
 
+def test_batches_of_short_sequences_have_a_group_for_each_row_block():
+    # two row blocks a workgroup only where they fill it, and where the keys are many enough for that to be worth a compute unit's wait for its next one
+    for H, KV, hd, B, cached, new, groups in [
+            (32, 8, 64, 64, 0, 40, 3), (32, 8, 64, 64, 0, 200, 3), (32, 8, 64, 48, 0, 65, 3), (32, 8, 64, 8, 16384, 32, 3),
+            (32, 8, 128, 8, 16384, 32, 3), (32, 32, 96, 25, 0, 100, 3), (32, 32, 96, 64, 500, 40, 3), (32, 32, 128, 64, 2000, 100, 3),
+            (32, 8, 64, 64, 500, 40, 1), (32, 8, 64, 64, 2000, 100, 1), (32, 8, 128, 64, 500, 100, 1), (32, 8, 64, 1, 0, 4096, 1)]:
+        plan = sa.describe_plan(H, KV, hd, [cached] * B, [new] * B)
+        assert plan["groups"] == groups, (H, KV, hd, B, cached, new, plan)
+        blocks = B * -(-new * (H // KV) // 128)
+        pairs = B * -(-new * (H // KV) // 256)
+        assert plan["workgroups"] == (blocks if groups == 3 else pairs) * KV * plan["key_chunks"], plan
+
+
 def test_decode_and_generic_paths_are_told_apart():
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [1] * 16)["path"] == sa.hip.PATH_DECODE
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [8] * 16)["path"] == sa.hip.PATH_DECODE  # two entries each
