@@ -1094,15 +1094,24 @@ PrefillLaunch plan_prefill_launch(const SeqTable &st, const Shape &sh, int items
   const int tile_hd = prefill_tile_head_dim(widest(sh, v_hd));
   p.groups = groups >= 1 && groups <= 3 ? groups : 2;
   if (p.groups != groups) {
+    int longest = 0;
     double tiles = 0, pair_tiles = 0, rows = 0;
     const long long pairs = block_pairs(st);
     for (int s = 0; s < st.n_seqs; ++s) {
+      const int n = (st.start_pos[s] + st.n_new[s] + 31) / 32;
+      longest = n > longest ? n : longest;
       tiles += st.work_off[s] * mean_tiles(st, sh, s, 1);
       pair_tiles += (st.work_off[s] + 1) / 2 * mean_tiles(st, sh, s, 2);
       rows += (double)st.n_new[s] * sh.g;
     }
-    if (p.n_wgs > 768) {
-      // More than three row blocks a compute unit: two blocks a workgroup, which share a tile's splits and of whose groups one has MFMAs while the other has none, or a workgroup a block,
+    if (p.n_wgs <= 768) {
+      // Up to three row blocks a compute unit: each in a workgroup of two groups that share its keys, but for ranges too short to share, which one group
+      // has walked through in the time of the two groups' merge, and of which two or three share a compute unit.  Us, two groups | one: 32 / 8 heads
+      // of 64, 20 rows 10.0 | 8.6, 45 rows 10.6 | 9.7, 100 rows 13.1 | 12.2, 128 rows 14.1 | 14.3, 200 rows 16.2 | 17.7; heads of 128, 45 rows 14.2 | 12.4, 64 rows
+      // 16.0 | 14.8, 128 rows 19.5 | 20.3; more than 256 blocks: 16 sequences of 100 rows 24.7 | 16.5 and 40 | 24.6, 8 of 200 rows 27.4 | 22.6 and 40.6 | 33.9.
+      if (ns == 1 && longest <= (p.n_wgs > 256 ? 8 : tile_hd == 64 ? 4 : 3)) p.groups = 3;
+    } else {
+      // More: two blocks a workgroup, which share a tile's splits and of whose groups one has MFMAs while the other has none, or a workgroup a block,
       // two or three on a compute unit, which start and end beside each other and leave no half empty where a sequence has an odd block.  What is
       // estimated to end first, in us: 256 pairs take 7 and, a key tile, 1.1 to 2.6 by how full they are (heads over 64: 12.5, 1.6 to 4.6), 256 blocks
       // 3.2 and 1.1 a tile, longer ranges 1.43 (5.5 and 2.45).

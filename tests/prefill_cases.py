@@ -16,6 +16,8 @@ CASES = [
     ("llama1b_prefill_t8192", 32, 8, 64, False, 0, 8192, (64, False, 1, 0)),
     ("llama1b_prefill_t2560", 32, 8, 64, False, 0, 2560, (64, False, 2, 0)),
     ("llama1b_prefill_t1024", 32, 8, 64, False, 0, 1024, (64, True, 2, 0)),
+    ("llama1b_prefill_t45", 32, 8, 64, False, 0, 45, (64, False, 3, 0)),
+    ("qwen3_8b_prefill_t45", 32, 8, 128, True, 0, 45, (128, False, 3, 0)),
     ("w1024_chunked_prefill_t2560_on_1000", 16, 2, 64, False, 1000, 2560, (64, True, 3, 0)),
     ("heads64_prefill_t2048", 64, 8, 64, False, 0, 2048, (64, False, 3, 0)),
     ("llama1b_chunked_prefill_t512_on_16384", 32, 8, 64, False, 16384, 512, (64, True, 1, 0)),

@@ -64,7 +64,8 @@ def test_one_group_of_zeros_and_a_tiny_value(hip, hd, KV, T, tiny, monkeypatch):
 
 
 # (cached, new) of each sequence; more row blocks than compute units
-@pytest.mark.parametrize("H,KV,hd,seqs,groups", [(32, 8, 64, [(0, 40)] * 60, 3), (32, 32, 96, [(0, 100), (30, 40)] * 13, 3), (32, 8, 64, [(700, 40)] * 50, 1)])
+@pytest.mark.parametrize("H,KV,hd,seqs,groups", [(32, 8, 64, [(0, 40)] * 60, 3), (32, 32, 96, [(0, 100), (30, 40)] * 13, 3), (8, 8, 128, [(0, 90 + i) for i in range(50)], 3),
+                                                 (32, 8, 64, [(700, 40)] * 50, 1)])
 def test_many_sequences_as_planned(hip, H, KV, hd, seqs, groups):  # noqa: F811
     plan = hip.describe_plan(H, KV, hd, [c for c, _ in seqs], [n for _, n in seqs])
     assert plan["groups"] == groups, plan

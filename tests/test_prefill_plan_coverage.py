@@ -65,6 +65,15 @@ def test_batches_of_short_sequences_have_a_group_for_each_row_block():
         assert plan["workgroups"] == (blocks if groups == 3 else pairs) * KV * plan["key_chunks"], plan
 
 
+def test_short_ranges_are_not_shared_by_two_groups():
+    for H, KV, hd, B, cached, new, groups in [
+            (32, 8, 64, 1, 0, 45, 3), (32, 8, 64, 1, 0, 128, 3), (32, 8, 64, 1, 0, 129, 2), (32, 8, 64, 1, 80, 45, 3), (32, 8, 64, 1, 90, 45, 2),
+            (32, 8, 128, 1, 0, 96, 3), (32, 8, 128, 1, 0, 97, 2), (32, 8, 64, 16, 0, 100, 3), (32, 8, 64, 8, 0, 256, 3), (32, 8, 64, 8, 0, 300, 2),
+            (32, 8, 128, 16, 0, 100, 3), (32, 8, 64, 1, 2000, 40, 2)]:
+        plan = sa.describe_plan(H, KV, hd, [cached] * B, [new] * B)
+        assert plan["groups"] == groups, (H, KV, hd, B, cached, new, plan)
+
+
 def test_decode_and_generic_paths_are_told_apart():
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [1] * 16)["path"] == sa.hip.PATH_DECODE
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [8] * 16)["path"] == sa.hip.PATH_DECODE  # two entries each
