@@ -1049,22 +1049,24 @@ int prefill_key_splits(const SeqTable &st, const Shape &sh, int items) {
   const int ns_1024 = (int)((1024 + wgs - 1) / wgs);
   if (longest / ns_1024 >= 32) return ns_1024 < 16 ? ns_1024 : 16;
   // Otherwise what is estimated to end first, in times of a key tile: a compute unit has one workgroup at a time, which costs three tiles beside
-  // its own; the launch that merges costs six for two chunks and one and a half for each further one (heads over 64, whose tiles take longer: four and a
-  // half, one and a quarter).
+  // its own; the launch that merges costs three and one and a half for each chunk, half of that where it has few rows (heads over 64, whose tiles take
+  // longer: two, one and a quarter).
   // Us, chunks by a target of 512 workgroups | these: 32 / 8 heads of 64, 800 rows 49 | 41, 200 on 2000 46 | 37, 400 on 4000 113 | 89; heads of 128, 800 rows 86 | 73,
-  // 32 / 4 heads, 512 on 4096 214 | 181; heads of 96, 777 rows 70 | 59.
+  // 32 / 4 heads, 512 on 4096 214 | 181; heads of 96, 777 rows 70 | 59.  Few rows, as many chunks as of many | these: 32 / 8 heads of 64, 17 on 2000 26.8 | 24.3, 40 on 2000
+  // 28.4 | 26.2, 40 on 8000 48.1 | 46.2.
   double blocks = 0, tiles = 0;
   for (int s = 0; s < st.n_seqs; ++s) {
     const double n = (st.n_new[s] * (double)sh.g + 127) / 128;
     blocks += n;
     tiles += n * ((st.start_pos[s] + st.n_new[s] * 0.5) / 32 + 1);
   }
+  const double a_chunk = wgs < 128 ? 0.75 + 0.75 * wgs / 128 : 1.5;
   const int cap = longest / 8;  // at least eight key tiles per chunk
   int best = 1;
   double least = 0;
   for (int ns = 1; ns == 1 || (ns <= cap && ns <= 16); ++ns) {
     const double rounds = (double)((wgs * ns + 255) / 256), one = (longest + ns - 1) / ns + 3, all = rounds * (tiles / blocks / ns + 3);
-    const double ends = (one > all ? one : all) + (ns == 1 ? 0 : sh.hd <= 64 ? 3 + 1.5 * ns : 2 + 1.25 * ns);
+    const double ends = (one > all ? one : all) + (ns == 1 ? 0 : sh.hd <= 64 ? 3 + a_chunk * ns : 2 + 1.25 * ns);
     if (ns == 1 || ends < least) {
       least = ends;
       best = ns;

@@ -65,6 +65,12 @@ def test_batches_of_short_sequences_have_a_group_for_each_row_block():
         assert plan["workgroups"] == (blocks if groups == 3 else pairs) * KV * plan["key_chunks"], plan
 
 
+def test_few_rows_on_many_are_cut_into_more_chunks():
+    # the launch that merges them is short: one chunk more costs it half as much as of many rows
+    for cached, new, chunks in [(2000, 17, 8), (2000, 40, 8), (8000, 40, 16), (2000, 200, 4), (4000, 400, 2)]:
+        assert sa.describe_plan(32, 8, 64, [cached], [new])["key_chunks"] == chunks, (cached, new)
+
+
 def test_short_ranges_are_not_shared_by_two_groups():
     for H, KV, hd, B, cached, new, groups in [
             (32, 8, 64, 1, 0, 45, 3), (32, 8, 64, 1, 0, 128, 3), (32, 8, 64, 1, 0, 129, 2), (32, 8, 64, 1, 80, 45, 3), (32, 8, 64, 1, 90, 45, 2),
