@@ -470,10 +470,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
 // which are requested behind them.
 // What bounds it: on zeros 2048 rows of 2048 -> 16384 (x itself) take 279 us, of which the MFMAs and fragments are 201, splits 26, writes to LDS 31 (17
 // cycles each while MFMAs run) and loads 21; on random numbers the clock is at 2.06 GHz.
-template <int WM, bool GUARD, bool SWIGLU, bool PLANES>
+// END: K ends with a step (kWhole; PLANES always); within one (kShifted): the last step is moved back until it ends with K, and what the steps before it
+// have had of x counts as zeros, so that no load hangs on a condition; or within the only one (kGuarded).  Us, every load behind a condition | this:
+// 512 rows of 2064 -> 16384 141 | 126, 777 rows of 1040 -> 16384 103 | 95, 1100 rows of 4112 -> 1028 58.5 | 49.8, 2048 rows of 2064 -> 2048 78.5 | 66.5, 8208 -> 2048
+// 193 | 171, 512 rows of 2060 -> 16384 130 | 116, 1300 rows of 36 -> 16380 41.4 | 28.4.
+constexpr int kWhole = 0, kShifted = 1, kGuarded = 2;
+template <int WM, int END, bool SWIGLU, bool PLANES>
 __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
   constexpr int WN = 8 / WM, MB = 4, NB = 2 * WM, TM = 64 * WM, TN = 256, NT = 512;
-  static_assert(!(GUARD && PLANES), "planes hold whole steps");
+  constexpr bool GUARD = END == kGuarded;
+  static_assert(END == kWhole || !PLANES, "planes hold whole steps");
   constexpr int NX = WM / 2;               // octets of x a thread stages (of W: two); PLANES: 16 rows of a part that a wavefront copies
   constexpr int kSets = WM == 4 ? 1 : 2;   // register sets: tiles are requested one step (of 3072 cycles) ahead, or two (of 1536)
   // units of 16 bytes; blocks of W a few units apart from 16, so that eight neighbouring threads' columns lie on eight different ones modulo 8
@@ -507,6 +513,7 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     const int m0 = tm * TM, n0 = tn * TN;
     const int k_begin = s_begin * kWideStep, k_end = min(K, s_end * kWideStep);
     const int nk = s_end - s_begin;
+    const int had = END == kShifted && s_end == steps ? steps * kWideStep - K : 0;  // of the last step's k
 
     int tid = threadIdx.x;  // (worked out again per tile, as above)
     asm volatile("" : "+v"(tid));
@@ -537,12 +544,19 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) w_row[i] = (unsigned)(((long long)(wk + i) * N + w_from) * 4);
-    const char *x_base = PLANES ? (const char *)(g.planes + (long long)k_begin * T) : (const char *)(g.x + k_begin), *w_base = (const char *)(g.w + (long long)k_begin * N);
+    const int k_first = k_begin - (nk == 1 ? had : 0);
+    const char *x_base = PLANES ? (const char *)(g.planes + (long long)k_begin * T) : (const char *)(g.x + k_first), *w_base = (const char *)(g.w + (long long)k_first * N);
     const long long plane = 2LL * T * K;
 
     f32x4 sx[kSets][NX][2];
     float sw[kSets][2][8];
-    int k_next = k_begin, to_load = nk, to_copy = nk;
+    int k_next = k_begin, to_load = nk, to_copy = nk, to_split = nk;
+    float lift[2];  // (kShifted) of an octet's halves
+    auto set_lift = [&]() {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) lift[h] = to_split == 1 && xk + 4 * h < had ? 0.f : kLift;
+    };
+    if constexpr (END == kShifted) set_lift();
     auto load_x = [&](const int set, const int u, const int h) {
       if constexpr (!PLANES) sx[set][u][h] = GUARD && k_next + xk + 4 * h >= k_end ? f32x4{0.f, 0.f, 0.f, 0.f} : load_from((const f32x4 *)(x_base + 16 * h), x_off[u]);
     };
@@ -551,8 +565,9 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     };
     auto advance = [&]() {
       if (--to_load > 0) {  // (behind the last step its tiles are requested again: the loop has no conditions)
-        if constexpr (!PLANES) x_base += kWideStep * 4;
-        w_base += (long long)kWideStep * N * 4;
+        const int by = kWideStep - (to_load == 1 ? had : 0);
+        if constexpr (!PLANES) x_base += by * 4;
+        w_base += (long long)by * N * 4;
         k_next += kWideStep;
       }
     };
@@ -576,8 +591,8 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
         } else if (m >= 16) {
           stage[x_unit + 128 * u + (m - 16) * kPartX] = whole[m - 16];
         } else if (m % 4 == 0) {
-          pa = sx[set][u][i / 2][i % 2 * 2] * kLift;
-          pb = sx[set][u][i / 2][i % 2 * 2 + 1] * kLift;
+          pa = sx[set][u][i / 2][i % 2 * 2] * (END == kShifted ? lift[i / 2] : kLift);
+          pb = sx[set][u][i / 2][i % 2 * 2 + 1] * (END == kShifted ? lift[i / 2] : kLift);
           whole[0][i] = pack_bf16(pa, pb);
         } else if (m % 4 == 1) {
           pa -= __builtin_bit_cast(float, whole[0][i] << 16);
@@ -598,7 +613,10 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
         else
           whole[0][m] = pack_high(sw[set][o][2 * m] * kLift, sw[set][o][2 * m + 1] * kLift);
       }
-      if (it == kItems - 1) advance();
+      if (it == kItems - 1) {
+        advance();
+        if constexpr (END == kShifted) --to_split, set_lift();
+      }
     };
     auto load_all = [&](const int set) {
 #pragma unroll
@@ -1689,16 +1707,23 @@ hipError_t launch_tiles(const GemmArgs &g, const GemmPlan &p, const GemmNext &ne
 template <int WM, bool PLANES>
 hipError_t launch_wide(const GemmArgs &g, const GemmPlan &p, const GemmNext &next, hipStream_t stream) {
   const dim3 grid((unsigned)p.workgroups);
-  const bool guard = g.K % kWideStep != 0, swiglu = next.swiglu && !g.pieces;
-  if (guard && PLANES) return hipErrorInvalidValue;
-  if (swiglu && guard)
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, !PLANES, true, PLANES>), grid, dim3(512), 0, stream, g);
-  else if (swiglu)
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, true, PLANES>), grid, dim3(512), 0, stream, g);
-  else if (guard)
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, !PLANES, false, PLANES>), grid, dim3(512), 0, stream, g);
+  const bool swiglu = next.swiglu && !g.pieces;
+  const int end = g.K % kWideStep == 0 ? kWhole : g.K > kWideStep ? kShifted : kGuarded;
+  if (end != kWhole && PLANES) return hipErrorInvalidValue;
+#define SHAINET_WIDE_LAUNCH(END_)                                                                          \
+  do {                                                                                                     \
+    if (swiglu)                                                                                            \
+      hipLaunchKernelGGL((sgemm_wide_kernel<WM, END_, true, PLANES>), grid, dim3(512), 0, stream, g);      \
+    else                                                                                                   \
+      hipLaunchKernelGGL((sgemm_wide_kernel<WM, END_, false, PLANES>), grid, dim3(512), 0, stream, g);     \
+  } while (0)
+  if (end == kWhole)
+    SHAINET_WIDE_LAUNCH(kWhole);
+  else if (end == kShifted)
+    SHAINET_WIDE_LAUNCH(PLANES ? kWhole : kShifted);
   else
-    hipLaunchKernelGGL((sgemm_wide_kernel<WM, false, false, PLANES>), grid, dim3(512), 0, stream, g);
+    SHAINET_WIDE_LAUNCH(PLANES ? kWhole : kGuarded);
+#undef SHAINET_WIDE_LAUNCH
   const hipError_t e = hipGetLastError();
   return e != hipSuccess || !g.pieces ? e : launch_sum<2 * WM>(g, PieceShape{64 * WM, 256, 64, 8 / WM, 512}, next, stream);
 }

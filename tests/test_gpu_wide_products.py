@@ -32,3 +32,35 @@ def test_wide_products_against_64_bits(T, K, N, tile, pieces, waits):
         for dim in (0, 1):
             off = float(((got.double() - want).norm(dim=dim) / want.norm(dim=dim)).max())
             assert off <= 2 * (3 * K / 32 + 4) ** 0.5 * 2.0 ** -24, off
+
+
+@pytest.mark.parametrize("T,K,N", [(257, 20, 8204), (1300, 28, 16380), (1300, 36, 16380), (257, 48, 8204), (2000, 60, 8188)])
+def test_products_that_end_within_their_first_or_second_step(T, K, N):
+    test_wide_products_against_64_bits(T, K, N, 128, False, False)
+
+
+@pytest.mark.parametrize("T,K,N", [(257, 28, 8204), (257, 52, 8204), (777, 1040, 16384), (1100, 4100, 1028), (3000, 548, 8204)])
+def test_last_step_and_what_is_not_finite(T, K, N):
+    """Values that are not finite, or too large to be lifted, among the last 32 of K, those counted in the last step and those that the step before it
+    had: a sum they take part in is what fp32 makes of it, every other one as if they were not there."""
+    import torch
+
+    import shainet_amd as sa
+    from shainet_amd import hip
+
+    assert sa.HIP.fully_available()
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn((T, K), generator=g, device="cuda")
+    w = torch.randn((K, N), generator=g, device="cuda").bfloat16().float()
+    for i, value in enumerate([float("inf"), float("nan"), -float("inf"), 2.0 ** 120]):
+        k = K - 1 - (9 * i) % min(K, 32)
+        x[5 + 50 * i, k] = value
+        w[k, 7 + 100 * i] = value
+    got = hip.matmul(x, w, bf16_weights=True)
+    want = x.cpu().double() @ w.cpu().double()
+    got = got.cpu().double()
+    finite = want.abs() < 3e38
+    assert torch.equal(got[finite].isfinite(), torch.ones(int(finite.sum()), dtype=torch.bool))
+    assert torch.equal(got.isnan()[~finite], want.isnan()[~finite]) and not got[~finite].isfinite().any()
+    # (K terms of size 1, taken again one after the other, round K^0.5 times at random by 2^-25 of a sum of K^0.5; the worst of 10^7 is 6 of these)
+    assert float((got - want)[finite & (want.abs() < 2.0 ** 100)].abs().max()) <= 6 * K * 2.0 ** -24
