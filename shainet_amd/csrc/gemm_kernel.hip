@@ -1567,7 +1567,7 @@ void describe_gemm(const GemmPlan &p, int K, int plan[7]) {
   plan[3] = p.workgroups;
   plan[4] = p.pieces > 1 ? p.pieces : 1;
   plan[5] = p.flag_words && p.quota % p.steps != 0;
-  plan[6] = p.mfma && K % (p.few ? step_k(p) : TK) != 0;
+  plan[6] = p.mfma && K % step_k(p) != 0;
 }
 
 bool gemm_takes_planes(const GemmPlan &p, int K) { return p.mfma && p.parts == 1 && !p.few && K % kWideStep == 0; }

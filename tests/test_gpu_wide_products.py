@@ -22,6 +22,7 @@ def test_wide_products_against_64_bits(T, K, N, tile, pieces, waits):
     assert sa.HIP.fully_available()
     plan = hip.describe_matmul(T, K, N, bf16_weights=True)
     assert (plan["kind"], plan["tile"], plan["pieces"] > 1, plan["waits"]) == ("tiles", (tile, 256), pieces, waits), plan
+    assert plan["ragged_k"] == (K % 32 != 0), plan
     g = torch.Generator(device="cuda").manual_seed(T + K + N)
     x = torch.randn((T, K + 4), generator=g, device="cuda")[:, :K]  # (rows of x need not be dense)
     w = torch.randn((K, N), generator=g, device="cuda").bfloat16().float()

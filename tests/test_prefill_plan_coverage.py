@@ -196,3 +196,12 @@ def test_no_more_rows_than_a_grid_has_are_cut_into_pieces():
     for T, K, N, bf16 in itertools.product((65536, 65537, 100000, 131072, 500000, 1 << 21), (4, 64, 100, 1024, 8192, 32768),
                                            (4, 32, 100, 132, 512, 1024, 3072, 16384), (False, True)):
         assert sa.hip.describe_matmul(T, K, N, bf16_weights=bf16)["pieces"] == 1, (T, K, N, bf16)
+
+
+def test_ragged_k_is_told_by_the_steps_of_the_kernel():
+    # large tiles take 32 of K at a time where the weights are bf16 numbers, 16 where they are not
+    for T, N in ((512, 16384), (2000, 8188), (1100, 1028), (3000, 8204)):
+        for K in (1008, 1024, 1040, 1044, 4112):
+            for bf16, step in ((True, 32), (False, 16)):
+                plan = sa.hip.describe_matmul(T, K, N, bf16)
+                assert plan["kind"] == "tiles" and plan["ragged_k"] == (K % step != 0), (T, K, N, bf16, plan)
