@@ -95,7 +95,7 @@ BF16_MATMULS = [
     (1300, 36, 16380, ("tiles", (128, 256), False, False, True)),
     (400, 640, 8200, ("tiles", (128, 256), False, True, False)),
     (200, 1044, 16384, ("tiles", (128, 256), False, True, True)),
-    (1000, 1024, 1028, ("tiles", (128, 256), True, False, False)),
+    (1100, 4096, 1028, ("tiles", (128, 256), True, False, False)),
     (1000, 1040, 1028, ("tiles", (128, 256), True, False, True)),
     (300, 1044, 4092, ("tiles", (128, 256), True, False, True)),
     (2000, 640, 8188, ("tiles", (256, 256), False, False, False)),
