@@ -186,6 +186,8 @@ struct Projector {
   // go to a second set of words nobody reads and waits end after 2000 polls, so that the report
   // of a given-up wait can be exercised without hanging anything
   bool lose_marks = false;
+  // SHAINET_HIP_TEST_NO_ROWS_AS_PARTS (read when the first such rows are to be written): as if there were no memory for them
+  bool no_parts = false, asked_parts = false;
   // where the split products' kernels report a given-up wait: the owner's pinned host word
   int *error = nullptr;
   // returns a SHAINET_HIP_* status; the message is left for shainet_hip_last_error
@@ -195,6 +197,7 @@ struct Projector {
 
  private:
   int reserve_flags(size_t n_flags, hipStream_t stream);
+  bool reserve_parts(DevF &to, size_t n);
   // res != nullptr: y = res + x W
   int gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N, hipStream_t stream, bool w_bf16,
            const float *res = nullptr, const float *bias = nullptr, Activation act = Activation(), bool swiglu = false, Handover *next = nullptr,

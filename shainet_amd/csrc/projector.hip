@@ -134,6 +134,13 @@ int Projector::reserve_flags(size_t n_flags, hipStream_t stream) {
   return SHAINET_HIP_OK;
 }
 
+// Room for the parts of n floats.  Rows for which there is none stay floats.
+bool Projector::reserve_parts(DevF &to, size_t n) {
+  if (!asked_parts) no_parts = getenv("SHAINET_HIP_TEST_NO_ROWS_AS_PARTS") != nullptr;
+  asked_parts = true;
+  return !no_parts && to.reserve(n / 2 * 3);
+}
+
 // y = (res +) x W with the library's own MFMA kernel; res == y is allowed.
 // swiglu: W is gate | up and y [T, N / 2].
 int Projector::gemm(const float *x, long long x_stride, const float *w, float *y, int T, int K, int N,
@@ -155,9 +162,10 @@ int Projector::gemm(const float *x, long long x_stride, const float *w, float *y
   if (int rc = reserve_flags(p.flag_words, stream)) return rc;
   // (what the product itself needs comes first: without the memory for these rows they are normed in front of the next product, as
   // after one that adds no pieces)
-  const bool as_planes = next && p.parts == 1 && next->n && gemm_takes_planes(plan_gemm(T, N, next->n, N, next->w_bf16), N);
-  if (next && next->norm->kind != kNormNone && !bias && aligned && gemm_takes_next(p, T, N, also) &&
-      handed.reserve((size_t)T * N / 2 * (as_planes ? 3 : 2))) {
+  const bool takes_norm = next && next->norm->kind != kNormNone && !bias && aligned && gemm_takes_next(p, T, N, also);
+  const bool as_planes = takes_norm && p.parts == 1 && next->n && gemm_takes_planes(plan_gemm(T, N, next->n, N, next->w_bf16), N) &&
+                         reserve_parts(handed, (size_t)T * N);
+  if (takes_norm && (as_planes || handed.reserve((size_t)T * N))) {
     also.norm.kind = next->norm->kind;
     also.norm.gamma = next->norm->gamma;
     also.norm.beta = next->norm->beta;
@@ -288,7 +296,7 @@ int Projector::project(const float *x, long long x_stride, const float *w, float
     // 151 and 131, 512 rows of 2048 -> 3072 32.8 and 30.6; a launch of its own for the parts would take 5 to 8 of these)
     planes = (x_stride & 3) == 0 && !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)f.res | (uintptr_t)f.bias) & 15) &&
              gemm_takes_planes(plan_gemm(T, K, swiglu ? 2 * N : N, K, f.w_bf16), K);
-    planes = planes && normed.reserve((size_t)T * K / 2 * 3);  // (without the memory for them they stay floats)
+    planes = planes && reserve_parts(normed, (size_t)T * K);
     if (!planes && !normed.reserve((size_t)T * K)) return llama_fail(SHAINET_HIP_ERR_ALLOC, "hipMalloc failed");
     e = f.norm == kNormDynTanh ? launch_dyn_tanh(x, x_stride, f.gamma, f.beta, f.alpha, normed.p, T, K, stream, planes)
                                : launch_rmsnorm(x, x_stride, f.gamma, normed.p, T, K, f.eps, stream, planes);

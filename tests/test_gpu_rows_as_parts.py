@@ -34,3 +34,25 @@ def test_rows_as_parts(hip, tmp_path, d, ff, T, tile, scales):  # noqa: F811
     got = model.run_rows(tokens, range(T)).astype(np.float64)
     off = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert off.max() <= 2 * 8196 ** 0.5 * 2.0 ** -24, off.max()
+
+
+@pytest.mark.parametrize("d,ff,T,tile,whole", [(1024, 4096, 301, (128, 256), "pieces"), (512, 8196, 1500, (256, 256), "shared"), (256, 4096, 399, (128, 256), "whole"),
+                                               (2048, 2052, 1500, (256, 256), "pieces"), (512, 4096, 700, (128, 256), "shared"), (512, 8192, 2048, (256, 256), "whole")])
+@pytest.mark.parametrize("scales", [{}, {7: -112, 9: -120}, {3: 106}])
+def test_rows_as_parts_and_as_floats_give_the_same_bits(hip, tmp_path, d, ff, T, tile, whole, scales, monkeypatch):  # noqa: F811
+    """Without memory for the parts both launches that write such rows write floats, and a product that reads floats makes the same parts of them itself.
+    (A part that is swapped, stale or missing is off by 2^-16 of a number at most: the sums' own rounding covers that.)"""
+    plan = hip.hip.describe_matmul(T, d, 2 * ff, bf16_weights=True)
+    assert plan["tile"] == tile and whole == ("pieces" if plan["pieces"] > 1 else "shared" if plan["waits"] else "whole"), plan
+    cfg, w = llama(d, ff, 260, d + T)
+    tokens = np.random.default_rng(1).integers(0, 260, T)
+    for p in ("model.layers.0.", "model.layers.1."):
+        for column, power in scales.items():
+            w[p + "post_attention_layernorm.weight"][column] *= np.float32(2.0 ** power)
+            for name in ("mlp.gate_proj", "mlp.up_proj"):
+                w[p + name + ".weight"][:, column] *= np.float32(2.0 ** -power)
+    folder = write(tmp_path / "m", cfg, w, lambda n: True, nudge=False)
+    parts = hip.HFLoader.load_model(folder).run_rows(tokens, range(T))
+    monkeypatch.setenv("SHAINET_HIP_TEST_NO_ROWS_AS_PARTS", "1")
+    floats = hip.HFLoader.load_model(folder).run_rows(tokens, range(T))
+    assert np.isfinite(parts).all() and np.array_equal(parts, floats)
