@@ -42,6 +42,7 @@
 //           key 4*j + r of the tile, where accumulator register r of S^T lives.
 #include "attn_kernels.hpp"
 #include "lane_quarters.hpp"
+#include "lds_copy.hpp"
 
 #include <math.h>
 #include <stdint.h>
@@ -857,8 +858,7 @@ __global__ __launch_bounds__(256, 1) void decode_rows_kernel(const float *__rest
     for (int i = 0; i < C::NKI; ++i) {  // (as issue_k_tile)
       const int slot = i * 64 + lane, row = slot / C::PPR, piece = slot % C::PPR ^ row;
       const unsigned off = (unsigned)(min(kb[u] + row, last_row) * C::ROW_BYTES + 16 * piece);
-      const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)LDS_PTR(&k_lds[wave][u][i * 1024]));
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(to), "v"(off), "s"(kbase) : "memory");
+      copy_to_lds<true>(&k_lds[wave][u][i * 1024], kbase, off);
     }
   }
 #pragma unroll

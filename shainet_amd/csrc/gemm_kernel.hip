@@ -40,6 +40,7 @@
 #include "gemm_kernel.hpp"
 
 #include "attn_kernels.hpp"
+#include "lds_copy.hpp"
 #include "split_mfma.hpp"
 
 #include <math.h>
@@ -581,8 +582,7 @@ __global__ __launch_bounds__(512, 2) void sgemm_wide_kernel(const GemmArgs g) {
     auto item = [&](const int it, const int set, u32x4 *stage) {
       if (PLANES && it < kItemsX) {
         const int u = it / 3, p = it % 3;
-        const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)(stage + p * kPartX + 64 * (wave + 8 * u)));
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(to), "v"(x_off[u]), "s"(x_base + p * plane) : "memory");
+        copy_to_lds<false>(stage + p * kPartX + 64 * (wave + 8 * u), x_base + p * plane, x_off[u]);
         if (it == kItemsX - 1 && --to_copy > 0) x_base += 64LL * T;
       } else if (it < kItemsX) {
         const int u = it / 21, m = it % 21, i = m / 4;
