@@ -127,8 +127,11 @@ struct TileUnits {
 // G = 3: heads of 64 keep within 168 registers so (three wavefronts on a SIMD); heads of 128 those of 24, or two workgroups would not fit.
 template <int HD, int G>
 constexpr int kThirds = HD == 128 ? (G == 2 ? 4 : 3) : G == 3 ? 2 : 0;
+// In LDS: the tiles' stages, behind them a wavefront's queries after another's.
 template <int HD, int G>
-constexpr int kLdsUnits = (G == 3 ? 1 : 2) * TileUnits<HD>::kTile + (G == 1 ? 8 : 4) * kThirds<HD, G> * 128;
+constexpr int kThirdsAt = (G == 3 ? 1 : 2) * TileUnits<HD>::kTile;
+template <int HD, int G>
+constexpr int kLdsUnits = kThirdsAt<HD, G> + (G == 1 ? 8 : 4) * kThirds<HD, G> * 128;
 static_assert(kLdsUnits<128, 1> * 16 <= 160 * 1024 && kLdsUnits<128, 2> * 16 <= 160 * 1024, "LDS of a compute unit");
 static_assert(2 * kLdsUnits<128, 3> * 16 <= 160 * 1024, "two workgroups of one group share a compute unit");
 
@@ -290,7 +293,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   }
   // the row's query, scaled by scale * log2(e): scores come out in log2 units
   u32x4 qf[KS][2][3];
-  u32x4 *const third = lds + 2 * U::kTile + (G == 1 ? 4 * gidx + wave : wave) * (kThirds<HD, G> * 128) + lane;
+  u32x4 *const third = lds + kThirdsAt<HD, G> + (G == 1 ? 4 * gidx + wave : wave) * (kThirds<HD, G> * 128) + lane;
   bool apart;  // some query of the wavefront needs its scores in fp32
   {
     float least = INFINITY, most = 0.f;

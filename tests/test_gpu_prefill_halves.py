@@ -78,3 +78,56 @@ def test_many_sequences_as_planned(hip, H, KV, hd, seqs, groups):  # noqa: F811
     assert parity.check_step(ctx, cache, blocks, r, [new for _, new in seqs], what=str(seqs[:2])) < 1e-4
     cache.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3])
+@pytest.mark.parametrize("hd,KV,T,cached", [(64, 2, 300, 0), (96, 4, 40, 33), (128, 2, 70, 100)])
+def test_scores_keep_all_24_bits_in_every_layout(hip, hd, KV, T, cached, groups, monkeypatch):  # noqa: F811
+    monkeypatch.setenv("SHAINET_HIP_PREFILL_GROUPS", str(groups))
+    parity.test_prefill_scores_keep_all_24_bits(hip, hd, KV, T, cached)
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3])
+@pytest.mark.parametrize("of_keys", [False, True])
+@pytest.mark.parametrize("hd,KV,T,splits", [(16, 2, 300, 0), (64, 2, 300, 3), (64, 8, 2300, 0), (96, 2, 300, 0), (128, 2, 300, 0), (128, 8, 2300, 0)])
+def test_third_parts_in_every_layout(hip, hd, KV, T, splits, of_keys, groups, monkeypatch):  # noqa: F811
+    """One operand is 1 + 2^-9 + 0.9 x 2^-17 in its even elements, of which the last summand is a bf16 part of its own, the other 1 and
+    -(1 + 2^-9) by turns: what is left of the scores of even keys, 2^18 times 0.9 x 2^-17, comes from third parts alone.  The odd keys have
+    the same score from one product of two leading parts.  A result is a difference of the weights of both, the bound what six products
+    leave out, the sums and the factor of the queries: 2^-23 of the sum of the products' sizes, 2^19, in log2 units.  2300 rows of 8 heads are
+    more workgroups than compute units: nothing pads their LDS."""
+    import numpy as np
+    import torch
+
+    monkeypatch.setenv("SHAINET_HIP_PREFILL_GROUPS", str(groups))
+    if splits:
+        monkeypatch.setenv("SHAINET_HIP_PREFILL_SPLITS", str(splits))
+    H, third = 2 * KV, 0.9 * 2.0 ** -17
+    c = float(np.float32(np.log2(np.e)) * np.float32(1 / np.sqrt(hd)))
+    size = 2.0 ** (13 - int(np.log2(hd)))
+    long, short = np.ones(hd), np.ones(hd)
+    long[0::2] = 1 + 2.0 ** -9 + third
+    short[1::2] = 1 + 2.0 ** -9
+    query, key = (short, long) if of_keys else (long, short)
+    key[1::2] *= -1
+    odd_key = np.zeros(hd)
+    odd_key[1] = hd / 2 * third
+    q = torch.tensor(np.tile(2.0 ** 6 / c * query, (T, H)), dtype=torch.float32, device="cuda")
+    keys = torch.tensor(np.where(np.arange(T)[:, None] % 2, odd_key, key) * size, dtype=torch.float32, device="cuda")
+    values = torch.ones((T, hd), device="cuda")
+    values[1::2] = -1
+    ctx = hip.AttnContext(H, KV, hd, rope_freqs=np.zeros(hd // 2, np.float32), max_positions=T)
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, T)
+    ctx.sync()
+    got = ctx.forward(cache, q, keys.repeat(1, KV), values.repeat(1, KV), [T])
+    ctx.sync()
+    got = got.cpu().numpy().reshape(T, H, hd).astype(np.float64)
+    s = keys.cpu().numpy().astype(np.float64) @ q[0, :hd].cpu().numpy().astype(np.float64) / np.sqrt(hd)  # every row's, every head's
+    sizes = float(np.abs(keys[0].cpu().numpy().astype(np.float64)) @ q[0, :hd].cpu().numpy().astype(np.float64) / np.sqrt(hd))
+    even, odd = np.exp(s[0] - s[:2].max()) * (np.arange(T) // 2 + 1), np.exp(s[1] - s[:2].max()) * ((np.arange(T) + 1) // 2)
+    bound = 0.5 * 2.0 ** -23 * sizes + 1e-5
+    assert 0.5 * (1 - np.exp(-abs(s[0]))) > 8 * bound  # (without those parts an even key's score is 0)
+    assert np.abs(got - ((even - odd) / (even + odd))[:, None, None]).max() <= bound
+    cache.close()
+    ctx.close()
