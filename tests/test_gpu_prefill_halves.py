@@ -131,3 +131,22 @@ def test_third_parts_in_every_layout(hip, hd, KV, T, splits, of_keys, groups, mo
     assert np.abs(got - ((even - odd) / (even + odd))[:, None, None]).max() <= bound
     cache.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3])
+@pytest.mark.parametrize("splits", [0, 3])
+@pytest.mark.parametrize("name", ["even", "narrow_values", "wide_values", "large"])
+def test_values_by_distance_in_every_layout(hip, tmp_path, name, splits, groups, monkeypatch):  # noqa: F811
+    """290 rows of one and of two heads a key's: 3 and 5 row blocks, rows on both sides of the table's reach."""
+    import numpy as np
+    import test_gpu_zabutar as zabutar
+
+    monkeypatch.setenv("SHAINET_HIP_PREFILL_GROUPS", str(groups))
+    if splits:
+        monkeypatch.setenv("SHAINET_HIP_PREFILL_SPLITS", str(splits))
+    cfg, rows = zabutar.attention_config(name)
+    p = zabutar.Pair(hip, tmp_path, cfg, rel_rows=rows)
+    x = np.random.default_rng(5).standard_normal((290, cfg["width"])).astype(np.float32)
+    want, b = p.layer(0, x), p.model.blocks[0]
+    zabutar.close(b.forward_cached(x), want)
+    zabutar.close(zabutar.block_cut(b, x, (33, 257)), want)
