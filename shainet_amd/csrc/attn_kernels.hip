@@ -1040,28 +1040,7 @@ static bool table_ok(const SeqTable &st, const Shape &sh) {
   return true;
 }
 
-// Heads of 64, prompts of more row blocks than half of the compute units and up to three quarters of them (520 to 760 rows of 32 / 8 heads): a block
-// each leaves the others idle, two chunks of each are a second round that is half empty.  Four chunks, of which a workgroup of one group takes one and a
-// compute unit two or three, fill it in one.  Only where most of the keys are new: of blocks of one length some units have two and others three.
-// Us, one or two chunks before the groups moved apart | since | these: 32 / 8 heads, 520 rows 29.9 | 30.7 | 28.9, 576 rows 32.3 | 33.4 | 31.0, 620 rows 33.5 | 33.9
-// | 31.6, 700 rows 36.1 | 36.4 | 34.8, 765 rows 46.8 | 38.5 | 35.7; 620 rows of heads of 48 31.4 | 32.3 | 30.0; 16 / 8 heads, 1090 rows 48.3 | 42.8 | 37.5; 32 / 32
-// heads, 600 rows 35.5 | 35.6 | 33.1; three chunks 31.9 and 36.4 at 576 and 700 rows, five 31.2 and 35.0; 640 rows on 2000 81.7 since | 84.7.
-// With values by distance only two such workgroups share a unit: a prompt of 520 to 760 rows of width 2048 took up to 1 % longer.
-constexpr int kChunksOfOneGroup = 4;
-static bool chunks_of_one_group(const SeqTable &st, const Shape &sh, int items, int v_hd) {
-  const long long blocks = (long long)items * sh.KV;
-  if (v_hd || prefill_tile_head_dim(sh.hd) != 64 || blocks <= 128 || blocks > 192) return false;
-  int longest = 0;
-  double tiles = 0;
-  for (int s = 0; s < st.n_seqs; ++s) {
-    const int n = (st.start_pos[s] + st.n_new[s] + 31) / 32;
-    longest = n > longest ? n : longest;
-    tiles += st.work_off[s] * ((st.start_pos[s] + 0.5 * st.n_new[s]) / 32 + 1);
-  }
-  return longest >= 4 * kChunksOfOneGroup && tiles <= 0.75 * longest * items;
-}
-
-int prefill_key_splits(const SeqTable &st, const Shape &sh, int items, int v_hd) {
+int prefill_key_splits(const SeqTable &st, const Shape &sh, int items) {
   const long long wgs = (long long)items * sh.KV;
   if (wgs >= 384) return 1;
   int longest = 0;  // key tiles of the longest row block
@@ -1084,7 +1063,6 @@ int prefill_key_splits(const SeqTable &st, const Shape &sh, int items, int v_hd)
     blocks += n;
     tiles += n * ((st.start_pos[s] + st.n_new[s] * 0.5) / 32 + 1);
   }
-  if (chunks_of_one_group(st, sh, items, v_hd)) return kChunksOfOneGroup;
   const double a_chunk = wgs < 128 ? 0.75 + 0.75 * wgs / 128 : 1.5;
   const int cap = longest / 8;  // at least eight key tiles per chunk
   int best = 1;
@@ -1136,8 +1114,7 @@ PrefillLaunch plan_prefill_launch(const SeqTable &st, const Shape &sh, int items
       // has walked through in the time of the two groups' merge, and of which two or three share a compute unit.  Us, two groups | one: 32 / 8 heads
       // of 64, 20 rows 10.0 | 8.6, 45 rows 10.6 | 9.7, 100 rows 13.1 | 12.2, 128 rows 14.1 | 14.3, 200 rows 16.2 | 17.7; heads of 128, 45 rows 14.2 | 12.4, 64 rows
       // 16.0 | 14.8, 128 rows 19.5 | 20.3; more than 256 blocks: 16 sequences of 100 rows 24.7 | 16.5 and 40 | 24.6, 8 of 200 rows 27.4 | 22.6 and 40.6 | 33.9.
-      if (ns == 1 ? longest <= (p.n_wgs > 256 ? 8 : tile_hd == 64 ? 4 : 3) : ns == kChunksOfOneGroup && chunks_of_one_group(st, sh, items, v_hd))
-        p.groups = 3;
+      if (ns == 1 && longest <= (p.n_wgs > 256 ? 8 : tile_hd == 64 ? 4 : 3)) p.groups = 3;
     } else {
       // More: two blocks a workgroup, which share a tile's splits and of whose groups one has MFMAs while the other has none, or a workgroup a block,
       // two or three on a compute unit, which start and end beside each other and leave no half empty where a sequence has an odd block.  What is
@@ -1187,7 +1164,7 @@ hipError_t launch_prefill(const float *q_rot, const float *kc, const float *vc, 
   if (bias && (!db.tab || (v_hd & 3) || (db.q_stride & 3) || v_hd < 4 || (long long)sh.cap * v_hd * 4 > 0xffffffffLL)) return hipErrorInvalidValue;
   if (!table_ok(st, sh) || !tile_hd || !prefill_tile_head_dim(sh.hd) || items < 1 || ns < 1 || (ns > 1 && !partials)) return hipErrorInvalidValue;
   const bool pad = tile_hd != sh.hd;
-  const PrefillLaunch plan = plan_prefill_launch(st, sh, items, ns, wgs_per_cu, groups_wanted, bias ? v_hd : 0);
+  const PrefillLaunch plan = plan_prefill_launch(st, sh, items, ns, wgs_per_cu, groups_wanted, v_hd);
   const long long n_wgs = plan.n_wgs;
   if (n_wgs > 0x7fffffffLL) return hipErrorInvalidValue;
   // the kernels address a row of a (sequence, kv head) by a 32-bit byte offset from its first row

@@ -174,7 +174,7 @@ bool decode_prepares(const PrepArgs &a, const SeqTable &st, const Shape &sh, con
 // Key splits of a prefill launch: 1 when the row blocks alone fill the chip, more
 // when they do not (few new rows on a long cached prefix); each split leaves
 // partial rows in `partials` (prefill_partial_floats) and a second kernel merges.
-int prefill_key_splits(const SeqTable &st, const Shape &sh, int items, int v_hd = 0);  // v_hd: of values by distance (0: none)
+int prefill_key_splits(const SeqTable &st, const Shape &sh, int items);
 size_t prefill_partial_floats(const Shape &sh, int items, int ns, int v_hd = 0);
 // The head dimension the MFMA prefill kernel lays its tiles out for when the data's is hd: 64 or
 // 128, the first that holds hd (a multiple of 4); 0 when neither does.

@@ -313,7 +313,7 @@ int run_attention(shainet_attn_ctx *c, const float *q_rot, float *kc, float *vc,
     }
     if (path == Path::kPrefillMfma) {
       const int items = plan_work(st, sh, path);
-      int ns = c->prefill_splits_override > 0 ? c->prefill_splits_override : prefill_key_splits(st, sh, items, bias ? v_hd : 0);
+      int ns = c->prefill_splits_override > 0 ? c->prefill_splits_override : prefill_key_splits(st, sh, items);
       int rc = c->partials.reserve(prefill_partial_floats(sh, items, ns, v_hd));
       if (rc) return rc;
       e = launch_prefill(q_rot, kc, vc, out, c->partials.p, st, sh, items, ns, scale, stream,

@@ -16,7 +16,6 @@ CASES = [
     ("llama1b_prefill_t8192", 32, 8, 64, False, 0, 8192, (64, False, 1, 0)),
     ("llama1b_prefill_t2560", 32, 8, 64, False, 0, 2560, (64, False, 2, 0)),
     ("llama1b_prefill_t1024", 32, 8, 64, False, 0, 1024, (64, True, 2, 0)),
-    ("llama1b_prefill_t600", 32, 8, 64, False, 0, 600, (64, True, 3, 0)),
     ("llama1b_prefill_t45", 32, 8, 64, False, 0, 45, (64, False, 3, 0)),
     ("qwen3_8b_prefill_t45", 32, 8, 128, True, 0, 45, (128, False, 3, 0)),
     ("w1024_chunked_prefill_t2560_on_1000", 16, 2, 64, False, 1000, 2560, (64, True, 3, 0)),

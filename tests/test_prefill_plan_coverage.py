@@ -80,18 +80,6 @@ def test_short_ranges_are_not_shared_by_two_groups():
         assert plan["groups"] == groups, (H, KV, hd, B, cached, new, plan)
 
 
-def test_prompts_of_half_to_three_quarters_of_the_compute_units_are_cut_for_one_group():
-    # a block each, or two chunks of each, would leave up to half of the compute units idle
-    for H, KV, hd, cached, new, chunks, groups in [
-            (32, 8, 64, 0, 512, 2, 2), (32, 8, 64, 0, 513, 4, 3), (32, 8, 64, 0, 620, 4, 3), (32, 8, 64, 0, 768, 4, 3), (32, 8, 64, 0, 769, 2, 2),
-            (32, 8, 48, 0, 620, 4, 3), (16, 8, 64, 0, 1200, 4, 3), (32, 32, 64, 0, 600, 4, 3), (32, 8, 64, 250, 600, 4, 3), (32, 8, 64, 2000, 640, 3, 2),
-            (32, 8, 128, 0, 620, 2, 2)]:
-        plan = sa.describe_plan(H, KV, hd, [cached], [new])
-        assert (plan["key_chunks"], plan["groups"]) == (chunks, groups), (H, KV, hd, cached, new, plan)
-        if groups == 3:
-            assert plan["workgroups"] == -(-new * (H // KV) // 128) * KV * 4 <= 768 and plan["turns"] == 0, plan
-
-
 def test_decode_and_generic_paths_are_told_apart():
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [1] * 16)["path"] == sa.hip.PATH_DECODE
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [8] * 16)["path"] == sa.hip.PATH_DECODE  # two entries each
