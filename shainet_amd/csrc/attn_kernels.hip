@@ -351,6 +351,15 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int b = 0; b < 2; ++b) o[t][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // O is a chain of sums, in which each of a tile's six products would be rounded to O's last place: twice the error of one rounding a tile (relative
+  // to 64 bits, 400 rows on 4000, 32 / 8 heads of 64, 5.4e-7 | 2.8e-7; 512 on 4096, 32 / 4 heads of 128, 6.1e-7 | 3.6e-7).
+  // kTwoSums: the five smaller products have a sum of their own, for which heads of 64 have the registers (2048 rows 97.4 | 97.6 us, 8192 rows 1156 | 1151).
+  // kOwnSum: a tile's products are added up before they join O (a sum more beside each six MFMAs: heads of 128, 2048 rows 192 | 193.5 us, 800 rows 71.9 | 73.1).
+  // Heads of 128 in two blocks a workgroup have neither: it would take 4 to 5 % (512 on 16384 558 | 586 us).  Nor have ranges of a few tiles.
+  constexpr bool kTwoSums = HD == 64 && G != 3, kOwnSum = G == 3 ? SPLIT : HD == 128 && G == 2;
+  f32x4 low[kTwoSums ? NT : 1][2];
+#pragma unroll
+  for (int t = 0; t < (kTwoSums ? NT : 1); ++t) low[t][0] = low[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   // A step of a group has two halves: MFMAs (O^T += V^T(sp - 1) P^T(sp - 1), scores of tile sp) and everything else (softmax of tile sp, P
   // split, V(sp) and K(sp + 1) parked, the next requested), a barrier behind each.  The second group is half a step behind: while a SIMD's
   // one wavefront has MFMAs only, its other one has none.  G = 2: each group stages its own tiles, one of K and one of V.  G = 1: both stage
@@ -463,6 +472,10 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
           l[b] *= alpha;
 #pragma unroll
           for (int t = 0; t < NT; ++t) o[t][b] *= alpha;
+          if constexpr (kTwoSums) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) low[t][b] *= alpha;
+          }
         }
       }
     }
@@ -483,6 +496,7 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
   auto outputs = [&](int sp) {  // O^T += V^T P^T
     const u32x4 *const vl = lds + v_at + (G == 1 && sp & 1 ? U::kTile : 0);
     u32x4 fr[2][3];
+    f32x4 before;  // (kOwnSum) the last block's sum, which joins O while the next one's MFMAs run
 #pragma unroll
     for (int w = 0; w < 3; ++w) fr[0][w] = vl[w * U::kPartV];
 #pragma unroll
@@ -493,11 +507,24 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < 2; ++b) {
+        if constexpr (kOwnSum) {
+          f32x4 own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < 6; ++w) o[t][b] = mfma_bf16_16(fr[t & 1][kPartA[w]], pf[b][kPartB[w]], o[t][b]);
+          for (int w = 0; w < 6; ++w) own = mfma_bf16_16(fr[t & 1][kPartA[w]], pf[b][kPartB[w]], own);
+          if (t + b > 0) o[b ? t : t - 1][b ^ 1] += before;
+          before = own;
+        } else {
+#pragma unroll
+          for (int w = 0; w < 6; ++w) {
+            f32x4 &to = kTwoSums && w < 5 ? low[t][b] : o[t][b];
+            to = mfma_bf16_16(fr[t & 1][kPartA[w]], pf[b][kPartB[w]], to);
+          }
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (kOwnSum) o[NT - 1][1] += before;
   };
   if (n_sp > 0) {
     park_k(0);
@@ -552,6 +579,12 @@ __device__ __forceinline__ void prefill_block(const int bid, const float *__rest
     if (!kScoresFirst && sp < n_mine) outputs(sp);
   }
   if (gidx == 0 && half_apart) __syncthreads();
+  if constexpr (kTwoSums) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) o[t][b] += low[t][b];
+  }
 
   // Some results are taken again, tile by tile in fp32:
   //   results that are not finite come from operands that are not, and fp32 says which (8192 rows, 32 / 8 heads of 64, NaN
@@ -1063,11 +1096,12 @@ int prefill_key_splits(const SeqTable &st, const Shape &sh, int items) {
     blocks += n;
     tiles += n * ((st.start_pos[s] + st.n_new[s] * 0.5) / 32 + 1);
   }
+  // (heads over 64: not so many that two blocks share a workgroup, which walks through a whole range there with six roundings a tile)
   const double a_chunk = wgs < 128 ? 0.75 + 0.75 * wgs / 128 : 1.5;
   const int cap = longest / 8;  // at least eight key tiles per chunk
   int best = 1;
   double least = 0;
-  for (int ns = 1; ns == 1 || (ns <= cap && ns <= 16); ++ns) {
+  for (int ns = 1; ns == 1 || (ns <= cap && ns <= 16 && (sh.hd <= 64 || wgs * ns <= 768)); ++ns) {
     const double rounds = (double)((wgs * ns + 255) / 256), one = (longest + ns - 1) / ns + 3, all = rounds * (tiles / blocks / ns + 3);
     const double ends = (one > all ? one : all) + (ns == 1 ? 0 : sh.hd <= 64 ? 3 + a_chunk * ns : 2 + 1.25 * ns);
     if (ns == 1 || ends < least) {

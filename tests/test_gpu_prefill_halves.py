@@ -150,3 +150,39 @@ def test_values_by_distance_in_every_layout(hip, tmp_path, name, splits, groups,
     want, b = p.layer(0, x), p.model.blocks[0]
     zabutar.close(b.forward_cached(x), want)
     zabutar.close(zabutar.block_cut(b, x, (33, 257)), want)
+
+
+@pytest.mark.parametrize("H,KV,hd,T,cached,chain", [(32, 8, 64, 400, 4000, 35), (32, 8, 64, 300, 8000, 44), (32, 8, 64, 800, 4000, 30), (32, 4, 128, 512, 4096, 36),
+                                                    (32, 8, 96, 300, 4000, 23)])
+def test_long_chains_are_rounded_once_a_tile(hip, H, KV, hd, T, cached, chain):  # noqa: F811
+    """chain: tiles that one group of wavefronts walks through, as planned.  A result is the sum of as many, rounded once for each (2^-24 of it at
+    most, at random), and comes from scores whose errors move it by four times that at most: the root of the sum of squares."""
+    import torch
+
+    plan = hip.describe_plan(H, KV, hd, [cached], [T])
+    tiles = -(-(-(-(cached + T) // 32)) // plan["key_chunks"])
+    assert plan["groups"] in (2, 3) and -(-tiles // (2 if plan["groups"] == 2 else 1)) == chain, plan
+    S, g = cached + T, H // KV
+    r = torch.Generator(device="cuda").manual_seed(hd + T)
+    q, k, v = (torch.randn((T, n * hd), generator=r, device="cuda") for n in (H, KV, KV))
+    kc, vc = (torch.randn((KV, cached, hd), generator=r, device="cuda") for _ in range(2))
+    ctx = hip.AttnContext(H, KV, hd, max_positions=S)
+    torch.cuda.synchronize()
+    cache = hip.KVCache(ctx, 1, S)
+    cache.fill(0, kc, vc)
+    ctx.sync()
+    got = ctx.forward(cache, q, k, v, [T])
+    ctx.sync()
+    got = got.double().reshape(T, H, hd)
+    qr = torch.tensor(ctx.last_q_rot(T), device="cuda").double().reshape(T, H, hd)
+    hidden = torch.arange(S, device="cuda")[None] > cached + torch.arange(T, device="cuda")[:, None]
+    off = size = 0.0
+    for h in range(0, H, g):  # one head of each group
+        kr, vr = (torch.tensor(a, device="cuda").double() for a in cache.read(0, h // g, 0, S))
+        s = (qr[:, h] @ kr.T.contiguous() / hd ** 0.5).masked_fill(hidden, float("-inf"))
+        want = torch.softmax(s, -1) @ vr
+        off += ((got[:, h] - want) ** 2).sum().item()
+        size += (want ** 2).sum().item()
+    assert (off / size) ** 0.5 <= 2.0 ** -24 * (chain + 16) ** 0.5, ((off / size) ** 0.5, 2.0 ** -24 * (chain + 16) ** 0.5)
+    cache.close()
+    ctx.close()
