@@ -112,13 +112,15 @@ struct TileUnits {
 // (split_mfma.hpp): the queries once, a key tile by the workgroup on its way to LDS, the probabilities in
 // the registers the scores came in.  A tile costs a wavefront HD / 16 x 12 + HD / 16 x 12 MFMAs of 16 cycles (64:
 // 1536) where the fp32 instruction took HD x 64 (4096).
-// Us, v_mfma_f32_32x32x16_bf16 with both wavefronts of a SIMD in step | this: 2048 rows, 32 / 8 heads of 64, 111 | 100, 4096 rows 380 | 317, 512 rows on
-// 16384 376 | 319; 512 rows on 16384, 32 / 4 heads of 128, 715 | 580, 2048 rows, 32 / 8 heads of 128, 225 | 204, 4096 rows 763 | 616; 2048 rows of 32 heads of 96
-// 219 | 186; 32 / 8 heads of 64, 45 rows 11.9 | 12.3, 600 and
-// 700 33.0 | 33.8 and 35.9 | 36.4 (start and end of a workgroup).  Errors against 64 bits 2 to 15 % smaller.
+// Us, v_mfma_f32_32x32x16_bf16 with both wavefronts of a SIMD in step | this: 2048 rows, 32 / 8 heads of 64, 108.5 | 97.6, 4096 rows 374 | 309, 512 rows on
+// 16384 369 | 308; 512 rows on 16384, 32 / 4 heads of 128, 700 | 558, 2048 rows, 32 / 8 heads of 128, 222 | 194, 4096 rows 748 | 601; 2048 rows of 32 heads of 96
+// 216 | 187; 32 / 8 heads of 64, 45 rows 12.4 | 11.7 (G = 3); 600 and 700 rows 33.1 | 34.2 and 36.1 | 36.6 one after the other (start and end of a workgroup, which leaves the
+// compute units that it does not need to others: 17.3 | 12.2 and 21.7 | 21.7 among calls of other contexts).  Errors against 64 bits: below, at kTwoSums.
 // What each part of it gave: half a step apart 104 | 100 and fragments a block ahead of their MFMAs 98; the layout of LDS without conflicts 96 | 92.6; a block's
-// products on one accumulator rather than two in turn 1 %; two row blocks a workgroup and the queries' third parts in LDS, which ended spills, 656 | 568 (512 rows on 16384, heads of 128).  In step
+// products on one accumulator rather than two in turn 1 %; two row blocks a workgroup and the queries' third parts in LDS 656 | 568 (512 rows on 16384, heads of 128).  In step
 // again (no group waits half a step at the start) short ranges take 2 to 10 % longer.
+// Registers: none spilled but for heads of 128 in turns (11, of padded tiles 14, with values by distance 33), with values by distance (2 to 20) and in padded tiles of G = 3
+// (2); mostly where a row block begins and ends (in the blocks of code that hold the MFMAs: none in turns, 2 or 3 accesses a tile with values by distance, 1 in padded G = 3).
 // What bounds it: heads of 128 the power the card may draw (matrix cores busy 78 % at 1.9 GHz); heads of 64 vector instructions: 281 and 16
 // exponentials a tile and wavefront, of which a SIMD issues two during an MFMA of 16 cycles.  (Queries and keys as two fp16 numbers and scores of three products
 // took 14 and 17 % less, but such numbers leave out up to 2^-21 of a product, and where a key's second parts have the signs of the

@@ -469,6 +469,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void sgemm_split_kernel(const Gemm
 // 2048 -> 16384 320 | 298, 777 rows 149 | 131, 512 rows 93 | 83, 300 rows 82 | 76, 512 rows of 2048 -> 3072 32.4 | 30.6, 2048 rows of 2048 -> 2048 58 | 55,
 // 8192 -> 2048 173 | 160, 512 rows 57 | 58.  The copies are not counted by the compiler: a step ends with a wait for all but its loads of W,
 // which are requested behind them.
+// Registers: tiles of 128 x 256 keep all, those of 256 x 256 spill 72 to 89 of a lane's (292 to 348 bytes of scratch), addresses and what a tile begins and ends with: none of it
+// in the block that holds the MFMAs.
 // What bounds it: on zeros 2048 rows of 2048 -> 16384 (x itself) take 279 us, of which the MFMAs and fragments are 201, splits 26, writes to LDS 31 (17
 // cycles each while MFMAs run) and loads 21; on random numbers the clock is at 2.06 GHz.
 // END: K ends with a step (kWhole; PLANES always); within one (kShifted): the last step is moved back until it ends with K, and what the steps before it
