@@ -80,6 +80,18 @@ def test_short_ranges_are_not_shared_by_two_groups():
         assert plan["groups"] == groups, (H, KV, hd, B, cached, new, plan)
 
 
+def test_chunks_of_heads_over_64_stay_with_a_row_block_a_workgroup():
+    # two row blocks a workgroup round a chain of sums six times a tile: only where ranges are long enough for 1024 blocks and chunks, as ever
+    for hd, (H, KV), S, T in itertools.product((96, 128), ((32, 8), (32, 4), (16, 8), (8, 8), (24, 4)), (0, 200, 1000, 3000, 6000, 12000),
+                                               (40, 100, 200, 400, 700, 1000, 1200, 1500, 2000, 2500)):
+        plan = plan_of(H, KV, hd, S, T)
+        if plan["path"] != sa.hip.PATH_PREFILL or plan["key_chunks"] == 1:
+            continue
+        blocks = -(-T * (H // KV) // 128) * KV
+        long = -(-(S + T) // 32) // -(-1024 // blocks) >= 32
+        assert long or blocks * plan["key_chunks"] <= 768 and plan["groups"] != 1, (hd, H, KV, S, T, plan)
+
+
 def test_decode_and_generic_paths_are_told_apart():
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [1] * 16)["path"] == sa.hip.PATH_DECODE
     assert sa.describe_plan(32, 8, 128, [5000] * 16, [8] * 16)["path"] == sa.hip.PATH_DECODE  # two entries each
